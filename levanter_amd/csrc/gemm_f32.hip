@@ -1,0 +1,192 @@
+// y = act(a . w^T + bias) + residual in 32 bits on the 32-bit matrix instruction (v_mfma_f32_16x16x4_f32: full 32-bit products and
+// sums, no reduced mode). a [M, K] (row stride lda), w [N, K], y [M, N].
+#include "common.h"
+#include <math.h>
+
+typedef __attribute__((ext_vector_type(4))) float gf_f32x4;
+
+// A workgroup of W waves owns 16 RT rows and 16 NT outputs; its waves split K (steps of 16 dealt in stretches) and the partial sums are
+// added through LDS in wave order. The product is transposed, out^T = w a^T, so that a lane ends with four neighbouring outputs of one
+// row. Both operands come straight from global memory, 16 bytes a lane (row = lane % 16, k = 4 (lane / 16) + j for the j-th of the
+// four products of a step): the 32-bit instruction takes 32 cycles for 1,024 multiply-adds, so that operands through LDS would buy
+// nothing that the caches do not give, but for tiles too small for their L2 traffic.
+// What bounds it: few rows, the read of the weights (4096 x 4096 at 4 rows 14.3 us, 4.7 TB/s; 768 x 768 4.8 us, a launch and a chain of
+// loads); some hundred rows, L2 at about 9.5 TB/s (1024 x 4096 at 203 rows 33 us) or the last round of tiles; many, the matrix pipe
+// (4096 x 4096 at 2,048 rows 532 us, 129 TFLOP/s of 157). The plain kernel of gemm_simple.hip (64 x 64 tiles, vector ALU, scalar loads)
+// took 84 us for 768 x 768 at 4 rows, 378 us for 768 x 3072, 2,417 us for 50257 x 1024 at 777 rows (now 4.8, 10 and 727).
+template <int RT, int NT, int W>
+__global__ void __launch_bounds__(64 * W)
+gemm_f32_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
+                const float* residual, long ldr, float* out, long ldo, int M, int N, int K, int act, int n_rows, int n_cols, int vec) {
+  extern __shared__ __attribute__((aligned(16))) float gf_part[];  // [W][RT * NT][64][4]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, g = lane >> 4;
+  // the chiplets (workgroups are dealt to the eight in turn) take neighbouring columns of tiles each, rows fastest: a weight is read by
+  // one chiplet's L2 only
+  const int n_tiles = n_rows * n_cols, per = (n_tiles + 7) / 8;
+  const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= per || tile >= n_tiles) return;  // the whole workgroup
+  const int m0 = (tile % n_rows) * 16 * RT, o0 = (tile / n_rows) * 16 * NT;
+  const float *ar[RT], *wr[NT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) ar[i] = a + (size_t)min(m0 + 16 * i + col, M - 1) * lda;  // rows beyond the matrix: read again, never stored
+#pragma unroll
+  for (int j = 0; j < NT; ++j) wr[j] = w + (size_t)min(o0 + 16 * j + col, N - 1) * K;
+  gf_f32x4 acc[RT][NT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+  const int share = (K + 16 * W - 1) / (16 * W) * 16;
+  const int k_lo = min(K, wave * share), k_hi = min(K, k_lo + share);
+  const int k_full = k_lo + (k_hi - k_lo) / 16 * 16;
+  auto load = [&](int k0, gf_f32x4 (&av)[RT], gf_f32x4 (&wv)[NT]) {
+    const int kk = k0 + 4 * g;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) wv[j] = *reinterpret_cast<const gf_f32x4*>(wr[j] + kk);
+#pragma unroll
+    for (int i = 0; i < RT; ++i) av[i] = *reinterpret_cast<const gf_f32x4*>(ar[i] + kk);
+  };
+  auto products = [&](const gf_f32x4 (&av)[RT], const gf_f32x4 (&wv)[NT]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[j][e], av[i][e], acc[i][j], 0, 0, 0);
+  };
+  // steps whose loads are on their way at a time; a wave with many products a step instead asks for the next step ahead of this one's products
+  constexpr bool AHEAD = RT * NT >= 4;
+  constexpr int U = AHEAD ? 2 : 4;
+  gf_f32x4 av[U][RT], wv[U][NT];
+  int k0 = k_lo;
+  if (AHEAD) {
+    if (k0 < k_full) load(k0, av[0], wv[0]);
+    for (; k0 + 32 <= k_full; k0 += 32) {
+      load(k0 + 16, av[1], wv[1]);
+      __builtin_amdgcn_sched_barrier(0);
+      products(av[0], wv[0]);
+      load(min(k0 + 32, k_full - 16), av[0], wv[0]);  // at the end: read again, not used
+      __builtin_amdgcn_sched_barrier(0);
+      products(av[1], wv[1]);
+    }
+    if (k0 < k_full) products(av[0], wv[0]);
+  } else {
+    for (; k0 + 16 * U <= k_full; k0 += 16 * U) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) load(k0 + 16 * u, av[u], wv[u]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) products(av[u], wv[u]);
+    }
+    for (; k0 < k_full; k0 += 16) {
+      load(k0, av[0], wv[0]);
+      products(av[0], wv[0]);
+    }
+  }
+  if (k_full < k_hi) {  // the last step of a K that is no multiple of 16: chunks beyond it count as zeros
+    const int kk = k_full + 4 * g, kc = min(kk, K - 4);
+    const bool in = kk < K;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      wv[0][j] = *reinterpret_cast<const gf_f32x4*>(wr[j] + kc);
+      if (!in) wv[0][j] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+      av[0][i] = *reinterpret_cast<const gf_f32x4*>(ar[i] + kc);
+      if (!in) av[0][i] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    products(av[0], wv[0]);
+  }
+  if (W > 1) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) *reinterpret_cast<gf_f32x4*>(gf_part + ((size_t)(wave * RT * NT + i * NT + j) * 64 + lane) * 4) = acc[i][j];
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int t = i * NT + j;
+      if (W > 1 && t % W != wave) continue;  // the waves finish a tile each in turn
+      gf_f32x4 v = acc[i][j];
+      if (W > 1) {
+        v = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < W; ++q) v += *reinterpret_cast<const gf_f32x4*>(gf_part + ((size_t)(q * RT * NT + t) * 64 + lane) * 4);
+      }
+      const int m = m0 + 16 * i + col, o = o0 + 16 * j + 4 * g;
+      if (m >= M || o >= N) continue;
+      if (vec && o + 4 <= N) {
+        if (bias) v += *reinterpret_cast<const gf_f32x4*>(bias + o);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = lev_activate(v[r], act);
+        if (residual) v += *reinterpret_cast<const gf_f32x4*>(residual + (size_t)m * ldr + o);
+        *reinterpret_cast<gf_f32x4*>(out + (size_t)m * ldo + o) = v;
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (o + r >= N) break;
+          float x = v[r];
+          if (bias) x += bias[o + r];
+          x = lev_activate(x, act);
+          if (residual) x += residual[(size_t)m * ldr + o + r];
+          out[(size_t)m * ldo + o + r] = x;
+        }
+      }
+    }
+  }
+}
+
+// Which tile: the fewest microseconds by an estimate from what was measured over 15 weights and 1 .. 2,048 rows (all eight tiles of the list):
+// a launch and its ramp of 4 us, and the longest of the weights' read from memory (5.2 TB/s), the operands that a CU pulls through
+// its L2 (37 GB/s and CU) and the products of the CU with the most workgroups (waves that fewer than four SIMDs hold leave the others idle).
+// Within 10 % of the best tile at nearly all of them; the ends: 16 x 16 for 768 x 768 at 4 rows (4.8 us; 64 x 64 19), 64 x 128 for
+// 4096 x 4096 at 2,048 rows (532 us; 16 x 16 1,790).
+struct GemmF32Tile {
+  int rt, nt, w;
+  float pipe;  // share of the matrix pipe that the tile reaches
+};
+static const GemmF32Tile GEMM_F32_TILES[] = {{1, 1, 8, 0.8f}, {2, 1, 8, 0.8f}, {1, 2, 8, 0.8f}, {1, 4, 8, 0.8f}, {2, 2, 4, 0.8f}, {2, 4, 4, 0.8f}, {4, 4, 4, 0.68f}, {4, 8, 2, 0.85f}};
+
+static int gemm_f32_choose(int M, int N, int K) {
+  int best = 0;
+  double best_us = 1e30;
+  for (int i = 0; i < (int)(sizeof(GEMM_F32_TILES) / sizeof(GEMM_F32_TILES[0])); ++i) {
+    const GemmF32Tile& t = GEMM_F32_TILES[i];
+    const double groups = (double)((M + 16 * t.rt - 1) / (16 * t.rt)) * ((N + 16 * t.nt - 1) / (16 * t.nt));
+    const double n = ceil(groups / 256.0), waves = n * t.w < 4.0 ? n * t.w : 4.0;
+    const double memory = 4.0 * N * K / 5.2e6;
+    const double l2 = n * ((16 * t.rt < M ? 16 * t.rt : M) + 16 * t.nt) * 4.0 * K / 37e3;
+    const double pipe = n * (K / 4.0) * t.rt * t.nt * 32.0 / waves / (2400.0 * t.pipe);
+    const double us = fmax(memory, fmax(l2, pipe));
+    if (us < best_us) best_us = us, best = i;
+  }
+  return best;
+}
+
+// 1: not for these operands (nothing has been launched): 16-byte loads need rows of a multiple of 4 numbers at 16-byte addresses
+int lev_gemm_f32(const float* a, long lda, const float* w, const float* bias, const float* residual, long ldr, float* out, long ldo, int M, int N, int K,
+                 int act, hipStream_t stream) {
+  if (K % 4 != 0 || lda % 4 != 0 || ((uintptr_t)a & 15) != 0 || ((uintptr_t)w & 15) != 0) return 1;
+  const int vec = ldo % 4 == 0 && ((uintptr_t)out & 15) == 0 && (!bias || ((uintptr_t)bias & 15) == 0) && (!residual || (ldr % 4 == 0 && ((uintptr_t)residual & 15) == 0));
+  const GemmF32Tile& t = GEMM_F32_TILES[gemm_f32_choose(M, N, K)];
+  const int n_rows = (M + 16 * t.rt - 1) / (16 * t.rt), n_cols = (N + 16 * t.nt - 1) / (16 * t.nt);
+  const long blocks = ((long)n_rows * n_cols + 7) / 8 * 8;
+  LEV_REQUIRE(blocks <= 0x7fffffffL, "linear: too many tiles (%ld)", blocks);
+#define GEMM_F32_CASE(RT, NT, W)                                                                                                                    \
+  if (t.rt == RT && t.nt == NT)                                                                                                                     \
+    gemm_f32_kernel<RT, NT, W><<<(unsigned)blocks, 64 * W, W * RT * NT * 1024, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act, n_rows, n_cols, vec)
+  GEMM_F32_CASE(1, 1, 8);
+  else GEMM_F32_CASE(2, 1, 8);
+  else GEMM_F32_CASE(1, 2, 8);
+  else GEMM_F32_CASE(1, 4, 8);
+  else GEMM_F32_CASE(2, 2, 4);
+  else GEMM_F32_CASE(2, 4, 4);
+  else GEMM_F32_CASE(4, 4, 4);
+  else GEMM_F32_CASE(4, 8, 2);
+#undef GEMM_F32_CASE
+  return lev_check_launch("linear (32-bit)");
+}

@@ -1,7 +1,10 @@
-// y = act(a . w^T + bias) + residual with plain fused multiply-adds in 32-bit: the matrix product
-// of the true 32-bit path (no matrix-core instruction, no reduced-precision mode) and a slow but
-// size-agnostic product for bfloat16 inputs.  a [M, K] (row stride lda), w [N, K], y [M, N].
+// y = act(a . w^T + bias) + residual with plain fused multiply-adds in 32-bit: a slow but size-agnostic product, for bfloat16 inputs that
+// the matrix-core kernels do not take and for 32-bit ones whose rows are no multiple of four numbers or not aligned (the others go to
+// gemm_f32.hip).  a [M, K] (row stride lda), w [N, K], y [M, N].
 #include "common.h"
+
+int lev_gemm_f32(const float* a, long lda, const float* w, const float* bias, const float* residual, long ldr, float* out, long ldo, int M, int N, int K,
+                 int act, hipStream_t stream);
 
 #define GS_TILE 64
 #define GS_BK 16
@@ -70,6 +73,10 @@ extern "C" int lev_linear_simple(const void* a, long lda, const void* w, const f
   LEV_REQUIRE(!residual || ldr >= N, "linear: residual row stride %ld is smaller than N=%d", ldr, N);
   LEV_REQUIRE(act >= LEV_ACT_NONE && act <= LEV_ACT_LAST, "linear: unknown activation %d", act);
   if (M == 0) return 0;
+  if (in_dtype == LEV_F32 && out_dtype == LEV_F32) {
+    const int rc = lev_gemm_f32((const float*)a, lda, (const float*)w, bias, residual, ldr, (float*)out, ldo, M, N, K, act, stream);
+    if (rc != 1) return rc;
+  }
   dim3 grid((N + GS_TILE - 1) / GS_TILE, (M + GS_TILE - 1) / GS_TILE);
   LEV_REQUIRE(grid.y <= 65535, "linear: too many rows (%d) for one launch", M);
   if (in_dtype == LEV_F32 && out_dtype == LEV_F32)
