@@ -1,0 +1,271 @@
+// Attention of a ragged batch over the paged cache in 32 bits, on the 32-bit matrix instruction (v_mfma_f32_16x16x4_f32), for head sizes
+// of 16 .. 128 in steps of 16. The problem is transposed, S^T = K Q^T and O^T = V^T P^T: both page layouts are then read 16 bytes a lane as
+// the instruction's first operand, and the probabilities leave the first product in the registers that the second one reads.
+//   q [T][H*HD] (row stride q_stride), out likewise; keys [page][kv_head][HD/8][PS][8], values [page][kv_head][HD][PS]
+//   scores, mask, pages that are not there and queries without a key as in attention_simple.hip
+//
+// A workgroup of W waves owns 16 columns: 16 consecutive query rows of one head (runs of several tokens), or up to 16 query heads of one
+// key/value head (single tokens). Its waves take the blocks of 16 KB keys in turn and merge through LDS in wave order.
+// What bounds it: prompts, the matrix pipe half of the time and the round trips between its batches the rest (777 rows of 16 heads of 64:
+// 35 us, 1.2 GFLOP of visible products); single tokens, the chain of one block's loads, products and merge (4 tokens of 12 heads over
+// 200 keys: 9.6 us). The plain kernel gives a wave one query row, reads keys 4 bytes at a time and walks the values key by key:
+// 1,187 us and 70 us.
+#include "common.h"
+#include <math.h>
+
+typedef __attribute__((ext_vector_type(4))) float af_f32x4;
+
+struct AttentionF32Args {
+  const float* q;
+  long q_stride;
+  float* out;
+  long o_stride;
+  const float *k_pages, *v_pages;
+  const int *positions, *token_seq, *block_tables;
+  int bt_stride, H, KVH, PS, window, bias_len;
+  float scale, softcap;
+  const float* score_bias;
+  const int* work;  // runs: (first token, rows) per tile of the list; single tokens: their indexes
+  int tile_rows, columns;  // rows of a tile of the list (runs); columns in use (single tokens: query heads of a key/value head, at most 16)
+};
+
+template <int HD, int KB, int W, bool RUNS>
+__global__ void __launch_bounds__(64 * W)
+attention_f32_kernel(const AttentionF32Args p) {
+  extern __shared__ __attribute__((aligned(16))) float af_lds[];  // [W][HD/16][4][columns] of four outputs, then maxima and sums [2][W][16] and a tile's weights [W][16][16]
+  constexpr int DT = HD / 16;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, g = lane >> 4;
+  const int group = p.H / p.KVH, nc = RUNS ? 16 : p.columns;
+  int token, head;
+  bool mine;  // this lane's column is one
+  if (RUNS) {
+    const int subs = (p.tile_rows + 15) / 16;
+    head = blockIdx.x % p.H;
+    const int sub = blockIdx.x / p.H % subs, tile = blockIdx.x / p.H / subs;
+    const int first = p.work[2 * tile], rows = p.work[2 * tile + 1] - 16 * sub;
+    if (rows <= 0) return;  // the whole workgroup
+    mine = col < rows;
+    token = first + 16 * sub + min(col, rows - 1);
+  } else {
+    const int sets = (group + 15) / 16, kvh = blockIdx.x / sets % p.KVH, set = blockIdx.x % sets;
+    token = p.work[blockIdx.x / sets / p.KVH];
+    const int n = min(16, group - 16 * set);
+    mine = col < n;
+    head = kvh * group + 16 * set + min(col, n - 1);
+  }
+  const int kvh = head / group;
+  const int pos = p.positions[token];
+  const int first = p.window > 0 ? max(0, pos - p.window + 1) : 0;
+  int last = pos, lo = first;  // over the columns
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) {
+    last = max(last, __shfl_xor(last, o, 64));
+    lo = min(lo, __shfl_xor(lo, o, 64));
+  }
+  const int* bt = p.block_tables + (size_t)p.token_seq[token] * p.bt_stride;
+  const size_t head_elems = (size_t)HD * p.PS;
+  const float* qr = p.q + (size_t)token * p.q_stride + (size_t)head * HD;
+  af_f32x4 q[DT], o_acc[DT];
+#pragma unroll
+  for (int d = 0; d < DT; ++d) {
+    q[d] = *reinterpret_cast<const af_f32x4*>(qr + 16 * d + 4 * g) * p.scale;
+    o_acc[d] = af_f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  float* ml = af_lds + (size_t)W * DT * 4 * nc * 4;
+  float* weights = ml + 2 * W * 16 + wave * 256;
+  float m = -INFINITY, l = 0.f;
+  const int t_last = last / 16;
+  for (int t0 = lo / 16 + wave * KB; t0 <= t_last; t0 += W * KB) {
+    int page[KB], off[KB];
+#pragma unroll
+    for (int t = 0; t < KB; ++t) {
+      const int key = min(t0 + t, t_last) * 16;  // tiles behind the last are read again and masked
+      page[t] = bt[key / p.PS];
+      off[t] = key % p.PS;
+    }
+    af_f32x4 s[KB], k[KB][DT], v[KB][DT];  // all of the block's loads are on their way before the first product
+#pragma unroll
+    for (int t = 0; t < KB; ++t) {
+      const float* kb = p.k_pages + ((size_t)max(page[t], 0) * p.KVH + kvh) * head_elems + (size_t)(off[t] + col) * 8 + (g & 1) * 4;
+#pragma unroll
+      for (int d = 0; d < DT; ++d) k[t][d] = *reinterpret_cast<const af_f32x4*>(kb + (size_t)(2 * d + (g >> 1)) * p.PS * 8);
+    }
+#pragma unroll
+    for (int t = 0; t < KB; ++t) {
+      const float* vb = p.v_pages + ((size_t)max(page[t], 0) * p.KVH + kvh) * head_elems + off[t] + 4 * g;
+#pragma unroll
+      for (int d = 0; d < DT; ++d) v[t][d] = *reinterpret_cast<const af_f32x4*>(vb + (size_t)(16 * d + col) * p.PS);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < KB; ++t) {
+      s[t] = af_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[t][d][e], q[d][e], s[t], 0, 0, 0);
+    }
+    float mx = -INFINITY;
+    bool masked = false;  // some column does not see some key of the block
+#pragma unroll
+    for (int t = 0; t < KB; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int key = (t0 + t) * 16 + 4 * g + r;
+        float x = s[t][r];
+        if (p.score_bias) x += p.score_bias[(size_t)head * p.bias_len + min(max(pos - key, 0), p.bias_len - 1)];
+        if (p.softcap > 0.f) x = p.softcap * tanhf(x / p.softcap);
+        const bool live = key <= pos && key >= first && page[t] >= 0;
+        masked |= !live;
+        s[t][r] = live ? x : -INFINITY;
+        mx = fmaxf(mx, s[t][r]);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float m_new = fmaxf(m, mx);
+    const float corr = m == -INFINITY ? 0.f : expf(m - m_new);
+    float sum = 0.f;
+#pragma unroll
+    for (int t = 0; t < KB; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float e = s[t][r] == -INFINITY ? 0.f : expf(s[t][r] - m_new);  // no live key so far: m_new = -inf, all are 0
+        s[t][r] = e;
+        sum += e;
+      }
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    l = l * corr + sum;
+    m = m_new;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) o_acc[d] *= corr;
+    const bool any_masked = __any(masked);
+#pragma unroll
+    for (int t = 0; t < KB; ++t) {
+      if (any_masked) {  // the whole wave
+        // keys that nobody sees (a page may hold anything behind the last token): zeros. Keys that some columns see and others do not:
+        // their weight is 0 in the others, and 0 times infinity or NaN must not reach those: such a tile takes the sum column by column.
+        bool odd = false;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int key = (t0 + t) * 16 + 4 * g + r;
+          const bool there = key <= last && page[t] >= 0;
+#pragma unroll
+          for (int d = 0; d < DT; ++d) {
+            if (!there) v[t][d][r] = 0.f;
+            odd |= !(fabsf(v[t][d][r]) < INFINITY);
+          }
+        }
+        if (__any(odd)) {  // rare, and kept small: the weights through LDS, a key at a time
+#pragma unroll
+          for (int r = 0; r < 4; ++r) weights[(4 * g + r) * 16 + col] = s[t][r];
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // within the wave
+          const float* at = p.v_pages + ((size_t)max(page[t], 0) * p.KVH + kvh) * head_elems + off[t] + (size_t)4 * g * p.PS;
+#pragma unroll 1
+          for (int j = 0; j < 16; ++j) {
+            const int key = (t0 + t) * 16 + j;
+            const bool live = key <= pos && key >= first && page[t] >= 0;
+            const float weight = weights[j * 16 + col];
+            const float* row = at + j;
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                asm volatile("" : "+v"(row));  // one address, moved on: the compiler would keep one for each of the sums
+                if (live) o_acc[d][e] = fmaf(weight, *row, o_acc[d][e]);
+                row += e < 3 ? p.PS : 13 * p.PS;
+              }
+          }
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          continue;
+        }
+      }
+#pragma unroll
+      for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o_acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][d][e], s[t][e], o_acc[d], 0, 0, 0);
+    }
+  }
+  if (col < nc) {
+#pragma unroll
+    for (int d = 0; d < DT; ++d) *reinterpret_cast<af_f32x4*>(af_lds + ((size_t)((wave * DT + d) * 4 + g) * nc + col) * 4) = o_acc[d];
+  }
+  if (g == 0) ml[wave * 16 + col] = m, ml[(W + wave) * 16 + col] = l;
+  __syncthreads();
+  if (!mine) return;
+  float top = -INFINITY, total = 0.f, factor[W];
+#pragma unroll
+  for (int w = 0; w < W; ++w) top = fmaxf(top, ml[w * 16 + col]);
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    const float mw = ml[w * 16 + col];
+    factor[w] = mw == -INFINITY ? 0.f : expf(mw - top);
+    total += ml[(W + w) * 16 + col] * factor[w];
+  }
+  const float inv = total > 0.f || total != total ? 1.0f / total : 0.f;  // a query without a key gives zeros, a score that is NaN gives NaN
+  float* orow = p.out + (size_t)token * p.o_stride + (size_t)head * HD;
+#pragma unroll
+  for (int d = 0; d < DT; ++d) {
+    if (d % W != wave) continue;  // the waves finish 16 dimensions each in turn
+    af_f32x4 sum = af_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const af_f32x4 part = *reinterpret_cast<const af_f32x4*>(af_lds + ((size_t)((w * DT + d) * 4 + g) * nc + col) * 4);
+      if (factor[w] != 0.f) sum += part * factor[w];
+    }
+    *reinterpret_cast<af_f32x4*>(orow + 16 * d + 4 * g) = sum * inv;
+  }
+}
+
+template <int HD>
+static int attention_f32_launch(const AttentionF32Args& common, const int* tiles, int n_tiles, int tile_rows, const int* tokens, int n_tokens, hipStream_t stream) {
+  AttentionF32Args p = common;
+  constexpr int DT = HD / 16, KB = HD <= 64 ? 4 : 2, KB1 = HD <= 96 ? 2 : 1;  // as many tiles of keys as fit the registers
+  if (n_tiles > 0) {
+    constexpr int W = 4, lds = W * DT * 4 * 16 * 16 + 2 * W * 16 * 4 + W * 1024;
+    p.work = tiles, p.tile_rows = tile_rows, p.columns = 16;
+    const long blocks = (long)n_tiles * ((tile_rows + 15) / 16) * p.H;
+    LEV_REQUIRE(blocks <= 0x7fffffffL, "attention: too many tiles (%ld)", blocks);
+    attention_f32_kernel<HD, KB, W, true><<<(unsigned)blocks, 64 * W, lds, stream>>>(p);
+  }
+  if (n_tokens > 0) {
+    constexpr int W = 8;
+    const int group = p.H / p.KVH, sets = (group + 15) / 16;
+    p.work = tokens, p.tile_rows = 0, p.columns = group < 16 ? group : 16;
+    const int lds = W * DT * 4 * p.columns * 16 + 2 * W * 16 * 4 + W * 1024;
+    const long blocks = (long)n_tokens * p.KVH * sets;
+    LEV_REQUIRE(blocks <= 0x7fffffffL, "attention: too many single tokens (%ld)", blocks);
+    if (lds > 64 * 1024) {
+      const hipError_t e = hipFuncSetAttribute((const void*)attention_f32_kernel<HD, KB1, W, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      LEV_REQUIRE(e == hipSuccess, "attention: %d bytes of LDS a workgroup: %s", lds, hipGetErrorString(e));
+    }
+    attention_f32_kernel<HD, KB1, W, false><<<(unsigned)blocks, 64 * W, lds, stream>>>(p);
+  }
+  return lev_check_launch("attention (32-bit)");
+}
+
+// 1: not for these operands (nothing has been launched): head sizes in steps of 16 up to 128, rows at 16-byte addresses. tiles: (first token,
+// rows <= tile_rows) of runs of several consecutive tokens; tokens: the single ones.
+extern "C" int lev_attention_f32(const float* q, long q_stride, float* out, long o_stride, const float* k_pages, const float* v_pages, const int* positions,
+                                 const int* token_seq, const int* block_tables, int bt_stride, const int* tiles, int n_tiles, int tile_rows, const int* tokens,
+                                 int n_tokens, int H, int KVH, int HD, int PS, float scale, int window, float softcap, const float* score_bias, int bias_len,
+                                 hipStream_t stream) {
+  LEV_REQUIRE(H > 0 && KVH > 0 && H % KVH == 0, "attention: bad head counts heads=%d kv_heads=%d", H, KVH);
+  LEV_REQUIRE(PS > 0 && PS % 16 == 0, "attention: page_size=%d must be a multiple of 16", PS);
+  LEV_REQUIRE(window >= 0, "attention: window=%d must not be negative", window);
+  LEV_REQUIRE(softcap >= 0.f && (!score_bias || bias_len >= 1), "attention: soft cap %g must not be negative and a bias table needs entries (%d)", (double)softcap, bias_len);
+  LEV_REQUIRE(n_tiles >= 0 && n_tokens >= 0 && (n_tiles == 0 || (tiles && tile_rows > 0)) && (n_tokens == 0 || tokens), "attention: a work list is missing");
+  if (HD % 16 != 0 || HD < 16 || HD > 128 || q_stride % 4 != 0 || o_stride % 4 != 0) return 1;
+  if ((((uintptr_t)q | (uintptr_t)out | (uintptr_t)k_pages | (uintptr_t)v_pages) & 15) != 0) return 1;
+  const AttentionF32Args p{q, q_stride, out, o_stride, k_pages, v_pages, positions, token_seq, block_tables, bt_stride, H, KVH, PS, window, bias_len, scale, softcap, score_bias, nullptr, 0, 0};
+  switch (HD / 16) {
+    case 1: return attention_f32_launch<16>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+    case 2: return attention_f32_launch<32>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+    case 3: return attention_f32_launch<48>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+    case 4: return attention_f32_launch<64>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+    case 5: return attention_f32_launch<80>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+    case 6: return attention_f32_launch<96>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+    case 7: return attention_f32_launch<112>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+    default: return attention_f32_launch<128>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+  }
+}

@@ -1,5 +1,5 @@
 // Attention of a ragged batch of query tokens over the paged cache, with plain 32-bit arithmetic:
-// the attention of the true 32-bit path, and a size-agnostic one for bfloat16 caches.
+// a size-agnostic attention for bfloat16 caches, and for 32-bit ones whose head sizes or rows attention_f32.hip does not take.
 // One wave per (query token, head). Keys are visited 64 at a time with an online softmax.
 //   q     [T][H*HD] (row stride q_stride), out likewise
 //   keys  [page][kv_head][HD/8][PS][8], values [page][kv_head][HD][PS]

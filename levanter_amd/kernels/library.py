@@ -1333,6 +1333,13 @@ class HipKernels:
                 _ptr(dest) if k_new is not None else None, ws_ptr, n_heads, n_kv_heads, head_dim, page_size,
                 splits, float(scale), w, cap, _ptr(score_bias), bias_len, self._s()))
             return k_new is not None
+        if dt == torch.float32:
+            rc = self.lib.lev_attention_f32(_ptr(q), qs, _ptr(out), os_, _ptr(k_pages), _ptr(v_pages), pos_ptr, seq_ptr, bt_ptr, bt_width, tiles_ptr,
+                                            meta.n_prefill_tiles, self.prefill_tile_rows, decode_ptr, meta.n_decode, n_heads, n_kv_heads, head_dim, page_size,
+                                            float(scale), w, cap, _ptr(score_bias), bias_len, self._s())
+            if rc <= 0:
+                self._check(rc)
+                return False
         self._check(self.lib.lev_attention_simple(
             _ptr(q), qs, _ptr(out), os_, _ptr(k_pages), _ptr(v_pages), pos_ptr, seq_ptr, bt_ptr, bt_width, T, n_heads, n_kv_heads,
             head_dim, page_size, float(scale), w, _DT[dt], cap, _ptr(score_bias), bias_len, self._s()))

@@ -58,3 +58,74 @@ def test_linear_float32_keeps_infinities_where_they_are(K):
     assert torch.equal(torch.isinf(out), torch.isinf(want)) and not bool(torch.isnan(out).any())
     keep = [r for r in range(20) if r != 7]
     torch.testing.assert_close(out[keep], want[keep], rtol=1e-5, atol=52 * EPS * 50)
+
+
+def _attention_float64(q, kp, vp, bt, runs, H, KVH, HD, PS, scale, window):
+    """Whole sequences from the pages in float64; only what a query sees is read."""
+    out, t = [], 0
+    for s, (n, kv) in enumerate(runs):
+        pages = bt[s, :(kv + PS - 1) // PS].long()
+        k = kp.view(-1, KVH, HD // 8, PS, 8)[pages].permute(1, 0, 3, 2, 4).reshape(KVH, -1, HD)[:, :kv].double()
+        v = vp.view(-1, KVH, HD, PS)[pages].permute(1, 0, 3, 2).reshape(KVH, -1, HD)[:, :kv].double()
+        for i in range(n):
+            pos = kv - n + i
+            lo = max(0, pos - window + 1) if window else 0
+            for h in range(H):
+                w = torch.softmax(k[h * KVH // H, lo:pos + 1] @ q[t, h * HD:(h + 1) * HD].double() * scale, 0)
+                out.append(w @ v[h * KVH // H, lo:pos + 1])
+            t += 1
+    return torch.stack(out).view(t, H * HD)
+
+
+# runs of (tokens, keys after the step): tiles of 16 rows with 1 to 16 in use, blocks of 64 and 32 keys at their edges, single tokens beside
+# them; groups of heads that fill a column set, more and less; every head size
+ATTENTION = [(4, 4, 64, 16, [(2, 2), (17, 17), (1, 64), (1, 65), (15, 80)], None), (16, 1, 16, 16, [(1, 1), (1, 33), (3, 130)], None),
+             (20, 1, 32, 32, [(1, 257), (18, 18)], 20), (6, 2, 48, 16, [(1, 300), (129, 140)], 64), (5, 5, 80, 48, [(33, 97), (1, 31)], None),
+             (3, 1, 96, 16, [(1, 128), (16, 16)], 17), (2, 2, 112, 64, [(1, 127), (31, 31)], None), (8, 4, 128, 16, [(1, 513), (40, 72), (1, 2)], 1)]
+
+
+@pytest.mark.parametrize("H,KVH,HD,PS,runs,window", ATTENTION)
+def test_attention_float32(K, H, KVH, HD, PS, runs, window):
+    """Weights are off by the scores' rounding, HD * 2^-24 of |q| |k| * scale (about 40 here) and a few units of the exponential: 2e-5 of the values."""
+    from helpers import make_meta
+    from test_gpu_kernels import _fill_cache
+
+    kv = [k for _, k in runs]
+    bt, kp, vp, kd, vd, _, _ = _fill_cache(K, torch.float32, kv, KVH, HD, PS, sum((k + PS - 1) // PS for k in kv) + 3, seed=5)
+    T = sum(n for n, _ in runs)
+    q = _rand(T, H * HD + 4, seed=6)
+    want = _attention_float64(q, kp, vp, bt, runs, H, KVH, HD, PS, HD ** -0.5, window)
+    for shift in (0, 1):  # the second time nothing is aligned: the plain kernel
+        qd = torch.empty(T * (H * HD + 4) + shift, device=DEV)[shift:].view(T, H * HD + 4)
+        qd.copy_(q)
+        got = torch.full((T, H * HD), float("nan"), device=DEV)
+        K.paged_attention(qd[:, :H * HD], got, kd, vd, make_meta(runs, DEV), n_heads=H, n_kv_heads=KVH, head_dim=HD, page_size=PS, scale=HD ** -0.5,
+                          window=window, block_tables=bt.to(DEV))
+        torch.testing.assert_close(got.cpu().double(), want, rtol=2e-5, atol=2e-5)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_attention_float32_values_that_are_not_seen_do_not_count(K, bad):
+    """Token 20's value is not a number: queries before it are what they are without it, the ones from it on carry it. A single token whose block
+    has no page (a request's page that was given back) gives zeros."""
+    from helpers import make_meta
+    from test_gpu_kernels import _fill_cache
+
+    H, KVH, HD, PS, runs = 4, 2, 64, 16, [(40, 40), (1, 30)]
+    bt, kp, vp, kd, vd, _, _ = _fill_cache(K, torch.float32, [40, 30], KVH, HD, PS, 8, seed=5)
+    q = _rand(41, H * HD, seed=6).to(DEV)
+    args = dict(n_heads=H, n_kv_heads=KVH, head_dim=HD, page_size=PS, scale=0.125, window=None)
+    clean, got = torch.empty(41, H * HD, device=DEV), torch.empty(41, H * HD, device=DEV)
+    K.paged_attention(q, clean, kd, vd, make_meta(runs, DEV), block_tables=bt.to(DEV), **args)
+    vd.view(-1, KVH, HD, PS)[int(bt[0, 1]), 1, 3, 4] = bad
+    bt[1, :] = -1
+    K.paged_attention(q, got, kd, vd, make_meta(runs, DEV), block_tables=bt.to(DEV), **args)
+    heads = got.view(41, H, HD)
+    hit = torch.zeros(41, H, HD, dtype=torch.bool, device=DEV)
+    hit[20:40, 2:, 3] = True
+    assert bool((~torch.isfinite(heads) == hit).all())
+    assert bool((got[40] == 0).all())
+    rest = ~hit
+    rest[40] = False
+    # the other sums of that tile go key by key: another order of at most 40 terms of at most 5, each off by 2^-24 of it
+    torch.testing.assert_close(heads[rest], clean.view(41, H, HD)[rest], rtol=0, atol=40 * 5 * EPS)
