@@ -422,14 +422,17 @@ moe_linear_splitk_kernel(const bf16_t* __restrict__ a, long a_stride, const bf16
   }
 }
 
-// Tiles of 128 rows (prompts, large batches): a workgroup of four waves owns 128 rows and 128 weight rows (with glu: 64 outputs' gate
-// rows and the same outputs' up rows), a wave 64 x 64 of them, so that a fragment from LDS feeds four products. K goes by in steps of 64,
-// two steps on their way in registers and two buffers in LDS (rows 72 elements apart), one barrier a step. Rows beyond the tile are
-// read again and never stored; a wave whose 64 rows all lie beyond it does not compute. The workgroups of a tile and of its neighbours
-// in the list (an expert's rows, its weights) follow each other on one of the eight chiplets (workgroups are dealt to them in turn).
+// Tiles of 128 rows (prompts, large batches): a workgroup of four waves owns 128 rows and BN weight rows (with glu: BN / 2 outputs' gate
+// rows and the same outputs' up rows), a wave 64 x BN / 2 of them in 32x32x16 products (the transposed product out^T = w a^T: a lane ends
+// with four neighbouring outputs of a row). K goes by in steps of 64, the step after next on its way in registers, two buffers in LDS,
+// one barrier a step that waits for LDS only; loads, LDS writes and fragment reads are issued one by one between the products. Rows
+// beyond the tile are read again and never stored. The workgroups of a tile and of its neighbours in the list (an expert's rows, its
+// weights) follow each other on one of the eight chiplets (workgroups are dealt to them in turn).
+#define MOE_BN 128
 #define MOE_BIG_K 64
 #define MOE_BIG_LD (MOE_BIG_K + 8)
-#define MOE_BIG_LDS (2 * 2 * MOE_BIG * MOE_BIG_LD * (int)sizeof(bf16_t))
+#define MOE_BIG_LDS(BN) (2 * (MOE_BIG + (BN)) * MOE_BIG_LD * (int)sizeof(bf16_t))
+typedef __attribute__((ext_vector_type(16))) float moe_f32x16;
 template <typename TO>
 __device__ __forceinline__ void moe_store4(TO* p, const float (&v)[4], int n, bool vec);
 template <>
@@ -449,108 +452,174 @@ __device__ __forceinline__ void moe_store4<bf16_t>(bf16_t* p, const float (&v)[4
       if (r < n) p[r] = float_to_bf16(v[r]);
 }
 
-template <typename TO, bool GLU>
-__global__ void __launch_bounds__(256, 2)
-moe_linear_big_kernel(const bf16_t* __restrict__ a, long a_stride, const bf16_t* __restrict__ w, TO* __restrict__ out, long o_stride,
-                      const int* __restrict__ tiles, const int* __restrict__ meta, const int* __restrict__ sorted, int top, int gather,
-                      int K, int N, int F, int act, float limit, float up_shift, int n_cols, int vec) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char moe_smem[];
-  bf16_t* sa = reinterpret_cast<bf16_t*>(moe_smem);    // [2][128][72]
-  bf16_t* sw = sa + 2 * MOE_BIG * MOE_BIG_LD;          // [2][128][72]
-  constexpr int BN = GLU ? MOE_BIG / 2 : MOE_BIG;      // outputs of a workgroup
-  const int n_tiles = meta[0], per = (n_tiles + 7) / 8;
-  if (per == 0) return;
-  const int slot = blockIdx.x >> 3, tile = (blockIdx.x & 7) * per + slot % per, ycol = slot / per;
-  if (ycol >= n_cols || tile >= n_tiles) return;  // the whole workgroup
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, g = lane >> 4;
-  const int wr = wave >> 1, wc = wave & 1;
-  const int o0 = ycol * BN;
-  const int e = tiles[3 * tile], first = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
-  // what this thread fetches: a chunk of 8 elements of four activation rows and of four weight rows per step
-  const int lrow = tid >> 3, lk = (tid & 7) * 8;
-  const bf16_t *ap[4], *wp[4];
+struct MoeLinearArgs {
+  const bf16_t* a;
+  long a_stride;
+  const bf16_t* w;
+  void* out;
+  long o_stride;
+  const int *tiles, *meta, *sorted;
+  int top, gather, K, N, F, act;
+  float limit, up_shift;
+  int n_cols, vec;
+};
+// BM: 128, or 64 for a tile whose rows fit that
+template <typename TO, bool GLU, int BN, int BM>
+__device__ __forceinline__ void moe_big_tile(const MoeLinearArgs& p, unsigned char* moe_smem, int e, int first, int rows, int ycol) {
+  constexpr int LD = MOE_BIG_LD, WM = BM / 2, WN = BN / 2, TI = WM / 32, TJ = WN / 32;
+  constexpr int CA = BM * (MOE_BIG_K / 8) / 256, CW = BN * (MOE_BIG_K / 8) / 256;  // 16-byte chunks a thread fetches a step
+  constexpr int OUT = GLU ? BN / 2 : BN;  // outputs of a workgroup
+  const int K = p.K, N = p.N, F = p.F, act = p.act;
+  bf16_t* sa = reinterpret_cast<bf16_t*>(moe_smem);  // [2][BM][LD]
+  bf16_t* sw = sa + 2 * BM * LD;                     // [2][BN][LD]
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
+  const int o0 = ycol * OUT;
+  const int kc = (tid & 7) * 8;
+  const bf16_t* we = p.w + (size_t)e * N * K;
+  const bf16_t *pa[CA], *pw[CW];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = lrow + 32 * i;
-    const int pos = first + min(r, rows - 1);
-    ap[i] = a + (size_t)(gather ? sorted[pos] / top : pos) * a_stride;
-    const int o = min(o0 + (r % BN), F - 1) + (r >= BN ? F : 0);
-    wp[i] = w + ((size_t)e * N + o) * K;
+  for (int i = 0; i < CA; ++i) {
+    const int pos = first + min((tid + 256 * i) >> 3, rows - 1);
+    pa[i] = p.a + (size_t)(p.gather ? p.sorted[pos] / p.top : pos) * p.a_stride;
   }
-  moe_f32x4 acc[4][4];
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) acc[rt][nt] = moe_f32x4{0.f, 0.f, 0.f, 0.f};
-  moe_u32x4 ra0[4], rw0[4], ra1[4], rw1[4];
-  auto fetch = [&](int k0, moe_u32x4 (&ra)[4], moe_u32x4 (&rw)[4]) {
-    const int kk = k0 + lk, kc = min(kk, K - 8);  // loads stand under no condition; a chunk beyond the row counts as zeros
-    const uint32_t keep = kk < K ? 0xffffffffu : 0u;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const moe_u32x4 x = *reinterpret_cast<const moe_u32x4*>(ap[i] + kc);
-      ra[i] = moe_u32x4{x[0] & keep, x[1] & keep, x[2] & keep, x[3] & keep};
-      rw[i] = *reinterpret_cast<const moe_u32x4*>(wp[i] + kc);
-    }
+  for (int i = 0; i < CW; ++i) {
+    const int r = (tid + 256 * i) >> 3, q = r % WN;  // with glu a wave's weight rows are its outputs' gate rows, then their up rows
+    const int o = GLU ? min(o0 + r / WN * (WN / 2) + q % (WN / 2), F - 1) + (q >= WN / 2 ? F : 0) : min(o0 + r, F - 1);
+    pw[i] = we + (size_t)o * K;
+  }
+  // the steps in the order they are taken: a partial one (K % 64 != 0) first, so that the loop needs no masks
+  const int tail = K % MOE_BIG_K, steps = (K + MOE_BIG_K - 1) / MOE_BIG_K, shift = tail ? 1 : 0;
+  auto k_of = [&](int t) { return max(min(t, steps - 1) - shift, 0) * MOE_BIG_K; };  // t >= 1; beyond the last: loaded again, not used
+  moe_u32x4 ra[2][CA], rw[2][CW];
+  auto fetch_one = [&](int set, int k, int i) {
+    if (i < CA) ra[set][i] = *reinterpret_cast<const moe_u32x4*>(pa[i] + k);
+    else rw[set][i - CA] = *reinterpret_cast<const moe_u32x4*>(pw[i - CA] + k);
   };
-  auto stage = [&](int buf, const moe_u32x4 (&ra)[4], const moe_u32x4 (&rw)[4]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      *reinterpret_cast<moe_u32x4*>(sa + ((size_t)buf * MOE_BIG + lrow + 32 * i) * MOE_BIG_LD + lk) = ra[i];
-      *reinterpret_cast<moe_u32x4*>(sw + ((size_t)buf * MOE_BIG + lrow + 32 * i) * MOE_BIG_LD + lk) = rw[i];
-    }
+  bf16_t* a_st = sa + (tid >> 3) * LD + kc;
+  bf16_t* w_st = sw + (tid >> 3) * LD + kc;
+  auto stage_one = [&](int set, int buf, int i) {
+    if (i < CA) *reinterpret_cast<moe_u32x4*>(a_st + (buf * BM + i * 32) * LD) = ra[set][i];
+    else *reinterpret_cast<moe_u32x4*>(w_st + (buf * BN + (i - CA) * 32) * LD) = rw[set][i - CA];
   };
-  const bool active = wr * 64 < rows;
-  auto multiply = [&](int buf) {
-    if (!active) return;  // the whole wave
+  moe_f32x16 acc[TI][TJ];
 #pragma unroll
-    for (int ks = 0; ks < MOE_BIG_K; ks += 32) {
-      moe_u32x4 av[4], wv[4];
+  for (int i = 0; i < TI; ++i)
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt)
-        av[rt] = *reinterpret_cast<const moe_u32x4*>(sa + ((size_t)buf * MOE_BIG + wr * 64 + 16 * rt + col) * MOE_BIG_LD + ks + 8 * g);
+    for (int j = 0; j < TJ; ++j)
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        const int r = GLU ? (nt < 2 ? wc * 32 + 16 * nt : BN + wc * 32 + 16 * (nt - 2)) : wc * 64 + 16 * nt;
-        wv[nt] = *reinterpret_cast<const moe_u32x4*>(sw + ((size_t)buf * MOE_BIG + r + col) * MOE_BIG_LD + ks + 8 * g);
-      }
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  {
+    const int k0 = tail ? K - tail : 0, k = min(k0 + kc, K - 8);
+    const bool in = k0 + kc < K;
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt)
+    for (int i = 0; i < CA + CW; ++i) fetch_one(0, k, i);
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt)
-          acc[rt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(moe_as_bf16x8(wv[nt]), moe_as_bf16x8(av[rt]), acc[rt][nt], 0, 0, 0);
-    }
-  };
-  const int steps = (K + MOE_BIG_K - 1) / MOE_BIG_K;
-  fetch(0, ra0, rw0);
-  fetch(MOE_BIG_K, ra1, rw1);  // beyond K: clamped and zero
-  stage(0, ra0, rw0);
+    for (int i = 0; i < CA; ++i) if (!in) ra[0][i] = moe_u32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < CW; ++i) if (!in) rw[0][i] = moe_u32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < CA + CW; ++i) stage_one(0, 0, i);
+    const int k1 = min(k_of(1) + kc, K - 8);
+#pragma unroll
+    for (int i = 0; i < CA + CW; ++i) fetch_one(1, k1, i);
+  }
   lds_barrier();
-  for (int st = 0; st < steps; st += 2) {  // the buffers and the register sets take turns; conditions are uniform over the workgroup
-    if (st + 2 < steps) fetch((st + 2) * MOE_BIG_K, ra0, rw0);
-    multiply(0);
-    if (st + 1 >= steps) break;
-    stage(1, ra1, rw1);  // nobody reads that buffer: every wave has passed the barrier behind the step that did
-    lds_barrier();
-    if (st + 3 < steps) fetch((st + 3) * MOE_BIG_K, ra1, rw1);
-    multiply(1);
-    if (st + 2 < steps) stage(0, ra0, rw0);
-    lds_barrier();
-  }
+  constexpr int KS = MOE_BIG_K / 16, NM = TI * TJ, NR = TI + TJ, PW = (CA + CW + KS - 2) / (KS - 1);
+  const bf16_t* a_rd = sa + (wm * WM + (lane & 31)) * LD + (lane >> 5) * 8;
+  const bf16_t* w_rd = sw + (wn * WN + (lane & 31)) * LD + (lane >> 5) * 8;
+  moe_u32x4 af[2][TI], wf[2][TJ];
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt) {
-    const int row = wr * 64 + 16 * rt + col;
+  for (int i = 0; i < TI; ++i) af[0][i] = *reinterpret_cast<const moe_u32x4*>(a_rd + i * 32 * LD);
+#pragma unroll
+  for (int j = 0; j < TJ; ++j) wf[0][j] = *reinterpret_cast<const moe_u32x4*>(w_rd + j * 32 * LD);
+  // step t: register set `cur` (step t + 1) goes to the other buffer, the other set receives step t + 2; the last products cover the first
+  // fragment reads of step t + 1 behind the barrier
+  auto step = [&](int t, int cur) {
+    const int buf = t & 1, k = min(k_of(t + 2) + kc, K - 8);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int c = ks & 1, nx = c ^ 1, from = ks + 1 < KS ? buf : buf ^ 1, at = ks + 1 < KS ? (ks + 1) * 16 : 0;
+      if (ks + 1 == KS) lds_barrier();
+#pragma unroll
+      for (int i = 0; i < TI; ++i) af[nx][i] = *reinterpret_cast<const moe_u32x4*>(a_rd + (from * BM + i * 32) * LD + at);
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) wf[nx][j] = *reinterpret_cast<const moe_u32x4*>(w_rd + (from * BN + j * 32) * LD + at);
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(moe_as_bf16x8(wf[c][j]), moe_as_bf16x8(af[c][i]), acc[i][j], 0, 0, 0);
+      if (ks + 1 < KS) {
+#pragma unroll
+        for (int q = 0; q < PW; ++q)
+          if (ks * PW + q < CA + CW) stage_one(cur, buf ^ 1, ks * PW + q);
+#pragma unroll
+        for (int q = 0; q < PW; ++q)
+          if (ks * PW + q < CA + CW) fetch_one(cur ^ 1, k, ks * PW + q);
+      }
+      constexpr int others = NR + 2 * PW;
+#pragma unroll
+      for (int m = 0; m < NM; ++m) {  // the order of issue: a product, then at most a few of the others
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        const int n = ks + 1 < KS ? others : NR, lo = m * n / NM, hi = (m + 1) * n / NM;
+#pragma unroll
+        for (int o = lo; o < hi; ++o) {
+          if (o < NR) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          else if (o < NR + PW) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+          else __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        }
+      }
+    }
+  };
+  int t = 0;
+  for (; t + 1 < steps; t += 2) {
+    step(t, 1);
+    step(t + 1, 0);
+  }
+  if (t < steps) step(t, 1);
+  // register r of a 32 x 32 tile: output 8 (r / 4) + 4 (lane / 32) + r % 4 of the tile, row lane % 32
+#pragma unroll
+  for (int i = 0; i < TI; ++i) {
+    const int row = wm * WM + 32 * i + (lane & 31);
     if (row >= rows) continue;
 #pragma unroll
-    for (int nt = 0; nt < (GLU ? 2 : 4); ++nt) {
-      const int o = o0 + wc * (GLU ? 32 : 64) + 16 * nt + 4 * g;
-      if (o >= F) continue;
-      float v[4];
+    for (int j = 0; j < (GLU ? TJ / 2 : TJ); ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = GLU ? moe_act(acc[rt][nt][r], acc[rt][(nt + 2) & 3][r], act, limit, up_shift) : lev_activate(acc[rt][nt][r], act);
-      moe_store4<TO>(out + (size_t)(first + row) * o_stride + o, v, F - o, vec);
-    }
+      for (int r4 = 0; r4 < 4; ++r4) {
+        const int o = o0 + wn * (GLU ? WN / 2 : WN) + 32 * j + 8 * r4 + 4 * (lane >> 5);
+        if (o >= F) continue;
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = GLU ? moe_act(acc[i][j][4 * r4 + r], acc[i][(j + TJ / 2) % TJ][4 * r4 + r], act, p.limit, p.up_shift) : lev_activate(acc[i][j][4 * r4 + r], act);
+        moe_store4<TO>(static_cast<TO*>(p.out) + (size_t)(first + row) * p.o_stride + o, v, F - o, p.vec);
+      }
   }
+}
+
+template <typename TO, bool GLU>
+__global__ void __launch_bounds__(256, 2)
+moe_linear_big_kernel(const MoeLinearArgs p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char moe_smem[];
+  const int n_tiles = p.meta[0], per = (n_tiles + 7) / 8;
+  if (per == 0) return;
+  const int lo = (blockIdx.x & 7) * per, n = min(per, n_tiles - lo), slot = blockIdx.x >> 3;
+  if (slot >= n * p.n_cols) return;  // the whole workgroup (n may be below 1)
+  int tile = lo + slot % n, ycol = slot / n;
+  if (n <= 64) {  // the chiplet's larger tiles first, in all columns: what runs last is short
+    const int lane = threadIdx.x & 63;
+    const bool large = lane < n && p.tiles[3 * (lo + lane) + 2] > MOE_BIG / 2;
+    const unsigned long long all = __ballot(lane < n), larger = __ballot(large);
+    const int n_larger = __popcll(larger);
+    const bool mine = slot < n_larger * p.n_cols;
+    const unsigned long long of = mine ? larger : all & ~larger;
+    const int at = mine ? slot : slot - n_larger * p.n_cols, kind = __popcll(of);
+    ycol = at / kind;
+    tile = lo + __ffsll(__ballot((of >> lane & 1) && __popcll(of & ((1ull << lane) - 1)) == at % kind)) - 1;
+  }
+  const int e = p.tiles[3 * tile], first = p.tiles[3 * tile + 1], rows = p.tiles[3 * tile + 2];
+  if (rows <= MOE_BIG / 2) moe_big_tile<TO, GLU, MOE_BN, MOE_BIG / 2>(p, moe_smem, e, first, rows, ycol);
+  else moe_big_tile<TO, GLU, MOE_BN, MOE_BIG>(p, moe_smem, e, first, rows, ycol);
 }
 
 // a [rows][K]; w [E][N][K] with N = F outputs, or with glu N = 2F: gate rows then up rows; out [P][F]
@@ -583,16 +652,16 @@ extern "C" int lev_moe_linear(const void* a, long a_stride, const void* w, void*
       return lev_check_launch("moe_linear (matrix cores, K split)");
     }
     if (tile_rows == MOE_BIG) {
-      const int bn = glu ? MOE_BIG / 2 : MOE_BIG, n_cols = (F + bn - 1) / bn;
+      const int bn = glu ? MOE_BN / 2 : MOE_BN, n_cols = (F + bn - 1) / bn;
       const long blocks = (long)((max_tiles + 7) / 8) * 8 * n_cols;
       LEV_REQUIRE(blocks <= 0x7fffffffL, "experts: too many tiles (%ld)", blocks);
       const int vec = o_stride % 4 == 0 && ((uintptr_t)out & (out_dtype == LEV_F32 ? 15 : 7)) == 0;
 #define MOE_BIG_CASE(TO, G)                                                                                                                       \
   do {                                                                                                                                            \
-    hipError_t e = hipFuncSetAttribute((const void*)moe_linear_big_kernel<TO, G>, hipFuncAttributeMaxDynamicSharedMemorySize, MOE_BIG_LDS);        \
-    LEV_REQUIRE(e == hipSuccess, "experts: %d bytes of LDS a workgroup: %s", MOE_BIG_LDS, hipGetErrorString(e));                                   \
-    moe_linear_big_kernel<TO, G><<<(unsigned)blocks, 256, MOE_BIG_LDS, stream>>>((const bf16_t*)a, a_stride, (const bf16_t*)w, (TO*)out, o_stride, tiles, \
-                                                                                meta, sorted, top, gather, K, N, F, act, limit, up_shift, n_cols, vec); \
+    hipError_t e = hipFuncSetAttribute((const void*)moe_linear_big_kernel<TO, G>, hipFuncAttributeMaxDynamicSharedMemorySize, MOE_BIG_LDS(MOE_BN)); \
+    LEV_REQUIRE(e == hipSuccess, "experts: %d bytes of LDS a workgroup: %s", MOE_BIG_LDS(MOE_BN), hipGetErrorString(e));                           \
+    moe_linear_big_kernel<TO, G><<<(unsigned)blocks, 256, MOE_BIG_LDS(MOE_BN), stream>>>(                                                         \
+        MoeLinearArgs{(const bf16_t*)a, a_stride, (const bf16_t*)w, out, o_stride, tiles, meta, sorted, top, gather, K, N, F, act, limit, up_shift, n_cols, vec}); \
   } while (0)
       if (out_dtype == LEV_F32) {
         if (glu) MOE_BIG_CASE(float, true); else MOE_BIG_CASE(float, false);
