@@ -4,14 +4,12 @@
 //   tile kernel   (M > 128): a 256x256, 256x192, 256x128, 128x128 or 128x64 tile per workgroup of 4 waves, 32x32x16 MFMA,
 //                 (K split into ranges, with a second kernel for the sums, where the tiles alone would leave CUs idle)
 //                 operands staged through LDS (two buffers), the next k-tile's global loads in registers meanwhile;
-//   stream kernel (M <= 128; up to 24 rows where an estimate puts it ahead of the skinny kernel: long sums, workgroup counts
-//                 that do not fit the CUs): the weights are the traffic; `a` is shared through LDS by the 4 to 16 waves of a
+//   stream kernel (M <= 128; up to 64 rows where an estimate puts it ahead of the skinny kernel: long sums, many rows): the weights are the traffic; `a` is shared through LDS by the 4 to 16 waves of a
 //                 workgroup, the weights go straight into MFMA operand registers, K is split over workgroups
 //                 and a second kernel adds the partial sums in a fixed order;
-//   skinny kernel (M <= 24, and up to 64 rows of narrow layers, see use_skinny): a workgroup owns 16 output columns;
-//                 its waves split K, load their part of w
-//                 straight into MFMA operand registers (16x16x32), and their partial sums are added
-//                 through LDS in a fixed order.
+//   skinny kernel (M <= 64, see use_skinny): a workgroup owns 8 to 64 output columns; its waves split K, bring whole lines of w
+//                 and a through an LDS area of their own into MFMA operand registers (16x16x32), and their partial sums are
+//                 added through LDS in a fixed order.
 // No atomics anywhere: results are deterministic. K and lda must be multiples of 8 (16-byte operand loads);
 // any M and N.
 #include "common.h"
@@ -332,75 +330,68 @@ static int launch_tile(const bf16_t* a, long lda, const bf16_t* w, const float* 
 }
 
 // ------------------------------------------------------------------------------------------------
-// Skinny kernel (M <= SKINNY_MAX_M: MT = 1, 2 or 4 tiles of 16 rows). A workgroup owns NT = 1 to 3 units of 16 output columns; its WAVES
-// waves split K. A wave takes pairs of adjacent 32-wide k-steps (64 k = 128 bytes of a row), U pairs in flight:
-//   weights: lane (row l%16, k-group l/16) loads 16 bytes straight into the MFMA operand, two loads per pair;
-//   `a`:     read as WHOLE 128-byte lines - lane (row l/8, 16-byte chunk l%8), one instruction for rows 0..7 and one
-//            for rows 8..15 of a pair - and turned into the operand layout (row l%16, k-group l/16) through a
-//            small LDS area of the wave's own. Reading `a` in operand layout (64 bytes of each of 16 rows per
-//            instruction) costs as much time in the memory pipeline as the weights themselves: every workgroup
-//            reads all of `a`, and half lines are fetched at half the rate.
-// The partial sums of the waves are added through LDS in wave order. ROT: every workgroup starts at another
+// Skinny kernel (M <= SKINNY_MAX_M: MT = 1 .. 4 tiles of 16 rows). A workgroup owns NT units of 16 output columns (or, HALF, one of 8); its
+// WAVES waves split K. A wave takes pairs of adjacent 32-wide k-steps (64 k = 128 bytes of a row), U pairs in flight. Weights and `a`
+// alike are read as WHOLE 128-byte lines - lane (row l/8, 16-byte chunk l%8), one instruction for 8 rows - and turned into the operand
+// layout (row l%16, k-group l/16) through a small LDS area of the wave's own. The vector cache looks lines up by neighbouring
+// lanes: read in operand layout (16 rows, 64 bytes of each) an instruction costs one look-up for every lane, 16 bytes a cycle and CU, and
+// weights and `a` together were bound by that and not by memory (of data in L2, 9.6 TB/s against 33 TB/s in whole lines).
+// The loads stand under no condition, from clamped addresses (a condition is a branch, and at its join everything in flight is waited
+// for); what lies beyond K is masked on its way into LDS, rows beyond M and columns beyond N are read again and never stored.
+// Measured in graphs over distinct weights, before (weights straight into the operand, conditional loads) and now, microseconds: 4800 x
+// 1600 at 6 / 24 rows 8.0 / 12.5 -> 6.4 / 8.9; 6400 x 1600 8.3 / 12.9 -> 7.0 / 9.2; 4608 x 2048 9.1 / 14.2 -> 6.8 / 9.0; 768 x 768 3.8 / 4.8 -> 3.5 /
+// 4.0; 4096 x 4096 8.6 / 12.5 -> 8.4 / 10.2; 16384 x 4096 25.0 -> 24.2 at 6 rows (memory: 5.5 TB/s); the same bits.
+// The partial sums of the waves are added through LDS in wave order. Every workgroup starts at another
 // place of the k range, so that they do not all read the same part of `a` and the same residue of the weight
 // rows at the same time; the order of the sum depends on the column tile only, never on M or the batch.
 #define SKINNY_SLOTS 72  // 16-byte slots of one staged instruction: 8 rows x (8 chunks + 1 of padding)
 #define SKINNY_MAX_M 64  // with four row tiles; which of these row counts it takes: use_skinny()
 
-template <typename TO, int WAVES, int U, int ROT, int MT, int NT>
+template <typename TO, int WAVES, int U, int MT, int NT, bool HALF>
 __global__ void __launch_bounds__(WAVES * 64)
 gemm_skinny_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restrict__ w, const float* __restrict__ bias,
                    const float* residual, long ldr, TO* out, long ldo, int M, int N, int K, int act) {
-  static_assert(NT >= 1 && NT <= WAVES, "wave j finishes column unit j");
-  constexpr int AI = 2 * MT;  // `a` instructions per pair of k-steps: 8 rows each
-  // With more than two row tiles the staging area holds one tile at a time (the LDS executes a wave's instructions in
-  // order, so the next tile's writes cannot overtake this one's reads): 16 waves x 8 instructions would not fit the LDS.
-  constexpr bool ONE_TILE = MT > 2;
-  constexpr int SI = ONE_TILE ? 2 : AI;
+  static_assert(NT * MT <= WAVES * 4 && (!HALF || NT == 1), "a wave finishes a few tiles; half a unit stands alone");
+  constexpr int AI = 2 * MT, WI = HALF ? 1 : 2;  // instructions per pair of k-steps and unit: 8 rows each
+  constexpr int COLS = HALF ? 8 : 16;
   __shared__ f32x4 red[WAVES][NT][MT][64];
-  __shared__ u32x4 stage[WAVES][SI][SKINNY_SLOTS];
+  __shared__ u32x4 stage[WAVES][2][SKINNY_SLOTS];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
-  const int n0 = blockIdx.x * 16 * NT;
+  const int n0 = blockIdx.x * COLS * NT;
   const int fr = lane & 15, kg = lane >> 4;
-  bool n_ok[NT];
-  const bf16_t* wrow[NT];
+  const int lr = lane >> 3, lc = lane & 7;  // loads: row (0..7, instruction i adds 8 i) and chunk of the line
+  const bf16_t* wrow[NT][WI];
 #pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    n_ok[j] = n0 + 16 * j + fr < N;
-    wrow[j] = w + (size_t)(n_ok[j] ? n0 + 16 * j + fr : 0) * K + kg * 8;
-  }
-  const int ar = lane >> 3, ac = lane & 7;  // `a` loads: row (0..7, instruction i adds 8 i) and chunk of the line
-  bool a_ok[AI];
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int i = 0; i < WI; ++i) wrow[j][i] = w + (size_t)min(n0 + 16 * j + 8 * i + lr, N - 1) * K;
   const bf16_t* arow[AI];
 #pragma unroll
-  for (int i = 0; i < AI; ++i) {
-    a_ok[i] = ar + 8 * i < M;
-    arow[i] = a + (size_t)(a_ok[i] ? ar + 8 * i : 0) * lda + ac * 8;
-  }
+  for (int i = 0; i < AI; ++i) arow[i] = a + (size_t)min(8 * i + lr, M - 1) * lda;
   u32x4* my_stage = &stage[wave][0][0];
-  const int st_slot = ar * 9 + ac;                       // where this lane's chunk is staged
+  const int st_slot = lr * 9 + lc;                                   // where this lane's chunk is staged
   const int ld_slot = (fr >> 3) * SKINNY_SLOTS + (fr & 7) * 9 + kg;  // operand (row fr, k-group kg) of the pair's first step
 
   // The lanes that will finish the sum fetch their bias and residual values now, so that the end of the kernel
   // (which no other workgroup's streaming overlaps: all of them finish together) has no dependent loads left.
-  // Unconditional loads from addresses that are always valid (clamped; `w` stands in for a missing operand):
-  // a load under a condition would make the compiler wait for it at the join, ahead of the whole k loop.
-  float pre_bias[NT];
-  f32x4 pre_res[NT][MT];
+  // `w` stands in for a missing operand.
+  constexpr int TURNS = (NT * MT + WAVES - 1) / WAVES;  // wave v finishes the tiles v, v + WAVES, ..
+  float pre_bias[TURNS];
+  f32x4 pre_res[TURNS];
 #pragma unroll
-  for (int j = 0; j < NT; ++j) {
+  for (int q = 0; q < TURNS; ++q) {
+    const int tile = min(wave + q * WAVES, NT * MT - 1), j = tile % NT, t = tile / NT;
     const int nn = min(n0 + 16 * j + fr, N - 1);
     const float* bp = bias ? bias + nn : reinterpret_cast<const float*>(w);
-    pre_bias[j] = *bp;
-    if (!bias) pre_bias[j] = 0.f;
+    pre_bias[q] = *bp;
+    if (!bias) pre_bias[q] = 0.f;
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = min(t * 16 + kg * 4 + r, M - 1);
-        const float* rp = residual ? residual + (size_t)m * ldr + nn : reinterpret_cast<const float*>(w);
-        pre_res[j][t][r] = *rp;
-      }
+    for (int r = 0; r < 4; ++r) {
+      const int m = min(t * 16 + kg * 4 + r, M - 1);
+      const float* rp = residual ? residual + (size_t)m * ldr + nn : reinterpret_cast<const float*>(w);
+      pre_res[q][r] = *rp;
+    }
   }
 
   f32x4 acc[NT][MT];
@@ -409,47 +400,47 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restr
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[j][t] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int npairs = (K + 63) / 64;
-  const int rot = ROT ? (int)((blockIdx.x * 2654435761u) % (unsigned)npairs) : 0;
+  const int rot = (int)((blockIdx.x * 2654435761u) % (unsigned)npairs);
   for (int p0 = wave; p0 < npairs; p0 += WAVES * U) {
-    u32x4 wv[U][NT][2], av[U][AI];
+    u32x4 wv[U][NT][WI], av[U][AI];
+    uint32_t keep[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       int pr = p0 + u * WAVES;
       const bool p_ok = pr < npairs;
-      if (ROT) {
-        pr += rot;
-        pr = pr >= npairs ? pr - npairs : pr;
-      }
-      const int k = pr * 64;
+      pr = min(pr, npairs - 1) + rot;
+      pr = pr >= npairs ? pr - npairs : pr;
+      const int k = pr * 64 + lc * 8, kc = min(k, K - 8);
+      keep[u] = p_ok && k < K ? 0xffffffffu : 0u;
 #pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        const bool w_ok = p_ok && n_ok[j];
-        wv[u][j][0] = (w_ok && k + kg * 8 < K) ? load16(wrow[j] + k) : u32x4{0, 0, 0, 0};
-        wv[u][j][1] = (w_ok && k + 32 + kg * 8 < K) ? load16(wrow[j] + k + 32) : u32x4{0, 0, 0, 0};
-      }
-      const bool c_ok = p_ok && k + ac * 8 < K;
+      for (int j = 0; j < NT; ++j)
 #pragma unroll
-      for (int i = 0; i < AI; ++i) av[u][i] = (c_ok && a_ok[i]) ? load16(arow[i] + k) : u32x4{0, 0, 0, 0};
+        for (int i = 0; i < WI; ++i) wv[u][j][i] = load16(wrow[j][i] + kc);
+#pragma unroll
+      for (int i = 0; i < AI; ++i) av[u][i] = load16(arow[i] + kc);
     }
+    __builtin_amdgcn_sched_barrier(0);  // all of them are on their way before the first is waited for
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      // LDS executes a wave's instructions in order: the area is reused pair after pair without a barrier
-      if (!ONE_TILE) {
+      // LDS executes a wave's instructions in order: the area is used again and again without a barrier
+      const u32x4 mk = u32x4{keep[u], keep[u], keep[u], keep[u]};
+      u32x4 wf[NT][2];
 #pragma unroll
-        for (int i = 0; i < AI; ++i) my_stage[i * SKINNY_SLOTS + st_slot] = av[u][i];
+      for (int j = 0; j < NT; ++j) {
+#pragma unroll
+        for (int i = 0; i < WI; ++i) my_stage[i * SKINNY_SLOTS + st_slot] = wv[u][j][i] & mk;
+        const int at = HALF ? (fr & 7) * 9 + kg : ld_slot;  // half a unit: columns 8 .. 15 repeat 0 .. 7
+        wf[j][0] = my_stage[at], wf[j][1] = my_stage[at + 4];
       }
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
-        if (ONE_TILE) {
-          my_stage[st_slot] = av[u][2 * t];
-          my_stage[SKINNY_SLOTS + st_slot] = av[u][2 * t + 1];
-        }
-        const int base = ONE_TILE ? 0 : 2 * t * SKINNY_SLOTS;
-        const u32x4 a_lo = my_stage[base + ld_slot], a_hi = my_stage[base + ld_slot + 4];
+        my_stage[st_slot] = av[u][2 * t] & mk;
+        my_stage[SKINNY_SLOTS + st_slot] = av[u][2 * t + 1] & mk;
+        const u32x4 a_lo = my_stage[ld_slot], a_hi = my_stage[ld_slot + 4];
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-          acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a_lo), as_bf16x8(wv[u][j][0]), acc[j][t], 0, 0, 0);
-          acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a_hi), as_bf16x8(wv[u][j][1]), acc[j][t], 0, 0, 0);
+          acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a_lo), as_bf16x8(wf[j][0]), acc[j][t], 0, 0, 0);
+          acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a_hi), as_bf16x8(wf[j][1]), acc[j][t], 0, 0, 0);
         }
       }
     }
@@ -460,87 +451,96 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restr
     for (int t = 0; t < MT; ++t) red[wave][j][t][lane] = acc[j][t];
   __syncthreads();
   // 16x16 accumulator: register r of lane l is row 4*(l/16) + r, column l%16. Partial sums are added in wave order.
-  if (wave < NT) {  // wave j finishes column unit j
-    const int j = wave;
+#pragma unroll
+  for (int q = 0; q < TURNS; ++q) {
+    const int tile = wave + q * WAVES, j = tile % NT, t = tile / NT;
+    if (tile >= NT * MT) break;
     const int nn = n0 + 16 * j + fr;
+    f32x4 s = red[0][j][t][lane];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      f32x4 s = red[0][j][t][lane];
+    for (int v = 1; v < WAVES; ++v) {
+      const f32x4 o = red[v][j][t][lane];
+      s[0] += o[0]; s[1] += o[1]; s[2] += o[2]; s[3] += o[3];
+    }
+    if (nn < N && fr < COLS) {
 #pragma unroll
-      for (int v = 1; v < WAVES; ++v) {
-        const f32x4 o = red[v][j][t][lane];
-        s[0] += o[0]; s[1] += o[1]; s[2] += o[2]; s[3] += o[3];
-      }
-      if (nn < N) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int m = t * 16 + kg * 4 + r;
-          if (m >= M) continue;
-          float pb = pre_bias[0], pr = pre_res[0][t][r];
-#pragma unroll
-          for (int j2 = 1; j2 < NT; ++j2)
-            if (j == j2) {
-              pb = pre_bias[j2];
-              pr = pre_res[j2][t][r];
-            }
-          float v = lev_activate(s[r] + pb, act);
-          if (residual) v += pr;
-          out[(size_t)m * ldo + nn] = from_float<TO>(v);
-        }
+      for (int r = 0; r < 4; ++r) {
+        const int m = t * 16 + kg * 4 + r;
+        if (m >= M) continue;
+        float v = lev_activate(s[r] + pre_bias[q], act);
+        if (residual) v += pre_res[q][r];
+        out[(size_t)m * ldo + nn] = from_float<TO>(v);
       }
     }
   }
 }
 
-// Choices measured on MI355X at K = 4096 .. 16384 and M = 1 .. 16 (graph replays over distinct weights): with many
-// column tiles 4 waves with 4 or 2 pairs in flight; with fewer than 512 the chip is only filled by 16 waves per
-// workgroup. The rotated start never costs and takes a third off the time where rows are long (K = 16384).
-// Two column units per workgroup (32 columns: every `a` fragment feeds two weight fragments, half the activation
-// traffic) pay where the halved number of workgroups still fills the chip evenly or the rows are many: 16384
-// columns x 4096 at 8 rows 28.1 -> 26.2 us, at 16 rows 33.4 -> 27.8 us; 24576 x 6144 at 16 rows 76 -> 64 us; at one
-// row and with workgroup counts that are no multiple of the CUs (18432 or 50257 columns) they lose up to 15 %.
-// Three units and 16 waves for 12288 columns x 4096: 25.1 -> 21.8 us at 16 rows, the same at 8 rows, 10 % slower at one.
+// Choices measured on MI355X (graphs over distinct weights, 1 to 64 rows, weights of 768 x 768 to 6144 x 24576). What decides is how many
+// columns the busiest CU streams, and that every `a` fragment feeds several of weights where the rows are many:
+//   up to 2,048 columns (256 workgroups of 8 columns): half units up to 32 rows: 1600 x 6400 at 6 rows 9.3 -> 7.7 us, at 24 rows 13.3 -> 11.6,
+//     2048 x 8192 11.0 -> 9.1; 16 waves with two pairs each for long rows and up to 8 rows of `a` (8.9 -> 7.7, 10.7 -> 9.1), else 8 waves;
+//   else as many units a workgroup as make one round of the CUs: two up to 512 units (4800 x 1600 at 6 rows 7.5 -> 6.4, 4608 x 2048 7.8 -> 6.8, 6144 x
+//     6144 18.0 -> 15.7), three up to 768 (12288 x 4096 at 24 rows 24.3 -> 21.2, 10752 x 2048 13.7 -> 10.6), four with 4 waves up to 1,024 (16384 x
+//     4096 at 24 rows 31.0 -> 26.4, at 48 rows 40.7 -> 28.4); above that three up to 32 rows (18432 x 6144 at 24 rows 55.8 -> 49.5), else four
+//     (32000 x 2048 at 48 rows 28.3 against 35.1 for the stream kernel, 50257 x 4096 89.5 against 105 with three);
+//   but up to 16 rows above 720 units one unit and 4 waves with four pairs in flight: 12288 x 4096 at 6 rows 20.7 -> 18.9, 16384 x 4096 29 -> 24.3.
 struct SkinnyShape {
   int waves, in_flight, row_tiles, units;  // the kernel's WAVES, U, MT, NT
+  bool half;
+  int cols() const { return half ? 8 : 16 * units; }
 };
-static SkinnyShape skinny_shape(int M, int N) {
+static SkinnyShape skinny_shape(int M, int N, int K) {
   const int tiles = (N + 15) / 16;
   if (M <= 16) {
-    const bool two_units = tiles >= 1024 && (M >= 12 || (tiles / 2) % 256 == 0);
-    if (two_units) return {4, 2, 1, 2};
-    if (M >= 12 && tiles >= 720 && tiles < 1024) return {16, 1, 1, 3};  // about 256 workgroups of 48 columns
-    if (tiles >= 1024) return {4, 4, 1, 1};
-    if (tiles >= 512) return {4, 2, 1, 1};
-    return {16, 1, 1, 1};
+    if (N <= 2048) return K > 4096 && M <= 8 ? SkinnyShape{16, 2, 1, 1, true} : SkinnyShape{8, 2, 1, 1, true};
+    if (tiles <= 256) return {8, 2, 1, 1, false};
+    if (tiles <= 512) return K < 1792 ? SkinnyShape{16, 1, 1, 2, false} : SkinnyShape{8, 2, 1, 2, false};
+    return tiles <= 720 ? SkinnyShape{16, 1, 1, 3, false} : SkinnyShape{4, 4, 1, 1, false};
   }
-  // 17 .. 32 rows: two row tiles share every weight load; up to SKINNY_MAX_M: four
-  if (M <= 32) return tiles >= 512 ? SkinnyShape{4, 2, 2, 1} : SkinnyShape{16, 1, 2, 1};
-  return tiles >= 512 ? SkinnyShape{4, 2, 4, 1} : SkinnyShape{16, 1, 4, 1};
+  if (M <= 32) {
+    if (N <= 2048) return {8, 2, 2, 1, true};
+    if (tiles <= 256) return {8, 2, 2, 1, false};
+    if (tiles <= 512) return {8, 2, 2, 2, false};
+    return tiles > 768 && tiles <= 1024 ? SkinnyShape{4, 1, 2, 4, false} : SkinnyShape{8, 1, 2, 3, false};
+  }
+  const int mt = M <= 48 ? 3 : 4;
+  if (tiles <= 768) return {8, 1, mt, tiles <= 256 ? 1 : tiles <= 512 ? 2 : 3, false};
+  return {4, 1, mt, 4, false};
 }
 
 template <typename TO>
 static void launch_skinny(const bf16_t* a, long lda, const bf16_t* w, const float* bias, const float* residual, long ldr,
                           TO* out, long ldo, int M, int N, int K, int act, hipStream_t stream) {
-  const int tiles = (N + 15) / 16;
-  const SkinnyShape sh = skinny_shape(M, N);
-#define LEV_SKINNY(W_, U_, MT_, NT_)                                                                                          \
-  if (sh.waves == W_ && sh.in_flight == U_ && sh.row_tiles == MT_ && sh.units == NT_)                                          \
-    gemm_skinny_kernel<TO, W_, U_, 1, MT_, NT_><<<(tiles + NT_ - 1) / NT_, W_ * 64, 0, stream>>>(a, lda, w, bias, residual, ldr, out, \
-                                                                                                 ldo, M, N, K, act)
-  LEV_SKINNY(4, 2, 1, 2);
-  LEV_SKINNY(16, 1, 1, 3);
-  LEV_SKINNY(4, 4, 1, 1);
-  LEV_SKINNY(4, 2, 1, 1);
-  LEV_SKINNY(16, 1, 1, 1);
-  LEV_SKINNY(4, 2, 2, 1);
-  LEV_SKINNY(16, 1, 2, 1);
-  LEV_SKINNY(4, 2, 4, 1);
-  LEV_SKINNY(16, 1, 4, 1);
+  const SkinnyShape sh = skinny_shape(M, N, K);
+  const int cols = sh.cols();
+#define LEV_SKINNY(W_, U_, MT_, NT_, H_)                                                                                          \
+  if (sh.waves == W_ && sh.in_flight == U_ && sh.row_tiles == MT_ && sh.units == NT_ && sh.half == H_)                             \
+    gemm_skinny_kernel<TO, W_, U_, MT_, NT_, H_><<<(N + cols - 1) / cols, W_ * 64, 0, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act)
+  LEV_SKINNY(16, 2, 1, 1, true);
+  LEV_SKINNY(8, 2, 1, 1, true);
+  LEV_SKINNY(8, 2, 1, 1, false);
+  LEV_SKINNY(16, 1, 1, 2, false);
+  LEV_SKINNY(8, 2, 1, 2, false);
+  LEV_SKINNY(16, 1, 1, 3, false);
+  LEV_SKINNY(4, 4, 1, 1, false);
+  LEV_SKINNY(8, 2, 2, 1, true);
+  LEV_SKINNY(8, 2, 2, 1, false);
+  LEV_SKINNY(8, 2, 2, 2, false);
+  LEV_SKINNY(8, 1, 2, 3, false);
+  LEV_SKINNY(4, 1, 2, 4, false);
+  LEV_SKINNY(8, 1, 3, 1, false);
+  LEV_SKINNY(8, 1, 4, 1, false);
+  LEV_SKINNY(8, 1, 3, 2, false);
+  LEV_SKINNY(8, 1, 4, 2, false);
+  LEV_SKINNY(8, 1, 3, 3, false);
+  LEV_SKINNY(8, 1, 4, 3, false);
+  LEV_SKINNY(4, 1, 3, 4, false);
+  LEV_SKINNY(4, 1, 4, 4, false);
 #undef LEV_SKINNY
 }
 
 // ------------------------------------------------------------------------------------------------
-// Stream kernel, for 24 < M <= 128: the weights are still the traffic that matters, but fetching the `a`
+// Stream kernel, for M <= 128 where the skinny kernel is not ahead: the weights are still the traffic that matters, but fetching the `a`
 // fragments from L2 once per wave (as the skinny kernel does) would cost more than the weights. Here a
 // workgroup of NW waves (4, 8, 12 or 16) owns NW x 16 output columns and all M rows; `a` goes through LDS in chunks
 // of 64 k and is shared by the waves, each wave loads its own 16 weight rows straight into MFMA operand
@@ -828,28 +828,21 @@ static TilePlan plan_tiles(int M, int N, int K) {
   return best;
 }
 
-// Which kernel takes M <= SKINNY_MAX_M rows. The skinny kernel's time grows with the rows, because every workgroup reads all
-// of `a` (out of L2, at about 20 TB/s for all CUs together), and with workgroup counts that are no multiple of the CUs; the
-// stream kernel's hardly does, but it pays for its K ranges. An estimate of the skinny kernel in the manner of
-// plan_stream's, and a factor between the two fitted to measurements at three model sizes (microseconds, skinny / stream):
-//   4096-wide layer:  8 rows 19.5 / 24.1, 8.6 / 14.7, 24.9 / 31.6, 23.9 / 32.9 (qkv, proj, fc, second MLP matrix);
-//                     24 rows 27.8 / 25.2, 12.6 / 15.9, 35.8 / 33.2, 35.3 / 33.6
-//   6144-wide layer:  8 rows 48.3 / 53.7, 20.6 / 21.4, 55.2 / 59.2, 67.0 / 60.3; 16 rows 55.3 / 54.5, 25.0 / 22.0, 60.3 / 60.3,
-//                     86.1 / 60.6 (384 workgroups of the skinny kernel: one and a half rounds); 24 rows 66 / 55, 32 / 23, 80 / 62, 104 / 62
-//   1600-wide layer:  8 rows 7.0 / 8.1, 4.7 / 7.1, 8.3 / 9.5, 10.8 / 10.8; 16 rows 7.3 / 8.2, 4.8 / 7.2, 9.0 / 10.0, 13.6 / 11.0
-//   heads (50257 columns) of 4096 / 6144 / 1600 / 768: 8 rows 81 / 87, 125 / 152, 34.6 / 34.3, 17.0 / 20.6; 24 rows 108 / 91, 169 / 156,
-//                     46.5 / 35.9, 24.3 / 22.2
-// Over the 112 cases measured (1 to 24 rows) the choice made here is on average 1 % behind the better kernel; the rule before
-// it (rows alone, with one exception for large weights) 4 %, and up to 70 % on the long sums of the 6144-wide layer.
+// Which kernel takes M <= SKINNY_MAX_M rows. An estimate of the skinny kernel in microseconds, from the measurements above: a launch and
+// its ramp, and the longest of the weights' read from memory, the share of it that falls to the busiest CU, and what that CU pulls
+// through its caches (its columns and all of `a`, for each of its workgroups). The stream kernel's time hardly grows with the
+// rows, but it pays for its K ranges: plan_stream's cost is about 0.8 of what it takes with the kernel that adds them (which the next norm may do in passing: 1.2). Measured,
+// skinny / stream: 1600 x 6400 at 16 / 24 / 32 / 64 rows 9.5 / 11.4, 11.6 / 11.7, 12.6 / 11.9, 20.0 / 13.8; 4096 x 16384 at 24 / 48 rows 28.1 / 33.4,
+// 39.1 / 35.1; 6144 x 24576 at 24 rows 67.7 / 61.0; 16384 x 4096 at 64 rows 32.2 / 37.1; 6144 x 6144 at 6 rows 15.7 / 21.1.
 static double skinny_estimate(int M, int N, int K) {
-  const SkinnyShape sh = skinny_shape(M, N);
-  const long wgs = ((N + 15) / 16 + sh.units - 1) / sh.units;
-  const long r = (wgs + 255) / 256;  // workgroups of the slowest CU
-  const double w_bytes = (double)N * K * 2.0, a_bytes = (double)wgs * M * K * 2.0;
-  const double t = w_bytes / 7.5e6 + a_bytes / 20e6;
-  double cost = 3.0 + t * (wgs >= 256 ? (double)r * 256.0 / wgs : 256.0 / wgs);
-  if (sh.row_tiles == 2) cost *= 1.2;
-  return cost;
+  const SkinnyShape sh = skinny_shape(M, N, K);
+  const long wgs = (N + sh.cols() - 1) / sh.cols(), r = (wgs + 255) / 256;  // r: workgroups of the busiest CU
+  const double memory = 2.0 * N * K / 5.5e6, own = r * (double)sh.cols() * K * 2.0 / 31e3;
+  const double rate = (long)N * K <= (1L << 23) ? 75e3 : sh.waves == 4 ? 37e3 : sh.units > 1 ? 45e3 : 50e3;  // small weights stay in the caches' reach
+  const double caches = r * (double)(sh.cols() + M) * K * 2.0 / rate;
+  double cost = memory > own ? memory : own;
+  if (caches > cost) cost = caches;
+  return 3.2 + cost + (sh.row_tiles > 1 && r > 4 ? 0.8 * (r - 1) : 0.0);
 }
 // 0: the estimate decides; 1 / 2: the skinny / the stream kernel wherever it takes the row count. For measurements of the
 // choice itself (a test times both candidates at widths the estimates were not fitted to); not used by the engine.
@@ -862,16 +855,7 @@ extern "C" int lev_linear_mfma_force(int kind) {
 static bool use_skinny(int M, int N, int K) {
   if (M > SKINNY_MAX_M) return false;
   if (g_force_kernel) return g_force_kernel == 1;
-  if (M > 24) {
-    // 25 to 64 rows (two or four row tiles), microseconds skinny / stream, second kernel included, at 32 and 64 rows: where
-    // the skinny kernel's workgroups of 16 waves make one round of the CUs and the sum is no longer than the output is wide
-    // it stays ahead (2304 x 768: 5.2 / 7.6, 7.6 / 9.4; 4096 x 1024: 6.1 / 8.6, 8.9 / 10.4; 1600 x 1600: 6.5 / 8.4, 9.5 / 10.2;
-    // 4096 x 4096: 13.4 / 15.0 but 18.6 / 16.7), elsewhere not (4800 x 1600, 300 workgroups: 14.1 / 11.1, 20.4 / 13.4;
-    // 1024 x 4096: 11.4 / 9.3, 16.2 / 11.0; 12288 x 4096: 32.1 / 26.4, 42.4 / 28.7).
-    const int tiles = (N + 15) / 16;
-    return tiles <= 256 && K <= N && (M <= 32 || (long)N * K <= (1L << 23));
-  }
-  return skinny_estimate(M, N, K) <= 1.3 * plan_stream(M, N, K).cost;
+  return skinny_estimate(M, N, K) <= 1.2 * plan_stream(M, N, K).cost;
 }
 
 // Into how many ranges the sum over K is split (1: the kernel finishes its outputs itself).

@@ -431,7 +431,7 @@ class HipKernels:
         return None
 
     LIBRARY_ACTIVATIONS = (ACTIVATIONS["none"], ACTIVATIONS["gelu_new"], ACTIVATIONS["relu"])
-    LIBRARY_MIN_ROWS = 25  # up to 24 rows the skinny kernel streams the weights at the rate a plain read reaches
+    LIBRARY_MIN_ROWS = 25  # up to 24 rows the skinny kernel is ahead everywhere, or behind by less than the library's first use costs
 
     @classmethod
     def use_library(cls, M: int, N: int, K: int, act: int) -> bool:
@@ -439,13 +439,16 @@ class HipKernels:
         ahead on MI355X (widths of GPT-2 7B and XL, with epilogues). From 256 rows: all but long sums into narrow outputs
         (K >= 4 N) below 1,024 rows and, below 320 rows, weights of a few MB unless the output is wide (a 1600-wide layer at 264
         rows, ours / library with its kernel timed: qkv 18.3 / 16.7, fc 24.8 / 18.8, proj 11.9 / 14.2, second MLP matrix 22.7 / 20.4 but
-        20.1 / 23.5 at 256 and 22.9 / 23.5 at 288). From 25 to 255 rows: wide outputs of large
-        weights (N >= 2 K, 32 MB and more: 7B qkv and fc at 64 rows 28.1 / 25.3 and 37.1 / 33.5 us, ours with the kernel that
-        adds its K ranges; at 160 rows 49.7 / 37.2 and 55.7 / 41.6); ours keep N = K (17.4 / 16.3 at 64 rows, 22.1 / 24.6 at
-        128) and K = 4 N (36.8 / 41.2, 43.5 / 81.1), and below 96 rows the largest weights (more than 256 MB: the fc of a
-        6144-wide layer 64.4 / 72.4 at 32 rows, 70.1 / 75.4 at 64, 85.0 / 84.4 at 128; its qkv, 216 MB, 58.9 / 57.6 and 62.3 / 59.7)."""
+        20.1 / 23.5 at 256 and 22.9 / 23.5 at 288). Up to 64 rows: the heads of narrow models (more than 16,384 outputs of sums below 2,048:
+        50257 x 1600 at 32 rows 35.5 / 31.8 us, 50257 x 768 22.9 / 19.0; but 32000 x 2048 28.3 / 33.0) and above 32 rows weights of 67 M to
+        134 M numbers (18432 x 6144 at 48 / 64 rows 57.3 / 54.0, 64.0 / 55.2); everything else is ours (12288 x 4096 at 32 / 64 rows 21.2 / 22.7
+        and 25.7 / 24.8, 16384 x 4096 26.3 / 33.5 and 31.6 / 33.0, 10752 x 2048 10.8 / 14.6 and 14.4 / 15.8). From 65 to 255 rows: wide outputs of large
+        weights (N >= 2 K, 32 MB and more: at 160 rows qkv and fc of a 4096-wide layer 49.7 / 37.2 and 55.7 / 41.6); ours keep N = K (22.1 /
+        24.6 at 128) and K = 4 N (43.5 / 81.1), and below 96 rows the largest weights (more than 256 MB)."""
         if act not in cls.LIBRARY_ACTIVATIONS or M < cls.LIBRARY_MIN_ROWS:
             return False
+        if M <= 64:
+            return (N > 16384 and K < 2048) or (M > 32 and N >= 2 * K and (1 << 26) < N * K <= (1 << 27))
         if M < 256:
             if N < 2 * K:
                 return False

@@ -1,0 +1,45 @@
+"""The bfloat16 product of up to 64 rows at the edges of its launch shapes: columns that make half units, one to four units a workgroup and their
+remainders, rows that fill one to four row tiles, inputs with a short last chunk and with fewer pairs than waves."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def K():
+    from levanter_amd.kernels import get_kernels
+
+    return get_kernels()
+
+
+@pytest.mark.parametrize("N", [1, 7, 9, 2047, 2049, 4090, 4100, 8190, 8200, 11530, 12280, 12300, 16390])
+@pytest.mark.parametrize("Ki", [8, 72, 200, 1784, 1800, 4168])
+def test_linear_skinny_against_float64(K, N, Ki, monkeypatch):
+    """bfloat16 operands are exact in float64; a sum of Ki products in 32 bits is off by at most Ki * 2^-24 of the sum of their absolute values."""
+    gemm = K._unit("gemm_mfma")
+    monkeypatch.setattr(K, "gemm_library", False)
+    g = torch.Generator(device=DEV).manual_seed(N * 31 + Ki)
+    w = torch.randn(N, Ki, device=DEV, generator=g).bfloat16()
+    bias = torch.randn(N, device=DEV, generator=g)
+    try:
+        K._check(gemm.lev_linear_mfma_force(1))
+        K._ws_need.clear()  # how much scratch memory a shape needs goes by the kernel that takes it
+        for M in (1, 8, 9, 16, 17, 32, 33, 48, 49, 64):
+            a = torch.randn(M, Ki + 8, device=DEV, generator=g).bfloat16()[:, :Ki]
+            res = torch.randn(M, N, device=DEV, generator=g)
+            want = a.double() @ w.double().T
+            size = a.double().abs() @ w.double().abs().T
+            out = torch.full((M, N + 3), float("nan"), device=DEV)
+            K.linear(a, w, bias, out[:, :N], residual=res)
+            err = (out[:, :N].double() - want - bias.double() - res.double()).abs()
+            assert bool((err <= (Ki + 4) * 2.0 ** -24 * (size + bias.double().abs() + res.double().abs())).all()), M
+            assert bool(torch.isnan(out[:, N:]).all())
+            half = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+            K.linear(a, w, None, half)
+            assert bool(((half.double() - want).abs() <= want.abs() * 2.0 ** -8 + Ki * 2.0 ** -24 * size).all()), M
+    finally:
+        K._check(gemm.lev_linear_mfma_force(0))
+        K._ws_need.clear()
