@@ -301,138 +301,17 @@ __device__ __forceinline__ moe_bf16x8 moe_as_bf16x8(moe_u32x4 v) {
   return c.b;
 }
 
-// bfloat16 on the matrix cores: a wave owns the tile's rows (RT row tiles of 16) and NT tiles of 16 outputs (with glu: of gate
-// and of up); the transposed product out^T = w a^T leaves each lane with four neighbouring outputs of one row. Every weight
-// fragment a wave loads is used for all its row tiles.
-template <typename TO, int NT, bool GLU, int RT>
-__global__ void __launch_bounds__(256)
-moe_linear_mfma_kernel(const bf16_t* __restrict__ a, long a_stride, const bf16_t* __restrict__ w, TO* __restrict__ out, long o_stride,
-                       const int* __restrict__ tiles, const int* __restrict__ meta, const int* __restrict__ sorted, int top, int gather,
-                       int K, int N, int F, int act, float limit, float up_shift) {
-  const int tile = blockIdx.x;
-  if (tile >= meta[0]) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, g = lane >> 4;
-  const int o0 = (blockIdx.y * 4 + wave) * 16 * NT;
-  if (o0 >= F) return;  // the whole wave
-  const int e = tiles[3 * tile], first = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
-  const bf16_t* ar[RT];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const int pos = first + min(16 * rt + col, rows - 1);  // rows beyond the tile: read again, never stored
-    ar[rt] = a + (size_t)(gather ? sorted[pos] / top : pos) * a_stride;
-  }
-  const bf16_t* we = w + (size_t)e * N * K;
-  const bf16_t* wr[NT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) wr[nt] = we + (size_t)min(o0 + 16 * nt + col, F - 1) * K;
-  moe_f32x4 acc[RT][NT], acc_up[RT][NT];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = acc_up[rt][nt] = moe_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int k0 = 0; k0 < K; k0 += 32) {
-    const int kk = k0 + 8 * g, kc = min(kk, K - 8);  // loads stand under no condition; a chunk beyond the row counts as zeros
-    const uint32_t keep = kk < K ? 0xffffffffu : 0u;
-    moe_u32x4 av[RT];
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      const moe_u32x4 x = *reinterpret_cast<const moe_u32x4*>(ar[rt] + kc);
-      av[rt] = moe_u32x4{x[0] & keep, x[1] & keep, x[2] & keep, x[3] & keep};
-    }
-    moe_u32x4 wv[NT], wu[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      wv[nt] = *reinterpret_cast<const moe_u32x4*>(wr[nt] + kc);
-      if (GLU) wu[nt] = *reinterpret_cast<const moe_u32x4*>(wr[nt] + (size_t)F * K + kc);
-    }
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        acc[rt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(moe_as_bf16x8(wv[nt]), moe_as_bf16x8(av[rt]), acc[rt][nt], 0, 0, 0);
-        if (GLU) acc_up[rt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(moe_as_bf16x8(wu[nt]), moe_as_bf16x8(av[rt]), acc_up[rt][nt], 0, 0, 0);
-      }
-  }
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    if (16 * rt + col >= rows) continue;
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int o = o0 + 16 * nt + 4 * g + r;
-        if (o < F)
-          out[(size_t)(first + 16 * rt + col) * o_stride + o] = from_float<TO>(GLU ? moe_act(acc[rt][nt][r], acc_up[rt][nt][r], act, limit, up_shift) : lev_activate(acc[rt][nt][r], act));
-      }
-  }
-}
-
-// Few tiles (a step of single tokens): the products are bound by reading the chosen experts' weights, and a tile's 16 rows give
-// the chip too few waves. A workgroup of MOE_KS waves owns one tile of 16 rows and 16 outputs; its waves split K, every wave has
-// all loads of its share in flight, and the partial sums are added through LDS in wave order.
-#define MOE_KS 8
-template <typename TO, bool GLU>
-__global__ void __launch_bounds__(64 * MOE_KS)
-moe_linear_splitk_kernel(const bf16_t* __restrict__ a, long a_stride, const bf16_t* __restrict__ w, TO* __restrict__ out, long o_stride,
-                         const int* __restrict__ tiles, const int* __restrict__ meta, const int* __restrict__ sorted, int top, int gather,
-                         int K, int N, int F, int act, float limit, float up_shift) {
-  __shared__ float part[MOE_KS][2][4][64];
-  const int tile = blockIdx.x;
-  if (tile >= meta[0]) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, g = lane >> 4;
-  const int o0 = blockIdx.y * 16;
-  const int e = tiles[3 * tile], first = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
-  const int pos = first + min(col, rows - 1);  // rows beyond the tile: read again, never stored
-  const bf16_t* ar = a + (size_t)(gather ? sorted[pos] / top : pos) * a_stride;
-  const bf16_t* wr = w + (size_t)e * N * K + (size_t)min(o0 + col, F - 1) * K;
-  const int share = ((K + MOE_KS * 32 - 1) / (MOE_KS * 32)) * 32;  // k steps of 32 a wave
-  const int k_lo = wave * share, k_hi = min(K, k_lo + share);
-  moe_f32x4 acc = moe_f32x4{0.f, 0.f, 0.f, 0.f}, acc_up = acc;
-#pragma unroll 4
-  for (int k0 = k_lo; k0 < k_hi; k0 += 32) {
-    const int kk = k0 + 8 * g, kc = min(kk, K - 8);  // loads stand under no condition; a chunk beyond the row counts as zeros
-    const uint32_t keep = kk < K ? 0xffffffffu : 0u;
-    const moe_u32x4 x = *reinterpret_cast<const moe_u32x4*>(ar + kc);
-    const moe_u32x4 av = moe_u32x4{x[0] & keep, x[1] & keep, x[2] & keep, x[3] & keep};
-    const moe_u32x4 wv = *reinterpret_cast<const moe_u32x4*>(wr + kc);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(moe_as_bf16x8(wv), moe_as_bf16x8(av), acc, 0, 0, 0);
-    if (GLU) {
-      const moe_u32x4 wu = *reinterpret_cast<const moe_u32x4*>(wr + (size_t)F * K + kc);
-      acc_up = __builtin_amdgcn_mfma_f32_16x16x32_bf16(moe_as_bf16x8(wu), moe_as_bf16x8(av), acc_up, 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    part[wave][0][r][lane] = acc[r];
-    if (GLU) part[wave][1][r][lane] = acc_up[r];
-  }
-  __syncthreads();
-  if (wave != 0 || col >= rows) return;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    float sum = 0.f, sum_up = 0.f;
-#pragma unroll
-    for (int q = 0; q < MOE_KS; ++q) {
-      sum += part[q][0][r][lane];
-      if (GLU) sum_up += part[q][1][r][lane];
-    }
-    const int o = o0 + 4 * g + r;
-    if (o < F) out[(size_t)(first + col) * o_stride + o] = from_float<TO>(GLU ? moe_act(sum, sum_up, act, limit, up_shift) : lev_activate(sum, act));
-  }
-}
-
-// Tiles of 128 rows (prompts, large batches): a workgroup of four waves owns 128 rows and BN weight rows (with glu: BN / 2 outputs' gate
-// rows and the same outputs' up rows), a wave 64 x BN / 2 of them in 32x32x16 products (the transposed product out^T = w a^T: a lane ends
-// with four neighbouring outputs of a row). K goes by in steps of 64, the step after next on its way in registers, two buffers in LDS,
-// one barrier a step that waits for LDS only; loads, LDS writes and fragment reads are issued one by one between the products. Rows
-// beyond the tile are read again and never stored. The workgroups of a tile and of its neighbours in the list (an expert's rows, its
-// weights) follow each other on one of the eight chiplets (workgroups are dealt to them in turn).
-#define MOE_BN 128
-#define MOE_BIG_K 64
-#define MOE_BIG_LD (MOE_BIG_K + 8)
-#define MOE_BIG_LDS(BN) (2 * (MOE_BIG + (BN)) * MOE_BIG_LD * (int)sizeof(bf16_t))
-typedef __attribute__((ext_vector_type(16))) float moe_f32x16;
+struct MoeLinearArgs {
+  const bf16_t* a;
+  long a_stride;
+  const bf16_t* w;
+  void* out;
+  long o_stride;
+  const int *tiles, *meta, *sorted;
+  int top, gather, K, N, F, act;
+  float limit, up_shift;
+  int n_cols, vec;
+};
 template <typename TO>
 __device__ __forceinline__ void moe_store4(TO* p, const float (&v)[4], int n, bool vec);
 template <>
@@ -452,17 +331,95 @@ __device__ __forceinline__ void moe_store4<bf16_t>(bf16_t* p, const float (&v)[4
       if (r < n) p[r] = float_to_bf16(v[r]);
 }
 
-struct MoeLinearArgs {
-  const bf16_t* a;
-  long a_stride;
-  const bf16_t* w;
-  void* out;
-  long o_stride;
-  const int *tiles, *meta, *sorted;
-  int top, gather, K, N, F, act;
-  float limit, up_shift;
-  int n_cols, vec;
-};
+// Tiles of 16 rows (steps of few tokens): the products are bound by reading the chosen experts' weights. A workgroup of KS waves owns one
+// tile and 16 outputs (with glu their gate and up rows; the transposed product out^T = w a^T leaves each lane with four neighbouring
+// outputs of a row); its waves split K in pairs of k-steps (64 k), U pairs on their way at once, and the partial sums are added through LDS
+// in wave order. Weights and rows are read as whole 128-byte lines (8 rows an instruction) and turned into operands in an LDS area of the
+// wave's own: read in operand layout, 64 bytes of each of 16 rows, a load costs the vector cache a look-up for every lane, which bounds
+// such a kernel at 16 bytes a cycle and CU. 33 experts of 2048 x 2048, 5 a token, microseconds of the up and of the gated product, before
+// (operand layout) and now: 1 token 16.6 and 25.5 / 12.6 and 19.8, 8 tokens (20 tiles, 168 MB) 40.7 and 70.5 / 32.6 and 60.3, 64 tokens
+// 81.7 and 136.8 / 54.8 and 99.2; 128 experts of 2048 to 768, 8 a token, 8 tokens: 65 and 127 / 30 and 56. Below K = 2,048 four waves are
+// enough: 1024 x 1024, 8 tokens 11.4 against 12.2 of eight, 768 to 2,048, 32 tokens 62 / 80; at 2,048 eight are: 1 token 12.6 / 13.8.
+#define MOE_SLOTS 72  // 16-byte slots of one staged instruction: 8 rows x (8 chunks + 1 of padding)
+template <typename TO, bool GLU, int KS, int U>
+__global__ void __launch_bounds__(64 * KS)
+moe_linear_few_kernel(const MoeLinearArgs p) {
+  constexpr int G = GLU ? 2 : 1;
+  __shared__ moe_f32x4 part[KS][G][64];
+  __shared__ moe_u32x4 stage[KS][2 * MOE_SLOTS];
+  const int tile = blockIdx.x;
+  if (tile >= p.meta[0]) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, g = lane >> 4, lr = lane >> 3, lc = lane & 7;
+  const int o0 = blockIdx.y * 16, K = p.K, F = p.F;
+  const int e = p.tiles[3 * tile], first = p.tiles[3 * tile + 1], rows = p.tiles[3 * tile + 2];
+  const bf16_t *ar[2], *wr[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int pos = first + min(8 * i + lr, rows - 1);  // rows beyond the tile: read again, never stored
+    ar[i] = p.a + (size_t)(p.gather ? p.sorted[pos] / p.top : pos) * p.a_stride;
+    wr[i] = p.w + (size_t)e * p.N * K + (size_t)min(o0 + 8 * i + lr, F - 1) * K;
+  }
+  moe_u32x4* mine = stage[wave];
+  const int st = lr * 9 + lc, ld = (col >> 3) * MOE_SLOTS + (col & 7) * 9 + g;
+  moe_f32x4 acc[G];
+#pragma unroll
+  for (int x = 0; x < G; ++x) acc[x] = moe_f32x4{0.f, 0.f, 0.f, 0.f};
+  const int pairs = (K + 63) / 64;
+  for (int p0 = wave; p0 < pairs; p0 += KS * U) {
+    moe_u32x4 av[U][2], wv[U][G][2];
+    uint32_t keep[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = (p0 + u * KS) * 64 + lc * 8, kc = min(k, K - 8);  // loads stand under no condition; a chunk beyond K counts as zeros
+      keep[u] = k < K ? 0xffffffffu : 0u;
+#pragma unroll
+      for (int x = 0; x < G; ++x)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) wv[u][x][i] = *reinterpret_cast<const moe_u32x4*>(wr[i] + (size_t)x * F * K + kc);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) av[u][i] = *reinterpret_cast<const moe_u32x4*>(ar[i] + kc);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // all of them are on their way before the first is waited for
+#pragma unroll
+    for (int u = 0; u < U; ++u) {  // LDS executes a wave's instructions in order: the area is used again and again without a barrier
+      const moe_u32x4 mk = moe_u32x4{keep[u], keep[u], keep[u], keep[u]};
+      mine[st] = av[u][0] & mk, mine[MOE_SLOTS + st] = av[u][1] & mk;
+      const moe_u32x4 a_lo = mine[ld], a_hi = mine[ld + 4];
+#pragma unroll
+      for (int x = 0; x < G; ++x) {
+        mine[st] = wv[u][x][0] & mk, mine[MOE_SLOTS + st] = wv[u][x][1] & mk;
+        const moe_u32x4 w_lo = mine[ld], w_hi = mine[ld + 4];
+        acc[x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(moe_as_bf16x8(w_lo), moe_as_bf16x8(a_lo), acc[x], 0, 0, 0);
+        acc[x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(moe_as_bf16x8(w_hi), moe_as_bf16x8(a_hi), acc[x], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int x = 0; x < G; ++x) part[wave][x][lane] = acc[x];
+  __syncthreads();
+  const int o = o0 + 4 * g;
+  if (wave != 0 || col >= rows || o >= F) return;
+#pragma unroll
+  for (int x = 0; x < G; ++x)
+#pragma unroll
+    for (int q = 1; q < KS; ++q) acc[x] += part[q][x][lane];
+  float v[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v[r] = GLU ? moe_act(acc[0][r], acc[G - 1][r], p.act, p.limit, p.up_shift) : lev_activate(acc[0][r], p.act);
+  moe_store4<TO>(static_cast<TO*>(p.out) + (size_t)(first + col) * p.o_stride + o, v, F - o, p.vec);
+}
+
+// Tiles of 128 rows (prompts, large batches): a workgroup of four waves owns 128 rows and BN weight rows (with glu: BN / 2 outputs' gate
+// rows and the same outputs' up rows), a wave 64 x BN / 2 of them in 32x32x16 products (the transposed product out^T = w a^T: a lane ends
+// with four neighbouring outputs of a row). K goes by in steps of 64, the step after next on its way in registers, two buffers in LDS,
+// one barrier a step that waits for LDS only; loads, LDS writes and fragment reads are issued one by one between the products. Rows
+// beyond the tile are read again and never stored. The workgroups of a tile and of its neighbours in the list (an expert's rows, its
+// weights) follow each other on one of the eight chiplets (workgroups are dealt to them in turn).
+#define MOE_BN 128
+#define MOE_BIG_K 64
+#define MOE_BIG_LD (MOE_BIG_K + 8)
+#define MOE_BIG_LDS(BN) (2 * (MOE_BIG + (BN)) * MOE_BIG_LD * (int)sizeof(bf16_t))
+typedef __attribute__((ext_vector_type(16))) float moe_f32x16;
 // BM: 128, or 64 for a tile whose rows fit that
 template <typename TO, bool GLU, int BN, int BM>
 __device__ __forceinline__ void moe_big_tile(const MoeLinearArgs& p, unsigned char* moe_smem, int e, int first, int rows, int ycol) {
@@ -636,26 +593,11 @@ extern "C" int lev_moe_linear(const void* a, long a_stride, const void* w, void*
   LEV_REQUIRE(a_stride >= K && o_stride >= F, "experts: row strides are smaller than the rows");
   if (max_tiles == 0) return 0;
   if (dtype == LEV_BF16 && use_mfma && K % 8 == 0 && a_stride % 8 == 0 && ((uintptr_t)a & 15) == 0 && ((uintptr_t)w & 15) == 0) {
-    if (tile_rows == MOE_TM && max_tiles <= 96) {  // a step of single tokens: K split over the waves of a workgroup
-      dim3 grid_k(max_tiles, (F + 15) / 16);
-#define MOE_SPLITK(TO)                                                                                                                           \
-  do {                                                                                                                                           \
-    if (glu)                                                                                                                                     \
-      moe_linear_splitk_kernel<TO, true><<<grid_k, 64 * MOE_KS, 0, stream>>>((const bf16_t*)a, a_stride, (const bf16_t*)w, (TO*)out, o_stride, tiles, \
-                                                                            meta, sorted, top, gather, K, N, F, act, limit, up_shift);                            \
-    else                                                                                                                                         \
-      moe_linear_splitk_kernel<TO, false><<<grid_k, 64 * MOE_KS, 0, stream>>>((const bf16_t*)a, a_stride, (const bf16_t*)w, (TO*)out, o_stride, tiles, \
-                                                                             meta, sorted, top, gather, K, N, F, act, limit, up_shift);                           \
-  } while (0)
-      if (out_dtype == LEV_F32) MOE_SPLITK(float); else MOE_SPLITK(bf16_t);
-#undef MOE_SPLITK
-      return lev_check_launch("moe_linear (matrix cores, K split)");
-    }
+    const int vec = o_stride % 4 == 0 && ((uintptr_t)out & (out_dtype == LEV_F32 ? 15 : 7)) == 0;
     if (tile_rows == MOE_BIG) {
       const int bn = glu ? MOE_BN / 2 : MOE_BN, n_cols = (F + bn - 1) / bn;
       const long blocks = (long)((max_tiles + 7) / 8) * 8 * n_cols;
       LEV_REQUIRE(blocks <= 0x7fffffffL, "experts: too many tiles (%ld)", blocks);
-      const int vec = o_stride % 4 == 0 && ((uintptr_t)out & (out_dtype == LEV_F32 ? 15 : 7)) == 0;
 #define MOE_BIG_CASE(TO, G)                                                                                                                       \
   do {                                                                                                                                            \
     hipError_t e = hipFuncSetAttribute((const void*)moe_linear_big_kernel<TO, G>, hipFuncAttributeMaxDynamicSharedMemorySize, MOE_BIG_LDS(MOE_BN)); \
@@ -671,20 +613,19 @@ extern "C" int lev_moe_linear(const void* a, long a_stride, const void* w, void*
 #undef MOE_BIG_CASE
       return lev_check_launch("moe_linear (matrix cores, tiles of 128 rows)");
     }
-    // many tiles of 16 rows: a wave per tile and 32 outputs, both operands straight from global memory
-    const int nt = 2;
-    dim3 grid(max_tiles, (F + 64 * nt - 1) / (64 * nt));
-#define MOE_CASE(TO)                                                                                                                             \
-  do {                                                                                                                                           \
-    if (glu)                                                                                                                                     \
-      moe_linear_mfma_kernel<TO, 2, true, 1><<<grid, 256, 0, stream>>>((const bf16_t*)a, a_stride, (const bf16_t*)w, (TO*)out, o_stride, tiles, meta, \
-                                                                      sorted, top, gather, K, N, F, act, limit, up_shift);                                        \
-    else                                                                                                                                         \
-      moe_linear_mfma_kernel<TO, 2, false, 1><<<grid, 256, 0, stream>>>((const bf16_t*)a, a_stride, (const bf16_t*)w, (TO*)out, o_stride, tiles,  \
-                                                                       meta, sorted, top, gather, K, N, F, act, limit, up_shift);                                 \
+    const MoeLinearArgs args{(const bf16_t*)a, a_stride, (const bf16_t*)w, out, o_stride, tiles, meta, sorted, top, gather, K, N, F, act, limit, up_shift, 0, vec};
+    const dim3 grid(max_tiles, (F + 15) / 16);
+#define MOE_FEW(TO, G)                                                                              \
+  do {                                                                                              \
+    if (K < 2048) moe_linear_few_kernel<TO, G, 4, 2><<<grid, 64 * 4, 0, stream>>>(args);            \
+    else moe_linear_few_kernel<TO, G, 8, 2><<<grid, 64 * 8, 0, stream>>>(args);                     \
   } while (0)
-    if (out_dtype == LEV_F32) MOE_CASE(float); else MOE_CASE(bf16_t);
-#undef MOE_CASE
+    if (out_dtype == LEV_F32) {
+      if (glu) MOE_FEW(float, true); else MOE_FEW(float, false);
+    } else {
+      if (glu) MOE_FEW(bf16_t, true); else MOE_FEW(bf16_t, false);
+    }
+#undef MOE_FEW
     return lev_check_launch("moe_linear (matrix cores)");
   }
   dim3 grid(max_tiles, (F + 15) / 16);

@@ -1209,10 +1209,10 @@ class HipKernels:
 
     @staticmethod
     def moe_tile_rows(pairs: int, n_experts: int) -> int:
-        """Rows of a tile of the experts' products: 128 where an expert has 12 rows or more on average, else 16 (32 experts of 2048 x 2048,
-        4 a token, microseconds of the two products, 16 / 128: 64 tokens 56 + 57 / 51 + 50 (gated 126 / 135 for the first), 128 tokens 96 + 89 /
-        53 + 51, 256 tokens 137 + 140 / 55 + 55)."""
-        return 128 if pairs >= 12 * n_experts else 16
+        """Rows of a tile of the experts' products: 128 where an expert has more than 16 rows on average, else 16 (32 experts of 2048 x 2048,
+        4 a token, microseconds of the two products, 16 / 128: 64 tokens 50 + 51 / 72 + 72 (gated 97 / 135 for the first), 128 tokens 65 + 73 /
+        72 + 73 (121 / 136), 192 tokens 82 + 119 / 73 + 74 (155 / 136))."""
+        return 128 if pairs > 16 * n_experts else 16
 
     def moe_max_tiles(self, pairs: int, n_experts: int, tile_rows: int = 16) -> int:
         return int(self.lib.lev_moe_max_tiles(int(pairs), int(n_experts), int(tile_rows)))
