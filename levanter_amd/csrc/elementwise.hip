@@ -296,6 +296,8 @@ extern "C" int lev_norm_pending(float* x, const float* partial, int S, const flo
 // contiguous on both sides: 16-byte (bf16) copies. Values are transposed through LDS: where 8 tokens in a row go
 // to 8 consecutive, aligned slots of one page (a prompt portion does, except at its ragged ends), a thread writes
 // its head-dim row for all 8 at once; other tokens are written element by element.
+// Small steps are bound by the chain of loads and waits of a thread, so a thread has as little to do as the head sizes allow
+// (256 tokens, 25 heads of 64, some of them single: 7.8 us with a wave a workgroup and tokens in turn, 5.6 now).
 #define KVW_TOKENS 16
 
 template <typename T>
@@ -318,64 +320,44 @@ __global__ void kv_write_kernel(const T* __restrict__ k, const T* __restrict__ v
   const int h = blockIdx.y;
   const int tid = threadIdx.x;
   if (tid < KVW_TOKENS) dst_s[tid] = t0 + tid < n_tokens ? dest[t0 + tid] : -1;
-  const int chunks = HD / 8, v_chunks = VD / 8;
-  // keys: one chunk of one token per thread and turn
-  for (int idx = tid; idx < KVW_TOKENS * chunks; idx += blockDim.x) {
-    const int i = idx / chunks, c = idx % chunks;
-    const int t = t0 + i;
+  const int chunks = HD / 8, n_k = KVW_TOKENS * chunks, v_chunks = VD / 8;
+  // one chunk of one token per thread and turn: keys into their pages, values into LDS (a value head may have another size than a key head)
+  for (int idx = tid; idx < n_k + KVW_TOKENS * v_chunks; idx += blockDim.x) {
+    const bool value = idx >= n_k;
+    const int per = value ? v_chunks : chunks, at = value ? idx - n_k : idx, i = at / per, c = at % per, t = t0 + i;
     if (t >= n_tokens) continue;
+    const T* from = value ? v + (size_t)t * v_stride + (size_t)h * VD + c * 8 : k + (size_t)t * k_stride + (size_t)h * HD + c * 8;
     const int dst = dest[t];
     if (dst < 0) continue;
-    const T* kr = k + (size_t)t * k_stride + (size_t)h * HD + c * 8;
-    const int page = dst / PS, off = dst % PS;
-    T* kd = k_pages + ((size_t)page * KVH + h) * (size_t)HD * PS + ((size_t)c * PS + off) * 8;
+    T* to = value ? vt + i * ldv + c * 8 : k_pages + ((size_t)(dst / PS) * KVH + h) * (size_t)HD * PS + ((size_t)c * PS + dst % PS) * 8;
     if (vec_ok) {
-      copy8<T>(kd, kr);
+      copy8<T>(to, from);
     } else {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) kd[e] = kr[e];
-    }
-  }
-  // values into LDS on the way (a value head may have another size than a key head)
-  for (int idx = tid; idx < KVW_TOKENS * v_chunks; idx += blockDim.x) {
-    const int i = idx / v_chunks, c = idx % v_chunks;
-    const int t = t0 + i;
-    if (t >= n_tokens) continue;
-    if (dest[t] < 0) continue;
-    const T* vr = v + (size_t)t * v_stride + (size_t)h * VD + c * 8;
-    if (vec_ok) {
-      copy8<T>(vt + i * ldv + c * 8, vr);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) vt[i * ldv + c * 8 + e] = vr[e];
+      for (int e = 0; e < 8; ++e) to[e] = from[e];
     }
   }
   __syncthreads();
-  for (int d = tid; d < VD; d += blockDim.x) {
-    int i = 0;
-    while (i < KVW_TOKENS) {
-      const int dst = dst_s[i];
-      if (dst < 0) {
-        ++i;
-        continue;
-      }
-      const int page = dst / PS, off = dst % PS;
-      T* vd = v_pages + ((size_t)page * KVH + h) * (size_t)VD * PS + (size_t)d * PS + off;
-      bool run = vec_ok && (off % 8 == 0) && i + 8 <= KVW_TOKENS;
-      if (run) {
+  // a head-dim row of up to 8 tokens per thread and turn; the tokens are cut where the first one's slots reach a multiple of 8
+  const int cut = dst_s[0] < 0 ? 0 : -dst_s[0] & 7, n_runs = KVW_TOKENS / 8 + (cut > 0);
+  for (int idx = tid; idx < n_runs * VD; idx += blockDim.x) {
+    const int r = idx / VD, d = idx - r * VD, lo = cut ? max(0, cut + 8 * (r - 1)) : 8 * r, n = min(cut ? cut + 8 * r : 8 * r + 8, KVW_TOKENS) - lo;
+    int dst[8];
 #pragma unroll
-        for (int j = 1; j < 8; ++j) run = run && dst_s[i + j] == dst + j;
-      }
-      if (run) {
-        __attribute__((aligned(16))) T row[8];
+    for (int j = 0; j < 8; ++j) dst[j] = j < n ? dst_s[lo + j] : -1;
+    bool run = vec_ok && dst[0] >= 0 && dst[0] % 8 == 0;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) row[j] = vt[(i + j) * ldv + d];
-        copy8<T>(vd, row);
-        i += 8;
-      } else {
-        *vd = vt[i * ldv + d];
-        ++i;
-      }
+    for (int j = 1; j < 8; ++j) run = run && dst[j] == dst[0] + j;
+    T* base = v_pages + (size_t)h * VD * PS + (size_t)d * PS;
+    if (run) {  // pages hold a multiple of 8 tokens: the slots lie in one
+      __attribute__((aligned(16))) T row[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) row[j] = vt[(lo + j) * ldv + d];
+      copy8<T>(base + (size_t)(dst[0] / PS) * KVH * VD * PS + dst[0] % PS, row);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (dst[j] >= 0) base[(size_t)(dst[j] / PS) * KVH * VD * PS + dst[j] % PS] = vt[(lo + j) * ldv + d];
     }
   }
 }
@@ -396,8 +378,7 @@ extern "C" int lev_kv_write(const void* k, const void* v, long k_stride, long v_
   const int vec_ok = ((uintptr_t)k % 16 == 0) && ((uintptr_t)v % 16 == 0) && (k_stride * esize % 16 == 0) && (v_stride * esize % 16 == 0) &&
                      ((uintptr_t)k_pages % 16 == 0) && ((uintptr_t)v_pages % 16 == 0);
   dim3 grid((T + KVW_TOKENS - 1) / KVW_TOKENS, KVH);
-  const int widest = HD > VD ? HD : VD;
-  const int nt = widest <= 64 ? 64 : (widest <= 128 ? 128 : 256);
+  const int nt = HD + VD <= 32 ? 64 : (HD + VD <= 64 ? 128 : 256);  // a chunk a thread, or two
   if (dtype == LEV_F32)
     kv_write_kernel<float><<<grid, nt, lds, stream>>>((const float*)k, (const float*)v, k_stride, v_stride, (float*)k_pages,
                                                       (float*)v_pages, dest, T, KVH, HD, VD, PS, vec_ok);
