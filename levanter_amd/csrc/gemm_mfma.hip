@@ -7,7 +7,7 @@
 //   stream kernel (M <= 128; up to 64 rows where an estimate puts it ahead of the skinny kernel: long sums, many rows): the weights are the traffic; `a` is shared through LDS by the 4 to 16 waves of a
 //                 workgroup, the weights go straight into MFMA operand registers, K is split over workgroups
 //                 and a second kernel adds the partial sums in a fixed order;
-//   skinny kernel (M <= 64, see use_skinny): a workgroup owns 8 to 64 output columns; its waves split K, bring whole lines of w
+//   skinny kernel (M <= 64, small weights to 256 rows, see use_skinny): a workgroup owns 8 to 64 output columns; its waves split K, bring whole lines of w
 //                 and a through an LDS area of their own into MFMA operand registers (16x16x32), and their partial sums are
 //                 added through LDS in a fixed order.
 // No atomics anywhere: results are deterministic. K and lda must be multiples of 8 (16-byte operand loads);
@@ -330,7 +330,7 @@ static int launch_tile(const bf16_t* a, long lda, const bf16_t* w, const float* 
 }
 
 // ------------------------------------------------------------------------------------------------
-// Skinny kernel (M <= SKINNY_MAX_M: MT = 1 .. 4 tiles of 16 rows). A workgroup owns NT units of 16 output columns (or, HALF, one of 8); its
+// Skinny kernel (M <= 64: MT = 1 .. 4 tiles of 16 rows; small weights up to 256 rows, in blocks of rows). A workgroup owns NT units of 16 output columns (or, HALF, one of 8); its
 // WAVES waves split K. A wave takes pairs of adjacent 32-wide k-steps (64 k = 128 bytes of a row), U pairs in flight. Weights and `a`
 // alike are read as WHOLE 128-byte lines - lane (row l/8, 16-byte chunk l%8), one instruction for 8 rows - and turned into the operand
 // layout (row l%16, k-group l/16) through a small LDS area of the wave's own. The vector cache looks lines up by neighbouring
@@ -345,9 +345,9 @@ static int launch_tile(const bf16_t* a, long lda, const bf16_t* w, const float* 
 // place of the k range, so that they do not all read the same part of `a` and the same residue of the weight
 // rows at the same time; the order of the sum depends on the column tile only, never on M or the batch.
 #define SKINNY_SLOTS 72  // 16-byte slots of one staged instruction: 8 rows x (8 chunks + 1 of padding)
-#define SKINNY_MAX_M 64  // with four row tiles; which of these row counts it takes: use_skinny()
+#define SKINNY_MAX_M 256  // which of these row counts it takes: use_skinny()
 
-template <typename TO, int WAVES, int U, int MT, int NT, bool HALF>
+template <typename TO, int WAVES, int U, int MT, int NT, bool HALF, bool BLOCKS>
 __global__ void __launch_bounds__(WAVES * 64)
 gemm_skinny_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restrict__ w, const float* __restrict__ bias,
                    const float* residual, long ldr, TO* out, long ldo, int M, int N, int K, int act) {
@@ -359,6 +359,14 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restr
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int n0 = blockIdx.x * COLS * NT;
+  if constexpr (BLOCKS) {
+    if (n0 >= N) return;  // the grid's columns are a multiple of 8
+    const int m0 = blockIdx.y * 16 * MT;
+    a += (size_t)m0 * lda;
+    out += (size_t)m0 * ldo;
+    if (residual) residual += (size_t)m0 * ldr;
+    M = min(M - m0, 16 * MT);
+  }
   const int fr = lane & 15, kg = lane >> 4;
   const int lr = lane >> 3, lc = lane & 7;  // loads: row (0..7, instruction i adds 8 i) and chunk of the line
   const bf16_t* wrow[NT][WI];
@@ -489,7 +497,25 @@ struct SkinnyShape {
   bool half;
   int cols() const { return half ? 8 : 16 * units; }
 };
+// Above 64 rows the rows are cut into blocks (the grid's y; its x a multiple of 8, so that the blocks of a column tile share a chiplet's L2):
+// every workgroup has a CU of its own, waves that split K need no barrier, and all their loads are out at once, where a tile kernel of
+// barriers and the library wait for memory at every step. Measured in graphs over distinct weights, microseconds, here / the better of
+// the library and the stream or tile kernel: 4800 x 1600 at 96 / 128 / 192 rows 9.6 / 12.7, 9.7 / 13.4, 10.3 / 16.8; 6400 x 1600 at 96 / 128 rows
+// 12.6 / 17.3, 13.0 / 17.7; 1600 x 1600 at 96 / 192 / 256 rows 7.0 / 11.0, 7.7 / 11.2, 7.7 / 12.4; 2304 x 768 5.4 / 7.1, 6.0 / 7.5, 7.4 / 7.7. In two
+// rounds it is behind (4800 x 1600 at 256 rows 17.0 / 17.2, 6400 x 1600 20.1 / 17.7, 12288 x 4096 at 96 rows 34.6 / 30.1), and for
+// long sums the kernels that split K over workgroups are ahead (1600 x 6400 at 96 rows 17.7 / 12.4).
+static bool skinny_blocks_fit(int M, int N, int row_tiles, int units) {
+  const long columns = (N + 16 * units - 1) / (16 * units);
+  return (M + 16 * row_tiles - 1) / (16 * row_tiles) * ((columns + 7) / 8 * 8) <= 256;
+}
+static bool skinny_in_blocks(int M, int N, int K) { return M > 64 && M <= SKINNY_MAX_M && K <= 2048 && skinny_blocks_fit(M, N, 4, 4); }
 static SkinnyShape skinny_shape(int M, int N, int K) {
+  if (M > 64) {  // the smallest blocks that make one round
+    if (skinny_blocks_fit(M, N, 2, 2)) return {8, 2, 2, 2, false};
+    for (int units = 2; units < 4; ++units)
+      if (skinny_blocks_fit(M, N, 4, units)) return {8, 1, 4, units, false};
+    return {8, 1, 4, 4, false};
+  }
   const int tiles = (N + 15) / 16;
   if (M <= 16) {
     if (N <= 2048) return K > 4096 && M <= 8 ? SkinnyShape{16, 2, 1, 1, true} : SkinnyShape{8, 2, 1, 1, true};
@@ -512,10 +538,23 @@ template <typename TO>
 static void launch_skinny(const bf16_t* a, long lda, const bf16_t* w, const float* bias, const float* residual, long ldr,
                           TO* out, long ldo, int M, int N, int K, int act, hipStream_t stream) {
   const SkinnyShape sh = skinny_shape(M, N, K);
-  const int cols = sh.cols();
+  const int cols = sh.cols(), columns = (N + cols - 1) / cols;
 #define LEV_SKINNY(W_, U_, MT_, NT_, H_)                                                                                          \
   if (sh.waves == W_ && sh.in_flight == U_ && sh.row_tiles == MT_ && sh.units == NT_ && sh.half == H_)                             \
-    gemm_skinny_kernel<TO, W_, U_, MT_, NT_, H_><<<(N + cols - 1) / cols, W_ * 64, 0, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act)
+    gemm_skinny_kernel<TO, W_, U_, MT_, NT_, H_, false><<<columns, W_ * 64, 0, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act)
+  // row blocks are a variant of their own: what finds them costs the small steps' kernels 0.2 - 0.4 us
+#define LEV_SKINNY_BLOCKS(U_, MT_, NT_)                                                                                           \
+  if (sh.row_tiles == MT_ && sh.units == NT_)                                                                                     \
+    gemm_skinny_kernel<TO, 8, U_, MT_, NT_, false, true><<<grid, 8 * 64, 0, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act)
+  if (M > 64) {
+    const dim3 grid((columns + 7) / 8 * 8, (M + 16 * sh.row_tiles - 1) / (16 * sh.row_tiles));
+    LEV_SKINNY_BLOCKS(2, 2, 2);
+    LEV_SKINNY_BLOCKS(1, 4, 2);
+    LEV_SKINNY_BLOCKS(1, 4, 3);
+    LEV_SKINNY_BLOCKS(1, 4, 4);
+    return;
+  }
+#undef LEV_SKINNY_BLOCKS
   LEV_SKINNY(16, 2, 1, 1, true);
   LEV_SKINNY(8, 2, 1, 1, true);
   LEV_SKINNY(8, 2, 1, 1, false);
@@ -828,7 +867,7 @@ static TilePlan plan_tiles(int M, int N, int K) {
   return best;
 }
 
-// Which kernel takes M <= SKINNY_MAX_M rows. An estimate of the skinny kernel in microseconds, from the measurements above: a launch and
+// Which kernel takes M <= 64 rows (above: skinny_in_blocks). An estimate of the skinny kernel in microseconds, from the measurements above: a launch and
 // its ramp, and the longest of the weights' read from memory, the share of it that falls to the busiest CU, and what that CU pulls
 // through its caches (its columns and all of `a`, for each of its workgroups). The stream kernel's time hardly grows with the
 // rows, but it pays for its K ranges: plan_stream's cost is about 0.8 of what it takes with the kernel that adds them (which the next norm may do in passing: 1.2). Measured,
@@ -853,7 +892,7 @@ extern "C" int lev_linear_mfma_force(int kind) {
   return 0;
 }
 static bool use_skinny(int M, int N, int K) {
-  if (M > SKINNY_MAX_M) return false;
+  if (M > 64) return skinny_in_blocks(M, N, K) && g_force_kernel != 2;
   if (g_force_kernel) return g_force_kernel == 1;
   return skinny_estimate(M, N, K) <= 1.2 * plan_stream(M, N, K).cost;
 }

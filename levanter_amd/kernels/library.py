@@ -444,16 +444,19 @@ class HipKernels:
         134 M numbers (18432 x 6144 at 48 / 64 rows 57.3 / 54.0, 64.0 / 55.2); everything else is ours (12288 x 4096 at 32 / 64 rows 21.2 / 22.7
         and 25.7 / 24.8, 16384 x 4096 26.3 / 33.5 and 31.6 / 33.0, 10752 x 2048 10.8 / 14.6 and 14.4 / 15.8). From 65 to 255 rows: wide outputs of large
         weights (N >= 2 K, 32 MB and more: at 160 rows qkv and fc of a 4096-wide layer 49.7 / 37.2 and 55.7 / 41.6); ours keep N = K (22.1 /
-        24.6 at 128) and K = 4 N (43.5 / 81.1), and below 96 rows the largest weights (more than 256 MB)."""
+        24.6 at 128) and K = 4 N (43.5 / 81.1), and below 96 rows the largest weights (more than 256 MB). Up to 256 rows our kernel
+        of row blocks keeps short sums (K to 2,048) whose blocks of 64 x 64 make one round of the CUs (4800 x 1600 at 96 / 192 rows 9.6 / 12.7, 10.3 / 16.8)."""
         if act not in cls.LIBRARY_ACTIVATIONS or M < cls.LIBRARY_MIN_ROWS:
             return False
         if M <= 64:
             return (N > 16384 and K < 2048) or (M > 32 and N >= 2 * K and (1 << 26) < N * K <= (1 << 27))
+        if M <= 256 and K <= 2048 and -(-M // 64) * (-(-N // 512) * 8) <= 256:
+            return False
         if M < 256:
             if N < 2 * K:
                 return False
             if N * K < (1 << 24):
-                return M >= 128  # a 1600-wide layer: qkv 16.5 / 14.2 at 128 rows, 17.3 / 14.5 at 192, but 12.8 / 14.3 at 64
+                return M >= 128  # a 1600-wide layer with the tile kernel: fc 20.5 / 17.7 at 128 rows, 19.1 / 18.7 at 192
             return not (M < 96 and N * K > (1 << 27))
         if M < 320 and N * K < (1 << 24):
             return N >= 2 * K

@@ -43,3 +43,25 @@ def test_linear_skinny_against_float64(K, N, Ki, monkeypatch):
     finally:
         K._check(gemm.lev_linear_mfma_force(0))
         K._ws_need.clear()
+
+
+@pytest.mark.parametrize("N", [1, 24, 511, 768, 1600, 2304, 4096])
+@pytest.mark.parametrize("Ki", [8, 72, 1600, 2040, 2048])
+def test_linear_in_row_blocks_against_float64(K, N, Ki, monkeypatch):
+    """65 to 256 rows of small weights, in blocks of 32 or 64 rows; the bound is the one above."""
+    gemm = K._unit("gemm_mfma")
+    monkeypatch.setattr(K, "gemm_library", False)
+    g = torch.Generator(device=DEV).manual_seed(N * 31 + Ki)
+    w = torch.randn(N, Ki, device=DEV, generator=g).bfloat16()
+    bias = torch.randn(N, device=DEV, generator=g)
+    for M in (65, 95, 128, 130, 193, 256):
+        taken = -(-M // 64) * (-(-N // 512) * 8) <= 256
+        assert not taken or gemm.lev_linear_mfma_ranges(M, N, Ki) == 1
+        a = torch.randn(M, Ki + 8, device=DEV, generator=g).bfloat16()[:, :Ki]
+        res = torch.randn(M, N, device=DEV, generator=g)
+        want = a.double() @ w.double().T + bias.double() + res.double()
+        size = a.double().abs() @ w.double().abs().T + bias.double().abs() + res.double().abs()
+        out = torch.full((M + 1, N + 3), float("nan"), device=DEV)
+        K.linear(a, w, bias, out[:M, :N], residual=res)
+        assert bool(((out[:M, :N].double() - want).abs() <= (Ki + 4) * 2.0 ** -24 * size).all()), M
+        assert bool(torch.isnan(out[:M, N:]).all()) and bool(torch.isnan(out[M]).all())
