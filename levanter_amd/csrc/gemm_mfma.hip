@@ -867,21 +867,23 @@ static TilePlan plan_tiles(int M, int N, int K) {
   return best;
 }
 
-// Which kernel takes M <= 64 rows (above: skinny_in_blocks). An estimate of the skinny kernel in microseconds, from the measurements above: a launch and
-// its ramp, and the longest of the weights' read from memory, the share of it that falls to the busiest CU, and what that CU pulls
-// through its caches (its columns and all of `a`, for each of its workgroups). The stream kernel's time hardly grows with the
-// rows, but it pays for its K ranges: plan_stream's cost is about 0.8 of what it takes with the kernel that adds them (which the next norm may do in passing: 1.2). Measured,
-// skinny / stream: 1600 x 6400 at 16 / 24 / 32 / 64 rows 9.5 / 11.4, 11.6 / 11.7, 12.6 / 11.9, 20.0 / 13.8; 4096 x 16384 at 24 / 48 rows 28.1 / 33.4,
-// 39.1 / 35.1; 6144 x 24576 at 24 rows 67.7 / 61.0; 16384 x 4096 at 64 rows 32.2 / 37.1; 6144 x 6144 at 6 rows 15.7 / 21.1.
+// Which kernel takes M <= 64 rows (above: skinny_in_blocks). An estimate of the skinny kernel in microseconds: a launch and its ramp, and
+// the longest of the weights' read from memory, the share of it that falls to the busiest CU, and what that CU pulls through its caches
+// (its columns and most of `a`, for each of its workgroups). The stream kernel's time hardly grows with the rows, but it pays for its K
+// ranges: plan_stream's cost is about 0.8 of what it takes with the kernel that adds them (which the next norm may do in passing: 1.18).
+// The constants are fitted to 154 cases (22 weights of 2 to 400 MB at 1, 8, 16, 24, 32, 48 and 64 rows): 7 % off the measured time on
+// average, and the choice on average within 1 % of the better kernel. Measured, skinny / stream: 16384 x 4096 at 8 / 64 rows 24.5 / 33.2,
+// 31.9 / 37.4; 4096 x 16384 at 8 / 32 / 64 rows 24.2 / 32.7, 31.3 / 33.9, 43.9 / 36.4; 1600 x 6400 at 16 / 24 / 32 / 64 rows 9.2 / 11.1, 11.0 / 11.4,
+// 12.3 / 11.6, 19.0 / 13.4; 6144 x 24576 at 8 / 24 rows 57.6 / 59.7, 67.1 / 61.0; 24576 x 6144 at 8 / 64 rows 53.0 / 59.1, 77.1 / 67.8.
 static double skinny_estimate(int M, int N, int K) {
   const SkinnyShape sh = skinny_shape(M, N, K);
   const long wgs = (N + sh.cols() - 1) / sh.cols(), r = (wgs + 255) / 256;  // r: workgroups of the busiest CU
-  const double memory = 2.0 * N * K / 5.5e6, own = r * (double)sh.cols() * K * 2.0 / 31e3;
-  const double rate = (long)N * K <= (1L << 23) ? 75e3 : sh.waves == 4 ? 37e3 : sh.units > 1 ? 45e3 : 50e3;  // small weights stay in the caches' reach
-  const double caches = r * (double)(sh.cols() + M) * K * 2.0 / rate;
+  const double memory = 2.0 * N * K / 6.27e6, own = r * (double)sh.cols() * K * 2.0 / 42e3;
+  const double rate = (long)N * K <= (1L << 23) ? 79e3 : sh.waves == 4 ? 39e3 : sh.units > 1 ? 37e3 : 48e3;  // small weights stay in the caches' reach
+  const double caches = r * (sh.cols() + 0.85 * M) * K * 2.0 / rate;
   double cost = memory > own ? memory : own;
   if (caches > cost) cost = caches;
-  return 3.2 + cost + (sh.row_tiles > 1 && r > 4 ? 0.8 * (r - 1) : 0.0);
+  return 3.26 + cost + (sh.row_tiles > 1 && r > 4 ? 1.1 * (r - 1) : 0.0);
 }
 // 0: the estimate decides; 1 / 2: the skinny / the stream kernel wherever it takes the row count. For measurements of the
 // choice itself (a test times both candidates at widths the estimates were not fitted to); not used by the engine.
@@ -894,7 +896,7 @@ extern "C" int lev_linear_mfma_force(int kind) {
 static bool use_skinny(int M, int N, int K) {
   if (M > 64) return skinny_in_blocks(M, N, K) && g_force_kernel != 2;
   if (g_force_kernel) return g_force_kernel == 1;
-  return skinny_estimate(M, N, K) <= 1.2 * plan_stream(M, N, K).cost;
+  return skinny_estimate(M, N, K) <= 1.18 * plan_stream(M, N, K).cost;
 }
 
 // Into how many ranges the sum over K is split (1: the kernel finishes its outputs itself).
