@@ -607,44 +607,16 @@ __device__ __forceinline__ void decode_wave(int idx, int kvh, int z, const bf16_
   // holds the token's position, which then has the copy ahead of its two or more blocks.
   const bool idle_last = splits > 1 && kb_first + (splits - 1) * per > kb_last;
   const bool owner = fused && (idle_last ? z == splits - 1 : (kb_begin <= kb_last && kb_last < kb_end));
-  const bf16_t* kn = fused ? k_new + (size_t)t * kv_stride + (size_t)kvh * HD : nullptr;
-  const bf16_t* vn = fused ? v_new + (size_t)t * kv_stride + (size_t)kvh * HD : nullptr;
-
-  if (owner) {  // read by later steps only: this step takes them from k_new / v_new
-    const int dst = dest[t];
-    if (dst >= 0) {
-      bf16_t* kb_ = k_pages + ((size_t)(dst >> ps_shift) * KVH + kvh) * head_elems;
-      bf16_t* vb_ = v_pages + ((size_t)(dst >> ps_shift) * KVH + kvh) * head_elems;
-      const int off = dst & ps_mask;
-      for (int c = lane; c < NCHUNK; c += 64)
-        *reinterpret_cast<u32x4*>(kb_ + ((size_t)c * PS + off) * 8) = *reinterpret_cast<const u32x4*>(kn + c * 8);
-      for (int d = lane; d < HD; d += 64) vb_[(size_t)d * PS + off] = vn[d];
-    }
-  }
-
-  u32x4 qf[NKS];
-#pragma unroll
-  for (int s = 0; s < NKS; ++s) {
-    const int c = 4 * s + g;
-    qf[s] = (q_pos >= 0 && c < NCHUNK) ? *reinterpret_cast<const u32x4*>(q + (size_t)t * q_stride + (size_t)head * HD + c * 8)
-                                        : u32x4{0, 0, 0, 0};
-  }
-  f32x4 o[NDT];
-#pragma unroll
-  for (int i = 0; i < NDT; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY, l = 0.f;
+  const bf16_t* q_row = q + (size_t)t * q_stride;
+  const bf16_t* kn = fused ? k_new + (size_t)t * kv_stride + (size_t)kvh * HD : q_row + (size_t)kvh * G * HD;  // unfused: read, not used
+  const bf16_t* vn = fused ? v_new + (size_t)t * kv_stride + (size_t)kvh * HD : q_row + (size_t)kvh * G * HD;
 
   // Every load below is unconditional, from a clamped address, and what it must not deliver is masked out afterwards:
   // a load under a condition becomes a branch, and at the join the compiler waits for all loads in flight, which
   // turned the 38 loads of a block into as many round trips to memory, one after the other.
-  // This lane's rows of the token's new value, read once, two to a register.
-  uint32_t nv2[(NDT + 1) / 2];
-#pragma unroll
-  for (int i = 0; i < (NDT + 1) / 2; ++i) nv2[i] = 0u;
-  if (fused) {
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) nv2[dt / 2] |= (uint32_t)vn[16 * dt + fr] << (16 * (dt & 1));
-  }
+  // The first block's page ids, the queries, the new value and what the owner copies are one round trip together, and the copy's
+  // stores come last: one after the other, with waits between, they took longer than a short context's keys. GPT-2 small, one
+  // token of 250 keys 5.4 -> 4.9 us; XL, a few of 500 keys 7.3 -> 6.5; 64 tokens of 32 heads of 128 at 100 keys 33.8 -> 31.5.
   // Page ids of a block of 64 keys, per lane: one per key tile (u, hh) and one per group of 8 values (u). They are read
   // one block ahead (behind the block's own loads, into the registers those have just used), so that no key or value
   // load waits for a table lookup. Positions beyond the token's own are clamped to it (its table entry exists);
@@ -666,6 +638,31 @@ __device__ __forceinline__ void decode_wave(int idx, int kvh, int z, const bf16_
     }
   };
   page_ids(min(kb_begin, kb_last));
+  u32x4 qf[NKS];
+#pragma unroll
+  for (int s = 0; s < NKS; ++s) qf[s] = *reinterpret_cast<const u32x4*>(q_row + (size_t)(kvh * G + min(fr, G - 1)) * HD + min(4 * s + g, NCHUNK - 1) * 8);
+  bf16_t nv[NDT];  // this lane's rows of the token's new value
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt) nv[dt] = vn[16 * dt + fr];
+  // the owner's copy: read by later steps only, this step takes the new key and value from k_new / v_new
+  const int copy_to = *(fused ? dest + t : decode_tokens + idx);
+  const u32x4 copy_k = *reinterpret_cast<const u32x4*>(kn + min(lane, NCHUNK - 1) * 8);
+  bf16_t copy_v[(HD + 63) / 64];
+#pragma unroll
+  for (int i = 0; i < (HD + 63) / 64; ++i) copy_v[i] = vn[min(64 * i + lane, HD - 1)];
+  __builtin_amdgcn_sched_barrier(0);  // all of them are on their way before the first is waited for
+#pragma unroll
+  for (int s = 0; s < NKS; ++s) {
+    const uint32_t mk = q_pos >= 0 && 4 * s + g < NCHUNK ? 0xffffffffu : 0u;
+    qf[s] = qf[s] & u32x4{mk, mk, mk, mk};
+  }
+  uint32_t nv2[(NDT + 1) / 2];  // two to a register
+#pragma unroll
+  for (int i = 0; i < (NDT + 1) / 2; ++i) nv2[i] = (uint32_t)nv[2 * i] | (2 * i + 1 < NDT ? (uint32_t)nv[min(2 * i + 1, NDT - 1)] << 16 : 0u);
+  f32x4 o[NDT];
+#pragma unroll
+  for (int i = 0; i < NDT; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
   for (int kb = kb_begin; kb < kb_end; ++kb) {
     const int key0 = kb * 64;
     // key operands: tile (u, hh), row fr is key tile_key(u, hh, fr)
@@ -745,6 +742,14 @@ __device__ __forceinline__ void decode_wave(int idx, int kvh, int z, const bf16_
 #pragma unroll
       for (int u = 0; u < 2; ++u)
         o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf[dt][u]), as_bf16x8(pf[u]), o[dt], 0, 0, 0);
+  }
+  if (owner && copy_to >= 0) {
+    const size_t page = ((size_t)(copy_to >> ps_shift) * KVH + kvh) * head_elems;
+    const int off = copy_to & ps_mask;
+    if (lane < NCHUNK) *reinterpret_cast<u32x4*>(k_pages + page + ((size_t)lane * PS + off) * 8) = copy_k;
+#pragma unroll
+    for (int i = 0; i < (HD + 63) / 64; ++i)
+      if (64 * i + lane < HD) v_pages[page + (size_t)(64 * i + lane) * PS + off] = copy_v[i];
   }
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
