@@ -125,32 +125,62 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
     block_first = z * per;
     block_last = min(block_last, block_first + per - 1);
   }
+  // Page ids of a block: of this lane's two groups of 8 keys (32u + 8g .. +7) and of its four operand rows. They are read one block
+  // ahead, behind the block's own loads, and a block's keys and values are asked for together: with the values behind the softmax and a
+  // key's page id ahead of each key, a short context (a block or two a wave) was a chain of round trips (8 tokens of 240 keys, heads of 256 and
+  // 224: 15.0 -> 7.7 us; 32 tokens, heads of 64: 10.4 -> 7.9).
+  // Loads stand under no condition: a branch would wait for everything in flight.
+  int pgv[2], pgk[2][2];
+  auto page_ids = [&](int bi) {
+    const int key0 = lev_block_key(bi, n_kept, first_block);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      pgv[u] = bt[min(key0 + 32 * u + 8 * g, p_max) / PS];
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) pgk[u][hh] = bt[min(key0 + 32 * u + 8 * (col >> 2) + 4 * hh + (col & 3), p_max) / PS];
+    }
+  };
+  page_ids(block_first);
   for (int bi = block_first; bi <= block_last; ++bi) {
     const int key0 = lev_block_key(bi, n_kept, first_block);
-    // pages of this lane's two groups of 8 keys (32u + 8g .. +7): for the mask and for the values
-    int pgv[2];
+    u32x4 kf[2][2][NKS], vf[NVC][NDT][2];
+    int page_of[2];  // of the two groups, -1: none
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        const int kpc = min(key0 + 32 * u + 8 * (col >> 2) + 4 * hh + (col & 3), p_max);  // the key of this lane's operand row
+        const int page = max(pgk[u][hh], 0);  // a key without a page or beyond the range is masked below; its operand may be anything that can be read
+        const bf16_t* kb = k_pages + ((size_t)page * KVH + kvh) * k_head + (size_t)(kpc % PS) * 8;
+#pragma unroll
+        for (int s = 0; s < NKS; ++s) kf[u][hh][s] = *reinterpret_cast<const u32x4*>(kb + (size_t)min(4 * s + g, HD / 8 - 1) * PS * 8);
+      }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int kp = key0 + 32 * u + 8 * g;
-      const int page = bt[min(kp, p_max) / PS];  // loads stand under no condition: a branch would wait for everything in flight
-      pgv[u] = kp <= p_max ? page : -1;
+      page_of[u] = kp <= p_max ? pgv[u] : -1;
+      const bf16_t* vb = v_pages + (size_t)max(page_of[u], 0) * KVH * v_head + (size_t)col * PS + kp % PS;
+#pragma unroll
+      for (int c = 0; c < NVC; ++c)
+        if (c == 0 || c < n_c) {  // the same for the whole wave
+#pragma unroll
+          for (int dt = 0; dt < NDT; ++dt) vf[c][dt][u] = *reinterpret_cast<const u32x4*>(vb + (size_t)(c0 + c) * v_head + (size_t)(16 * dt) * PS);
+        }
     }
+    page_ids(bi + 1);
+    __builtin_amdgcn_sched_barrier(0);  // all of them are on their way before the first is waited for
     // scores: S^T tiles (u, h)
     f32x4 st[2][2];
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) {
-        const int kp = key0 + 32 * u + 8 * (col >> 2) + 4 * hh + (col & 3);  // the key of this lane's operand row
-        const int kpc = min(kp, p_max);
-        const int page = max(bt[kpc / PS], 0);  // a key without a page or beyond the range is masked below; its operand may be anything that can be read
-        const bf16_t* kb = k_pages + ((size_t)page * KVH + kvh) * k_head + (size_t)(kpc % PS) * 8;
         f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s = 0; s < NKS; ++s) {
-          u32x4 kf = u32x4{0u, 0u, 0u, 0u};
-          if (HD % 32 == 0 || 32 * s + 8 * g < HD) kf = *reinterpret_cast<const u32x4*>(kb + (size_t)(4 * s + g) * PS * 8);
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf), as_bf16x8(qf[s]), acc, 0, 0, 0);
+          u32x4 k = kf[u][hh][s];
+          if (HD % 32 != 0 && 4 * s + g >= HD / 8) k = u32x4{0u, 0u, 0u, 0u};
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k), as_bf16x8(qf[s]), acc, 0, 0, 0);
         }
         st[u][hh] = acc;
       }
@@ -163,7 +193,7 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int kp = key0 + 32 * u + 8 * g + 4 * hh + r;
-          const bool ok = valid && lev_key_visible(kp, pos, lo, keep) && pgv[u] >= 0;
+          const bool ok = valid && lev_key_visible(kp, pos, lo, keep) && page_of[u] >= 0;
           float s = st[u][hh][r] * scale;
           if (softcap > 0.f) s = softcap * fast_tanh(s * __builtin_amdgcn_rcpf(softcap));
           s = (s - slope * (float)(pos - kp)) * LOG2E;
@@ -203,10 +233,8 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
 #pragma unroll
           for (int u = 0; u < 2; ++u) {
             const int kp = key0 + 32 * u + 8 * g;
-            const bf16_t* vb = v_pages + ((size_t)max(pgv[u], 0) * KVH + (c0 + c)) * v_head + (size_t)(16 * dt + col) * PS + kp % PS;
-            u32x4 vf = *reinterpret_cast<const u32x4*>(vb);
-            vf = first_keys(vf, pgv[u] >= 0 ? min(8, max(0, p_max - kp + 1)) : 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf), as_bf16x8(pf[u]), acc, 0, 0, 0);
+            const u32x4 v = first_keys(vf[c][dt][u], page_of[u] >= 0 ? min(8, max(0, p_max - kp + 1)) : 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v), as_bf16x8(pf[u]), acc, 0, 0, 0);
           }
           o[c][dt] = acc;
         }
