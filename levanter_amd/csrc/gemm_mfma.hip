@@ -348,12 +348,16 @@ static int launch_tile(const bf16_t* a, long lda, const bf16_t* w, const float* 
 #define SKINNY_MAX_M 256  // which of these row counts it takes: use_skinny()
 
 template <typename TO, int WAVES, int U, int MT, int NT, bool HALF, bool BLOCKS>
-__global__ void __launch_bounds__(WAVES * 64)
+__global__ void __launch_bounds__(WAVES * 64, U == 2 && NT * MT == 4 ? 4 : 1)  // 128 registers: 130 cost 7 % at 2048 x 2048 and 96 rows
 gemm_skinny_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restrict__ w, const float* __restrict__ bias,
                    const float* residual, long ldr, TO* out, long ldo, int M, int N, int K, int act) {
   static_assert(NT * MT <= WAVES * 4 && (!HALF || NT == 1), "a wave finishes a few tiles; half a unit stands alone");
   constexpr int AI = 2 * MT, WI = HALF ? 1 : 2;  // instructions per pair of k-steps and unit: 8 rows each
   constexpr int COLS = HALF ? 8 : 16;
+  // Partial sums of a wave: 16 of them a workgroup, so that none is a longer chain of roundings than with 16 waves (the error against
+  // 64 bits of a 4096-long sum is 1.15e-7 with 16 chains, 1.37e-7 with 8, 1.9e-7 with 4). Not where the registers would cost a workgroup
+  // its place beside another: many rows times many columns.
+  constexpr int SUMS = WAVES >= 16 || NT * MT >= 12 ? 1 : (WAVES == 4 && U >= 2 ? 4 : 2);
   __shared__ f32x4 red[WAVES][NT][MT][64];
   __shared__ u32x4 stage[WAVES][2][SKINNY_SLOTS];
   const int tid = threadIdx.x;
@@ -402,11 +406,13 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restr
     }
   }
 
-  f32x4 acc[NT][MT];
+  f32x4 acc[SUMS][NT][MT];
 #pragma unroll
-  for (int j = 0; j < NT; ++j)
+  for (int s = 0; s < SUMS; ++s)
 #pragma unroll
-    for (int t = 0; t < MT; ++t) acc[j][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) acc[s][j][t] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int npairs = (K + 63) / 64;
   const int rot = (int)((blockIdx.x * 2654435761u) % (unsigned)npairs);
   for (int p0 = wave; p0 < npairs; p0 += WAVES * U) {
@@ -447,8 +453,9 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restr
         const u32x4 a_lo = my_stage[ld_slot], a_hi = my_stage[ld_slot + 4];
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-          acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a_lo), as_bf16x8(wf[j][0]), acc[j][t], 0, 0, 0);
-          acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a_hi), as_bf16x8(wf[j][1]), acc[j][t], 0, 0, 0);
+          f32x4 &lo = acc[2 * u % SUMS][j][t], &hi = acc[(2 * u + 1) % SUMS][j][t];
+          lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a_lo), as_bf16x8(wf[j][0]), lo, 0, 0, 0);
+          hi = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a_hi), as_bf16x8(wf[j][1]), hi, 0, 0, 0);
         }
       }
     }
@@ -456,7 +463,11 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restr
 #pragma unroll
   for (int j = 0; j < NT; ++j)
 #pragma unroll
-    for (int t = 0; t < MT; ++t) red[wave][j][t][lane] = acc[j][t];
+    for (int t = 0; t < MT; ++t) {
+#pragma unroll
+      for (int s = 1; s < SUMS; ++s) acc[0][j][t] += acc[s][j][t];
+      red[wave][j][t][lane] = acc[0][j][t];
+    }
   __syncthreads();
   // 16x16 accumulator: register r of lane l is row 4*(l/16) + r, column l%16. Partial sums are added in wave order.
 #pragma unroll
@@ -646,9 +657,14 @@ gemm_stream_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restr
       wr[set][s] = load16(wrow + (k < K ? k : K - 8));  // beyond K the a fragment is zero, whatever this holds
     }
   };
-  f32x4 acc[MT];
+  // up to 32 rows four sums in turn (a k-step's, of even and of odd chunks): a short chain of roundings each, as the skinny kernel's; more
+  // rows have no registers for that
+  constexpr int SUMS = MT <= 2 ? 4 : 1;
+  f32x4 acc[SUMS][MT];
 #pragma unroll
-  for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < SUMS; ++s)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[s][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   if (c_begin < c_end) {
     load_x(0, c_begin);
@@ -670,7 +686,8 @@ gemm_stream_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restr
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
           const u32x4 af = *reinterpret_cast<const u32x4*>(xb + t * 16 * SK_LDS_STRIDE + s * 32);
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(af), as_bf16x8(wr[set][s]), acc[t], 0, 0, 0);
+          f32x4& sum = acc[(set * KS + s) % SUMS][t];
+          sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(af), as_bf16x8(wr[set][s]), sum, 0, 0, 0);
         }
       // the weight registers are refilled behind the products that read them: refilled ahead of them (from a copy),
       // the new values landed in other registers and were moved into place at the end of the loop, which waits for
@@ -689,6 +706,10 @@ gemm_stream_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restr
     }
     if (c < c_end) chunk(c, 0);
   }
+#pragma unroll
+  for (int s = 1; s < SUMS; ++s)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[0][t] += acc[s][t];
   // 16x16 accumulator: register r of lane l is row 4*(l/16) + r, column l%16
   if (n < N) {
 #pragma unroll
@@ -698,9 +719,9 @@ gemm_stream_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restr
         const int m = t * 16 + (lane >> 4) * 4 + r;
         if (m < M) {
           if (S == 1)
-            epilogue_store<TO>(acc[t][r], m, n, bias, residual, ldr, out, ldo, act);
+            epilogue_store<TO>(acc[0][t][r], m, n, bias, residual, ldr, out, ldo, act);
           else
-            partial[((size_t)split * M + m) * N + n] = acc[t][r];
+            partial[((size_t)split * M + m) * N + n] = acc[0][t][r];
         }
       }
   }

@@ -361,9 +361,9 @@ moe_linear_few_kernel(const MoeLinearArgs p) {
   }
   moe_u32x4* mine = stage[wave];
   const int st = lr * 9 + lc, ld = (col >> 3) * MOE_SLOTS + (col & 7) * 9 + g;
-  moe_f32x4 acc[G];
+  moe_f32x4 acc[G], acc_hi[G];  // a pair's first and second k-steps: 8 or 16 partial sums a workgroup, so that none is a long chain of roundings
 #pragma unroll
-  for (int x = 0; x < G; ++x) acc[x] = moe_f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int x = 0; x < G; ++x) acc[x] = acc_hi[x] = moe_f32x4{0.f, 0.f, 0.f, 0.f};
   const int pairs = (K + 63) / 64;
   for (int p0 = wave; p0 < pairs; p0 += KS * U) {
     moe_u32x4 av[U][2], wv[U][G][2];
@@ -390,12 +390,12 @@ moe_linear_few_kernel(const MoeLinearArgs p) {
         mine[st] = wv[u][x][0] & mk, mine[MOE_SLOTS + st] = wv[u][x][1] & mk;
         const moe_u32x4 w_lo = mine[ld], w_hi = mine[ld + 4];
         acc[x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(moe_as_bf16x8(w_lo), moe_as_bf16x8(a_lo), acc[x], 0, 0, 0);
-        acc[x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(moe_as_bf16x8(w_hi), moe_as_bf16x8(a_hi), acc[x], 0, 0, 0);
+        acc_hi[x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(moe_as_bf16x8(w_hi), moe_as_bf16x8(a_hi), acc_hi[x], 0, 0, 0);
       }
     }
   }
 #pragma unroll
-  for (int x = 0; x < G; ++x) part[wave][x][lane] = acc[x];
+  for (int x = 0; x < G; ++x) part[wave][x][lane] = acc[x] += acc_hi[x];
   __syncthreads();
   const int o = o0 + 4 * g;
   if (wave != 0 || col >= rows || o >= F) return;

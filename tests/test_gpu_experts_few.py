@@ -46,3 +46,20 @@ def test_products_over_tiles_of_16_rows_against_float64(K, F, Kd):
                     bound = err + 1e-30 + (2.0 ** -8 * (y.abs() + err) if dtype is torch.bfloat16 else 0)
                     assert bool(((out[:, :F].double() - y).abs() <= bound).all()), (glu, gather, dtype, width)
                     assert bool(torch.isnan(out[:, F:]).all())
+
+
+@pytest.mark.parametrize("Kd,sums", [(1024, 8), (2048, 16)])
+def test_the_sums_chains_of_roundings_stay_short(K, Kd, sums):
+    """The error in root mean square of Kd products in ``sums`` partial sums, derived as in the test of the same name in test_gpu_skinny.py."""
+    g = torch.Generator(device=DEV).manual_seed(Kd)
+    T, E, F = 8, 4, 1024
+    chosen = (torch.arange(T) % E).to(torch.int32).to(DEV).unsqueeze(1)
+    h, w = torch.randn(T, Kd, device=DEV, generator=g).bfloat16(), torch.randn(E, F, Kd, device=DEV, generator=g).bfloat16()
+    tables = torch.empty(2 * T + 1 + 3 * K.moe_max_tiles(T, E, 16), dtype=torch.int32, device=DEV)
+    sp, po, meta, tiles = tables[:T], tables[T:2 * T], tables[2 * T:2 * T + 1], tables[2 * T + 1:]
+    K.moe_sort(chosen, E, sp, po, tiles, meta, tile_rows=16)
+    out = torch.empty(T, F, device=DEV)
+    K.moe_linear(h, w, out, tiles, meta, sp, top=1, gather=True, tile_rows=16)
+    want = torch.stack([w[t % E].double() @ h[t].double() for t in sp.tolist()])
+    error, n = float((out.double() - want).norm() / want.norm()), Kd / 32 / sums
+    assert error <= 1.06 * 0.40 * 2.0 ** -24 * ((4 * n + 1) / 2 + (sums + 1) / 2) ** 0.5, error

@@ -65,3 +65,21 @@ def test_linear_in_row_blocks_against_float64(K, N, Ki, monkeypatch):
         K.linear(a, w, bias, out[:M, :N], residual=res)
         assert bool(((out[:M, :N].double() - want).abs() <= (Ki + 4) * 2.0 ** -24 * size).all()), M
         assert bool(torch.isnan(out[:M, N:]).all()) and bool(torch.isnan(out[M]).all())
+
+
+@pytest.mark.parametrize("M,N,Ki,sums", [(8, 768, 3072, 16), (8, 4096, 4096, 16), (48, 4096, 4096, 16), (16, 2048, 8192, 16), (8, 6144, 6144, 16), (8, 4096, 16384, 16),
+                                         (16, 12288, 4096, 16), (16, 50257, 768, 4), (16, 32000, 2048, 4)])
+def test_the_sums_chains_of_roundings_stay_short(K, M, N, Ki, sums, monkeypatch):
+    """Ki products in ``sums`` partial sums of n = Ki / 32 / sums instructions each, whose 32 products are added in four groups; the partial sums are then added in a
+    row. After i of n equal steps a sum of random terms has i / n of its final variance, and each addition is off by 0.40 * 2^-24 of its result in root mean square
+    (rounding to nearest, mantissas spread over their logarithm), so that the whole is off by that times sqrt((4 n + 1) / 2 + (sums + 1) / 2); 6 % more for
+    the scatter over the outputs. Half as many sums would be 18 to 40 % above."""
+    monkeypatch.setattr(K, "gemm_library", False)
+    g = torch.Generator(device=DEV).manual_seed(N + Ki)
+    a, w = torch.randn(M, Ki, device=DEV, generator=g).bfloat16(), torch.randn(N, Ki, device=DEV, generator=g).bfloat16()
+    out = torch.empty(M, N, device=DEV)
+    K.linear(a, w, None, out)
+    want = a.double() @ w.double().T
+    error = float((out.double() - want).norm() / want.norm())
+    n = Ki / 32 / sums
+    assert error <= 1.06 * 0.40 * 2.0 ** -24 * ((4 * n + 1) / 2 + (sums + 1) / 2) ** 0.5, error
