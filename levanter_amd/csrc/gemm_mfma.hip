@@ -13,6 +13,7 @@
 // No atomics anywhere: results are deterministic. K and lda must be multiples of 8 (16-byte operand loads);
 // any M and N.
 #include "common.h"
+#include <type_traits>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -348,7 +349,9 @@ static int launch_tile(const bf16_t* a, long lda, const bf16_t* w, const float* 
 #define SKINNY_MAX_M 256  // which of these row counts it takes: use_skinny()
 
 template <typename TO, int WAVES, int U, int MT, int NT, bool HALF, bool BLOCKS>
-__global__ void __launch_bounds__(WAVES * 64, U == 2 && NT * MT == 4 ? 4 : 1)  // 128 registers: 130 cost 7 % at 2048 x 2048 and 96 rows
+// at most 128 registers a lane for 2 x 2 tiles (130 cost 7 % at 2048 x 2048 and 96 rows); with four waves at most 256, so that the sums stay in
+// registers that every instruction reads (where 512 are allowed the compiler moves them to and fro: 16384 x 4096 at 64 rows 34.2 us)
+__global__ void __launch_bounds__(WAVES * 64, U == 2 && NT * MT == 4 ? 4 : WAVES == 4 ? 2 : 1)
 gemm_skinny_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restrict__ w, const float* __restrict__ bias,
                    const float* residual, long ldr, TO* out, long ldo, int M, int N, int K, int act) {
   static_assert(NT * MT <= WAVES * 4 && (!HALF || NT == 1), "a wave finishes a few tiles; half a unit stands alone");
@@ -415,11 +418,12 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restr
       for (int t = 0; t < MT; ++t) acc[s][j][t] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int npairs = (K + 63) / 64;
   const int rot = (int)((blockIdx.x * 2654435761u) % (unsigned)npairs);
-  for (int p0 = wave; p0 < npairs; p0 += WAVES * U) {
-    u32x4 wv[U][NT][WI], av[U][AI];
-    uint32_t keep[U];
+  auto take = [&](auto pairs, int p0) {
+    constexpr int UU = decltype(pairs)::value;
+    u32x4 wv[UU][NT][WI], av[UU][AI];
+    uint32_t keep[UU];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (int u = 0; u < UU; ++u) {
       int pr = p0 + u * WAVES;
       const bool p_ok = pr < npairs;
       pr = min(pr, npairs - 1) + rot;
@@ -435,7 +439,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restr
     }
     __builtin_amdgcn_sched_barrier(0);  // all of them are on their way before the first is waited for
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (int u = 0; u < UU; ++u) {
       // LDS executes a wave's instructions in order: the area is used again and again without a barrier
       const u32x4 mk = u32x4{keep[u], keep[u], keep[u], keep[u]};
       u32x4 wf[NT][2];
@@ -459,6 +463,19 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restr
         }
       }
     }
+  };
+  // U pairs at a time; of the few that are left a half or a quarter as many, so that short sums do not read their last pairs twice or more
+  // (34768 x 320 at 13 rows 10.7 -> 7.9 us, 55128 x 576 at one row 15.6 -> 13.5)
+  int p0 = U > 1 ? __builtin_amdgcn_readfirstlane(wave) : wave;
+  for (; p0 + WAVES * (U / 2) < npairs; p0 += WAVES * U) take(std::integral_constant<int, U>(), p0);
+  if constexpr (U == 4) {
+    if (p0 + WAVES < npairs) {
+      take(std::integral_constant<int, 2>(), p0);
+      p0 = npairs;
+    }
+  }
+  if constexpr (U > 1) {
+    if (p0 < npairs) take(std::integral_constant<int, 1>(), p0);
   }
 #pragma unroll
   for (int j = 0; j < NT; ++j)
@@ -532,7 +549,9 @@ static SkinnyShape skinny_shape(int M, int N, int K) {
     if (N <= 2048) return K > 4096 && M <= 8 ? SkinnyShape{16, 2, 1, 1, true} : SkinnyShape{8, 2, 1, 1, true};
     if (tiles <= 256) return {8, 2, 1, 1, false};
     if (tiles <= 512) return K < 1792 ? SkinnyShape{16, 1, 1, 2, false} : SkinnyShape{8, 2, 1, 2, false};
-    return tiles <= 720 ? SkinnyShape{16, 1, 1, 3, false} : SkinnyShape{4, 4, 1, 1, false};
+    if (tiles <= 720) return {16, 1, 1, 3, false};
+    if (K <= 256 && tiles >= 1024) return {4, 1, 1, 2, false};  // a pair a wave at most: two units share `a`
+    return {4, 4, 1, 1, false};
   }
   if (M <= 32) {
     if (N <= 2048) return {8, 2, 2, 1, true};
@@ -573,6 +592,7 @@ static void launch_skinny(const bf16_t* a, long lda, const bf16_t* w, const floa
   LEV_SKINNY(8, 2, 1, 2, false);
   LEV_SKINNY(16, 1, 1, 3, false);
   LEV_SKINNY(4, 4, 1, 1, false);
+  LEV_SKINNY(4, 1, 1, 2, false);
   LEV_SKINNY(8, 2, 2, 1, true);
   LEV_SKINNY(8, 2, 2, 1, false);
   LEV_SKINNY(8, 2, 2, 2, false);
@@ -600,7 +620,7 @@ static void launch_skinny(const bf16_t* a, long lda, const bf16_t* w, const floa
 #define SK_LDS_STRIDE (SK_CHUNK + 8)
 
 template <typename TO, int MT, int NW>
-__global__ void __launch_bounds__(NW * 64)
+__global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1)
 gemm_stream_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restrict__ w, const float* __restrict__ bias,
                    const float* residual, long ldr, TO* out, long ldo, float* __restrict__ partial, int M, int N, int K, int act,
                    int S) {

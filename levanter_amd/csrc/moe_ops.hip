@@ -342,7 +342,7 @@ __device__ __forceinline__ void moe_store4<bf16_t>(bf16_t* p, const float (&v)[4
 // enough: 1024 x 1024, 8 tokens 11.4 against 12.2 of eight, 768 to 2,048, 32 tokens 62 / 80; at 2,048 eight are: 1 token 12.6 / 13.8.
 #define MOE_SLOTS 72  // 16-byte slots of one staged instruction: 8 rows x (8 chunks + 1 of padding)
 template <typename TO, bool GLU, int KS, int U>
-__global__ void __launch_bounds__(64 * KS)
+__global__ void __launch_bounds__(64 * KS, KS == 4 ? 2 : 1)
 moe_linear_few_kernel(const MoeLinearArgs p) {
   constexpr int G = GLU ? 2 : 1;
   __shared__ moe_f32x4 part[KS][G][64];

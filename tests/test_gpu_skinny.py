@@ -83,3 +83,26 @@ def test_the_sums_chains_of_roundings_stay_short(K, M, N, Ki, sums, monkeypatch)
     error = float((out.double() - want).norm() / want.norm())
     n = Ki / 32 / sums
     assert error <= 1.06 * 0.40 * 2.0 ** -24 * ((4 * n + 1) / 2 + (sums + 1) / 2) ** 0.5, error
+
+
+@pytest.mark.parametrize("N", [40, 2500, 9000, 11536, 16400])
+@pytest.mark.parametrize("pairs", [1, 2, 3, 4, 5, 6, 8, 9, 11, 12, 13, 17, 19, 33])
+def test_linear_skinny_with_few_pairs_left(K, N, pairs, monkeypatch):
+    """What is left of a sum behind the whole rounds of a workgroup's waves, for every number of it; every product once: ones give whole numbers, exactly."""
+    gemm = K._unit("gemm_mfma")
+    monkeypatch.setattr(K, "gemm_library", False)
+    try:
+        K._check(gemm.lev_linear_mfma_force(1))
+        K._ws_need.clear()
+        for Ki in (64 * pairs, 64 * pairs - 24):
+            w = torch.ones(N, Ki, device=DEV, dtype=torch.bfloat16)
+            w[:, Ki // 2] = 3.0
+            for M in (1, 16, 17, 33, 64):
+                a = torch.ones(M, Ki, device=DEV, dtype=torch.bfloat16)
+                a[:, -1] = 5.0
+                out = torch.full((M, N), float("nan"), device=DEV)
+                K.linear(a, w, None, out)
+                assert bool((out == (a[0].double() @ w[0].double()).item()).all()), (Ki, M)
+    finally:
+        K._check(gemm.lev_linear_mfma_force(0))
+        K._ws_need.clear()
