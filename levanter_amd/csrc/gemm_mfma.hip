@@ -910,21 +910,27 @@ static TilePlan plan_tiles(int M, int N, int K) {
 
 // Which kernel takes M <= 64 rows (above: skinny_in_blocks). An estimate of the skinny kernel in microseconds: a launch and its ramp, and
 // the longest of the weights' read from memory, the share of it that falls to the busiest CU, and what that CU pulls through its caches
-// (its columns and most of `a`, for each of its workgroups). The stream kernel's time hardly grows with the rows, but it pays for its K
-// ranges: plan_stream's cost is about 0.8 of what it takes with the kernel that adds them (which the next norm may do in passing: 1.18).
-// The constants are fitted to 154 cases (22 weights of 2 to 400 MB at 1, 8, 16, 24, 32, 48 and 64 rows): 7 % off the measured time on
-// average, and the choice on average within 1 % of the better kernel. Measured, skinny / stream: 16384 x 4096 at 8 / 64 rows 24.5 / 33.2,
-// 31.9 / 37.4; 4096 x 16384 at 8 / 32 / 64 rows 24.2 / 32.7, 31.3 / 33.9, 43.9 / 36.4; 1600 x 6400 at 16 / 24 / 32 / 64 rows 9.2 / 11.1, 11.0 / 11.4,
-// 12.3 / 11.6, 19.0 / 13.4; 6144 x 24576 at 8 / 24 rows 57.6 / 59.7, 67.1 / 61.0; 24576 x 6144 at 8 / 64 rows 53.0 / 59.1, 77.1 / 67.8.
+// (its columns and most of `a`, for each of its workgroups: the rate depends on how much of that is waited for at once). The stream
+// kernel's time hardly grows with the rows, but it pays for its K ranges: plan_stream's cost and a launch; unsplit, its workgroups all
+// start at their rows' beginnings, and rows a multiple of 4 KB apart (K = 2,048 n) then meet on the same memory channels.
+// The constants are those that choose best over 2,400 cases (weights of 0.15 M to 206 M numbers, sums of 64 to 24,576, 1 to 64 rows; 400 weights
+// drawn, 32 of layers), under the condition that weights of 17 MB and more at 64 rows, which the norm behind them adds up, stay split. The choice
+// is 0.3 % behind the better kernel on average, and more than 5 % at 2 % of the cases; the estimate of the one that is chosen is 15 % off on average. The
+// fit before it, to 154 cases of layers, took no account of the stream kernel's own launch and of long sums of few outputs and was 3.2 %
+// behind: 65024 x 2048 at 25 rows 73 us (stream) for 53, 464 x 16384 at 22 rows 17.2 (skinny) for 12.0, 3118 x 128 at 64 rows 7.0 (stream)
+// for 3.7. Measured, skinny / stream: 16384 x 4096 at 8 / 64 rows 24.9 / 32.6, 30.6 / 37.6; 4096 x 16384 at 8 / 24 / 64 rows 24.5 / 33.0,
+// 28.9 / 34.1, 44.8 / 36.7; 1600 x 6400 at 16 / 64 rows 9.2 / 11.5, 19.4 / 13.6; 6144 x 24576 at 4 / 24 rows 55.4 / 60.0, 68.1 / 61.2.
 static double skinny_estimate(int M, int N, int K) {
   const SkinnyShape sh = skinny_shape(M, N, K);
   const long wgs = (N + sh.cols() - 1) / sh.cols(), r = (wgs + 255) / 256;  // r: workgroups of the busiest CU
-  const double memory = 2.0 * N * K / 6.27e6, own = r * (double)sh.cols() * K * 2.0 / 42e3;
-  const double rate = (long)N * K <= (1L << 23) ? 79e3 : sh.waves == 4 ? 39e3 : sh.units > 1 ? 37e3 : 48e3;  // small weights stay in the caches' reach
-  const double caches = r * (sh.cols() + 0.85 * M) * K * 2.0 / rate;
+  const double memory = 2.0 * N * K / 7.3e6, own = r * (double)sh.cols() * K * 2.0 / 34e3;
+  double rate = (long)N * K <= (1L << 23) ? 66e3 : sh.waves == 4 ? 34.7e3 : sh.units > 1 ? 45e3 : 39e3;  // small weights stay in the caches' reach
+  const double most = sh.units > 1 ? 34e3 : 38.4e3;
+  if (K >= 8192 && rate > most) rate = most;  // long sums: a chain of round trips a workgroup
+  const double caches = r * (sh.cols() + (M > 32 ? 0.93 : 0.74) * M) * K * 2.0 / rate;
   double cost = memory > own ? memory : own;
   if (caches > cost) cost = caches;
-  return 3.26 + cost + (sh.row_tiles > 1 && r > 4 ? 1.1 * (r - 1) : 0.0);
+  return 2.4 + cost + (sh.row_tiles > 1 ? 0.75 * (r - 1) : 0.0);
 }
 // 0: the estimate decides; 1 / 2: the skinny / the stream kernel wherever it takes the row count. For measurements of the
 // choice itself (a test times both candidates at widths the estimates were not fitted to); not used by the engine.
@@ -937,7 +943,8 @@ extern "C" int lev_linear_mfma_force(int kind) {
 static bool use_skinny(int M, int N, int K) {
   if (M > 64) return skinny_in_blocks(M, N, K) && g_force_kernel != 2;
   if (g_force_kernel) return g_force_kernel == 1;
-  return skinny_estimate(M, N, K) <= 1.18 * plan_stream(M, N, K).cost;
+  const StreamPlan plan = plan_stream(M, N, K);
+  return skinny_estimate(M, N, K) <= 2.3 + 1.17 * plan.cost * (plan.splits == 1 && K % 2048 == 0 ? 1.2 : 1.0);
 }
 
 // Into how many ranges the sum over K is split (1: the kernel finishes its outputs itself).

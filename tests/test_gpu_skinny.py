@@ -106,3 +106,34 @@ def test_linear_skinny_with_few_pairs_left(K, N, pairs, monkeypatch):
     finally:
         K._check(gemm.lev_linear_mfma_force(0))
         K._ws_need.clear()
+
+
+# Beyond the layers that the estimate was once fitted to: heads of some 50,000 outputs at a few and at 32 rows, long sums of a few hundred outputs, short sums
+CHOICES = [(2, 59904, 1024), (25, 65024, 2048), (32, 50256, 2048), (22, 464, 16384), (25, 304, 11264), (9, 656, 16384), (58, 9696, 12992), (64, 3112, 128), (5, 1600, 256),
+           (21, 6080, 256), (13, 50768, 256), (64, 34968, 1216)]
+
+
+def test_the_choice_between_the_two_kernels_is_within_a_quarter_of_the_better_one(K):
+    from test_gpu_kernels import _time_products
+
+    gemm = K._unit("gemm_mfma")
+
+    def timed(M, N, Ki, reps):
+        weights = [torch.randn(N, Ki, device=DEV).bfloat16() for _ in range(max(3, min(12, int(6e8 / (N * Ki * 2)))))]
+        a, bias, out = torch.randn(M, Ki, device=DEV).bfloat16(), torch.randn(N, device=DEV), torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+        times = []
+        for kind in (0, 1, 2):
+            K._check(gemm.lev_linear_mfma_force(kind))
+            K._ws_need.clear()
+            times.append(_time_products(lambda w: K.linear(a, w, bias, out), weights, reps=reps))
+        return times
+
+    was, K.gemm_library = K.gemm_library, False
+    try:
+        report = [(c, timed(*c, 5)) for c in CHOICES]
+        report = [(c, timed(*c, 15) if t[0] > 1.25 * min(t[1:]) else t) for c, t in report]  # over the line: once more, longer, before it counts
+    finally:
+        K.gemm_library = was
+        K._check(gemm.lev_linear_mfma_force(0))
+        K._ws_need.clear()
+    assert not [x for x in report if x[1][0] > 1.25 * min(x[1][1:])], report
