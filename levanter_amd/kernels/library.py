@@ -439,17 +439,14 @@ class HipKernels:
         ahead on MI355X (widths of GPT-2 7B and XL, with epilogues). From 256 rows: all but long sums into narrow outputs
         (K >= 4 N) below 1,024 rows and, below 320 rows, weights of a few MB unless the output is wide (a 1600-wide layer at 264
         rows, ours / library with its kernel timed: qkv 18.3 / 16.7, fc 24.8 / 18.8, proj 11.9 / 14.2, second MLP matrix 22.7 / 20.4 but
-        20.1 / 23.5 at 256 and 22.9 / 23.5 at 288). Up to 64 rows: the heads of narrow models (more than 16,384 outputs of sums below 2,048:
-        50257 x 1600 at 32 rows 35.5 / 31.8 us, 50257 x 768 22.9 / 19.0; but 32000 x 2048 28.3 / 33.0) and above 32 rows weights of 67 M to
-        134 M numbers (18432 x 6144 at 48 / 64 rows 57.3 / 54.0, 64.0 / 55.2); everything else is ours (12288 x 4096 at 32 / 64 rows 21.2 / 22.7
-        and 25.7 / 24.8, 16384 x 4096 26.3 / 33.5 and 31.6 / 33.0, 10752 x 2048 10.8 / 14.6 and 14.4 / 15.8). From 65 to 255 rows: wide outputs of large
+        20.1 / 23.5 at 256 and 22.9 / 23.5 at 288). Up to 64 rows see ``_library_reads_weights_faster``. From 65 to 255 rows: wide outputs of large
         weights (N >= 2 K, 32 MB and more: at 160 rows qkv and fc of a 4096-wide layer 49.7 / 37.2 and 55.7 / 41.6); ours keep N = K (22.1 /
         24.6 at 128) and K = 4 N (43.5 / 81.1), and below 96 rows the largest weights (more than 256 MB). Up to 256 rows our kernel
         of row blocks keeps short sums (K to 2,048) whose blocks of 64 x 64 make one round of the CUs (4800 x 1600 at 96 / 192 rows 9.6 / 12.7, 10.3 / 16.8)."""
         if act not in cls.LIBRARY_ACTIVATIONS or M < cls.LIBRARY_MIN_ROWS:
             return False
         if M <= 64:
-            return (N > 16384 and K < 2048) or (M > 32 and N >= 2 * K and (1 << 26) < N * K <= (1 << 27))
+            return cls._library_reads_weights_faster(M, N, K)
         if M <= 256 and K <= 2048 and -(-M // 64) * (-(-N // 512) * 8) <= 256:
             return False
         if M < 256:
@@ -461,6 +458,30 @@ class HipKernels:
         if M < 320 and N * K < (1 << 24):
             return N >= 2 * K
         return not (K >= 4 * N and M < 1024)
+
+    @staticmethod
+    def _library_reads_weights_faster(M: int, N: int, K: int) -> bool:
+        """25 to 64 rows, where a product is the read of its weights: which of them the library's kernel reads faster. It has tiles of up to
+        256 outputs, which make one round of the CUs, a fifth full or more, from 12,000 to 65,536 outputs (fewer: ours ahead by 4 - 40 %; more: by
+        up to 3 times); its rates suggest that it starts every row at its beginning: rows 4 KB or a multiple of that apart (K a multiple of 2,048), which then meet on the
+        same memory channels, it reads at 4.4 - 5 TB/s instead of 5.5 - 6; and it is slow on rows that are no whole number of 256 bytes (K % 128: 14896 x 4544 at 32 / 64
+        rows ours 28.3 / 33.4 us, library 36.8 / 41.9; 14480 x 4608 28.3 / 33.8, 26.1 / 29.5), unless its 256-wide tiles alone fill half of the CUs
+        (50257 x 1600 at 32 / 64 rows ours 35.4 / 40.6, library 32.2 / 34.6). Ours start at another place in every workgroup and read at 5 to 6
+        TB/s up to 32 rows whatever K; above, more rows share a line's look-ups (4 - 5 TB/s), and from K = 2,048 n only an uneven last round of
+        workgroups of 64 outputs, less than four fifths of all full, lets the library ahead (22528 x 4096 at 64 rows 51.9 / 44.7, but 16384 x 4096
+        30.6 / 32.8 and 32768 x 4096 55.4 / 60.5). Short sums are ours up to 32 rows (24000 x 1024 12.6 / 31.3) but for wide outputs.
+        Weights of less than 2^24 and more than 2^27 numbers are ours whatever is faster (the library's lead there is 6 % on average): it adds a sum up in
+        one chain (off from 64 bits by 4.0e-7 at K = 4,096, ours by 1.1e-7).
+        Over 1,007 cases (176 weights of 17 to 270 M numbers, biased bfloat16 and plain float32 outputs) the choice is on average 0.9 % behind the
+        better of the two; ours everywhere 5.0 %, the library everywhere 9.3 %."""
+        if N < 2 * K or K < 768 or not 12000 <= N <= 65536 or not (1 << 24) <= N * K <= (1 << 27):
+            return False
+        if M <= 32:
+            return N > 36000 if K < 2048 else K % 128 == 0 and K % 2048 != 0
+        if K % 2048 == 0:
+            groups = -(-N // 64)
+            return N > 16384 and groups < 0.8 * 256 * -(-groups // 256)
+        return N > 32768 or (K % 128 == 0 and (K >= 1280 or N < 25600))
 
     # ---- cache write -----------------------------------------------------------------------
     def kv_write(self, k, v, k_pages, v_pages, dest, n_kv_heads: int, head_dim: int, page_size: int, value_dim: Optional[int] = None) -> None:
