@@ -59,7 +59,10 @@ __device__ __forceinline__ float fast_tanh(float x) {  // 1 - 2 / (1 + e^(2x)) w
   return 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * 2.8853900817779268f));
 }
 
-template <bool SINGLE>
+// NC: value heads that a wave has room for (1, or a power of two up to NVC). The operands of all of them are on their way together, so room
+// for more than there are costs registers and a launch that is 0.3 - 0.5 us longer (16 x 16 heads of 64 / 64, 8 tokens of 60 keys 5.1 us, 5.6 with
+// room for four; 16 x 4 of 64 / 32 with all 4 value heads 6.2 us, 6.6 with room for eight).
+template <bool SINGLE, int NC>
 __global__ void __launch_bounds__(64)
 attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float* __restrict__ out, const bf16_t* __restrict__ k_pages,
                              const bf16_t* __restrict__ v_pages, const int* __restrict__ positions, const int* __restrict__ token_seq,
@@ -97,8 +100,8 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
   }
   const int* bt = block_tables + (size_t)token_seq[tok] * bt_stride;
   const float slope = slopes ? slopes[head] : 0.f;
-  const int c0 = NV == 1 ? kvh : blockIdx.z * NVC;             // first value head of this wave
-  const int n_c = NV == 1 ? 1 : min(NVC, NV - blockIdx.z * NVC);  // and how many
+  const int c0 = NV == 1 ? kvh : blockIdx.z * NC;              // first value head of this wave
+  const int n_c = NV == 1 ? 1 : min(NC, NV - blockIdx.z * NC);  // and how many
 
   u32x4 qf[NKS];
 #pragma unroll
@@ -107,9 +110,9 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
     if (valid && 32 * s + 8 * g < HD)
       qf[s] = *reinterpret_cast<const u32x4*>(q + (size_t)tok * q_stride + (size_t)head * HD + 32 * s + 8 * g);
   }
-  f32x4 o[NVC][NDT];
+  f32x4 o[NC][NDT];
 #pragma unroll
-  for (int c = 0; c < NVC; ++c)
+  for (int c = 0; c < NC; ++c)
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) o[c][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
@@ -143,7 +146,7 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
   page_ids(block_first);
   for (int bi = block_first; bi <= block_last; ++bi) {
     const int key0 = lev_block_key(bi, n_kept, first_block);
-    u32x4 kf[2][2][NKS], vf[NVC][NDT][2];
+    u32x4 kf[2][2][NKS], vf[NC][NDT][2];
     int page_of[2];  // of the two groups, -1: none
 #pragma unroll
     for (int u = 0; u < 2; ++u)
@@ -161,7 +164,7 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
       page_of[u] = kp <= p_max ? pgv[u] : -1;
       const bf16_t* vb = v_pages + (size_t)max(page_of[u], 0) * KVH * v_head + (size_t)col * PS + kp % PS;
 #pragma unroll
-      for (int c = 0; c < NVC; ++c)
+      for (int c = 0; c < NC; ++c)
         if (c == 0 || c < n_c) {  // the same for the whole wave
 #pragma unroll
           for (int dt = 0; dt < NDT; ++dt) vf[c][dt][u] = *reinterpret_cast<const u32x4*>(vb + (size_t)(c0 + c) * v_head + (size_t)(16 * dt) * PS);
@@ -225,7 +228,7 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
     l = l * corr + psum;
     // values of every value head of this wave
 #pragma unroll
-    for (int c = 0; c < NVC; ++c) {
+    for (int c = 0; c < NC; ++c) {
       if (c < n_c) {
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt) {
@@ -251,7 +254,7 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
       part_ml[2 * slot + 1] = l;
     }
 #pragma unroll
-    for (int c = 0; c < NVC; ++c) {
+    for (int c = 0; c < NC; ++c) {
       if (c < n_c) {
         float* ob = part_o + (slot * NV + (NV == 1 ? 0 : c0 + c)) * VD;
 #pragma unroll
@@ -263,7 +266,7 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
   if (sinks != nullptr) l = m == -INFINITY ? 1.0f : l + __builtin_amdgcn_exp2f(sinks[head] * LOG2E - m);  // m is in base 2
   const float inv = l > 0.f ? 1.0f / l : 0.f;
 #pragma unroll
-  for (int c = 0; c < NVC; ++c) {
+  for (int c = 0; c < NC; ++c) {
     if (c < n_c) {
       float* ob = out + (((size_t)tok * H + head) * NV + (NV == 1 ? 0 : c0 + c)) * VD;
 #pragma unroll
@@ -545,7 +548,22 @@ extern "C" int lev_attention_values_mfma(const void* q, long q_stride, float* ou
                   ((uintptr_t)out & 15) == 0,
               "attention: operands must be 16-byte aligned");
   const int chunks = NV == 1 ? 1 : (NV + NVC - 1) / NVC;
+  int room = 1;  // value heads of a wave of the kernels without shared operands
+  while (room < NV && room < NVC) room *= 2;
   LEV_REQUIRE(H <= 65535 && chunks <= 65535, "attention: too many heads (%d)", H);
+#define AV_ROOM(SINGLE, NC, GRID, WORK, SPLITS, PART_O, PART_ML)                                                                                    \
+  if constexpr (NC <= NVC)                                                                                                                          \
+    if (room == NC)                                                                                                                                 \
+      attention_values_mfma_kernel<SINGLE, NC><<<GRID, 64, 0, stream>>>((const bf16_t*)q, q_stride, out, (const bf16_t*)k_pages,                   \
+                                                                        (const bf16_t*)v_pages, positions, token_seq, block_tables, bt_stride, WORK, \
+                                                                        H, KVH, NV, PS, scale, window, chunk, keep, softcap, slopes, SPLITS, PART_O, PART_ML, sinks)
+#define AV_ROOMS(SINGLE, GRID, WORK, SPLITS, PART_O, PART_ML)   \
+  do {                                                          \
+    AV_ROOM(SINGLE, 1, GRID, WORK, SPLITS, PART_O, PART_ML);    \
+    AV_ROOM(SINGLE, 2, GRID, WORK, SPLITS, PART_O, PART_ML);    \
+    AV_ROOM(SINGLE, 4, GRID, WORK, SPLITS, PART_O, PART_ML);    \
+    AV_ROOM(SINGLE, 8, GRID, WORK, SPLITS, PART_O, PART_ML);    \
+  } while (0)
   if (n_tiles > 0) {
     dim3 grid(n_tiles, H, chunks);
     const size_t lds = ((size_t)HD * 64 + (size_t)(NV == 1 ? 1 : (NV < NVC ? NV : NVC)) * VD * VS_STRIDE) * sizeof(bf16_t);
@@ -563,9 +581,7 @@ extern "C" int lev_attention_values_mfma(const void* q, long q_stride, float* ou
                                                                          (const bf16_t*)v_pages, positions, token_seq, block_tables,
                                                                          bt_stride, tiles, H, KVH, NV, PS, scale, window, chunk, keep, softcap, slopes, sinks);
     else  // the longest ranges: every wave by itself, operands straight from the pages
-      attention_values_mfma_kernel<false><<<dim3(n_tiles * SUB_TILES, H, chunks), 64, 0, stream>>>(
-          (const bf16_t*)q, q_stride, out, (const bf16_t*)k_pages, (const bf16_t*)v_pages, positions, token_seq, block_tables, bt_stride,
-          tiles, H, KVH, NV, PS, scale, window, chunk, keep, softcap, slopes, 1, nullptr, nullptr, sinks);
+      AV_ROOMS(false, dim3(n_tiles * SUB_TILES, H, chunks), tiles, 1, nullptr, nullptr);
     if (lev_check_launch("attention_values_mfma (runs)")) return -1;
   }
   if (n_singles > 0) {
@@ -573,10 +589,9 @@ extern "C" int lev_attention_values_mfma(const void* q, long q_stride, float* ou
     dim3 grid(n_singles * splits, KVH * ((group + 15) / 16), chunks);
     float* part_o = workspace;
     float* part_ml = splits > 1 ? workspace + (size_t)n_singles * splits * H * NV * VD : nullptr;
-    attention_values_mfma_kernel<true><<<grid, 64, 0, stream>>>((const bf16_t*)q, q_stride, out, (const bf16_t*)k_pages,
-                                                               (const bf16_t*)v_pages, positions, token_seq, block_tables, bt_stride,
-                                                               singles, H, KVH, NV, PS, scale, window, chunk, keep, softcap, slopes, splits, part_o,
-                                                               part_ml, sinks);
+    AV_ROOMS(true, grid, singles, splits, part_o, part_ml);
+#undef AV_ROOMS
+#undef AV_ROOM
     if (lev_check_launch("attention_values_mfma (single tokens)")) return -1;
     if (splits > 1) {
       attention_values_merge_kernel<<<dim3(n_singles, H), 64, 0, stream>>>(part_o, part_ml, singles, out, H, NV * VD, splits, sinks);
