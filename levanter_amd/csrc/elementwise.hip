@@ -297,8 +297,11 @@ extern "C" int lev_norm_pending(float* x, const float* partial, int S, const flo
 // to 8 consecutive, aligned slots of one page (a prompt portion does, except at its ragged ends), a thread writes
 // its head-dim row for all 8 at once; other tokens are written element by element.
 // Small steps are bound by the chain of loads and waits of a thread, so a thread has as little to do as the head sizes allow
-// (256 tokens, 25 heads of 64, some of them single: 7.8 us with a wave a workgroup and tokens in turn, 5.6 now).
+// (256 tokens, 25 heads of 64, some of them single: 7.1 us with a wave a workgroup and tokens in turn, 4.3 now). The tokens' slots are cut into runs wherever
+// one ends, so that a portion's rows are found also behind single tokens or in the middle of a workgroup's tokens: with cuts at the slots of the
+// first token alone 9 single tokens ahead of 2,039 took 11.4 us (heads of 64) and 23.5 (32 of 128), now 10.4 and 21.6.
 #define KVW_TOKENS 16
+#define KVW_TABLE ((3 * KVW_TOKENS + 4) * (int)sizeof(int))
 
 template <typename T>
 __device__ __forceinline__ void copy8(T* dst, const T* src) {  // 8 elements, both 16-byte aligned
@@ -308,56 +311,106 @@ __device__ __forceinline__ void copy8(T* dst, const T* src) {  // 8 elements, bo
     reinterpret_cast<u32x4*>(dst)[i] = reinterpret_cast<const u32x4*>(src)[i];
 }
 
-template <typename T>
+// PAIRED: a key's chunk and a value's per thread and turn, both on their way together, where a chunk a thread takes more threads than there are
+template <typename T, bool PAIRED>
 __global__ void kv_write_kernel(const T* __restrict__ k, const T* __restrict__ v, long k_stride, long v_stride,
                                 T* __restrict__ k_pages, T* __restrict__ v_pages, const int* __restrict__ dest, int n_tokens,
                                 int KVH, int HD, int VD, int PS, int vec_ok) {
   extern __shared__ __attribute__((aligned(16))) unsigned char kvw_smem[];
-  int* dst_s = reinterpret_cast<int*>(kvw_smem);                       // [KVW_TOKENS]
-  T* vt = reinterpret_cast<T*>(kvw_smem + KVW_TOKENS * sizeof(int));   // [KVW_TOKENS][VD + 8]
+  int* run_s = reinterpret_cast<int*>(kvw_smem);           // [KVW_TOKENS]: first slot of a run of tokens whose slots follow each other
+  int* run_at = run_s + KVW_TOKENS;                        // [KVW_TOKENS]: its first token, and its number of tokens in the upper half
+  int* slot_s = run_at + KVW_TOKENS;                       // [KVW_TOKENS]: every token's
+  int* n_runs = slot_s + KVW_TOKENS;                       // [1]
+  T* vt = reinterpret_cast<T*>(kvw_smem + KVW_TABLE);      // [KVW_TOKENS][VD + 8]
   const int ldv = VD + 8;
   const int t0 = blockIdx.x * KVW_TOKENS;
   const int h = blockIdx.y;
   const int tid = threadIdx.x;
-  if (tid < KVW_TOKENS) dst_s[tid] = t0 + tid < n_tokens ? dest[t0 + tid] : -1;
-  const int chunks = HD / 8, n_k = KVW_TOKENS * chunks, v_chunks = VD / 8;
-  // one chunk of one token per thread and turn: keys into their pages, values into LDS (a value head may have another size than a key head)
-  for (int idx = tid; idx < n_k + KVW_TOKENS * v_chunks; idx += blockDim.x) {
-    const bool value = idx >= n_k;
-    const int per = value ? v_chunks : chunks, at = value ? idx - n_k : idx, i = at / per, c = at % per, t = t0 + i;
-    if (t >= n_tokens) continue;
-    const T* from = value ? v + (size_t)t * v_stride + (size_t)h * VD + c * 8 : k + (size_t)t * k_stride + (size_t)h * HD + c * 8;
-    const int dst = dest[t];
-    if (dst < 0) continue;
-    T* to = value ? vt + i * ldv + c * 8 : k_pages + ((size_t)(dst / PS) * KVH + h) * (size_t)HD * PS + ((size_t)c * PS + dst % PS) * 8;
-    if (vec_ok) {
-      copy8<T>(to, from);
-    } else {
+  if (tid < 64) {  // runs end where a token is dropped, where the next slot is another one, and in front of every multiple of 8
+    const int d = tid < KVW_TOKENS && t0 + tid < n_tokens ? dest[t0 + tid] : -1, before = __shfl_up(d, 1, 64);
+    const bool starts = d >= 0 && (tid == 0 || d != before + 1 || d % 8 == 0);
+    const unsigned long long all = __ballot(starts), ends = all | __ballot(d < 0);  // lanes beyond the tokens count as dropped ones
+    if (starts) {
+      const int r = __popcll(all & ((1ull << tid) - 1));
+      run_s[r] = d;
+      run_at[r] = tid | (__ffsll((long long)(ends >> (tid + 1))) << 16);
+    }
+    if (tid < KVW_TOKENS) slot_s[tid] = d;
+    if (tid == 0) *n_runs = __popcll(all);
+  }
+  // keys into their pages, values into LDS (a value head may have another size than a key head)
+  const int k_chunks = HD / 8, v_chunks = VD / 8;
+  if (PAIRED) {
+    const int chunks = max(k_chunks, v_chunks);
+    for (int idx = tid; idx < KVW_TOKENS * chunks; idx += blockDim.x) {
+      const int i = idx / chunks, c = idx - i * chunks, t = t0 + i;
+      if (t >= n_tokens) continue;
+      const int dst = dest[t];
+      if (dst < 0) continue;
+      const bool has_k = c < k_chunks, has_v = c < v_chunks;
+      const T* kr = k + (size_t)t * k_stride + (size_t)h * HD + (has_k ? c : 0) * 8;
+      const T* vr = v + (size_t)t * v_stride + (size_t)h * VD + (has_v ? c : 0) * 8;
+      __attribute__((aligned(16))) T kc[8], vc[8];
+      if (vec_ok) {
+        copy8<T>(kc, kr);
+        copy8<T>(vc, vr);
+      } else {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) to[e] = from[e];
+        for (int e = 0; e < 8; ++e) kc[e] = kr[e], vc[e] = vr[e];
+      }
+      T* kd = k_pages + ((size_t)(dst / PS) * KVH + h) * (size_t)HD * PS + ((size_t)c * PS + dst % PS) * 8;
+      if (has_k) {
+        if (vec_ok) {
+          copy8<T>(kd, kc);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) kd[e] = kc[e];
+        }
+      }
+      if (has_v) copy8<T>(vt + i * ldv + c * 8, vc);
+    }
+  } else {
+    const int n_k = KVW_TOKENS * k_chunks;
+    for (int idx = tid; idx < n_k + KVW_TOKENS * v_chunks; idx += blockDim.x) {
+      const bool value = idx >= n_k;
+      const int per = value ? v_chunks : k_chunks, at = value ? idx - n_k : idx, i = at / per, c = at % per, t = t0 + i;
+      if (t >= n_tokens) continue;
+      const T* from = value ? v + (size_t)t * v_stride + (size_t)h * VD + c * 8 : k + (size_t)t * k_stride + (size_t)h * HD + c * 8;
+      const int dst = dest[t];
+      if (dst < 0) continue;
+      T* to = value ? vt + i * ldv + c * 8 : k_pages + ((size_t)(dst / PS) * KVH + h) * (size_t)HD * PS + ((size_t)c * PS + dst % PS) * 8;
+      if (vec_ok) {
+        copy8<T>(to, from);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) to[e] = from[e];
+      }
     }
   }
   __syncthreads();
-  // a head-dim row of up to 8 tokens per thread and turn; the tokens are cut where the first one's slots reach a multiple of 8
-  const int cut = dst_s[0] < 0 ? 0 : -dst_s[0] & 7, n_runs = KVW_TOKENS / 8 + (cut > 0);
-  for (int idx = tid; idx < n_runs * VD; idx += blockDim.x) {
-    const int r = idx / VD, d = idx - r * VD, lo = cut ? max(0, cut + 8 * (r - 1)) : 8 * r, n = min(cut ? cut + 8 * r : 8 * r + 8, KVW_TOKENS) - lo;
-    int dst[8];
+  if (*n_runs > 10) {  // mostly single tokens: a head-dim row of 8 tokens per thread and turn, element by element (16 of them, 12 heads of 64: 3.8 us, 4.0 run by run)
+    for (int idx = tid; idx < KVW_TOKENS / 8 * VD; idx += blockDim.x) {
+      const int lo = idx < VD ? 0 : 8, d = idx < VD ? idx : idx - VD;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) dst[j] = j < n ? dst_s[lo + j] : -1;
-    bool run = vec_ok && dst[0] >= 0 && dst[0] % 8 == 0;
-#pragma unroll
-    for (int j = 1; j < 8; ++j) run = run && dst[j] == dst[0] + j;
-    T* base = v_pages + (size_t)h * VD * PS + (size_t)d * PS;
-    if (run) {  // pages hold a multiple of 8 tokens: the slots lie in one
+      for (int j = 0; j < 8; ++j) {
+        const int slot = slot_s[lo + j];
+        if (slot >= 0) v_pages[((size_t)(slot / PS) * KVH + h) * VD * PS + (size_t)d * PS + slot % PS] = vt[(lo + j) * ldv + d];
+      }
+    }
+    return;
+  }
+  // a head-dim row of a run per thread and turn
+  const int work = *n_runs * VD;
+  for (int idx = tid; idx < work; idx += blockDim.x) {
+    const int r = idx / VD, d = idx - r * VD, slot = run_s[r], lo = run_at[r] & 0xffff, n = run_at[r] >> 16;
+    T* to = v_pages + ((size_t)(slot / PS) * KVH + h) * VD * PS + (size_t)d * PS + slot % PS;  // pages hold a multiple of 8 tokens: a run lies in one
+    if (n == 8 && vec_ok) {
       __attribute__((aligned(16))) T row[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) row[j] = vt[(lo + j) * ldv + d];
-      copy8<T>(base + (size_t)(dst[0] / PS) * KVH * VD * PS + dst[0] % PS, row);
+      copy8<T>(to, row);
     } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (dst[j] >= 0) base[(size_t)(dst[j] / PS) * KVH * VD * PS + dst[j] % PS] = vt[(lo + j) * ldv + d];
+      for (int j = 0; j < n; ++j) to[j] = vt[(lo + j) * ldv + d];
     }
   }
 }
@@ -372,19 +425,23 @@ extern "C" int lev_kv_write(const void* k, const void* v, long k_stride, long v_
   LEV_REQUIRE(dtype == LEV_F32 || dtype == LEV_BF16, "kv_write: unknown dtype %d", dtype);
   if (T == 0) return 0;
   const size_t esize = dtype == LEV_F32 ? 4 : 2;
-  const size_t lds = KVW_TOKENS * sizeof(int) + (size_t)KVW_TOKENS * (VD + 8) * esize;
+  const size_t lds = KVW_TABLE + (size_t)KVW_TOKENS * (VD + 8) * esize;
   LEV_REQUIRE(lds <= 64 * 1024, "kv_write: a value head of %d is too large", VD);
   // 16-byte copies of the source rows need aligned rows (the pages always are: page_size and head sizes are multiples of 8)
   const int vec_ok = ((uintptr_t)k % 16 == 0) && ((uintptr_t)v % 16 == 0) && (k_stride * esize % 16 == 0) && (v_stride * esize % 16 == 0) &&
                      ((uintptr_t)k_pages % 16 == 0) && ((uintptr_t)v_pages % 16 == 0);
   dim3 grid((T + KVW_TOKENS - 1) / KVW_TOKENS, KVH);
   const int nt = HD + VD <= 32 ? 64 : (HD + VD <= 64 ? 128 : 256);  // a chunk a thread, or two
-  if (dtype == LEV_F32)
-    kv_write_kernel<float><<<grid, nt, lds, stream>>>((const float*)k, (const float*)v, k_stride, v_stride, (float*)k_pages,
-                                                      (float*)v_pages, dest, T, KVH, HD, VD, PS, vec_ok);
-  else
-    kv_write_kernel<bf16_t><<<grid, nt, lds, stream>>>((const bf16_t*)k, (const bf16_t*)v, k_stride, v_stride,
-                                                       (bf16_t*)k_pages, (bf16_t*)v_pages, dest, T, KVH, HD, VD, PS, vec_ok);
+  const bool paired = KVW_TOKENS * (HD / 8 + VD / 8) > nt;
+#define KVW_CASE(T_, PAIRED)                                                                                                                       \
+  kv_write_kernel<T_, PAIRED><<<grid, nt, lds, stream>>>((const T_*)k, (const T_*)v, k_stride, v_stride, (T_*)k_pages, (T_*)v_pages, dest, T, KVH, \
+                                                         HD, VD, PS, vec_ok)
+  if (dtype == LEV_F32) {
+    if (paired) KVW_CASE(float, true); else KVW_CASE(float, false);
+  } else {
+    if (paired) KVW_CASE(bf16_t, true); else KVW_CASE(bf16_t, false);
+  }
+#undef KVW_CASE
   return lev_check_launch("kv_write");
 }
 
