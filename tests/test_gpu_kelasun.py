@@ -260,7 +260,7 @@ def test_routing_and_sorting_in_one_kernel(T, E, G, keep, top, scoring, extra):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("T,D,F,E,top,shared", [(37, 64, 24, 6, 3, 24), (1, 32, 8, 2, 2, None), (300, 96, 48, 4, 2, 40), (5, 40, 13, 9, 1, 16), (5, 40, 16, 9, 2, 16), (16, 64, 32, 7, 1, 32), (20, 64, 32, 16, 3, 32), (700, 64, 24, 30, 4, 64), (400, 64, 160, 5, 2, None)])
+@pytest.mark.parametrize("T,D,F,E,top,shared", [(37, 64, 24, 6, 3, 24), (1, 32, 8, 2, 2, None), (300, 96, 48, 4, 2, 40), (5, 40, 13, 9, 1, 16), (5, 40, 16, 9, 2, 16), (28, 64, 32, 5, 2, 32), (32, 64, 32, 5, 2, 32), (33, 64, 32, 5, 2, 32), (16, 64, 32, 7, 1, 32), (20, 64, 32, 16, 3, 32), (700, 64, 24, 30, 4, 64), (400, 64, 160, 5, 2, None)])
 def test_experts_without_gates_beside_a_shared_one(dtype, T, D, F, E, top, shared):
     """Few tokens, tiles of 16 rows and of 64: the part's own result, the result added to a stream, and the sum left to the pass that reads it."""
     from levanter_amd.parts import BuildEnv, PartSpec, TensorSpec, part_class
@@ -295,7 +295,7 @@ def test_experts_without_gates_beside_a_shared_one(dtype, T, D, F, E, top, share
     y = torch.full((T, D), float("nan"), device=DEV)
     left = part.compute_unsummed(dev(h, dtype), y, ctx)
     # a shared expert of the experts' size (filled up to a multiple of 8) is the last choice of every token where the experts have few rows each
-    assert left.alone == (shared is None or (shared == (F + 7) // 8 * 8 and T * (top + 1) < 12 * (E + 1)))
+    assert left.alone == (shared is None or (shared == (F + 7) // 8 * 8 and T * (top + 1) <= 16 * (E + 1)))
     product = ctx.take_product_pending(y)
     x, nw = dev(x0), torch.ones(D, device=DEV)
     K().finish(K().sum_norm_step(x, alpha=2.0, y=None if left.alone or product is not None else y, product=product, experts=left, write_norm=(nw, None, 1e-5, False), defer=True))
