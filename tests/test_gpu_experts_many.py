@@ -1,0 +1,71 @@
+"""The experts' products over tiles of 128 rows at the edges of the kernel that carries them: outputs that end inside a tile, inner sizes of one step, of an
+odd and an even number and with a short step, stretches of one row, of half a tile, a tile and one more or less, output rows without alignment, and lists of
+more tiles a chiplet than a wave has lanes."""
+import pytest
+import torch
+import torch.nn.functional as F_
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def K():
+    from levanter_amd.kernels import get_kernels
+
+    return get_kernels()
+
+
+def _sorted(K, counts):
+    """One token a pair, in a drawn order; the experts of the sorted pairs beside the lists."""
+    E, P = len(counts), sum(counts)
+    order = torch.randperm(P, generator=torch.Generator().manual_seed(P))
+    chosen = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[order].to(torch.int32).to(DEV).unsqueeze(1)
+    tables = torch.empty(2 * P + 1 + 3 * K.moe_max_tiles(P, E, 128), dtype=torch.int32, device=DEV)
+    sp, po, meta, tiles = tables[:P], tables[P:2 * P], tables[2 * P:2 * P + 1], tables[2 * P + 1:]
+    K.moe_sort(chosen, E, sp, po, tiles, meta, tile_rows=128)
+    return sp, tiles, meta, chosen[:, 0].long()[sp.long()]
+
+
+def _check(K, counts, Fo, Kd, widths, dtypes=(torch.float32, torch.bfloat16)):
+    """bfloat16 operands are exact in float64; a sum of Kd products in 32 bits is off by at most Kd * 2^-24 of the sum of their absolute values (e), and
+    silu(gate) * up by 1.1 e_gate |up| + |silu(gate)| e_up + 1.1 e_gate e_up (silu's slope stays below 1.1) and 2^-20 of itself."""
+    g = torch.Generator(device=DEV).manual_seed(Fo * 31 + Kd)
+    E, P = len(counts), sum(counts)
+    sp, tiles, meta, expert = _sorted(K, counts)
+    h = torch.randn(P, Kd + 8, device=DEV, generator=g).bfloat16()[:, :Kd]
+    first = [sum(counts[:e]) for e in range(E)]
+    for glu in (False, True):
+        w = (torch.randn(E, Fo * (2 if glu else 1), Kd, device=DEV, generator=g) / Kd ** 0.5).bfloat16()
+        for gather in (False, True):
+            rows = h[sp.long()] if gather else h
+            parts = [(rows[first[e]:first[e] + n].double(), w[e].double()) for e, n in enumerate(counts)]
+            y = torch.cat([r @ m.T for r, m in parts])
+            err = (Kd + 8) * 2.0 ** -24 * torch.cat([r.abs() @ m.abs().T for r, m in parts])
+            if glu:
+                gate, up, eg, eu = F_.silu(y[:, :Fo]), y[:, Fo:], err[:, :Fo], err[:, Fo:]
+                y, err = gate * up, 1.1 * eg * up.abs() + gate.abs() * eu + 1.1 * eg * eu + 2.0 ** -20 * (gate * up).abs()
+            for dtype in dtypes:
+                for width in widths:
+                    out = torch.full((P, width), float("nan"), device=DEV, dtype=dtype)
+                    K.moe_linear(h, w, out[:, :Fo], tiles, meta, sp, top=1, gather=gather, glu=glu, activation="silu" if glu else "none", tile_rows=128)
+                    bound = err + 1e-30 + (2.0 ** -8 * (y.abs() + err) if dtype is torch.bfloat16 else 0)
+                    assert bool(((out[:, :Fo].double() - y).abs() <= bound).all()), (glu, gather, dtype, width)
+                    assert bool(torch.isnan(out[:, Fo:]).all())
+
+
+@pytest.mark.parametrize("Fo", [1, 63, 64, 65, 129])
+@pytest.mark.parametrize("Kd", [8, 64, 72, 136, 192, 2056])
+def test_products_over_tiles_of_128_rows_against_float64(K, Fo, Kd):
+    _check(K, [1, 63, 0, 64, 65, 128, 129], Fo, Kd, (Fo, Fo + 3, (Fo + 3) // 4 * 4 + 4))
+
+
+@pytest.mark.parametrize("experts", [511, 513, 700])
+def test_more_tiles_than_lanes_a_chiplet(K, experts):
+    """Up to 512 tiles a chiplet's larger ones come first, beyond that the list's order holds."""
+    counts = [(1, 130, 200, 70)[e % 4] for e in range(experts - experts // 2)]
+    while sum((n + 127) // 128 for n in counts) < experts:
+        counts.append(2)
+    assert sum((n + 127) // 128 for n in counts) == experts
+    _check(K, counts, 72, 136, (72,), (torch.float32,))
