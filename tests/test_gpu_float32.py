@@ -20,9 +20,10 @@ def _rand(*shape, seed=0):
 
 
 # rows, inputs, outputs: every tile of the list (rows x outputs of 16 x 16 .. 64 x 128), at its edges, one more and one less; inputs that are
-# no multiple of a step of 16, fewer than the waves have steps, and (no multiple of 4) none that 16-byte loads take
+# no multiple of a step of 16, fewer than the waves have steps, and (no multiple of 4) none that 16-byte loads take. (13, 264, 50257) takes
+# 16 x 32 and (15, 264, 11531) 16 x 64.
 LINEAR = [(1, 4, 1), (1, 64, 50), (3, 768, 768), (16, 100, 48), (17, 772, 33), (31, 1024, 130), (33, 20, 65), (64, 256, 4096), (65, 300, 1024), (129, 1028, 257),
-          (203, 516, 1000), (400, 128, 1030), (777, 260, 1024), (1031, 96, 3000), (5, 6, 40), (70, 333, 129)]
+          (203, 516, 1000), (400, 128, 1030), (777, 260, 1024), (1031, 96, 3000), (15, 264, 11531), (13, 264, 50257), (5, 6, 40), (70, 333, 129)]
 
 
 @pytest.mark.parametrize("M,Ki,N", LINEAR)
@@ -78,10 +79,11 @@ def _attention_float64(q, kp, vp, bt, runs, H, KVH, HD, PS, scale, window):
 
 
 # runs of (tokens, keys after the step): tiles of 16 rows with 1 to 16 in use, blocks of 64 and 32 keys at their edges, single tokens beside
-# them; groups of heads that fill a column set, more and less; every head size
+# them; groups of heads that fill a column set, more and less; every head size; single tokens that need more than 64 KB of LDS (the last two)
 ATTENTION = [(4, 4, 64, 16, [(2, 2), (17, 17), (1, 64), (1, 65), (15, 80)], None), (16, 1, 16, 16, [(1, 1), (1, 33), (3, 130)], None),
              (20, 1, 32, 32, [(1, 257), (18, 18)], 20), (6, 2, 48, 16, [(1, 300), (129, 140)], 64), (5, 5, 80, 48, [(33, 97), (1, 31)], None),
-             (3, 1, 96, 16, [(1, 128), (16, 16)], 17), (2, 2, 112, 64, [(1, 127), (31, 31)], None), (8, 4, 128, 16, [(1, 513), (40, 72), (1, 2)], 1)]
+             (3, 1, 96, 16, [(1, 128), (16, 16)], 17), (2, 2, 112, 64, [(1, 127), (31, 31)], None), (8, 4, 128, 16, [(1, 513), (40, 72), (1, 2)], 1),
+             (16, 1, 128, 16, [(1, 300), (1, 16), (20, 20), (1, 1)], None), (32, 2, 112, 32, [(1, 200), (1, 33)], 100)]
 
 
 @pytest.mark.parametrize("H,KVH,HD,PS,runs,window", ATTENTION)
@@ -129,3 +131,30 @@ def test_attention_float32_values_that_are_not_seen_do_not_count(K, bad):
     rest[40] = False
     # the other sums of that tile go key by key: another order of at most 40 terms of at most 5, each off by 2^-24 of it
     torch.testing.assert_close(heads[rest], clean.view(41, H, HD)[rest], rtol=0, atol=40 * 5 * EPS)
+
+
+@pytest.mark.parametrize("HD,H", [(64, 4), (128, 16), (16, 20)])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_attention_float32_values_outside_the_window_do_not_count(K, bad, HD, H):
+    """Key 20 holds a value that is not a number, the window 10 keys: of a run and of single tokens only those that see the key carry it."""
+    from helpers import make_meta
+    from test_gpu_kernels import _fill_cache
+
+    KVH, PS, window, runs = 1, 16, 10, [(40, 40), (1, 30), (1, 31), (1, 21)]
+    kv = [k for _, k in runs]
+    bt, kp, vp, kd, vd, _, _ = _fill_cache(K, torch.float32, kv, KVH, HD, PS, 12, seed=7)
+    T = sum(n for n, _ in runs)
+    q = _rand(T, H * HD, seed=8).to(DEV)
+    args = dict(n_heads=H, n_kv_heads=KVH, head_dim=HD, page_size=PS, scale=HD ** -0.5, window=window, block_tables=bt.to(DEV))
+    clean, got = torch.empty(T, H * HD, device=DEV), torch.empty(T, H * HD, device=DEV)
+    K.paged_attention(q, clean, kd, vd, make_meta(runs, DEV), **args)
+    for s in range(len(runs)):
+        vd.view(-1, KVH, HD, PS)[int(bt[s, 1]), 0, 5, 4] = bad
+    K.paged_attention(q, got, kd, vd, make_meta(runs, DEV), **args)
+    hit = torch.zeros(T, H, HD, dtype=torch.bool, device=DEV)
+    hit[20:30, :, 5] = True  # positions 20 .. 29 see keys 11 .. 29
+    hit[[40, 42], :, 5] = True  # positions 29 and 20; position 30 sees 21 .. 30
+    heads = got.view(T, H, HD)
+    assert bool((~torch.isfinite(heads) == hit).all())
+    # the other sums of such a tile go key by key: another order of at most 10 terms of at most 5, each off by 2^-24 of it
+    torch.testing.assert_close(heads[~hit], clean.view(T, H, HD)[~hit], rtol=0, atol=10 * 5 * EPS)
