@@ -604,7 +604,7 @@ __device__ __forceinline__ void decode_wave(int idx, int kvh, int z, const bf16_
   const bool fused = k_new != nullptr;
   // The new key and value are copied to their page by one wave of the (token, kv head): the last one if it has no keys
   // of its own (the ranges are rounded up, so with few blocks the last waves are idle), else the wave whose range
-  // holds the token's position, which then has the copy ahead of its two or more blocks.
+  // holds the token's position, which then has the copy's loads ahead of its two or more blocks and its stores behind them.
   const bool idle_last = splits > 1 && kb_first + (splits - 1) * per > kb_last;
   const bool owner = fused && (idle_last ? z == splits - 1 : (kb_begin <= kb_last && kb_last < kb_end));
   const bf16_t* q_row = q + (size_t)t * q_stride;

@@ -8,8 +8,8 @@ typedef __attribute__((ext_vector_type(4))) float gf_f32x4;
 // A workgroup of W waves owns 16 RT rows and 16 NT outputs; its waves split K (steps of 16 dealt in stretches) and the partial sums are
 // added through LDS in wave order. The product is transposed, out^T = w a^T, so that a lane ends with four neighbouring outputs of one
 // row. Both operands come straight from global memory, 16 bytes a lane (row = lane % 16, k = 4 (lane / 16) + j for the j-th of the
-// four products of a step): the 32-bit instruction takes 32 cycles for 1,024 multiply-adds, so that operands through LDS would buy
-// nothing that the caches do not give, but for tiles too small for their L2 traffic.
+// four products of a step): the 32-bit instruction takes 32 cycles for 1,024 multiply-adds, which hides much of what such loads cost
+// the vector cache (a look-up for every lane); whole lines turned into operands in LDS, as the bfloat16 kernels read them, have not been tried.
 // What bounds it: few rows, the read of the weights (4096 x 4096 at 4 rows 14.3 us, 4.7 TB/s; 768 x 768 4.8 us, a launch and a chain of
 // loads); some hundred rows, L2 at about 9.5 TB/s (1024 x 4096 at 203 rows 33 us) or the last round of tiles; many, the matrix pipe
 // (4096 x 4096 at 2,048 rows 532 us, 129 TFLOP/s of 157). The plain kernel of gemm_simple.hip (64 x 64 tiles, vector ALU, scalar loads)

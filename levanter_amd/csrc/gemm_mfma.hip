@@ -341,12 +341,13 @@ static int launch_tile(const bf16_t* a, long lda, const bf16_t* w, const float* 
 // for); what lies beyond K is masked on its way into LDS, rows beyond M and columns beyond N are read again and never stored.
 // Measured in graphs over distinct weights, before (weights straight into the operand, conditional loads) and now, microseconds: 4800 x
 // 1600 at 6 / 24 rows 8.0 / 12.5 -> 6.4 / 8.9; 6400 x 1600 8.3 / 12.9 -> 7.0 / 9.2; 4608 x 2048 9.1 / 14.2 -> 6.8 / 9.0; 768 x 768 3.8 / 4.8 -> 3.5 /
-// 4.0; 4096 x 4096 8.6 / 12.5 -> 8.4 / 10.2; 16384 x 4096 25.0 -> 24.2 at 6 rows (memory: 5.5 TB/s); the same bits.
+// 4.0; 4096 x 4096 8.6 / 12.5 -> 8.4 / 10.2; 16384 x 4096 25.0 -> 24.2 at 6 rows (memory: 5.5 TB/s).
 // The partial sums of the waves are added through LDS in wave order. Every workgroup starts at another
 // place of the k range, so that they do not all read the same part of `a` and the same residue of the weight
-// rows at the same time; the order of the sum depends on the column tile only, never on M or the batch.
+// rows at the same time; the order of a sum depends on the column tile
+// and, through the launch's shape (skinny_shape), on the number of rows, never on what other rows hold.
 #define SKINNY_SLOTS 72  // 16-byte slots of one staged instruction: 8 rows x (8 chunks + 1 of padding)
-#define SKINNY_MAX_M 256  // which of these row counts it takes: use_skinny()
+#define SKINNY_MAX_M 256  // which of these row counts it takes: use_skinny(); blocks of more rows have not been measured
 
 template <typename TO, int WAVES, int U, int MT, int NT, bool HALF, bool BLOCKS>
 // at most 128 registers a lane for 2 x 2 tiles (130 cost 7 % at 2048 x 2048 and 96 rows); with four waves at most 256, so that the sums stay in
