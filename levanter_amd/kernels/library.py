@@ -1233,10 +1233,14 @@ class HipKernels:
 
     @staticmethod
     def moe_tile_rows(pairs: int, n_experts: int) -> int:
-        """Rows of a tile of the experts' products: 128 where an expert has more than 16 rows on average, else 16 (32 experts of 2048 x 2048,
-        4 a token, microseconds of the two products, 16 / 128: 64 tokens 50 + 51 / 72 + 72 (gated 97 / 135 for the first), 128 tokens 65 + 73 /
-        72 + 73 (121 / 136), 192 tokens 82 + 119 / 73 + 74 (155 / 136))."""
-        return 128 if pairs > 16 * n_experts else 16
+        """Rows of a tile of the experts' products: 16 up to 12, 14 or 16 rows an expert on average, else 128. Tiles of 16 read the weights faster (5.4 TB/s
+        of distinct ones against 3.9, and 2.6 where few experts leave CUs without a tile of 128), but every expert with a 17th row has a second tile; the more
+        experts, the more workgroups of 128 rows there are to hide behind each other. Up and down product of distinct weights, microseconds, 16 / 128 rows a
+        tile: 16 experts of 2048 x 2048 at 14 / 16 rows 66 / 75, 73 / 75; 32 of 4096 x 2048 at 14 / 15 / 16 rows 233 / 255, 249 / 255, 292 / 256; 33 of 2048 x 2048 at 16 rows
+        150 / 184; 64 of 2048 x 2048 at 13 / 14 / 16 rows 248 / 258, 268 / 256, 299 / 253; 128 of 2048 x 1024 at 12 / 13 / 16 rows 242 / 247, 254 / 245, 305 / 244
+        (gated 336 / 305, 349 / 306, 420 / 310); 256 of 1024 x 512 at 12 / 13 / 16 rows 126 / 128, 132 / 129, 155 / 130."""
+        rows = 12 if n_experts >= 96 else 14 if n_experts >= 48 else 16
+        return 128 if pairs > rows * n_experts else 16
 
     def moe_max_tiles(self, pairs: int, n_experts: int, tile_rows: int = 16) -> int:
         return int(self.lib.lev_moe_max_tiles(int(pairs), int(n_experts), int(tile_rows)))

@@ -432,7 +432,7 @@ class EmulatedKernels:
 
     @staticmethod
     def moe_tile_rows(pairs, n_experts) -> int:
-        return 128 if pairs > 16 * n_experts else 16
+        return 128 if pairs > (12 if n_experts >= 96 else 14 if n_experts >= 48 else 16) * n_experts else 16
 
     def moe_max_tiles(self, pairs, n_experts, tile_rows=16) -> int:
         return pairs // tile_rows + n_experts + 1

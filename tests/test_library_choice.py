@@ -31,3 +31,15 @@ def test_below_25_rows_and_for_other_activations_never():
 def test_sums_that_the_librarys_single_chain_would_make_less_exact_stay_ours():
     for N, K in ((50257, 4096), (27648, 5120), (12000, 1280), (65024, 2560)):
         assert not any(HipKernels.use_library(M, N, K, 0) for M in range(1, 65))
+
+
+# experts, width, inner width, rows an expert, microseconds of the up and the down product with tiles of 16 and of 128 rows
+EXPERTS = [(8, 2048, 4096, 12, 61.9, 87.5), (16, 2048, 2048, 14, 65.9, 74.5), (16, 1024, 1024, 16, 23.3, 27.2), (32, 2048, 1024, 13, 63.8, 66.5), (33, 2048, 2048, 16, 150.2, 183.5),
+           (32, 4096, 2048, 14, 232.9, 254.6), (64, 1024, 512, 13, 30.5, 34.1), (64, 2048, 2048, 14, 268.1, 256.2), (64, 2048, 1024, 15, 136.6, 127.5), (64, 2048, 2048, 16, 298.5, 253.2),
+           (128, 1024, 768, 12, 95.1, 95.2), (128, 2048, 1024, 13, 253.8, 245.4), (128, 2048, 1024, 16, 305.1, 243.5), (256, 1024, 512, 14, 141.1, 129.3), (256, 1024, 512, 12, 125.8, 127.9)]
+
+
+@pytest.mark.parametrize("experts,width,inner,rows,few,many", EXPERTS)
+def test_the_tiles_of_the_experts_products_are_the_faster_ones(experts, width, inner, rows, few, many):
+    taken = {16: few, 128: many}[HipKernels.moe_tile_rows(rows * experts, experts)]
+    assert taken <= 1.05 * min(few, many)
