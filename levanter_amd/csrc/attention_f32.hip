@@ -229,7 +229,7 @@ static int attention_f32_launch(const AttentionF32Args& common, const int* tiles
     attention_f32_kernel<HD, KB, W, true><<<(unsigned)blocks, 64 * W, lds, stream>>>(p);
   }
   if (n_tokens > 0) {
-    constexpr int W = 8;
+    constexpr int W = 8;  // at most 256 registers a lane: head size 128 keeps 52 bytes of them in scratch memory
     const int group = p.H / p.KVH, sets = (group + 15) / 16;
     p.work = tokens, p.tile_rows = 0, p.columns = group < 16 ? group : 16;
     const int lds = W * DT * 4 * p.columns * 16 + 2 * W * 16 * 4 + W * 1024;

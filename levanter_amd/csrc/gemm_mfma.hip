@@ -521,6 +521,9 @@ gemm_skinny_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restr
 //     4096 at 24 rows 31.0 -> 26.4, at 48 rows 40.7 -> 28.4); above that three up to 32 rows (18432 x 6144 at 24 rows 55.8 -> 49.5), else four
 //     (32000 x 2048 at 48 rows 28.3 against 35.1 for the stream kernel, 50257 x 4096 89.5 against 105 with three);
 //   but up to 16 rows above 720 units one unit and 4 waves with four pairs in flight: 12288 x 4096 at 6 rows 20.7 -> 18.9, 16384 x 4096 29 -> 24.3.
+// Beside the lines, at 6 rows: 16 / 8 waves of two units, 7600 outputs, sums of 1,664 / 1,920: 7.5 / 7.4, 8.6 / 8.0; three units / one with 4 waves, sums of
+// 2,048: 10752 outputs 10.6 / 11.1, 12288 11.4 / 11.7, 14336 17.1 / 13.5, sums of 4,096: 18.8 / 18.7, 20.9 / 19.6, 30.6 / 23.6; 16 / 8 waves of half a unit, 2048
+// outputs, sums of 4,096 / 5,120 / 8,192: 5.9 / 6.1, 7.3 / 7.9, 9.2 / 10.7.
 struct SkinnyShape {
   int waves, in_flight, row_tiles, units;  // the kernel's WAVES, U, MT, NT
   bool half;
