@@ -415,18 +415,57 @@ moe_linear_few_kernel(const MoeLinearArgs p) {
 // one barrier a step that waits for LDS only; loads, LDS writes and fragment reads are issued one by one between the products. Rows
 // beyond the tile are read again and never stored. The workgroups of a tile and of its neighbours in the list (an expert's rows, its
 // weights) follow each other on one of the eight chiplets (workgroups are dealt to them in turn).
+// What bounds it: the read of the weights with up to about 128 rows an expert (4.7 - 5.0 TB/s), else what the CUs pull through L2 (32 KB a
+// step and workgroup at 15 TB/s) and the last round of tiles. The outputs leave through LDS as whole lines, after one decision on the activation
+// for all of them: stored from the products' registers, 8 or 16 bytes of each of 32 rows, with the decision at every value, the last 64 KB of a
+// workgroup cost 15 us a round: 2048 outputs of 2048 (bfloat16 / 32-bit, microseconds), 32 experts of 256 rows 126 / 137 -> 110 / 116,
+// 4 of 2,048 93 / 105 -> 78 / 80. Where the weights' read is the bound, fewer than two rounds of a chiplet's 64 workgroups, these begin at places of
+// their own along K: rows a power of two apart lie in the same channels of the memory, and workgroups that walk together ask those alone: 32
+// experts of 128 rows 97 -> 65 us, of 40 72 -> 56, of 90 99 -> 83; from two rounds on they have drifted apart (254 rows 136 either way, 8 experts of
+// 4,096 rows 190 in order, 197 spread). Measured and not kept: tiles of 256 rows by 8 waves (32 of 256 rows 107, of 254 drawn ones 153 against 136),
+// workgroups that stay and fetch the next tile's first steps ahead of the last outputs (spills; 4 of 2,048 rows 82 - 107), weights three
+// steps ahead (no gain), chiplets' shares by cost (of 40 rows 77 against 55).
 #define MOE_BN 128
 #define MOE_BIG_K 64
 #define MOE_BIG_LD (MOE_BIG_K + 8)
+#define MOE_BIG_SPREAD 128  // a chiplet's workgroups of two rounds
 #define MOE_BIG_LDS(BN) (2 * (MOE_BIG + (BN)) * MOE_BIG_LD * (int)sizeof(bf16_t))
 typedef __attribute__((ext_vector_type(16))) float moe_f32x16;
+// the sums become outputs in place; with glu the first half of a row's registers takes them
+template <int ACT, bool GLU, int TI, int TJ>
+__device__ __forceinline__ void moe_big_activate(moe_f32x16 (&acc)[TI][TJ], const MoeLinearArgs& p) {
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < (GLU ? TJ / 2 : TJ); ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = GLU ? moe_act(acc[i][j][r], acc[i][(j + TJ / 2) % TJ][r], ACT, p.limit, p.up_shift) : lev_activate(acc[i][j][r], ACT);
+}
+
+// eight (bfloat16) or four (float32) neighbouring outputs of a row; `vec`: 1: rows allow half of such a store, 2: a whole one
+__device__ __forceinline__ void moe_big_store(float* to, const moe_u32x4& v, int left, int vec) {
+  if (vec && left >= 4) *reinterpret_cast<moe_u32x4*>(to) = v;
+  else
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (r < left) to[r] = __uint_as_float(v[r]);
+}
+__device__ __forceinline__ void moe_big_store(bf16_t* to, const moe_u32x4& v, int left, int vec) {
+  if (vec == 2 && left >= 8) *reinterpret_cast<moe_u32x4*>(to) = v;
+  else if (vec && left >= 8) reinterpret_cast<uint2*>(to)[0] = make_uint2(v[0], v[1]), reinterpret_cast<uint2*>(to)[1] = make_uint2(v[2], v[3]);
+  else
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      if (r < left) to[r] = (bf16_t)(v[r / 2] >> (r % 2 * 16));
+}
+
 // BM: 128, or 64 for a tile whose rows fit that
 template <typename TO, bool GLU, int BN, int BM>
-__device__ __forceinline__ void moe_big_tile(const MoeLinearArgs& p, unsigned char* moe_smem, int e, int first, int rows, int ycol) {
+__device__ __forceinline__ void moe_big_tile(const MoeLinearArgs& p, unsigned char* moe_smem, int e, int first, int rows, int ycol, bool spread) {
   constexpr int LD = MOE_BIG_LD, WM = BM / 2, WN = BN / 2, TI = WM / 32, TJ = WN / 32;
   constexpr int CA = BM * (MOE_BIG_K / 8) / 256, CW = BN * (MOE_BIG_K / 8) / 256;  // 16-byte chunks a thread fetches a step
   constexpr int OUT = GLU ? BN / 2 : BN;  // outputs of a workgroup
-  const int K = p.K, N = p.N, F = p.F, act = p.act;
+  const int K = p.K, N = p.N, F = p.F;
   bf16_t* sa = reinterpret_cast<bf16_t*>(moe_smem);  // [2][BM][LD]
   bf16_t* sw = sa + 2 * BM * LD;                     // [2][BN][LD]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
@@ -447,7 +486,11 @@ __device__ __forceinline__ void moe_big_tile(const MoeLinearArgs& p, unsigned ch
   }
   // the steps in the order they are taken: a partial one (K % 64 != 0) first, so that the loop needs no masks
   const int tail = K % MOE_BIG_K, steps = (K + MOE_BIG_K - 1) / MOE_BIG_K, shift = tail ? 1 : 0;
-  auto k_of = [&](int t) { return max(min(t, steps - 1) - shift, 0) * MOE_BIG_K; };  // t >= 1; beyond the last: loaded again, not used
+  const int turn = spread && !tail ? ycol * 5 % steps : 0;  // whole steps then begin at a place of the workgroup's own
+  auto k_of = [&](int t) {  // t >= 1; beyond the last: loaded again, not used
+    const unsigned i = max(min(t, steps - 1) - shift, 0) + turn;
+    return (int)min(i, i - (unsigned)steps) * MOE_BIG_K;  // i, or i - steps if that is not below 0
+  };
   moe_u32x4 ra[2][CA], rw[2][CW];
   auto fetch_one = [&](int set, int k, int i) {
     if (i < CA) ra[set][i] = *reinterpret_cast<const moe_u32x4*>(pa[i] + k);
@@ -467,7 +510,7 @@ __device__ __forceinline__ void moe_big_tile(const MoeLinearArgs& p, unsigned ch
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
   {
-    const int k0 = tail ? K - tail : 0, k = min(k0 + kc, K - 8);
+    const int k0 = tail ? K - tail : turn * MOE_BIG_K, k = min(k0 + kc, K - 8);
     const bool in = k0 + kc < K;
 #pragma unroll
     for (int i = 0; i < CA + CW; ++i) fetch_one(0, k, i);
@@ -535,23 +578,44 @@ __device__ __forceinline__ void moe_big_tile(const MoeLinearArgs& p, unsigned ch
     step(t + 1, 0);
   }
   if (t < steps) step(t, 1);
-  // register r of a 32 x 32 tile: output 8 (r / 4) + 4 (lane / 32) + r % 4 of the tile, row lane % 32
-#pragma unroll
-  for (int i = 0; i < TI; ++i) {
-    const int row = wm * WM + 32 * i + (lane & 31);
-    if (row >= rows) continue;
-#pragma unroll
-    for (int j = 0; j < (GLU ? TJ / 2 : TJ); ++j)
-#pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4) {
-        const int o = o0 + wn * (GLU ? WN / 2 : WN) + 32 * j + 8 * r4 + 4 * (lane >> 5);
-        if (o >= F) continue;
-        float v[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = GLU ? moe_act(acc[i][j][4 * r4 + r], acc[i][(j + TJ / 2) % TJ][4 * r4 + r], act, p.limit, p.up_shift) : lev_activate(acc[i][j][4 * r4 + r], act);
-        moe_store4<TO>(static_cast<TO*>(p.out) + (size_t)(first + row) * p.o_stride + o, v, F - o, p.vec);
-      }
+  lds_barrier();  // nobody reads the buffers any more
+  switch (p.act) {  // one decision for all outputs
+    case LEV_ACT_GELU_TANH: moe_big_activate<LEV_ACT_GELU_TANH, GLU, TI, TJ>(acc, p); break;
+    case LEV_ACT_GELU_ERF: moe_big_activate<LEV_ACT_GELU_ERF, GLU, TI, TJ>(acc, p); break;
+    case LEV_ACT_RELU: moe_big_activate<LEV_ACT_RELU, GLU, TI, TJ>(acc, p); break;
+    case LEV_ACT_SILU: moe_big_activate<LEV_ACT_SILU, GLU, TI, TJ>(acc, p); break;
+    case LEV_ACT_QUICK_GELU: moe_big_activate<LEV_ACT_QUICK_GELU, GLU, TI, TJ>(acc, p); break;
+    case LEV_ACT_TANH: moe_big_activate<LEV_ACT_TANH, GLU, TI, TJ>(acc, p); break;
+    case LEV_ACT_RELU_SQUARED: moe_big_activate<LEV_ACT_RELU_SQUARED, GLU, TI, TJ>(acc, p); break;
+    default: moe_big_activate<LEV_ACT_NONE, GLU, TI, TJ>(acc, p);
   }
+  // Whole lines go out: 32 rows and 128 bytes of each (64 where a wave has no more) turn round in a part of the LDS that is the wave's own.
+  // Register r of a 32 x 32 tile: output 8 (r / 4) + 4 (lane / 32) + r % 4, row lane % 32
+  constexpr bool F32 = sizeof(TO) == 4;
+  constexpr int TO_J = GLU ? TJ / 2 : TJ, JB = F32 ? 1 : TO_J, PER = 16 / (int)sizeof(TO), WIDTH = 32 * JB, LR = WIDTH / PER;  // lanes a row
+  constexpr int STRIDE = 36 * 4 / (int)sizeof(TO);
+  TO* lines = reinterpret_cast<TO*>(moe_smem + wave * 32 * 36 * 4);
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int jb = 0; jb < TO_J / JB; ++jb) {
+#pragma unroll
+      for (int j = 0; j < JB; ++j)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+          const moe_f32x16& v = acc[i][jb * JB + j];
+          TO* at = lines + (lane & 31) * STRIDE + 32 * j + 8 * r4 + 4 * (lane >> 5);
+          if constexpr (F32) *reinterpret_cast<float4*>(at) = make_float4(v[4 * r4], v[4 * r4 + 1], v[4 * r4 + 2], v[4 * r4 + 3]);
+          else *reinterpret_cast<uint2*>(at) = make_uint2(float2_to_bf16x2(v[4 * r4], v[4 * r4 + 1]), float2_to_bf16x2(v[4 * r4 + 2], v[4 * r4 + 3]));
+        }
+#pragma unroll
+      for (int x = 0; x < 32 * LR / 64; ++x) {
+        const int r = (64 * x + lane) / LR, c = lane % LR * PER, at = wm * WM + 32 * i + r;
+        const int o = o0 + wn * (GLU ? WN / 2 : WN) + 32 * jb * JB + c;
+        const moe_u32x4 v = *reinterpret_cast<const moe_u32x4*>(lines + r * STRIDE + c);
+        if (at < rows && o < F) moe_big_store(static_cast<TO*>(p.out) + (size_t)(first + at) * p.o_stride + o, v, F - o, p.vec);
+      }
+    }
 }
 
 template <typename TO, bool GLU>
@@ -574,9 +638,10 @@ moe_linear_big_kernel(const MoeLinearArgs p) {
     ycol = at / kind;
     tile = lo + __ffsll(__ballot((of >> lane & 1) && __popcll(of & ((1ull << lane) - 1)) == at % kind)) - 1;
   }
+  const bool spread = n * p.n_cols < MOE_BIG_SPREAD;
   const int e = p.tiles[3 * tile], first = p.tiles[3 * tile + 1], rows = p.tiles[3 * tile + 2];
-  if (rows <= MOE_BIG / 2) moe_big_tile<TO, GLU, MOE_BN, MOE_BIG / 2>(p, moe_smem, e, first, rows, ycol);
-  else moe_big_tile<TO, GLU, MOE_BN, MOE_BIG>(p, moe_smem, e, first, rows, ycol);
+  if (rows <= MOE_BIG / 2) moe_big_tile<TO, GLU, MOE_BN, MOE_BIG / 2>(p, moe_smem, e, first, rows, ycol, spread);
+  else moe_big_tile<TO, GLU, MOE_BN, MOE_BIG>(p, moe_smem, e, first, rows, ycol, spread);
 }
 
 // a [rows][K]; w [E][N][K] with N = F outputs, or with glu N = 2F: gate rows then up rows; out [P][F]
@@ -593,7 +658,7 @@ extern "C" int lev_moe_linear(const void* a, long a_stride, const void* w, void*
   LEV_REQUIRE(a_stride >= K && o_stride >= F, "experts: row strides are smaller than the rows");
   if (max_tiles == 0) return 0;
   if (dtype == LEV_BF16 && use_mfma && K % 8 == 0 && a_stride % 8 == 0 && ((uintptr_t)a & 15) == 0 && ((uintptr_t)w & 15) == 0) {
-    const int vec = o_stride % 4 == 0 && ((uintptr_t)out & (out_dtype == LEV_F32 ? 15 : 7)) == 0;
+    const int vec = o_stride % 8 == 0 && ((uintptr_t)out & 15) == 0 ? 2 : o_stride % 4 == 0 && ((uintptr_t)out & (out_dtype == LEV_F32 ? 15 : 7)) == 0;
     if (tile_rows == MOE_BIG) {
       const int bn = glu ? MOE_BN / 2 : MOE_BN, n_cols = (F + bn - 1) / bn;
       const long blocks = (long)((max_tiles + 7) / 8) * 8 * n_cols;

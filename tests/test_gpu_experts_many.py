@@ -61,6 +61,33 @@ def test_products_over_tiles_of_128_rows_against_float64(K, Fo, Kd):
     _check(K, [1, 63, 0, 64, 65, 128, 129], Fo, Kd, (Fo, Fo + 3, (Fo + 3) // 4 * 4 + 4))
 
 
+@pytest.mark.parametrize("Fo,Kd", [(520, 512), (640, 576), (1032, 1024), (2048, 128)])
+def test_columns_that_begin_at_places_of_their_own(K, Fo, Kd):
+    """Fewer than two rounds of workgroups: every column of tiles walks K from another step on; (2048, 128) has as many as two rounds with glu."""
+    _check(K, [130, 5, 64, 128], Fo, Kd, (Fo,))
+
+
+@pytest.mark.parametrize("activation", ["none", "gelu_new", "gelu", "relu", "silu", "quick_gelu", "tanh", "relu_squared"])
+def test_every_activation(K, activation):
+    """Against the same sums without one, in float64: an activation's own error is at most 2^-20 of the sum (its slope stays below 1.13; relu_squared's
+    is twice the sum), the 32-bit sums are the same in both."""
+    f = {"none": lambda x: x, "gelu_new": lambda x: F_.gelu(x, approximate="tanh"), "gelu": F_.gelu, "relu": F_.relu, "silu": F_.silu, "tanh": torch.tanh,
+         "quick_gelu": lambda x: x * torch.sigmoid(1.702 * x), "relu_squared": lambda x: F_.relu(x) ** 2}[activation]
+    counts, Fo, Kd = [100, 20], 96, 64
+    g = torch.Generator(device=DEV).manual_seed(5)
+    sp, tiles, meta, _ = _sorted(K, counts)
+    h = torch.randn(sum(counts), Kd, device=DEV, generator=g).bfloat16()
+    for glu in (False, True):
+        w = (torch.randn(2, Fo * (2 if glu else 1), Kd, device=DEV, generator=g) / 6).bfloat16()
+        run = lambda w, act, glu: [K.moe_linear(h, w, out := torch.empty(sum(counts), w.shape[1] // (2 if glu else 1), device=DEV), tiles, meta, sp, top=1, gather=False, glu=glu,
+                                                activation=act, tile_rows=128), out][1]
+        y = run(w, "none", False).double()
+        want = f(y[:, :Fo]) * (y[:, Fo:] if glu else 1)
+        got = run(w, activation, glu).double()
+        bound = 2.0 ** -20 * (1 + y[:, :Fo].abs()) ** 2 * (1 + y[:, Fo:].abs() if glu else 1)
+        assert bool(((got - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("experts", [511, 513, 700])
 def test_more_tiles_than_lanes_a_chiplet(K, experts):
     """Up to 512 tiles a chiplet's larger ones come first, beyond that the list's order holds."""
