@@ -278,19 +278,26 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
 // Runs of several tokens: one workgroup of PF_WAVES waves per (tile of up to PF_ROWS consecutive query tokens, query head,
 // set of value heads). The keys and values of a block of 64 positions are staged once for all waves: global -> registers
 // (requested two blocks ahead, while the blocks before are computed) -> LDS, keys as [HD/8][64][8], values transposed as
-// [value head][VD][64 + 8] with everything beyond the last written key made zero on the way.
+// [value head][VD][64 + 8] with everything beyond the last written key made zero on the way (from the registers, not when they are asked
+// for: that would wait for them).
+// What bounds it: the chain of a block (two barriers, scores, softmax, values) in the workgroups of the longest tiles, few of which share a CU.
+// Two prompts of 1,000, 16 heads of 256 / 224 and of 128 / 64, microseconds a layer: 102 -> 65; three of 1,000, 960 and 90 of 128 / 64: 77 -> 49. What went:
+// waits for loads that had just been asked for (zeros were put in at once), a division and its branches per chunk (now one a block), masks on the
+// scores of blocks that all rows see (most), room for four value heads where there is one (three quarters of the value loads were repeats).
 #define VS_STRIDE 72
 #define RUN_MAX_LDS (80 * 1024)  // bytes a workgroup may take: two workgroups a CU
 #define RUN_PAGES 2048  // page ids of a tile's key range that are kept in LDS
-#define K_STAGE ((HD * 8 + PF_THREADS - 1) / PF_THREADS)        // 16-byte chunks of a key block per thread
-#define V_STAGE ((NVC * VD * 8 + PF_THREADS - 1) / PF_THREADS)  // and of the value blocks
+#define K_STAGE ((HD * 8 + PF_THREADS - 1) / PF_THREADS)  // 16-byte chunks of a key block per thread
 
+// NC: value heads that a wave has room for, as above: 1, or NVC for layers with more
+template <int NC>
 __global__ void __launch_bounds__(PF_THREADS)
 attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, float* __restrict__ out, const bf16_t* __restrict__ k_pages,
                                   const bf16_t* __restrict__ v_pages, const int* __restrict__ positions, const int* __restrict__ token_seq,
                                   const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tiles, int H, int KVH, int NV,
                                   int PS, float scale, int window, int chunk, int keep, float softcap, const float* __restrict__ slopes,
                                   const float* __restrict__ sinks) {
+  constexpr int V_STAGE = (NC * VD * 8 + PF_THREADS - 1) / PF_THREADS;  // 16-byte chunks of the value blocks per thread
   extern __shared__ __attribute__((aligned(16))) unsigned char av_smem[];
   bf16_t* ks = reinterpret_cast<bf16_t*>(av_smem);  // [HD/8][64][8]
   bf16_t* vs = ks + HD * 64;                        // [n_c][VD][VS_STRIDE]
@@ -306,28 +313,38 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
   const int pos = pos0 + (tok - first);         // a run's tokens stand at consecutive positions
   const int lo = lev_first_visible(pos, window, chunk);
   const int p_max_wg = pos0 + n - 1, lo_wg = lev_first_visible(pos0, window, chunk);
-  const int p_max = min(p_max_wg, pos0 + wave * 16 + 15);                                   // this wave's rows
-  const int lo_min = lev_first_visible(pos0 + wave * 16, window, chunk);
+  const int p_min = pos0 + wave * 16, p_max = min(p_max_wg, p_min + 15);                    // this wave's rows
+  const int lo_min = lev_first_visible(p_min, window, chunk), lo_max = lev_first_visible(p_max, window, chunk);
   const int* bt = block_tables + (size_t)token_seq[first] * bt_stride;
   const float slope = slopes ? slopes[head] : 0.f;
-  const int c0 = NV == 1 ? kvh : blockIdx.z * NVC;
-  const int n_c = NV == 1 ? 1 : min(NVC, NV - blockIdx.z * NVC);
+  const int c0 = NV == 1 ? kvh : blockIdx.z * NC;
+  const int n_c = NV == 1 ? 1 : min(NC, NV - blockIdx.z * NC);
   const int key_begin = (lo_wg / 64) * 64;
   // A key's page: from LDS, where the page ids of the tile's whole key range were put once (a look-up in global memory ahead
   // of every operand load would put two memory latencies in a row into every block). Pages are powers of two in practice:
   // a shift then, a division otherwise.
   const int sh = (PS & (PS - 1)) == 0 ? __builtin_ctz(PS) : -1;
-  const int pg0 = sh >= 0 ? key_begin >> sh : key_begin / PS;
-  const int n_pg = (sh >= 0 ? p_max_wg >> sh : p_max_wg / PS) - pg0 + 1;
+  auto block_of = [&](int kp) { return sh >= 0 ? kp >> sh : kp / PS; };
+  const int pg0 = block_of(key_begin), n_pg = block_of(p_max_wg) - pg0 + 1;
   // with kept first positions the tile also reads the n_kept blocks of 64 keys that hold them and lie before key_begin: their
   // page ids stand at the table's start, those of the range from key_begin on behind them
   const int first_block = lo_wg / 64, n_kept = lev_kept_blocks(lo_wg, keep), n_blocks = n_kept + p_max_wg / 64 - first_block + 1;
-  const int n_kpg = n_kept > 0 ? (sh >= 0 ? (n_kept * 64 - 1) >> sh : (n_kept * 64 - 1) / PS) + 1 : 0;
-  for (int i = tid; i < min(n_kpg, RUN_PAGES); i += PF_THREADS) pages_s[i] = bt[i];
-  for (int i = tid; i < min(n_pg, RUN_PAGES - n_kpg); i += PF_THREADS) pages_s[n_kpg + i] = bt[pg0 + i];  // the host sends longer ranges elsewhere
-  auto block_of = [&](int kp) { return sh >= 0 ? kp >> sh : kp / PS; };
-  auto page_of = [&](int kp) {  // kp within the tile's range or among the kept blocks
-    const int b = block_of(kp);
+  const int n_kpg = n_kept > 0 ? block_of(n_kept * 64 - 1) + 1 : 0;
+  int none = 0;  // negative: a page that holds a key in sight is missing
+  for (int i = tid; i < min(n_kpg, RUN_PAGES); i += PF_THREADS) {
+    const int page = bt[i];
+    pages_s[i] = page, none |= i * PS < keep ? page : 0;
+  }
+  for (int i = tid; i < min(n_pg, RUN_PAGES - n_kpg); i += PF_THREADS) {  // the host sends longer ranges elsewhere
+    const int page = bt[pg0 + i];
+    pages_s[n_kpg + i] = page, none |= (pg0 + i + 1) * PS > lo_wg ? page : 0;
+  }
+  // The page of a key of the block at key0 (within the tile's range or among the kept blocks) and the key's place in it, from the number and the
+  // first key of the page that key0 lies in (one division a block). The distance from there is below PS + 64: its quotient in 16 bits is exact.
+  const int sixteenths = PS < 64 ? (65536 + PS - 1) / PS : 0;
+  auto place_of = [&](int kp, int page_no, int page_key, int& at) {
+    const int r = kp - page_key, over = PS < 64 ? r * sixteenths >> 16 : r >= PS, b = page_no + over;
+    at = r - over * PS;
     return pages_s[b >= pg0 ? n_kpg + b - pg0 : b];
   };
 
@@ -338,43 +355,44 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
     if (valid && 32 * s + 8 * g < HD)
       qf[s] = *reinterpret_cast<const u32x4*>(q + (size_t)tok * q_stride + (size_t)head * HD + 32 * s + 8 * g);
   }
-  f32x4 o[NVC][NDT];
+  f32x4 o[NC][NDT];
 #pragma unroll
-  for (int c = 0; c < NVC; ++c)
+  for (int c = 0; c < NC; ++c)
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) o[c][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
   constexpr float LOG2E = 1.4426950408889634f;
   const size_t k_head = (size_t)HD * PS, v_head = (size_t)VD * PS;
-  __syncthreads();  // the page ids are there
+  const bool all_pages = __syncthreads_or(none < 0) == 0;  // the page ids are there, and every key in sight has a page
 
   u32x4 kst_a[K_STAGE], vst_a[V_STAGE], kst_b[K_STAGE], vst_b[V_STAGE];  // two blocks on their way at any time
-  // this thread's chunks of the block at key0, from the pages into registers
+  // This thread's chunks of the block at key0, from the pages into registers: chunks of one key, and of one group of 8 keys' values.
   // Every load stands under no condition (a load in a branch makes the compiler wait for all loads in flight where the
-  // branch ends): addresses are clamped into what can be read, what must not count is made zero afterwards.
-  auto fetch = [&](int key0, u32x4* kst, u32x4* vst) {
+  // branch ends): addresses are clamped into what can be read, what must not count is made zero when it goes to LDS.
+  auto fetch = [&](int key0, u32x4 (&kst)[K_STAGE], u32x4 (&vst)[V_STAGE]) {
+    const int page_no = block_of(key0), page_key = page_no * PS;
+    int ka, va;
+    const int kpage = place_of(min(key0 + (tid & 63), p_max_wg), page_no, page_key, ka);
+    const int vpage = place_of(min(key0 + 8 * (tid & 7), p_max_wg & ~7), page_no, page_key, va);
+    const bf16_t* kb = k_pages + ((size_t)max(kpage, 0) * KVH + kvh) * k_head + (size_t)ka * 8;
+    const bf16_t* vb = v_pages + ((size_t)max(vpage, 0) * KVH + c0) * v_head + va;
 #pragma unroll
-    for (int i = 0; i < K_STAGE; ++i) {
-      const int ci = min(tid + PF_THREADS * i, HD * 8 - 1);  // (chunk of 8 dims, key)
-      const int kp = key0 + (ci & 63), kpc = min(kp, p_max_wg);
-      const int page = page_of(kpc);
-      const u32x4 v = *reinterpret_cast<const u32x4*>(k_pages + ((size_t)max(page, 0) * KVH + kvh) * k_head +
-                                                      ((size_t)(ci >> 6) * PS + (kpc - block_of(kpc) * PS)) * 8);
-      const uint32_t keep = (kp <= p_max_wg && page >= 0) ? 0xffffffffu : 0u;
-      kst[i] = u32x4{v[0] & keep, v[1] & keep, v[2] & keep, v[3] & keep};
-    }
+    for (int i = 0; i < K_STAGE; ++i) kst[i] = *reinterpret_cast<const u32x4*>(kb + min((tid >> 6) + PF_THREADS / 64 * i, HD / 8 - 1) * PS * 8);
 #pragma unroll
-    for (int i = 0; i < V_STAGE; ++i) {
-      const int ci = min(tid + PF_THREADS * i, n_c * VD * 8 - 1);  // (value head, dim, group of 8 keys)
-      const int kp = key0 + 8 * (ci & 7), row = ci >> 3;         // row = c * VD + dim
-      const int kpc = min(kp, p_max_wg & ~7);
-      const int page = page_of(kpc);
-      const u32x4 v = *reinterpret_cast<const u32x4*>(v_pages + ((size_t)max(page, 0) * KVH + c0 + row / VD) * v_head +
-                                                      (size_t)(row % VD) * PS + (kpc - block_of(kpc) * PS));
-      vst[i] = first_keys(v, page >= 0 ? min(8, max(0, p_max_wg - kp + 1)) : 0);
-    }
+    for (int i = 0; i < V_STAGE; ++i) vst[i] = *reinterpret_cast<const u32x4*>(vb + (size_t)min((tid >> 3) + PF_THREADS / 8 * i, n_c * VD - 1) * PS);
   };
-  auto stage = [&](const u32x4* kst, const u32x4* vst) {
+  auto stage = [&](int key0, u32x4 (&kst)[K_STAGE], u32x4 (&vst)[V_STAGE]) {
+    if (!all_pages || key0 + 63 > p_max_wg || !(key0 >= lo_wg || key0 + 63 < keep)) {  // keys without values: the same for the whole workgroup
+      const int page_no = block_of(key0), page_key = page_no * PS, kp = key0 + (tid & 63), vp = key0 + 8 * (tid & 7);
+      int at;
+      const bool in = kp <= p_max_wg && place_of(min(kp, p_max_wg), page_no, page_key, at) >= 0;
+      const int count = place_of(min(vp, p_max_wg & ~7), page_no, page_key, at) >= 0 ? min(8, max(0, p_max_wg - vp + 1)) : 0;
+#pragma unroll
+      for (int i = 0; i < K_STAGE; ++i)
+        if (!in) kst[i] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int i = 0; i < V_STAGE; ++i) vst[i] = first_keys(vst[i], count);
+    }
 #pragma unroll
     for (int i = 0; i < K_STAGE; ++i) {
       const int ci = tid + PF_THREADS * i;
@@ -395,22 +413,15 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
     // the register sets take turns: this block's goes to LDS and is asked for again two blocks ahead (conditions uniform
     // over the workgroup)
     if (it & 1) {
-      stage(kst_b, vst_b);
+      stage(key0, kst_b, vst_b);
       lds_barrier();
       if (it + 2 < n_blocks) fetch(lev_block_key(it + 2, n_kept, first_block), kst_b, vst_b);
     } else {
-      stage(kst_a, vst_a);
+      stage(key0, kst_a, vst_a);
       lds_barrier();
       if (it + 2 < n_blocks) fetch(lev_block_key(it + 2, n_kept, first_block), kst_a, vst_a);
     }
     if (!active || key0 > p_max || (key0 + 63 < lo_min && key0 >= keep)) continue;  // none of this wave's rows sees a key of this block
-    int pgv[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int kp = key0 + 32 * u + 8 * g;
-      const int page = page_of(min(kp, p_max_wg));
-      pgv[u] = kp <= p_max ? page : -1;
-    }
     f32x4 st[2][2];
 #pragma unroll
     for (int u = 0; u < 2; ++u)
@@ -426,22 +437,39 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
         }
         st[u][hh] = acc;
       }
+    // scale, cap, distance term; in base 2 from here on
     float mx = -INFINITY;
+    const float dist0 = (float)(pos - key0 - 8 * g);  // whole numbers: exact
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float far = dist0 - (float)(32 * u + 4 * hh + r);
+          if (softcap > 0.f) st[u][hh][r] = fmaf(-slope, far, softcap * fast_tanh(st[u][hh][r] * scale * __builtin_amdgcn_rcpf(softcap))) * LOG2E;
+          else st[u][hh][r] = fmaf(st[u][hh][r], scale, -(slope * far)) * LOG2E;
+        }
+      }
+    if (!all_pages || key0 + 63 > p_min || !(key0 >= lo_max || key0 + 63 < keep)) {  // a row that does not see every key: the same for the whole wave
+      const int page_no = block_of(key0), page_key = page_no * PS;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int kg = key0 + 32 * u + 8 * g;
+        int at;
+        const bool there = valid && kg <= p_max && place_of(min(kg, p_max_wg), page_no, page_key, at) >= 0;
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) st[u][hh][r] = there && lev_key_visible(kg + 4 * hh + r, pos, lo, keep) ? st[u][hh][r] : -INFINITY;
+      }
+    }
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int kp = key0 + 32 * u + 8 * g + 4 * hh + r;
-          const bool ok = valid && lev_key_visible(kp, pos, lo, keep) && pgv[u] >= 0;
-          float sc = st[u][hh][r] * scale;
-          if (softcap > 0.f) sc = softcap * fast_tanh(sc * __builtin_amdgcn_rcpf(softcap));
-          sc = (sc - slope * (float)(pos - kp)) * LOG2E;
-          sc = ok ? sc : -INFINITY;
-          st[u][hh][r] = sc;
-          mx = fmaxf(mx, sc);
-        }
+        for (int r = 0; r < 4; ++r) mx = fmaxf(mx, st[u][hh][r]);
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     const float m_new = fmaxf(m, mx);
@@ -457,7 +485,9 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
       for (int hh = 0; hh < 2; ++hh)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          p[4 * hh + r] = __builtin_amdgcn_exp2f(st[u][hh][r] - m_use);
+#pragma clang fp contract(off)  // the rounded score, as the maximum holds it
+          const float below = st[u][hh][r] - m_use;
+          p[4 * hh + r] = __builtin_amdgcn_exp2f(below);
           psum += p[4 * hh + r];
         }
 #pragma unroll
@@ -465,8 +495,8 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
     }
     l = l * corr + psum;
 #pragma unroll
-    for (int c = 0; c < NVC; ++c) {
-      if (c < n_c) {
+    for (int c = 0; c < NC; ++c) {
+      if (c == 0 || c < n_c) {
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt) {
           f32x4 acc = o[c][dt] * corr;
@@ -486,7 +516,7 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
   if (sinks != nullptr) l = m == -INFINITY ? 1.0f : l + __builtin_amdgcn_exp2f(sinks[head] * LOG2E - m);  // m is in base 2
   const float inv = l > 0.f ? 1.0f / l : 0.f;
 #pragma unroll
-  for (int c = 0; c < NVC; ++c) {
+  for (int c = 0; c < NC; ++c) {
     if (c < n_c) {
       float* ob = out + (((size_t)tok * H + head) * NV + (NV == 1 ? 0 : c0 + c)) * VD;
 #pragma unroll
@@ -573,13 +603,19 @@ extern "C" int lev_attention_values_mfma(const void* q, long q_stride, float* ou
     reach += PF_ROWS + 64 + (keep > 0 ? keep + 64 + PS : 0);
     const size_t all_lds = lds + RUN_PAGES * sizeof(int);
     if (all_lds > 64 * 1024 && all_lds <= RUN_MAX_LDS) {  // more than a kernel gets unasked
-      hipError_t e = hipFuncSetAttribute((const void*)attention_values_mfma_runs_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      hipError_t e = hipFuncSetAttribute(NV == 1 ? (const void*)attention_values_mfma_runs_kernel<1> : (const void*)attention_values_mfma_runs_kernel<NVC>,
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
       LEV_REQUIRE(e == hipSuccess, "attention: %zu bytes of LDS a workgroup: %s", all_lds, hipGetErrorString(e));
     }
-    if (all_lds <= RUN_MAX_LDS && reach / PS + 2 <= RUN_PAGES)
-      attention_values_mfma_runs_kernel<<<grid, PF_THREADS, lds, stream>>>((const bf16_t*)q, q_stride, out, (const bf16_t*)k_pages,
-                                                                         (const bf16_t*)v_pages, positions, token_seq, block_tables,
-                                                                         bt_stride, tiles, H, KVH, NV, PS, scale, window, chunk, keep, softcap, slopes, sinks);
+#define AV_RUNS(NC)                                                                                                                                    \
+  attention_values_mfma_runs_kernel<NC><<<grid, PF_THREADS, lds, stream>>>((const bf16_t*)q, q_stride, out, (const bf16_t*)k_pages, (const bf16_t*)v_pages, \
+                                                                           positions, token_seq, block_tables, bt_stride, tiles, H, KVH, NV, PS, scale, window, \
+                                                                           chunk, keep, softcap, slopes, sinks)
+    if (all_lds <= RUN_MAX_LDS && reach / PS + 2 <= RUN_PAGES) {
+      if (NV == 1) AV_RUNS(1);
+      else AV_RUNS(NVC);
+    }
+#undef AV_RUNS
     else  // the longest ranges: every wave by itself, operands straight from the pages
       AV_ROOMS(false, dim3(n_tiles * SUB_TILES, H, chunks), tiles, 1, nullptr, nullptr);
     if (lev_check_launch("attention_values_mfma (runs)")) return -1;
