@@ -5,15 +5,35 @@
 
 typedef __attribute__((ext_vector_type(4))) float gf_f32x4;
 
+// four neighbouring outputs of a row
+__device__ __forceinline__ void gemm_f32_store(gf_f32x4 v, const float* bias, const float* residual, long ldr, float* out, long ldo, int m, int o, int N, int act, int vec) {
+  if (vec && o + 4 <= N) {
+    if (bias) v += *reinterpret_cast<const gf_f32x4*>(bias + o);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = lev_activate(v[r], act);
+    if (residual) v += *reinterpret_cast<const gf_f32x4*>(residual + (size_t)m * ldr + o);
+    *reinterpret_cast<gf_f32x4*>(out + (size_t)m * ldo + o) = v;
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (o + r >= N) break;
+      float x = v[r];
+      if (bias) x += bias[o + r];
+      x = lev_activate(x, act);
+      if (residual) x += residual[(size_t)m * ldr + o + r];
+      out[(size_t)m * ldo + o + r] = x;
+    }
+  }
+}
+
 // A workgroup of W waves owns 16 RT rows and 16 NT outputs; its waves split K (steps of 16 dealt in stretches) and the partial sums are
 // added through LDS in wave order. The product is transposed, out^T = w a^T, so that a lane ends with four neighbouring outputs of one
 // row. Both operands come straight from global memory, 16 bytes a lane (row = lane % 16, k = 4 (lane / 16) + j for the j-th of the
 // four products of a step): the 32-bit instruction takes 32 cycles for 1,024 multiply-adds, which hides much of what such loads cost
-// the vector cache (a look-up for every lane); whole lines turned into operands in LDS, as the bfloat16 kernels read them, have not been tried.
+// the vector cache (a look-up for every lane).
 // What bounds it: few rows, the read of the weights (4096 x 4096 at 4 rows 14.3 us, 4.7 TB/s; 768 x 768 4.8 us, a launch and a chain of
-// loads); some hundred rows, L2 at about 9.5 TB/s (1024 x 4096 at 203 rows 33 us) or the last round of tiles; many, the matrix pipe
-// (4096 x 4096 at 2,048 rows 532 us, 129 TFLOP/s of 157). The plain kernel of gemm_simple.hip (64 x 64 tiles, vector ALU, scalar loads)
-// took 84 us for 768 x 768 at 4 rows, 378 us for 768 x 3072, 2,417 us for 50257 x 1024 at 777 rows (now 4.8, 10 and 727).
+// loads); some hundred rows, L2 at about 9.5 TB/s (1024 x 4096 at 203 rows 33 us) or the last round of tiles. The plain kernel of
+// gemm_simple.hip (64 x 64 tiles, vector ALU, scalar loads) took 84 us for 768 x 768 at 4 rows, 378 us for 768 x 3072 (now 4.8 and 10).
 template <int RT, int NT, int W>
 __global__ void __launch_bounds__(64 * W)
 gemm_f32_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
@@ -118,51 +138,184 @@ gemm_f32_kernel(const float* __restrict__ a, long lda, const float* __restrict__
         for (int q = 0; q < W; ++q) v += *reinterpret_cast<const gf_f32x4*>(gf_part + ((size_t)(q * RT * NT + t) * 64 + lane) * 4);
       }
       const int m = m0 + 16 * i + col, o = o0 + 16 * j + 4 * g;
-      if (m >= M || o >= N) continue;
-      if (vec && o + 4 <= N) {
-        if (bias) v += *reinterpret_cast<const gf_f32x4*>(bias + o);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = lev_activate(v[r], act);
-        if (residual) v += *reinterpret_cast<const gf_f32x4*>(residual + (size_t)m * ldr + o);
-        *reinterpret_cast<gf_f32x4*>(out + (size_t)m * ldo + o) = v;
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          if (o + r >= N) break;
-          float x = v[r];
-          if (bias) x += bias[o + r];
-          x = lev_activate(x, act);
-          if (residual) x += residual[(size_t)m * ldr + o + r];
-          out[(size_t)m * ldo + o + r] = x;
-        }
-      }
+      if (m < M && o < N) gemm_f32_store(v, bias, residual, ldr, out, ldo, m, o, N, act, vec);
     }
   }
 }
 
-// Which tile: the fewest microseconds by an estimate from what was measured over 15 weights and 1 .. 2,048 rows (all eight tiles of the list):
-// a launch and its ramp of 4 us, and the longest of the weights' read from memory (5.2 TB/s), the operands that a CU pulls through
-// its L2 (37 GB/s and CU) and the products of the CU with the most workgroups (waves that fewer than four SIMDs hold leave the others idle).
-// Within 10 % of the best tile at nearly all of them; the ends: 16 x 16 for 768 x 768 at 4 rows (4.8 us; 64 x 64 19), 64 x 128 for
-// 4096 x 4096 at 2,048 rows (532 us; 16 x 16 1,790).
+// Some hundred rows and more: a workgroup of four waves (2 x 2) owns 32 RT rows and 32 NT outputs, a wave 16 RT x 16 NT of them over the whole
+// of K. Both operands come as whole lines (32 numbers of a row a step, the step after next on its way in registers) and are turned into the
+// instruction's operands by two buffers in LDS, rows of 36 numbers: 16 lanes' reads of 16 bytes fall on all banks. A load's four products of a tile
+// go to SETS sums in turn (so many that none waits for the one before it), which join the tile's sum every 128 or 256 k: no chain of roundings is
+// longer than those of the kernel above (errors against 64 bits at 777 rows: K = 1,024 2.1e-7, before 2.9e-7; 4,096 2.1e-7, before 5.7e-7).
+// What bounds it: the matrix pipe (64 x 128 tiles, 4096 x 4096 at 2,048 rows 495 us, 139 TFLOP/s; before 531), of some hundred rows the last round of
+// tiles. A mask on the chunks in the loop cost it 15 %: it waited for loads that had just gone out.
+#define GF_LD 36
+template <int RT, int NT, int SETS>
+__global__ void __launch_bounds__(256, RT * NT > 8 ? 1 : 2)
+gemm_f32_tile_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias, const float* residual, long ldr,
+                     float* out, long ldo, int M, int N, int K, int act, int n_rows, int n_cols, int vec) {
+  constexpr int BM = 32 * RT, BN = 32 * NT, PIECE = SETS == 1 ? 4 : 8;  // steps whose products are added up before they join the sum
+  __shared__ __attribute__((aligned(16))) float sm[2][BM + BN][GF_LD];  // rows of a, then of w
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, g = lane >> 4, wm = wave >> 1, wn = wave & 1;
+  const int n_tiles = n_rows * n_cols, per = (n_tiles + 7) / 8;  // neighbouring columns of tiles on a chiplet, as above
+  const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= per || tile >= n_tiles) return;  // the whole workgroup
+  const int m0 = (tile % n_rows) * BM, o0 = (tile / n_rows) * BN;
+  const int row = tid >> 3, kc = (tid & 7) * 4;
+  const float* src[RT + NT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) src[i] = a + (size_t)min(m0 + 32 * i + row, M - 1) * lda;  // rows beyond the matrix: read again, never stored
+#pragma unroll
+  for (int j = 0; j < NT; ++j) src[RT + j] = w + (size_t)min(o0 + 32 * j + row, N - 1) * K;
+  gf_f32x4 ahead[2][RT + NT];
+  // the steps in the order they are taken: a partial one (K % 32 != 0) first, so that the loop needs no masks (one there waits for its load)
+  const int tail = K % 32, steps = (K + 31) / 32;
+  auto fetch = [&](gf_f32x4 (&to)[RT + NT], int t) {  // t >= 1; beyond the end: loaded again, not used
+    const int k = min(max(min(t, steps - 1) - (tail ? 1 : 0), 0) * 32 + kc, K - 4);
+#pragma unroll
+    for (int i = 0; i < RT + NT; ++i) to[i] = *reinterpret_cast<const gf_f32x4*>(src[i] + k);
+  };
+  auto stage = [&](gf_f32x4 (&from)[RT + NT], int buf) {
+#pragma unroll
+    for (int i = 0; i < RT + NT; ++i) *reinterpret_cast<gf_f32x4*>(&sm[buf][32 * i + row][kc]) = from[i];
+  };
+  gf_f32x4 sum[RT][NT], acc[SETS][RT][NT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      sum[i][j] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < SETS; ++e) acc[e][i][j] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  auto settle = [&]() {
+#pragma unroll
+    for (int e = 0; e < SETS; ++e)
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) sum[i][j] += acc[e][i][j], acc[e][i][j] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  gf_f32x4 av[2][RT], wv[2][NT];
+  auto read = [&](int set, int buf, int half) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i) av[set][i] = *reinterpret_cast<const gf_f32x4*>(&sm[buf][16 * (wm * RT + i) + col][16 * half + 4 * g]);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) wv[set][j] = *reinterpret_cast<const gf_f32x4*>(&sm[buf][BM + 16 * (wn * NT + j) + col][16 * half + 4 * g]);
+  };
+  auto products = [&](int half) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          gf_f32x4& c = acc[(4 * half + e) % SETS][i][j];
+          c = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[half][j][e], av[half][i][e], c, 0, 0, 0);
+        }
+  };
+  const int k0 = (tail ? K - tail : 0) + kc;
+#pragma unroll
+  for (int i = 0; i < RT + NT; ++i) ahead[0][i] = *reinterpret_cast<const gf_f32x4*>(src[i] + min(k0, K - 4));
+  fetch(ahead[1], 1);
+  if (k0 >= K)  // chunks beyond K count as zeros
+#pragma unroll
+    for (int i = 0; i < RT + NT; ++i) ahead[0][i] = gf_f32x4{0.f, 0.f, 0.f, 0.f};
+  stage(ahead[0], 0);
+  lds_barrier();
+  read(0, 0, 0);
+  // Step t: step t + 1 goes to the other buffer and step t + 2 is asked for between the first half's products, the operands of a half are read
+  // while those of the half before are multiplied. The barrier in the middle: the other buffer is whole, this one has been read.
+  auto step = [&](int t, int buf) {
+    constexpr int NM = 4 * RT * NT, NR = RT + NT;
+    read(1, buf, 1);
+    products(0);
+    stage(ahead[buf ^ 1], buf ^ 1);  // behind the last step: numbers that nobody uses
+    fetch(ahead[buf], t + 2);
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {  // the order of issue: a product, then at most a few of the others
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+#pragma unroll
+      for (int o = m * 3 * NR / NM; o < (m + 1) * 3 * NR / NM; ++o) {
+        if (o < NR) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        else if (o < 2 * NR) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+        else __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+      }
+    }
+    lds_barrier();
+    read(0, buf ^ 1, 0);
+    products(1);
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+#pragma unroll
+      for (int o = m * NR / NM; o < (m + 1) * NR / NM; ++o) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+  };
+  int t = 0;
+  while (t + 1 < steps) {
+    const int stop = min(t + PIECE, steps - 1);
+    for (; t < stop; t += 2) {
+      step(t, 0);
+      step(t + 1, 1);
+    }
+    settle();
+  }
+  if (t < steps) {
+    step(t, 0);
+    settle();
+  }
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int m = m0 + 16 * (wm * RT + i) + col, o = o0 + 16 * (wn * NT + j) + 4 * g;
+      if (m < M && o < N) gemm_f32_store(sum[i][j], bias, residual, ldr, out, ldo, m, o, N, act, vec);
+    }
+  }
+}
+
+// Which tile: the fewest microseconds by an estimate from what was measured over 14 weights and 17 .. 2,048 rows (all tiles of both lists).
+// Of the first kernel: the longest of the weights' read from memory (5.2 TB/s), the operands that a CU pulls through its L2 (37 GB/s and CU) and
+// the products of the CU with the most workgroups (waves that fewer than four SIMDs hold leave the others idle). Of the second: its steps on that
+// CU. Within 8 % of the best tile at nearly all of them; the ends: 16 x 16 for 768 x 768 at 4 rows (4.8 us; 64 x 64 19), 64 x 128 of the second for
+// 4096 x 4096 at 2,048 rows (495 us; 16 x 16 of the first 1,790). With the second kernel, before / after: 3072 x 1024 at 777 rows 61 / 48 us, 4096 x 1024
+// 75 / 66, 1024 x 1024 25 / 22, 1024 x 4096 78 / 73, 50257 x 1024 733 / 625, 3072 x 768 at 606 rows 41 / 30, 4096 x 4096 at 404 rows 173 / 133. Below about 100 rows
+// and for long sums into few outputs the first stays ahead: its waves split K (1024 x 4096 at 203 rows 33 us, the second 46).
 struct GemmF32Tile {
   int rt, nt, w;
-  float pipe;  // share of the matrix pipe that the tile reaches
+  float pipe;   // share of the matrix pipe that the tile reaches
+  float start;  // microseconds before and behind the products that smaller tiles do not have
 };
-static const GemmF32Tile GEMM_F32_TILES[] = {{1, 1, 8, 0.8f}, {2, 1, 8, 0.8f}, {1, 2, 8, 0.8f}, {1, 4, 8, 0.8f}, {2, 2, 4, 0.8f}, {2, 4, 4, 0.8f}, {4, 4, 4, 0.68f}, {4, 8, 2, 0.85f}};
+static const GemmF32Tile GEMM_F32_TILES[] = {{1, 1, 8, 0.8f, 0.f}, {2, 1, 8, 0.8f, 0.f}, {1, 2, 8, 0.8f, 0.f}, {1, 4, 8, 0.8f, 0.f}, {2, 2, 4, 0.8f, 0.f}, {2, 4, 4, 0.8f, 0.f}, {4, 4, 4, 0.85f, 7.f}};
+struct GemmF32LineTile {
+  int rt, nt, sets;
+  float alone, among;  // microseconds of a step: of the one workgroup on a CU, and of one among several
+  float start;
+};
+static const GemmF32LineTile GEMM_F32_LINE_TILES[] = {{1, 1, 4, 0.32f, 0.155f, 0.f},  {1, 2, 2, 0.37f, 0.28f, 0.5f}, {1, 3, 2, 0.44f, 0.395f, 1.f},
+                                                      {2, 2, 1, 0.6f, 0.5f, 1.f},     {2, 3, 1, 0.76f, 0.73f, 2.f},  {2, 4, 1, 0.98f, 0.96f, 2.5f}};
+#define GEMM_F32_N_TILES (int)(sizeof(GEMM_F32_TILES) / sizeof(GEMM_F32_TILES[0]))
 
-static int gemm_f32_choose(int M, int N, int K) {
+static int gemm_f32_choose(int M, int N, int K) {  // an index into the first list, or behind its end into the second
   int best = 0;
   double best_us = 1e30;
-  for (int i = 0; i < (int)(sizeof(GEMM_F32_TILES) / sizeof(GEMM_F32_TILES[0])); ++i) {
+  const double memory = 4.0 * N * K / 5.2e6;
+  for (int i = 0; i < GEMM_F32_N_TILES; ++i) {
     const GemmF32Tile& t = GEMM_F32_TILES[i];
     const double groups = (double)((M + 16 * t.rt - 1) / (16 * t.rt)) * ((N + 16 * t.nt - 1) / (16 * t.nt));
     const double n = ceil(groups / 256.0), waves = n * t.w < 4.0 ? n * t.w : 4.0;
-    const double memory = 4.0 * N * K / 5.2e6;
     const double l2 = n * ((16 * t.rt < M ? 16 * t.rt : M) + 16 * t.nt) * 4.0 * K / 37e3;
     const double pipe = n * (K / 4.0) * t.rt * t.nt * 32.0 / waves / (2400.0 * t.pipe);
-    const double us = fmax(memory, fmax(l2, pipe));
+    const double us = t.start + fmax(memory, fmax(l2, pipe));
     if (us < best_us) best_us = us, best = i;
+  }
+  for (int i = 0; i < (int)(sizeof(GEMM_F32_LINE_TILES) / sizeof(GEMM_F32_LINE_TILES[0])); ++i) {
+    const GemmF32LineTile& t = GEMM_F32_LINE_TILES[i];
+    const double n = ceil((double)((M + 32 * t.rt - 1) / (32 * t.rt)) * ((N + 32 * t.nt - 1) / (32 * t.nt)) / 256.0);
+    const double us = t.start + fmax(memory, (K + 31) / 32 * fmax(t.alone + 0.15 * (n - 1) * t.among, n * t.among));
+    if (us < best_us) best_us = us, best = GEMM_F32_N_TILES + i;
   }
   return best;
 }
@@ -172,13 +325,17 @@ int lev_gemm_f32(const float* a, long lda, const float* w, const float* bias, co
                  int act, hipStream_t stream) {
   if (K % 4 != 0 || lda % 4 != 0 || ((uintptr_t)a & 15) != 0 || ((uintptr_t)w & 15) != 0) return 1;
   const int vec = ldo % 4 == 0 && ((uintptr_t)out & 15) == 0 && (!bias || ((uintptr_t)bias & 15) == 0) && (!residual || (ldr % 4 == 0 && ((uintptr_t)residual & 15) == 0));
-  const GemmF32Tile& t = GEMM_F32_TILES[gemm_f32_choose(M, N, K)];
-  const int n_rows = (M + 16 * t.rt - 1) / (16 * t.rt), n_cols = (N + 16 * t.nt - 1) / (16 * t.nt);
+  const int choice = gemm_f32_choose(M, N, K), line = choice - GEMM_F32_N_TILES;
+  const int rt = line < 0 ? GEMM_F32_TILES[choice].rt : 2 * GEMM_F32_LINE_TILES[line].rt, nt = line < 0 ? GEMM_F32_TILES[choice].nt : 2 * GEMM_F32_LINE_TILES[line].nt;
+  const int n_rows = (M + 16 * rt - 1) / (16 * rt), n_cols = (N + 16 * nt - 1) / (16 * nt);
   const long blocks = ((long)n_rows * n_cols + 7) / 8 * 8;
   LEV_REQUIRE(blocks <= 0x7fffffffL, "linear: too many tiles (%ld)", blocks);
 #define GEMM_F32_CASE(RT, NT, W)                                                                                                                    \
-  if (t.rt == RT && t.nt == NT)                                                                                                                     \
+  if (line < 0 && rt == RT && nt == NT)                                                                                                             \
     gemm_f32_kernel<RT, NT, W><<<(unsigned)blocks, 64 * W, W * RT * NT * 1024, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act, n_rows, n_cols, vec)
+#define GEMM_F32_LINE_CASE(RT, NT, SETS)                                                                                                            \
+  if (rt == 2 * RT && nt == 2 * NT)                                                                                                                 \
+    gemm_f32_tile_kernel<RT, NT, SETS><<<(unsigned)blocks, 256, 0, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act, n_rows, n_cols, vec)
   GEMM_F32_CASE(1, 1, 8);
   else GEMM_F32_CASE(2, 1, 8);
   else GEMM_F32_CASE(1, 2, 8);
@@ -186,7 +343,13 @@ int lev_gemm_f32(const float* a, long lda, const float* w, const float* bias, co
   else GEMM_F32_CASE(2, 2, 4);
   else GEMM_F32_CASE(2, 4, 4);
   else GEMM_F32_CASE(4, 4, 4);
-  else GEMM_F32_CASE(4, 8, 2);
+  else GEMM_F32_LINE_CASE(1, 1, 4);
+  else GEMM_F32_LINE_CASE(1, 2, 2);
+  else GEMM_F32_LINE_CASE(1, 3, 2);
+  else GEMM_F32_LINE_CASE(2, 2, 1);
+  else GEMM_F32_LINE_CASE(2, 3, 1);
+  else GEMM_F32_LINE_CASE(2, 4, 1);
+#undef GEMM_F32_LINE_CASE
 #undef GEMM_F32_CASE
   return lev_check_launch("linear (32-bit)");
 }

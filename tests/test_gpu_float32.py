@@ -24,6 +24,10 @@ def _rand(*shape, seed=0):
 # 16 x 32 and (15, 264, 11531) 16 x 64.
 LINEAR = [(1, 4, 1), (1, 64, 50), (3, 768, 768), (16, 100, 48), (17, 772, 33), (31, 1024, 130), (33, 20, 65), (64, 256, 4096), (65, 300, 1024), (129, 1028, 257),
           (203, 516, 1000), (400, 128, 1030), (777, 260, 1024), (1031, 96, 3000), (15, 264, 11531), (13, 264, 50257), (5, 6, 40), (70, 333, 129)]
+# the tiles whose operands come through LDS (32 x 32, 32 x 64, 32 x 96, 64 x 64, 64 x 96, 64 x 128): ends inside a tile, K of one step, with a short one, of
+# odd and even numbers of steps, of pieces of 128 and 256 and one step more
+LINEAR += [(404, 768, 3072), (289, 100, 2051), (1031, 32, 3001), (801, 1028, 1030), (777, 300, 3072), (2047, 292, 4097), (609, 516, 2310), (2047, 260, 2310),
+           (1000, 260, 4097), (1030, 1028, 4100), (2047, 516, 3071)]
 
 
 @pytest.mark.parametrize("M,Ki,N", LINEAR)
