@@ -173,7 +173,7 @@ norm_reg_kernel(float* __restrict__ x, const float* __restrict__ w, const float*
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
-    mean = block_sum<NT>(s, red) / (float)D;
+    mean = block_sum<NT, true>(s, red) / (float)D;
   }
   float s2 = 0.f;
 #pragma unroll
@@ -184,7 +184,7 @@ norm_reg_kernel(float* __restrict__ x, const float* __restrict__ w, const float*
       s2 += (c0 * c0 + c1 * c1) + (c2 * c2 + c3 * c3);
     }
   }
-  const float var = block_sum<NT>(s2, red) / (float)D;
+  const float var = block_sum<NT, true>(s2, red) / (float)D;
   const float rstd = 1.0f / sqrtf(var + eps);
   TO* o = out + (size_t)r * D;
 #pragma unroll

@@ -33,9 +33,9 @@ __device__ __forceinline__ void group_inverse_rms(const float (&v)[PER], const i
     s = wave_sum(s);
     if (lane == 0) part[wave * G + g] = s;
   }
-  __syncthreads();
+  lds_barrier();  // the row's own loads and stores are not waited for
   if (tid < G) total[tid] = 1.0f / sqrtf(((part[tid] + part[G + tid]) + (part[2 * G + tid] + part[3 * G + tid])) * inv_n + eps);
-  __syncthreads();
+  lds_barrier();
 }
 
 template <typename TG, typename TO, int PER>
@@ -49,18 +49,31 @@ group_norm_step_kernel(float* __restrict__ x, const float* __restrict__ y, const
   const int r = blockIdx.x, row = rows ? rows[r] : r;
   const int group_size = D / G;
   const float inv_n = 1.0f / (float)group_size;
-  float xv[PER], z[PER], pw[PER], wv[PER];
+  float xv[PER], z[PER] = {}, pw[PER] = {}, wv[PER] = {};
   int gid[PER];  // the group of each of this thread's elements; -1 beyond the row
-  // every load of the row is asked for before anything is computed: the kernel is a chain of a few memory latencies otherwise
+  // every load of the row is asked for before anything is computed: the kernel is a chain of a few memory latencies otherwise (with the gate and
+  // the zeros beyond the row in the loop of the loads, every turn of it waited for its own)
+  float gt[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) xv[i] = x[(size_t)row * D + min(tid + GN_NT * i, D - 1)];
+  if (y != nullptr)
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int ec = min(tid + GN_NT * i, D - 1);
+      z[i] = y[(size_t)row * D + ec], pw[i] = post_w[ec];
+    }
+  if (h_out != nullptr && w != nullptr)
+#pragma unroll
+    for (int i = 0; i < PER; ++i) wv[i] = w[min(tid + GN_NT * i, D - 1)];
+  if (gate != nullptr) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) gt[i] = to_float<TG>(gate[(size_t)row * gate_stride + min(tid + GN_NT * i, D - 1)]);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) z[i] = z[i] / (1.0f + expf(-gt[i]));
+  }
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
-    const int e = tid + GN_NT * i, ec = min(e, D - 1);
-    xv[i] = x[(size_t)row * D + ec];
-    z[i] = y != nullptr ? y[(size_t)row * D + ec] : 0.f;
-    pw[i] = y != nullptr ? post_w[ec] : 0.f;
-    wv[i] = (h_out != nullptr && w != nullptr) ? w[ec] : 0.f;
-    const float gt = gate != nullptr ? to_float<TG>(gate[(size_t)row * gate_stride + ec]) : 0.f;
-    if (gate != nullptr) z[i] = z[i] / (1.0f + expf(-gt));
+    const int e = tid + GN_NT * i;
     if (e >= D) xv[i] = 0.f, z[i] = 0.f;
     gid[i] = e < D ? e / group_size : -1;
   }
@@ -88,7 +101,7 @@ group_norm_step_kernel(float* __restrict__ x, const float* __restrict__ y, const
         if (rows == nullptr) x[(size_t)row * D + e] = xv[i];
       }
     }
-    __syncthreads();  // the groups' sums are read before the next use of the scratch arrays
+    lds_barrier();  // the groups' sums are read before the next use of the scratch arrays
   }
   if (h_out != nullptr && w == nullptr) {
 #pragma unroll

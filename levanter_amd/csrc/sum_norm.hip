@@ -73,7 +73,7 @@ __device__ __forceinline__ void sn_norm(float (&v)[PER][VEC], const float (&w)[P
     for (int i = 0; i < PER; ++i)
 #pragma unroll
       for (int e = 0; e < VEC; ++e) s += v[i][e];  // numbers beyond the row are zeros
-    mean = block_sum<SN_NT>(s, red) * inv_n;
+    mean = block_sum<SN_NT, true>(s, red) * inv_n;
   }
   float ss = 0.f;
 #pragma unroll
@@ -84,7 +84,7 @@ __device__ __forceinline__ void sn_norm(float (&v)[PER][VEC], const float (&w)[P
         v[i][e] -= mean;
         ss = fmaf(v[i][e], v[i][e], ss);
       }
-  const float r = 1.0f / sqrtf(block_sum<SN_NT>(ss, red + SN_NT / 64) * inv_n + eps);
+  const float r = 1.0f / sqrtf(block_sum<SN_NT, true>(ss, red + SN_NT / 64) * inv_n + eps);
 #pragma unroll
   for (int i = 0; i < PER; ++i)
     if (e0 + SN_NT * VEC * i < D)
