@@ -62,14 +62,16 @@ __device__ __forceinline__ float fast_tanh(float x) {  // 1 - 2 / (1 + e^(2x)) w
 // NC: value heads that a wave has room for (1, or a power of two up to NVC). The operands of all of them are on their way together, so room
 // for more than there are costs registers and a launch that is 0.3 - 0.5 us longer (16 x 16 heads of 64 / 64, 8 tokens of 60 keys 5.1 us, 5.6 with
 // room for four; 16 x 4 of 64 / 32 with all 4 value heads 6.2 us, 6.6 with room for eight).
-template <bool SINGLE, int NC>
-__global__ void __launch_bounds__(64)
+// WAVES > 1: up to so many ranges of a single token's keys are the waves of one workgroup, which merge through LDS; more of them go through scratch
+// memory and a second kernel.
+template <bool SINGLE, int NC, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES)
 attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float* __restrict__ out, const bf16_t* __restrict__ k_pages,
                              const bf16_t* __restrict__ v_pages, const int* __restrict__ positions, const int* __restrict__ token_seq,
                              const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ work, int H, int KVH, int NV,
                              int PS, float scale, int window, int chunk, int keep, float softcap, const float* __restrict__ slopes, int splits,
                              float* __restrict__ part_o, float* __restrict__ part_ml, const float* __restrict__ sinks) {
-  const int lane = threadIdx.x, col = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
   const int group = H / KVH;
   int tok = 0, head = 0, kvh = 0;
   bool valid;
@@ -79,7 +81,7 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
     const int c = (blockIdx.y % col_sets) * 16 + col;
     valid = c < group;
     head = kvh * group + (valid ? c : 0);
-    tok = work[blockIdx.x / splits];
+    tok = work[WAVES > 1 ? blockIdx.x : blockIdx.x / splits];
   } else {
     const int tile = blockIdx.x / SUB_TILES, sub = blockIdx.x % SUB_TILES;
     const int first = work[2 * tile], n = work[2 * tile + 1];
@@ -124,7 +126,7 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
   const int first_block = lo_min / 64, n_kept = lev_kept_blocks(lo_min, keep);
   int block_first = 0, block_last = n_kept + p_max / 64 - first_block;
   if (SINGLE && splits > 1) {
-    const int per = (block_last + splits) / splits, z = blockIdx.x % splits;
+    const int per = (block_last + splits) / splits, z = WAVES > 1 ? (int)threadIdx.x >> 6 : blockIdx.x % splits;
     block_first = z * per;
     block_last = min(block_last, block_first + per - 1);
   }
@@ -246,6 +248,45 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
   }
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
+  if (WAVES > 1) {  // the merge of the kernel below (the same sums in the same order), a wave some tiles of the result
+    extern __shared__ __attribute__((aligned(16))) unsigned char av_merge[];
+    f32x4* po = reinterpret_cast<f32x4*>(av_merge);                       // [splits][NC * NDT][64]
+    float2* ml = reinterpret_cast<float2*>(po + splits * NC * NDT * 64);  // [splits][16]
+    const int wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      if (c == 0 || c < n_c) {
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) po[(wave * NC * NDT + c * NDT + dt) * 64 + lane] = o[c][dt];
+      }
+    if (g == 0) ml[wave * 16 + col] = make_float2(m, l);
+    lds_barrier();
+    float w[8], M = -INFINITY;
+#pragma unroll
+    for (int s = 0; s < WAVES; ++s) M = fmaxf(M, ml[min(s, splits - 1) * 16 + col].x);
+    float v[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const float2 q2 = ml[min(s, splits - 1) * 16 + col];
+      w[s] = s < splits ? __builtin_amdgcn_exp2f(q2.x - (M == -INFINITY ? 0.f : M)) : 0.f;
+      v[s] = s < splits ? w[s] * q2.y : 0.f;
+    }
+    float L = ((v[0] + v[4]) + (v[2] + v[6])) + ((v[1] + v[5]) + (v[3] + v[7]));
+    if (sinks != nullptr) L = M == -INFINITY ? 1.0f : L + __builtin_amdgcn_exp2f(sinks[head] * LOG2E - M);
+    const float inv = L > 0.f ? 1.0f / L : 0.f;
+    float* ob = out + (((size_t)tok * H + head) * NV + (NV == 1 ? 0 : c0)) * VD + 4 * g;
+    for (int t = wave; t < n_c * NDT; t += splits) {
+      f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < WAVES; ++s) {  // beyond the ranges: weight 0
+        const f32x4 part = po[(min(s, splits - 1) * NC * NDT + t) * 64 + lane];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] = fmaf(w[s], part[r], acc[r]);
+      }
+      if (valid) *reinterpret_cast<f32x4*>(ob + 16 * t) = acc * inv;
+    }
+    return;
+  }
   if (!valid) return;
   if (SINGLE && splits > 1) {  // unnormalised sums, the maximum and the sum of weights: merged by the kernel below
     const size_t slot = ((size_t)blockIdx.x * H + head);  // (token index, split) major, then head
@@ -556,6 +597,25 @@ attention_values_merge_kernel(const float* __restrict__ part_o, const float* __r
   }
 }
 
+// Key ranges that one workgroup's waves take: eight where a wave's operands and sums leave it half of a lane's 512 registers, else four
+template <int NC>
+constexpr int av_waves() { return 20 * NKS + 12 * NDT * NC > 160 ? 4 : 8; }
+static int av_room(int NV) {  // value heads of a wave of the kernels without shared operands
+  int room = 1;
+  while (room < NV && room < NVC) room *= 2;
+  return room;
+}
+// Whether a token's ranges are the waves of one workgroup. That saves a launch and a way through memory (4 - 5 us) and puts their reads on one CU, which
+// takes about 50 KB a microsecond: not where that CU then reads over 192 KB more than if the waves lay apart. 8 tokens of 240 keys, four ranges: heads of
+// 256 / 224 (184 KB more) 0.6 us ahead as one workgroup, 4 heads of 128 / 64 (74 KB) 12.1 us before, 8.3 now, 32 tokens of 180 keys (25 KB) 12.4 / 7.9.
+static bool av_merged(int splits, int NV, int groups, long reach) {
+  const int room = av_room(NV);
+  if (splits <= 1 || splits > (room == 1 ? av_waves<1>() : room == 2 ? av_waves<2>() : room == 4 ? av_waves<4>() : av_waves<8>())) return false;
+  const long wave_bytes = ((reach + 63) / 64 + splits - 1) / splits * 64 * (HD + (NV < room ? NV : room) * VD) * 2;
+  const long apart = ((long)groups * splits + 255) / 256, together = ((long)groups + 255) / 256 * splits;
+  return (together - apart) * wave_bytes <= 192 * 1024;
+}
+
 // bytes of scratch memory for n single tokens whose keys are split `splits` ways
 extern "C" long lev_attention_values_mfma_workspace(int n_singles, int splits, int H, int NV) {
   return splits <= 1 ? 0 : (long)n_singles * splits * H * ((long)NV * VD + 2) * (long)sizeof(float);
@@ -578,22 +638,31 @@ extern "C" int lev_attention_values_mfma(const void* q, long q_stride, float* ou
                   ((uintptr_t)out & 15) == 0,
               "attention: operands must be 16-byte aligned");
   const int chunks = NV == 1 ? 1 : (NV + NVC - 1) / NVC;
-  int room = 1;  // value heads of a wave of the kernels without shared operands
-  while (room < NV && room < NVC) room *= 2;
+  const int room = av_room(NV);
   LEV_REQUIRE(H <= 65535 && chunks <= 65535, "attention: too many heads (%d)", H);
-#define AV_ROOM(SINGLE, NC, GRID, WORK, SPLITS, PART_O, PART_ML)                                                                                    \
-  if constexpr (NC <= NVC)                                                                                                                          \
-    if (room == NC)                                                                                                                                 \
-      attention_values_mfma_kernel<SINGLE, NC><<<GRID, 64, 0, stream>>>((const bf16_t*)q, q_stride, out, (const bf16_t*)k_pages,                   \
-                                                                        (const bf16_t*)v_pages, positions, token_seq, block_tables, bt_stride, WORK, \
-                                                                        H, KVH, NV, PS, scale, window, chunk, keep, softcap, slopes, SPLITS, PART_O, PART_ML, sinks)
-#define AV_ROOMS(SINGLE, GRID, WORK, SPLITS, PART_O, PART_ML)   \
-  do {                                                          \
-    AV_ROOM(SINGLE, 1, GRID, WORK, SPLITS, PART_O, PART_ML);    \
-    AV_ROOM(SINGLE, 2, GRID, WORK, SPLITS, PART_O, PART_ML);    \
-    AV_ROOM(SINGLE, 4, GRID, WORK, SPLITS, PART_O, PART_ML);    \
-    AV_ROOM(SINGLE, 8, GRID, WORK, SPLITS, PART_O, PART_ML);    \
+#define AV_ROOM(SINGLE, NC, WAVES, LDS, GRID, WORK, SPLITS, PART_O, PART_ML)                                                                              \
+  if constexpr (NC <= NVC)                                                                                                                              \
+    if (room == NC) {                                                                                                                                   \
+      const size_t lds = LDS(NC);                                                                                                                       \
+      if (lds > 64 * 1024) { /* more than a kernel gets unasked */                                                                                      \
+        hipError_t e = hipFuncSetAttribute((const void*)attention_values_mfma_kernel<SINGLE, NC, WAVES>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+        LEV_REQUIRE(e == hipSuccess, "attention: %zu bytes of LDS a workgroup: %s", lds, hipGetErrorString(e));                                         \
+      }                                                                                                                                                 \
+      attention_values_mfma_kernel<SINGLE, NC, WAVES><<<GRID, WAVES > 1 ? 64 * SPLITS : 64, lds, stream>>>(                                             \
+          (const bf16_t*)q, q_stride, out, (const bf16_t*)k_pages, (const bf16_t*)v_pages, positions, token_seq, block_tables, bt_stride, WORK, H, KVH, \
+          NV, PS, scale, window, chunk, keep, softcap, slopes, SPLITS, PART_O, PART_ML, sinks);                                                         \
+    }
+#define AV_NO_LDS(NC) 0
+#define AV_MERGE_LDS(NC) ((size_t)splits * (NC * NDT * 64 * sizeof(f32x4) + 16 * sizeof(float2)))
+#define AV_ROOMS(SINGLE, WAVES, LDS, GRID, WORK, SPLITS, PART_O, PART_ML)       \
+  do {                                                                          \
+    AV_ROOM(SINGLE, 1, WAVES(1), LDS, GRID, WORK, SPLITS, PART_O, PART_ML);     \
+    AV_ROOM(SINGLE, 2, WAVES(2), LDS, GRID, WORK, SPLITS, PART_O, PART_ML);     \
+    AV_ROOM(SINGLE, 4, WAVES(4), LDS, GRID, WORK, SPLITS, PART_O, PART_ML);     \
+    AV_ROOM(SINGLE, 8, WAVES(8), LDS, GRID, WORK, SPLITS, PART_O, PART_ML);     \
   } while (0)
+#define AV_ONE_WAVE(NC) 1
+#define AV_MANY_WAVES(NC) av_waves<NC>()
   if (n_tiles > 0) {
     dim3 grid(n_tiles, H, chunks);
     const size_t lds = ((size_t)HD * 64 + (size_t)(NV == 1 ? 1 : (NV < NVC ? NV : NVC)) * VD * VS_STRIDE) * sizeof(bf16_t);
@@ -617,19 +686,27 @@ extern "C" int lev_attention_values_mfma(const void* q, long q_stride, float* ou
     }
 #undef AV_RUNS
     else  // the longest ranges: every wave by itself, operands straight from the pages
-      AV_ROOMS(false, dim3(n_tiles * SUB_TILES, H, chunks), tiles, 1, nullptr, nullptr);
+      AV_ROOMS(false, AV_ONE_WAVE, AV_NO_LDS, dim3(n_tiles * SUB_TILES, H, chunks), tiles, 1, nullptr, nullptr);
     if (lev_check_launch("attention_values_mfma (runs)")) return -1;
   }
   if (n_singles > 0) {
     const int group = H / KVH;
-    dim3 grid(n_singles * splits, KVH * ((group + 15) / 16), chunks);
+    long reach = window > 0 && window < max_keys ? window : max_keys;
+    if (chunk > 0 && chunk < reach) reach = chunk;
+    const bool merged = av_merged(splits, NV, n_singles * KVH * ((group + 15) / 16) * chunks, reach + (keep > 0 ? keep : 0));
+    dim3 grid(merged ? n_singles : n_singles * splits, KVH * ((group + 15) / 16), chunks);
     float* part_o = workspace;
-    float* part_ml = splits > 1 ? workspace + (size_t)n_singles * splits * H * NV * VD : nullptr;
-    AV_ROOMS(true, grid, singles, splits, part_o, part_ml);
+    float* part_ml = splits > 1 && !merged ? workspace + (size_t)n_singles * splits * H * NV * VD : nullptr;
+    if (merged) AV_ROOMS(true, AV_MANY_WAVES, AV_MERGE_LDS, grid, singles, splits, nullptr, nullptr);
+    else AV_ROOMS(true, AV_ONE_WAVE, AV_NO_LDS, grid, singles, splits, part_o, part_ml);
+#undef AV_MANY_WAVES
+#undef AV_ONE_WAVE
 #undef AV_ROOMS
+#undef AV_MERGE_LDS
+#undef AV_NO_LDS
 #undef AV_ROOM
     if (lev_check_launch("attention_values_mfma (single tokens)")) return -1;
-    if (splits > 1) {
+    if (splits > 1 && !merged) {
       attention_values_merge_kernel<<<dim3(n_singles, H), 64, 0, stream>>>(part_o, part_ml, singles, out, H, NV * VD, splits, sinks);
       if (lev_check_launch("attention_values_mfma (merge)")) return -1;
     }

@@ -72,3 +72,19 @@ def test_pages_out_of_sight_are_not_there(ps, window, keep):
                               scale=dk ** -0.5, window=window, block_tables=bt, keep_first=keep)
         outs.append(out)
     assert bool(torch.isfinite(outs[0]).all()) and torch.equal(*outs)
+
+
+@pytest.mark.parametrize("G,dk,dv,talking", [(1, 128, 64, False), (2, 64, 32, True), (1, 256, 224, False), (3, 32, 32, True)])
+@pytest.mark.parametrize("keys", [65, 128, 129, 250, 257, 449, 512, 513])
+@pytest.mark.parametrize("window", [None, 100])
+def test_ranges_of_keys_that_one_workgroup_merges(G, dk, dv, talking, keys, window):
+    """Two to nine ranges of a single token's keys, beside tokens with fewer keys than there are ranges: up to four or eight are merged by the waves of a
+    workgroup, more by a kernel of their own."""
+    H = 2 * G
+    g = torch.Generator().manual_seed(keys + dk)
+    runs = [(1, keys), (1, 1), (1, 64), (1, max(1, keys - 1))]
+    q, k = ([as_bf16_numbers(Z.unit_rms(torch.randn(r[i], n, dk, generator=g), 1e-6).reshape(r[i], -1)) for r in runs] for i, n in ((0, H), (1, G)))
+    v = [as_bf16_numbers(torch.randn(kl, G * dv, generator=g)) for _, kl in runs]
+    talk = as_bf16_numbers(torch.eye(H) + 0.5 * torch.randn(H, H, generator=g)) if talking else None
+    args = (H, G, dk, dv, runs, window, None, 4.0 / math.sqrt(dk), q, k, v, talk, None)
+    torch.testing.assert_close(run_attention(torch.bfloat16, *args), plain_attention(*args), **tol(torch.bfloat16, bf16=3e-2))
