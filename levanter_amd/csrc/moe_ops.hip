@@ -39,7 +39,8 @@ struct MoeRouteArgs {
   int* chosen;
   float* weights;
 };
-__device__ __forceinline__ void moe_route_token(const MoeRouteArgs& a, int t, bool store, float* s_s, float* c_s, float* g_s) {
+// chosen_s: a copy of the choices in LDS, for a sort in the same workgroup
+__device__ __forceinline__ void moe_route_token(const MoeRouteArgs& a, int t, bool store, float* s_s, float* c_s, float* g_s, int* chosen_s) {
   const int lane = threadIdx.x & 63, E = a.E, G = a.G, top = a.top;
   const int per = E / G;
   const float* zt = a.z + (size_t)t * a.z_stride;
@@ -98,12 +99,13 @@ __device__ __forceinline__ void moe_route_token(const MoeRouteArgs& a, int t, bo
       const float c = c_s[e];
       if (!(taken >> i & 1u) && (c > best || (c == best && e < best_e))) best = c, best_e = e;
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ob = __shfl_xor(best, o, 64);
-      const int oe = __shfl_xor(best_e, o, 64);
-      if (ob > best || (ob == best && oe < best_e)) best = ob, best_e = oe;
-    }
+    // the largest, and of its owners' experts the first: those of the lowest 64 before others, then the lowest lane's
+    const float largest = wave_max(best);
+    const bool owner = best == largest && best_e < E;
+    unsigned long long owners = 0;
+    int block = 0;
+    for (; block * 64 < E && owners == 0; ++block) owners = __ballot(owner && best_e >> 6 == block);
+    best_e = owners != 0 ? (block - 1) * 64 + __ffsll(owners) - 1 : E;
     if (best_e >= E) best_e = 0;  // nothing left to choose from (a configuration that keeps fewer experts than it uses)
     if ((best_e & 63) == lane) taken |= 1u << (best_e >> 6);
     if (lane == n) mine = best_e;
@@ -121,9 +123,11 @@ __device__ __forceinline__ void moe_route_token(const MoeRouteArgs& a, int t, bo
   if (!store) return;
   if (lane < top) {
     a.chosen[at + lane] = mine;
+    if (chosen_s != nullptr) chosen_s[at + lane] = mine;
     a.weights[at + lane] = weight;
   } else if (lane == top && a.extra) {
     a.chosen[at + top] = E;
+    if (chosen_s != nullptr) chosen_s[at + top] = E;
     a.weights[at + top] = 1.0f;
   }
 }
@@ -131,7 +135,7 @@ __device__ __forceinline__ void moe_route_token(const MoeRouteArgs& a, int t, bo
 __global__ void __launch_bounds__(64)
 moe_route_kernel(const MoeRouteArgs a) {
   __shared__ float s_s[MOE_MAX_E], c_s[MOE_MAX_E], g_s[MOE_MAX_E];
-  moe_route_token(a, blockIdx.x, true, s_s, c_s, g_s);
+  moe_route_token(a, blockIdx.x, true, s_s, c_s, g_s, nullptr);
 }
 
 // ---- sort --------------------------------------------------------------------------------------
@@ -145,9 +149,9 @@ __device__ __forceinline__ void moe_sort_pairs(MoeSortLds& l, const int* chosen,
                                                int* __restrict__ pos_of, int* __restrict__ tiles, int* __restrict__ meta) {
   const int tid = threadIdx.x;
   for (int e = tid; e < E; e += MOE_SORT_NT) l.count[e] = 0, l.cursor[e] = 0;
-  __syncthreads();
+  lds_barrier();
   for (int p = tid; p < P; p += MOE_SORT_NT) atomicAdd(&l.count[chosen[p]], 1);
-  __syncthreads();
+  lds_barrier();
   if (tid < 64) {  // running sums over the experts: each lane a stretch of neighbours, then across the lanes
     const int c = (E + 63) / 64, lo = min(E, tid * c), hi = min(E, lo + c);
     int n = 0, nt = 0;
@@ -170,7 +174,7 @@ __device__ __forceinline__ void moe_sort_pairs(MoeSortLds& l, const int* chosen,
       if (e < n_real) tile += (l.count[e] + tile_rows - 1) / tile_rows;
     }
   }
-  __syncthreads();
+  lds_barrier();
   for (int p = tid; p < P; p += MOE_SORT_NT) {
     const int e = chosen[p];
     const int pos = l.start[e] + atomicAdd(&l.cursor[e], 1);
@@ -203,12 +207,13 @@ moe_route_sort_kernel(const MoeRouteArgs a, int T, int n_real, int tile_rows, in
                       int* __restrict__ meta) {
   __shared__ MoeSortLds l;
   __shared__ float s_s[MOE_SMALL_T][MOE_SMALL_E], c_s[MOE_SMALL_T][MOE_SMALL_E];
+  __shared__ int chosen_s[MOE_SMALL_T * (MOE_MAX_TOP + 1)];
   const int wave = threadIdx.x >> 6;
   // the groups' scores take the place of the sort's counters, which nobody needs before the routing is done
   float* g_s = reinterpret_cast<float*>(l.count) + (size_t)wave * MOE_SMALL_E / 4;
-  moe_route_token(a, min(wave, T - 1), wave < T, s_s[wave], c_s[wave], g_s);
-  __syncthreads();  // the choices, in global memory, are the whole workgroup's
-  moe_sort_pairs(l, a.chosen, T * (a.top + a.extra), a.E + a.extra, n_real, tile_rows, sorted, pos_of, tiles, meta);
+  moe_route_token(a, min(wave, T - 1), wave < T, s_s[wave], c_s[wave], g_s, chosen_s);
+  lds_barrier();  // (the choices in global memory are on their way: the sort reads the copy)
+  moe_sort_pairs(l, chosen_s, T * (a.top + a.extra), a.E + a.extra, n_real, tile_rows, sorted, pos_of, tiles, meta);
 }
 
 static int moe_route_check(const MoeRouteArgs& a, int T) {
