@@ -489,7 +489,7 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
         for (int r = 0; r < 4; ++r) {
           const float far = dist0 - (float)(32 * u + 4 * hh + r);
           if (softcap > 0.f) st[u][hh][r] = fmaf(-slope, far, softcap * fast_tanh(st[u][hh][r] * scale * __builtin_amdgcn_rcpf(softcap))) * LOG2E;
-          else st[u][hh][r] = fmaf(st[u][hh][r], scale, -(slope * far)) * LOG2E;
+          else st[u][hh][r] = fmaf(-slope, far, st[u][hh][r] * scale) * LOG2E;
         }
       }
     if (!all_pages || key0 + 63 > p_min || !(key0 >= lo_max || key0 + 63 < keep)) {  // a row that does not see every key: the same for the whole wave

@@ -424,16 +424,16 @@ moe_linear_few_kernel(const MoeLinearArgs p) {
 // step and workgroup at 15 TB/s) and the last round of tiles. The outputs leave through LDS as whole lines, after one decision on the activation
 // for all of them: stored from the products' registers, 8 or 16 bytes of each of 32 rows, with the decision at every value, the last 64 KB of a
 // workgroup cost 15 us a round: 2048 outputs of 2048 (bfloat16 / 32-bit, microseconds), 32 experts of 256 rows 126 / 137 -> 110 / 116,
-// 4 of 2,048 93 / 105 -> 78 / 80. Where the weights' read is the bound, fewer than two rounds of a chiplet's 64 workgroups, these begin at places of
+// 4 of 2,048 93 / 105 -> 78 / 80. Where the weights' read is the bound, up to one and a half rounds of a chiplet's 64 workgroups, these begin at places of
 // their own along K: rows a power of two apart lie in the same channels of the memory, and workgroups that walk together ask those alone: 32
-// experts of 128 rows 97 -> 65 us, of 40 72 -> 56, of 90 99 -> 83; from two rounds on they have drifted apart (254 rows 136 either way, 8 experts of
+// experts of 128 rows 97 -> 65 us, of 40 72 -> 56, of 90 99 -> 83; from two rounds on they have drifted apart (256 rows 110 -> 105, 254 136 either way, 8 of
 // 4,096 rows 190 in order, 197 spread). Measured and not kept: tiles of 256 rows by 8 waves (32 of 256 rows 107, of 254 drawn ones 153 against 136),
 // workgroups that stay and fetch the next tile's first steps ahead of the last outputs (spills; 4 of 2,048 rows 82 - 107), weights three
 // steps ahead (no gain), chiplets' shares by cost (of 40 rows 77 against 55).
 #define MOE_BN 128
 #define MOE_BIG_K 64
 #define MOE_BIG_LD (MOE_BIG_K + 8)
-#define MOE_BIG_SPREAD 128  // a chiplet's workgroups of two rounds
+#define MOE_BIG_SPREAD 96  // a chiplet's workgroups of one and a half rounds
 #define MOE_BIG_LDS(BN) (2 * (MOE_BIG + (BN)) * MOE_BIG_LD * (int)sizeof(bf16_t))
 typedef __attribute__((ext_vector_type(16))) float moe_f32x16;
 // the sums become outputs in place; with glu the first half of a row's registers takes them
@@ -643,7 +643,7 @@ moe_linear_big_kernel(const MoeLinearArgs p) {
     ycol = at / kind;
     tile = lo + __ffsll(__ballot((of >> lane & 1) && __popcll(of & ((1ull << lane) - 1)) == at % kind)) - 1;
   }
-  const bool spread = n * p.n_cols < MOE_BIG_SPREAD;
+  const bool spread = per * p.n_cols <= MOE_BIG_SPREAD;  // the same for all chiplets
   const int e = p.tiles[3 * tile], first = p.tiles[3 * tile + 1], rows = p.tiles[3 * tile + 2];
   if (rows <= MOE_BIG / 2) moe_big_tile<TO, GLU, MOE_BN, MOE_BIG / 2>(p, moe_smem, e, first, rows, ycol, spread);
   else moe_big_tile<TO, GLU, MOE_BN, MOE_BIG>(p, moe_smem, e, first, rows, ycol, spread);
