@@ -104,25 +104,27 @@ sum_norm_kernel(const SumNormArgs a) {
   const bool write = a.w1 != nullptr;
   float v[PER][VEC], w[PER][VEC], b[PER][VEC];
   int at[PER];
-  if (a.top > 0) {
-    if (tid < a.top) {
-      pos_s[tid] = a.pos_of[(size_t)row * a.top + tid];
-      wt_s[tid] = a.weights[(size_t)row * a.top + tid];
-    }
-    __syncthreads();
-  }
-  // loads stand under no condition (clamped into the row): all of them are in flight before the first is used
+  // loads stand under no condition (clamped into the row): all of them are in flight before the first is used, the places of the experts' outputs
+  // ahead of the others, which are not waited for at the barrier behind which the outputs themselves are asked for
+  int pos = 0;
+  float wt = 0.f;
+  if (a.top > 0) pos = a.pos_of[(size_t)row * a.top + min(tid, a.top - 1)], wt = a.weights[(size_t)row * a.top + min(tid, a.top - 1)];
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     at[i] = min((tid + SN_NT * i) * VEC, D - VEC);
     sn_load<VEC>(a.x + base + at[i], v[i]);
     if (write) sn_load<VEC>(a.w1 + at[i], w[i]);
   }
+  float y[PER][VEC];
+  if (write && a.y != nullptr)
+#pragma unroll
+    for (int i = 0; i < PER; ++i) sn_load<VEC>(a.y + base + at[i], y[i]);
+  if (a.top > 0) {
+    if (tid < a.top) pos_s[tid] = pos, wt_s[tid] = wt;
+    lds_barrier();
+  }
   if (write) {
     if (a.y != nullptr) {
-      float y[PER][VEC];
-#pragma unroll
-      for (int i = 0; i < PER; ++i) sn_load<VEC>(a.y + base + at[i], y[i]);
 #pragma unroll
       for (int i = 0; i < PER; ++i)
 #pragma unroll
@@ -162,9 +164,9 @@ sum_norm_kernel(const SumNormArgs a) {
         for (int c = 0; c < a.top; ++c) {
           float p[VEC];
           sn_load<VEC>(a.expert_out + (size_t)pos_s[c] * D + at[i], p);
-          const float wt = wt_s[c];
+          const float share = wt_s[c];
 #pragma unroll
-          for (int e = 0; e < VEC; ++e) sum[e] = fmaf(wt, p[e], sum[e]);
+          for (int e = 0; e < VEC; ++e) sum[e] = fmaf(share, p[e], sum[e]);
         }
 #pragma unroll
         for (int e = 0; e < VEC; ++e) v[i][e] += sum[e];
