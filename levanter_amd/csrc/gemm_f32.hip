@@ -32,7 +32,7 @@ __device__ __forceinline__ void gemm_f32_store(gf_f32x4 v, const float* bias, co
 // four products of a step): the 32-bit instruction takes 32 cycles for 1,024 multiply-adds, which hides much of what such loads cost
 // the vector cache (a look-up for every lane).
 // What bounds it: few rows, the read of the weights (4096 x 4096 at 4 rows 14.3 us, 4.7 TB/s; 768 x 768 4.8 us, a launch and a chain of
-// loads); some hundred rows, L2 at about 9.5 TB/s (1024 x 4096 at 203 rows 33 us) or the last round of tiles. The plain kernel of
+// loads); some dozens, L2 at about 9.5 TB/s (1024 x 4096 at 203 rows 33 us) or the last round of tiles. The plain kernel of
 // gemm_simple.hip (64 x 64 tiles, vector ALU, scalar loads) took 84 us for 768 x 768 at 4 rows, 378 us for 768 x 3072 (now 4.8 and 10).
 template <int RT, int NT, int W>
 __global__ void __launch_bounds__(64 * W)
@@ -276,6 +276,63 @@ gemm_f32_tile_kernel(const float* __restrict__ a, long lda, const float* __restr
   }
 }
 
+// Up to eight rows and few outputs: 16 of them a workgroup would leave most CUs without one. A workgroup of eight waves owns four outputs; a thread
+// multiplies 16 bytes of each weight row with every row of a, two stretches of 2,048 k on their way at once, and the partial sums go over the lanes
+// and, through LDS, over the waves: chains of a dozen roundings (errors 0.8e-7 .. 1.1e-7; the 16-output tiles 1.9e-7 .. 5e-7).
+// What bounds it: a launch, one read of the weights (768 x 3072 at 4 rows 5.9 us, 1.6 TB/s) and 4 sums over the lanes for every row.
+#define GF_FEW_OUT 4
+template <int MR>
+__global__ void __launch_bounds__(512)
+gemm_f32_few_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias, const float* residual, long ldr,
+                    float* out, long ldo, int M, int N, int K, int act) {
+  __shared__ float part[8][GF_FEW_OUT * MR];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, o0 = blockIdx.x * GF_FEW_OUT;
+  const float *ar[MR], *wr[GF_FEW_OUT];
+#pragma unroll
+  for (int m = 0; m < MR; ++m) ar[m] = a + (size_t)min(m, M - 1) * lda;  // rows and outputs beyond the matrices: read again, never stored
+#pragma unroll
+  for (int j = 0; j < GF_FEW_OUT; ++j) wr[j] = w + (size_t)min(o0 + j, N - 1) * K;
+  float acc[GF_FEW_OUT][MR] = {};
+  for (int k0 = 0; k0 < K; k0 += 4096) {
+    gf_f32x4 av[2][MR], wv[2][GF_FEW_OUT];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int kc = min(k0 + 2048 * u + 4 * tid, K - 4);
+#pragma unroll
+      for (int j = 0; j < GF_FEW_OUT; ++j) wv[u][j] = *reinterpret_cast<const gf_f32x4*>(wr[j] + kc);
+#pragma unroll
+      for (int m = 0; m < MR; ++m) av[u][m] = *reinterpret_cast<const gf_f32x4*>(ar[m] + kc);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (k0 + 2048 * u + 4 * tid < K)
+#pragma unroll
+        for (int j = 0; j < GF_FEW_OUT; ++j)
+#pragma unroll
+          for (int m = 0; m < MR; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[j][m] = fmaf(wv[u][j][e], av[u][m][e], acc[j][m]);
+  }
+#pragma unroll
+  for (int j = 0; j < GF_FEW_OUT; ++j)
+#pragma unroll
+    for (int m = 0; m < MR; ++m) {
+      const float s = wave_sum(acc[j][m]);
+      if (lane == 0) part[wave][j * MR + m] = s;
+    }
+  __syncthreads();
+  const int m = tid % MR, o = o0 + tid / MR;
+  if (tid >= GF_FEW_OUT * MR || m >= M || o >= N) return;
+  float x = 0.f;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) x += part[q][tid];
+  if (bias) x += bias[o];
+  x = lev_activate(x, act);
+  if (residual) x += residual[(size_t)m * ldr + o];
+  out[(size_t)m * ldo + o] = x;
+}
+
 // Which tile: the fewest microseconds by an estimate from what was measured over 14 weights and 17 .. 2,048 rows (all tiles of both lists).
 // Of the first kernel: the longest of the weights' read from memory (5.2 TB/s), the operands that a CU pulls through its L2 (37 GB/s and CU) and
 // the products of the CU with the most workgroups (waves that fewer than four SIMDs hold leave the others idle). Of the second: its steps on that
@@ -325,6 +382,21 @@ int lev_gemm_f32(const float* a, long lda, const float* w, const float* bias, co
                  int act, hipStream_t stream) {
   if (K % 4 != 0 || lda % 4 != 0 || ((uintptr_t)a & 15) != 0 || ((uintptr_t)w & 15) != 0) return 1;
   const int vec = ldo % 4 == 0 && ((uintptr_t)out & 15) == 0 && (!bias || ((uintptr_t)bias & 15) == 0) && (!residual || (ldr % 4 == 0 && ((uintptr_t)residual & 15) == 0));
+  // Measured against the best tile, 1 / 2 / 4 / 8 rows, microseconds before and now: 768 x 768 4.5, 4.6, 4.8, 5.0 / 2.8, 3.3, 3.9, 5.3; 768 x 3072 9.8, 10.0, 10.8,
+  // 11.7 / 4.2, 5.0, 5.9, 7.7; 1024 x 4096 12.0, 12.2, 13.3, 14.6 / 5.1, 5.6, 6.6, 8.7; 1600 x 1600 7.1, 7.1, 7.3, 7.8 / 4.9, 5.6, 6.6, 11.9; 1600 x 6400 17.8, 18.1, 19.3,
+  // 21.3 / 10.1, 11.1, 12.9, 20.2; 3072 x 1024 6.0, 6.1, 5.9, 6.3 / 5.3, 5.9, 8.0, 14.9; 4096 x 4096 15.6, 15.0, 14.9, 15.7 / 12.9, 13.1, 15.3, 27.3: the more rows, the
+  // fewer outputs (sums over the lanes), the longer K, the more (the tiles' few workgroups read it).
+  const int few = M > 8 ? 0 : M > 4 ? 8 : M > 2 ? 4 : M;
+  if (few > 0 && (long)few * N <= (K >= 2048 ? 12800 : 6400) && (few < 8 || K >= 1024)) {
+#define GEMM_F32_FEW(MR) \
+  if (few == MR) gemm_f32_few_kernel<MR><<<(N + GF_FEW_OUT - 1) / GF_FEW_OUT, 512, 0, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act)
+    GEMM_F32_FEW(1);
+    else GEMM_F32_FEW(2);
+    else GEMM_F32_FEW(4);
+    else GEMM_F32_FEW(8);
+#undef GEMM_F32_FEW
+    return lev_check_launch("linear (32-bit, few rows)");
+  }
   const int choice = gemm_f32_choose(M, N, K), line = choice - GEMM_F32_N_TILES;
   const int rt = line < 0 ? GEMM_F32_TILES[choice].rt : 2 * GEMM_F32_LINE_TILES[line].rt, nt = line < 0 ? GEMM_F32_TILES[choice].nt : 2 * GEMM_F32_LINE_TILES[line].nt;
   const int n_rows = (M + 16 * rt - 1) / (16 * rt), n_cols = (N + 16 * nt - 1) / (16 * nt);

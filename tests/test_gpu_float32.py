@@ -28,6 +28,9 @@ LINEAR = [(1, 4, 1), (1, 64, 50), (3, 768, 768), (16, 100, 48), (17, 772, 33), (
 # odd and even numbers of steps, of pieces of 128 and 256 and one step more
 LINEAR += [(404, 768, 3072), (289, 100, 2051), (1031, 32, 3001), (801, 1028, 1030), (777, 300, 3072), (2047, 292, 4097), (609, 516, 2310), (2047, 260, 2310),
            (1000, 260, 4097), (1030, 1028, 4100), (2047, 516, 3071)]
+# up to eight rows and four outputs a workgroup: 1, 2, 4 and 8 rows' room full and not, outputs that end inside a workgroup, K of less than a thread each,
+# one stretch of 2,048, two, a short one more; and just beyond the rule's lines
+LINEAR += [(1, 8196, 64), (2, 1028, 3001), (3, 4100, 130), (4, 2048, 1601), (5, 2052, 33), (8, 1024, 777), (7, 4096, 1600), (8, 1020, 40), (4, 1600, 1601), (1, 100, 6401)]
 
 
 @pytest.mark.parametrize("M,Ki,N", LINEAR)
