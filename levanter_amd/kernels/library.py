@@ -1238,7 +1238,9 @@ class HipKernels:
         experts, the more workgroups of 128 rows there are to hide behind each other. Up and down product of distinct weights, microseconds, 16 / 128 rows a
         tile: 16 experts of 2048 x 2048 at 14 / 16 rows 66 / 75, 73 / 75; 32 of 4096 x 2048 at 14 / 15 / 16 rows 233 / 255, 249 / 255, 292 / 256; 33 of 2048 x 2048 at 16 rows
         150 / 184; 64 of 2048 x 2048 at 13 / 14 / 16 rows 248 / 258, 268 / 256, 299 / 253; 128 of 2048 x 1024 at 12 / 13 / 16 rows 242 / 247, 254 / 245, 305 / 244
-        (gated 336 / 305, 349 / 306, 420 / 310); 256 of 1024 x 512 at 12 / 13 / 16 rows 126 / 128, 132 / 129, 155 / 130."""
+        (gated 336 / 305, 349 / 306, 420 / 310); 256 of 1024 x 512 at 12 / 13 / 16 rows 126 / 128, 132 / 129, 155 / 130. Since then tiles of 128 write whole
+        lines and begin apart along K: over drawn choices 16 of 2048 x 2048 at 14 rows 71 / 60, 32 of 2048 x 4096 at 14 rows 272 / 251, 33 of 2048 x 2048 at 12 / 16
+        rows 113 / 138, 152 / 139, 64 of them at 8 / 13 rows 207 / 250, 294 / 251: the lines lie a row or two late for some numbers of experts."""
         rows = 12 if n_experts >= 96 else 14 if n_experts >= 48 else 16
         return 128 if pairs > rows * n_experts else 16
 
