@@ -84,6 +84,14 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// Between what a wave's lanes write to LDS and what its other lanes read of it (and before they write there again). LDS works a wave's accesses off in
+// order, so nothing is waited for; but to the compiler they are accesses of one thread to other addresses, which it may exchange.
+__device__ __forceinline__ void lds_wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // sum over a block of NT threads (NT a multiple of 64, at most 1024); every thread gets the result.
 // `red` is shared memory of at least NT/64 floats. Safe to call repeatedly (syncs before reuse).
 // LDS_ONLY: its barriers do not wait for global loads and stores in flight, which must be the thread's own.

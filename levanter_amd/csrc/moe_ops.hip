@@ -613,6 +613,7 @@ __device__ __forceinline__ void moe_big_tile(const MoeLinearArgs& p, unsigned ch
           if constexpr (F32) *reinterpret_cast<float4*>(at) = make_float4(v[4 * r4], v[4 * r4 + 1], v[4 * r4 + 2], v[4 * r4 + 3]);
           else *reinterpret_cast<uint2*>(at) = make_uint2(float2_to_bf16x2(v[4 * r4], v[4 * r4 + 1]), float2_to_bf16x2(v[4 * r4 + 2], v[4 * r4 + 3]));
         }
+      lds_wave_order();
 #pragma unroll
       for (int x = 0; x < 32 * LR / 64; ++x) {
         const int r = (64 * x + lane) / LR, c = lane % LR * PER, at = wm * WM + 32 * i + r;
@@ -620,6 +621,7 @@ __device__ __forceinline__ void moe_big_tile(const MoeLinearArgs& p, unsigned ch
         const moe_u32x4 v = *reinterpret_cast<const moe_u32x4*>(lines + r * STRIDE + c);
         if (at < rows && o < F) moe_big_store(static_cast<TO*>(p.out) + (size_t)(first + at) * p.o_stride + o, v, F - o, p.vec);
       }
+      lds_wave_order();
     }
 }
 
