@@ -316,6 +316,7 @@ struct MoeLinearArgs {
   int top, gather, K, N, F, act;
   float limit, up_shift;
   int n_cols, vec;
+  bool spread;  // tiles of 128 rows: their columns begin at places of their own along K
 };
 template <typename TO>
 __device__ __forceinline__ void moe_store4(TO* p, const float (&v)[4], int n, bool vec);
@@ -424,10 +425,14 @@ moe_linear_few_kernel(const MoeLinearArgs p) {
 // step and workgroup at 15 TB/s) and the last round of tiles. The outputs leave through LDS as whole lines, after one decision on the activation
 // for all of them: stored from the products' registers, 8 or 16 bytes of each of 32 rows, with the decision at every value, the last 64 KB of a
 // workgroup cost 15 us a round: 2048 outputs of 2048 (bfloat16 / 32-bit, microseconds), 32 experts of 256 rows 126 / 137 -> 110 / 116,
-// 4 of 2,048 93 / 105 -> 78 / 80. Where the weights' read is the bound, up to one and a half rounds of a chiplet's 64 workgroups, these begin at places of
+// 4 of 2,048 93 / 105 -> 78 / 80. Where the weights' read is the bound the workgroups begin at places of
 // their own along K: rows a power of two apart lie in the same channels of the memory, and workgroups that walk together ask those alone: 32
-// experts of 128 rows 97 -> 65 us, of 40 72 -> 56, of 90 99 -> 83; from two rounds on they have drifted apart (256 rows 110 -> 105, 254 136 either way, 8 of
-// 4,096 rows 190 in order, 197 spread). Measured and not kept: tiles of 256 rows by 8 waves (32 of 256 rows 107, of 254 drawn ones 153 against 136),
+// experts of 128 rows 97 -> 65 us, of 40 72 -> 56, of 160 160 -> 114, 64 of 30 140 -> 103. With many rounds or rows they drift apart by themselves (8 of 4,096
+// rows 190 in order, 197 spread; 64 of 160 with gates, 512 workgroups a chiplet, 416 / 463), so: up to one and a half rounds of a chiplet's 64 workgroups,
+// counted with as many tiles as the step's sizes allow, and up to three where that is twice what most routings make, at 128 rows an expert on average
+// or fewer. How the routing dealt the tokens out has no say: a token's sums would be in another order when others of the step chose otherwise. Over 780
+// shapes 2 are slower by 4 - 5 % than with the actual number of tiles (128 experts of 1024 x 1024 with 60 rows), 50 faster by 4 % and up to 40 %.
+// Measured and not kept: tiles of 256 rows by 8 waves (32 of 256 rows 107, of 254 drawn ones 153 against 136),
 // workgroups that stay and fetch the next tile's first steps ahead of the last outputs (spills; 4 of 2,048 rows 82 - 107), weights three
 // steps ahead (no gain), chiplets' shares by cost (of 40 rows 77 against 55).
 #define MOE_BN 128
@@ -466,7 +471,7 @@ __device__ __forceinline__ void moe_big_store(bf16_t* to, const moe_u32x4& v, in
 
 // BM: 128, or 64 for a tile whose rows fit that
 template <typename TO, bool GLU, int BN, int BM>
-__device__ __forceinline__ void moe_big_tile(const MoeLinearArgs& p, unsigned char* moe_smem, int e, int first, int rows, int ycol, bool spread) {
+__device__ __forceinline__ void moe_big_tile(const MoeLinearArgs& p, unsigned char* moe_smem, int e, int first, int rows, int ycol) {
   constexpr int LD = MOE_BIG_LD, WM = BM / 2, WN = BN / 2, TI = WM / 32, TJ = WN / 32;
   constexpr int CA = BM * (MOE_BIG_K / 8) / 256, CW = BN * (MOE_BIG_K / 8) / 256;  // 16-byte chunks a thread fetches a step
   constexpr int OUT = GLU ? BN / 2 : BN;  // outputs of a workgroup
@@ -491,7 +496,7 @@ __device__ __forceinline__ void moe_big_tile(const MoeLinearArgs& p, unsigned ch
   }
   // the steps in the order they are taken: a partial one (K % 64 != 0) first, so that the loop needs no masks
   const int tail = K % MOE_BIG_K, steps = (K + MOE_BIG_K - 1) / MOE_BIG_K, shift = tail ? 1 : 0;
-  const int turn = spread && !tail ? ycol * 5 % steps : 0;  // whole steps then begin at a place of the workgroup's own
+  const int turn = p.spread && !tail ? ycol * 5 % steps : 0;  // whole steps then begin at a place of the workgroup's own
   auto k_of = [&](int t) {  // t >= 1; beyond the last: loaded again, not used
     const unsigned i = max(min(t, steps - 1) - shift, 0) + turn;
     return (int)min(i, i - (unsigned)steps) * MOE_BIG_K;  // i, or i - steps if that is not below 0
@@ -645,15 +650,14 @@ moe_linear_big_kernel(const MoeLinearArgs p) {
     ycol = at / kind;
     tile = lo + __ffsll(__ballot((of >> lane & 1) && __popcll(of & ((1ull << lane) - 1)) == at % kind)) - 1;
   }
-  const bool spread = per * p.n_cols <= MOE_BIG_SPREAD;  // the same for all chiplets
   const int e = p.tiles[3 * tile], first = p.tiles[3 * tile + 1], rows = p.tiles[3 * tile + 2];
-  if (rows <= MOE_BIG / 2) moe_big_tile<TO, GLU, MOE_BN, MOE_BIG / 2>(p, moe_smem, e, first, rows, ycol, spread);
-  else moe_big_tile<TO, GLU, MOE_BN, MOE_BIG>(p, moe_smem, e, first, rows, ycol, spread);
+  if (rows <= MOE_BIG / 2) moe_big_tile<TO, GLU, MOE_BN, MOE_BIG / 2>(p, moe_smem, e, first, rows, ycol);
+  else moe_big_tile<TO, GLU, MOE_BN, MOE_BIG>(p, moe_smem, e, first, rows, ycol);
 }
 
 // a [rows][K]; w [E][N][K] with N = F outputs, or with glu N = 2F: gate rows then up rows; out [P][F]
 extern "C" int lev_moe_linear(const void* a, long a_stride, const void* w, void* out, long o_stride, const int* tiles, const int* meta,
-                              const int* sorted, int max_tiles, int tile_rows, int top, int gather, int K, int N, int glu, int act, float limit,
+                              const int* sorted, int max_tiles, int tile_rows, int E, int top, int gather, int K, int N, int glu, int act, float limit,
                               float up_shift, int dtype, int out_dtype, int use_mfma, hipStream_t stream) {
   LEV_REQUIRE(a && w && out && tiles && meta && sorted, "experts: a tensor is missing");
   LEV_REQUIRE(K > 0 && N > 0 && (!glu || N % 2 == 0) && top > 0 && max_tiles >= 0, "experts: bad sizes K=%d N=%d", K, N);
@@ -670,12 +674,13 @@ extern "C" int lev_moe_linear(const void* a, long a_stride, const void* w, void*
       const int bn = glu ? MOE_BN / 2 : MOE_BN, n_cols = (F + bn - 1) / bn;
       const long blocks = (long)((max_tiles + 7) / 8) * 8 * n_cols;
       LEV_REQUIRE(blocks <= 0x7fffffffL, "experts: too many tiles (%ld)", blocks);
+      const bool spread = blocks / 8 <= (max_tiles <= 2L * E + 1 ? 2 * MOE_BIG_SPREAD : MOE_BIG_SPREAD);  // by sizes alone, not by what the routing made of them
 #define MOE_BIG_CASE(TO, G)                                                                                                                       \
   do {                                                                                                                                            \
     hipError_t e = hipFuncSetAttribute((const void*)moe_linear_big_kernel<TO, G>, hipFuncAttributeMaxDynamicSharedMemorySize, MOE_BIG_LDS(MOE_BN)); \
     LEV_REQUIRE(e == hipSuccess, "experts: %d bytes of LDS a workgroup: %s", MOE_BIG_LDS(MOE_BN), hipGetErrorString(e));                           \
     moe_linear_big_kernel<TO, G><<<(unsigned)blocks, 256, MOE_BIG_LDS(MOE_BN), stream>>>(                                                         \
-        MoeLinearArgs{(const bf16_t*)a, a_stride, (const bf16_t*)w, out, o_stride, tiles, meta, sorted, top, gather, K, N, F, act, limit, up_shift, n_cols, vec}); \
+        MoeLinearArgs{(const bf16_t*)a, a_stride, (const bf16_t*)w, out, o_stride, tiles, meta, sorted, top, gather, K, N, F, act, limit, up_shift, n_cols, vec, spread}); \
   } while (0)
       if (out_dtype == LEV_F32) {
         if (glu) MOE_BIG_CASE(float, true); else MOE_BIG_CASE(float, false);
@@ -685,7 +690,7 @@ extern "C" int lev_moe_linear(const void* a, long a_stride, const void* w, void*
 #undef MOE_BIG_CASE
       return lev_check_launch("moe_linear (matrix cores, tiles of 128 rows)");
     }
-    const MoeLinearArgs args{(const bf16_t*)a, a_stride, (const bf16_t*)w, out, o_stride, tiles, meta, sorted, top, gather, K, N, F, act, limit, up_shift, 0, vec};
+    const MoeLinearArgs args{(const bf16_t*)a, a_stride, (const bf16_t*)w, out, o_stride, tiles, meta, sorted, top, gather, K, N, F, act, limit, up_shift, 0, vec, false};
     const dim3 grid(max_tiles, (F + 15) / 16);
 #define MOE_FEW(TO, G)                                                                              \
   do {                                                                                              \

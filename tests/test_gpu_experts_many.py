@@ -96,3 +96,23 @@ def test_more_tiles_than_lanes_a_chiplet(K, experts):
         counts.append(2)
     assert sum((n + 127) // 128 for n in counts) == experts
     _check(K, counts, 72, 136, (72,), (torch.float32,))
+
+
+@pytest.mark.parametrize("Fo,glu", [(2176, False), (1088, True)])
+def test_other_tokens_choices_do_not_change_a_tokens_outputs(K, Fo, glu):
+    """The same bits for the tokens of expert 0 beside 31 experts of 128 rows each and beside 16 of 192 and 15 of the rest: 32 and 48 tiles, on either side of
+    one and a half rounds of workgroups."""
+    E, Kd, P = 32, 512, 4096
+    g = torch.Generator(device=DEV).manual_seed(3)
+    h = torch.randn(P, Kd, device=DEV, generator=g).bfloat16()
+    w = (torch.randn(E, Fo * (2 if glu else 1), Kd, device=DEV, generator=g) / Kd ** 0.5).bfloat16()
+    outs = []
+    for counts in ([128] * 32, [128] + [192] * 16 + [60] * 11 + [59] * 4):
+        chosen = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).to(torch.int32).to(DEV).unsqueeze(1)
+        tables = torch.empty(2 * P + 1 + 3 * K.moe_max_tiles(P, E, 128), dtype=torch.int32, device=DEV)
+        sp, po, meta, tiles = tables[:P], tables[P:2 * P], tables[2 * P:2 * P + 1], tables[2 * P + 1:]
+        K.moe_sort(chosen, E, sp, po, tiles, meta, tile_rows=128)
+        out = torch.empty(P, Fo, device=DEV)
+        K.moe_linear(h, w, out, tiles, meta, sp, top=1, gather=True, glu=glu, activation="silu" if glu else "none", tile_rows=128)
+        outs.append(out[po.long()][:128])
+    assert torch.equal(*outs)
