@@ -146,16 +146,19 @@ gemm_f32_kernel(const float* __restrict__ a, long lda, const float* __restrict__
 // Some hundred rows and more: a workgroup of four waves (2 x 2) owns 32 RT rows and 32 NT outputs, a wave 16 RT x 16 NT of them over the whole
 // of K. Both operands come as whole lines (32 numbers of a row a step, the step after next on its way in registers) and are turned into the
 // instruction's operands by two buffers in LDS, rows of 36 numbers: 16 lanes' reads of 16 bytes fall on all banks. A load's four products of a tile
-// go to SETS sums in turn (so many that none waits for the one before it), which join the tile's sum every 128 or 256 k: no chain of roundings is
-// longer than those of the kernel above (errors against 64 bits at 777 rows: K = 1,024 2.1e-7, before 2.9e-7; 4,096 2.1e-7, before 5.7e-7).
+// go to SETS sums in turn (so many that none waits for the one before it), which join the tile's sum every 128 or 256 k, below GF_SHORT every 64: chains of
+// 128, 128 and 64 numbers for 1, 2 and 4 sets, and of 32 and 16 for 2 and 4 sets of short sums, about a quarter of K as in the kernel above (errors against
+// 64 bits at 777 rows, that kernel's / this one's: K = 1,024 2.9e-7 / 2.1e-7; 4,096 5.7e-7 / 2.1e-7; 256 1.5e-7 / 1.1e-7, with chains of 128 2.05e-7).
 // What bounds it: the matrix pipe (64 x 128 tiles, 4096 x 4096 at 2,048 rows 495 us, 139 TFLOP/s; before 531), of some hundred rows the last round of
 // tiles. A mask on the chunks in the loop cost it 15 %: it waited for loads that had just gone out.
 #define GF_LD 36
+#define GF_SHORT 512  // inputs: below, single chains of 128 would be less exact than the split of K
 template <int RT, int NT, int SETS>
-__global__ void __launch_bounds__(256, RT * NT > 8 ? 1 : 2)
+__global__ void __launch_bounds__(256, 2)
 gemm_f32_tile_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias, const float* residual, long ldr,
                      float* out, long ldo, int M, int N, int K, int act, int n_rows, int n_cols, int vec) {
-  constexpr int BM = 32 * RT, BN = 32 * NT, PIECE = SETS == 1 ? 4 : 8;  // steps whose products are added up before they join the sum
+  constexpr int BM = 32 * RT, BN = 32 * NT;
+  const int piece = K < GF_SHORT ? 2 : SETS == 1 ? 4 : 8;  // steps whose products are added up before they join the sum
   __shared__ __attribute__((aligned(16))) float sm[2][BM + BN][GF_LD];  // rows of a, then of w
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, g = lane >> 4, wm = wave >> 1, wn = wave & 1;
   const int n_tiles = n_rows * n_cols, per = (n_tiles + 7) / 8;  // neighbouring columns of tiles on a chiplet, as above
@@ -255,7 +258,7 @@ gemm_f32_tile_kernel(const float* __restrict__ a, long lda, const float* __restr
   };
   int t = 0;
   while (t + 1 < steps) {
-    const int stop = min(t + PIECE, steps - 1);
+    const int stop = min(t + piece, steps - 1);
     for (; t < stop; t += 2) {
       step(t, 0);
       step(t + 1, 1);
@@ -370,6 +373,7 @@ static int gemm_f32_choose(int M, int N, int K) {  // an index into the first li
   }
   for (int i = 0; i < (int)(sizeof(GEMM_F32_LINE_TILES) / sizeof(GEMM_F32_LINE_TILES[0])); ++i) {
     const GemmF32LineTile& t = GEMM_F32_LINE_TILES[i];
+    if (t.sets < (K < 128 ? 4 : K < GF_SHORT ? 2 : 1)) continue;  // chains longer than a quarter of K
     const double n = ceil((double)((M + 32 * t.rt - 1) / (32 * t.rt)) * ((N + 32 * t.nt - 1) / (32 * t.nt)) / 256.0);
     const double us = t.start + fmax(memory, (K + 31) / 32 * fmax(t.alone + 0.15 * (n - 1) * t.among, n * t.among));
     if (us < best_us) best_us = us, best = GEMM_F32_N_TILES + i;

@@ -56,6 +56,20 @@ def test_linear_float32(K, M, Ki, N, form):
     assert bool(((out.double() - want.clamp(min=0) ** 2 - res.double()).abs() <= (2 * Ki + 8) * EPS * (size ** 2 + res.double().abs())).all())
 
 
+@pytest.mark.parametrize("M,N,Ki", [(2048, 4096, 64), (1024, 3072, 96), (1024, 3072, 128), (2048, 4096, 128), (2048, 2304, 192), (777, 2304, 256), (404, 4096, 384),
+                                    (777, 2304, 384), (777, 1024, 512), (777, 1024, 1024)])
+def test_short_sums_are_no_long_chains(K, M, N, Ki):
+    """Relative error in the 2-norm of products of normal numbers. A rounding is off by 0.42 * 2^-24 of its result (2^-23 / sqrt(12), times the root mean square of
+    1 / x over a power of two); the sums in a chain of c of the K numbers are j / K of the whole's square, j = 1 .. c: chains of c and their K / c joins make
+    0.42 * 2^-24 * sqrt(c / 2 + K / (2 c)). Chains: a quarter of K in steps of 16, at most 128; 15 % for what is drawn and for products of 4 at a time."""
+    a, w = _rand(M, Ki, seed=1).to(DEV), _rand(N, Ki, seed=2).to(DEV)
+    out = torch.empty(M, N, device=DEV)
+    K.linear(a, w, None, out)
+    want = a.double() @ w.double().T
+    c = min(128, -(-Ki // 64) * 16)
+    assert float((out.double() - want).norm() / want.norm()) <= 1.15 * 0.42 * EPS * (c / 2 + Ki / (2 * c)) ** 0.5
+
+
 def test_linear_float32_keeps_infinities_where_they_are(K):
     """An infinite input reaches the outputs of its own row only, also from the last, short step of a wave's inputs."""
     a, w = _rand(20, 52, seed=1).to(DEV), _rand(40, 52, seed=2).to(DEV)
