@@ -147,8 +147,8 @@ gemm_f32_kernel(const float* __restrict__ a, long lda, const float* __restrict__
 // of K. Both operands come as whole lines (32 numbers of a row a step, the step after next on its way in registers) and are turned into the
 // instruction's operands by two buffers in LDS, rows of 36 numbers: 16 lanes' reads of 16 bytes fall on all banks. A load's four products of a tile
 // go to SETS sums in turn (so many that none waits for the one before it), which join the tile's sum every 128 or 256 k, below GF_SHORT every 64: chains of
-// 128, 128 and 64 numbers for 1, 2 and 4 sets, and of 32 and 16 for 2 and 4 sets of short sums, about a quarter of K as in the kernel above (errors against
-// 64 bits at 777 rows, that kernel's / this one's: K = 1,024 2.9e-7 / 2.1e-7; 4,096 5.7e-7 / 2.1e-7; 256 1.5e-7 / 1.1e-7, with chains of 128 2.05e-7).
+// 128, 128 and 64 numbers for 1, 2 and 4 sets, in short sums of 64, 32 and 16, no more than a quarter of K as in the kernel above (errors against
+// 64 bits at 777 rows, that kernel's / this one's: K = 1,024 2.9e-7 / 2.1e-7; 4,096 5.7e-7 / 2.1e-7; 256 1.5e-7 / 1.1e-7 - 1.5e-7, with chains of 128 2.05e-7).
 // What bounds it: the matrix pipe (64 x 128 tiles, 4096 x 4096 at 2,048 rows 495 us, 139 TFLOP/s; before 531), of some hundred rows the last round of
 // tiles. A mask on the chunks in the loop cost it 15 %: it waited for loads that had just gone out.
 #define GF_LD 36
@@ -339,10 +339,12 @@ gemm_f32_few_kernel(const float* __restrict__ a, long lda, const float* __restri
 // Which tile: the fewest microseconds by an estimate from what was measured over 14 weights and 17 .. 2,048 rows (all tiles of both lists).
 // Of the first kernel: the longest of the weights' read from memory (5.2 TB/s), the operands that a CU pulls through its L2 (37 GB/s and CU) and
 // the products of the CU with the most workgroups (waves that fewer than four SIMDs hold leave the others idle). Of the second: its steps on that
-// CU. Within 8 % of the best tile at nearly all of them; the ends: 16 x 16 for 768 x 768 at 4 rows (4.8 us; 64 x 64 19), 64 x 128 of the second for
-// 4096 x 4096 at 2,048 rows (495 us; 16 x 16 of the first 1,790). With the second kernel, before / after: 3072 x 1024 at 777 rows 61 / 48 us, 4096 x 1024
-// 75 / 66, 1024 x 1024 25 / 22, 1024 x 4096 78 / 73, 50257 x 1024 733 / 625, 3072 x 768 at 606 rows 41 / 30, 4096 x 4096 at 404 rows 173 / 133. Below about 100 rows
-// and for long sums into few outputs the first stays ahead: its waves split K (1024 x 4096 at 203 rows 33 us, the second 46).
+// CU (a lone workgroup of 32 x 96 at what it takes with weights that no cache holds; 0.44 us a step with weights in the last cache made it the choice where it is up to
+// 15 % behind: 5120 x 6400 at 100 rows 129 us, 64 x 64 of the first 113). Checked over 1,386 shapes of 512 inputs and more, weights that no cache holds: 0.3 % behind the
+// best tile on average, 18 by more than 5 %, and behind the first kernel's best alone by 4 - 7 % at six, where the second's shorter chains are taken (6400 x 3072 at 100 rows 65 us, the
+// first 61). The ends: 16 x 16 for 16 rows of 768 x 768, 64 x 128 of the second for 4096 x 4096 at 2,048 rows (520 us; 16 x 16 of the first 1,790). Before the second kernel /
+// now: 3072 x 1024 at 777 rows 66 / 54 us, 4096 x 1024 76 / 65, 1024 x 1024 24 / 21, 50257 x 1024 751 / 673, 3072 x 768 at 606 rows 41 / 30, 4096 x 4096 at 404 rows 172 / 135.
+// Below about 100 rows and for long sums into few outputs the first stays ahead: its waves split K (1024 x 4096 at 203 rows 32 us, the second 61; at 777 rows 74 and 76).
 struct GemmF32Tile {
   int rt, nt, w;
   float pipe;   // share of the matrix pipe that the tile reaches
@@ -354,7 +356,7 @@ struct GemmF32LineTile {
   float alone, among;  // microseconds of a step: of the one workgroup on a CU, and of one among several
   float start;
 };
-static const GemmF32LineTile GEMM_F32_LINE_TILES[] = {{1, 1, 4, 0.32f, 0.155f, 0.f},  {1, 2, 2, 0.37f, 0.28f, 0.5f}, {1, 3, 2, 0.44f, 0.395f, 1.f},
+static const GemmF32LineTile GEMM_F32_LINE_TILES[] = {{1, 1, 4, 0.32f, 0.155f, 0.f},  {1, 2, 2, 0.37f, 0.28f, 0.5f}, {1, 3, 2, 0.6f, 0.395f, 1.f},
                                                       {2, 2, 1, 0.6f, 0.5f, 1.f},     {2, 3, 1, 0.76f, 0.73f, 2.f},  {2, 4, 1, 0.98f, 0.96f, 2.5f}};
 #define GEMM_F32_N_TILES (int)(sizeof(GEMM_F32_TILES) / sizeof(GEMM_F32_TILES[0]))
 
@@ -373,13 +375,15 @@ static int gemm_f32_choose(int M, int N, int K) {  // an index into the first li
   }
   for (int i = 0; i < (int)(sizeof(GEMM_F32_LINE_TILES) / sizeof(GEMM_F32_LINE_TILES[0])); ++i) {
     const GemmF32LineTile& t = GEMM_F32_LINE_TILES[i];
-    if (t.sets < (K < 128 ? 4 : K < GF_SHORT ? 2 : 1)) continue;  // chains longer than a quarter of K
+    if (t.sets < (K < 128 ? 4 : K < 256 ? 2 : 1)) continue;  // chains longer than a quarter of K
     const double n = ceil((double)((M + 32 * t.rt - 1) / (32 * t.rt)) * ((N + 32 * t.nt - 1) / (32 * t.nt)) / 256.0);
     const double us = t.start + fmax(memory, (K + 31) / 32 * fmax(t.alone + 0.15 * (n - 1) * t.among, n * t.among));
     if (us < best_us) best_us = us, best = GEMM_F32_N_TILES + i;
   }
   return best;
 }
+
+extern "C" int lev_linear_f32_choice(int M, int N, int K) { return gemm_f32_choose(M, N, K); }  // the tile's place in the two lists, one behind the other
 
 // 1: not for these operands (nothing has been launched): 16-byte loads need rows of a multiple of 4 numbers at 16-byte addresses
 int lev_gemm_f32(const float* a, long lda, const float* w, const float* bias, const float* residual, long ldr, float* out, long ldo, int M, int N, int K,
