@@ -383,19 +383,33 @@ static int gemm_f32_choose(int M, int N, int K) {  // an index into the first li
   return best;
 }
 
-extern "C" int lev_linear_f32_choice(int M, int N, int K) { return gemm_f32_choose(M, N, K); }  // the tile's place in the two lists, one behind the other
+// Rows that the few-row kernel has room for, or 0 where it would be behind the tiles: it reads longer sums faster than their few workgroups, and pays for
+// every row and output with sums over the lanes. The inputs from which on it is level, by its room (1, 2, 4, 8) and the outputs in rounds of 256 workgroups
+// (the last: all further ones), from 317 weights of 16 .. 12,800 outputs and 64 .. 16,384 inputs at 1 .. 8 rows: 4 of the 2,536 shapes are 5 % behind the tiles, none
+// further. Tiles / few, microseconds, 1 / 2 / 4 / 8 rows: 768 x 768 4.5, 4.6, 4.8, 5.0 / 2.8, 3.3, 3.9, 5.3; 768 x 3072 9.8, 10.0, 10.8, 11.7 / 4.2, 5.0, 5.9, 7.7; 1024 x 4096 12.0,
+// 12.2, 13.3, 14.6 / 5.1, 5.6, 6.6, 8.7; 1600 x 1600 7.1, 7.1, 7.3, 7.8 / 4.9, 5.6, 6.6, 11.9; 1600 x 2048 at 8 rows 9.0 / 12.4, 1600 x 4096 14.8 / 14.9; 1200 x 256 at 4
+// rows 3.4 / 4.6; 3072 x 1024 6.0, 6.1, 5.9, 6.3 / 5.3, 5.9, 8.0, 14.9; 4096 x 4096 15.6, 15.0, 14.9, 15.7 / 12.9, 13.1, 15.3, 27.3.
+static const int GEMM_F32_FEW_INPUTS[4][5] = {{0, 0, 256, 256, 768}, {256, 384, 768, 1280, 2048}, {512, 768, 2560, 8192, 8192}, {1024, 4096, 4096, 4096, 4096}};
+static int gemm_f32_few(int M, int N, int K) {
+  if (M < 1 || M > 8 || N < 1) return 0;
+  const int i = M > 4 ? 3 : M > 2 ? 2 : M - 1, rounds = (N - 1) / (256 * GF_FEW_OUT);
+  if (((long)N << i) > (K >= 2048 ? 12800 : 6400)) return 0;
+  return K >= GEMM_F32_FEW_INPUTS[i][rounds < 4 ? rounds : 4] ? 1 << i : 0;
+}
+
+// the kernel of a product: 0 less the few-row kernel's room, or the tile's place in the two lists, one behind the other
+extern "C" int lev_linear_f32_choice(int M, int N, int K) {
+  const int few = gemm_f32_few(M, N, K);
+  return few > 0 ? -few : gemm_f32_choose(M, N, K);
+}
 
 // 1: not for these operands (nothing has been launched): 16-byte loads need rows of a multiple of 4 numbers at 16-byte addresses
 int lev_gemm_f32(const float* a, long lda, const float* w, const float* bias, const float* residual, long ldr, float* out, long ldo, int M, int N, int K,
                  int act, hipStream_t stream) {
   if (K % 4 != 0 || lda % 4 != 0 || ((uintptr_t)a & 15) != 0 || ((uintptr_t)w & 15) != 0) return 1;
   const int vec = ldo % 4 == 0 && ((uintptr_t)out & 15) == 0 && (!bias || ((uintptr_t)bias & 15) == 0) && (!residual || (ldr % 4 == 0 && ((uintptr_t)residual & 15) == 0));
-  // Measured against the best tile, 1 / 2 / 4 / 8 rows, microseconds before and now: 768 x 768 4.5, 4.6, 4.8, 5.0 / 2.8, 3.3, 3.9, 5.3; 768 x 3072 9.8, 10.0, 10.8,
-  // 11.7 / 4.2, 5.0, 5.9, 7.7; 1024 x 4096 12.0, 12.2, 13.3, 14.6 / 5.1, 5.6, 6.6, 8.7; 1600 x 1600 7.1, 7.1, 7.3, 7.8 / 4.9, 5.6, 6.6, 11.9; 1600 x 6400 17.8, 18.1, 19.3,
-  // 21.3 / 10.1, 11.1, 12.9, 20.2; 3072 x 1024 6.0, 6.1, 5.9, 6.3 / 5.3, 5.9, 8.0, 14.9; 4096 x 4096 15.6, 15.0, 14.9, 15.7 / 12.9, 13.1, 15.3, 27.3: the more rows, the
-  // fewer outputs (sums over the lanes), the longer K, the more (the tiles' few workgroups read it).
-  const int few = M > 8 ? 0 : M > 4 ? 8 : M > 2 ? 4 : M;
-  if (few > 0 && (long)few * N <= (K >= 2048 ? 12800 : 6400) && (few < 8 || K >= 1024)) {
+  const int choice = lev_linear_f32_choice(M, N, K), few = -choice, line = choice - GEMM_F32_N_TILES;
+  if (few > 0) {
 #define GEMM_F32_FEW(MR) \
   if (few == MR) gemm_f32_few_kernel<MR><<<(N + GF_FEW_OUT - 1) / GF_FEW_OUT, 512, 0, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act)
     GEMM_F32_FEW(1);
@@ -405,7 +419,6 @@ int lev_gemm_f32(const float* a, long lda, const float* w, const float* bias, co
 #undef GEMM_F32_FEW
     return lev_check_launch("linear (32-bit, few rows)");
   }
-  const int choice = gemm_f32_choose(M, N, K), line = choice - GEMM_F32_N_TILES;
   const int rt = line < 0 ? GEMM_F32_TILES[choice].rt : 2 * GEMM_F32_LINE_TILES[line].rt, nt = line < 0 ? GEMM_F32_TILES[choice].nt : 2 * GEMM_F32_LINE_TILES[line].nt;
   const int n_rows = (M + 16 * rt - 1) / (16 * rt), n_cols = (N + 16 * nt - 1) / (16 * nt);
   const long blocks = ((long)n_rows * n_cols + 7) / 8 * 8;
