@@ -13,7 +13,8 @@
 //   * a run of several tokens: 16 consecutive query tokens of one query head; the 8 waves of a workgroup are a tile of up
 //     to 128 tokens and share every block of keys and values through LDS (attention_values_mfma_runs_kernel);
 //   * a single token: the query heads of one key/value head (up to 16 at a time); operands go from the pages straight
-//     into registers, and a token's keys may be split over several waves whose results a second kernel merges.
+//     into registers, and a token's keys may be split over several waves, whose results their workgroup merges through LDS or, where there
+//     are too many or their reads would crowd one CU, a second kernel.
 // A wave walks the keys in blocks of 64, keeps a running maximum and sum per column, and applies the weights to the
 // values of up to NVC value heads (blockIdx.z picks which): its own one, or, for layers that mix the weights over the
 // heads afterwards, every key/value head in turn.
@@ -605,20 +606,26 @@ static int av_room(int NV) {  // value heads of a wave of the kernels without sh
   while (room < NV && room < NVC) room *= 2;
   return room;
 }
-// Whether a token's ranges are the waves of one workgroup. That saves a launch and a way through memory (4 - 5 us) and puts their reads on one CU, which
-// takes about 50 KB a microsecond: not where that CU then reads over 192 KB more than if the waves lay apart. 8 tokens of 240 keys, four ranges: heads of
-// 256 / 224 (184 KB more) 0.6 us ahead as one workgroup, 4 heads of 128 / 64 (74 KB) 12.1 us before, 8.3 now, 32 tokens of 180 keys (25 KB) 12.4 / 7.9.
-static bool av_merged(int splits, int NV, int groups, long reach) {
+// Whether a token's ranges are the waves of one workgroup. That saves a launch and a way through memory and puts their reads on one CU, which takes about 50
+// KB a microsecond: not where that CU then reads over 192 KB more than if the waves lay apart. Over 11 pairs of head sizes, 1 .. 128 tokens of 70 .. 2,000 keys (pages that
+// no cache holds) 541 launches merge, at 0.94 - 1.61 times the speed of two, 1.29 on average; 5 of them, with ranges of 1,000 keys or right at the limit, are 3 - 6 % slower. 8 tokens
+// of 240 keys, four ranges, before / now: heads of 256 / 224 (180 KB more) 11.3 / 8.7 us, 4 heads of 128 / 64 (72 KB) 8.6 / 6.9.
+static bool av_merged(int n_singles, int splits, int H, int KVH, int NV, int window, int chunk, int keep, int max_keys) {
   const int room = av_room(NV);
   if (splits <= 1 || splits > (room == 1 ? av_waves<1>() : room == 2 ? av_waves<2>() : room == 4 ? av_waves<4>() : av_waves<8>())) return false;
+  const long groups = (long)n_singles * KVH * ((H / KVH + 15) / 16) * (NV == 1 ? 1 : (NV + NVC - 1) / NVC);
+  long reach = window > 0 && window < max_keys ? window : max_keys;
+  if (chunk > 0 && chunk < reach) reach = chunk;
+  reach += keep > 0 ? keep : 0;
   const long wave_bytes = ((reach + 63) / 64 + splits - 1) / splits * 64 * (HD + (NV < room ? NV : room) * VD) * 2;
-  const long apart = ((long)groups * splits + 255) / 256, together = ((long)groups + 255) / 256 * splits;
+  const long apart = (groups * splits + 255) / 256, together = (groups + 255) / 256 * splits;
   return (together - apart) * wave_bytes <= 192 * 1024;
 }
 
-// bytes of scratch memory for n single tokens whose keys are split `splits` ways
-extern "C" long lev_attention_values_mfma_workspace(int n_singles, int splits, int H, int NV) {
-  return splits <= 1 ? 0 : (long)n_singles * splits * H * ((long)NV * VD + 2) * (long)sizeof(float);
+// bytes of scratch memory for n single tokens whose keys are split `splits` ways; none where a workgroup merges them
+extern "C" long lev_attention_values_mfma_workspace(int n_singles, int splits, int H, int KVH, int NV, int window, int chunk, int keep, int max_keys) {
+  if (splits <= 1 || n_singles <= 0 || KVH <= 0 || av_merged(n_singles, splits, H, KVH, NV, window, chunk, keep, max_keys)) return 0;
+  return (long)n_singles * splits * H * ((long)NV * VD + 2) * (long)sizeof(float);
 }
 
 extern "C" int lev_attention_values_mfma(const void* q, long q_stride, float* out, const void* k_pages, const void* v_pages,
@@ -631,8 +638,9 @@ extern "C" int lev_attention_values_mfma(const void* q, long q_stride, float* ou
   LEV_REQUIRE(NV == 1 || NV == KVH, "attention: %d value heads per query head (1 or kv_heads=%d)", NV, KVH);
   LEV_REQUIRE(PS > 0 && PS % 16 == 0, "attention: page_size=%d must be a multiple of 16", PS);
   LEV_REQUIRE(window >= 0 && chunk >= 0 && keep >= 0 && softcap >= 0.f, "attention: window=%d, chunk=%d, kept positions %d and soft cap %g must not be negative", window, chunk, keep, (double)softcap);
-  LEV_REQUIRE(splits >= 1 && splits <= MERGE_MAX_SPLITS && (splits == 1 || workspace), "attention: %d splits (at most %d) need scratch memory", splits,
-              MERGE_MAX_SPLITS);
+  LEV_REQUIRE(splits >= 1 && splits <= MERGE_MAX_SPLITS, "attention: %d splits (at most %d)", splits, MERGE_MAX_SPLITS);
+  const bool merged = n_singles > 0 && av_merged(n_singles, splits, H, KVH, NV, window, chunk, keep, max_keys);
+  LEV_REQUIRE(splits == 1 || merged || workspace, "attention: %d splits (at most %d) need scratch memory", splits, MERGE_MAX_SPLITS);
   LEV_REQUIRE(n_tiles >= 0 && n_singles >= 0 && (n_tiles == 0 || tiles) && (n_singles == 0 || singles), "attention: bad work lists");
   LEV_REQUIRE(((uintptr_t)q & 15) == 0 && q_stride % 8 == 0 && ((uintptr_t)k_pages & 15) == 0 && ((uintptr_t)v_pages & 15) == 0 &&
                   ((uintptr_t)out & 15) == 0,
@@ -691,9 +699,6 @@ extern "C" int lev_attention_values_mfma(const void* q, long q_stride, float* ou
   }
   if (n_singles > 0) {
     const int group = H / KVH;
-    long reach = window > 0 && window < max_keys ? window : max_keys;
-    if (chunk > 0 && chunk < reach) reach = chunk;
-    const bool merged = av_merged(splits, NV, n_singles * KVH * ((group + 15) / 16) * chunks, reach + (keep > 0 ? keep : 0));
     dim3 grid(merged ? n_singles : n_singles * splits, KVH * ((group + 15) / 16), chunks);
     float* part_o = workspace;
     float* part_ml = splits > 1 && !merged ? workspace + (size_t)n_singles * splits * H * NV * VD : nullptr;

@@ -754,7 +754,7 @@ class HipKernels:
             # single tokens: the keys of one token are split over several waves where the step's tokens alone leave the chip
             # empty (about 1,024 waves are aimed at, a block of 64 keys at least per wave); the step's description keeps the
             # choice and the scratch memory for all layers with these sizes
-            key = ("values", n_heads, n_kv_heads, value_dim, nv, int(window) if window else 0, int(chunk) if chunk else 0, int(keep_first))
+            key = ("values", n_heads, n_kv_heads, head_dim, value_dim, nv, int(window) if window else 0, int(chunk) if chunk else 0, int(keep_first))
             plan = meta.plans.get(key)
             if plan is None:
                 splits = 1
@@ -765,7 +765,7 @@ class HipKernels:
                         reach = min(reach, int(chunk))
                     most = max(1, (reach + 63) // 64 + (1 if window or chunk else 0) + ((int(keep_first) + 63) // 64 if window or chunk else 0))
                     splits = int(max(1, min(most, 32, 1024 // max(1, meta.n_decode * n_kv_heads * chunks))))
-                need = lib.lev_attention_values_mfma_workspace(meta.n_decode, splits, n_heads, nv) if splits > 1 else 0
+                need = lib.lev_attention_values_mfma_workspace(meta.n_decode, splits, n_heads, n_kv_heads, nv, *key[-3:], int(meta.max_kv_len)) if splits > 1 else 0
                 ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
                 plan = meta.plans[key] = (splits, ws)
             splits, ws = plan

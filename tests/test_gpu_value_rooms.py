@@ -88,3 +88,38 @@ def test_ranges_of_keys_that_one_workgroup_merges(G, dk, dv, talking, keys, wind
     talk = as_bf16_numbers(torch.eye(H) + 0.5 * torch.randn(H, H, generator=g)) if talking else None
     args = (H, G, dk, dv, runs, window, None, 4.0 / math.sqrt(dk), q, k, v, talk, None)
     torch.testing.assert_close(run_attention(torch.bfloat16, *args), plain_attention(*args), **tol(torch.bfloat16, bf16=3e-2))
+
+
+@pytest.mark.parametrize("G,dk,dv,talking", [(1, 128, 64, False), (2, 64, 32, True), (1, 256, 224, False), (3, 32, 32, True)])
+@pytest.mark.parametrize("keys", [65, 129, 250, 449])
+def test_a_workgroups_merge_is_the_second_kernels(G, dk, dv, talking, keys):
+    """The same ranges, merged by their workgroup without scratch memory and, the step said to reach so many keys that its reads would crowd a CU, by the
+    second kernel: the same bits."""
+    from levanter_amd.kernels import build, get_kernels
+
+    kern, H, ps, dev = get_kernels(), 2 * G, 16, "cuda:0"
+    lens = [keys, 1, 64, keys - 1]
+    g = torch.Generator(device=dev).manual_seed(keys + dk)
+    pages = sum(-(-n // ps) for n in lens)
+    bt = random_block_tables(lens, ps, pages, 1, dev)
+    q = torch.randn(len(lens), H * dk, device=dev, generator=g).bfloat16()
+    k_pages, v_pages = (torch.randn(pages, G * d * ps, device=dev, generator=g).bfloat16() for d in (dk, dv))
+    nv = G if talking else 1
+    sinks = torch.randn(H, device=dev, generator=g)
+    meta, outs = make_meta([(1, n) for n in lens], dev), []
+    lib = kern._unit(build.attention_values_unit(dk, dv))
+    for many in (False, True):
+        if many:
+            ((key, (splits, scratch)),) = meta.plans.items()
+            if splits == 1 or (splits > 4 and dk == 256):
+                return  # one range, or more than a workgroup merges
+            assert scratch is None
+            meta.max_kv_len = 1 << 20
+            need = lib.lev_attention_values_mfma_workspace(len(lens), splits, H, G, nv, 0, 0, 0, meta.max_kv_len)
+            assert need == len(lens) * splits * H * (nv * dv + 2) * 4
+            meta.plans[key] = (splits, torch.empty(need, dtype=torch.uint8, device=dev))
+        out = torch.empty(len(lens), H, nv, dv, device=dev)
+        kern.attention_values(q, out, k_pages, v_pages, meta, n_heads=H, n_kv_heads=G, head_dim=dk, value_dim=dv, all_value_heads=talking, page_size=ps,
+                              scale=dk ** -0.5, window=None, block_tables=bt, sinks=sinks)
+        outs.append(out)
+    assert torch.equal(*outs)
