@@ -19,9 +19,9 @@ def _rand(*shape, seed=0):
     return torch.randn(*shape, generator=torch.Generator().manual_seed(seed))
 
 
-# rows, inputs, outputs: every tile of the list (rows x outputs of 16 x 16 .. 64 x 128), at its edges, one more and one less; inputs that are
-# no multiple of a step of 16, fewer than the waves have steps, and (no multiple of 4) none that 16-byte loads take. (13, 264, 50257) takes
-# 16 x 32 and (15, 264, 11531) 16 x 64.
+# rows, inputs, outputs: every tile whose operands come straight from memory (16 x 16 .. 32 x 64 here, 64 x 64 at the end), at its edges, one more and one less; inputs
+# that are no multiple of a step of 16, fewer than the waves have steps, and (no multiple of 4) none that 16-byte loads take. (13, 264, 50257) takes
+# 16 x 32 and (15, 264, 11531) 16 x 64. That all kernels are among them is a test below.
 LINEAR = [(1, 4, 1), (1, 64, 50), (3, 768, 768), (16, 100, 48), (17, 772, 33), (31, 1024, 130), (33, 20, 65), (64, 256, 4096), (65, 300, 1024), (129, 1028, 257),
           (203, 516, 1000), (400, 128, 1030), (777, 260, 1024), (1031, 96, 3000), (15, 264, 11531), (13, 264, 50257), (5, 6, 40), (70, 333, 129)]
 # the tiles whose operands come through LDS (32 x 32, 32 x 64, 32 x 96, 64 x 64, 64 x 96, 64 x 128): ends inside a tile, K of one step, with a short one, of
@@ -29,8 +29,16 @@ LINEAR = [(1, 4, 1), (1, 64, 50), (3, 768, 768), (16, 100, 48), (17, 772, 33), (
 LINEAR += [(404, 768, 3072), (289, 100, 2051), (1031, 32, 3001), (801, 1028, 1030), (777, 300, 3072), (2047, 292, 4097), (609, 516, 2310), (2047, 260, 2310),
            (1000, 260, 4097), (1030, 1028, 4100), (2047, 516, 3071)]
 # up to eight rows and four outputs a workgroup: 1, 2, 4 and 8 rows' room full and not, outputs that end inside a workgroup, K of less than a thread each,
-# one stretch of 2,048, two, a short one more; and just beyond the rule's lines
+# one stretch of 2,048, two, a short one more; and shapes that the rule gives to the tiles
 LINEAR += [(1, 8196, 64), (2, 1028, 3001), (3, 4100, 130), (4, 2048, 1601), (5, 2052, 33), (8, 1024, 777), (7, 4096, 1600), (8, 1020, 40), (4, 1600, 1601), (1, 100, 6401)]
+
+# 64 x 64 straight from memory: rows and outputs that end inside a tile, K with a short last step, of short and long sums
+LINEAR += [(935, 228, 8317), (129, 3396, 4949), (195, 3364, 3558), (777, 4100, 1030)]
+
+
+def test_every_kernel_is_among_the_shapes(K):
+    """Room for 8, 4, 2 and 1 rows (-8 .. -1), seven tiles straight from memory, six through LDS."""
+    assert {K.lib.lev_linear_f32_choice(M, N, Ki) for M, Ki, N in LINEAR if Ki % 4 == 0} == {-8, -4, -2, -1, *range(13)}
 
 
 @pytest.mark.parametrize("M,Ki,N", LINEAR)
@@ -80,6 +88,42 @@ def test_linear_float32_keeps_infinities_where_they_are(K):
     assert torch.equal(torch.isinf(out), torch.isinf(want)) and not bool(torch.isnan(out).any())
     keep = [r for r in range(20) if r != 7]
     torch.testing.assert_close(out[keep], want[keep], rtol=1e-5, atol=52 * EPS * 50)
+
+
+@pytest.mark.parametrize("M,Ki,N", [(289, 100, 2051), (609, 516, 2310), (1030, 1028, 4100), (129, 3396, 4949), (1, 8196, 64), (3, 4100, 130), (8, 1028, 777)])
+def test_linear_float32_keeps_infinities_where_they_are_in_every_kernel(K, M, Ki, N):
+    """Tiles through LDS with a short step of one, two and four sums, 64 x 64 straight from memory, and rooms for 1, 4 and 8 rows whose last stretch is short: an infinite last
+    input reaches its own row, an infinite last weight its own output, and nothing else is anything but finite."""
+    a, w = _rand(M, Ki, seed=1).to(DEV), _rand(N, Ki, seed=2).to(DEV)
+    row, col = M // 2, N // 2
+    a[row, Ki - 1] = float("inf")
+    w[col, Ki - 1] = float("-inf")
+    out = torch.empty(M, N, device=DEV)
+    K.linear(a, w, None, out)
+    want = torch.zeros(M, N, dtype=torch.bool, device=DEV)
+    want[row] = want[:, col] = True
+    assert torch.equal(torch.isinf(out), want) and not bool(torch.isnan(out).any())
+    assert torch.equal(out[row] > 0, w[:, Ki - 1] > 0)
+
+
+def test_a_waves_sum_is_the_tree_over_lane_numbers(K):
+    """Every lane's number is exact (one of four inputs counts), so that the sums are those of the 64 lanes, halves first, then of neighbours 16, 8, 4, 2 and 1 apart, and of the
+    eight waves in order, bit by bit."""
+    a = torch.randn(1, 2048, generator=torch.Generator().manual_seed(1)) * torch.logspace(-3, 3, 2048)
+    w = torch.zeros(64, 2048)
+    for n in range(64):
+        w[n, n % 4::4] = 1.0
+    assert K.lib.lev_linear_f32_choice(1, 64, 2048) == -1
+    out = torch.empty(1, 64, device=DEV)
+    K.linear(a.to(DEV), w.to(DEV), None, out)
+    for n in range(4):
+        v = a[0, n::4].reshape(8, 64)
+        for apart in (32, 16, 8, 4, 2, 1):
+            v = v + v[:, torch.arange(64) ^ apart]
+        total = torch.zeros(())
+        for part in v[:, 0]:
+            total = total + part
+        assert bool((out[0, n::4].cpu() == total).all())
 
 
 def _attention_float64(q, kp, vp, bt, runs, H, KVH, HD, PS, scale, window):
