@@ -31,9 +31,10 @@ __device__ __forceinline__ void gemm_f32_store(gf_f32x4 v, const float* bias, co
 // row. Both operands come straight from global memory, 16 bytes a lane (row = lane % 16, k = 4 (lane / 16) + j for the j-th of the
 // four products of a step): the 32-bit instruction takes 32 cycles for 1,024 multiply-adds, which hides much of what such loads cost
 // the vector cache (a look-up for every lane).
-// What bounds it: few rows, the read of the weights (4096 x 4096 at 4 rows 14.3 us, 4.7 TB/s; 768 x 768 4.8 us, a launch and a chain of
-// loads); some dozens, L2 at about 9.5 TB/s (1024 x 4096 at 203 rows 33 us) or the last round of tiles. The plain kernel of
-// gemm_simple.hip (64 x 64 tiles, vector ALU, scalar loads) took 84 us for 768 x 768 at 4 rows, 378 us for 768 x 3072 (now 4.8 and 10).
+// What bounds it: few rows, the read of the weights (4096 x 4096 at 4 rows 14.3 us, 4.7 TB/s; 768 x 768 at 16 rows 5.3 us, a launch and a chain of
+// loads); some dozens, L2 at about 9.5 TB/s (1024 x 4096 at 203 rows 32 us) or the last round of tiles. The plain kernel of
+// gemm_simple.hip (64 x 64 tiles, vector ALU, scalar loads) took 84 us for 768 x 768 at 4 rows, 378 us for 768 x 3072 (this one 4.8 and 10; with so few rows
+// and outputs the few-row kernel below goes before it, 3.9 and 5.9).
 template <int RT, int NT, int W>
 __global__ void __launch_bounds__(64 * W)
 gemm_f32_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
@@ -281,7 +282,7 @@ gemm_f32_tile_kernel(const float* __restrict__ a, long lda, const float* __restr
 
 // Up to eight rows and few outputs: 16 of them a workgroup would leave most CUs without one. A workgroup of eight waves owns four outputs; a thread
 // multiplies 16 bytes of each weight row with every row of a, two stretches of 2,048 k on their way at once, and the partial sums go over the lanes
-// and, through LDS, over the waves: chains of a dozen roundings (errors 0.8e-7 .. 1.1e-7; the 16-output tiles 1.9e-7 .. 5e-7).
+// and, through LDS, over the waves: chains of 4 ceil(K / 2048) + 13 roundings (errors 0.8e-7 .. 1.1e-7 up to K = 6,400; the 16-output tiles 1.9e-7 .. 5e-7).
 // What bounds it: a launch, one read of the weights (768 x 3072 at 4 rows 5.9 us, 1.6 TB/s) and 4 sums over the lanes for every row.
 #define GF_FEW_OUT 4
 template <int MR>
