@@ -1,18 +1,20 @@
 // bfloat16 matrix products on the matrix cores (MFMA), 32-bit accumulation, fused epilogue:
 //   y = act(a . w^T + bias) (+ residual),  a [M, K] (row stride lda), w [N, K], y [M, N] bf16 or f32.
-// Three kernels, chosen by M:
-//   tile kernel   (M > 128): a 256x256, 256x192, 256x128, 128x128 or 128x64 tile per workgroup of 4 waves, 32x32x16 MFMA,
+// Three kernels here and one in gemm_ring.hip, chosen by the sizes:
+//   ring kernel   (M > 64 and fewer than four million outputs: use_ring): in gemm_ring.hip;
+//   tile kernel   (more outputs, M > 128): a 256x256, 256x192, 256x128 or 128x128 tile per workgroup of 4 waves, 32x32x16 MFMA,
 //                 (K split into ranges, with a second kernel for the sums, where the tiles alone would leave CUs idle)
 //                 operands staged through LDS (two buffers), the next k-tile's global loads in registers meanwhile;
-//   stream kernel (M <= 128; up to 64 rows where an estimate puts it ahead of the skinny kernel: long sums, many rows): the weights are the traffic; `a` is shared through LDS by the 4 to 16 waves of a
+//   stream kernel (M <= 64, and up to 128 rows of more than 32,768 outputs; where an estimate puts it ahead of the skinny kernel: long sums, many rows): the weights are the traffic; `a` is shared through LDS by the 4 to 16 waves of a
 //                 workgroup, the weights go straight into MFMA operand registers, K is split over workgroups
 //                 and a second kernel adds the partial sums in a fixed order;
-//   skinny kernel (M <= 64, small weights to 256 rows, see use_skinny): a workgroup owns 8 to 64 output columns; its waves split K, bring whole lines of w
+//   skinny kernel (M <= 64, the smallest weights to 256 rows, see use_skinny): a workgroup owns 8 to 64 output columns; its waves split K, bring whole lines of w
 //                 and a through an LDS area of their own into MFMA operand registers (16x16x32), and their partial sums are
 //                 added through LDS in a fixed order.
 // No atomics anywhere: results are deterministic. K and lda must be multiples of 8 (16-byte operand loads);
 // any M and N.
 #include "common.h"
+#include "gemm_ring.h"
 #include <type_traits>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
@@ -529,25 +531,16 @@ struct SkinnyShape {
   bool half;
   int cols() const { return half ? 8 : 16 * units; }
 };
-// Above 64 rows the rows are cut into blocks (the grid's y; its x a multiple of 8, so that the blocks of a column tile share a chiplet's L2):
-// every workgroup has a CU of its own, waves that split K need no barrier, and all their loads are out at once, where a tile kernel of
-// barriers and the library wait for memory at every step. Measured in graphs over distinct weights, microseconds, here / the better of
-// the library and the stream or tile kernel: 4800 x 1600 at 96 / 128 / 192 rows 9.6 / 12.7, 9.7 / 13.4, 10.3 / 16.8; 6400 x 1600 at 96 / 128 rows
-// 12.6 / 17.3, 13.0 / 17.7; 1600 x 1600 at 96 / 192 / 256 rows 7.0 / 11.0, 7.7 / 11.2, 7.7 / 12.4; 2304 x 768 5.4 / 7.1, 6.0 / 7.5, 7.4 / 7.7. In two
-// rounds it is behind (4800 x 1600 at 256 rows 17.0 / 17.2, 6400 x 1600 20.1 / 17.7, 12288 x 4096 at 96 rows 34.6 / 30.1), and for
-// long sums the kernels that split K over workgroups are ahead (1600 x 6400 at 96 rows 17.7 / 12.4).
-static bool skinny_blocks_fit(int M, int N, int row_tiles, int units) {
-  const long columns = (N + 16 * units - 1) / (16 * units);
-  return (M + 16 * row_tiles - 1) / (16 * row_tiles) * ((columns + 7) / 8 * 8) <= 256;
+// Above 64 rows the rows are cut into blocks of 32 (the grid's y; its x a multiple of 8, so that the blocks of a column tile share a chiplet's L2) where 32 x 32
+// outputs a workgroup make one round of the CUs: waves that split K need no barrier, and all their loads are out at once. Measured in graphs over
+// distinct weights, microseconds, here / the ring kernel: 768 x 768 at 96 / 256 rows 4.5 / 5.0, 5.1 / 5.5; 1024 x 1024 at 256 rows 5.8 / 6.4; 2048 x 2048 at 96 /
+// 128 rows 6.5 / 7.1, 7.3 / 7.5; 2304 x 768 at 96 rows 5.0 / 5.2. Beyond one round the ring kernel is ahead (2304 x 768 at 128 rows 5.7 / 5.2, 2048 x 2048 at 160 rows
+// 8.5 / 7.6, 4800 x 1600 at 96 rows in blocks of 64 x 48 9.6 / 6.9), and for long sums.
+static bool skinny_in_blocks(int M, int N, int K) {
+  return M > 64 && M <= SKINNY_MAX_M && K <= 2048 && (long)((M + 31) / 32) * (((N + 31) / 32 + 7) / 8 * 8) <= 256;
 }
-static bool skinny_in_blocks(int M, int N, int K) { return M > 64 && M <= SKINNY_MAX_M && K <= 2048 && skinny_blocks_fit(M, N, 4, 4); }
 static SkinnyShape skinny_shape(int M, int N, int K) {
-  if (M > 64) {  // the smallest blocks that make one round
-    if (skinny_blocks_fit(M, N, 2, 2)) return {8, 2, 2, 2, false};
-    for (int units = 2; units < 4; ++units)
-      if (skinny_blocks_fit(M, N, 4, units)) return {8, 1, 4, units, false};
-    return {8, 1, 4, 4, false};
-  }
+  if (M > 64) return {8, 2, 2, 2, false};
   const int tiles = (N + 15) / 16;
   if (M <= 16) {
     if (N <= 2048) return K > 4096 && M <= 8 ? SkinnyShape{16, 2, 1, 1, true} : SkinnyShape{8, 2, 1, 1, true};
@@ -576,19 +569,11 @@ static void launch_skinny(const bf16_t* a, long lda, const bf16_t* w, const floa
 #define LEV_SKINNY(W_, U_, MT_, NT_, H_)                                                                                          \
   if (sh.waves == W_ && sh.in_flight == U_ && sh.row_tiles == MT_ && sh.units == NT_ && sh.half == H_)                             \
     gemm_skinny_kernel<TO, W_, U_, MT_, NT_, H_, false><<<columns, W_ * 64, 0, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act)
-  // row blocks are a variant of their own: what finds them costs the small steps' kernels 0.2 - 0.4 us
-#define LEV_SKINNY_BLOCKS(U_, MT_, NT_)                                                                                           \
-  if (sh.row_tiles == MT_ && sh.units == NT_)                                                                                     \
-    gemm_skinny_kernel<TO, 8, U_, MT_, NT_, false, true><<<grid, 8 * 64, 0, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act)
-  if (M > 64) {
-    const dim3 grid((columns + 7) / 8 * 8, (M + 16 * sh.row_tiles - 1) / (16 * sh.row_tiles));
-    LEV_SKINNY_BLOCKS(2, 2, 2);
-    LEV_SKINNY_BLOCKS(1, 4, 2);
-    LEV_SKINNY_BLOCKS(1, 4, 3);
-    LEV_SKINNY_BLOCKS(1, 4, 4);
+  if (M > 64) {  // row blocks are a variant of their own: what finds them costs the small steps' kernels 0.2 - 0.4 us
+    const dim3 grid((columns + 7) / 8 * 8, (M + 31) / 32);
+    gemm_skinny_kernel<TO, 8, 2, 2, 2, false, true><<<grid, 8 * 64, 0, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act);
     return;
   }
-#undef LEV_SKINNY_BLOCKS
   LEV_SKINNY(16, 2, 1, 1, true);
   LEV_SKINNY(8, 2, 1, 1, true);
   LEV_SKINNY(8, 2, 1, 1, false);
@@ -869,28 +854,26 @@ static StreamPlan plan_stream(int M, int N, int K) {
   return best;
 }
 
-// Tile shape and number of k ranges for M > 128. Estimated time of each tile shape: rounds of workgroups over the 256
+// Tile shape and number of k ranges of the tile kernel. Estimated time of each tile shape: rounds of workgroups over the 256
 // CUs times (k-tiles x the shape's time per k-tile + a fixed cost for a tile's first loads and its epilogue). Two
 // 128 x 128 workgroups fit a CU and then share it; up to 256 of them have a CU each. Where the output has so few
 // tiles that most CUs would idle (a few hundred rows times a narrow weight), K is split into ranges, as in the
 // stream kernel: the second kernel then costs its launch and the traffic of the partial sums. The constants are
 // microseconds measured on MI355X.
 struct TilePlan {
-  int shape;   // 0: 256 x 256, 1: 256 x 192, 2: 256 x 128, 3: 128 x 128, 4: 128 x 64
+  int shape;   // 0: 256 x 256, 1: 256 x 192, 2: 256 x 128, 3: 128 x 128
   int splits;  // k ranges (1: none)
 };
 static TilePlan plan_tiles(int M, int N, int K) {
-  static const int bm[5] = {256, 256, 256, 128, 128}, bn[5] = {256, 192, 128, 128, 64};
-  static const double us_per_ktile[5] = {1.72, 1.36, 0.97, 0.6, 0.4}, fixed[5] = {13.0, 11.0, 9.0, 7.0, 6.0};
+  static const int bm[4] = {256, 256, 256, 128}, bn[4] = {256, 192, 128, 128};
+  static const double us_per_ktile[4] = {1.72, 1.36, 0.97, 0.6}, fixed[4] = {13.0, 11.0, 9.0, 7.0};
   const long nk = (K + TK - 1) / TK;
   TilePlan best = {0, 1};
   double best_cost = 1e30;
-  for (int i = 0; i < 5; ++i) {
+  for (int i = 0; i < 4; ++i) {
     const long tiles = (long)((M + bm[i] - 1) / bm[i]) * ((N + bn[i] - 1) / bn[i]);
     double cost;
-    if (i == 4 && tiles > 256)
-      continue;  // the small tile is for outputs that would leave CUs idle otherwise
-    else if (i == 3 && tiles > 256)
+    if (i == 3 && tiles > 256)
       cost = (double)((tiles + 511) / 512) * (nk * 1.05 + 9.0);
     else
       cost = (double)((tiles + 255) / 256) * (nk * us_per_ktile[i] + fixed[i]);
@@ -951,9 +934,22 @@ static bool use_skinny(int M, int N, int K) {
   return skinny_estimate(M, N, K) <= 2.3 + 1.17 * plan.cost * (plan.splits == 1 && K % 2048 == 0 ? 1.2 : 1.0);
 }
 
+// Where the ring kernel is ahead of the library and of the kernels here, measured at 25 weights of 512 x 2048 to 16384 x 4096 and 65 to 2,048 rows (microseconds, before /
+// ring; the library's kernels are chosen by timing): below 2^22 outputs 0.9 to 1.9 times as fast; above, 12288 x 4096 at 400 / 512 rows 54.7 / 59, 55.8 / 77, 6400 x 1600
+// at 1,000 28.9 / 37, 4096 x 2048 at 2,048 34 / 45. Heads of more outputs than a layer has stay where they were: 50257 x 768 at 65 rows 23.4 / 29.8.
+static bool use_ring(int M, int N, int K) { return M > 64 && N <= 32768 && (long)M * N < (1L << 22) && !use_skinny(M, N, K); }
+
+// The tile and the ranges of the ring kernel, 16 x tile + ranges; -1 where another kernel takes the product.
+extern "C" int lev_linear_mfma_ring(int M, int N, int K) {
+  if (!use_ring(M, N, K)) return -1;
+  const RingPlan plan = lev_ring_plan(M, N, K);
+  return 16 * plan.shape + plan.splits;
+}
+
 // Into how many ranges the sum over K is split (1: the kernel finishes its outputs itself).
 extern "C" int lev_linear_mfma_ranges(int M, int N, int K) {
   if (use_skinny(M, N, K)) return 1;
+  if (use_ring(M, N, K)) return lev_ring_plan(M, N, K).splits;
   return M <= 128 ? plan_stream(M, N, K).splits : plan_tiles(M, N, K).splits;
 }
 
@@ -1008,6 +1004,11 @@ static int linear_mfma_typed(const bf16_t* a, long lda, const bf16_t* w, const f
                              TO* out, long ldo, float* workspace, int M, int N, int K, int act, int defer, hipStream_t stream) {
   if (use_skinny(M, N, K)) {
     launch_skinny<TO>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act, stream);
+  } else if (use_ring(M, N, K)) {
+    const RingPlan plan = lev_ring_plan(M, N, K);
+    const int rc = lev_ring_launch(plan, a, lda, w, bias, residual, ldr, out, ldo, workspace, M, N, K, act, sizeof(TO) == 4 ? LEV_F32 : LEV_BF16, stream);
+    if (rc || plan.splits == 1 || defer) return rc;
+    return launch_splitk_reduce<TO>(workspace, bias, residual, ldr, out, ldo, M, N, plan.splits, act, stream);
   } else if (M <= 128) {
     return launch_stream<TO>(a, lda, w, bias, residual, ldr, out, ldo, workspace, M, N, K, act, defer, stream);
   } else {
@@ -1021,10 +1022,8 @@ static int linear_mfma_typed(const bf16_t* a, long lda, const bf16_t* w, const f
       rc = launch_tile<TO, 256, 192>(a, lda, w, bias, residual, ldr, out, ldo, workspace, M, N, K, act, plan.splits, defer, stream);
     else if (plan.shape == 2)
       rc = launch_tile<TO, 256, 128>(a, lda, w, bias, residual, ldr, out, ldo, workspace, M, N, K, act, plan.splits, defer, stream);
-    else if (plan.shape == 3)
-      rc = launch_tile<TO, 128, 128>(a, lda, w, bias, residual, ldr, out, ldo, workspace, M, N, K, act, plan.splits, defer, stream);
     else
-      rc = launch_tile<TO, 128, 64>(a, lda, w, bias, residual, ldr, out, ldo, workspace, M, N, K, act, plan.splits, defer, stream);
+      rc = launch_tile<TO, 128, 128>(a, lda, w, bias, residual, ldr, out, ldo, workspace, M, N, K, act, plan.splits, defer, stream);
     if (rc) return rc;
   }
   return lev_check_launch("linear_mfma");

@@ -436,27 +436,21 @@ class HipKernels:
     @classmethod
     def use_library(cls, M: int, N: int, K: int, act: int) -> bool:
         """Which products go to the vendor library: those with an epilogue it has, at the shapes where it was measured
-        ahead on MI355X (widths of GPT-2 7B and XL, with epilogues). From 256 rows: all but long sums into narrow outputs
-        (K >= 4 N) below 1,024 rows and, below 320 rows, weights of a few MB unless the output is wide (a 1600-wide layer at 264
-        rows, ours / library with its kernel timed: qkv 18.3 / 16.7, fc 24.8 / 18.8, proj 11.9 / 14.2, second MLP matrix 22.7 / 20.4 but
-        20.1 / 23.5 at 256 and 22.9 / 23.5 at 288). Up to 64 rows see ``_library_reads_weights_faster``. From 65 to 255 rows: wide outputs of large
-        weights (N >= 2 K, 32 MB and more: at 160 rows qkv and fc of a 4096-wide layer 49.7 / 37.2 and 55.7 / 41.6); ours keep N = K (22.1 /
-        24.6 at 128) and K = 4 N (43.5 / 81.1), and below 96 rows the largest weights (more than 256 MB). Up to 256 rows our kernel
-        of row blocks keeps short sums (K to 2,048) whose blocks of 64 x 64 make one round of the CUs (4800 x 1600 at 96 / 192 rows 9.6 / 12.7, 10.3 / 16.8)."""
+        ahead on MI355X (with epilogues). Up to 64 rows see ``_library_reads_weights_faster``. Above, ours keep outputs below 2^22 numbers, 32,768 columns at
+        most (figures beside the ring kernel's rule), and the library takes the rest: from 256 rows all but the longest sums (K >= 4 N) below 1,024 rows, and of 65 to
+        255 rows (heads of tens of thousands of outputs) those with N >= 2 K, but below 128 rows no weights of less than 32 MB and below 96 rows none of more than 256 MB."""
         if act not in cls.LIBRARY_ACTIVATIONS or M < cls.LIBRARY_MIN_ROWS:
             return False
         if M <= 64:
             return cls._library_reads_weights_faster(M, N, K)
-        if M <= 256 and K <= 2048 and -(-M // 64) * (-(-N // 512) * 8) <= 256:
+        if N <= 32768 and M * N < (1 << 22):
             return False
         if M < 256:
             if N < 2 * K:
                 return False
             if N * K < (1 << 24):
-                return M >= 128  # a 1600-wide layer with the tile kernel: fc 20.5 / 17.7 at 128 rows, 19.1 / 18.7 at 192
+                return M >= 128
             return not (M < 96 and N * K > (1 << 27))
-        if M < 320 and N * K < (1 << 24):
-            return N >= 2 * K
         return not (K >= 4 * N and M < 1024)
 
     @staticmethod

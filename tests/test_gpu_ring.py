@@ -1,0 +1,65 @@
+"""The bfloat16 product through a ring of k-tiles in LDS: every tile, sums that end inside a k-tile, outputs that end inside a tile, ranges of K, strides, every epilogue."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+# rows, outputs, inputs; together they reach all eight tiles, one range and several (asserted below)
+SHAPES = [(97, 2304, 768), (65, 4100, 40), (100, 2321, 8), (129, 2049, 72), (200, 3072, 824), (264, 4800, 1600), (264, 1600, 6400), (300, 1601, 6408), (65, 4096, 16384), (100, 1000, 4096),
+          (264, 6400, 1600), (333, 6400, 1592), (777, 4800, 1600), (600, 2048, 5376), (1000, 3072, 776), (264, 12288, 520), (300, 12289, 392), (2047, 2048, 512), (1299, 2052, 1024), (511, 8190, 72)]
+
+
+@pytest.fixture(scope="module")
+def K():
+    from levanter_amd.kernels import get_kernels
+
+    return get_kernels()
+
+
+def test_the_shapes_reach_every_tile(K):
+    gemm = K._unit("gemm_mfma")
+    plans = {gemm.lev_linear_mfma_ring(*s) for s in SHAPES}
+    assert -1 not in plans
+    assert {p // 16 for p in plans} == set(range(8)) and {p % 16 > 1 for p in plans} == {True, False}
+
+
+@pytest.mark.parametrize("M,N,Ki", SHAPES)
+def test_against_float64(K, M, N, Ki):
+    """|error| <= (roundings of one chain) 2^-24 (sum of the absolute terms), K at the most; bfloat16 results besides rounded once."""
+    g = torch.Generator(device=DEV).manual_seed(M * 7 + N + Ki)
+    w = torch.randn(N, Ki, device=DEV, generator=g).bfloat16()
+    bias = torch.randn(N, device=DEV, generator=g)
+    a = torch.randn(M, Ki + 8, device=DEV, generator=g).bfloat16()[:, :Ki]
+    res = torch.randn(M, N, device=DEV, generator=g)
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    out = torch.full((M, N + 3), float("nan"), device=DEV)
+    K.linear(a, w, bias, out[:, :N], residual=res)  # rows that are not 16 bytes apart
+    err = (out[:, :N].double() - want - bias.double() - res.double()).abs()
+    assert bool((err <= (Ki + 4) * 2.0 ** -24 * (size + bias.double().abs() + res.double().abs())).all())
+    assert bool(torch.isnan(out[:, N:]).all())
+    again = res.clone()
+    K.linear(a, w, bias, again, residual=again)
+    assert torch.equal(again, out[:, :N])
+    half = torch.full((M, N), float("nan"), device=DEV, dtype=torch.bfloat16)
+    K.linear(a, w, None, half)
+    assert bool(((half.double() - want).abs() <= want.abs() * 2.0 ** -8 + Ki * 2.0 ** -24 * size).all())
+    small = (w.float() * Ki ** -0.5).bfloat16()
+    want = a.double() @ small.double().T + bias.double()
+    for act, f in (("gelu_new", lambda u: torch.nn.functional.gelu(u, approximate="tanh")), ("gelu", torch.nn.functional.gelu), ("silu", torch.nn.functional.silu),
+                   ("relu_squared", lambda u: torch.relu(u) ** 2)):
+        K.linear(a, small, bias, half, activation=act)
+        assert float((half.double() - f(want)).abs().max() / f(want).abs().max()) < 2e-2, act
+
+
+@pytest.mark.parametrize("M,N,Ki", [(100, 2304, 104), (264, 1600, 6408), (300, 6400, 1600)])
+def test_infinities_and_nan_stay_in_their_row_and_column(K, M, N, Ki):
+    """Neither what lies beyond a row's end nor the rows read again in place of those beyond the matrix reach another output."""
+    a, w = torch.randn(M, Ki, device=DEV).bfloat16(), torch.randn(N, Ki, device=DEV).bfloat16()
+    a[M - 1, 0], a[3, Ki - 1], w[N - 1, 1], w[5, Ki - 2] = float("inf"), float("nan"), float("nan"), float("inf")
+    out = torch.empty(M, N, device=DEV)
+    K.linear(a, w, None, out)
+    bad = ~torch.isfinite(out)
+    want = torch.zeros_like(bad)
+    want[M - 1], want[3], want[:, N - 1], want[:, 5] = True, True, True, True
+    assert torch.equal(bad, want)
