@@ -16,6 +16,7 @@
 // workgroup (up to 40 % slower where neighbours then no longer wait for the same line, 2 - 9 % faster at K = 16384 alone), a ring twice as deep (8 % slower), a
 // CU for every workgroup where two fit (the same).
 #include "gemm_ring.h"
+#include "ring.h"
 #include <math.h>
 #include <type_traits>
 
@@ -27,21 +28,6 @@ __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) {
   union { u32x4 u; bf16x8 b; } c;
   c.u = v;
   return c.b;
-}
-
-// Which chunk of its line a row keeps at place 0 of LDS (at place p: p ^ that). LDS has 64 banks, so 16 lanes' chunks (two rows' worth of banks) are served at
-// once: 16 rows of `a` one behind the other, or the 16 rows 8 q + r (r < 4) of w that one operand takes, each have their own.
-__device__ __forceinline__ int ring_swap_a(int row) { return (row >> 1) & 7; }
-__device__ __forceinline__ int ring_swap_w(int row) { return ((row >> 1) & 1) | ((row >> 2) & 6); }
-
-// 16 bytes a lane from base + off straight into LDS, at lds + 16 * lane. In assembly because the compiler waits for all such loads before any read of LDS; no
-// register is written, and vmcnt is waited for below.
-__device__ __forceinline__ void lines_to_lds(uint32_t lds, uint32_t off, const void* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
 // A workgroup of WGM x WGN waves computes BM x BN outputs, a wave BM / WGM x BN / WGN, in 16 x 16 x 32 products with w as the first operand: a lane then holds four
@@ -72,14 +58,14 @@ gemm_ring_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, uin
 #pragma unroll
   for (int i = 0; i < LA; ++i) {
     const int r = (wave * LA + i) * 8 + lr;
-    off[i] = (uint32_t)min(m0 + r, M - 1) * lda * 2 + (uint32_t)((lc ^ ring_swap_a(r)) * 16);
+    off[i] = (uint32_t)min(m0 + r, M - 1) * lda * 2 + (uint32_t)((lc ^ ring_swap_rows(r)) * 16);
   }
 #pragma unroll
   for (int i = 0; i < LW; ++i) {
     const int r = (wave * LW + i) * 8 + lr;
-    off[LA + i] = (uint32_t)min(n0 + r, N - 1) * (uint32_t)K * 2 + (uint32_t)((lc ^ ring_swap_w(r)) * 16);
+    off[LA + i] = (uint32_t)min(n0 + r, N - 1) * (uint32_t)K * 2 + (uint32_t)((lc ^ ring_swap_columns(r)) * 16);
   }
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds_ring;
+  const uint32_t lds0 = lds_offset(lds_ring);
   const long first = tail ? (t0 == 0 ? 0 : (long)t0 * 64 - (64 - tail)) : (long)t0 * 64;
   const char *ab = reinterpret_cast<const char*>(a + first), *wb = reinterpret_cast<const char*>(w + first);
   auto load_one = [&](uint32_t at, int i) {
@@ -92,7 +78,7 @@ gemm_ring_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, uin
 #pragma unroll
     for (int i = 0; i < L; ++i) {
       const int r = ((i < LA ? wave * LA + i : wave * LW + i - LA)) * 8 + lr;
-      const int c = lc ^ (i < LA ? ring_swap_a(r) : ring_swap_w(r));
+      const int c = lc ^ (i < LA ? ring_swap_rows(r) : ring_swap_columns(r));
       const uint32_t o = off[i] - (uint32_t)((c - min(c, chunks - 1)) * 16);
       if (i < LA) lines_to_lds(lds0 + (wave * LA + i) * 1024, o, ab);
       else lines_to_lds(lds0 + BM * 128 + (wave * LW + i - LA) * 1024, o, wb);
@@ -107,20 +93,6 @@ gemm_ring_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, uin
     for (int i = 0; i < L; ++i) load_one(lds0 + ahead * TILE, i);
     ab += 128, wb += 128;
   }
-  auto wait_for = [&](int newer) {  // all but the loads of the `newer` youngest k-tiles have landed
-    static_assert((R - 1) * L <= 63, "vmcnt counts to 63");
-    switch (newer) {
-      case 7: wait_vmcnt<R >= 8 ? 7 * L : 0>(); break;
-      case 6: wait_vmcnt<R >= 7 ? 6 * L : 0>(); break;
-      case 5: wait_vmcnt<R >= 6 ? 5 * L : 0>(); break;
-      case 4: wait_vmcnt<R >= 5 ? 4 * L : 0>(); break;
-      case 3: wait_vmcnt<R >= 4 ? 3 * L : 0>(); break;
-      case 2: wait_vmcnt<2 * L>(); break;
-      case 1: wait_vmcnt<L>(); break;
-      default: wait_vmcnt<0>();
-    }
-  };
-
   // Sums in turn, joined at the end: with four no chain of roundings is longer than K / 128 products, about what the row blocks and waves that split K leave. Larger
   // tiles run 15 - 40 % slower with as many (registers: 128 x 128 at 1,300 rows of 2048 x 2048 21.8 us with four, 17.8 with fewer); the kernels they replace have one.
   constexpr int SUMS = TI * TJ <= 6 ? 4 : W == 8 ? 2 : 1;
@@ -134,8 +106,8 @@ gemm_ring_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, uin
   auto& acc = sums[0];
   // operand (row l % 16, k-group l / 16) of a k-step of 32; column tile j = 2 p + h takes the rows 32 p + 8 (l % 16 / 4) + 4 h + l % 4 of w
   const int fr = lane & 15, kg = lane >> 4, wr = 8 * (fr >> 2) + (fr & 3);
-  const int a_at = (wm * WM + fr) * 128 + ((kg ^ ring_swap_a(fr)) * 16);
-  const int w_at[2] = {(BM + wn * WN + wr) * 128 + ((kg ^ ring_swap_w(wr)) * 16), (BM + wn * WN + wr + 4) * 128 + ((kg ^ ring_swap_w(wr + 4)) * 16)};
+  const int a_at = (wm * WM + fr) * 128 + ((kg ^ ring_swap_rows(fr)) * 16);
+  const int w_at[2] = {(BM + wn * WN + wr) * 128 + ((kg ^ ring_swap_columns(wr)) * 16), (BM + wn * WN + wr + 4) * 128 + ((kg ^ ring_swap_columns(wr + 4)) * 16)};
   u32x4 af[2][2][TI], wf[2][2][TJ];
   constexpr int READS = 2 * (TI + TJ), PRODUCTS = 2 * TI * TJ;
   auto read_one = [&](auto set, const char* kt, int o) {  // the o-th of a k-tile's operands
@@ -152,14 +124,14 @@ gemm_ring_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, uin
   };
   typedef std::integral_constant<int, 0> Zero;
   typedef std::integral_constant<int, 1> One;
-  wait_for(most - 1);
+  ring_wait_for<R, L>(most - 1);
   if (tail && t0 == 0) {
     const int chunks = tail >> 3;
 #pragma unroll
     for (int i = 0; i < L; ++i) {
       const int at = i < LA ? (wave * LA + i) * 1024 : BM * 128 + (wave * LW + i - LA) * 1024;
       const int r = ((i < LA ? wave * LA + i : wave * LW + i - LA)) * 8 + lr;
-      if ((lc ^ (i < LA ? ring_swap_a(r) : ring_swap_w(r))) >= chunks) *reinterpret_cast<u32x4*>(lds_ring + at + lane * 16) = u32x4{0, 0, 0, 0};
+      if ((lc ^ (i < LA ? ring_swap_rows(r) : ring_swap_columns(r))) >= chunks) *reinterpret_cast<u32x4*>(lds_ring + at + lane * 16) = u32x4{0, 0, 0, 0};
     }
   }
   lds_barrier();
@@ -171,7 +143,7 @@ gemm_ring_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, uin
   int place = 0;
   auto step = [&](auto set, auto loads, int kt) {
     constexpr bool on = decltype(loads)::value;
-    if constexpr (on) wait_vmcnt<(R - 2) * L>(); else wait_for(min(R - 2, nk - 2 - kt));
+    if constexpr (on) ring_wait<(R - 2) * L>(); else ring_wait_for<R, L>(min(R - 2, nk - 2 - kt));
     lds_barrier();
     const uint32_t into = lds0 + place * TILE;
     place = place + 1 == R ? 0 : place + 1;

@@ -20,10 +20,9 @@
 //   combine   y[t] = sum_c weight[t][c] * out[pos_of[t * top + c]], c in order, float32; with `accumulate` added to what y holds.
 //   identity  router outputs n_real .. E-1 may stand for experts without weights whose result is their input: sort gives their pairs
 //             places but no tiles (the products never see them), and combine takes the token's own row of `identity_in` for them.
-#include "common.h"
+#include "moe.h"
 
 #define MOE_TM 16          // rows of a matrix-core row tile, and of a tile of the list in steps of few tokens
-#define MOE_BIG 128        // rows of a tile of the list in the others
 #define MOE_MAX_E 1024     // experts (at most 32 a lane)
 #define MOE_MAX_TOP 32
 
@@ -264,11 +263,6 @@ extern "C" int lev_moe_route_sort(const float* z, long z_stride, const float* co
 }
 
 // ---- the experts' products ------------------------------------------------------------------------
-__device__ __forceinline__ float moe_act(float gate, float up, int act, float limit, float up_shift) {
-  if (limit > 0.f) gate = fminf(gate, limit), up = fminf(fmaxf(up, -limit), limit);
-  return lev_activate(gate, act) * (up + up_shift);
-}
-
 // float32: a thread per (row of the tile, output); 16 x 16 a workgroup
 template <typename T, typename TO>
 __global__ void __launch_bounds__(256)
@@ -306,18 +300,6 @@ __device__ __forceinline__ moe_bf16x8 moe_as_bf16x8(moe_u32x4 v) {
   return c.b;
 }
 
-struct MoeLinearArgs {
-  const bf16_t* a;
-  long a_stride;
-  const bf16_t* w;
-  void* out;
-  long o_stride;
-  const int *tiles, *meta, *sorted;
-  int top, gather, K, N, F, act;
-  float limit, up_shift;
-  int n_cols, vec;
-  bool spread;  // tiles of 128 rows: their columns begin at places of their own along K
-};
 template <typename TO>
 __device__ __forceinline__ void moe_store4(TO* p, const float (&v)[4], int n, bool vec);
 template <>
@@ -415,7 +397,7 @@ moe_linear_few_kernel(const MoeLinearArgs p) {
   moe_store4<TO>(static_cast<TO*>(p.out) + (size_t)(first + col) * p.o_stride + o, v, F - o, p.vec);
 }
 
-// Tiles of 128 rows (prompts, large batches): a workgroup of four waves owns 128 rows and BN weight rows (with glu: BN / 2 outputs' gate
+// Tiles of 128 rows (prompts, large batches) of sums that are no multiple of 128 or below 512 (moe_ring.hip has the others): a workgroup of four waves owns 128 rows and BN weight rows (with glu: BN / 2 outputs' gate
 // rows and the same outputs' up rows), a wave 64 x BN / 2 of them in 32x32x16 products (the transposed product out^T = w a^T: a lane ends
 // with four neighbouring outputs of a row). K goes by in steps of 64, the step after next on its way in registers, two buffers in LDS,
 // one barrier a step that waits for LDS only; loads, LDS writes and fragment reads are issued one by one between the products. Rows
@@ -656,7 +638,7 @@ moe_linear_big_kernel(const MoeLinearArgs p) {
 }
 
 // a [rows][K]; w [E][N][K] with N = F outputs, or with glu N = 2F: gate rows then up rows; out [P][F]
-extern "C" int lev_moe_linear(const void* a, long a_stride, const void* w, void* out, long o_stride, const int* tiles, const int* meta,
+extern "C" int lev_moe_linear(const void* a, long a_rows, long a_stride, const void* w, void* out, long o_stride, const int* tiles, const int* meta,
                               const int* sorted, int max_tiles, int tile_rows, int E, int top, int gather, int K, int N, int glu, int act, float limit,
                               float up_shift, int dtype, int out_dtype, int use_mfma, hipStream_t stream) {
   LEV_REQUIRE(a && w && out && tiles && meta && sorted, "experts: a tensor is missing");
@@ -675,12 +657,14 @@ extern "C" int lev_moe_linear(const void* a, long a_stride, const void* w, void*
       const long blocks = (long)((max_tiles + 7) / 8) * 8 * n_cols;
       LEV_REQUIRE(blocks <= 0x7fffffffL, "experts: too many tiles (%ld)", blocks);
       const bool spread = blocks / 8 <= (max_tiles <= 2L * E + 1 ? 2 * MOE_BIG_SPREAD : MOE_BIG_SPREAD);  // by sizes alone, not by what the routing made of them
+      const MoeLinearArgs args{(const bf16_t*)a, a_stride, (const bf16_t*)w, out, o_stride, tiles, meta, sorted, top, gather, K, N, F, act, limit, up_shift, n_cols, vec, spread};
+      const int ring = lev_moe_ring(args, a_rows, out_dtype, glu, max_tiles, stream);
+      if (ring <= 0) return ring;
 #define MOE_BIG_CASE(TO, G)                                                                                                                       \
   do {                                                                                                                                            \
     hipError_t e = hipFuncSetAttribute((const void*)moe_linear_big_kernel<TO, G>, hipFuncAttributeMaxDynamicSharedMemorySize, MOE_BIG_LDS(MOE_BN)); \
     LEV_REQUIRE(e == hipSuccess, "experts: %d bytes of LDS a workgroup: %s", MOE_BIG_LDS(MOE_BN), hipGetErrorString(e));                           \
-    moe_linear_big_kernel<TO, G><<<(unsigned)blocks, 256, MOE_BIG_LDS(MOE_BN), stream>>>(                                                         \
-        MoeLinearArgs{(const bf16_t*)a, a_stride, (const bf16_t*)w, out, o_stride, tiles, meta, sorted, top, gather, K, N, F, act, limit, up_shift, n_cols, vec, spread}); \
+    moe_linear_big_kernel<TO, G><<<(unsigned)blocks, 256, MOE_BIG_LDS(MOE_BN), stream>>>(args);                                                   \
   } while (0)
       if (out_dtype == LEV_F32) {
         if (glu) MOE_BIG_CASE(float, true); else MOE_BIG_CASE(float, false);

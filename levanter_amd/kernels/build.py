@@ -277,7 +277,7 @@ _P, _I, _L, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_long, ctypes.c_float
 
 register_unit("core", ["errors.hip", "elementwise.hip", "layer_ops.hip", "gemm_simple.hip", "gemm_f32.hip", "attention_simple.hip", "attention_f32.hip", "attention_values.hip",
                        "attention_common.hip", "stream_ops.hip", "rotary.hip", "block_linear.hip", "recurrent_ops.hip", "group_norm.hip", "delta_rule.hip",
-                       "moe_ops.hip", "linear_attention.hip", "state_recurrence.hip", "state_chunks.hip", "sum_norm.hip"], signatures={
+                       "moe_ops.hip", "moe_ring.hip", "linear_attention.hip", "state_recurrence.hip", "state_chunks.hip", "sum_norm.hip"], signatures={
     "lev_embed": [_P] * 5 + [_I, _I, _I, _F, _P],
     "lev_pair_embed_add": [_P] * 6 + [_I, _I, _I, _L, _L, _I, _P],
     "lev_streams_step": [_P, _I, _I, _I, _P, _P, _P, _P, _P, _P, _F, _P, _P, _P, _I, _I, _P, _I, _P, _P],
@@ -293,7 +293,7 @@ register_unit("core", ["errors.hip", "elementwise.hip", "layer_ops.hip", "gemm_s
     "lev_moe_route_sort": [_P, _L, _P] + [_I] * 9 + [_P, _P, _I, _I] + [_P] * 5,
     "lev_moe_max_tiles": [_I, _I, _I],
     "lev_moe_sort": [_P, _I, _I, _I, _I, _P, _P, _P, _P, _P],
-    "lev_moe_linear": [_P, _L, _P, _P, _L, _P, _P, _P] + [_I] * 9 + [_F, _F, _I, _I, _I, _P],
+    "lev_moe_linear": [_P, _L, _L, _P, _P, _L, _P, _P, _P] + [_I] * 9 + [_F, _F, _I, _I, _I, _P],
     "lev_moe_combine": [_P, _P, _P, _P, _I, _I, _I, _I, _P, _I, _P, _L, _I, _P],
     "lev_block_linear": [_P, _L, _P, _P, _P, _L, _P, _L] + [_I] * 7 + [_P],
     "lev_block_linear_mfma": [_P, _L, _P, _P, _P, _L, _P, _L] + [_I] * 6 + [_P],

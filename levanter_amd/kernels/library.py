@@ -1268,7 +1268,7 @@ class HipKernels:
         F_ = N // 2 if glu else N
         _req(out.dim() == 2 and out.shape[1] == F_ and out.dtype in _DT and (a.dtype == torch.bfloat16 or out.dtype == torch.float32), "experts: bad output")
         max_tiles = tiles.numel() // 3
-        self._check(self.lib.lev_moe_linear(_ptr(a), _rows(a, "experts: a"), _ptr(w), _ptr(out), _rows(out, "experts: out"), _ptr(tiles), _ptr(meta),
+        self._check(self.lib.lev_moe_linear(_ptr(a), a.shape[0], _rows(a, "experts: a"), _ptr(w), _ptr(out), _rows(out, "experts: out"), _ptr(tiles), _ptr(meta),
                                             _ptr(sorted_pairs), max_tiles, int(tile_rows), E, int(top), int(gather), K, N, int(glu), ACTIVATIONS[activation], float(limit), float(up_shift), _DT[a.dtype],
                                             _DT[out.dtype], int(self.use_mfma), self._s()))
 
