@@ -582,7 +582,7 @@ __device__ __forceinline__ void decode_wave(int idx, int kvh, int z, const bf16_
                                             const int* __restrict__ decode_tokens, const bf16_t* __restrict__ k_new,
                                             const bf16_t* __restrict__ v_new, long kv_stride, const int* __restrict__ dest,
                                             float* __restrict__ ws_m, float* __restrict__ ws_l, float* __restrict__ ws_o, int H,
-                                            int KVH, int ps_shift, int splits, float scale, int window, int wg_merge, float softcap,
+                                            int KVH, int ps_shift, int splits, float scale, int window, float* merge, float softcap,
                                             const float* __restrict__ score_bias, int bias_len) {
   const int PS = 1 << ps_shift, ps_mask = PS - 1;
   const float scale_log2 = scale * 1.4426950408889634f;
@@ -765,10 +765,9 @@ __device__ __forceinline__ void decode_wave(int idx, int kvh, int z, const bf16_
     }
     return;
   }
-  if (wg_merge) {
+  if (merge) {
     // partial results of this wave into LDS [split][query head of the group]: m, l, o[HD]
-    extern __shared__ float merge_s[];
-    float* ms = merge_s;
+    float* ms = merge;
     float* ls = ms + splits * G;
     float* os = ls + splits * G;
     if (fr < G) {
@@ -782,7 +781,7 @@ __device__ __forceinline__ void decode_wave(int idx, int kvh, int z, const bf16_
     }
     __syncthreads();
     bf16_t* orow = out + (size_t)t * o_stride + (size_t)kvh * G * HD;
-    for (int e = threadIdx.x; e < G * HD; e += blockDim.x) {
+    for (int e = z * 64 + lane; e < G * HD; e += splits * 64) {  // by the waves of this token and kv head
       const int hq = e / HD, d = e - hq * HD;
       float mx = -INFINITY;
       for (int zz = 0; zz < splits; ++zz) mx = fmaxf(mx, ms[zz * G + hq]);
@@ -818,22 +817,25 @@ LEV_NAME(attn_decode_hd)(const bf16_t* __restrict__ q, long q_stride, bf16_t* __
                          float* __restrict__ ws_m, float* __restrict__ ws_l, float* __restrict__ ws_o,
                          int H, int KVH, int ps_shift, int splits, float scale, int window, int wg_merge, float softcap,
                          const float* __restrict__ score_bias, int bias_len) {
+  extern __shared__ float merge_s[];
   decode_wave(blockIdx.x, blockIdx.y, wg_merge ? (int)(threadIdx.x >> 6) : (int)blockIdx.z, q, q_stride, out, o_stride, k_pages, v_pages,
               positions, token_seq, block_tables, bt_stride, decode_tokens, k_new, v_new, kv_stride, dest, ws_m, ws_l, ws_o, H, KVH,
-              ps_shift, splits, scale, window, wg_merge, softcap, score_bias, bias_len);
+              ps_shift, splits, scale, window, wg_merge ? merge_s : nullptr, softcap, score_bias, bias_len);
 }
 
-// A step of prompt portions beside single tokens whose key ranges are not split: both kinds of work in one launch, so that
+// A step of prompt portions beside single tokens: both kinds of work in one launch, so that
 // the single tokens' waves (bound by memory) fill the CUs that the portions' few workgroups (bound by latency) leave idle,
 // and the step has one kernel boundary fewer a layer. Workgroups below n_pf_wgs are the prefill kernel's, with its
-// numbering; each of the others is DECODE_WG_WAVES waves with a (single token, kv head) each, whose new keys and values
-// the KV-write kernel has written before.
+// numbering; each of the others is DECODE_WG_WAVES waves with the key ranges of as many (single token, kv head) as they hold, whose new
+// keys and values the KV-write kernel has written before; the ranges are merged as in the kernel of single tokens (same bits), in the LDS that the
+// portions' workgroups have their keys in. Split ranges used to take the two kernels one behind the other: GPT-2 XL, 256 tokens of portions beside 8 to 24
+// single tokens of 100 to 300 keys, a session of 24 requests 124.9 -> 117.8 ms (9 + 12 us a layer before).
 __global__ void __launch_bounds__(PF_THREADS)
 LEV_NAME(attn_mixed_hd)(const bf16_t* __restrict__ q, long q_stride, bf16_t* __restrict__ out, long o_stride,
                         bf16_t* __restrict__ k_pages, bf16_t* __restrict__ v_pages, const int* __restrict__ positions,
                         const int* __restrict__ token_seq, const int* __restrict__ block_tables, int bt_stride,
                         const int* __restrict__ tiles, int n_tiles, int pair, int n_pf_wgs, const int* __restrict__ decode_tokens,
-                        int n_decode, int H, int KVH, int ps_shift, float scale, int window, float softcap,
+                        int n_decode, int H, int KVH, int ps_shift, int splits, float scale, int window, float softcap,
                         const float* __restrict__ score_bias, int bias_len) {
   static_assert(PF_THREADS == 64 * DECODE_WG_WAVES, "one workgroup size for both kinds of work");
   __shared__ __attribute__((aligned(16))) bf16_t Ks[2][4][NCHUNK][16][8];
@@ -849,10 +851,15 @@ LEV_NAME(attn_mixed_hd)(const bf16_t* __restrict__ q, long q_stride, bf16_t* __r
                    tiles[2 * second + 1], h, H, KVH, ps_shift, scale, window, softcap, score_bias, bias_len, Ks, Vs);
     return;
   }
-  const int item = ((int)blockIdx.x - n_pf_wgs) * DECODE_WG_WAVES + (int)(threadIdx.x >> 6);
-  if (item >= n_decode * KVH) return;
-  decode_wave(item / KVH, item % KVH, 0, q, q_stride, out, o_stride, k_pages, v_pages, positions, token_seq, block_tables, bt_stride,
-              decode_tokens, nullptr, nullptr, 0, nullptr, nullptr, nullptr, nullptr, H, KVH, ps_shift, 1, scale, window, 0, softcap,
+  const int wave = threadIdx.x >> 6, held = DECODE_WG_WAVES / splits, mine = wave / splits;
+  const int item = ((int)blockIdx.x - n_pf_wgs) * held + mine;
+  if (mine >= held || item >= n_decode * KVH) {
+    if (splits > 1) __syncthreads();  // the others' merge
+    return;
+  }
+  float* merge = splits > 1 ? reinterpret_cast<float*>(&Ks[0][0][0][0][0]) + (size_t)mine * splits * (H / KVH) * (HD + 2) : nullptr;
+  decode_wave(item / KVH, item % KVH, wave % splits, q, q_stride, out, o_stride, k_pages, v_pages, positions, token_seq, block_tables, bt_stride,
+              decode_tokens, nullptr, nullptr, 0, nullptr, nullptr, nullptr, nullptr, H, KVH, ps_shift, splits, scale, window, merge, softcap,
               score_bias, bias_len);
 }
 
@@ -899,14 +906,17 @@ extern "C" int LEV_NAME(lev_attention_mfma_hd)(const void* q, long q_stride, voi
   int ps_shift = 0;
   while ((1 << ps_shift) < PS) ++ps_shift;
   if ((1 << ps_shift) != PS) return lev_fail("attention (matrix cores): page_size=%d must be a power of two", PS);
-  if (n_prefill_tiles > 0 && n_decode > 0 && splits == 1 && !k_new) {
+  // ranges that a workgroup merges, with room for them in the portions' keys
+  const size_t range_bytes = (size_t)(H / KVH) * (HD + 2) * sizeof(float);
+  const bool merged = splits > 1 && splits <= DECODE_WG_WAVES && splits * range_bytes <= 48 * 1024;
+  if (n_prefill_tiles > 0 && n_decode > 0 && !k_new && (splits == 1 || (merged && DECODE_WG_WAVES * range_bytes <= 2 * 4 * NCHUNK * 16 * 8 * sizeof(bf16_t)))) {
     const int pair = (long)n_prefill_tiles * H >= 512;
     const int n_pf_wgs = (pair ? (n_prefill_tiles + 1) / 2 : n_prefill_tiles) * H;
-    const long items = (long)n_decode * KVH;
-    dim3 grid((unsigned)(n_pf_wgs + (items + DECODE_WG_WAVES - 1) / DECODE_WG_WAVES));
+    const long items = (long)n_decode * KVH, held = DECODE_WG_WAVES / splits;
+    dim3 grid((unsigned)(n_pf_wgs + (items + held - 1) / held));
     LEV_NAME(attn_mixed_hd)<<<grid, PF_THREADS, 0, stream>>>(
         (const bf16_t*)q, q_stride, (bf16_t*)out, o_stride, (bf16_t*)k_pages, (bf16_t*)v_pages, positions, token_seq, block_tables,
-        bt_stride, prefill_tiles, n_prefill_tiles, pair, n_pf_wgs, decode_tokens, n_decode, H, KVH, ps_shift, scale, window, softcap,
+        bt_stride, prefill_tiles, n_prefill_tiles, pair, n_pf_wgs, decode_tokens, n_decode, H, KVH, ps_shift, splits, scale, window, softcap,
         score_bias, bias_len);
     return lev_check_launch("attention of a mixed step");
   }
@@ -926,9 +936,8 @@ extern "C" int LEV_NAME(lev_attention_mfma_hd)(const void* q, long q_stride, voi
     float* ws_m = (float*)workspace;
     float* ws_l = ws_m + rows;
     float* ws_o = ws_l + rows;
-    const int G = H / KVH;
-    const size_t merge_bytes = (size_t)splits * G * (HD + 2) * sizeof(float);
-    const int wg_merge = splits > 1 && splits <= DECODE_WG_WAVES && merge_bytes <= 48 * 1024;
+    const size_t merge_bytes = splits * range_bytes;
+    const int wg_merge = merged;
     dim3 grid(n_decode, KVH, wg_merge ? 1 : splits);
     LEV_NAME(attn_decode_hd)<<<grid, wg_merge ? 64 * splits : 64, wg_merge ? merge_bytes : 0, stream>>>(
         (const bf16_t*)q, q_stride, (bf16_t*)out, o_stride, (bf16_t*)k_pages, (bf16_t*)v_pages, positions, token_seq, block_tables,
