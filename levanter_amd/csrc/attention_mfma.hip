@@ -809,14 +809,12 @@ __device__ __forceinline__ void decode_wave(int idx, int kvh, int z, const bf16_
 }
 
 __global__ void __launch_bounds__(64 * DECODE_WG_WAVES)
-LEV_NAME(attn_decode_hd)(const bf16_t* __restrict__ q, long q_stride, bf16_t* __restrict__ out, long o_stride,
-                         bf16_t* __restrict__ k_pages, bf16_t* __restrict__ v_pages, const int* __restrict__ positions,
-                         const int* __restrict__ token_seq, const int* __restrict__ block_tables, int bt_stride,
-                         const int* __restrict__ decode_tokens, const bf16_t* __restrict__ k_new,
-                         const bf16_t* __restrict__ v_new, long kv_stride, const int* __restrict__ dest,
-                         float* __restrict__ ws_m, float* __restrict__ ws_l, float* __restrict__ ws_o,
-                         int H, int KVH, int ps_shift, int splits, float scale, int window, int wg_merge, float softcap,
-                         const float* __restrict__ score_bias, int bias_len) {
+LEV_NAME(attn_decode_hd)(const int* __restrict__ decode_tokens, const int* __restrict__ positions, const int* __restrict__ token_seq,
+                         const int* __restrict__ block_tables, int bt_stride, int H, int KVH, int splits, int wg_merge, int ps_shift,  // in registers when the waves start
+                         const bf16_t* __restrict__ q, long q_stride, bf16_t* __restrict__ k_pages, bf16_t* __restrict__ v_pages,
+                         const bf16_t* __restrict__ k_new, const bf16_t* __restrict__ v_new, long kv_stride, const int* __restrict__ dest,
+                         bf16_t* __restrict__ out, long o_stride, float* __restrict__ ws_m, float* __restrict__ ws_l, float* __restrict__ ws_o,
+                         float scale, int window, float softcap, const float* __restrict__ score_bias, int bias_len) {
   extern __shared__ float merge_s[];
   decode_wave(blockIdx.x, blockIdx.y, wg_merge ? (int)(threadIdx.x >> 6) : (int)blockIdx.z, q, q_stride, out, o_stride, k_pages, v_pages,
               positions, token_seq, block_tables, bt_stride, decode_tokens, k_new, v_new, kv_stride, dest, ws_m, ws_l, ws_o, H, KVH,
@@ -940,9 +938,9 @@ extern "C" int LEV_NAME(lev_attention_mfma_hd)(const void* q, long q_stride, voi
     const int wg_merge = merged;
     dim3 grid(n_decode, KVH, wg_merge ? 1 : splits);
     LEV_NAME(attn_decode_hd)<<<grid, wg_merge ? 64 * splits : 64, wg_merge ? merge_bytes : 0, stream>>>(
-        (const bf16_t*)q, q_stride, (bf16_t*)out, o_stride, (bf16_t*)k_pages, (bf16_t*)v_pages, positions, token_seq, block_tables,
-        bt_stride, decode_tokens, (const bf16_t*)k_new, (const bf16_t*)v_new, kv_stride, dest, ws_m, ws_l, ws_o, H, KVH, ps_shift,
-        splits, scale, window, wg_merge, softcap, score_bias, bias_len);
+        decode_tokens, positions, token_seq, block_tables, bt_stride, H, KVH, splits, wg_merge, ps_shift, (const bf16_t*)q, q_stride, (bf16_t*)k_pages,
+        (bf16_t*)v_pages, (const bf16_t*)k_new, (const bf16_t*)v_new, kv_stride, dest, (bf16_t*)out, o_stride, ws_m, ws_l, ws_o, scale, window, softcap,
+        score_bias, bias_len);
     if (int rc = lev_check_launch("attention decode")) return rc;
     if (splits > 1 && !wg_merge) {
       dim3 cgrid(n_decode, H);

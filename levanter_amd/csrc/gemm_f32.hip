@@ -37,8 +37,9 @@ __device__ __forceinline__ void gemm_f32_store(gf_f32x4 v, const float* bias, co
 // and outputs the few-row kernel below goes before it, 3.9 and 5.9).
 template <int RT, int NT, int W>
 __global__ void __launch_bounds__(64 * W)
-gemm_f32_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias,
-                const float* residual, long ldr, float* out, long ldo, int M, int N, int K, int act, int n_rows, int n_cols, int vec) {
+gemm_f32_kernel(const float* __restrict__ w, const float* __restrict__ a, uint32_t lda4, int K, int N, int M, int n_rows, int n_cols, int vec, int act,
+                const float* __restrict__ bias, const float* residual, float* out, long ldr, long ldo) {  // up to bias in registers when the waves start
+  const size_t lda = (size_t)lda4 * 4;
   extern __shared__ __attribute__((aligned(16))) float gf_part[];  // [W][RT * NT][64][4]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, g = lane >> 4;
   // the chiplets (workgroups are dealt to the eight in turn) take neighbouring columns of tiles each, rows fastest: a weight is read by
@@ -287,8 +288,9 @@ gemm_f32_tile_kernel(const float* __restrict__ a, long lda, const float* __restr
 #define GF_FEW_OUT 4
 template <int MR>
 __global__ void __launch_bounds__(512)
-gemm_f32_few_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias, const float* residual, long ldr,
-                    float* out, long ldo, int M, int N, int K, int act) {
+gemm_f32_few_kernel(const float* __restrict__ w, const float* __restrict__ a, uint32_t lda4, int K, int N, int M, const float* __restrict__ bias,
+                    const float* residual, float* out, long ldr, long ldo, int act) {  // in registers when the waves start: all but the last three
+  const size_t lda = (size_t)lda4 * 4;
   __shared__ float part[8][GF_FEW_OUT * MR];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, o0 = blockIdx.x * GF_FEW_OUT;
   const float *ar[MR], *wr[GF_FEW_OUT];
@@ -412,7 +414,7 @@ int lev_gemm_f32(const float* a, long lda, const float* w, const float* bias, co
   const int choice = lev_linear_f32_choice(M, N, K), few = -choice, line = choice - GEMM_F32_N_TILES;
   if (few > 0) {
 #define GEMM_F32_FEW(MR) \
-  if (few == MR) gemm_f32_few_kernel<MR><<<(N + GF_FEW_OUT - 1) / GF_FEW_OUT, 512, 0, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act)
+  if (few == MR) gemm_f32_few_kernel<MR><<<(N + GF_FEW_OUT - 1) / GF_FEW_OUT, 512, 0, stream>>>(w, a, (uint32_t)(lda / 4), K, N, M, bias, residual, out, ldr, ldo, act)
     GEMM_F32_FEW(1);
     else GEMM_F32_FEW(2);
     else GEMM_F32_FEW(4);
@@ -426,7 +428,7 @@ int lev_gemm_f32(const float* a, long lda, const float* w, const float* bias, co
   LEV_REQUIRE(blocks <= 0x7fffffffL, "linear: too many tiles (%ld)", blocks);
 #define GEMM_F32_CASE(RT, NT, W)                                                                                                                    \
   if (line < 0 && rt == RT && nt == NT)                                                                                                             \
-    gemm_f32_kernel<RT, NT, W><<<(unsigned)blocks, 64 * W, W * RT * NT * 1024, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act, n_rows, n_cols, vec)
+    gemm_f32_kernel<RT, NT, W><<<(unsigned)blocks, 64 * W, W * RT * NT * 1024, stream>>>(w, a, (uint32_t)(lda / 4), K, N, M, n_rows, n_cols, vec, act, bias, residual, out, ldr, ldo)
 #define GEMM_F32_LINE_CASE(RT, NT, SETS)                                                                                                            \
   if (rt == 2 * RT && nt == 2 * NT)                                                                                                                 \
     gemm_f32_tile_kernel<RT, NT, SETS><<<(unsigned)blocks, 256, 0, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act, n_rows, n_cols, vec)

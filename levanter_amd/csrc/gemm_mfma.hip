@@ -355,8 +355,9 @@ template <typename TO, int WAVES, int U, int MT, int NT, bool HALF, bool BLOCKS>
 // at most 128 registers a lane for 2 x 2 tiles (130 cost 7 % at 2048 x 2048 and 96 rows); with four waves at most 256, so that the sums stay in
 // registers that every instruction reads (where 512 are allowed the compiler moves them to and fro: 16384 x 4096 at 64 rows 34.2 us)
 __global__ void __launch_bounds__(WAVES * 64, U == 2 && NT * MT == 4 ? 4 : WAVES == 4 ? 2 : 1)
-gemm_skinny_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restrict__ w, const float* __restrict__ bias,
-                   const float* residual, long ldr, TO* out, long ldo, int M, int N, int K, int act) {
+gemm_skinny_kernel(const bf16_t* __restrict__ w, const bf16_t* __restrict__ a, uint32_t lda8, int K, int N, int M, const float* __restrict__ bias,
+                   const float* residual, TO* out, long ldr, long ldo, int act) {  // in registers when the waves start: all but the last three
+  const size_t lda = (size_t)lda8 * 8;
   static_assert(NT * MT <= WAVES * 4 && (!HALF || NT == 1), "a wave finishes a few tiles; half a unit stands alone");
   constexpr int AI = 2 * MT, WI = HALF ? 1 : 2;  // instructions per pair of k-steps and unit: 8 rows each
   constexpr int COLS = HALF ? 8 : 16;
@@ -568,10 +569,10 @@ static void launch_skinny(const bf16_t* a, long lda, const bf16_t* w, const floa
   const int cols = sh.cols(), columns = (N + cols - 1) / cols;
 #define LEV_SKINNY(W_, U_, MT_, NT_, H_)                                                                                          \
   if (sh.waves == W_ && sh.in_flight == U_ && sh.row_tiles == MT_ && sh.units == NT_ && sh.half == H_)                             \
-    gemm_skinny_kernel<TO, W_, U_, MT_, NT_, H_, false><<<columns, W_ * 64, 0, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act)
+    gemm_skinny_kernel<TO, W_, U_, MT_, NT_, H_, false><<<columns, W_ * 64, 0, stream>>>(w, a, (uint32_t)(lda / 8), K, N, M, bias, residual, out, ldr, ldo, act)
   if (M > 64) {  // row blocks are a variant of their own: what finds them costs the small steps' kernels 0.2 - 0.4 us
     const dim3 grid((columns + 7) / 8 * 8, (M + 31) / 32);
-    gemm_skinny_kernel<TO, 8, 2, 2, 2, false, true><<<grid, 8 * 64, 0, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act);
+    gemm_skinny_kernel<TO, 8, 2, 2, 2, false, true><<<grid, 8 * 64, 0, stream>>>(w, a, (uint32_t)(lda / 8), K, N, M, bias, residual, out, ldr, ldo, act);
     return;
   }
   LEV_SKINNY(16, 2, 1, 1, true);
@@ -610,9 +611,9 @@ static void launch_skinny(const bf16_t* a, long lda, const bf16_t* w, const floa
 
 template <typename TO, int MT, int NW>
 __global__ void __launch_bounds__(NW * 64, NW == 4 ? 2 : 1)
-gemm_stream_kernel(const bf16_t* __restrict__ a, long lda, const bf16_t* __restrict__ w, const float* __restrict__ bias,
-                   const float* residual, long ldr, TO* out, long ldo, float* __restrict__ partial, int M, int N, int K, int act,
-                   int S) {
+gemm_stream_kernel(const bf16_t* __restrict__ w, const bf16_t* __restrict__ a, uint32_t lda8, int K, int N, int M, int S, float* __restrict__ partial,
+                   const float* __restrict__ bias, const float* residual, TO* out, long ldr, long ldo, int act) {
+  const size_t lda = (size_t)lda8 * 8;
   constexpr int BM = MT * 16;
   constexpr int NT = NW * 64;
   constexpr int A_CHUNKS = BM * (SK_CHUNK / 8);       // 16-byte chunks of the a tile
@@ -977,7 +978,7 @@ static int launch_stream(const bf16_t* a, long lda, const bf16_t* w, const float
   if (S > 1 && !workspace) return lev_fail("linear: M=%d N=%d K=%d needs a workspace of lev_linear_mfma_workspace bytes", M, N, K);
   dim3 grid((N + plan.waves * 16 - 1) / (plan.waves * 16), S);
 #define LEV_STREAM(MT_, NW_) \
-  gemm_stream_kernel<TO, MT_, NW_><<<grid, NW_ * 64, 0, stream>>>(a, lda, w, bias, residual, ldr, out, ldo, workspace, M, N, K, act, S)
+  gemm_stream_kernel<TO, MT_, NW_><<<grid, NW_ * 64, 0, stream>>>(w, a, (uint32_t)(lda / 8), K, N, M, S, workspace, bias, residual, out, ldr, ldo, act)
 #define LEV_STREAM_MT(MT_)                 \
   switch (plan.waves) {                    \
     case 4: LEV_STREAM(MT_, 4); break;     \

@@ -104,8 +104,9 @@ def lib_name(unit: str) -> str:
 # -packed-fp32-ops off: no packed 32-bit float instructions (v_pk_*_f32) are generated; some forms have given wrong results on MI355X
 # kernarg-preload: the first 14 registers' worth of a kernel's arguments (as many as are left of the 16) is there when its waves start, instead of being
 # read from memory first (a step of single tokens is dozens of kernels of 3 to 8 us, one behind the other: GPT-2 small, one request 0.327 -> 0.318 ms a step, XL, 6
-# requests 2.05 -> 2.00, small in 32 bits 0.79 -> 0.77). Kernels that take a struct (the experts' products and routing, the norms of sums, the 32-bit attention)
-# keep reading all of it, and the others what lies behind: the sizes of the products, the work lists of the decode attentions.
+# requests 2.05 -> 2.00, small in 32 bits 0.79 -> 0.77). The products of few rows and the attention of single tokens therefore name what their first loads need
+# first: pointers and sizes, the work lists (sessions: GPT-2 small, one request 7.71 -> 7.54 ms, XL, a few 63.6 -> 62.9, small in 32 bits 10.97 -> 10.78). Kernels that take a
+# struct (the experts' products and routing, the norms of sums, the 32-bit attention) keep reading all of it, and the others what lies behind.
 HIPCC_FLAGS = [
     f"--offload-arch={ARCH}",
     "-O3",
