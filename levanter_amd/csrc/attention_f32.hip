@@ -9,7 +9,9 @@
 // What bounds it: prompts, the matrix pipe half of the time and the round trips between its batches the rest (777 rows of 16 heads of 64:
 // 35 us, 1.2 GFLOP of visible products); single tokens, the chain of one block's loads, products and merge (4 tokens of 12 heads over
 // 200 keys: 9.6 us). The plain kernel gives a wave one query row, reads keys 4 bytes at a time and walks the values key by key:
-// 1,187 us and 70 us.
+// 1,187 us and 70 us. A step of single tokens alone brings its new keys and values along: the wave whose keys they are takes them from the projection's output, and
+// the wave behind it, which has none in a short context, writes them to their page; the kernel that wrote them first took 4 us a layer (GPT-2 small, 4 requests of
+// 100 to 200 tokens, with the arguments of the first loads in registers besides: 10.78 -> 9.99 ms a session, same bits).
 #include "common.h"
 #include <math.h>
 
@@ -20,41 +22,44 @@ struct AttentionF32Args {
   long q_stride;
   float* out;
   long o_stride;
-  const float *k_pages, *v_pages;
-  const int *positions, *token_seq, *block_tables;
-  int bt_stride, H, KVH, PS, window, bias_len;
+  float *k_pages, *v_pages;
+  int window, bias_len;
   float scale, softcap;
   const float* score_bias;
-  const int* work;  // runs: (first token, rows) per tile of the list; single tokens: their indexes
-  int tile_rows, columns;  // rows of a tile of the list (runs); columns in use (single tokens: query heads of a key/value head, at most 16)
+  const float *k_new, *v_new;  // single tokens: the step's new keys and values (rows kv_stride apart), not in their pages yet; or null
+  long kv_stride;
+  const int* dest;  // where they go, by token: page * PS + offset
 };
 
 template <int HD, int KB, int W, bool RUNS>
 __global__ void __launch_bounds__(64 * W)
-attention_f32_kernel(const AttentionF32Args p) {
+attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows) per tile of the list; single tokens: their indexes
+                     const int* __restrict__ positions, const int* __restrict__ token_seq, const int* __restrict__ block_tables, int bt_stride, int H, int KVH, int PS,
+                     int tile_rows, int columns,  // rows of a tile of the list (runs); columns in use (single tokens: query heads of a key/value head, at most 16)
+                     const AttentionF32Args p) {  // all before p is in registers when the waves start
   extern __shared__ __attribute__((aligned(16))) float af_lds[];  // [W][HD/16][4][columns] of four outputs, then maxima and sums [2][W][16] and a tile's weights [W][16][16]
   constexpr int DT = HD / 16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, g = lane >> 4;
-  const int group = p.H / p.KVH, nc = RUNS ? 16 : p.columns;
+  const int group = H / KVH, nc = RUNS ? 16 : columns;
   int token, head;
   bool mine;  // this lane's column is one
   if (RUNS) {
-    const int subs = (p.tile_rows + 15) / 16;
-    head = blockIdx.x % p.H;
-    const int sub = blockIdx.x / p.H % subs, tile = blockIdx.x / p.H / subs;
-    const int first = p.work[2 * tile], rows = p.work[2 * tile + 1] - 16 * sub;
+    const int subs = (tile_rows + 15) / 16;
+    head = blockIdx.x % H;
+    const int sub = blockIdx.x / H % subs, tile = blockIdx.x / H / subs;
+    const int first = work[2 * tile], rows = work[2 * tile + 1] - 16 * sub;
     if (rows <= 0) return;  // the whole workgroup
     mine = col < rows;
     token = first + 16 * sub + min(col, rows - 1);
   } else {
-    const int sets = (group + 15) / 16, kvh = blockIdx.x / sets % p.KVH, set = blockIdx.x % sets;
-    token = p.work[blockIdx.x / sets / p.KVH];
+    const int sets = (group + 15) / 16, kvh = blockIdx.x / sets % KVH, set = blockIdx.x % sets;
+    token = work[blockIdx.x / sets / KVH];
     const int n = min(16, group - 16 * set);
     mine = col < n;
     head = kvh * group + 16 * set + min(col, n - 1);
   }
   const int kvh = head / group;
-  const int pos = p.positions[token];
+  const int pos = positions[token];
   const int first = p.window > 0 ? max(0, pos - p.window + 1) : 0;
   int last = pos, lo = first;  // over the columns
 #pragma unroll
@@ -62,8 +67,8 @@ attention_f32_kernel(const AttentionF32Args p) {
     last = max(last, __shfl_xor(last, o, 64));
     lo = min(lo, __shfl_xor(lo, o, 64));
   }
-  const int* bt = p.block_tables + (size_t)p.token_seq[token] * p.bt_stride;
-  const size_t head_elems = (size_t)HD * p.PS;
+  const int* bt = block_tables + (size_t)token_seq[token] * bt_stride;
+  const size_t head_elems = (size_t)HD * PS;
   const float* qr = p.q + (size_t)token * p.q_stride + (size_t)head * HD;
   af_f32x4 q[DT], o_acc[DT];
 #pragma unroll
@@ -75,28 +80,49 @@ attention_f32_kernel(const AttentionF32Args p) {
   float* weights = ml + 2 * W * 16 + wave * 256;
   float m = -INFINITY, l = 0.f;
   const int t_last = last / 16;
+  const bool fused = !RUNS && p.k_new != nullptr;
+  const float* kn = fused ? p.k_new + (size_t)token * p.kv_stride + (size_t)kvh * HD : qr;  // not fused: read, not used
+  const float* vn = fused ? p.v_new + (size_t)token * p.kv_stride + (size_t)kvh * HD : qr;
+  float nv[DT];  // the token's new value in this lane's dimensions
+  int to = -1;
+  if (!RUNS) {
+#pragma unroll
+    for (int d = 0; d < DT; ++d) nv[d] = vn[16 * d + col];
+    to = *(fused ? p.dest + token : work);
+    to = fused ? to : -1;
+  }
   for (int t0 = lo / 16 + wave * KB; t0 <= t_last; t0 += W * KB) {
     int page[KB], off[KB];
 #pragma unroll
     for (int t = 0; t < KB; ++t) {
       const int key = min(t0 + t, t_last) * 16;  // tiles behind the last are read again and masked
-      page[t] = bt[key / p.PS];
-      off[t] = key % p.PS;
+      page[t] = bt[key / PS];
+      off[t] = key % PS;
     }
     af_f32x4 s[KB], k[KB][DT], v[KB][DT];  // all of the block's loads are on their way before the first product
 #pragma unroll
     for (int t = 0; t < KB; ++t) {
-      const float* kb = p.k_pages + ((size_t)max(page[t], 0) * p.KVH + kvh) * head_elems + (size_t)(off[t] + col) * 8 + (g & 1) * 4;
+      const bool is_new = fused && (t0 + t) * 16 + col == pos;
+      const float* kb = is_new ? kn + 4 * g : p.k_pages + ((size_t)max(page[t], 0) * KVH + kvh) * head_elems + (size_t)(off[t] + col) * 8 + (g & 1) * 4 + (size_t)(g >> 1) * PS * 8;
+      const size_t next = is_new ? 16 : (size_t)PS * 16;
 #pragma unroll
-      for (int d = 0; d < DT; ++d) k[t][d] = *reinterpret_cast<const af_f32x4*>(kb + (size_t)(2 * d + (g >> 1)) * p.PS * 8);
+      for (int d = 0; d < DT; ++d) k[t][d] = *reinterpret_cast<const af_f32x4*>(kb + d * next);
     }
 #pragma unroll
     for (int t = 0; t < KB; ++t) {
-      const float* vb = p.v_pages + ((size_t)max(page[t], 0) * p.KVH + kvh) * head_elems + off[t] + 4 * g;
+      const float* vb = p.v_pages + ((size_t)max(page[t], 0) * KVH + kvh) * head_elems + off[t] + 4 * g;
 #pragma unroll
-      for (int d = 0; d < DT; ++d) v[t][d] = *reinterpret_cast<const af_f32x4*>(vb + (size_t)(16 * d + col) * p.PS);
+      for (int d = 0; d < DT; ++d) v[t][d] = *reinterpret_cast<const af_f32x4*>(vb + (size_t)(16 * d + col) * PS);
     }
     __builtin_amdgcn_sched_barrier(0);
+    if (!RUNS) {
+#pragma unroll
+      for (int t = 0; t < KB; ++t)
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[t][d][e] = fused && (t0 + t) * 16 + 4 * g + e == pos ? nv[d] : v[t][d][e];
+    }
 #pragma unroll
     for (int t = 0; t < KB; ++t) {
       s[t] = af_f32x4{0.f, 0.f, 0.f, 0.f};
@@ -160,20 +186,22 @@ attention_f32_kernel(const AttentionF32Args p) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) weights[(4 * g + r) * 16 + col] = s[t][r];
           asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // within the wave
-          const float* at = p.v_pages + ((size_t)max(page[t], 0) * p.KVH + kvh) * head_elems + off[t] + (size_t)4 * g * p.PS;
+          const float* at = p.v_pages + ((size_t)max(page[t], 0) * KVH + kvh) * head_elems + off[t] + (size_t)4 * g * PS;
 #pragma unroll 1
           for (int j = 0; j < 16; ++j) {
             const int key = (t0 + t) * 16 + j;
             const bool live = key <= pos && key >= first && page[t] >= 0;
             const float weight = weights[j * 16 + col];
-            const float* row = at + j;
+            const bool is_new = fused && key == pos;  // not in its page yet
+            const float* row = is_new ? vn + 4 * g : at + j;
+            const int next = is_new ? 1 : PS;
 #pragma unroll
             for (int d = 0; d < DT; ++d)
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
                 asm volatile("" : "+v"(row));  // one address, moved on: the compiler would keep one for each of the sums
                 if (live) o_acc[d][e] = fmaf(weight, *row, o_acc[d][e]);
-                row += e < 3 ? p.PS : 13 * p.PS;
+                row += e < 3 ? next : 13 * next;
               }
           }
           asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -184,6 +212,16 @@ attention_f32_kernel(const AttentionF32Args p) {
       for (int d = 0; d < DT; ++d)
 #pragma unroll
         for (int e = 0; e < 4; ++e) o_acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][d][e], s[t][e], o_acc[d], 0, 0, 0);
+    }
+  }
+  // the new key and value go to their page: read by later steps only. By the wave behind the one with the last keys, which has none where there are few
+  if (!RUNS && to >= 0 && blockIdx.x % ((group + 15) / 16) == 0 && wave == ((t_last - lo / 16) / KB + 1) % W) {
+    const size_t page = ((size_t)(to / PS) * KVH + kvh) * head_elems;
+    const int at = to % PS;
+#pragma unroll
+    for (int i = lane; i < HD; i += 64) {
+      p.k_pages[page + ((size_t)(i >> 3) * PS + at) * 8 + (i & 7)] = kn[i];
+      p.v_pages[page + (size_t)i * PS + at] = vn[i];
     }
   }
   if (col < nc) {
@@ -218,54 +256,54 @@ attention_f32_kernel(const AttentionF32Args p) {
 }
 
 template <int HD>
-static int attention_f32_launch(const AttentionF32Args& common, const int* tiles, int n_tiles, int tile_rows, const int* tokens, int n_tokens, hipStream_t stream) {
-  AttentionF32Args p = common;
+static int attention_f32_launch(const AttentionF32Args& p, const int* positions, const int* token_seq, const int* block_tables, int bt_stride, int H, int KVH, int PS,
+                                const int* tiles, int n_tiles, int tile_rows, const int* tokens, int n_tokens, hipStream_t stream) {
   constexpr int DT = HD / 16, KB = HD <= 64 ? 4 : 2, KB1 = HD <= 96 ? 2 : 1;  // as many tiles of keys as fit the registers
   if (n_tiles > 0) {
     constexpr int W = 4, lds = W * DT * 4 * 16 * 16 + 2 * W * 16 * 4 + W * 1024;
-    p.work = tiles, p.tile_rows = tile_rows, p.columns = 16;
-    const long blocks = (long)n_tiles * ((tile_rows + 15) / 16) * p.H;
+    const long blocks = (long)n_tiles * ((tile_rows + 15) / 16) * H;
     LEV_REQUIRE(blocks <= 0x7fffffffL, "attention: too many tiles (%ld)", blocks);
-    attention_f32_kernel<HD, KB, W, true><<<(unsigned)blocks, 64 * W, lds, stream>>>(p);
+    attention_f32_kernel<HD, KB, W, true><<<(unsigned)blocks, 64 * W, lds, stream>>>(tiles, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tile_rows, 16, p);
   }
   if (n_tokens > 0) {
     constexpr int W = 8;  // at most 256 registers a lane: head size 128 keeps 52 bytes of them in scratch memory
-    const int group = p.H / p.KVH, sets = (group + 15) / 16;
-    p.work = tokens, p.tile_rows = 0, p.columns = group < 16 ? group : 16;
-    const int lds = W * DT * 4 * p.columns * 16 + 2 * W * 16 * 4 + W * 1024;
-    const long blocks = (long)n_tokens * p.KVH * sets;
+    const int group = H / KVH, sets = (group + 15) / 16, columns = group < 16 ? group : 16;
+    const int lds = W * DT * 4 * columns * 16 + 2 * W * 16 * 4 + W * 1024;
+    const long blocks = (long)n_tokens * KVH * sets;
     LEV_REQUIRE(blocks <= 0x7fffffffL, "attention: too many single tokens (%ld)", blocks);
     if (lds > 64 * 1024) {
       const hipError_t e = hipFuncSetAttribute((const void*)attention_f32_kernel<HD, KB1, W, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
       LEV_REQUIRE(e == hipSuccess, "attention: %d bytes of LDS a workgroup: %s", lds, hipGetErrorString(e));
     }
-    attention_f32_kernel<HD, KB1, W, false><<<(unsigned)blocks, 64 * W, lds, stream>>>(p);
+    attention_f32_kernel<HD, KB1, W, false><<<(unsigned)blocks, 64 * W, lds, stream>>>(tokens, positions, token_seq, block_tables, bt_stride, H, KVH, PS, 0, columns, p);
   }
   return lev_check_launch("attention (32-bit)");
 }
 
 // 1: not for these operands (nothing has been launched): head sizes in steps of 16 up to 128, rows at 16-byte addresses. tiles: (first token,
-// rows <= tile_rows) of runs of several consecutive tokens; tokens: the single ones.
-extern "C" int lev_attention_f32(const float* q, long q_stride, float* out, long o_stride, const float* k_pages, const float* v_pages, const int* positions,
+// rows <= tile_rows) of runs of several consecutive tokens; tokens: the single ones. k_new (a step of single tokens alone): the step's keys and values (rows kv_stride
+// apart) are not in the cache yet and are written to dest[t] = page * PS + offset on the way.
+extern "C" int lev_attention_f32(const float* q, long q_stride, float* out, long o_stride, float* k_pages, float* v_pages, const int* positions,
                                  const int* token_seq, const int* block_tables, int bt_stride, const int* tiles, int n_tiles, int tile_rows, const int* tokens,
-                                 int n_tokens, int H, int KVH, int HD, int PS, float scale, int window, float softcap, const float* score_bias, int bias_len,
+                                 int n_tokens, const float* k_new, const float* v_new, long kv_stride, const int* dest, int H, int KVH, int HD, int PS, float scale, int window, float softcap, const float* score_bias, int bias_len,
                                  hipStream_t stream) {
   LEV_REQUIRE(H > 0 && KVH > 0 && H % KVH == 0, "attention: bad head counts heads=%d kv_heads=%d", H, KVH);
   LEV_REQUIRE(PS > 0 && PS % 16 == 0, "attention: page_size=%d must be a multiple of 16", PS);
   LEV_REQUIRE(window >= 0, "attention: window=%d must not be negative", window);
   LEV_REQUIRE(softcap >= 0.f && (!score_bias || bias_len >= 1), "attention: soft cap %g must not be negative and a bias table needs entries (%d)", (double)softcap, bias_len);
   LEV_REQUIRE(n_tiles >= 0 && n_tokens >= 0 && (n_tiles == 0 || (tiles && tile_rows > 0)) && (n_tokens == 0 || tokens), "attention: a work list is missing");
-  if (HD % 16 != 0 || HD < 16 || HD > 128 || q_stride % 4 != 0 || o_stride % 4 != 0) return 1;
-  if ((((uintptr_t)q | (uintptr_t)out | (uintptr_t)k_pages | (uintptr_t)v_pages) & 15) != 0) return 1;
-  const AttentionF32Args p{q, q_stride, out, o_stride, k_pages, v_pages, positions, token_seq, block_tables, bt_stride, H, KVH, PS, window, bias_len, scale, softcap, score_bias, nullptr, 0, 0};
+  LEV_REQUIRE(!k_new || (v_new && dest && n_tiles == 0), "attention: new keys come with values and destinations, in steps of single tokens");
+  if (HD % 16 != 0 || HD < 16 || HD > 128 || q_stride % 4 != 0 || o_stride % 4 != 0 || (k_new && kv_stride % 4 != 0)) return 1;
+  if ((((uintptr_t)q | (uintptr_t)out | (uintptr_t)k_pages | (uintptr_t)v_pages | (uintptr_t)k_new) & 15) != 0) return 1;
+  const AttentionF32Args p{q, q_stride, out, o_stride, k_pages, v_pages, window, bias_len, scale, softcap, score_bias, k_new, v_new, kv_stride, dest};
   switch (HD / 16) {
-    case 1: return attention_f32_launch<16>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
-    case 2: return attention_f32_launch<32>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
-    case 3: return attention_f32_launch<48>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
-    case 4: return attention_f32_launch<64>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
-    case 5: return attention_f32_launch<80>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
-    case 6: return attention_f32_launch<96>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
-    case 7: return attention_f32_launch<112>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
-    default: return attention_f32_launch<128>(p, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+    case 1: return attention_f32_launch<16>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+    case 2: return attention_f32_launch<32>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+    case 3: return attention_f32_launch<48>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+    case 4: return attention_f32_launch<64>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+    case 5: return attention_f32_launch<80>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+    case 6: return attention_f32_launch<96>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+    case 7: return attention_f32_launch<112>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
+    default: return attention_f32_launch<128>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tiles, n_tiles, tile_rows, tokens, n_tokens, stream);
   }
 }

@@ -331,7 +331,7 @@ register_unit("core", ["errors.hip", "elementwise.hip", "layer_ops.hip", "gemm_s
     "lev_linear_f32_choice": [_I, _I, _I],
     "lev_linear_simple": [_P, _L, _P, _P, _P, _L, _P, _L] + [_I] * 6 + [_P],
     "lev_attention_simple": [_P, _L, _P, _L, _P, _P, _P, _P, _P] + [_I] * 6 + [_F, _I, _I, _F, _P, _I, _P],
-    "lev_attention_f32": [_P, _L, _P, _L, _P, _P, _P, _P, _P, _I, _P, _I, _I, _P, _I] + [_I] * 4 + [_F, _I, _F, _P, _I, _P],
+    "lev_attention_f32": [_P, _L, _P, _L, _P, _P, _P, _P, _P, _I, _P, _I, _I, _P, _I, _P, _P, _L, _P] + [_I] * 4 + [_F, _I, _F, _P, _I, _P],
     "lev_attention_mfma_workspace": [_I] * 5,
 })
 register_unit("gemm_mfma", ["gemm_mfma.hip", "gemm_ring.hip"], signatures={

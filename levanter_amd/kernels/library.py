@@ -1344,7 +1344,7 @@ class HipKernels:
         qs, os_ = _rows(q, "attention: q"), _rows(out, "attention: out")
         kvs = 0
         if k_new is not None:
-            fusable = mfma and meta.n_prefill_tiles == 0 and meta.n_decode == T
+            fusable = (mfma or dt == torch.float32) and meta.n_prefill_tiles == 0 and meta.n_decode == T
             if not fusable:
                 return False
             _dev(k_new, v_new, dest)
@@ -1362,10 +1362,13 @@ class HipKernels:
             return k_new is not None
         if dt == torch.float32:
             rc = self.lib.lev_attention_f32(_ptr(q), qs, _ptr(out), os_, _ptr(k_pages), _ptr(v_pages), pos_ptr, seq_ptr, bt_ptr, bt_width, tiles_ptr,
-                                            meta.n_prefill_tiles, self.prefill_tile_rows, decode_ptr, meta.n_decode, n_heads, n_kv_heads, head_dim, page_size,
+                                            meta.n_prefill_tiles, self.prefill_tile_rows, decode_ptr, meta.n_decode, _ptr(k_new), _ptr(v_new), kvs,
+                                            _ptr(dest) if k_new is not None else None, n_heads, n_kv_heads, head_dim, page_size,
                                             float(scale), w, cap, _ptr(score_bias), bias_len, self._s())
             if rc <= 0:
                 self._check(rc)
+                return k_new is not None
+            if k_new is not None:  # not for these operands: nothing has been launched
                 return False
         self._check(self.lib.lev_attention_simple(
             _ptr(q), qs, _ptr(out), os_, _ptr(k_pages), _ptr(v_pages), pos_ptr, seq_ptr, bt_ptr, bt_width, T, n_heads, n_kv_heads,
