@@ -5,8 +5,9 @@
 //   DELTA:  P_ij = exp(cs_i - cs_j) (q_i . k_j), j <= i;         A_ij = w_i exp(cs_i - cs_j) (k_i . k_j), j < i;     T = (1 + A)^-1
 //           R_i  = w_i (v_i - exp(cs_i) S0^T k_i);               U = T R;     o_i = exp(cs_i) S0^T q_i + sum_j P_ij u_j
 //           S    = exp(cs_end) S0 + sum_j exp(cs_end - cs_j) k_j u_j^T
-// P and T do not depend on the state: a first kernel makes them for all blocks and heads in parallel (entries between tokens of different
-// runs are zero, so T is block-diagonal by itself), a second one goes along each run and carries the state from chunk to chunk. Entries of
+// P, T and the running sums do not depend on the state: a first kernel makes them (of the sums exp(cs_i) and exp(cs_end - cs_i)) for all blocks and heads in parallel
+// (entries between tokens of different runs are zero, so T is block-diagonal by itself), a second one goes along each run and carries the state from chunk to chunk.
+// Its chain of one block after the other is the time of a long prompt: what can be done ahead is, and products that only add up go in sums of their own. Entries of
 // T are bounded: with unit keys and write rates below one, 1 - w k k^T does not lengthen a vector.
 //
 // Exactness. q, k and v are bfloat16 numbers (their unit norms are a float32 factor a row, applied behind the product), so q . k is a
@@ -34,6 +35,11 @@ __device__ __forceinline__ sc_f32x4 sc_mfma(sc_u32x4 a, sc_u32x4 b, sc_f32x4 c) 
   union { sc_u32x4 u; sc_bf16x8 v; } x, y;
   x.u = a, y.u = b;
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.v, y.v, c, 0, 0, 0);
+}
+// the same in four sums that do not wait for each other
+__device__ __forceinline__ void sc_mfma32(sc_f32x4 a, sc_f32x4 b, sc_f32x4 (&c)[4]) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) c[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], c[r], 0, 0, 0);
 }
 __device__ __forceinline__ sc_f32x4 sc_mfma32(sc_f32x4 a, sc_f32x4 b, sc_f32x4 c) {  // 16 of the K dimension: register r is k slot (lane / 16, r)
 #pragma unroll
@@ -97,7 +103,7 @@ __device__ __forceinline__ sc_u32x4 sc_mask8(sc_u32x4 v, int i0, int dk) {
 template <int DKM, int RULE, bool VEC>
 __global__ void __launch_bounds__(256)
 sc_inner_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, const int* __restrict__ token_slots, float* __restrict__ P_out,
-                float* __restrict__ T_out, SrShape s) {
+                float* __restrict__ T_out, float2* __restrict__ E_out, SrShape s) {
   constexpr int LDK = DKM + 8, KS = DKM / 32, QI = DKM / 32;
   constexpr bool DELTA = RULE == SR_DELTA;
   __shared__ __attribute__((aligned(16))) bf16_t s_q[SC_Q][LDK], s_k[SC_Q][LDK];
@@ -120,16 +126,23 @@ sc_inner_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
   if (wave == 0) {
     const int t = min(tb + lane, s.Tn - 1), slot = tb + lane < s.Tn ? token_slots[t] : -1;
     const float* sc = scal + (size_t)t * n_scal;
+    const float w = sc[s.H + h], rk = sc[2 * s.H + g], rq = sc[2 * s.H + s.G + g];
     double cs = slot >= 0 ? (double)sc[h] : 0.0;
+    // running sums within the runs: `begin` is the first of the lane's own, `end` its last
+    const int before = __shfl_up(slot, 1, 64);  // by all lanes
+    const unsigned long long begins = __ballot(lane == 0 || slot != before), behind = begins >> lane >> 1;
+    const int begin = 63 - __clzll(begins & (~0ull >> (63 - lane))), end = behind ? lane + __ffsll(behind) - 1 : 63;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
       const double up = __shfl_up(cs, d, 64);
-      if (lane >= d) cs += up;
+      if (lane - d >= begin) cs += up;
     }
     s_cs[lane] = cs;
     s_slot[lane] = slot;
-    s_w[lane] = sc[s.H + h];
-    s_rk[lane] = sc[2 * s.H + g], s_rq[lane] = sc[2 * s.H + s.G + g];
+    s_w[lane] = w;
+    s_rk[lane] = rk, s_rq[lane] = rq;
+    // what the walk along the runs needs of them: exp(cs_i), and exp(cs_end - cs_i) times the key's weight
+    E_out[((size_t)blockIdx.y * s.H + h) * SC_Q + lane] = make_float2(expf((float)cs), expf((float)(__shfl(cs, end, 64) - cs)) * (DELTA ? rk : w));
   }
   __syncthreads();
   const double cs_i = s_cs[16 * wave + col];  // of the token that is this lane's row in the tiles below
@@ -221,7 +234,7 @@ sc_inner_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
 template <int DKM, int RULE, bool VEC>
 __global__ void __launch_bounds__(256)
 sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, const float* __restrict__ P_in, const float* __restrict__ T_in,
-                float* __restrict__ state, const int* __restrict__ token_slots, float* __restrict__ o, SrShape s) {
+                const float2* __restrict__ E_in, float* __restrict__ state, const int* __restrict__ token_slots, float* __restrict__ o, SrShape s) {
   constexpr int LDK = DKM + 8, KS = DKM / 32, NTW = DKM / 64, KI = DKM / 64, QI = DKM / 32;
   constexpr bool DELTA = RULE == SR_DELTA;
   __shared__ __attribute__((aligned(16))) bf16_t s_q[SC_Q][LDK], s_k[DELTA ? SC_Q : 1][LDK], s_kt[DKM][SC_LDT], s_S[3][SC_VB][LDK];
@@ -262,7 +275,8 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
   sc_u32x4 nk[KI][2], nq[QI];
   bf16_t nv[4];
   sc_f32x4 nP[4], nT[4];
-  float n_ld = 0.f, n_w = 0.f, n_rk = 0.f, n_rq = 0.f;
+  float2 n_e = make_float2(0.f, 0.f);
+  float n_w = 0.f, n_rk = 0.f, n_rq = 0.f;
   auto fetch = [&](int tb) {
 #pragma unroll
     for (int n = 0; n < KI; ++n) {
@@ -290,8 +304,8 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
     }
     if (wave == 0) {
       const float* sc = scal + (size_t)min(tb + lane, s.Tn - 1) * n_scal;
-      n_ld = sc[h], n_w = sc[s.H + h];
-      if (DELTA) n_rk = sc[2 * s.H + g], n_rq = sc[2 * s.H + s.G + g];
+      n_e = E_in[((size_t)(tb / SC_Q) * s.H + h) * SC_Q + lane];
+      if (DELTA) n_w = sc[s.H + h], n_rk = sc[2 * s.H + g], n_rq = sc[2 * s.H + s.G + g];
     }
   };
   auto stage = [&](int tb) {
@@ -332,19 +346,11 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
       }
     }
     if (wave == 0) {
-      const float in = tb + lane >= t0 && tb + lane < t_end ? 1.f : 0.f;  // the block's tokens of other runs: no decay, no weight
-      n_ld *= in, n_w *= in, n_rk *= in, n_rq *= in;
-      double cs = (double)n_ld;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const double up = __shfl_up(cs, d, 64);
-        if (lane >= d) cs += up;
-      }
-      const double end = __shfl(cs, 63, 64);
-      s_ecs[lane] = expf((float)cs);
-      s_wend[lane] = expf((float)(end - cs)) * (DELTA ? n_rk : n_w);
-      s_w[lane] = n_w, s_rk[lane] = n_rk, s_rq[lane] = n_rq;
-      if (lane == 0) s_end = expf((float)end);
+      const bool in = tb + lane >= t0 && tb + lane < t_end;  // the block's tokens of other runs: no weight
+      s_ecs[lane] = in ? n_e.x : 0.f;
+      s_wend[lane] = in ? n_e.y : 0.f;
+      if (DELTA) s_w[lane] = in ? n_w : 0.f, s_rk[lane] = in ? n_rk : 0.f, s_rq[lane] = in ? n_rq : 0.f;
+      if (tb + lane == min(t_end, tb + SC_Q) - 1) s_end = n_e.x;  // the decay of the chunk
     }
   };
 
@@ -364,7 +370,8 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
     if (tb + SC_Q < t_end) fetch(tb + SC_Q);
 
     // rows of the result: tokens 16 wave + .. ; S0^T q and (DELTA) S0^T k, two sums each
-    sc_f32x4 oq = {0.f, 0.f, 0.f, 0.f}, ok = {0.f, 0.f, 0.f, 0.f};
+    const sc_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    sc_f32x4 oq3[3] = {zero, zero, zero}, ok3[3] = {zero, zero, zero};  // a sum for each part of the state: the longest wait in a block is for products in turn
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const sc_u32x4 aq = sc_read16(&s_q[16 * wave + col][32 * ks + 8 * grp]);
@@ -373,10 +380,12 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
 #pragma unroll
       for (int p = 2; p >= 0; --p) {
         const sc_u32x4 b = sc_read16(&s_S[p][col][32 * ks + 8 * grp]);
-        oq = sc_mfma(aq, b, oq);
-        if (DELTA) ok = sc_mfma(ak, b, ok);
+        oq3[p] = sc_mfma(aq, b, oq3[p]);
+        if (DELTA) ok3[p] = sc_mfma(ak, b, ok3[p]);
       }
     }
+    sc_f32x4 oq = (oq3[2] + oq3[1]) + oq3[0];
+    const sc_f32x4 ok = (ok3[2] + ok3[1]) + ok3[0];
     const sc_f32x4 ecs_rows = *reinterpret_cast<const sc_f32x4*>(&s_ecs[16 * wave + 4 * grp]);
     if (DELTA) {
       const sc_f32x4 w_rows = *reinterpret_cast<const sc_f32x4*>(&s_w[16 * wave + 4 * grp]), rk_rows = *reinterpret_cast<const sc_f32x4*>(&s_rk[16 * wave + 4 * grp]);
@@ -389,22 +398,24 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
       }
       s_R[wave][lane] = R;
       lds_barrier();
-      sc_f32x4 U0 = {0.f, 0.f, 0.f, 0.f};
+      sc_f32x4 U4[4] = {zero, zero, zero, zero};
 #pragma unroll
       for (int jt = 0; jt < 4; ++jt) {
         if (jt > wave) break;
-        U0 = sc_mfma32(T[jt], s_R[jt][lane], U0);
+        sc_mfma32(T[jt], s_R[jt][lane], U4);
       }
-      s_U[wave][lane] = U0;
+      s_U[wave][lane] = (U4[0] + U4[1]) + (U4[2] + U4[3]);
       lds_barrier();
       sc_f32x4 U[4];
 #pragma unroll
       for (int jt = 0; jt < 4; ++jt) U[jt] = s_U[jt][lane];
+      sc_f32x4 PU[4] = {zero, zero, zero, zero};
 #pragma unroll
       for (int jt = 0; jt < 4; ++jt) {
         if (jt > wave) break;
-        oq = sc_mfma32(P[jt], U[jt], oq);
+        sc_mfma32(P[jt], U[jt], PU);
       }
+      oq += (PU[0] + PU[1]) + (PU[2] + PU[3]);
       const float dend = s_end;
 #pragma unroll
       for (int n = 0; n < NTW; ++n) S[n] = S[n] * dend;
@@ -476,7 +487,7 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
   }
 }
 
-long sr_chunks_workspace(int rule, int Tn, int H) { return (long)((Tn + SC_Q - 1) / SC_Q) * H * 10 * 256 * (rule == SR_DELTA ? 2 : 1); }
+long sr_chunks_workspace(int rule, int Tn, int H) { return (long)((Tn + SC_Q - 1) / SC_Q) * H * (10 * 256 * (rule == SR_DELTA ? 2 : 1) + 2 * SC_Q); }
 
 int sr_chunks_launch(int rule, const bf16_t* u, const float* scal, float* state, const int* token_slots, float* o, float* workspace, int max_runs,
                      const SrShape& s, hipStream_t stream) {
@@ -485,12 +496,13 @@ int sr_chunks_launch(int rule, const bf16_t* u, const float* scal, float* state,
   LEV_REQUIRE(max_runs <= 65535 && n_blocks <= 65535 && ((uintptr_t)workspace & 15) == 0, "state recurrence: too many runs (%d) or tokens (%d)", max_runs, s.Tn);
   float* P = workspace;
   float* T = workspace + (size_t)n_blocks * s.H * 10 * 256;
+  float2* E = reinterpret_cast<float2*>(rule == SR_DELTA ? T + (size_t)n_blocks * s.H * 10 * 256 : T);
   const dim3 inner(s.H, n_blocks), grid(s.H * ((s.dv + SC_VB - 1) / SC_VB), max_runs);
 #define SC_RUN(DKM, RULE, VEC)                                                                                   \
   do {                                                                                                           \
-    sc_inner_kernel<DKM, RULE, VEC><<<inner, 256, 0, stream>>>(u, scal, token_slots, P, T, s);                    \
+    sc_inner_kernel<DKM, RULE, VEC><<<inner, 256, 0, stream>>>(u, scal, token_slots, P, T, E, s);                 \
     if (lev_check_launch("state recurrence (blocks)")) return -1;                                                \
-    sc_chunk_kernel<DKM, RULE, VEC><<<grid, 256, 0, stream>>>(u, scal, P, T, state, token_slots, o, s);           \
+    sc_chunk_kernel<DKM, RULE, VEC><<<grid, 256, 0, stream>>>(u, scal, P, T, E, state, token_slots, o, s);        \
   } while (0)
 #define SC_GO(DKM)                                          \
   do {                                                      \
