@@ -147,8 +147,8 @@ class StateSlots:
             self.tensors[unit] = torch.zeros((self.n_slots,) + tuple(req.shape), dtype=_TORCH_DTYPES[req.dtype], device=device)
 
     def reset_slot(self, slot: int) -> None:
-        for t in self.tensors.values():
-            t[slot].zero_()
+        if self.tensors:  # one launch for all units
+            torch._foreach_zero_([t[slot] for t in self.tensors.values()])
 
 
 @dataclass
