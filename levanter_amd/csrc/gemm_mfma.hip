@@ -1,7 +1,7 @@
 // bfloat16 matrix products on the matrix cores (MFMA), 32-bit accumulation, fused epilogue:
 //   y = act(a . w^T + bias) (+ residual),  a [M, K] (row stride lda), w [N, K], y [M, N] bf16 or f32.
 // Three kernels here and one in gemm_ring.hip, chosen by the sizes:
-//   ring kernel   (M > 64 and fewer than four million outputs: use_ring): in gemm_ring.hip;
+//   ring kernel   (M > 64 and fewer than four million outputs, long sums from 17 rows: use_ring): in gemm_ring.hip;
 //   tile kernel   (more outputs, M > 128): a 256x256, 256x192, 256x128 or 128x128 tile per workgroup of 4 waves, 32x32x16 MFMA,
 //                 (K split into ranges, with a second kernel for the sums, where the tiles alone would leave CUs idle)
 //                 operands staged through LDS (two buffers), the next k-tile's global loads in registers meanwhile;
@@ -938,7 +938,14 @@ static bool use_skinny(int M, int N, int K) {
 // Where the ring kernel is ahead of the library and of the kernels here, measured at 25 weights of 512 x 2048 to 16384 x 4096 and 65 to 2,048 rows (microseconds, before /
 // ring; the library's kernels are chosen by timing): below 2^22 outputs 0.9 to 1.9 times as fast; above, 12288 x 4096 at 400 / 512 rows 54.7 / 59, 55.8 / 77, 6400 x 1600
 // at 1,000 28.9 / 37, 4096 x 2048 at 2,048 34 / 45. Heads of more outputs than a layer has stay where they were: 50257 x 768 at 65 rows 23.4 / 29.8.
-static bool use_ring(int M, int N, int K) { return M > 64 && N <= 32768 && (long)M * N < (1L << 22) && !use_skinny(M, N, K); }
+// Of 17 to 64 rows it takes long sums up to 48 million weights, and from 41 rows other large ones: the kernels for them have few outputs a CU or a range too
+// many. Microseconds without the pass that adds the ranges, before / ring: 1600 x 6400 at 24 / 64 rows 11.4 / 7.1, 10.3 / 8.8; 768 x 3072 6.2 / 4.5, 9.3 / 5.0; 4096 x 4096
+// at 64 rows 12.9 / 10.5; 4096 x 16384 at 64 rows 31.9 / 32.0. Not 1600 x 1600 at 24 rows (5.1 / 4.3, less than the norm then pays for the ranges) nor gated inner sizes (2048 x 5376 at
+// 32 rows 11.0 / 7.4, but a session of Lelatar 33.1 -> 33.8 ms: a kernel of its own adds the ranges there). Sessions: GPT-2 XL, 24 requests 116.3 -> 115.0 ms, 7B, 64 requests 170.8 -> 169.7.
+static bool use_ring(int M, int N, int K) {
+  if (M > 16 && M <= 64) return !g_force_kernel && N <= K && (long)N * K < 48000000L && ((K >= 4L * N && K >= 3072) || (M > 40 && (long)N * K >= (1L << 24)));
+  return M > 64 && N <= 32768 && (long)M * N < (1L << 22) && !use_skinny(M, N, K);
+}
 
 // The tile and the ranges of the ring kernel, 16 x tile + ranges; -1 where another kernel takes the product.
 extern "C" int lev_linear_mfma_ring(int M, int N, int K) {
@@ -949,8 +956,8 @@ extern "C" int lev_linear_mfma_ring(int M, int N, int K) {
 
 // Into how many ranges the sum over K is split (1: the kernel finishes its outputs itself).
 extern "C" int lev_linear_mfma_ranges(int M, int N, int K) {
-  if (use_skinny(M, N, K)) return 1;
   if (use_ring(M, N, K)) return lev_ring_plan(M, N, K).splits;
+  if (use_skinny(M, N, K)) return 1;
   return M <= 128 ? plan_stream(M, N, K).splits : plan_tiles(M, N, K).splits;
 }
 
@@ -1003,13 +1010,13 @@ static int launch_stream(const bf16_t* a, long lda, const bf16_t* w, const float
 template <typename TO>
 static int linear_mfma_typed(const bf16_t* a, long lda, const bf16_t* w, const float* bias, const float* residual, long ldr,
                              TO* out, long ldo, float* workspace, int M, int N, int K, int act, int defer, hipStream_t stream) {
-  if (use_skinny(M, N, K)) {
-    launch_skinny<TO>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act, stream);
-  } else if (use_ring(M, N, K)) {
+  if (use_ring(M, N, K)) {
     const RingPlan plan = lev_ring_plan(M, N, K);
     const int rc = lev_ring_launch(plan, a, lda, w, bias, residual, ldr, out, ldo, workspace, M, N, K, act, sizeof(TO) == 4 ? LEV_F32 : LEV_BF16, stream);
     if (rc || plan.splits == 1 || defer) return rc;
     return launch_splitk_reduce<TO>(workspace, bias, residual, ldr, out, ldo, M, N, plan.splits, act, stream);
+  } else if (use_skinny(M, N, K)) {
+    launch_skinny<TO>(a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act, stream);
   } else if (M <= 128) {
     return launch_stream<TO>(a, lda, w, bias, residual, ldr, out, ldo, workspace, M, N, K, act, defer, stream);
   } else {

@@ -311,7 +311,9 @@ static const RingShape kRing[8] = {
 };
 
 // An estimate of every tile and number of ranges: rounds of the CUs times a workgroup's k-tiles, joined (exponent 1.27: neither hides the other wholly) with the time the
-// weights take from memory, and what writing the sums costs; of ranges also the pass that adds them, which the norm behind the product does for less. Fitted to
+// weights take from memory, and what writing the sums costs; of ranges also the pass that adds them: a kernel of its own, or,
+// for the longest sums (K >= 4 N), which lead into a residual stream, what the norm behind the product pays for them (64 rows of 1600: 2.5 us, with 2 / 4 / 8 ranges 3.2 / 3.4 / 4.1; 264 rows
+// 2.8, 4.4 / 5.0 / 6.1). Fitted to
 // 13,000 launches (25 weights of 512 x 2048 to 16384 x 4096, 64 to 2,048 rows, up to five million outputs): off by 6 % on average, and the tile it chooses is 0.7 %
 // behind the best on average, more than 8 % in 8 of 383 shapes (2048 rows of 2048 x 5376: 57.2 us for 50.5).
 static RingPlan ring_choice(int M, int N, int K) {
@@ -336,7 +338,8 @@ static RingPlan ring_choice(int M, int N, int K) {
       }
       cus *= 1.0 + 0.110 * (beyond < 0.0 ? 0.0 : beyond > 1.0 ? 1.0 : beyond);
       double us = 1.63 + pow(pow(cus, 1.27) + pow(memory, 1.27), 1.0 / 1.27) + 0.214 * s * outputs;
-      if (s > 1) us += 1.5 + (s + 1) * outputs / 4.5;
+      if (K >= 4L * N) us += s > 1 ? 0.6 + s * outputs / 4.5 : 0.5;
+      else if (s > 1) us += 1.5 + (s + 1) * outputs / 4.5;
       if (us < best.us) best = {i, s, us};
     }
   }

@@ -7,7 +7,8 @@ DEV = "cuda:0"
 
 # rows, outputs, inputs; together they reach all eight tiles, one range and several (asserted below)
 SHAPES = [(97, 2304, 768), (65, 4100, 40), (100, 2321, 8), (129, 2049, 72), (200, 3072, 824), (264, 4800, 1600), (264, 1600, 6400), (300, 1601, 6408), (65, 4096, 16384), (100, 1000, 4096),
-          (264, 6400, 1600), (333, 6400, 1592), (777, 4800, 1600), (600, 2048, 5376), (1000, 3072, 776), (264, 12288, 520), (300, 12289, 392), (2047, 2048, 512), (1299, 2052, 1024), (511, 8190, 72)]
+          (264, 6400, 1600), (333, 6400, 1592), (777, 4800, 1600), (600, 2048, 5376), (1000, 3072, 776), (264, 12288, 520), (300, 12289, 392), (2047, 2048, 512), (1299, 2052, 1024), (511, 8190, 72),
+          (17, 768, 3072), (33, 1601, 6408), (64, 1600, 6400), (50, 4096, 4096)]
 
 
 @pytest.fixture(scope="module")
