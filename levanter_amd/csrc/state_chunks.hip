@@ -229,16 +229,18 @@ sc_inner_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
 }
 
 // ---- along the runs -------------------------------------------------------------------------------------------------------------
-// One workgroup of four waves per (run, head, 16 value columns); wave w has the tokens 16 w .. of the block as rows of the result and a quarter
-// of the state's key channels, in accumulator registers.
-template <int DKM, int RULE, bool VEC>
+// One workgroup of four waves per (run, head, 16 CT value columns); wave w has the tokens 16 w .. of the block as rows of the result and a quarter
+// of the state's key channels, in accumulator registers. SSD takes up to 64 columns at once where there are many runs: what a block stages in LDS (keys, queries, weights)
+// is the same for all of them (64 heads of 128 / 64, microseconds with 16 / 64 columns: 32 runs of 40 to 150 tokens 205 / 158, but three of 300 to 999, whose chain is the bound, 62 / 100). DELTA stays at 16: its products with two 32-bit sides are four times as long.
+template <int DKM, int RULE, bool VEC, int CT>
 __global__ void __launch_bounds__(256)
 sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, const float* __restrict__ P_in, const float* __restrict__ T_in,
                 const float2* __restrict__ E_in, float* __restrict__ state, const int* __restrict__ token_slots, float* __restrict__ o, SrShape s) {
   constexpr int LDK = DKM + 8, KS = DKM / 32, NTW = DKM / 64, KI = DKM / 64, QI = DKM / 32;
   constexpr bool DELTA = RULE == SR_DELTA;
-  __shared__ __attribute__((aligned(16))) bf16_t s_q[SC_Q][LDK], s_k[DELTA ? SC_Q : 1][LDK], s_kt[DKM][SC_LDT], s_S[3][SC_VB][LDK];
-  __shared__ __attribute__((aligned(16))) bf16_t s_x[DELTA ? 1 : SC_VB][SC_LDT];
+  static_assert(!DELTA || CT == 1, "one tile of columns");
+  __shared__ __attribute__((aligned(16))) bf16_t s_q[SC_Q][LDK], s_k[DELTA ? SC_Q : 1][LDK], s_kt[DKM][SC_LDT], s_S[3][SC_VB * CT][LDK];
+  __shared__ __attribute__((aligned(16))) bf16_t s_x[DELTA ? 1 : SC_VB * CT][SC_LDT];
   __shared__ __attribute__((aligned(16))) float s_ecs[SC_Q], s_wend[SC_Q], s_w[SC_Q], s_rk[SC_Q], s_rq[SC_Q];
   __shared__ float s_end;
   __shared__ __attribute__((aligned(16))) sc_f32x4 s_R[DELTA ? 4 : 1][64], s_U[DELTA ? 4 : 1][64];
@@ -247,33 +249,39 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
   // the slowest index; and the heads of a chiplet are neighbours, which read the same keys and queries through its cache.
   const int n_items = gridDim.x, per_xcd = n_items / 8;
   const int item = n_items % 8 == 0 ? (blockIdx.x % 8) * per_xcd + blockIdx.x / 8 : blockIdx.x;
-  const int n_blocks = (s.dv + SC_VB - 1) / SC_VB, h = item / n_blocks;
+  const int n_blocks = (s.dv + SC_VB * CT - 1) / (SC_VB * CT), h = item / n_blocks;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, grp = lane >> 4;
   const int g = h / (s.H / s.G), n_scal = 2 * s.H + 2 * s.G, dk = s.dk, dv = s.dv;
-  const int j = (item - h * n_blocks) * SC_VB + col;  // this lane's value column
-  const bool live = j < dv;
+  const int j = (item - h * n_blocks) * SC_VB * CT + col;  // this lane's value column, and every 16th behind it
+  bool live[CT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c) live[c] = j + 16 * c < dv;
   int t0, t_end, slot;
   if (!sr_find_run<256>(blockIdx.y, token_slots, s.Tn, tmp, t0, t_end, slot)) return;
   const bf16_t* uk = u + s.k_off + (size_t)g * dk;
   const bf16_t* uq = u + s.q_off + (size_t)g * dk;
   const bf16_t* uv = u + s.v_off + (size_t)h * dv;
-  const int jc = live ? j : 0;
-  float* sp = state + (size_t)slot * s.slot_stride + (size_t)s.K * s.C + (size_t)h * dk * dv + jc;
+  int jc[CT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c) jc[c] = live[c] ? j + 16 * c : 0;
+  float* sp = state + (size_t)slot * s.slot_stride + (size_t)s.K * s.C + (size_t)h * dk * dv;
 
   // the state: key channels 16 (wave * NTW + n) + 4 grp + r of column j
-  sc_f32x4 S[NTW];
+  sc_f32x4 S[CT][NTW];
 #pragma unroll
-  for (int n = 0; n < NTW; ++n)
+  for (int c = 0; c < CT; ++c)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = 16 * (wave * NTW + n) + 4 * grp + r;
-      S[n][r] = live && i < dk ? sp[(size_t)i * dv] : 0.f;
-    }
+    for (int n = 0; n < NTW; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = 16 * (wave * NTW + n) + 4 * grp + r;
+        S[c][n][r] = live[c] && i < dk ? sp[(size_t)i * dv + jc[c]] : 0.f;
+      }
 
   // what of the next block is on its way: keys (two neighbouring tokens, eight channels), queries, values, scalars, this wave's rows of P and T.
   // Raw loads only, under no condition: whatever is computed from them here would wait for their way through the memory.
   sc_u32x4 nk[KI][2], nq[QI];
-  bf16_t nv[4];
+  bf16_t nv[CT][4];
   sc_f32x4 nP[4], nT[4];
   float2 n_e = make_float2(0.f, 0.f);
   float n_w = 0.f, n_rk = 0.f, n_rq = 0.f;
@@ -293,7 +301,8 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
     for (int r = 0; r < 4; ++r) {
       // DELTA: the rows and the column of this lane's part of R; SSD: 16 columns of four tokens per thread, for the transposed copy
       const int t = DELTA ? tb + 16 * wave + 4 * grp + r : tb + (tid >> 4) + 16 * r;
-      nv[r] = uv[(size_t)min(t, s.Tn - 1) * s.C + jc];
+#pragma unroll
+      for (int c = 0; c < CT; ++c) nv[c][r] = uv[(size_t)min(t, s.Tn - 1) * s.C + jc[c]];
     }
     const size_t tile = ((size_t)(tb / SC_Q) * s.H + h) * 10 + wave * (wave + 1) / 2;
 #pragma unroll
@@ -331,20 +340,24 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
     }
     if (!DELTA)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) s_x[col][(tid >> 4) + 16 * r] = live ? nv[r] : (bf16_t)0;
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-    for (int n = 0; n < NTW; ++n) {
-      float rest[4];
+        for (int c = 0; c < CT; ++c) s_x[16 * c + col][(tid >> 4) + 16 * r] = live[c] ? nv[c][r] : (bf16_t)0;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) rest[r] = S[n][r];
+    for (int c = 0; c < CT; ++c)
 #pragma unroll
-      for (int p = 0; p < 3; ++p) {
-        const uint32_t lo = float2_to_bf16x2(rest[0], rest[1]), hi = float2_to_bf16x2(rest[2], rest[3]);
-        *reinterpret_cast<sc_u32x2*>(&s_S[p][col][16 * (wave * NTW + n) + 4 * grp]) = sc_u32x2{lo, hi};
-        rest[0] -= __uint_as_float(lo << 16), rest[1] -= __uint_as_float(lo & 0xffff0000u);
-        rest[2] -= __uint_as_float(hi << 16), rest[3] -= __uint_as_float(hi & 0xffff0000u);
+      for (int n = 0; n < NTW; ++n) {
+        float rest[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) rest[r] = S[c][n][r];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          const uint32_t lo = float2_to_bf16x2(rest[0], rest[1]), hi = float2_to_bf16x2(rest[2], rest[3]);
+          *reinterpret_cast<sc_u32x2*>(&s_S[p][16 * c + col][16 * (wave * NTW + n) + 4 * grp]) = sc_u32x2{lo, hi};
+          rest[0] -= __uint_as_float(lo << 16), rest[1] -= __uint_as_float(lo & 0xffff0000u);
+          rest[2] -= __uint_as_float(hi << 16), rest[3] -= __uint_as_float(hi & 0xffff0000u);
+        }
       }
-    }
     if (wave == 0) {
       const bool in = tb + lane >= t0 && tb + lane < t_end;  // the block's tokens of other runs: no weight
       s_ecs[lane] = in ? n_e.x : 0.f;
@@ -362,7 +375,7 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
     stage(tb);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      v_now[r] = live ? to_float<bf16_t>(nv[r]) : 0.f;
+      v_now[r] = live[0] ? to_float<bf16_t>(nv[0][r]) : 0.f;  // DELTA
       P[r] = nP[r];
       if (DELTA) T[r] = nT[r];
     }
@@ -371,20 +384,26 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
 
     // rows of the result: tokens 16 wave + .. ; S0^T q and (DELTA) S0^T k, two sums each
     const sc_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    sc_f32x4 oq3[3] = {zero, zero, zero}, ok3[3] = {zero, zero, zero};  // a sum for each part of the state: the longest wait in a block is for products in turn
+    sc_f32x4 oq3[CT][3], ok3[3] = {zero, zero, zero};  // a sum for each part of the state: the longest wait in a block is for products in turn
+#pragma unroll
+    for (int c = 0; c < CT; ++c) oq3[c][0] = oq3[c][1] = oq3[c][2] = zero;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const sc_u32x4 aq = sc_read16(&s_q[16 * wave + col][32 * ks + 8 * grp]);
       sc_u32x4 ak;
       if (DELTA) ak = sc_read16(&s_k[DELTA ? 16 * wave + col : 0][32 * ks + 8 * grp]);
 #pragma unroll
-      for (int p = 2; p >= 0; --p) {
-        const sc_u32x4 b = sc_read16(&s_S[p][col][32 * ks + 8 * grp]);
-        oq3[p] = sc_mfma(aq, b, oq3[p]);
-        if (DELTA) ok3[p] = sc_mfma(ak, b, ok3[p]);
-      }
+      for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int p = 2; p >= 0; --p) {
+          const sc_u32x4 b = sc_read16(&s_S[p][16 * c + col][32 * ks + 8 * grp]);
+          oq3[c][p] = sc_mfma(aq, b, oq3[c][p]);
+          if (DELTA) ok3[p] = sc_mfma(ak, b, ok3[p]);
+        }
     }
-    sc_f32x4 oq = (oq3[2] + oq3[1]) + oq3[0];
+    sc_f32x4 oq[CT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) oq[c] = (oq3[c][2] + oq3[c][1]) + oq3[c][0];
     const sc_f32x4 ok = (ok3[2] + ok3[1]) + ok3[0];
     const sc_f32x4 ecs_rows = *reinterpret_cast<const sc_f32x4*>(&s_ecs[16 * wave + 4 * grp]);
     if (DELTA) {
@@ -394,7 +413,7 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         R[r] = w_rows[r] * (v_now[r] - ecs_rows[r] * rk_rows[r] * ok[r]);
-        oq[r] *= ecs_rows[r] * rq_rows[r];
+        oq[0][r] *= ecs_rows[r] * rq_rows[r];
       }
       s_R[wave][lane] = R;
       lds_barrier();
@@ -415,10 +434,10 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
         if (jt > wave) break;
         sc_mfma32(P[jt], U[jt], PU);
       }
-      oq += (PU[0] + PU[1]) + (PU[2] + PU[3]);
+      oq[0] += (PU[0] + PU[1]) + (PU[2] + PU[3]);
       const float dend = s_end;
 #pragma unroll
-      for (int n = 0; n < NTW; ++n) S[n] = S[n] * dend;
+      for (int n = 0; n < NTW; ++n) S[0][n] = S[0][n] * dend;
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
         const sc_f32x4 w0 = *reinterpret_cast<const sc_f32x4*>(&s_wend[32 * half + 4 * grp]), w1 = *reinterpret_cast<const sc_f32x4*>(&s_wend[32 * half + 16 + 4 * grp]);
@@ -432,59 +451,73 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
           const bf16_t* row = s_kt[16 * (wave * NTW + n) + col];
           const sc_u32x4 a = sc_read8x2(row + 32 * half + 4 * grp, row + 32 * half + 16 + 4 * grp);
 #pragma unroll
-          for (int p = 2; p >= 0; --p) S[n] = sc_mfma(a, b[p], S[n]);
+          for (int p = 2; p >= 0; --p) S[0][n] = sc_mfma(a, b[p], S[0][n]);
         }
       }
     } else {
-      oq = oq * ecs_rows;
       const float dend = s_end;
 #pragma unroll
-      for (int n = 0; n < NTW; ++n) S[n] = S[n] * dend;
+      for (int c = 0; c < CT; ++c) {
+        oq[c] = oq[c] * ecs_rows;
+#pragma unroll
+        for (int n = 0; n < NTW; ++n) S[c][n] = S[c][n] * dend;
+      }
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
-        const sc_u32x4 x8 = sc_read8x2(&s_x[DELTA ? 0 : col][32 * half + 4 * grp], &s_x[DELTA ? 0 : col][32 * half + 16 + 4 * grp]);
-        float v8[8];
-        sc_u32x4 b[3];
-        if (2 * half <= wave) {
+        sc_u32x4 pb[3];
+        if (2 * half <= wave) {  // the block's weights, the same for all columns
           const float second = 2 * half + 1 <= wave ? 1.f : 0.f;
+          float p8[8];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v8[e] = P[2 * half][e], v8[4 + e] = P[2 * half + 1][e] * second;
-          sc_split(v8, b);
-#pragma unroll
-          for (int p = 2; p >= 0; --p) oq = sc_mfma(b[p], x8, oq);
+          for (int e = 0; e < 4; ++e) p8[e] = P[2 * half][e], p8[4 + e] = P[2 * half + 1][e] * second;
+          sc_split(p8, pb);
         }
         const sc_f32x4 w0 = *reinterpret_cast<const sc_f32x4*>(&s_wend[32 * half + 4 * grp]), w1 = *reinterpret_cast<const sc_f32x4*>(&s_wend[32 * half + 16 + 4 * grp]);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float xv = __uint_as_float((e & 1) ? x8[e >> 1] & 0xffff0000u : x8[e >> 1] << 16);
-          v8[e] = xv * (e < 4 ? w0[e] : w1[e - 4]);
-        }
-        sc_split(v8, b);
+        for (int c = 0; c < CT; ++c) {
+          const int xr = DELTA ? 0 : 16 * c + col;
+          const sc_u32x4 x8 = sc_read8x2(&s_x[xr][32 * half + 4 * grp], &s_x[xr][32 * half + 16 + 4 * grp]);
+          if (2 * half <= wave)
 #pragma unroll
-        for (int n = 0; n < NTW; ++n) {
-          const bf16_t* row = s_kt[16 * (wave * NTW + n) + col];
-          const sc_u32x4 a = sc_read8x2(row + 32 * half + 4 * grp, row + 32 * half + 16 + 4 * grp);
+            for (int p = 2; p >= 0; --p) oq[c] = sc_mfma(pb[p], x8, oq[c]);
+          float v8[8];
+          sc_u32x4 b[3];
 #pragma unroll
-          for (int p = 2; p >= 0; --p) S[n] = sc_mfma(a, b[p], S[n]);
+          for (int e = 0; e < 8; ++e) {
+            const float xv = __uint_as_float((e & 1) ? x8[e >> 1] & 0xffff0000u : x8[e >> 1] << 16);
+            v8[e] = xv * (e < 4 ? w0[e] : w1[e - 4]);
+          }
+          sc_split(v8, b);
+#pragma unroll
+          for (int n = 0; n < NTW; ++n) {
+            const bf16_t* row = s_kt[16 * (wave * NTW + n) + col];
+            const sc_u32x4 a = sc_read8x2(row + 32 * half + 4 * grp, row + 32 * half + 16 + 4 * grp);
+#pragma unroll
+            for (int p = 2; p >= 0; --p) S[c][n] = sc_mfma(a, b[p], S[c][n]);
+          }
         }
       }
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = tb + 16 * wave + 4 * grp + r;
-      if (live && t >= t0 && t < t_end) o[((size_t)t * s.H + h) * dv + j] = oq[r];
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+        if (live[c] && t >= t0 && t < t_end) o[((size_t)t * s.H + h) * dv + j + 16 * c] = oq[c][r];
     }
     lds_barrier();  // the block's tiles have been read by every wave
   }
-  if (live) {
 #pragma unroll
-    for (int n = 0; n < NTW; ++n)
+  for (int c = 0; c < CT; ++c)
+    if (live[c]) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = 16 * (wave * NTW + n) + 4 * grp + r;
-        if (i < dk) sp[(size_t)i * dv] = S[n][r];
-      }
-  }
+      for (int n = 0; n < NTW; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = 16 * (wave * NTW + n) + 4 * grp + r;
+          if (i < dk) sp[(size_t)i * dv + jc[c]] = S[c][n][r];
+        }
+    }
 }
 
 long sr_chunks_workspace(int rule, int Tn, int H) { return (long)((Tn + SC_Q - 1) / SC_Q) * H * (10 * 256 * (rule == SR_DELTA ? 2 : 1) + 2 * SC_Q); }
@@ -497,12 +530,21 @@ int sr_chunks_launch(int rule, const bf16_t* u, const float* scal, float* state,
   float* P = workspace;
   float* T = workspace + (size_t)n_blocks * s.H * 10 * 256;
   float2* E = reinterpret_cast<float2*>(rule == SR_DELTA ? T + (size_t)n_blocks * s.H * 10 * 256 : T);
-  const dim3 inner(s.H, n_blocks), grid(s.H * ((s.dv + SC_VB - 1) / SC_VB), max_runs);
+  const dim3 inner(s.H, n_blocks);
+  // columns at once: 64 (or as many as there are) where even so the runs give every CU four workgroups, else 16; of heads of 256 keys, which fill the LDS, 16. A token's
+  // sums are the same.
+  const long items = (long)max_runs * s.H * ((s.dv + SC_VB - 1) / SC_VB);
+  const int tiles = rule == SR_DELTA || s.dk > 128 || items < 4096 ? 1 : s.dv > 32 ? 4 : s.dv > 16 ? 2 : 1;
+  const dim3 grid(s.H * ((s.dv + SC_VB * tiles - 1) / (SC_VB * tiles)), max_runs);
+#define SC_CHUNK(DKM, RULE, VEC, CT) sc_chunk_kernel<DKM, RULE, VEC, CT><<<grid, 256, 0, stream>>>(u, scal, P, T, E, state, token_slots, o, s)
 #define SC_RUN(DKM, RULE, VEC)                                                                                   \
   do {                                                                                                           \
     sc_inner_kernel<DKM, RULE, VEC><<<inner, 256, 0, stream>>>(u, scal, token_slots, P, T, E, s);                 \
     if (lev_check_launch("state recurrence (blocks)")) return -1;                                                \
-    sc_chunk_kernel<DKM, RULE, VEC><<<grid, 256, 0, stream>>>(u, scal, P, T, E, state, token_slots, o, s);        \
+    if constexpr (RULE == SR_DELTA || DKM > 128) SC_CHUNK(DKM, RULE, VEC, 1);                                    \
+    else if (tiles == 4) SC_CHUNK(DKM, RULE, VEC, 4);                                                            \
+    else if (tiles == 2) SC_CHUNK(DKM, RULE, VEC, 2);                                                            \
+    else SC_CHUNK(DKM, RULE, VEC, 1);                                                                            \
   } while (0)
 #define SC_GO(DKM)                                          \
   do {                                                      \
@@ -516,5 +558,6 @@ int sr_chunks_launch(int rule, const bf16_t* u, const float* scal, float* state,
   else SC_GO(256);
 #undef SC_GO
 #undef SC_RUN
+#undef SC_CHUNK
   return lev_check_launch("state recurrence (chunks)");
 }
