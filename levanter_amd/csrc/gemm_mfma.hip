@@ -14,6 +14,7 @@
 // No atomics anywhere: results are deterministic. K and lda must be multiples of 8 (16-byte operand loads);
 // any M and N.
 #include "common.h"
+#include "gemm_norm.h"
 #include "gemm_ring.h"
 #include <type_traits>
 
@@ -1057,4 +1058,23 @@ extern "C" int lev_linear_mfma(const void* a, long lda, const void* w, const flo
     return linear_mfma_typed<bf16_t>((const bf16_t*)a, lda, (const bf16_t*)w, bias, residual, ldr, (bf16_t*)out, ldo,
                                      (float*)workspace, M, N, K, act, leave_ranges, stream);
   return lev_fail("linear: unknown output dtype %d", out_dtype);
+}
+
+// Which products of a few rows take the norm ahead of them along (gemm_norm.hip, with the figures): those of the skinny kernel whose workgroups make one
+// round of the CUs (more would normalise in vain), but none that spreads a short sum over many outputs (11520 x 256 at 4 / 8 rows 6.4 / 6.2, 6.5 / 6.8). Sums
+// below 256 have not been measured, half units (up to 2,048 outputs) are shapes of products that follow no norm.
+extern "C" int lev_linear_normed_takes(int M, int N, int K) {
+  if (M < 1 || M > NORMED_MAX_M || K < 256 || K > NORMED_MAX_K || K % 8 || N <= 2048 || N > 16 * 720 || (K < 512 && N > 8192) || g_force_kernel == 2 || !use_skinny(M, N, K)) return 0;
+  return !skinny_shape(M, N, K).half;
+}
+
+// out = act(norm(x) . w^T + bias): the norm of lev_norm into bfloat16 and the product of lev_linear_mfma, bit for bit, in one kernel. x [M][K] float32.
+extern "C" int lev_linear_normed(const float* x, const float* norm_w, const float* norm_b, float eps, int rms, const void* w, const float* bias, void* out,
+                                 long ldo, int M, int N, int K, int act, hipStream_t stream) {
+  LEV_REQUIRE(x && norm_w && w && out && lev_linear_normed_takes(M, N, K), "norm and linear: no kernel for M=%d N=%d K=%d", M, N, K);
+  LEV_REQUIRE((((uintptr_t)x | (uintptr_t)norm_w | (uintptr_t)norm_b | (uintptr_t)w) & 15) == 0, "norm and linear: operands must be 16-byte aligned");
+  LEV_REQUIRE(ldo >= N && eps > 0.f && act >= LEV_ACT_NONE && act <= LEV_ACT_LAST, "norm and linear: bad ldo=%ld, eps=%g or activation %d", ldo, eps, act);
+  const SkinnyShape sh = skinny_shape(M, N, K);
+  const int rc = lev_normed_launch(sh.waves, sh.units, x, norm_w, norm_b, eps, rms, (const bf16_t*)w, bias, (bf16_t*)out, ldo, M, N, K, act, stream);
+  return rc < 0 ? lev_fail("norm and linear: no kernel of %d waves and %d units", sh.waves, sh.units) : rc;
 }

@@ -334,12 +334,14 @@ register_unit("core", ["errors.hip", "elementwise.hip", "layer_ops.hip", "gemm_s
     "lev_attention_f32": [_P, _L, _P, _L, _P, _P, _P, _P, _P, _I, _P, _I, _I, _P, _I, _P, _P, _L, _P] + [_I] * 4 + [_F, _I, _F, _P, _I, _P],
     "lev_attention_mfma_workspace": [_I] * 5,
 })
-register_unit("gemm_mfma", ["gemm_mfma.hip", "gemm_ring.hip"], signatures={
+register_unit("gemm_mfma", ["gemm_mfma.hip", "gemm_ring.hip", "gemm_norm.hip"], signatures={
     "lev_linear_mfma": [_P, _L, _P, _P, _P, _L, _P, _L, _P] + [_I] * 6 + [_P],
     "lev_linear_mfma_workspace": [_I, _I, _I],
     "lev_linear_mfma_ranges": [_I, _I, _I],
     "lev_linear_mfma_ring": [_I, _I, _I],
     "lev_linear_mfma_force": [_I],
+    "lev_linear_normed": [_P, _P, _P, _F, _I, _P, _P, _P, _L, _I, _I, _I, _I, _P],
+    "lev_linear_normed_takes": [_I, _I, _I],
     "lev_linear_mfma_finish": [_P, _P, _P, _L, _P, _L] + [_I] * 5 + [_P],
 })
 # the vendor library's GEMM (hipBLASLt) behind the same interface

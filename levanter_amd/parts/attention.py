@@ -61,6 +61,10 @@ class CausalSelfAttention(Mixer):
             self.rotary = part_class(rotary.kind, rotary.family or "position")(rotary, tensors_of_nested("rotary", tensors), env)
             self.graph_safe = bool(self.rotary.graph_safe)  # the rotation runs inside this mixer's forward
 
+    @property
+    def first_product(self):
+        return self.qkv
+
     def cache_requirement(self):
         return PagedKv(self.n_kv_heads, self.head_dim, self.window)
 

@@ -157,6 +157,10 @@ class Norm(Part):
     def __call__(self, x: torch.Tensor, ctx: StepContext, rows: Optional[torch.Tensor] = None) -> torch.Tensor:
         raise NotImplementedError
 
+    def ahead_of(self, product, x: torch.Tensor, ctx: StepContext):
+        """``self(x, ctx)`` for a part whose ``first_product`` alone reads it: the rows, or what that product makes them out of itself."""
+        return self(x, ctx)
+
 
 class PositionEncoding(Part):
     """Two hooks; a position encoding uses one of them.
@@ -182,6 +186,8 @@ class Mixer(Part):
     ``[T, dim]``) to the residual ``x`` (float32 ``[T, dim]``) in place; reads (and, if
     ``writes_cache``, first writes) ``unit``."""
 
+    first_product = None  # the ``Linear`` through which alone ``forward`` reads ``h`` (besides its shape), if there is one
+
     def cache_requirement(self):
         return None
 
@@ -198,6 +204,8 @@ class Mixer(Part):
 
 class FeedForward(Part):
     """``forward(h, x, ctx)``: adds the feed-forward's output for ``h`` to the residual ``x`` in place."""
+
+    first_product = None  # as a mixer's
 
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext) -> None:
         raise NotImplementedError

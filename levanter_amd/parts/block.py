@@ -31,13 +31,18 @@ class PreNormBlock(Block):
         # a product that the part before has left unfinished is folded into the norm that follows it, or finished first
         if not self.norm1.folds_pending:
             ctx.settle()
-        self.mixer.forward(self.norm1(x, ctx), x, ctx, unit, writes_cache)
+        self.mixer.forward(self._normed(self.norm1, self.mixer, x, ctx), x, ctx, unit, writes_cache)
         if self.feed_forward is not None:
             if not self.norm2.folds_pending:
                 ctx.settle()
-            self.feed_forward.forward(self.norm2(x, ctx), x, ctx)
+            self.feed_forward.forward(self._normed(self.norm2, self.feed_forward, x, ctx), x, ctx)
         if self.token_input is not None:
             self.token_input.add(x, ctx)
+
+    @staticmethod
+    def _normed(norm, part, x: torch.Tensor, ctx: StepContext):
+        product = part.first_product
+        return norm(x, ctx) if product is None else norm.ahead_of(product, x, ctx)
 
 
 @BLOCKS.register("parallel")

@@ -29,6 +29,10 @@ class DenseMlp(FeedForward):
         if (self.up.n_in, self.up.n_out) != (p["dim"], p["inner_dim"]) or (self.down.n_in, self.down.n_out) != (p["inner_dim"], p["dim"]):
             raise ValueError("dense_mlp: weights do not have the sizes of the description")
 
+    @property
+    def first_product(self):
+        return self.up
+
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext) -> None:
         m = self.up(h, ctx, activation=self.activation)
         self.down(m, ctx, residual=x, final=True)
@@ -77,6 +81,10 @@ class GatedMlp(FeedForward):
         w_down = torch.zeros(D, Fp)
         w_down[:, :F] = f32("down.weight", (D, F))
         self.down = Linear(w_down, tensors.get("down.bias"), "out_in", env)
+
+    @property
+    def first_product(self):
+        return self.up
 
     def _inner(self, h: torch.Tensor, ctx: StepContext) -> torch.Tensor:
         z = self.up(h, ctx)

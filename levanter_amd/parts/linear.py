@@ -8,6 +8,16 @@ import torch
 from .base import BuildEnv, StepContext
 
 
+class RowsAhead:
+    """Rows that a norm has yet to make out of the float32 ``x``: what ``Norm.ahead_of`` gives to the one product that reads them, whose kernel
+    normalises them on the way. ``x`` stays as it is until that product has been launched."""
+
+    __slots__ = ("x", "norm", "shape")
+
+    def __init__(self, x: torch.Tensor, norm):
+        self.x, self.norm, self.shape = x, norm, x.shape
+
+
 class Linear:
     def __init__(self, weight: torch.Tensor, bias: Optional[torch.Tensor], layout: str, env: BuildEnv):
         """``layout``: "in_out" (stored [in, out], as GPT-2 checkpoints do) or "out_in"."""
@@ -27,6 +37,12 @@ class Linear:
         (``ctx.may_defer``) the product may then leave the sum of its K ranges to the norm that follows. ``may_leave`` (a
         float32 ``out`` without a residual): the product may leave its K ranges in ``ctx.product_pending`` for the kernel that
         reads ``out`` next."""
+        if type(a) is RowsAhead:
+            if out is None:
+                out = ctx.empty(a.shape[0], self.n_out, out_dtype)
+            n = a.norm
+            ctx.kernels.linear_normed(a.x, n.weight, n.bias, n.eps, n.rms, self.weight, self.bias, out, activation)
+            return out
         if ctx.pending is not None or ctx.product_pending is not None:
             ctx.settle()  # the unfinished product's ranges live in the workspace that this one is about to use
         if out is None:

@@ -8,6 +8,7 @@ from typing import Dict, Optional
 import torch
 
 from .base import BuildEnv, Norm, StepContext
+from .linear import RowsAhead
 from .registry import NORMS
 from .spec import PartSpec
 
@@ -39,6 +40,13 @@ class LayerNorm(Norm):
         else:
             ctx.kernels.norm(x, self.weight, self.bias, self.eps, out, rows=rows, rms=self.rms, pending=pending)
         return out
+
+    def ahead_of(self, product, x: torch.Tensor, ctx: StepContext):
+        kernels = ctx.kernels
+        if (product.weight.dtype == torch.bfloat16 and ctx.pending is None and ctx.product_pending is None and hasattr(kernels, "takes_norm")
+                and kernels.takes_norm(x.shape[0], product.n_out, product.n_in)):
+            return RowsAhead(x, self)
+        return self(x, ctx)
 
 
 @NORMS.register("rmsnorm")
