@@ -11,8 +11,10 @@
 // chunks one behind the other, so the lane's address does the swapping.
 // Measured in graphs over distinct weights, microseconds, before (the library, the tile kernel through registers or row blocks) / here: 264 rows of 4800 x
 // 1600 14.5 / 9.9, 6400 x 1600 19.3 / 13.9, 1600 x 1600 11.8 / 7.1, 1600 x 6400 22.3 / 18.7 (15.0 where the norm behind it adds the ranges); 128 rows of 4800 x 1600 9.5 / 8.1,
-// 768 x 3072 12.8 / 8.1, 2048 x 5376 at 600 rows 31.2 / 26.1, 4096 x 16384 at 264 rows 73 / 56. Errors against 64 bits, before / here: 264 rows of 4800 x 1600
-// 2.4e-7 / 1.2e-7, 1600 x 6400 1.95e-7 / 1.4e-7, 2048 x 5376 at 700 rows 4.6e-7 / 2.2e-7. Taken back: k-tiles that begin at another place in every
+// 768 x 3072 12.8 / 8.1, 2048 x 5376 at 600 rows 31.2 / 26.1, 4096 x 16384 at 264 rows 73 / 56. Errors against 64 bits, before / here: 264 rows of 4800 x
+// 1600 2.4e-7 / 1.2e-7, 1600 x 6400 1.95e-7 / 1.4e-7, 2048 x 5376 at 400 rows 4.6e-7 / 2.2e-7; of the row blocks and ranges of K (with one chain of K / 128 here they were
+// exceeded, 1.3e-7 at 2,048 inputs: the joins are for these) 96 rows of 3072 x 2048 8.6e-8 / 8.2e-8, 256 of 1600 x 1600 8.3e-8 / 7.9e-8, 192 of 2560 x 1024 7.5e-8 / 7.4e-8, 128 of
+// 4096 x 4096 1.24e-7 / 0.92e-7, 600 of 4096 x 16384 3.5e-7 / 2.8e-7; of 386 shapes (28 weights, 65 to 1,328 rows) none is further off. Taken back: k-tiles that begin at another place in every
 // workgroup (up to 40 % slower where neighbours then no longer wait for the same line, 2 - 9 % faster at K = 16384 alone), a ring twice as deep (8 % slower), a
 // CU for every workgroup where two fit (the same).
 #include "gemm_ring.h"
@@ -30,12 +32,17 @@ __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) {
   return c.b;
 }
 
+// How many sums in turn a wave of so many 16 x 16 tiles has registers for, one of so many waves of a workgroup, and whether for a total beside them. (128 x 128 at 1,300
+// rows of 2048 x 2048 21.8 us with four sums, 17.8 with two.)
+constexpr int ring_sums(int tiles, int waves) { return tiles <= 6 ? 4 : waves == 8 ? 2 : 1; }
+constexpr bool ring_joins(int tiles) { return tiles <= 6; }
+
 // A workgroup of WGM x WGN waves computes BM x BN outputs, a wave BM / WGM x BN / WGN, in 16 x 16 x 32 products with w as the first operand: a lane then holds four
 // neighbouring outputs of a row, and eight of a pair of tiles, whose rows of w are dealt out for that. R: k-tiles of the ring.
 template <typename TO, int BM, int BN, int WGM, int WGN, int R>
 __global__ void __launch_bounds__(WGM * WGN * 64, R * (BM + BN) * 128 <= 80 * 1024 ? WGM * WGN / 2 : WGM * WGN / 4)
 gemm_ring_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, uint32_t lda, int K, int M, int N, int tiles_m, int tiles_n, int S, int act,
-                 const float* __restrict__ bias, const float* residual, TO* out, float* __restrict__ partial, long ldr, long ldo, int vec_ok) {
+                 const float* __restrict__ bias, const float* residual, TO* out, float* __restrict__ partial, long ldr, long ldo, int vec_ok, int fold) {
   constexpr int W = WGM * WGN, WM = BM / WGM, WN = BN / WGN, TI = WM / 16, TJ = WN / 16;
   static_assert(TJ % 2 == 0 && WM % 16 == 0 && BM % (8 * W) == 0 && BN % (8 * W) == 0 && R >= 3, "pairs of column tiles; whole loads a wave");
   constexpr int LA = BM / 8 / W, LW = BN / 8 / W, L = LA + LW;  // a wave's loads a k-tile, 8 lines each
@@ -93,16 +100,41 @@ gemm_ring_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, uin
     for (int i = 0; i < L; ++i) load_one(lds0 + ahead * TILE, i);
     ab += 128, wb += 128;
   }
-  // Sums in turn, joined at the end: with four no chain of roundings is longer than K / 128 products, about what the row blocks and waves that split K leave. Larger
-  // tiles run 15 - 40 % slower with as many (registers: 128 x 128 at 1,300 rows of 2048 x 2048 21.8 us with four, 17.8 with fewer); the kernels they replace have one.
-  constexpr int SUMS = TI * TJ <= 6 ? 4 : W == 8 ? 2 : 1;
-  f32x4 sums[SUMS][TI][TJ];
+  // Sums in turn, joined at the end and on the way: a chain of roundings is at most `fold` * 2 / SUMS products long (ring_fold says why).
+  constexpr int SUMS = ring_sums(TI * TJ, W);
+  constexpr bool JOINS = ring_joins(TI * TJ);
+  f32x4 sums[SUMS][TI][TJ], joined[JOINS ? TI : 1][JOINS ? TJ : 1];
 #pragma unroll
-  for (int s = 0; s < SUMS; ++s)
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {
+      if constexpr (JOINS) joined[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < SUMS; ++s) sums[s][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  auto join = [&](bool last) __attribute__((always_inline)) {  // last: what all outputs take is in sums[0]
 #pragma unroll
     for (int i = 0; i < TI; ++i)
 #pragma unroll
-      for (int j = 0; j < TJ; ++j) sums[s][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < TJ; ++j) {
+        if constexpr (SUMS == 4) sums[2][i][j] += sums[3][i][j];
+        if constexpr (SUMS >= 2) sums[0][i][j] += sums[1][i][j];
+        if constexpr (SUMS == 4) sums[0][i][j] += sums[2][i][j];
+        if constexpr (JOINS) {
+          if (last) {
+            sums[0][i][j] += joined[i][j];
+            continue;
+          }
+          joined[i][j] += sums[0][i][j];
+#pragma unroll
+          for (int s = 0; s < SUMS; ++s) sums[s][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+  };
+  auto join_in_time = [&](int kt) __attribute__((always_inline)) {  // kt: k-tiles summed up
+    if constexpr (JOINS)
+      if (((kt + (fold >> 1)) & (fold - 1)) == 0) join(false);
+  };
   auto& acc = sums[0];
   // operand (row l % 16, k-group l / 16) of a k-step of 32; column tile j = 2 p + h takes the rows 32 p + 8 (l % 16 / 4) + 4 h + l % 4 of w
   const int fr = lane & 15, kg = lane >> 4, wr = 8 * (fr >> 2) + (fr & 3);
@@ -169,6 +201,7 @@ gemm_ring_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, uin
   for (; kt + 1 + R < nk; kt += 2) {
     step(Zero(), One(), kt);
     step(One(), One(), kt + 1);
+    join_in_time(kt + 2);
   }
   bool odd = false;  // the next k-tile's operands are in the second set
   if (kt + R < nk) {
@@ -177,25 +210,20 @@ gemm_ring_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, uin
     if (kt + 1 < nk) {
       step(One(), Zero(), kt++);
       odd = false;
+      join_in_time(kt);
     }
   }
   for (; kt + 2 < nk; kt += 2) {
     step(Zero(), Zero(), kt);
     step(One(), Zero(), kt + 1);
+    join_in_time(kt + 2);
   }
   if (kt + 1 < nk) {
     step(Zero(), Zero(), kt);
     odd = true;
   }
   if (odd) last(One()); else last(Zero());
-#pragma unroll
-  for (int i = 0; i < TI; ++i)
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) {
-      if constexpr (SUMS == 4) sums[2][i][j] += sums[3][i][j];
-      if constexpr (SUMS >= 2) acc[i][j] += sums[1][i][j];
-      if constexpr (SUMS == 4) acc[i][j] += sums[2][i][j];
-    }
+  join(true);
 
   // register r of lane l: column 8 (l / 16) + 4 h + r of a pair of tiles, row l % 16
   if (S > 1) {
@@ -328,6 +356,7 @@ static RingPlan ring_choice(int M, int N, int K) {
       const int per = (nk + s - 1) / s;
       if (s > 1 && (wgs > 520 || nk / s < 2)) break;
       if (per * (s - 1) >= nk) continue;  // a range would be empty
+      if ((i == 7 && per > 96) || (i > 4 && M <= 128)) continue;  // no registers for a total: chains would be longer than before
       const double beyond = 2e-6 * M * K / s / 4.2 - 1.0;  // activations of a range that an L2 does not hold
       double cus;
       if (sh.two) {
@@ -354,6 +383,15 @@ RingPlan lev_ring_plan(int M, int N, int K) {
   return slot.plan;
 }
 
+// Every how many k-tiles (a power of two; the first time after half as many) a wave's sums join its total: so that no chain of roundings is longer than in the kernels that
+// had these products before. Those were row blocks up to 256 rows (2 to 4 products a chain), ranges of K up to 128 rows of larger weights (10 and more) and up to 320 rows of
+// small ones, and above the library's kernels and tiles of one chain. In 64 x 64 tiles a join every 8 k-tiles costs 2 - 3 %.
+static int ring_fold(int BM, int BN, int M) {
+  const int never = 1 << 20;
+  if (BM * BN > 64 * 64) return M <= 128 ? 16 : never;
+  return M <= 256 ? 8 : M <= 320 ? 16 : never;
+}
+
 template <typename TO, int BM, int BN, int WGM, int WGN, int R>
 static int launch_ring(const bf16_t* a, long lda, const bf16_t* w, const float* bias, const float* residual, long ldr, TO* out, long ldo, float* partial, int M,
                        int N, int K, int act, int S, int vec_ok, hipStream_t stream) {
@@ -365,8 +403,9 @@ static int launch_ring(const bf16_t* a, long lda, const bf16_t* w, const float* 
     if (e != hipSuccess) return lev_fail("linear: cannot reserve %d bytes of LDS: %s", lds, hipGetErrorString(e));
     configured = true;
   }
+  const int fold = ring_fold(BM, BN, M);
   gemm_ring_kernel<TO, BM, BN, WGM, WGN, R><<<tiles_m * tiles_n * S, WGM * WGN * 64, lds, stream>>>(a, w, (uint32_t)lda, K, M, N, tiles_m, tiles_n, S, act, bias, residual,
-                                                                                                   out, partial, ldr, ldo, vec_ok);
+                                                                                                   out, partial, ldr, ldo, vec_ok, fold);
   return lev_check_launch("linear_ring");
 }
 
