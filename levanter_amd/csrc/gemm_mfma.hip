@@ -921,7 +921,7 @@ static double skinny_estimate(int M, int N, int K) {
   if (caches > cost) cost = caches;
   return 2.4 + cost + (sh.row_tiles > 1 ? 0.75 * (r - 1) : 0.0);
 }
-// 0: the estimate decides; 1 / 2: the skinny / the stream kernel wherever it takes the row count. For measurements of the
+// 0: the estimate decides; 1 / 2: the skinny / the stream kernel wherever it takes the row count (up to 64 rows and where use_skinny has blocks / to 128 rows), the tile kernel above. For measurements of the
 // choice itself (a test times both candidates at widths the estimates were not fitted to); not used by the engine.
 static int g_force_kernel = 0;
 extern "C" int lev_linear_mfma_force(int kind) {
@@ -940,30 +940,39 @@ static bool use_skinny(int M, int N, int K) {
 // ring; the library's kernels are chosen by timing): below 2^22 outputs 0.9 to 1.9 times as fast; above, 12288 x 4096 at 400 / 512 rows 54.7 / 59, 55.8 / 77, 6400 x 1600
 // at 1,000 28.9 / 37, 4096 x 2048 at 2,048 34 / 45. Heads of more outputs than a layer has stay where they were: 50257 x 768 at 65 rows 23.4 / 29.8.
 // Of 17 to 64 rows it takes long sums up to 48 million weights, and from 41 rows other large ones: the kernels for them have few outputs a CU or a range too
-// many. Microseconds without the pass that adds the ranges, before / ring: 1600 x 6400 at 24 / 64 rows 11.4 / 7.1, 10.3 / 8.8; 768 x 3072 6.2 / 4.5, 9.3 / 5.0; 4096 x 4096
-// at 64 rows 12.9 / 10.5; 4096 x 16384 at 64 rows 31.9 / 32.0. Not 1600 x 1600 at 24 rows (5.1 / 4.3, less than the norm then pays for the ranges) nor gated inner sizes (2048 x 5376 at
-// 32 rows 11.0 / 7.4, but a session of Lelatar 33.1 -> 33.8 ms: a kernel of its own adds the ranges there). Sessions: GPT-2 XL, 24 requests 116.3 -> 115.0 ms, 7B, 64 requests 170.8 -> 169.7.
-static bool use_ring(int M, int N, int K) {
-  if (M > 16 && M <= 64) return !g_force_kernel && N <= K && (long)N * K < 48000000L && ((K >= 4L * N && K >= 3072) || (M > 40 && (long)N * K >= (1L << 24)));
+// many. Microseconds with what adds the ranges, before / ring. By the norm behind the product (left): 1600 x 6400 at 24 / 64 rows 13.2 / 10.5, 14.2 / 12.0; 768 x 3072 8.0 / 7.4, 11.0 / 7.9; 32 x 4096 at 24
+// 7.9 / 6.6; from 41 rows 4096 x 4096 at 64 18.1 / 13.7, 3072 x 6144 at 48 / 64 18.4 / 14.6, 19.3 / 15.6, 5120 x 5120 23.4 / 18.6, 22.6 / 19.5, 3584 x 4864 17.7 / 14.1, 18.7 / 14.7, 4096 x 11008 30.1 / 25.4, 30.9 / 26.3.
+// By a pass of its own, which is all that up to 24 rows of the smaller weights gain: 768 x 3072 at 24 rows 5.6 / 7.1, 32 x 4096 5.8 / 6.3, 1024 x 4096 at 17 8.3 / 8.9, but at 28 9.7 / 8.9, and
+// 1280 x 5120 at 17 / 24 8.9 / 8.4, 9.8 / 8.9; 768 x 3072 at 64 8.7 / 7.5. Not 1600 x 1600 at 24 rows (5.1 / 4.3, less than the norm then pays for the ranges) nor gated inner sizes (2048 x 5376 at
+// 32 rows 11.0 / 7.4, but a session of Lelatar 33.1 -> 33.8 ms: a kernel of its own adds the ranges there). A forced kernel is not this one.
+static bool use_ring(int M, int N, int K, bool left) {
+  if (g_force_kernel) return false;
+  const long weights = (long)N * K;
+  if (M > 16 && M <= 64) return N <= K && weights < 48000000L && ((K >= 4L * N && K >= 3072 && (left || M > 24 || weights > (1L << 22))) || (M > 40 && weights >= (1L << 24)));
   return M > 64 && N <= 32768 && (long)M * N < (1L << 22) && !use_skinny(M, N, K);
 }
 
 // The tile and the ranges of the ring kernel, 16 x tile + ranges; -1 where another kernel takes the product.
-extern "C" int lev_linear_mfma_ring(int M, int N, int K) {
-  if (!use_ring(M, N, K)) return -1;
-  const RingPlan plan = lev_ring_plan(M, N, K);
+extern "C" int lev_linear_mfma_ring_of(int M, int N, int K, int left) {
+  if (!use_ring(M, N, K, left != 0)) return -1;
+  const RingPlan plan = lev_ring_plan(M, N, K, left != 0);
   return 16 * plan.shape + plan.splits;
 }
 
+// the same of a product whose ranges may be left
+extern "C" int lev_linear_mfma_ring(int M, int N, int K) { return lev_linear_mfma_ring_of(M, N, K, 1); }
+
 // Into how many ranges the sum over K is split (1: the kernel finishes its outputs itself).
-extern "C" int lev_linear_mfma_ranges(int M, int N, int K) {
-  if (use_ring(M, N, K)) return lev_ring_plan(M, N, K).splits;
+extern "C" int lev_linear_mfma_ranges_of(int M, int N, int K, int left) {
+  if (use_ring(M, N, K, left != 0)) return lev_ring_plan(M, N, K, left != 0).splits;
   if (use_skinny(M, N, K)) return 1;
   return M <= 128 ? plan_stream(M, N, K).splits : plan_tiles(M, N, K).splits;
 }
 
-extern "C" long lev_linear_mfma_workspace(int M, int N, int K) {
-  const int S = lev_linear_mfma_ranges(M, N, K);
+extern "C" int lev_linear_mfma_ranges(int M, int N, int K) { return lev_linear_mfma_ranges_of(M, N, K, 1); }
+
+extern "C" long lev_linear_mfma_workspace(int M, int N, int K, int left) {
+  const int S = lev_linear_mfma_ranges_of(M, N, K, left);
   return S > 1 ? (long)S * M * N * (long)sizeof(float) : 0;
 }
 
@@ -1011,8 +1020,8 @@ static int launch_stream(const bf16_t* a, long lda, const bf16_t* w, const float
 template <typename TO>
 static int linear_mfma_typed(const bf16_t* a, long lda, const bf16_t* w, const float* bias, const float* residual, long ldr,
                              TO* out, long ldo, float* workspace, int M, int N, int K, int act, int defer, hipStream_t stream) {
-  if (use_ring(M, N, K)) {
-    const RingPlan plan = lev_ring_plan(M, N, K);
+  if (use_ring(M, N, K, defer != 0)) {
+    const RingPlan plan = lev_ring_plan(M, N, K, defer != 0);
     const int rc = lev_ring_launch(plan, a, lda, w, bias, residual, ldr, out, ldo, workspace, M, N, K, act, sizeof(TO) == 4 ? LEV_F32 : LEV_BF16, stream);
     if (rc || plan.splits == 1 || defer) return rc;
     return launch_splitk_reduce<TO>(workspace, bias, residual, ldr, out, ldo, M, N, plan.splits, act, stream);

@@ -20,6 +20,7 @@
 #include "gemm_ring.h"
 #include "ring.h"
 #include <math.h>
+#include <algorithm>
 #include <type_traits>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
@@ -339,12 +340,15 @@ static const RingShape kRing[8] = {
 };
 
 // An estimate of every tile and number of ranges: rounds of the CUs times a workgroup's k-tiles, joined (exponent 1.27: neither hides the other wholly) with the time the
-// weights take from memory, and what writing the sums costs; of ranges also the pass that adds them: a kernel of its own, or,
-// for the longest sums (K >= 4 N), which lead into a residual stream, what the norm behind the product pays for them (64 rows of 1600: 2.5 us, with 2 / 4 / 8 ranges 3.2 / 3.4 / 4.1; 264 rows
-// 2.8, 4.4 / 5.0 / 6.1). Fitted to
-// 13,000 launches (25 weights of 512 x 2048 to 16384 x 4096, 64 to 2,048 rows, up to five million outputs): off by 6 % on average, and the tile it chooses is 0.7 %
-// behind the best on average, more than 8 % in 8 of 383 shapes (2048 rows of 2048 x 5376: 57.2 us for 50.5).
-static RingPlan ring_choice(int M, int N, int K) {
+// weights take from memory, and what writing the sums costs; of ranges also the pass that adds them: a kernel of its own, or, where they are left, what
+// the norm behind the product pays for them (64 rows of 1600: 2.5 us, with 2 / 4 / 8 ranges 3.2 / 3.4 / 4.1; 264 rows 2.8, 4.4 / 5.0 / 6.1), which gives a row a thousand threads then:
+// beyond two rows a CU they take turns. One price for all sums of K >= 4 N, as if a norm always followed, put 2,020 rows of 128 x 2048 into two ranges and a pass (9.5 us; in one 8.7), 128 x 512 at
+// 1,024 into four (6.6, 4.9), and with the norm 64 x 4096 at 4,000 into four (21.6, 20.2). It stands for longer sums with a pass of their own: in one range their small tiles take up to 30 % more
+// than the estimate, about what the pass costs (700 rows of 1280 x 5120 28.7 us in one, 23.9 in three). The tiles' numbers are fitted to
+// 13,000 launches (25 weights of 512 x 2048 to 16384 x 4096, 64 to 2,048 rows, up to five million outputs), off by 6 % on average; the prices of ranges to 16,000 more (34 weights of
+// 16 x 2048 to 4096 x 16384 in no cache, 17 to 4,000 rows, each with its own pass and with the norm): the choice is 1.0 and 1.5 % behind the best on average, more than 8 % at 12 and 21 of
+// 440 shapes (512 rows of 1600 x 6400 27.5 us for 26.1, 4,000 of 512 x 2048, which the library has, 24.5 for 17.8).
+static RingPlan ring_choice(int M, int N, int K, bool left) {
   const int nk = (K + 63) >> 6;
   const double memory = 2e-6 * N * K * 0.140, outputs = 4e-6 * M * N;
   RingPlan best = {0, 1, 1e30};
@@ -367,19 +371,23 @@ static RingPlan ring_choice(int M, int N, int K) {
       }
       cus *= 1.0 + 0.110 * (beyond < 0.0 ? 0.0 : beyond > 1.0 ? 1.0 : beyond);
       double us = 1.63 + pow(pow(cus, 1.27) + pow(memory, 1.27), 1.0 / 1.27) + 0.214 * s * outputs;
-      if (K >= 4L * N) us += s > 1 ? 0.6 + s * outputs / 4.5 : 0.5;
-      else if (s > 1) us += 1.5 + (s + 1) * outputs / 4.5;
+      if (s > 1) {
+        const int more_rows = std::max(0, M - 512);
+        if (left) us += 0.1 + s * outputs / 4.5 + 1.5e-3 * more_rows;
+        else if (K >= 4L * N && (long)N * K >= (3L << 19)) us += 0.1 + s * outputs / 4.5;
+        else us += 1.5 + 0.22 * (s + 1) * outputs + 0.8e-3 * more_rows;
+      }
       if (us < best.us) best = {i, s, us};
     }
   }
   return best;
 }
 
-// The choice takes the host 3 us, a launch less: the last ones are kept, by the sizes alone.
-RingPlan lev_ring_plan(int M, int N, int K) {
-  static thread_local struct { int M, N, K; RingPlan plan; } kept[64];
-  auto& slot = kept[((unsigned)M * 31u + (unsigned)N * 7u + (unsigned)K) * 2654435769u >> 26];
-  if (slot.M != M || slot.N != N || slot.K != K) slot = {M, N, K, ring_choice(M, N, K)};
+// The choice takes the host 3 us, a launch less: the last ones are kept, by the sizes and `left` alone.
+RingPlan lev_ring_plan(int M, int N, int K, bool left) {
+  static thread_local struct { int M, N, K; bool left; RingPlan plan; } kept[64];
+  auto& slot = kept[((unsigned)M * 31u + (unsigned)N * 7u + (unsigned)K * 2u + left) * 2654435769u >> 26];
+  if (slot.M != M || slot.N != N || slot.K != K || slot.left != left) slot = {M, N, K, left, ring_choice(M, N, K, left)};
   return slot.plan;
 }
 

@@ -336,9 +336,11 @@ register_unit("core", ["errors.hip", "elementwise.hip", "layer_ops.hip", "gemm_s
 })
 register_unit("gemm_mfma", ["gemm_mfma.hip", "gemm_ring.hip", "gemm_norm.hip"], signatures={
     "lev_linear_mfma": [_P, _L, _P, _P, _P, _L, _P, _L, _P] + [_I] * 6 + [_P],
-    "lev_linear_mfma_workspace": [_I, _I, _I],
+    "lev_linear_mfma_workspace": [_I, _I, _I, _I],
     "lev_linear_mfma_ranges": [_I, _I, _I],
+    "lev_linear_mfma_ranges_of": [_I, _I, _I, _I],
     "lev_linear_mfma_ring": [_I, _I, _I],
+    "lev_linear_mfma_ring_of": [_I, _I, _I, _I],
     "lev_linear_mfma_force": [_I],
     "lev_linear_normed": [_P, _P, _P, _F, _I, _P, _P, _P, _L, _I, _I, _I, _I, _P],
     "lev_linear_normed_takes": [_I, _I, _I],

@@ -400,7 +400,7 @@ class HipKernels:
             ldr = ldo if residual is out else _rows(residual, "linear: residual")
         act = ACTIVATIONS[activation]
         if adt == torch.bfloat16 and self.use_mfma and K % 8 == 0 and lda % 8 == 0 and a.data_ptr() % 16 == 0:
-            if self.gemm_library and self.use_library(M, N, K, act):
+            if self.gemm_library and (self.use_library(M, N, K, act) or (residual is not None and self.library_adds_faster(M, N, K, act))):
                 key = (M, N, K, act, bias is None, residual is None, odt)
                 # never while a HIP graph is being recorded: what the library records besides its kernel is not ours to vouch for
                 if key not in self._library_refused and (self.library_in_graphs or not torch.cuda.is_current_stream_capturing()):
@@ -417,14 +417,14 @@ class HipKernels:
                         self._check(rc)
                     self._library_refused.add(key)  # the library has no kernel for it: ours from now on
             gemm = self._units.get("gemm_mfma") or self._unit("gemm_mfma")
-            need = self._ws_need.get((M, N, K))
-            if need is None:  # partial sums of a K range split over workgroups
-                need = self._ws_need[(M, N, K)] = gemm.lev_linear_mfma_workspace(M, N, K)
+            leave = may_leave_pending and (residual is out or (residual is None and odt == torch.float32)) and act == 0 and ldo == N
+            need = self._ws_need.get((M, N, K, leave))
+            if need is None:  # partial sums of a K range split over workgroups; into how many goes by who adds them
+                need = self._ws_need[(M, N, K, leave)] = gemm.lev_linear_mfma_workspace(M, N, K, int(leave))
             ws = self._workspace(need, a.device) if need > 0 else None
-            leave = may_leave_pending and need > 0 and (residual is out or (residual is None and odt == torch.float32)) and act == 0 and ldo == N
             self._check(gemm.lev_linear_mfma(_ptr(a), lda, _ptr(w), _ptr(bias), _ptr(residual), ldr, _ptr(out), ldo, _ptr(ws),
                                              M, N, K, act, _DT[odt], int(leave), self._s()))
-            if leave:
+            if leave and need > 0:
                 return (PendingSum if residual is out else PendingProduct)(out, ws, need // (M * N * 4), bias, ldo)
         else:
             self._check(self.lib.lev_linear_simple(_ptr(a), lda, _ptr(w), _ptr(bias), _ptr(residual), ldr, _ptr(out), ldo,
@@ -462,14 +462,16 @@ class HipKernels:
     def use_library(cls, M: int, N: int, K: int, act: int) -> bool:
         """Which products go to the vendor library: those with an epilogue it has, at the shapes where it was measured
         ahead on MI355X (with epilogues). Up to 64 rows see ``_library_reads_weights_faster``. Above, ours keep outputs below 2^22 numbers, 32,768 columns at
-        most (figures beside the ring kernel's rule), and the library takes the rest: from 256 rows all but the longest sums (K >= 4 N) below 1,024 rows, and of 65 to
+        most (figures beside the ring kernel's rule), but from 1,024 rows not 24 columns and fewer (16 x 2048 at 2,020 rows, library / ours 5.9 / 7.4 us, 24 x 3072 7.1 / 8.2, 32 x 2048
+        7.8 / 7.1), and from 2,048 rows not sums of K >= 4 N, 1,536 and more, whose output fills the chip without ranges of K (3,000 rows of 512 x 3584 23.1 / 27.7,
+        1024 x 4096 33.9 / 36.5; shorter sums 256 x 1024 at 4,000 12.0 / 7.9, fewer rows 1600 x 6400 at 1,024 45.5 / 36.5). The library takes the rest: from 256 rows all but the longest sums (K >= 4 N) below 1,024 rows, and of 65 to
         255 rows (heads of tens of thousands of outputs) those with N >= 2 K, but below 128 rows no weights of less than 32 MB and below 96 rows none of more than 256 MB."""
         if act not in cls.LIBRARY_ACTIVATIONS or M < cls.LIBRARY_MIN_ROWS:
             return False
         if M <= 64:
             return cls._library_reads_weights_faster(M, N, K)
         if N <= 32768 and M * N < (1 << 22):
-            return False
+            return M >= 1024 and (N <= 24 or (M >= 2048 and M * N >= (1 << 20) and K >= max(4 * N, 1536)))
         if M < 256:
             if N < 2 * K:
                 return False
@@ -477,6 +479,13 @@ class HipKernels:
                 return M >= 128
             return not (M < 96 and N * K > (1 << 27))
         return not (K >= 4 * N and M < 1024)
+
+    @classmethod
+    def library_adds_faster(cls, M: int, N: int, K: int, act: int) -> bool:
+        """Products with a residual that the library has beside those of ``use_library``: from three million outputs on, of 1,024 rows and more and sums of K <= 2 N
+        (library / ours with the norm behind them: 2048 x 2048 at 2,020 rows 32.2 / 35.2 us, 3072 x 1536 at 1,300 29.8 / 34.6; longer sums 2048 x 5376 at 1,800 56.7 / 53.1, fewer
+        rows 4096 x 4096 at 777 47.3 / 44.3, 1600 x 1600 at 1,024 22.5 / 20.3)."""
+        return act in cls.LIBRARY_ACTIVATIONS and M >= 1024 and N <= 32768 and 3 << 20 <= M * N < 1 << 22 and K <= 2 * N
 
     @staticmethod
     def _library_reads_weights_faster(M: int, N: int, K: int) -> bool:

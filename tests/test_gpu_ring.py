@@ -80,3 +80,30 @@ def test_the_sums_chains_of_roundings_stay_short(K, M, N, Ki, chain):
     error = float((out.double() - want).norm() / want.norm())
     sums = Ki / 32 / chain
     assert error <= 1.06 * 0.40 * 2.0 ** -24 * ((4 * chain + 1) / 2 + (sums + 1) / 2) ** 0.5, error
+
+
+@pytest.mark.parametrize("M,N,Ki", SHAPES + [(24, 32, 4096), (1024, 128, 512), (2020, 128, 2048)])
+def test_ranges_that_are_left(K, M, N, Ki, monkeypatch):
+    """A product whose ranges somebody else adds has a plan of its own; scratch memory and ranges are that plan's. The bound is the first test's."""
+    monkeypatch.setattr(K, "gemm_library", False)
+    gemm = K._unit("gemm_mfma")
+    g = torch.Generator(device=DEV).manual_seed(M + N * 3 + Ki)
+    a, w = torch.randn(M, Ki, device=DEV, generator=g).bfloat16(), torch.randn(N, Ki, device=DEV, generator=g).bfloat16()
+    res = torch.randn(M, N, device=DEV, generator=g)
+    want = a.double() @ w.double().T + res.double()
+    size = a.double().abs() @ w.double().abs().T + res.double().abs()
+    for left in (True, False):
+        out = res.clone()
+        pending = K.linear(a, w, None, out, residual=out, may_leave_pending=left)
+        ranges = gemm.lev_linear_mfma_ranges_of(M, N, Ki, int(left))
+        assert (pending is not None) == (left and ranges > 1)
+        if pending is not None:
+            assert pending.n_ranges == ranges and torch.equal(out, res)
+            K.finish(pending)
+        assert bool(((out.double() - want).abs() <= (Ki + 4) * 2.0 ** -24 * size).all()), left
+
+
+@pytest.mark.parametrize("M,N,Ki", [(17, 768, 3072), (24, 768, 3072), (24, 32, 4096), (1024, 128, 512), (777, 384, 1536), (2020, 128, 2048)])
+def test_no_ranges_whose_own_pass_costs_more_than_they_give(K, M, N, Ki):
+    """Each was 5 to 25 % slower in ranges and a second kernel than in one."""
+    assert K._unit("gemm_mfma").lev_linear_mfma_ranges_of(M, N, Ki, 0) == 1

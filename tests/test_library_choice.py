@@ -102,3 +102,12 @@ def test_the_tile_of_a_32_bit_product_is_among_the_fastest(core, M, N, K, us):
 @pytest.mark.parametrize("M,N,K,few,tiles", FEW_ROWS)
 def test_few_rows_of_a_32_bit_product_take_the_faster_kernel(core, M, N, K, few, tiles):
     assert (few if core.lev_linear_f32_choice(M, N, K) < 0 else tiles) <= 1.07 * min(few, tiles)
+
+
+def test_tall_products_that_the_library_keeps():
+    """Narrow outputs and long sums of many rows, and large residual products; beside each a neighbour where our kernel is ahead."""
+    use = HipKernels.use_library
+    assert use(2020, 16, 2048, 0) and use(1024, 24, 3072, 0) and not use(2020, 32, 2048, 0) and not use(777, 16, 2048, 0)
+    assert use(3000, 512, 3584, 0) and use(4000, 768, 3072, 0) and not use(4000, 256, 1024, 0) and not use(1024, 1600, 6400, 0)
+    adds = HipKernels.library_adds_faster
+    assert adds(2020, 2048, 2048, 0) and not use(2020, 2048, 2048, 0) and not adds(777, 4096, 4096, 0) and not adds(1800, 2048, 5376, 0)
