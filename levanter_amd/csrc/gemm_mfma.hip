@@ -946,7 +946,7 @@ static bool use_skinny(int M, int N, int K) {
 // 1280 x 5120 at 17 / 24 8.9 / 8.4, 9.8 / 8.9; 768 x 3072 at 64 8.7 / 7.5. Not 1600 x 1600 at 24 rows (5.1 / 4.3, less than the norm then pays for the ranges) nor gated inner sizes (2048 x 5376 at
 // 32 rows 11.0 / 7.4, but a session of Lelatar 33.1 -> 33.8 ms: a kernel of its own adds the ranges there). A forced kernel is not this one.
 static bool use_ring(int M, int N, int K, bool left) {
-  if (g_force_kernel) return false;
+  if (g_force_kernel || K > RING_MAX_K) return false;
   const long weights = (long)N * K;
   if (M > 16 && M <= 64) return N <= K && weights < 48000000L && ((K >= 4L * N && K >= 3072 && (left || M > 24 || weights > (1L << 22))) || (M > 40 && weights >= (1L << 24)));
   return M > 64 && N <= 32768 && (long)M * N < (1L << 22) && !use_skinny(M, N, K);

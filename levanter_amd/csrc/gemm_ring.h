@@ -2,6 +2,7 @@
 #pragma once
 #include "common.h"
 
+#define RING_MAX_K (1 << 24)  // 128 rows of w within 2^32 bytes
 struct RingPlan {
   int shape;   // place in the kernel's list of tiles
   int splits;  // ranges of K (1: none)

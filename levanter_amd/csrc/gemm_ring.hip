@@ -43,7 +43,7 @@ constexpr bool ring_joins(int tiles) { return tiles <= 6; }
 template <typename TO, int BM, int BN, int WGM, int WGN, int R>
 __global__ void __launch_bounds__(WGM * WGN * 64, R * (BM + BN) * 128 <= 80 * 1024 ? WGM * WGN / 2 : WGM * WGN / 4)
 gemm_ring_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, uint32_t lda, int K, int M, int N, int tiles_m, int tiles_n, int S, int act,
-                 const float* __restrict__ bias, const float* residual, TO* out, float* __restrict__ partial, long ldr, long ldo, int vec_ok, int fold) {
+                 const float* __restrict__ bias, const float* residual, TO* out, float* __restrict__ partial, long ldr, long ldo, int vec_ok, int fold, size_t range) {  // range: numbers of a range's sums
   constexpr int W = WGM * WGN, WM = BM / WGM, WN = BN / WGN, TI = WM / 16, TJ = WN / 16;
   static_assert(TJ % 2 == 0 && WM % 16 == 0 && BM % (8 * W) == 0 && BN % (8 * W) == 0 && R >= 3, "pairs of column tiles; whole loads a wave");
   constexpr int LA = BM / 8 / W, LW = BN / 8 / W, L = LA + LW;  // a wave's loads a k-tile, 8 lines each
@@ -60,22 +60,22 @@ gemm_ring_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, uin
   // k = 64 t - (64 - K % 64), or 64 t. This workgroup takes t0 .. t0 + nk - 1.
   const int tail = K & 63, nk_all = (K + 63) >> 6, per = (nk_all + S - 1) / S, t0 = split * per, nk = min(nk_all, t0 + per) - t0;
 
-  // Rows beyond the matrix read the last one; their products are never stored. Offsets and sizes are below 2^32 bytes (the caller checks).
+  // Rows beyond the matrix read the last one; their products are never stored. Offsets are within the tile, below 2^32 bytes (the launch sees to that).
   uint32_t off[L];
   const int lr = lane >> 3, lc = lane & 7;
 #pragma unroll
   for (int i = 0; i < LA; ++i) {
     const int r = (wave * LA + i) * 8 + lr;
-    off[i] = (uint32_t)min(m0 + r, M - 1) * lda * 2 + (uint32_t)((lc ^ ring_swap_rows(r)) * 16);
+    off[i] = (uint32_t)min(r, M - 1 - m0) * lda * 2 + (uint32_t)((lc ^ ring_swap_rows(r)) * 16);
   }
 #pragma unroll
   for (int i = 0; i < LW; ++i) {
     const int r = (wave * LW + i) * 8 + lr;
-    off[LA + i] = (uint32_t)min(n0 + r, N - 1) * (uint32_t)K * 2 + (uint32_t)((lc ^ ring_swap_columns(r)) * 16);
+    off[LA + i] = (uint32_t)min(r, N - 1 - n0) * (uint32_t)K * 2 + (uint32_t)((lc ^ ring_swap_columns(r)) * 16);
   }
   const uint32_t lds0 = lds_offset(lds_ring);
   const long first = tail ? (t0 == 0 ? 0 : (long)t0 * 64 - (64 - tail)) : (long)t0 * 64;
-  const char *ab = reinterpret_cast<const char*>(a + first), *wb = reinterpret_cast<const char*>(w + first);
+  const char *ab = reinterpret_cast<const char*>(a + (size_t)m0 * lda + first), *wb = reinterpret_cast<const char*>(w + (size_t)n0 * K + first);
   auto load_one = [&](uint32_t at, int i) {
     if (i < LA) lines_to_lds(at + (wave * LA + i) * 1024, off[i], ab);
     else lines_to_lds(at + BM * 128 + (wave * LW + i - LA) * 1024, off[i], wb);
@@ -235,7 +235,7 @@ gemm_ring_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w, uin
       for (int i = 0; i < TI; ++i) {
         const int m = m0 + wm * WM + i * 16 + fr;
         if (m >= M) continue;
-        float* o = partial + ((size_t)split * M + m) * N + n;
+        float* o = partial + split * range + (size_t)m * N + n;
         if ((vec_ok & 2) && n + 7 < N) {
           reinterpret_cast<f32x4*>(o)[0] = acc[i][2 * p];
           reinterpret_cast<f32x4*>(o)[1] = acc[i][2 * p + 1];
@@ -403,7 +403,6 @@ static int ring_fold(int BM, int BN, int M) {
 template <typename TO, int BM, int BN, int WGM, int WGN, int R>
 static int launch_ring(const bf16_t* a, long lda, const bf16_t* w, const float* bias, const float* residual, long ldr, TO* out, long ldo, float* partial, int M,
                        int N, int K, int act, int S, int vec_ok, hipStream_t stream) {
-  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   constexpr int lds = R * (BM + BN) * 128;
   static bool configured = false;  // per instantiation
   if (!configured) {
@@ -411,17 +410,23 @@ static int launch_ring(const bf16_t* a, long lda, const bf16_t* w, const float* 
     if (e != hipSuccess) return lev_fail("linear: cannot reserve %d bytes of LDS: %s", lds, hipGetErrorString(e));
     configured = true;
   }
-  const int fold = ring_fold(BM, BN, M);
-  gemm_ring_kernel<TO, BM, BN, WGM, WGN, R><<<tiles_m * tiles_n * S, WGM * WGN * 64, lds, stream>>>(a, w, (uint32_t)lda, K, M, N, tiles_m, tiles_n, S, act, bias, residual,
-                                                                                                   out, partial, ldr, ldo, vec_ok, fold);
+  const int fold = ring_fold(BM, BN, M), tiles_n = (N + BN - 1) / BN;
+  // as many rows a launch as a tile's offsets reach (rows of a tile are 70 MB and more apart, if that is fewer than a tile has: a column block of a very wide matrix)
+  const long reach = ((1L << 32) - 256) / (2 * lda) + 1;
+  const int rows = reach >= std::min(BM, M) ? M : (int)reach;
+  for (int m = 0; m < M; m += rows) {
+    const int here = std::min(rows, M - m), tiles_m = (here + BM - 1) / BM;
+    gemm_ring_kernel<TO, BM, BN, WGM, WGN, R><<<tiles_m * tiles_n * S, WGM * WGN * 64, lds, stream>>>(
+        a + m * lda, w, (uint32_t)(here > 1 ? lda : 0), K, here, N, tiles_m, tiles_n, S, act, bias, residual ? residual + m * ldr : nullptr, out + m * ldo,
+        partial ? partial + (size_t)m * N : nullptr, ldr, ldo, vec_ok, fold, (size_t)M * N);
+  }
   return lev_check_launch("linear_ring");
 }
 
 template <typename TO>
 static int launch_ring_typed(const RingPlan& plan, const bf16_t* a, long lda, const bf16_t* w, const float* bias, const float* residual, long ldr, TO* out, long ldo,
                              float* partial, int M, int N, int K, int act, hipStream_t stream) {
-  if ((size_t)M * lda >= (1ull << 31) || (size_t)N * K >= (1ull << 31))
-    return lev_fail("linear: operands of more than 2^31 elements are not supported (M=%d lda=%ld N=%d K=%d)", M, lda, N, K);
+  if (K > RING_MAX_K) return lev_fail("linear: a sum of %d products is too long for the ring kernel", K);
   const int S = plan.splits;
   if (S > 1 && !partial) return lev_fail("linear: M=%d N=%d K=%d needs a workspace of lev_linear_mfma_workspace bytes", M, N, K);
   const int vec_out = ldo % (sizeof(TO) == 4 ? 4 : 8) == 0 && ((uintptr_t)out & 15) == 0 && (!residual || (ldr % 4 == 0 && ((uintptr_t)residual & 15) == 0));

@@ -107,3 +107,26 @@ def test_ranges_that_are_left(K, M, N, Ki, monkeypatch):
 def test_no_ranges_whose_own_pass_costs_more_than_they_give(K, M, N, Ki):
     """Each was 5 to 25 % slower in ranges and a second kernel than in one."""
     assert K._unit("gemm_mfma").lev_linear_mfma_ranges_of(M, N, Ki, 0) == 1
+
+
+# row strides at which a matrix takes more than 4 GiB, and at which a tile's rows do; weights of more than 2^31 numbers
+@pytest.mark.parametrize("M,N,Ki,stride,left", [(64, 1600, 6400, 40_000_000, True), (100, 2304, 1024, 36_000_000, False), (17, 768, 3072, 280_000_000, True), (33, 1600, 6400, 150_000_000, False),
+                                                (100, 32768, 65544, 65544, False)])
+def test_operands_of_more_than_4_gib(K, M, N, Ki, stride, left, monkeypatch):
+    monkeypatch.setattr(K, "gemm_library", False)
+    assert K._unit("gemm_mfma").lev_linear_mfma_ring_of(M, N, Ki, int(left)) != -1
+    a = torch.empty((M - 1) * stride + Ki, dtype=torch.bfloat16, device=DEV).as_strided((M, Ki), (stride, 1))
+    a.copy_(torch.randn(M, Ki, device=DEV))
+    w = torch.empty(N, Ki, dtype=torch.bfloat16, device=DEV)
+    for n in range(0, N, 4096):
+        w[n:n + 4096] = torch.randn(min(4096, N - n), Ki, device=DEV)
+    res = torch.randn(M, N, device=DEV)
+    out = res.clone()
+    pending = K.linear(a, w, None, out, residual=out, may_leave_pending=left)
+    if pending is not None:
+        K.finish(pending)
+    x = a.double()
+    for n in range(0, N, 4096):
+        y, r = w[n:n + 4096].double(), res[:, n:n + 4096].double()
+        err = (out[:, n:n + 4096].double() - x @ y.T - r).abs()
+        assert bool((err <= (Ki + 4) * 2.0 ** -24 * (x.abs() @ y.T.abs() + r.abs())).all()), n
