@@ -38,11 +38,14 @@ class Linear:
         float32 ``out`` without a residual): the product may leave its K ranges in ``ctx.product_pending`` for the kernel that
         reads ``out`` next."""
         if type(a) is RowsAhead:
-            if out is None:
-                out = ctx.empty(a.shape[0], self.n_out, out_dtype)
             n = a.norm
-            ctx.kernels.linear_normed(a.x, n.weight, n.bias, n.eps, n.rms, self.weight, self.bias, out, activation)
-            return out
+            if (residual is None and not may_leave and (ctx.dtype if out is None and out_dtype is None else out_dtype or out.dtype) == torch.bfloat16
+                    and ctx.kernels.takes_norm(a.shape[0], self.n_out, self.n_in)):
+                if out is None:
+                    out = ctx.empty(a.shape[0], self.n_out, out_dtype)
+                ctx.kernels.linear_normed(a.x, n.weight, n.bias, n.eps, n.rms, self.weight, self.bias, out, activation)
+                return out
+            a = n(a.x, ctx)  # a product that the kernel is not for
         if ctx.pending is not None or ctx.product_pending is not None:
             ctx.settle()  # the unfinished product's ranges live in the workspace that this one is about to use
         if out is None:
