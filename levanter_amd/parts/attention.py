@@ -63,7 +63,7 @@ class CausalSelfAttention(Mixer):
 
     @property
     def first_product(self):
-        return self.qkv
+        return self.qkv if self.keeps(CausalSelfAttention, "forward") else None
 
     def cache_requirement(self):
         return PagedKv(self.n_kv_heads, self.head_dim, self.window)

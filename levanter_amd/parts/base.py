@@ -146,6 +146,10 @@ class Part:
         self.spec = spec
         self.env = env
 
+    def keeps(self, cls, *methods: str) -> bool:
+        """Whether these methods are ``cls``'s own, neither a subclass's nor put on this object."""
+        return all(getattr(getattr(self, m), "__func__", None) is getattr(cls, m) for m in methods)
+
 
 class Norm(Part):
     """``__call__(x_f32 [T, dim], ctx, rows=None) -> h [T or len(rows), dim]`` in the compute dtype.
@@ -186,7 +190,7 @@ class Mixer(Part):
     ``[T, dim]``) to the residual ``x`` (float32 ``[T, dim]``) in place; reads (and, if
     ``writes_cache``, first writes) ``unit``."""
 
-    first_product = None  # the ``Linear`` through which alone ``forward`` reads ``h`` (besides its shape), if there is one
+    first_product = None  # the ``Linear`` through which alone ``forward`` reads ``h`` (besides its shape), if there is one; a part that inherits another ``forward`` has none
 
     def cache_requirement(self):
         return None

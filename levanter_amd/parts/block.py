@@ -7,7 +7,7 @@ from typing import Dict
 
 import torch
 
-from .base import Block, CacheUnitView, Part, StepContext
+from .base import Block, CacheUnitView, Norm, Part, StepContext
 from .linear import Linear
 from .registry import BLOCKS
 
@@ -41,8 +41,8 @@ class PreNormBlock(Block):
 
     @staticmethod
     def _normed(norm, part, x: torch.Tensor, ctx: StepContext):
-        product = part.first_product
-        return norm(x, ctx) if product is None else norm.ahead_of(product, x, ctx)
+        product = getattr(part, "first_product", None)
+        return norm.ahead_of(product, x, ctx) if product is not None and isinstance(norm, Norm) else norm(x, ctx)
 
 
 @BLOCKS.register("parallel")

@@ -31,7 +31,7 @@ class DenseMlp(FeedForward):
 
     @property
     def first_product(self):
-        return self.up
+        return self.up if self.keeps(DenseMlp, "forward") else None
 
     def forward(self, h: torch.Tensor, x: torch.Tensor, ctx: StepContext) -> None:
         m = self.up(h, ctx, activation=self.activation)
@@ -84,7 +84,7 @@ class GatedMlp(FeedForward):
 
     @property
     def first_product(self):
-        return self.up
+        return self.up if self.keeps(GatedMlp, "forward", "_inner") else None
 
     def _inner(self, h: torch.Tensor, ctx: StepContext) -> torch.Tensor:
         z = self.up(h, ctx)

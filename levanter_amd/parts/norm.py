@@ -8,7 +8,7 @@ from typing import Dict, Optional
 import torch
 
 from .base import BuildEnv, Norm, StepContext
-from .linear import RowsAhead
+from .linear import Linear, RowsAhead
 from .registry import NORMS
 from .spec import PartSpec
 
@@ -43,8 +43,9 @@ class LayerNorm(Norm):
 
     def ahead_of(self, product, x: torch.Tensor, ctx: StepContext):
         kernels = ctx.kernels
-        if (product.weight.dtype == torch.bfloat16 and ctx.pending is None and ctx.product_pending is None and hasattr(kernels, "takes_norm")
-                and kernels.takes_norm(x.shape[0], product.n_out, product.n_in)):
+        if (type(product) is Linear and product.weight.dtype == torch.bfloat16 and type(self).__call__ is LayerNorm.__call__
+                and ctx.pending is None and ctx.product_pending is None and hasattr(kernels, "takes_norm")
+                and x.is_contiguous() and x.data_ptr() % 16 == 0 and kernels.takes_norm(x.shape[0], product.n_out, product.n_in)):
             return RowsAhead(x, self)
         return self(x, ctx)
 

@@ -1,10 +1,11 @@
-"""What becomes of rows that a product normalises itself in a product that does more than read them: on the CPU, with plain
+"""Which parts are given rows that their first product normalises itself, and what becomes of such rows in a product that does more than read them: on the CPU, with plain
 kernels that say they take every norm along."""
 import torch
 
 from emulated_kernels import EmulatedKernels
 from levanter_amd.kernels.library import KernelError
 from levanter_amd.parts.base import BuildEnv, StepContext
+from levanter_amd.parts.block import PreNormBlock
 from levanter_amd.parts.feed_forward import DenseMlp, GatedMlp
 from levanter_amd.parts.linear import Linear, RowsAhead
 from levanter_amd.parts.norm import LayerNorm
@@ -40,6 +41,65 @@ def _parts(norm=LayerNorm, mlp=DenseMlp):
     tensors = {"down.weight": torch.randn(D, F, generator=g), **{k: torch.randn(F, D, generator=g) for k in names}}
     m = mlp(PartSpec("mlp", dict(dim=D, inner_dim=F, activation="silu")), tensors, env)
     return n, m, ctx, env.kernels, torch.randn(T, D, generator=g)
+
+
+def _run(norm, mlp, x, ctx):
+    x = x.clone()
+    mlp.forward(PreNormBlock._normed(norm, mlp, x, ctx), x, ctx)
+    return x
+
+
+def _check(norm, mlp, ctx, kernels, x, taken):
+    want = x.clone()
+    mlp.forward(norm(want, ctx), want, ctx)
+    assert torch.equal(_run(norm, mlp, x, ctx), want) and kernels.taken == taken
+
+
+def test_parts_as_they_are():
+    for mlp in (DenseMlp, GatedMlp):
+        _check(*(p := _parts(mlp=mlp))[:4], p[4], taken=1)
+
+
+def test_a_part_that_reads_its_rows_elsewhere_gets_rows():
+    class Reads(DenseMlp):
+        def forward(self, h, x, ctx):
+            x += h.float() * 0.5
+            super().forward(h, x, ctx)
+
+    class Inner(GatedMlp):
+        def _inner(self, h, ctx):
+            return super()._inner(h * 2, ctx)
+
+    for mlp in (Reads, Inner):
+        _check(*(p := _parts(mlp=mlp))[:4], p[4], taken=0)
+    n, m, ctx, k, x = _parts()
+    own, seen = m.forward, []
+    m.forward = lambda h, x, ctx: (seen.append(h), own(h, x, ctx))
+    _check(n, m, ctx, k, x, taken=0)
+    assert all(isinstance(h, torch.Tensor) for h in seen)
+
+
+def test_a_norm_of_its_own_is_not_passed_by():
+    class Scaled(LayerNorm):
+        def __call__(self, x, ctx, rows=None):
+            return super().__call__(x, ctx, rows) * 2
+
+    _check(*(p := _parts(norm=Scaled))[:4], p[4], taken=0)
+
+
+def test_another_product_in_the_linears_place():
+    n, m, ctx, k, x = _parts()
+    up = m.up
+    m.up = lambda h, ctx, **args: up(h, ctx, **args) + 1
+    _check(n, m, ctx, k, x, taken=0)
+
+
+def test_rows_that_the_kernel_cannot_read():
+    n, m, ctx, k, x = _parts()
+    storage = torch.empty(T * D + 1)
+    odd = storage[1:].view(T, D).copy_(x)
+    assert isinstance(PreNormBlock._normed(n, m, odd, ctx), torch.Tensor)
+    assert isinstance(PreNormBlock._normed(n, m, torch.empty(D, T).t().copy_(x), ctx), torch.Tensor)
 
 
 def test_a_product_that_does_more_than_the_kernel_makes_the_rows_first():
