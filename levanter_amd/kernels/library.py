@@ -170,8 +170,8 @@ class HipKernels:
         self._units = {}
         self._held_stream = None  # see hold_stream
         self._library_ws_bytes = None
-        self._takes_norm = {}  # (M, N, K) -> bool
-        self._ws, self._ws_outgrown, self._ws_need = {}, [], {}  # GEMM scratch memory per device, see _workspace
+        self._ws, self._ws_outgrown = {}, []  # GEMM scratch memory per device, see _workspace
+        self._ws_need = {}  # what the products' rules say of sizes (how much scratch memory, whether a norm comes along): empty it when a kernel is forced
         self._ws_last = None
         L.lev_attention_prefill_tile_rows.restype = c_int
         self.prefill_tile_rows = int(L.lev_attention_prefill_tile_rows())
@@ -433,10 +433,10 @@ class HipKernels:
 
     def takes_norm(self, M: int, N: int, K: int) -> bool:
         """Whether ``linear_normed`` has a kernel for these sizes (in bfloat16) that is ahead of the norm and the product apart."""
-        takes = self._takes_norm.get((M, N, K))
+        takes = self._ws_need.get((M, N, K))
         if takes is None:
             gemm = self._units.get("gemm_mfma") or self._unit("gemm_mfma")
-            takes = self._takes_norm[(M, N, K)] = gemm.lev_linear_normed_takes(M, N, K) == 1
+            takes = self._ws_need[(M, N, K)] = gemm.lev_linear_normed_takes(M, N, K) == 1
         return takes and self.use_mfma
 
     def linear_normed(self, x, norm_weight, norm_bias, eps: float, rms: bool, w, bias, out, activation: str = "none") -> None:

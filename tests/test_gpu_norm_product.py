@@ -58,3 +58,26 @@ def test_sizes_that_keep_the_two_kernels():
     x, w = torch.zeros(9, 768, device=DEV), torch.zeros(3072, 768, dtype=torch.bfloat16, device=DEV)
     with pytest.raises(KernelError, match="no kernel"):
         kern.linear_normed(x, torch.ones(768, device=DEV), None, 1e-5, True, w, None, torch.empty(9, 3072, dtype=torch.bfloat16, device=DEV))
+
+
+def test_a_forced_kernel_is_asked_anew():
+    """The answer for a size goes by the kernel that takes its product, as the scratch memory does, and is forgotten with it."""
+    from levanter_amd.kernels import KernelError, get_kernels
+
+    kern = get_kernels()
+    gemm = kern._unit("gemm_mfma")
+    x, w, out = torch.ones(2, 768, device=DEV), torch.ones(3072, 768, dtype=torch.bfloat16, device=DEV), torch.empty(2, 3072, dtype=torch.bfloat16, device=DEV)
+    args = (x, torch.ones(768, device=DEV), None, 1e-5, True, w, None, out)
+    assert kern.takes_norm(2, 3072, 768)
+    try:
+        kern._check(gemm.lev_linear_mfma_force(2))
+        kern._ws_need.clear()
+        assert not kern.takes_norm(2, 3072, 768)
+        with pytest.raises(KernelError, match="no kernel"):
+            kern.linear_normed(*args)
+    finally:
+        kern._check(gemm.lev_linear_mfma_force(0))
+        kern._ws_need.clear()
+    assert kern.takes_norm(2, 3072, 768)
+    kern.linear_normed(*args)
+    assert bool((out.float() == 768).all())
