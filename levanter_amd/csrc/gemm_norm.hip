@@ -166,8 +166,10 @@ gemm_norm_kernel(const bf16_t* __restrict__ w, const float* __restrict__ x, int 
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       // LDS executes a wave's instructions in order: the area is used again and again without a barrier
+      lds_wave_order();
       my_stage[st_slot] = wv[p][j][0] & mk;
       my_stage[STAGE_SLOTS + st_slot] = wv[p][j][1] & mk;
+      lds_wave_order();
       const u32x4 w_lo = my_stage[ld_slot], w_hi = my_stage[ld_slot + 4];
       acc[0][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a_lo), as_bf16x8(w_lo), acc[0][j], 0, 0, 0);
       acc[1 % SUMS][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a_hi), as_bf16x8(w_hi), acc[1 % SUMS][j], 0, 0, 0);

@@ -8,7 +8,8 @@ __device__ __forceinline__ int ring_swap_rows(int row) { return (row >> 1) & 7; 
 __device__ __forceinline__ int ring_swap_columns(int row) { return ((row >> 1) & 1) | ((row >> 2) & 6); }
 
 // 16 bytes a lane from base + off straight into LDS, at lds + 16 * lane. In assembly because the compiler waits for all such loads before any read of LDS; no
-// register is written, and whoever reads the LDS waits for vmcnt (ring_wait) and a barrier first.
+// register is written, and whoever reads the LDS waits for vmcnt (ring_wait) and a barrier first. m0 is reserved to the compiler, which keeps nothing in it from one
+// instruction to the next and takes no clobber of it; the kernels here have no other instruction that reads it.
 __device__ __forceinline__ void lines_to_lds(uint32_t lds, uint32_t off, const void* base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
 }
