@@ -4,6 +4,7 @@
 #include <stdint.h>
 #include <stdio.h>
 #include <stdarg.h>
+#include <atomic>
 
 enum LevDtype { LEV_F32 = 0, LEV_BF16 = 1 };
 enum LevAct { LEV_ACT_NONE = 0, LEV_ACT_GELU_TANH = 1, LEV_ACT_GELU_ERF = 2, LEV_ACT_RELU = 3, LEV_ACT_SILU = 4,
@@ -19,6 +20,18 @@ int lev_check_launch(const char* what);
   do {                                    \
     if (!(cond)) return lev_fail(__VA_ARGS__); \
   } while (0)
+
+// More LDS a workgroup than a kernel has unasked: once on each device (a bit of `done` each), whichever thread comes first.
+inline int lev_reserve_lds(const void* kernel, int bytes, std::atomic<unsigned long long>& done) {
+  int device = 0;
+  hipError_t e = hipGetDevice(&device);
+  const unsigned long long bit = 1ull << (device & 63);
+  if (e == hipSuccess && (done.load(std::memory_order_acquire) & bit)) return 0;
+  if (e == hipSuccess) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  LEV_REQUIRE(e == hipSuccess, "%d bytes of LDS a workgroup: %s", bytes, hipGetErrorString(e));
+  done.fetch_or(bit, std::memory_order_release);
+  return 0;
+}
 
 // ---- bf16 as raw 16 bits -----------------------------------------------------------------
 typedef uint16_t bf16_t;

@@ -311,12 +311,8 @@ static int launch_tile(const bf16_t* a, long lda, const bf16_t* w, const float* 
   const size_t lds_ops = (size_t)2 * (BM + BN) * LDS_STRIDE * sizeof(bf16_t);
   const size_t lds_out = (size_t)4 * 32 * (BN / 2 + 4) * sizeof(float);
   const size_t lds = lds_ops > lds_out ? lds_ops : lds_out;
-  static bool configured = false;  // per instantiation
-  if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_tile_kernel<TO, BM, BN>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return lev_fail("linear: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
-    configured = true;
-  }
+  static std::atomic<unsigned long long> reserved{0};  // per instantiation
+  if (int rc = lev_reserve_lds((const void*)gemm_tile_kernel<TO, BM, BN>, (int)lds, reserved)) return rc;
   if (S > 1 && !workspace) return lev_fail("linear: M=%d N=%d K=%d needs a workspace of lev_linear_mfma_workspace bytes", M, N, K);
   // rows of 4 outputs are stored (and bias / residual read) as vectors when everything is aligned for it
   const int vec_out = (ldo % 4 == 0) && (((uintptr_t)out & 15) == 0) && (!residual || (ldr % 4 == 0 && ((uintptr_t)residual & 15) == 0)) &&

@@ -404,12 +404,8 @@ template <typename TO, int BM, int BN, int WGM, int WGN, int R>
 static int launch_ring(const bf16_t* a, long lda, const bf16_t* w, const float* bias, const float* residual, long ldr, TO* out, long ldo, float* partial, int M,
                        int N, int K, int act, int S, int vec_ok, hipStream_t stream) {
   constexpr int lds = R * (BM + BN) * 128;
-  static bool configured = false;  // per instantiation
-  if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_ring_kernel<TO, BM, BN, WGM, WGN, R>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (e != hipSuccess) return lev_fail("linear: cannot reserve %d bytes of LDS: %s", lds, hipGetErrorString(e));
-    configured = true;
-  }
+  static std::atomic<unsigned long long> reserved{0};  // per instantiation
+  if (int rc = lev_reserve_lds((const void*)gemm_ring_kernel<TO, BM, BN, WGM, WGN, R>, lds, reserved)) return rc;
   const int fold = ring_fold(BM, BN, M), tiles_n = (N + BN - 1) / BN;
   // as many rows a launch as a tile's offsets reach (rows of a tile are 70 MB and more apart, if that is fewer than a tile has: a column block of a very wide matrix)
   const long reach = ((1L << 32) - 256) / (2 * lda) + 1;
