@@ -231,7 +231,9 @@ sc_inner_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
 // ---- along the runs -------------------------------------------------------------------------------------------------------------
 // One workgroup of four waves per (run, head, 16 CT value columns); wave w has the tokens 16 w .. of the block as rows of the result and a quarter
 // of the state's key channels, in accumulator registers. SSD takes up to 64 columns at once where there are many runs: what a block stages in LDS (keys, queries, weights)
-// is the same for all of them (64 heads of 128 / 64, microseconds with 16 / 64 columns: 32 runs of 40 to 150 tokens 205 / 158, but three of 300 to 999, whose chain is the bound, 62 / 100). DELTA stays at 16: its products with two 32-bit sides are four times as long.
+// is the same for all of them (64 heads of 128 / 64, microseconds with 16 / 64 columns: 32 runs of 40 to 150 tokens 205 / 158, but three of 300 to 999, whose chain is the bound, 62 / 100).
+// Runs of several tokens begin first: behind 31 single tokens, as a step has them, one of 1,000 would begin last and its chain be the end of the step (with all that stands around the kernel, 16 columns / 64 / 64 and
+// long runs first: 246 / 254 / 188; of 3,000 406 / 484 / 365; 32 of 40 to 150, in a scan that reads every slot once, 386 / 306 / 282). DELTA stays at 16: its products with two 32-bit sides are four times as long.
 template <int DKM, int RULE, bool VEC, int CT>
 __global__ void __launch_bounds__(256)
 sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, const float* __restrict__ P_in, const float* __restrict__ T_in,
@@ -257,7 +259,7 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
 #pragma unroll
   for (int c = 0; c < CT; ++c) live[c] = j + 16 * c < dv;
   int t0, t_end, slot;
-  if (!sr_find_run<256>(blockIdx.y, token_slots, s.Tn, tmp, t0, t_end, slot)) return;
+  if (!sr_find_run<256, true>(blockIdx.y, token_slots, s.Tn, tmp, t0, t_end, slot)) return;
   const bf16_t* uk = u + s.k_off + (size_t)g * dk;
   const bf16_t* uq = u + s.q_off + (size_t)g * dk;
   const bf16_t* uv = u + s.v_off + (size_t)h * dv;

@@ -22,32 +22,47 @@ struct SrShape {
 
 // ---- the run-th run of a step: its first token, the token behind its last, its slot; false: there are fewer ------------------
 // A token starts a run if it has a slot and the token before it has another. Each thread counts the starts of its stretch of
-// tokens; the thread whose stretch holds the run-th one finds it. `tmp`: NT + 2 ints of LDS.
-template <int NT>
+// tokens; the thread whose stretch holds the run-th one finds it. `tmp`: NT + 2 ints of LDS. LONG_FIRST: runs of several tokens have the first numbers (at most 65,535 runs).
+template <int NT, bool LONG_FIRST = false>
 __device__ __forceinline__ bool sr_find_run(int run, const int* __restrict__ token_slots, int Tn, int* tmp, int& t0, int& t_end, int& slot) {
   const int tid = threadIdx.x;
   const int per = (Tn + NT - 1) / NT, lo = min(Tn, tid * per), hi = min(Tn, lo + per);
-  int mine = 0;
-  for (int t = lo; t < hi; ++t) mine += (token_slots[t] >= 0 && (t == 0 || token_slots[t - 1] != token_slots[t])) ? 1 : 0;
+  // visit(t, what a start there counts): 1; behind the long runs those of one token 1 << 16
+  auto starts = [&](auto visit) {
+    int prev = lo > 0 ? token_slots[lo - 1] : -1, here = lo < hi ? token_slots[lo] : -1;
+    for (int t = lo; t < hi; ++t) {
+      const int next = token_slots[min(t + 1, Tn - 1)];
+      if (here >= 0 && here != prev) visit(t, LONG_FIRST && (t + 1 >= Tn || next != here) ? 1u << 16 : 1u);
+      prev = here, here = next;
+    }
+  };
+  unsigned mine = 0;
+  starts([&](int, unsigned counts) { mine += counts; });
   if (tid == 0) tmp[NT] = -1, tmp[NT + 1] = Tn;
   // the starts in the stretches before this thread's: across the lanes of its wave, then the waves before it
-  int upto = mine;
+  unsigned upto = mine;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
-    const int up = __shfl_up(upto, d, 64);
+    const unsigned up = __shfl_up(upto, d, 64);
     if ((tid & 63) >= d) upto += up;
   }
-  if ((tid & 63) == 63) tmp[tid >> 6] = upto;
+  if ((tid & 63) == 63) tmp[tid >> 6] = (int)upto;
   __syncthreads();
-  int before = upto - mine;
-  for (int i = 0; i < (tid >> 6); ++i) before += tmp[i];
-  if (run >= before && run < before + mine) {
-    int seen = before;
-    for (int t = lo; t < hi; ++t)
-      if (token_slots[t] >= 0 && (t == 0 || token_slots[t - 1] != token_slots[t])) {
-        if (seen == run) tmp[NT] = t;
-        ++seen;
-      }
+  unsigned before = upto - mine;
+  for (int i = 0; i < (tid >> 6); ++i) before += (unsigned)tmp[i];
+  unsigned unit = 1u, shift = 0u, mask = ~0u;  // the kind of start that is looked for, and its count
+  if (LONG_FIRST) {
+    unsigned n_long = 0;
+#pragma unroll
+    for (int i = 0; i < NT / 64; ++i) n_long += (unsigned)tmp[i] & 0xffffu;
+    mask = 0xffffu;
+    if (run >= (int)n_long) run -= (int)n_long, unit = 1u << 16, shift = 16u;
+  }
+  int seen = (int)(before >> shift & mask);
+  if (run >= seen && run < seen + (int)(mine >> shift & mask)) {
+    starts([&](int t, unsigned counts) {
+      if (counts == unit && seen++ == run) tmp[NT] = t;
+    });
   }
   __syncthreads();
   t0 = tmp[NT];
