@@ -965,7 +965,8 @@ extern "C" int lev_linear_mfma_ranges_of(int M, int N, int K, int left) {
   return M <= 128 ? plan_stream(M, N, K).splits : plan_tiles(M, N, K).splits;
 }
 
-extern "C" int lev_linear_mfma_ranges(int M, int N, int K) { return lev_linear_mfma_ranges_of(M, N, K, 1); }
+// the same of a product that adds them itself
+extern "C" int lev_linear_mfma_ranges(int M, int N, int K) { return lev_linear_mfma_ranges_of(M, N, K, 0); }
 
 extern "C" long lev_linear_mfma_workspace(int M, int N, int K, int left) {
   const int S = lev_linear_mfma_ranges_of(M, N, K, left);

@@ -12,9 +12,10 @@ def K():
     return get_kernels()
 
 
-# 512: the shortest sum that goes this way; one workgroup has up to 1, 2 and 7 units
+# 384: the shortest sum that goes this way (six k-tiles a unit, a workgroup's only unit as long as the ring needs); one workgroup has up to 1, 2 and 7 units
 @pytest.mark.parametrize("counts,Fo,Kd", [([1, 31, 0, 32, 33, 64, 65, 127, 128, 129, 260], 1, 512), ([1, 31, 0, 32, 33, 64, 65, 127, 128, 129, 260], 63, 640),
-                                          ([200, 0, 5], 129, 2048), ([97, 300, 0, 33] * 8, 776, 512), ([129] * 300, 200, 512), ([40] * 90, 1000, 768)])
+                                          ([200, 0, 5], 129, 2048), ([97, 300, 0, 33] * 8, 776, 512), ([129] * 300, 200, 512), ([40] * 90, 1000, 768),
+                                          ([5], 40, 384), ([1, 31, 0, 32, 33, 64, 65, 127, 128, 129, 260], 63, 384), ([129] * 300, 200, 384)])
 def test_against_float64(K, counts, Fo, Kd):
     from test_gpu_experts_many import _check
 

@@ -86,16 +86,16 @@ def test_norm_constant_row_gives_bias(K):
     torch.testing.assert_close(got.cpu(), b.expand(2, 96), rtol=0, atol=1e-6)
 
 
-# M <= 24: weight-streaming kernel (its three launch shapes by N: 16, 4 and 4 waves; K with and without a partial
-# pair of k-steps; rows 8..15; two row tiles above 16 rows); 25..128: split-K kernel; above: tile kernels (the last shape takes 256 x 256 tiles
-# and a partial k-tile)
+# In bfloat16, M <= 25: the kernel of few rows (its launch shapes by N; K with and without a partial pair of k-steps; rows 8..15; two row tiles above
+# 16 rows), which has 65 and 130 rows in row blocks; 64 rows of K = 4096 and 256 to 320 rows of long sums: the ring kernel in ranges of K, 300 of 1600 x 520 and of 72 x 12288 and 257
+# of 64 x 6282 in one; of more than 2^22 outputs: the tile kernel, or the library where that is ahead
 LINEAR_SHAPES = [(1, 64, 192), (2, 96, 320), (7, 320, 96), (16, 64, 1000), (9, 4104, 200), (12, 1096, 8200), (5, 520, 16400),
                  (17, 96, 50257 // 16), (24, 200, 8200), (21, 1096, 16400), (25, 96, 300), (64, 4096, 528), (65, 256, 257), (130, 96, 300), (300, 1600, 520),
                  (257, 64, 50257 // 8), (520, 72, 33000),
                  (13, 264, 50257), (16, 1096, 16400), (2, 72, 16384),  # 1,024 column units and more: two units per workgroup
                  (12, 520, 12288), (15, 264, 11531),  # 720 to 1,023 units at 12 to 16 rows: three units per workgroup
                  (300, 72, 12288), (300, 1032, 22002), (2048, 64, 6144), (256, 6144, 96),
-                 (200, 8200, 300), (320, 6400, 1600), (300, 1600, 520)]  # few tiles and a long K: K is split into ranges  # the last four take the 128x128, 256x256, 256x128 and 256x192 tiles
+                 (200, 8200, 300), (320, 6400, 1600), (300, 1600, 520)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
@@ -130,7 +130,7 @@ def test_linear_plain_and_epilogues(K, dtype, M, K_, N):
 
 
 def test_linear_bf16_random_shapes_strides_and_epilogues(K):
-    """Sixty random shapes through the bfloat16 kernels (skinny, stream, tiles of every shape, K split into ranges),
+    """Sixty random shapes of up to two million outputs through the bfloat16 kernels (few rows, row blocks, ring; one range of K and several),
     with row strides above K, every epilogue and both output types, against the float64 statement."""
     import random
 

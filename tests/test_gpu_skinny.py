@@ -45,18 +45,19 @@ def test_linear_skinny_against_float64(K, N, Ki, monkeypatch):
         K._ws_need.clear()
 
 
-@pytest.mark.parametrize("N", [1, 24, 511, 768, 1600, 2304, 4096])
+@pytest.mark.parametrize("N", [1, 24, 511, 768, 1024, 1025, 1600, 2048, 2049, 2304, 4096])
 @pytest.mark.parametrize("Ki", [8, 72, 1600, 2040, 2048])
 def test_linear_in_row_blocks_against_float64(K, N, Ki, monkeypatch):
-    """65 to 256 rows of small weights, in blocks of 32 or 64 rows; the bound is the one above."""
+    """65 to 256 rows of small weights, in blocks of 32 rows and columns where they make one round of the CUs, in the ring kernel beyond; the bound is the one above."""
     gemm = K._unit("gemm_mfma")
     monkeypatch.setattr(K, "gemm_library", False)
     g = torch.Generator(device=DEV).manual_seed(N * 31 + Ki)
     w = torch.randn(N, Ki, device=DEV, generator=g).bfloat16()
     bias = torch.randn(N, device=DEV, generator=g)
     for M in (65, 95, 128, 130, 193, 256):
-        taken = -(-M // 64) * (-(-N // 512) * 8) <= 256
-        assert not taken or gemm.lev_linear_mfma_ranges(M, N, Ki) == 1
+        taken = -(-M // 32) * (-(-N // 256) * 8) <= 256
+        assert (gemm.lev_linear_mfma_ring_of(M, N, Ki, 0) == -1) == taken
+        assert not taken or gemm.lev_linear_mfma_ranges_of(M, N, Ki, 0) == 1
         a = torch.randn(M, Ki + 8, device=DEV, generator=g).bfloat16()[:, :Ki]
         res = torch.randn(M, N, device=DEV, generator=g)
         want = a.double() @ w.double().T + bias.double() + res.double()
@@ -137,3 +138,40 @@ def test_the_choice_between_the_two_kernels_is_within_a_quarter_of_the_better_on
         K._check(gemm.lev_linear_mfma_force(0))
         K._ws_need.clear()
     assert not [x for x in report if x[1][0] > 1.25 * min(x[1][1:])], report
+
+
+# beyond the ring kernel's sizes: 65 to 128 rows of more than 32,768 outputs (the kernel of streamed weights, all of a column's rows at once), more rows of four million outputs and more
+# (tiles of 256 x 256, 256 x 192, 256 x 128 and 128 x 128, K in one range and in two and three)
+BEYOND = [(65, 33001, 1608, 1), (100, 50257, 768, 1), (127, 32776, 4104, 1), (128, 40001, 200, 1), (512, 8192, 16384, 2), (385, 12288, 6400, 2), (700, 6400, 12288, 3), (257, 16390, 1032, 1),
+          (2048, 6144, 72, 1), (513, 12289, 392, 1), (300, 22002, 1032, 1), (1300, 4004, 520, 1), (130, 33001, 264, 1), (4100, 1032, 72, 1)]
+
+
+@pytest.mark.parametrize("M,N,Ki,ranges", BEYOND)
+def test_products_beyond_the_ring_kernel(K, M, N, Ki, ranges, monkeypatch):
+    """Every epilogue, outputs that end inside a tile, and sums whose ranges are left; the bound is the first test's."""
+    gemm = K._unit("gemm_mfma")
+    monkeypatch.setattr(K, "gemm_library", False)
+    for left in (0, 1):
+        assert gemm.lev_linear_mfma_ring_of(M, N, Ki, left) == -1 and gemm.lev_linear_mfma_ranges_of(M, N, Ki, left) == ranges
+    g = torch.Generator(device=DEV).manual_seed(N + Ki)
+    w = (torch.randn(N, Ki, device=DEV, generator=g) * Ki ** -0.5).bfloat16()
+    a = torch.randn(M, Ki + 8, device=DEV, generator=g).bfloat16()[:, :Ki]
+    bias, res = torch.randn(N, device=DEV, generator=g), torch.randn(M, N, device=DEV, generator=g)
+    x, y = a.double(), w.double().T
+    want, size = x @ y, x.abs() @ y.abs()
+    bound = (Ki + 4) * 2.0 ** -24 * (size + bias.double().abs() + res.double().abs())
+    out = torch.full((M, N + 3), float("nan"), device=DEV)
+    K.linear(a, w, bias, out[:, :N], residual=res)
+    assert bool(((out[:, :N].double() - want - bias.double() - res.double()).abs() <= bound).all()) and bool(torch.isnan(out[:, N:]).all())
+    left = res.clone()
+    pending = K.linear(a, w, bias, left, residual=left, may_leave_pending=True)
+    assert (pending is not None) == (ranges > 1)
+    if pending is not None:
+        assert pending.n_ranges == ranges and torch.equal(left, res)
+        K.finish(pending)
+    assert bool(((left.double() - want - bias.double() - res.double()).abs() <= bound).all())
+    half = torch.full((M, N), float("nan"), device=DEV, dtype=torch.bfloat16)
+    for act, f in (("none", lambda u: u), ("gelu_new", lambda u: torch.nn.functional.gelu(u, approximate="tanh")), ("gelu", torch.nn.functional.gelu), ("silu", torch.nn.functional.silu)):
+        K.linear(a, w, bias, half, activation=act)
+        u = f(want + bias.double())
+        assert float((half.double() - u).abs().max() / u.abs().max()) < 2e-2, act
