@@ -342,15 +342,15 @@ static const RingShape kRing[8] = {
 // An estimate of every tile and number of ranges: rounds of the CUs times a workgroup's k-tiles, joined (exponent 1.27: neither hides the other wholly) with the time the
 // weights take from memory, and what writing the sums costs; of ranges also the pass that adds them: a kernel of its own, or, where they are left, what
 // the norm behind the product pays for them (64 rows of 1600: 2.5 us, with 2 / 4 / 8 ranges 3.2 / 3.4 / 4.1; 264 rows 2.8, 4.4 / 5.0 / 6.1), which gives a row a thousand threads then:
-// beyond two rows a CU they take turns. One price for all sums of K >= 4 N, as if a norm always followed, put 2,020 rows of 128 x 2048 into two ranges and a pass (9.5 us; in one 8.7), 128 x 512 at
+// beyond two rows a CU they take turns; activations that no L2 holds are read by each column of tiles (4,000 rows of 512 x 2048: 128 columns a tile 17.8 us, 64 24.5). One price for all sums of K >= 4 N, as if a norm always followed, put 2,020 rows of 128 x 2048 into two ranges and a pass (9.5 us; in one 8.7), 128 x 512 at
 // 1,024 into four (6.6, 4.9), and with the norm 64 x 4096 at 4,000 into four (21.6, 20.2). It stands for longer sums with a pass of their own: in one range their small tiles take up to 30 % more
 // than the estimate, about what the pass costs (700 rows of 1280 x 5120 28.7 us in one, 23.9 in three). The tiles' numbers are fitted to
 // 13,000 launches (25 weights of 512 x 2048 to 16384 x 4096, 64 to 2,048 rows, up to five million outputs), off by 6 % on average; the prices of ranges to 16,000 more (34 weights of
-// 16 x 2048 to 4096 x 16384 in no cache, 17 to 4,000 rows, each with its own pass and with the norm): the choice is 1.0 and 1.5 % behind the best on average, more than 8 % at 12 and 21 of
-// 440 shapes (512 rows of 1600 x 6400 27.5 us for 26.1, 4,000 of 512 x 2048, which the library has, 24.5 for 17.8).
+// 16 x 2048 to 4096 x 16384 in no cache, 17 to 4,000 rows, each with its own pass and with the norm): the choice is 1.0 and 1.5 % behind the best on average, more than 8 % at 10 and 19 of
+// 440 shapes (264 rows of 2048 x 5376 22.8 us for 20.4).
 static RingPlan ring_choice(int M, int N, int K, bool left) {
   const int nk = (K + 63) >> 6;
-  const double memory = 2e-6 * N * K * 0.140, outputs = 4e-6 * M * N;
+  const double weights = 2e-6 * N * K * 0.140, outputs = 4e-6 * M * N;
   RingPlan best = {0, 1, 1e30};
   for (int i = 0; i < 8; ++i) {
     const RingShape& sh = kRing[i];
@@ -360,7 +360,7 @@ static RingPlan ring_choice(int M, int N, int K, bool left) {
       const int per = (nk + s - 1) / s;
       if (s > 1 && (wgs > 520 || nk / s < 2)) break;
       if (per * (s - 1) >= nk) continue;  // a range would be empty
-      if ((i == 7 && per > 96) || (i > 4 && M <= 128)) continue;  // no registers for a total: chains would be longer than before
+      if ((i == 7 && per > 96) || (i == 5 && per > 64) || (i > 4 && M <= 128)) continue;  // no registers for a total (96 x 128: for a second sum): chains would be longer than before
       const double beyond = 2e-6 * M * K / s / 4.2 - 1.0;  // activations of a range that an L2 does not hold
       double cus;
       if (sh.two) {
@@ -370,7 +370,8 @@ static RingPlan ring_choice(int M, int N, int K, bool left) {
         cus = (double)((wgs + 255) / 256) * (per * sh.alone + sh.ends);
       }
       cus *= 1.0 + 0.110 * (beyond < 0.0 ? 0.0 : beyond > 1.0 ? 1.0 : beyond);
-      double us = 1.63 + pow(pow(cus, 1.27) + pow(memory, 1.27), 1.0 / 1.27) + 0.214 * s * outputs;
+      const double rows = 2e-6 * M * K / s > 16.0 ? 0.028 * ((N + sh.bn - 1) / sh.bn) * 2e-6 * M * K : 0.0;  // every column of tiles reads them from beyond the caches of a chiplet
+      double us = 1.63 + pow(pow(cus, 1.27) + pow(weights + rows, 1.27), 1.0 / 1.27) + 0.214 * s * outputs;
       if (s > 1) {
         const int more_rows = std::max(0, M - 512);
         if (left) us += 0.1 + s * outputs / 4.5 + 1.5e-3 * more_rows;
@@ -392,12 +393,12 @@ RingPlan lev_ring_plan(int M, int N, int K, bool left) {
 }
 
 // Every how many k-tiles (a power of two; the first time after half as many) a wave's sums join its total: so that no chain of roundings is longer than in the kernels that
-// had these products before. Those were row blocks up to 256 rows (2 to 4 products a chain), ranges of K up to 128 rows of larger weights (10 and more) and up to 320 rows of
-// small ones, and above the library's kernels and tiles of one chain. In 64 x 64 tiles a join every 8 k-tiles costs 2 - 3 %.
+// had these products before. Those were row blocks up to 256 rows (2 to 4 products a chain), ranges of K up to 128 rows of larger weights (10 and more), up to 320 rows of
+// small ones and of long sums of narrow outputs (700 rows of 384 x 1536: 9.9e-8 then, 1.14e-7 in one chain), and else above 256 rows the library's kernels and tiles of one chain. In 64 x 64 tiles a join every 8 k-tiles costs 2 - 3 %.
 static int ring_fold(int BM, int BN, int M) {
   const int never = 1 << 20;
   if (BM * BN > 64 * 64) return M <= 128 ? 16 : never;
-  return M <= 256 ? 8 : M <= 320 ? 16 : never;
+  return M <= 256 ? 8 : 16;
 }
 
 template <typename TO, int BM, int BN, int WGM, int WGN, int R>

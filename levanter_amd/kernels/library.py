@@ -400,7 +400,7 @@ class HipKernels:
             ldr = ldo if residual is out else _rows(residual, "linear: residual")
         act = ACTIVATIONS[activation]
         if adt == torch.bfloat16 and self.use_mfma and K % 8 == 0 and lda % 8 == 0 and a.data_ptr() % 16 == 0:
-            if self.gemm_library and (self.use_library(M, N, K, act) or (residual is not None and self.library_adds_faster(M, N, K, act))):
+            if self.gemm_library and self.use_library(M, N, K, act):
                 key = (M, N, K, act, bias is None, residual is None, odt)
                 # never while a HIP graph is being recorded: what the library records besides its kernel is not ours to vouch for
                 if key not in self._library_refused and (self.library_in_graphs or not torch.cuda.is_current_stream_capturing()):
@@ -462,16 +462,15 @@ class HipKernels:
     def use_library(cls, M: int, N: int, K: int, act: int) -> bool:
         """Which products go to the vendor library: those with an epilogue it has, at the shapes where it was measured
         ahead on MI355X (with epilogues). Up to 64 rows see ``_library_reads_weights_faster``. Above, ours keep outputs below 2^22 numbers, 32,768 columns at
-        most (figures beside the ring kernel's rule), but from 1,024 rows not 24 columns and fewer (16 x 2048 at 2,020 rows, library / ours 5.9 / 7.4 us, 24 x 3072 7.1 / 8.2, 32 x 2048
-        7.8 / 7.1), and from 2,048 rows not sums of K >= 4 N, 1,536 and more, whose output fills the chip without ranges of K (3,000 rows of 512 x 3584 23.1 / 27.7,
-        1024 x 4096 33.9 / 36.5; shorter sums 256 x 1024 at 4,000 12.0 / 7.9, fewer rows 1600 x 6400 at 1,024 45.5 / 36.5). The library takes the rest: from 256 rows all but the longest sums (K >= 4 N) below 1,024 rows, and of 65 to
+        most (figures beside the ring kernel's rule; the library is up to a fifth ahead where 1,024 rows and more meet 48 columns and fewer, 16 x 2048 at 2,020 rows 5.9 / 7.4 us, or
+        three million outputs with a residual, 2048 x 2048 at 2,020 32.2 / 35.2, but its one chain of sums is 1.5 to 2.5 times as far off, 2.7e-7 / 1.9e-7 there), and the library takes the rest: from 256 rows all but the longest sums (K >= 4 N) below 1,024 rows, and of 65 to
         255 rows (heads of tens of thousands of outputs) those with N >= 2 K, but below 128 rows no weights of less than 32 MB and below 96 rows none of more than 256 MB."""
         if act not in cls.LIBRARY_ACTIVATIONS or M < cls.LIBRARY_MIN_ROWS:
             return False
         if M <= 64:
             return cls._library_reads_weights_faster(M, N, K)
         if N <= 32768 and M * N < (1 << 22):
-            return M >= 1024 and (N <= 24 or (M >= 2048 and M * N >= (1 << 20) and K >= max(4 * N, 1536)))
+            return False
         if M < 256:
             if N < 2 * K:
                 return False
@@ -479,13 +478,6 @@ class HipKernels:
                 return M >= 128
             return not (M < 96 and N * K > (1 << 27))
         return not (K >= 4 * N and M < 1024)
-
-    @classmethod
-    def library_adds_faster(cls, M: int, N: int, K: int, act: int) -> bool:
-        """Products with a residual that the library has beside those of ``use_library``: from three million outputs on, of 1,024 rows and more and sums of K <= 2 N
-        (library / ours with the norm behind them: 2048 x 2048 at 2,020 rows 32.2 / 35.2 us, 3072 x 1536 at 1,300 29.8 / 34.6; longer sums 2048 x 5376 at 1,800 56.7 / 53.1, fewer
-        rows 4096 x 4096 at 777 47.3 / 44.3, 1600 x 1600 at 1,024 22.5 / 20.3)."""
-        return act in cls.LIBRARY_ACTIVATIONS and M >= 1024 and N <= 32768 and 3 << 20 <= M * N < 1 << 22 and K <= 2 * N
 
     @staticmethod
     def _library_reads_weights_faster(M: int, N: int, K: int) -> bool:

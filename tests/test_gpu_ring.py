@@ -67,7 +67,7 @@ def test_infinities_and_nan_stay_in_their_row_and_column(K, M, N, Ki):
 
 
 @pytest.mark.parametrize("M,N,Ki,chain", [(65, 3072, 2048, 4), (160, 2048, 2048, 4), (256, 1600, 1600, 4), (192, 2560, 1024, 4), (128, 4096, 4096, 4), (96, 4096, 16384, 8), (264, 1024, 2048, 8),
-                                          (600, 4096, 16384, 96)])
+                                          (600, 4096, 16384, 96), (700, 384, 1536, 8), (1300, 2048, 5376, 64)])
 def test_the_sums_chains_of_roundings_stay_short(K, M, N, Ki, chain):
     """Sums of ``chain`` products of 32 at most, joined in a row: the bound is derived beside the test of this name for a few rows. The kernels that had these products before
     had such chains; twice as long ones are 10 to 40 % above."""
