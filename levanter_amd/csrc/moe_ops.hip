@@ -397,7 +397,7 @@ moe_linear_few_kernel(const MoeLinearArgs p) {
   moe_store4<TO>(static_cast<TO*>(p.out) + (size_t)(first + col) * p.o_stride + o, v, F - o, p.vec);
 }
 
-// Tiles of 128 rows (prompts, large batches) of sums that are no multiple of 128 or below 384 (moe_ring.hip has the others): a workgroup of four waves owns 128 rows and BN weight rows (with glu: BN / 2 outputs' gate
+// Tiles of 128 rows (prompts, large batches) of sums that are no multiple of 128 or below 384, and of fewer units than fill the CUs (moe_ring.hip has the others): a workgroup of four waves owns 128 rows and BN weight rows (with glu: BN / 2 outputs' gate
 // rows and the same outputs' up rows), a wave 64 x BN / 2 of them in 32x32x16 products (the transposed product out^T = w a^T: a lane ends
 // with four neighbouring outputs of a row). K goes by in steps of 64, the step after next on its way in registers, two buffers in LDS,
 // one barrier a step that waits for LDS only; loads, LDS writes and fragment reads are issued one by one between the products. Rows

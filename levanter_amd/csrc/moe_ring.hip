@@ -273,8 +273,16 @@ static int launch_moe_ring(const MoeLinearArgs& args, hipStream_t stream) {
   return lev_check_launch("moe_linear (ring)");
 }
 
+// Which products: N rows of w an expert, K numbers each, as many tiles as the step's sizes allow. Below 0.6 full units a CU the CUs that have one walk it alone, and twice as many tiles of 128 x 128, two
+// a CU, are ahead. Measured over 192 shapes (4 to 128 experts, 300 to 12,000 rows, 64 to 2,048 outputs of 384 to 2048; microseconds, tiles of 128 x 128 / here, at so many full units a CU): 0.12 8 experts, 1,000 rows, 384 outputs of
+// 768 16.0 / 21.4; 0.23 1024 of 2048 34.3 / 44.0; 0.47 2048 of 1408 30.5 / 39.1; 0.59 12,000 rows, 384 of 768 23.3 / 23.5; 0.61 32 experts, 1,000 rows, 1024 of 2048 45.4 / 48.4; 0.64 8 experts, gated 1408 of 2048 56.3 / 47.9; 0.73 32
+// experts, 12,000 rows, 384 of 768 28.8 / 26.3; 0.98 4,000 rows, 1024 of 2048 63.1 / 55.6; 1.95 12,000 rows 104 / 87.
+extern "C" int lev_moe_ring_takes(int max_tiles, int K, int N) {
+  return K % 128 == 0 && K >= 128 * MOE_RING_TILES && 5L * max_tiles * N >= 3L * 8 * MOE_RING_CUS * MOE_RING_BN;
+}
+
 int lev_moe_ring(const MoeLinearArgs& args, long a_rows, int out_dtype, int glu, int max_tiles, hipStream_t stream) {
-  if (args.K % 128 || args.K < 128 * MOE_RING_TILES || (size_t)a_rows * args.a_stride >= (1ull << 31) || (size_t)args.N * args.K >= (1ull << 31)) return 1;
+  if (!lev_moe_ring_takes(max_tiles, args.K, args.N) || (size_t)a_rows * args.a_stride >= (1ull << 31) || (size_t)args.N * args.K >= (1ull << 31)) return 1;
   MoeLinearArgs p = args;
   const int out = glu ? MOE_RING_BN / 2 : MOE_RING_BN;
   p.n_cols = (p.F + out - 1) / out;
