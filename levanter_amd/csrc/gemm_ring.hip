@@ -14,7 +14,8 @@
 // 768 x 3072 12.8 / 8.1, 2048 x 5376 at 600 rows 31.2 / 26.1, 4096 x 16384 at 264 rows 73 / 56. Errors against 64 bits, before / here: 264 rows of 4800 x
 // 1600 2.4e-7 / 1.2e-7, 1600 x 6400 1.95e-7 / 1.4e-7, 2048 x 5376 at 400 rows 4.6e-7 / 2.2e-7; of the row blocks and ranges of K (with one chain of K / 128 here they were
 // exceeded, 1.3e-7 at 2,048 inputs: the joins are for these) 96 rows of 3072 x 2048 8.6e-8 / 8.2e-8, 256 of 1600 x 1600 8.3e-8 / 7.9e-8, 192 of 2560 x 1024 7.5e-8 / 7.4e-8, 128 of
-// 4096 x 4096 1.24e-7 / 0.92e-7, 600 of 4096 x 16384 3.5e-7 / 2.8e-7; of 386 shapes (28 weights, 65 to 1,328 rows) none is further off. Taken back: k-tiles that begin at another place in every
+// 4096 x 4096 1.24e-7 / 0.92e-7, 700 of 384 x 1536 9.9e-8 / 9.1e-8; of 856 sizes (45 weights, 17 to 2,020 rows), with
+// the ranges left and not, none is further off. Taken back: k-tiles that begin at another place in every
 // workgroup (up to 40 % slower where neighbours then no longer wait for the same line, 2 - 9 % faster at K = 16384 alone), a ring twice as deep (8 % slower), a
 // CU for every workgroup where two fit (the same).
 #include "gemm_ring.h"
@@ -346,7 +347,7 @@ static const RingShape kRing[8] = {
 // 1,024 into four (6.6, 4.9), and with the norm 64 x 4096 at 4,000 into four (21.6, 20.2). It stands for longer sums with a pass of their own: in one range their small tiles take up to 30 % more
 // than the estimate, about what the pass costs (700 rows of 1280 x 5120 28.7 us in one, 23.9 in three). The tiles' numbers are fitted to
 // 13,000 launches (25 weights of 512 x 2048 to 16384 x 4096, 64 to 2,048 rows, up to five million outputs), off by 6 % on average; the prices of ranges to 16,000 more (34 weights of
-// 16 x 2048 to 4096 x 16384 in no cache, 17 to 4,000 rows, each with its own pass and with the norm): the choice is 1.0 and 1.5 % behind the best on average, more than 8 % at 10 and 19 of
+// 16 x 2048 to 4096 x 16384 in no cache, 17 to 4,000 rows, each with its own pass and with the norm): the choice is 0.9 and 1.5 % behind the best on average, more than 8 % at 9 and 19 of
 // 440 shapes (264 rows of 2048 x 5376 22.8 us for 20.4).
 static RingPlan ring_choice(int M, int N, int K, bool left) {
   const int nk = (K + 63) >> 6;
