@@ -1,30 +1,7 @@
 // y = act(a . w^T + bias) + residual in 32 bits on the 32-bit matrix instruction (v_mfma_f32_16x16x4_f32: full 32-bit products and
-// sums, no reduced mode). a [M, K] (row stride lda), w [N, K], y [M, N].
-#include "common.h"
+// sums, no reduced mode). a [M, K] (row stride lda), w [N, K], y [M, N]. Some hundred rows and more go to gemm_f32_split.hip by the rule at this file's end.
+#include "gemm_f32.h"
 #include <math.h>
-
-typedef __attribute__((ext_vector_type(4))) float gf_f32x4;
-
-// four neighbouring outputs of a row
-__device__ __forceinline__ void gemm_f32_store(gf_f32x4 v, const float* bias, const float* residual, long ldr, float* out, long ldo, int m, int o, int N, int act, int vec) {
-  if (vec && o + 4 <= N) {
-    if (bias) v += *reinterpret_cast<const gf_f32x4*>(bias + o);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = lev_activate(v[r], act);
-    if (residual) v += *reinterpret_cast<const gf_f32x4*>(residual + (size_t)m * ldr + o);
-    *reinterpret_cast<gf_f32x4*>(out + (size_t)m * ldo + o) = v;
-  } else {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      if (o + r >= N) break;
-      float x = v[r];
-      if (bias) x += bias[o + r];
-      x = lev_activate(x, act);
-      if (residual) x += residual[(size_t)m * ldr + o + r];
-      out[(size_t)m * ldo + o + r] = x;
-    }
-  }
-}
 
 // A workgroup of W waves owns 16 RT rows and 16 NT outputs; its waves split K (steps of 16 dealt in stretches) and the partial sums are
 // added through LDS in wave order. The product is transposed, out^T = w a^T, so that a lane ends with four neighbouring outputs of one
@@ -363,7 +340,7 @@ static const GemmF32LineTile GEMM_F32_LINE_TILES[] = {{1, 1, 4, 0.32f, 0.155f, 0
                                                       {2, 2, 1, 0.6f, 0.5f, 1.f},     {2, 3, 1, 0.76f, 0.73f, 2.f},  {2, 4, 1, 0.98f, 0.96f, 2.5f}};
 #define GEMM_F32_N_TILES (int)(sizeof(GEMM_F32_TILES) / sizeof(GEMM_F32_TILES[0]))
 
-static int gemm_f32_choose(int M, int N, int K) {  // an index into the first list, or behind its end into the second
+static int gemm_f32_choose(int M, int N, int K, double* estimate = nullptr) {  // an index into the first list, or behind its end into the second
   int best = 0;
   double best_us = 1e30;
   const double memory = 4.0 * N * K / 5.2e6;
@@ -383,6 +360,7 @@ static int gemm_f32_choose(int M, int N, int K) {  // an index into the first li
     const double us = t.start + fmax(memory, (K + 31) / 32 * fmax(t.alone + 0.15 * (n - 1) * t.among, n * t.among));
     if (us < best_us) best_us = us, best = GEMM_F32_N_TILES + i;
   }
+  if (estimate) *estimate = best_us;
   return best;
 }
 
@@ -400,10 +378,29 @@ static int gemm_f32_few(int M, int N, int K) {
   return K >= GEMM_F32_FEW_INPUTS[i][rounds < 4 ? rounds : 4] ? 1 << i : 0;
 }
 
-// the kernel of a product: 0 less the few-row kernel's room, or the tile's place in the two lists, one behind the other
+// the kernel of a product on the 32-bit instruction: 0 less the few-row kernel's room, or the tile's place in the two lists, one behind the other
 extern "C" int lev_linear_f32_choice(int M, int N, int K) {
   const int few = gemm_f32_few(M, N, K);
   return few > 0 ? -few : gemm_f32_choose(M, N, K);
+}
+
+// The tile of the kernel that splits its operands into bfloat16 numbers (gemm_f32_split.hip), or -1 where the kernels above are not behind by an estimate as theirs, fitted
+// to 208 shapes of 70 .. 2,048 rows (0.2 % behind the best on average, 14 % at worst: 2048 x 256 at 1,000 rows 13.4 us, 11.8 with 64 x 128; none behind the kernels above). Below 256
+// inputs those stay ahead of it, or level; and it knows no rows more than GEMM_F32_SPLIT_MOST apart. Kernels above / this one, microseconds: 4096 x 1024 at 777 rows 62 / 47, 1024 x 4096 72 / 63,
+// 50257 x 768 at 300 rows 209 / 166, 4096 x 4096 at 2,048 502 / 366, 1600 x 1600 at 512 34 / 27; not taken: 768 x 3072 at 606 rows 35 / 47, 1024 x 1024 at 404 15 / 19.
+extern "C" int lev_linear_f32_split(int M, int N, int K) {
+  if (K % 4 != 0 || K < 256 || K > GEMM_F32_SPLIT_MOST || lev_linear_f32_choice(M, N, K) < 0) return -1;
+  double us, best_us;
+  gemm_f32_choose(M, N, K, &best_us);
+  best_us *= 0.949;  // the estimates' own errors: of 190 shapes none is slower than before
+  int best = -1;
+  for (int i = 0; i < GEMM_F32_N_SPLIT_TILES; ++i) {
+    const GemmF32SplitTile& t = GEMM_F32_SPLIT_TILES[i];
+    const double n = ceil((double)((M + t.rows - 1) / t.rows) * ((N + t.outputs - 1) / t.outputs) / 256.0);
+    us = t.start + fmax(4.0 * N * K / 5.2e6, ((K + 31) / 32 + t.groups - 1) / t.groups * (n <= 1.0 ? t.alone : n * t.among));
+    if (us < best_us) best_us = us, best = i;
+  }
+  return best;
 }
 
 // 1: not for these operands (nothing has been launched): 16-byte loads need rows of a multiple of 4 numbers at 16-byte addresses
@@ -411,6 +408,8 @@ int lev_gemm_f32(const float* a, long lda, const float* w, const float* bias, co
                  int act, hipStream_t stream) {
   if (K % 4 != 0 || lda % 4 != 0 || ((uintptr_t)a & 15) != 0 || ((uintptr_t)w & 15) != 0) return 1;
   const int vec = ldo % 4 == 0 && ((uintptr_t)out & 15) == 0 && (!bias || ((uintptr_t)bias & 15) == 0) && (!residual || (ldr % 4 == 0 && ((uintptr_t)residual & 15) == 0));
+  const int split = lda <= GEMM_F32_SPLIT_MOST ? lev_linear_f32_split(M, N, K) : -1;
+  if (split >= 0) return lev_gemm_f32_split(split, a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act, vec, stream);
   const int choice = lev_linear_f32_choice(M, N, K), few = -choice, line = choice - GEMM_F32_N_TILES;
   if (few > 0) {
 #define GEMM_F32_FEW(MR) \

@@ -106,6 +106,71 @@ def test_linear_float32_keeps_infinities_where_they_are_in_every_kernel(K, M, Ki
     assert torch.equal(out[row] > 0, w[:, Ki - 1] > 0)
 
 
+# products whose operands are split into bfloat16 numbers: tiles of 128 x 128, 64 x 128 and 64 x 64 outputs that end inside a tile, whole steps of 32 inputs, a partial one of 4 and of 28,
+# odd and even numbers of steps, numbers that the two groups of a 64 x 64 tile share unevenly, sums that are joined once and often, and long ones
+SPLIT = [(0, 777, 260, 4097), (0, 513, 284, 6401), (0, 1030, 288, 3071), (0, 1030, 4100, 2051), (1, 1030, 256, 3071), (1, 513, 516, 3071), (1, 257, 540, 6401), (1, 609, 516, 3071), (2, 777, 772, 1030),
+         (2, 100, 1028, 6401), (2, 65, 3396, 6401), (2, 777, 4100, 1030), (2, 404, 796, 2051)]
+
+
+@pytest.mark.parametrize("tile,M,Ki,N", SPLIT)
+def test_split_products(K, tile, M, Ki, N):
+    """Bound: Ki roundings, at most, of what has been added up so far, and at most 2^-23 of every product for the parts that are left out; bias and residual two more."""
+    assert K.lib.lev_linear_f32_split(M, N, Ki) == tile
+    a_all, w, b, res = _rand(M, Ki + 8, seed=1).to(DEV), _rand(N, Ki, seed=2).to(DEV), _rand(N, seed=3).to(DEV), _rand(M, N, seed=4).to(DEV)
+    a = a_all[:, :Ki]
+    want = a.double() @ w.double().T + b.double()
+    size = a.double().abs() @ w.double().abs().T + b.double().abs()
+    out = torch.full((M, N + 3), float("nan"), device=DEV)
+    K.linear(a, w, b, out[:, :N], residual=res)
+    assert bool(((out[:, :N].double() - want - res.double()).abs() <= (Ki + 6) * EPS * (size + res.double().abs())).all())
+    assert bool(torch.isnan(out[:, N:]).all())
+    got = torch.empty(M, N, device=DEV)
+    K.linear(a, w, None, got)
+    exact = a.double() @ w.double().T
+    # in the 2-norm as below, with sums of their own for at most 256 numbers: 0.42 * 2^-24 * sqrt(c / 2 + K / (2 c)), c = 128
+    assert float((got.double() - exact).norm() / exact.norm()) <= 1.15 * 0.42 * EPS * (64 + Ki / 256) ** 0.5
+
+
+@pytest.mark.parametrize("tile,M,Ki,N", [(0, 513, 284, 6401), (1, 609, 516, 3071), (2, 404, 796, 2051)])
+def test_split_products_of_the_smallest_and_largest_numbers(K, tile, M, Ki, N):
+    """Powers of two on the operands change nothing, down to numbers whose last bits are the smallest there are and up to the largest, which have no bfloat16 parts."""
+    assert K.lib.lev_linear_f32_split(M, N, Ki) == tile
+    a, w = _rand(M, Ki, seed=1).to(DEV), _rand(N, Ki, seed=2).to(DEV)
+    a = a.sign() * a.abs().clamp(min=2.0 ** -6)
+    exact = a.double() @ w.double().T
+    for up, other in ((-119, 40), (119, -60), (60, -60)):
+        got = torch.empty(M, N, device=DEV)
+        K.linear(a * 2.0 ** up, w * 2.0 ** other, None, got)
+        assert float((got.double() * 2.0 ** -(up + other) - exact).norm() / exact.norm()) <= 1.15 * 0.42 * EPS * (64 + Ki / 256) ** 0.5
+    a[M // 2, 5], w[N // 2, 7] = 3.4e38, float("nan")
+    a[3, Ki - 1] = float("-inf")
+    a[M - 1, 0], w[0, 0] = 0.0, float("inf")
+    got = torch.empty(M, N, device=DEV)
+    K.linear(a, w, None, got)
+    want = (a.double() @ w.double().T).float()  # the same places beyond the range of 32 bits
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    inf = torch.isinf(want)
+    assert torch.equal(got[inf] > 0, want[inf] > 0)
+    size = (a.double().abs() @ w.double().abs().T)
+    fine = ~inf & ~torch.isnan(want)
+    assert bool(((got.double() - want.double()).abs() <= (Ki + 6) * EPS * size)[fine].all())
+
+
+@pytest.mark.parametrize("choice,M,Ki,N", [(8, 273, 772, 9001), (9, 129, 516, 9001), (10, 177, 516, 9001), (11, 465, 256, 9001), (12, 417, 772, 9001)])
+def test_rows_too_far_apart_to_be_split(K, choice, M, Ki, N):
+    """Rows more than 2^22 numbers apart: the tiles through LDS on the 32-bit instruction."""
+    assert K.lib.lev_linear_f32_choice(M, N, Ki) == choice
+    far = 2 ** 22 + 4
+    a = torch.empty(M * far, device=DEV).as_strided((M, Ki), (far, 1))
+    a.copy_(_rand(M, Ki, seed=1))
+    w, b, res = _rand(N, Ki, seed=2).to(DEV), _rand(N, seed=3).to(DEV), _rand(M, N, seed=4).to(DEV)
+    out = torch.empty(M, N, device=DEV)
+    K.linear(a, w, b, out, residual=res)
+    want = a.double() @ w.double().T + b.double() + res.double()
+    size = a.double().abs() @ w.double().abs().T + b.double().abs() + res.double().abs()
+    assert bool(((out.double() - want).abs() <= (Ki + 4) * EPS * size).all())
+
+
 def test_a_waves_sum_is_the_tree_over_lane_numbers(K):
     """Every lane's number is exact (one of four inputs counts), so that the sums are those of the 64 lanes, halves first, then of neighbours 16, 8, 4, 2 and 1 apart, and of the
     eight waves in order, bit by bit."""
