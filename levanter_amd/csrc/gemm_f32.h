@@ -12,6 +12,7 @@ struct GemmF32SplitTile {
 };
 static const GemmF32SplitTile GEMM_F32_SPLIT_TILES[] = {{128, 128, 1, 5.789f, 0.998f, 1.051f}, {64, 128, 1, 4.353f, 0.732f, 0.579f}, {64, 64, 2, 4.205f, 0.644f, 1.135f}};
 #define GEMM_F32_N_SPLIT_TILES (int)(sizeof(GEMM_F32_SPLIT_TILES) / sizeof(GEMM_F32_SPLIT_TILES[0]))
+extern "C" int lev_linear_f32_choice(int M, int N, int K);
 extern "C" int lev_linear_f32_split(int M, int N, int K);
 int lev_gemm_f32_split(int tile, const float* a, long lda, const float* w, const float* bias, const float* residual, long ldr, float* out, long ldo, int M, int N, int K,
                        int act, int vec, hipStream_t stream);

@@ -276,7 +276,7 @@ def ensure_built(unit: str = "core") -> str:
 # ---- the units of this package --------------------------------------------------------------------------------
 _P, _I, _L, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_long, ctypes.c_float
 
-register_unit("core", ["errors.hip", "elementwise.hip", "layer_ops.hip", "gemm_simple.hip", "gemm_f32.hip", "gemm_f32_split.hip", "attention_simple.hip", "attention_f32.hip", "attention_values.hip",
+register_unit("core", ["errors.hip", "elementwise.hip", "layer_ops.hip", "gemm_simple.hip", "gemm_f32.hip", "gemm_f32_split.hip", "gemm_f32_norm.hip", "attention_simple.hip", "attention_f32.hip", "attention_values.hip",
                        "attention_common.hip", "stream_ops.hip", "rotary.hip", "block_linear.hip", "recurrent_ops.hip", "group_norm.hip", "delta_rule.hip",
                        "moe_ops.hip", "moe_ring.hip", "linear_attention.hip", "state_recurrence.hip", "state_chunks.hip", "sum_norm.hip"], signatures={
     "lev_embed": [_P] * 5 + [_I, _I, _I, _F, _P],
@@ -331,6 +331,8 @@ register_unit("core", ["errors.hip", "elementwise.hip", "layer_ops.hip", "gemm_s
     "lev_feed_tokens": [_P, _P, _P, _I, _P],
     "lev_linear_f32_choice": [_I, _I, _I],
     "lev_linear_f32_split": [_I, _I, _I],
+    "lev_linear_f32_normed": [_P, _P, _P, _F, _I, _P, _P, _P, _L, _I, _I, _I, _I, _P],
+    "lev_linear_f32_normed_takes": [_I, _I, _I],
     "lev_linear_simple": [_P, _L, _P, _P, _P, _L, _P, _L] + [_I] * 6 + [_P],
     "lev_attention_simple": [_P, _L, _P, _L, _P, _P, _P, _P, _P] + [_I] * 6 + [_F, _I, _I, _F, _P, _I, _P],
     "lev_attention_f32": [_P, _L, _P, _L, _P, _P, _P, _P, _P, _I, _P, _I, _I, _P, _I, _P, _P, _L, _P] + [_I] * 4 + [_F, _I, _F, _P, _I, _P],

@@ -439,21 +439,28 @@ class HipKernels:
             takes = self._ws_need[(M, N, K)] = gemm.lev_linear_normed_takes(M, N, K) == 1
         return takes and self.use_mfma
 
+    def takes_norm_float32(self, M: int, N: int, K: int) -> bool:
+        """``takes_norm`` of products in float32."""
+        takes = self._ws_need.get((M, N, K, "float32"))
+        if takes is None:
+            takes = self._ws_need[(M, N, K, "float32")] = self.lib.lev_linear_f32_normed_takes(M, N, K) == 1
+        return takes
+
     def linear_normed(self, x, norm_weight, norm_bias, eps: float, rms: bool, w, bias, out, activation: str = "none") -> None:
-        """out = act(norm(x) @ w.T + bias): ``norm`` of the float32 rows x [M, K] into bfloat16 and ``linear`` behind it, bit for bit, in one
-        kernel, where ``takes_norm(M, N, K)``."""
+        """out = act(norm(x) @ w.T + bias): ``norm`` of the float32 rows x [M, K] into the weight's type and ``linear`` behind it, bit for bit, in one
+        kernel, where ``takes_norm(M, N, K)`` (of float32 weights ``takes_norm_float32``)."""
         _dev(x, norm_weight, norm_bias, w, bias, out)
         M, K = x.shape
         N = w.shape[0]
         _req(x.dtype == torch.float32 and x.is_contiguous(), "linear_normed: x must be contiguous float32")
         for t in (norm_weight, norm_bias):
             _req(t is None or (t.dtype == torch.float32 and t.numel() == K and t.is_contiguous()), "linear_normed: scale and shift must be float32 [K]")
-        _req(w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] == K and w.is_contiguous(), f"linear_normed: weight must be contiguous bfloat16 [N, {K}]")
+        _req(w.dtype in _DT and w.dim() == 2 and w.shape[1] == K and w.is_contiguous(), f"linear_normed: weight must be contiguous [N, {K}] in bfloat16 or float32")
         _req(bias is None or (bias.dtype == torch.float32 and bias.numel() == N and bias.is_contiguous()), "linear_normed: bias must be float32 [N]")
-        _req(out.dtype == torch.bfloat16 and tuple(out.shape) == (M, N), "linear_normed: bad out")
-        gemm = self._units.get("gemm_mfma") or self._unit("gemm_mfma")
-        self._check(gemm.lev_linear_normed(_ptr(x), _ptr(norm_weight), _ptr(norm_bias), float(eps), int(rms), _ptr(w), _ptr(bias), _ptr(out),
-                                           _rows(out, "linear_normed: out"), M, N, K, ACTIVATIONS[activation], self._s()))
+        _req(out.dtype == w.dtype and tuple(out.shape) == (M, N), "linear_normed: bad out")
+        entry = self.lib.lev_linear_f32_normed if w.dtype == torch.float32 else (self._units.get("gemm_mfma") or self._unit("gemm_mfma")).lev_linear_normed
+        self._check(entry(_ptr(x), _ptr(norm_weight), _ptr(norm_bias), float(eps), int(rms), _ptr(w), _ptr(bias), _ptr(out),
+                          _rows(out, "linear_normed: out"), M, N, K, ACTIVATIONS[activation], self._s()))
 
     LIBRARY_ACTIVATIONS = (ACTIVATIONS["none"], ACTIVATIONS["gelu_new"], ACTIVATIONS["relu"])
     LIBRARY_MIN_ROWS = 25  # up to 24 rows the skinny kernel is ahead everywhere, or behind by less than the library's first use costs

@@ -30,6 +30,11 @@ class Linear:
         self.bias = None if bias is None else bias.to(env.device, torch.float32).contiguous()
         self.n_out, self.n_in = self.weight.shape
 
+    def takes_norm(self, kernels, rows: int) -> bool:
+        """Whether the product of so many rows has a kernel that normalises them on the way."""
+        takes = getattr(kernels, "takes_norm" if self.weight.dtype == torch.bfloat16 else "takes_norm_float32", None)
+        return takes is not None and self.weight.data_ptr() % 16 == 0 and takes(rows, self.n_out, self.n_in)
+
     def __call__(self, a: torch.Tensor, ctx: StepContext, *, activation: str = "none", residual: Optional[torch.Tensor] = None,
                  out: Optional[torch.Tensor] = None, out_dtype: Optional[torch.dtype] = None, final: bool = False,
                  may_leave: bool = False) -> torch.Tensor:
@@ -39,8 +44,8 @@ class Linear:
         reads ``out`` next."""
         if type(a) is RowsAhead:
             n = a.norm
-            if (residual is None and not may_leave and (ctx.dtype if out is None and out_dtype is None else out_dtype or out.dtype) == torch.bfloat16
-                    and ctx.kernels.takes_norm(a.shape[0], self.n_out, self.n_in)):
+            if (residual is None and not may_leave and (ctx.dtype if out is None and out_dtype is None else out_dtype or out.dtype) == self.weight.dtype
+                    and self.takes_norm(ctx.kernels, a.shape[0])):
                 if out is None:
                     out = ctx.empty(a.shape[0], self.n_out, out_dtype)
                 ctx.kernels.linear_normed(a.x, n.weight, n.bias, n.eps, n.rms, self.weight, self.bias, out, activation)

@@ -42,10 +42,9 @@ class LayerNorm(Norm):
         return out
 
     def ahead_of(self, product, x: torch.Tensor, ctx: StepContext):
-        kernels = ctx.kernels
-        if (type(product) is Linear and product.weight.dtype == torch.bfloat16 and type(self).__call__ is LayerNorm.__call__
-                and ctx.pending is None and ctx.product_pending is None and hasattr(kernels, "takes_norm")
-                and x.is_contiguous() and x.data_ptr() % 16 == 0 and kernels.takes_norm(x.shape[0], product.n_out, product.n_in)):
+        if (type(product) is Linear and type(self).__call__ is LayerNorm.__call__
+                and ctx.pending is None and ctx.product_pending is None
+                and x.is_contiguous() and x.data_ptr() % 16 == 0 and product.takes_norm(ctx.kernels, x.shape[0])):
             return RowsAhead(x, self)
         return self(x, ctx)
 
