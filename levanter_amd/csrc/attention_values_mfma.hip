@@ -317,35 +317,40 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
   }
 }
 
-// Runs of several tokens: one workgroup of PF_WAVES waves per (tile of up to PF_ROWS consecutive query tokens, query head,
+// Runs of several tokens: one workgroup per (tile of up to PF_ROWS consecutive query tokens or half of one, query head,
 // set of value heads). The keys and values of a block of 64 positions are staged once for all waves: global -> registers
-// (requested two blocks ahead, while the blocks before are computed) -> LDS, keys as [HD/8][64][8], values transposed as
-// [value head][VD][64 + 8] with everything beyond the last written key made zero on the way (from the registers, not when they are asked
+// (requested a block ahead) -> LDS, with everything beyond the last written key made zero on the way (from the registers, not when they are asked
 // for: that would wait for them).
-// What bounds it: the chain of a block (two barriers, scores, softmax, values) in the workgroups of the longest tiles, few of which share a CU.
-// Two prompts of 1,000, 16 heads of 256 / 224 and of 128 / 64, microseconds a layer: 102 -> 65; three of 1,000, 960 and 90 of 128 / 64: 77 -> 49. What went:
-// waits for loads that had just been asked for (zeros were put in at once), a division and its branches per chunk (now one a block), masks on the
-// scores of blocks that all rows see (most), room for four value heads where there is one (three quarters of the value loads were repeats).
-#define VS_STRIDE 72
+// What bounds it: the chain of a block (two barriers, scores, softmax, values) in the workgroups of the longest tiles, few of which share a CU. So the operands of the products
+// come from LDS four at a time, two groups ahead (one, where a workgroup is half a tile) instead of each ahead of its product; a block has no branch for its scores; the maximum goes over the lanes by swaps, and the outputs
+// are scaled only when one was raised. The next block is asked for in one set of registers: of two sets, one of which a branch picked, the loads went to a third, were waited for
+// and copied there, in every block.
+// Before / now, microseconds a layer, 16 heads of 128 / 64, 256 / 224, 64 / 32: 1,000 tokens 38 / 24, 60 / 49, 30 / 20; two of 1,015 41 / 31, 64 / 54, 31 / 24; 2,000 70 / 54, 111 / 87, 54 / 41; twelve of 150
+// 12.8 / 11.4, 27 / 29, 9.9 / 9.4. (Wide heads take the registers of two workgroups of which one is left a CU: many runs of one to three blocks are 4 - 15 % slower there.)
 #define RUN_MAX_LDS (80 * 1024)  // bytes a workgroup may take: two workgroups a CU
 #define RUN_PAGES 2048  // page ids of a tile's key range that are kept in LDS
-#define K_STAGE ((HD * 8 + PF_THREADS - 1) / PF_THREADS)  // 16-byte chunks of a key block per thread
+
+// Waves of a workgroup, 16 query tokens each: half a tile's, where three such workgroups fit a CU's registers (heads of 128 / 64, microseconds, whole tiles / halves: 1,000 tokens 28.3 / 24.5, six
+// of 1,000 82 / 68, two of 1,015 30.7 / 30.4; of 256 / 224 two of 1,015 55 / 100: the loads of a block are twice as many registers a thread).
+#define RUN_WAVES(NC) ((NC) == 1 && HD + VD <= 192 ? PF_WAVES / 2 : PF_WAVES)
 
 // NC: value heads that a wave has room for, as above: 1, or NVC for layers with more
-template <int NC>
-__global__ void __launch_bounds__(PF_THREADS)
+template <int NC, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES, WAVES == PF_WAVES ? 2 : 3)
 attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, float* __restrict__ out, const bf16_t* __restrict__ k_pages,
                                   const bf16_t* __restrict__ v_pages, const int* __restrict__ positions, const int* __restrict__ token_seq,
                                   const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tiles, int H, int KVH, int NV,
                                   int PS, float scale, int window, int chunk, int keep, float softcap, const float* __restrict__ slopes,
                                   const float* __restrict__ sinks) {
-  constexpr int V_STAGE = (NC * VD * 8 + PF_THREADS - 1) / PF_THREADS;  // 16-byte chunks of the value blocks per thread
+  constexpr int THREADS = 64 * WAVES, PARTS = PF_ROWS / (16 * WAVES);
+  constexpr int K_STAGE = (HD * 8 + THREADS - 1) / THREADS, V_STAGE = (NC * VD * 8 + THREADS - 1) / THREADS;  // 16-byte chunks of a block of keys, of values per thread
   extern __shared__ __attribute__((aligned(16))) unsigned char av_smem[];
   bf16_t* ks = reinterpret_cast<bf16_t*>(av_smem);  // [HD/8][64][8]
-  bf16_t* vs = ks + HD * 64;                        // [n_c][VD][VS_STRIDE]
+  bf16_t* vs = ks + HD * 64;                        // [8 chunks][n_c VD][8]
   __shared__ int pages_s[RUN_PAGES];                // page ids of the blocks that the tile's keys lie in
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, g = lane >> 4;
-  const int first = tiles[2 * blockIdx.x], n = tiles[2 * blockIdx.x + 1];
+  const int tile = blockIdx.x / PARTS, skip = (blockIdx.x - tile * PARTS) * 16 * WAVES;
+  const int first = tiles[2 * tile] + skip, n = min(tiles[2 * tile + 1] - skip, 16 * WAVES);
   if (n <= 0) return;  // the whole workgroup
   const int head = blockIdx.y, group = H / KVH, kvh = head / group;
   const bool active = wave * 16 < n;            // this wave has query rows
@@ -373,11 +378,11 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
   const int first_block = lo_wg / 64, n_kept = lev_kept_blocks(lo_wg, keep), n_blocks = n_kept + p_max_wg / 64 - first_block + 1;
   const int n_kpg = n_kept > 0 ? block_of(n_kept * 64 - 1) + 1 : 0;
   int none = 0;  // negative: a page that holds a key in sight is missing
-  for (int i = tid; i < min(n_kpg, RUN_PAGES); i += PF_THREADS) {
+  for (int i = tid; i < min(n_kpg, RUN_PAGES); i += THREADS) {
     const int page = bt[i];
     pages_s[i] = page, none |= i * PS < keep ? page : 0;
   }
-  for (int i = tid; i < min(n_pg, RUN_PAGES - n_kpg); i += PF_THREADS) {  // the host sends longer ranges elsewhere
+  for (int i = tid; i < min(n_pg, RUN_PAGES - n_kpg); i += THREADS) {  // the host sends longer ranges elsewhere
     const int page = bt[pg0 + i];
     pages_s[n_kpg + i] = page, none |= (pg0 + i + 1) * PS > lo_wg ? page : 0;
   }
@@ -407,11 +412,17 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
   const size_t k_head = (size_t)HD * PS, v_head = (size_t)VD * PS;
   const bool all_pages = __syncthreads_or(none < 0) == 0;  // the page ids are there, and every key in sight has a page
 
-  u32x4 kst_a[K_STAGE], vst_a[V_STAGE], kst_b[K_STAGE], vst_b[V_STAGE];  // two blocks on their way at any time
+  // In LDS a chunk of 8 dimensions has its 64 keys in the order in which the score tiles have them as rows, and a chunk of 8 keys' values its rows in their
+  // order but for a turn by twice the chunk's number: 16 lanes' reads, and what neighbouring lanes write, fall on all banks.
+  const int v_rows = NC == 1 ? VD : n_c * VD;
+  const bf16_t* ks_get = ks + (g * 64 + col) * 8;
+  const bf16_t* vs_get[2] = {vs + (g * v_rows + (col ^ 2 * g)) * 8, vs + ((4 + g) * v_rows + (col ^ (8 + 2 * g))) * 8};
+  bf16_t* ks_put = ks + ((tid & ~63) + (tid & 32) + 16 * (tid >> 2 & 1) + 4 * (tid >> 3 & 3) + (tid & 3)) * 8;
+  u32x4 kst[K_STAGE], vst[V_STAGE];  // the next block, on its way
   // This thread's chunks of the block at key0, from the pages into registers: chunks of one key, and of one group of 8 keys' values.
   // Every load stands under no condition (a load in a branch makes the compiler wait for all loads in flight where the
   // branch ends): addresses are clamped into what can be read, what must not count is made zero when it goes to LDS.
-  auto fetch = [&](int key0, u32x4 (&kst)[K_STAGE], u32x4 (&vst)[V_STAGE]) {
+  auto fetch = [&](int key0) __attribute__((always_inline)) {
     const int page_no = block_of(key0), page_key = page_no * PS;
     int ka, va;
     const int kpage = place_of(min(key0 + (tid & 63), p_max_wg), page_no, page_key, ka);
@@ -419,11 +430,11 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
     const bf16_t* kb = k_pages + ((size_t)max(kpage, 0) * KVH + kvh) * k_head + (size_t)ka * 8;
     const bf16_t* vb = v_pages + ((size_t)max(vpage, 0) * KVH + c0) * v_head + va;
 #pragma unroll
-    for (int i = 0; i < K_STAGE; ++i) kst[i] = *reinterpret_cast<const u32x4*>(kb + min((tid >> 6) + PF_THREADS / 64 * i, HD / 8 - 1) * PS * 8);
+    for (int i = 0; i < K_STAGE; ++i) kst[i] = *reinterpret_cast<const u32x4*>(kb + min((tid >> 6) + THREADS / 64 * i, HD / 8 - 1) * PS * 8);
 #pragma unroll
-    for (int i = 0; i < V_STAGE; ++i) vst[i] = *reinterpret_cast<const u32x4*>(vb + (size_t)min((tid >> 3) + PF_THREADS / 8 * i, n_c * VD - 1) * PS);
+    for (int i = 0; i < V_STAGE; ++i) vst[i] = *reinterpret_cast<const u32x4*>(vb + (size_t)min((tid >> 3) + THREADS / 8 * i, n_c * VD - 1) * PS);
   };
-  auto stage = [&](int key0, u32x4 (&kst)[K_STAGE], u32x4 (&vst)[V_STAGE]) {
+  auto stage = [&](int key0) __attribute__((always_inline)) {
     if (!all_pages || key0 + 63 > p_max_wg || !(key0 >= lo_wg || key0 + 63 < keep)) {  // keys without values: the same for the whole workgroup
       const int page_no = block_of(key0), page_key = page_no * PS, kp = key0 + (tid & 63), vp = key0 + 8 * (tid & 7);
       int at;
@@ -436,63 +447,79 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
       for (int i = 0; i < V_STAGE; ++i) vst[i] = first_keys(vst[i], count);
     }
 #pragma unroll
-    for (int i = 0; i < K_STAGE; ++i) {
-      const int ci = tid + PF_THREADS * i;
-      if (ci < HD * 8) *reinterpret_cast<u32x4*>(ks + (size_t)ci * 8) = kst[i];
-    }
+    for (int i = 0; i < K_STAGE; ++i)
+      if (HD * 8 % THREADS == 0 || tid + THREADS * i < HD * 8) *reinterpret_cast<u32x4*>(ks_put + THREADS * 8 * i) = kst[i];
 #pragma unroll
     for (int i = 0; i < V_STAGE; ++i) {
-      const int ci = tid + PF_THREADS * i;
-      if (ci < n_c * VD * 8) *reinterpret_cast<u32x4*>(vs + (size_t)(ci >> 3) * VS_STRIDE + 8 * (ci & 7)) = vst[i];
+      const int row = (tid >> 3) + THREADS / 8 * i;
+      if ((NC == 1 && VD * 8 % THREADS == 0) || row < v_rows) *reinterpret_cast<u32x4*>(vs + ((tid & 7) * v_rows + (row ^ 2 * (tid & 7))) * 8) = vst[i];
     }
   };
 
-  fetch(lev_block_key(0, n_kept, first_block), kst_a, vst_a);
-  if (n_blocks > 1) fetch(lev_block_key(1, n_kept, first_block), kst_b, vst_b);
+  fetch(lev_block_key(0, n_kept, first_block));
   for (int it = 0; it < n_blocks; ++it) {
     const int key0 = lev_block_key(it, n_kept, first_block);
     lds_barrier();  // the block before has been read by every wave (a barrier for LDS only: the loads on their way stay there)
-    // the register sets take turns: this block's goes to LDS and is asked for again two blocks ahead (conditions uniform
-    // over the workgroup)
-    if (it & 1) {
-      stage(key0, kst_b, vst_b);
-      lds_barrier();
-      if (it + 2 < n_blocks) fetch(lev_block_key(it + 2, n_kept, first_block), kst_b, vst_b);
-    } else {
-      stage(key0, kst_a, vst_a);
-      lds_barrier();
-      if (it + 2 < n_blocks) fetch(lev_block_key(it + 2, n_kept, first_block), kst_a, vst_a);
-    }
+    stage(key0);
+    fetch(lev_block_key(min(it + 1, n_blocks - 1), n_kept, first_block));  // under no condition: behind the last the last again
+    lds_barrier();
     if (!active || key0 > p_max || (key0 + 63 < lo_min && key0 >= keep)) continue;  // none of this wave's rows sees a key of this block
+    // Four operands at a time come from LDS, two such groups ahead of the products: keys (a score tile and up to four k-steps; the tiles in turn), then values (two tiles of 16
+    // dimensions), the first of them before the softmax.
+    constexpr int KC = (NKS + 3) / 4, NGK = 4 * KC, NGV1 = (NDT + 1) / 2, NGV = NC * NGV1;
+    constexpr int D = WAVES == PF_WAVES ? 3 : 2;
+    u32x4 fr[D][4];
     f32x4 st[2][2];
+    auto read = [&](int group) __attribute__((always_inline)) {
+      u32x4 (&to)[4] = fr[group % D];
+      if (group < NGK) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const int key_row = 32 * u + 8 * (col >> 2) + 4 * hh + (col & 3);
-        f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < NKS; ++s) {
-          u32x4 kf = u32x4{0u, 0u, 0u, 0u};
-          if (HD % 32 == 0 || 32 * s + 8 * g < HD) kf = *reinterpret_cast<const u32x4*>(ks + ((size_t)(4 * s + g) * 64 + key_row) * 8);
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf), as_bf16x8(qf[s]), acc, 0, 0, 0);
+        for (int e = 0; e < 4; ++e) {
+          const int s = group / 4 * 4 + e;
+          if (s >= NKS) break;
+          const bool in = HD % 32 == 0 || 32 * s + 8 * g < HD;  // beyond: read at another place, and zeros
+          to[e] = *reinterpret_cast<const u32x4*>(ks_get + ((in ? 4 * s * 64 : 0) + 16 * (group % 4)) * 8);
+          if (!in) to[e] = u32x4{0u, 0u, 0u, 0u};
         }
-        st[u][hh] = acc;
+      } else if (group < NGK + NGV) {
+        const int c = (group - NGK) / NGV1, dt0 = (group - NGK) % NGV1 * 2;
+        const int row0 = (NC == 1 ? 0 : min(c, n_c - 1)) * VD + 16 * dt0;  // of heads beyond the last: read, not used
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (dt0 + e / 2 < NDT) to[e] = *reinterpret_cast<const u32x4*>(vs_get[e & 1] + (row0 + e / 2 * 16) * 8);
       }
+    };
+#pragma unroll
+    for (int group = 0; group < D - 1; ++group) read(group);
+#pragma unroll
+    for (int group = 0; group < NGK; ++group) {
+      read(group + D - 1);
+      __builtin_amdgcn_sched_barrier(0);
+      f32x4& acc = st[group % 4 >> 1][group & 1];
+      if (group < 4) acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (group / 4 * 4 + e < NKS) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(fr[group % D][e]), as_bf16x8(qf[group / 4 * 4 + e]), acc, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     // scale, cap, distance term; in base 2 from here on
     float mx = -INFINITY;
     const float dist0 = (float)(pos - key0 - 8 * g);  // whole numbers: exact
+    if (softcap > 0.f) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
+        for (int hh = 0; hh < 2; ++hh)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float far = dist0 - (float)(32 * u + 4 * hh + r);
-          if (softcap > 0.f) st[u][hh][r] = fmaf(-slope, far, softcap * fast_tanh(st[u][hh][r] * scale * __builtin_amdgcn_rcpf(softcap))) * LOG2E;
-          else st[u][hh][r] = fmaf(-slope, far, st[u][hh][r] * scale) * LOG2E;
-        }
-      }
+          for (int r = 0; r < 4; ++r) st[u][hh][r] = fmaf(-slope, dist0 - (float)(32 * u + 4 * hh + r), softcap * fast_tanh(st[u][hh][r] * scale * __builtin_amdgcn_rcpf(softcap))) * LOG2E;
+    } else {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) st[u][hh][r] = fmaf(-slope, dist0 - (float)(32 * u + 4 * hh + r), st[u][hh][r] * scale) * LOG2E;
+    }
     if (!all_pages || key0 + 63 > p_min || !(key0 >= lo_max || key0 + 63 < keep)) {  // a row that does not see every key: the same for the whole wave
       const int page_no = block_of(key0), page_key = page_no * PS;
 #pragma unroll
@@ -512,8 +539,13 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
       for (int hh = 0; hh < 2; ++hh)
 #pragma unroll
         for (int r = 0; r < 4; ++r) mx = fmaxf(mx, st[u][hh][r]);
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    {  // over the lanes 16, 32 and 48 further on, by the lane-swap instructions
+      typedef __attribute__((ext_vector_type(2))) uint32_t pair_t;
+      const pair_t a = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+      const pair_t b = __builtin_amdgcn_permlane16_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+    }
     const float m_new = fmaxf(m, mx);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
     const float corr = __builtin_amdgcn_exp2f(m - m_use);
@@ -536,20 +568,25 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
       for (int e = 0; e < 4; ++e) pf[u][e] = float2_to_bf16x2(p[2 * e], p[2 * e + 1]);
     }
     l = l * corr + psum;
+    if (__any(corr != 1.f)) {  // some row's maximum was raised
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      if (c == 0 || c < n_c) {
+      for (int c = 0; c < NC; ++c)
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) {
-          f32x4 acc = o[c][dt] * corr;
+        for (int dt = 0; dt < NDT; ++dt) o[c][dt] *= corr;
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const u32x4 vf = *reinterpret_cast<const u32x4*>(vs + (size_t)(c * VD + 16 * dt + col) * VS_STRIDE + 32 * u + 8 * g);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf), as_bf16x8(pf[u]), acc, 0, 0, 0);
-          }
-          o[c][dt] = acc;
-        }
-      }
+    for (int v = 0; v < NGV; ++v) {
+      const int c = v / NGV1, dt0 = v % NGV1 * 2;
+      if (NC > 1 && c > 0 && c >= n_c) break;
+      if (v + D - 1 < NGV) read(NGK + v + D - 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          if (dt0 + t < NDT) o[c][dt0 + t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(fr[(NGK + v) % D][2 * t + u]), as_bf16x8(pf[u]), o[c][dt0 + t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
   l += __shfl_xor(l, 16, 64);
@@ -672,22 +709,21 @@ extern "C" int lev_attention_values_mfma(const void* q, long q_stride, float* ou
 #define AV_ONE_WAVE(NC) 1
 #define AV_MANY_WAVES(NC) av_waves<NC>()
   if (n_tiles > 0) {
-    dim3 grid(n_tiles, H, chunks);
-    const size_t lds = ((size_t)HD * 64 + (size_t)(NV == 1 ? 1 : (NV < NVC ? NV : NVC)) * VD * VS_STRIDE) * sizeof(bf16_t);
+    const size_t lds = ((size_t)HD * 64 + (size_t)(NV == 1 ? 1 : (NV < NVC ? NV : NVC)) * VD * 64) * sizeof(bf16_t);
     // the page ids of a tile's key range (the window, or all keys so far, and the tile itself) must fit their LDS table
     long reach = window > 0 && window < max_keys ? window : max_keys;
     if (chunk > 0 && chunk < reach) reach = chunk;
     reach += PF_ROWS + 64 + (keep > 0 ? keep + 64 + PS : 0);
     const size_t all_lds = lds + RUN_PAGES * sizeof(int);
     if (all_lds > 64 * 1024 && all_lds <= RUN_MAX_LDS) {  // more than a kernel gets unasked
-      hipError_t e = hipFuncSetAttribute(NV == 1 ? (const void*)attention_values_mfma_runs_kernel<1> : (const void*)attention_values_mfma_runs_kernel<NVC>,
+      hipError_t e = hipFuncSetAttribute(NV == 1 ? (const void*)attention_values_mfma_runs_kernel<1, RUN_WAVES(1)> : (const void*)attention_values_mfma_runs_kernel<NVC, RUN_WAVES(NVC)>,
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
       LEV_REQUIRE(e == hipSuccess, "attention: %zu bytes of LDS a workgroup: %s", all_lds, hipGetErrorString(e));
     }
 #define AV_RUNS(NC)                                                                                                                                    \
-  attention_values_mfma_runs_kernel<NC><<<grid, PF_THREADS, lds, stream>>>((const bf16_t*)q, q_stride, out, (const bf16_t*)k_pages, (const bf16_t*)v_pages, \
-                                                                           positions, token_seq, block_tables, bt_stride, tiles, H, KVH, NV, PS, scale, window, \
-                                                                           chunk, keep, softcap, slopes, sinks)
+  attention_values_mfma_runs_kernel<NC, RUN_WAVES(NC)><<<dim3(n_tiles * (PF_WAVES / RUN_WAVES(NC)), H, chunks), 64 * RUN_WAVES(NC), lds, stream>>>(    \
+      (const bf16_t*)q, q_stride, out, (const bf16_t*)k_pages, (const bf16_t*)v_pages, positions, token_seq, block_tables, bt_stride, tiles, H, KVH, NV, PS, scale, window, \
+      chunk, keep, softcap, slopes, sinks)
     if (all_lds <= RUN_MAX_LDS && reach / PS + 2 <= RUN_PAGES) {
       if (NV == 1) AV_RUNS(1);
       else AV_RUNS(NVC);
