@@ -231,7 +231,8 @@ sc_inner_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
 // ---- along the runs -------------------------------------------------------------------------------------------------------------
 // One workgroup of four waves per (run, head, 16 CT value columns); wave w has the tokens 16 w .. of the block as rows of the result and a quarter
 // of the state's key channels, in accumulator registers. SSD takes up to 64 columns at once where there are many runs: what a block stages in LDS (keys, queries, weights)
-// is the same for all of them (64 heads of 128 / 64, microseconds with 16 / 64 columns: 32 runs of 40 to 150 tokens 205 / 158, but three of 300 to 999, whose chain is the bound, 62 / 100).
+// is the same for all of them (64 heads of 128 / 64, microseconds with 16 / 64 columns: 32 runs of 40 to 150 tokens 205 / 158, but three of 300 to 999, whose chain is the bound, 62 / 100; with the next block's loads kept
+// from waits - copies of registers for a branch's sake, the block's own stores - and operands read ahead of their products 57; DELTA, 16 heads, 64 / 55).
 // Runs of several tokens begin first: behind 31 single tokens, as a step has them, one of 1,000 would begin last and its chain be the end of the step (with all that stands around the kernel, 16 columns / 64 / 64 and
 // long runs first: 246 / 254 / 188; of 3,000 406 / 484 / 365; 32 of 40 to 150, in a scan that reads every slot once, 386 / 306 / 282). DELTA stays at 16: its products with two 32-bit sides are four times as long.
 template <int DKM, int RULE, bool VEC, int CT>
@@ -280,14 +281,15 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
         S[c][n][r] = live[c] && i < dk ? sp[(size_t)i * dv + jc[c]] : 0.f;
       }
 
-  // what of the next block is on its way: keys (two neighbouring tokens, eight channels), queries, values, scalars, this wave's rows of P and T.
-  // Raw loads only, under no condition: whatever is computed from them here would wait for their way through the memory.
+  // what of the next block is on its way: keys (two neighbouring tokens, eight channels), queries, values, scalars; and, once this block's have been used, this wave's rows
+  // of P and T. Raw loads only, under no condition (the last block is written out apart): whatever is computed from them here, or copied for the sake of a branch, would wait for their way
+  // through the memory.
   sc_u32x4 nk[KI][2], nq[QI];
   bf16_t nv[CT][4];
-  sc_f32x4 nP[4], nT[4];
+  sc_f32x4 P[4], T[4];
   float2 n_e = make_float2(0.f, 0.f);
   float n_w = 0.f, n_rk = 0.f, n_rq = 0.f;
-  auto fetch = [&](int tb) {
+  auto fetch = [&](int tb) __attribute__((always_inline)) {
 #pragma unroll
     for (int n = 0; n < KI; ++n) {
       const int idx = tid + 256 * n, pair = idx & 31, i0 = (idx >> 5) * 8;
@@ -306,20 +308,20 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
 #pragma unroll
       for (int c = 0; c < CT; ++c) nv[c][r] = uv[(size_t)min(t, s.Tn - 1) * s.C + jc[c]];
     }
+    const float* sc = scal + (size_t)min(tb + lane, s.Tn - 1) * n_scal;
+    n_e = E_in[((size_t)(tb / SC_Q) * s.H + h) * SC_Q + lane];
+    if (DELTA) n_w = sc[s.H + h], n_rk = sc[2 * s.H + g], n_rq = sc[2 * s.H + s.G + g];
+  };
+  auto fetch_tiles = [&](int tb) __attribute__((always_inline)) {
     const size_t tile = ((size_t)(tb / SC_Q) * s.H + h) * 10 + wave * (wave + 1) / 2;
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt) {
       const size_t at = ((tile + min(jt, wave)) * 64 + lane) * 4;
-      nP[jt] = *reinterpret_cast<const sc_f32x4*>(P_in + at);
-      if (DELTA) nT[jt] = *reinterpret_cast<const sc_f32x4*>(T_in + at);
-    }
-    if (wave == 0) {
-      const float* sc = scal + (size_t)min(tb + lane, s.Tn - 1) * n_scal;
-      n_e = E_in[((size_t)(tb / SC_Q) * s.H + h) * SC_Q + lane];
-      if (DELTA) n_w = sc[s.H + h], n_rk = sc[2 * s.H + g], n_rq = sc[2 * s.H + s.G + g];
+      P[jt] = *reinterpret_cast<const sc_f32x4*>(P_in + at);
+      if (DELTA) T[jt] = *reinterpret_cast<const sc_f32x4*>(T_in + at);
     }
   };
-  auto stage = [&](int tb) {
+  auto stage = [&](int tb) __attribute__((always_inline)) {
 #pragma unroll
     for (int n = 0; n < KI; ++n) {
       const int idx = tid + 256 * n, pair = idx & 31, i0 = (idx >> 5) * 8;
@@ -369,39 +371,48 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
     }
   };
 
-  const int first = t0 / SC_Q * SC_Q;
+  const int first = t0 / SC_Q * SC_Q, last = (t_end - 1) / SC_Q * SC_Q;
   fetch(first);
-  for (int tb = first; tb < t_end; tb += SC_Q) {
+  __builtin_amdgcn_sched_barrier(0);  // in this order, here as in the loop: rows are waited for first
+  fetch_tiles(first);
+  __builtin_amdgcn_sched_barrier(0);
+  auto block = [&](int tb, bool more) __attribute__((always_inline)) {
     float v_now[4];
-    sc_f32x4 P[4], T[4];
     stage(tb);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      v_now[r] = live[0] ? to_float<bf16_t>(nv[0][r]) : 0.f;  // DELTA
-      P[r] = nP[r];
-      if (DELTA) T[r] = nT[r];
-    }
+    for (int r = 0; r < 4; ++r) v_now[r] = live[0] ? to_float<bf16_t>(nv[0][r]) : 0.f;  // DELTA
     lds_barrier();  // the loads and stores in flight are the thread's own and are not waited for
-    if (tb + SC_Q < t_end) fetch(tb + SC_Q);
+    if (more) fetch(tb + SC_Q);
+    __builtin_amdgcn_sched_barrier(0);
 
     // rows of the result: tokens 16 wave + .. ; S0^T q and (DELTA) S0^T k, two sums each
     const sc_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     sc_f32x4 oq3[CT][3], ok3[3] = {zero, zero, zero};  // a sum for each part of the state: the longest wait in a block is for products in turn
 #pragma unroll
     for (int c = 0; c < CT; ++c) oq3[c][0] = oq3[c][1] = oq3[c][2] = zero;
+    // operands of a step of 32 channels and 16 columns, read a step ahead of their products
+    sc_u32x4 aq[2], ak[2], sb[2][3];
+    auto read = [&](int at) __attribute__((always_inline)) {
+      const int ks = at / CT, c = at % CT;
+      if (c == 0) {
+        aq[ks & 1] = sc_read16(&s_q[16 * wave + col][32 * ks + 8 * grp]);
+        if (DELTA) ak[ks & 1] = sc_read16(&s_k[DELTA ? 16 * wave + col : 0][32 * ks + 8 * grp]);
+      }
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const sc_u32x4 aq = sc_read16(&s_q[16 * wave + col][32 * ks + 8 * grp]);
-      sc_u32x4 ak;
-      if (DELTA) ak = sc_read16(&s_k[DELTA ? 16 * wave + col : 0][32 * ks + 8 * grp]);
+      for (int p = 2; p >= 0; --p) sb[at & 1][p] = sc_read16(&s_S[p][16 * c + col][32 * ks + 8 * grp]);
+    };
+    read(0);
 #pragma unroll
-      for (int c = 0; c < CT; ++c)
+    for (int at = 0; at < KS * CT; ++at) {
+      const int ks = at / CT, c = at % CT;
+      if (at + 1 < KS * CT) read(at + 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int p = 2; p >= 0; --p) {
-          const sc_u32x4 b = sc_read16(&s_S[p][16 * c + col][32 * ks + 8 * grp]);
-          oq3[c][p] = sc_mfma(aq, b, oq3[c][p]);
-          if (DELTA) ok3[p] = sc_mfma(ak, b, ok3[p]);
-        }
+      for (int p = 2; p >= 0; --p) {
+        oq3[c][p] = sc_mfma(aq[ks & 1], sb[at & 1][p], oq3[c][p]);
+        if (DELTA) ok3[p] = sc_mfma(ak[ks & 1], sb[at & 1][p], ok3[p]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
     sc_f32x4 oq[CT];
 #pragma unroll
@@ -500,15 +511,23 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
         }
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
+    if (more) fetch_tiles(tb + SC_Q);
+    // through a buffer of the wave's 16 rows, beyond whose end nothing is written: a branch round a store makes the next block's loads wait for it
+    const auto rows = __builtin_amdgcn_make_buffer_rsrc(o + (size_t)(tb + 16 * wave) * s.H * dv, 0, 16 * s.H * dv * (int)sizeof(float), 0x00027000);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int t = tb + 16 * wave + 4 * grp + r;
+      const int t = 4 * grp + r, at = tb + 16 * wave + t;
+      const bool in = at >= t0 && at < t_end;
 #pragma unroll
       for (int c = 0; c < CT; ++c)
-        if (live[c] && t >= t0 && t < t_end) o[((size_t)t * s.H + h) * dv + j + 16 * c] = oq[c][r];
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(oq[c][r]), rows, in && live[c] ? ((t * s.H + h) * dv + j + 16 * c) * (int)sizeof(float) : 0x7ffffff0, 0, 0);
     }
     lds_barrier();  // the block's tiles have been read by every wave
-  }
+  };
+  int tb = first;
+  for (; tb < last; tb += SC_Q) block(tb, true);
+  block(last, false);
 #pragma unroll
   for (int c = 0; c < CT; ++c)
     if (live[c]) {
@@ -528,6 +547,7 @@ int sr_chunks_launch(int rule, const bf16_t* u, const float* scal, float* state,
                      const SrShape& s, hipStream_t stream) {
   const int vec = s.C % 8 == 0 && s.dk % 8 == 0 && s.k_off % 8 == 0 && s.q_off % 8 == 0 && ((uintptr_t)u & 15) == 0;
   const int n_blocks = (s.Tn + SC_Q - 1) / SC_Q;
+  LEV_REQUIRE((long)s.H * s.dv < (1L << 25), "state recurrence: rows of %ld numbers are too long", (long)s.H * s.dv);
   LEV_REQUIRE(max_runs <= 65535 && n_blocks <= 65535 && ((uintptr_t)workspace & 15) == 0, "state recurrence: too many runs (%d) or tokens (%d)", max_runs, s.Tn);
   float* P = workspace;
   float* T = workspace + (size_t)n_blocks * s.H * 10 * 256;
