@@ -41,7 +41,7 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
   constexpr int DT = HD / 16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, g = lane >> 4;
   const int group = H / KVH, nc = RUNS ? 16 : columns;
-  int token, head;
+  int token, head, pos, seq;
   bool mine;  // this lane's column is one
   if (RUNS) {
     const int subs = (tile_rows + 15) / 16;
@@ -51,23 +51,27 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
     if (rows <= 0) return;  // the whole workgroup
     mine = col < rows;
     token = first + 16 * sub + min(col, rows - 1);
+    pos = positions[token], seq = token_seq[token];
   } else {
     const int sets = (group + 15) / 16, kvh = blockIdx.x / sets % KVH, set = blockIdx.x % sets;
-    token = work[blockIdx.x / sets / KVH];
+    // which token, its position and its row in one trip: the i-th single token of a step is mostly its i-th token, and if not they are asked for again
+    const int i = blockIdx.x / sets / KVH;
+    token = work[i], pos = positions[i], seq = token_seq[i];
+    if (token != i) pos = positions[token], seq = token_seq[token];
     const int n = min(16, group - 16 * set);
     mine = col < n;
     head = kvh * group + 16 * set + min(col, n - 1);
   }
   const int kvh = head / group;
-  const int pos = positions[token];
   const int first = p.window > 0 ? max(0, pos - p.window + 1) : 0;
   int last = pos, lo = first;  // over the columns
+  if (RUNS)
 #pragma unroll
-  for (int o = 8; o > 0; o >>= 1) {
-    last = max(last, __shfl_xor(last, o, 64));
-    lo = min(lo, __shfl_xor(lo, o, 64));
-  }
-  const int* bt = block_tables + (size_t)token_seq[token] * bt_stride;
+    for (int o = 8; o > 0; o >>= 1) {
+      last = max(last, __shfl_xor(last, o, 64));
+      lo = min(lo, __shfl_xor(lo, o, 64));
+    }
+  const int* bt = block_tables + (size_t)seq * bt_stride;
   const size_t head_elems = (size_t)HD * PS;
   const float* qr = p.q + (size_t)token * p.q_stride + (size_t)head * HD;
   af_f32x4 q[DT], o_acc[DT];

@@ -74,7 +74,7 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
                              float* __restrict__ part_o, float* __restrict__ part_ml, const float* __restrict__ sinks) {
   const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
   const int group = H / KVH;
-  int tok = 0, head = 0, kvh = 0;
+  int tok = 0, head = 0, kvh = 0, pos, seq;
   bool valid;
   if (SINGLE) {
     const int col_sets = (group + 15) / 16;
@@ -82,7 +82,10 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
     const int c = (blockIdx.y % col_sets) * 16 + col;
     valid = c < group;
     head = kvh * group + (valid ? c : 0);
-    tok = work[WAVES > 1 ? blockIdx.x : blockIdx.x / splits];
+    // which token, its position and its row in one trip: the i-th single token of a step is mostly its i-th token, and if not they are asked for again
+    const int i = WAVES > 1 ? blockIdx.x : blockIdx.x / splits;
+    tok = work[i], pos = positions[i], seq = token_seq[i];
+    if (tok != i) pos = positions[tok], seq = token_seq[tok];
   } else {
     const int tile = blockIdx.x / SUB_TILES, sub = blockIdx.x % SUB_TILES;
     const int first = work[2 * tile], n = work[2 * tile + 1];
@@ -91,17 +94,18 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
     kvh = head / group;
     valid = sub * 16 + col < n;
     tok = first + (valid ? sub * 16 + col : sub * 16);
+    pos = positions[tok], seq = token_seq[tok];
   }
-  const int pos = positions[tok];
   const int lo = lev_first_visible(pos, window, chunk);
-  // the wave's range of keys; every column belongs to the same request
-  int p_max = valid ? pos : -1, lo_min = valid ? lo : 0x7fffffff;
+  // the wave's range of keys; every column belongs to the same request, those of a single token to one position
+  int p_max = SINGLE || valid ? pos : -1, lo_min = SINGLE || valid ? lo : 0x7fffffff;
+  if (!SINGLE)
 #pragma unroll
-  for (int o = 8; o > 0; o >>= 1) {
-    p_max = max(p_max, __shfl_xor(p_max, o, 64));
-    lo_min = min(lo_min, __shfl_xor(lo_min, o, 64));
-  }
-  const int* bt = block_tables + (size_t)token_seq[tok] * bt_stride;
+    for (int o = 8; o > 0; o >>= 1) {
+      p_max = max(p_max, __shfl_xor(p_max, o, 64));
+      lo_min = min(lo_min, __shfl_xor(lo_min, o, 64));
+    }
+  const int* bt = block_tables + (size_t)seq * bt_stride;
   const float slope = slopes ? slopes[head] : 0.f;
   const int c0 = NV == 1 ? kvh : blockIdx.z * NC;              // first value head of this wave
   const int n_c = NV == 1 ? 1 : min(NC, NV - blockIdx.z * NC);  // and how many
