@@ -69,7 +69,7 @@ template <bool SINGLE, int NC, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES)
 attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float* __restrict__ out, const bf16_t* __restrict__ k_pages,
                              const bf16_t* __restrict__ v_pages, const int* __restrict__ positions, const int* __restrict__ token_seq,
-                             const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ work, int H, int KVH, int NV,
+                             const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ work, int n_positions, int H, int KVH, int NV,
                              int PS, float scale, int window, int chunk, int keep, float softcap, const float* __restrict__ slopes, int splits,
                              float* __restrict__ part_o, float* __restrict__ part_ml, const float* __restrict__ sinks) {
   const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
@@ -83,9 +83,9 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
     valid = c < group;
     head = kvh * group + (valid ? c : 0);
     // which token, its position and its row in one trip: the i-th single token of a step is mostly its i-th token, and if not they are asked for again
-    const int i = WAVES > 1 ? blockIdx.x : blockIdx.x / splits;
-    tok = work[i], pos = positions[i], seq = token_seq[i];
-    if (tok != i) pos = positions[tok], seq = token_seq[tok];
+    const int i = WAVES > 1 ? blockIdx.x : blockIdx.x / splits, guess = min(i, n_positions - 1);
+    tok = work[i], pos = positions[guess], seq = token_seq[guess];
+    if (tok != guess) pos = positions[tok], seq = token_seq[tok];
   } else {
     const int tile = blockIdx.x / SUB_TILES, sub = blockIdx.x % SUB_TILES;
     const int first = work[2 * tile], n = work[2 * tile + 1];
@@ -671,7 +671,7 @@ extern "C" long lev_attention_values_mfma_workspace(int n_singles, int splits, i
 
 extern "C" int lev_attention_values_mfma(const void* q, long q_stride, float* out, const void* k_pages, const void* v_pages,
                                          const int* positions, const int* token_seq, const int* block_tables, int bt_stride,
-                                         const int* tiles, int n_tiles, const int* singles, int n_singles, int H, int KVH, int HD_,
+                                         const int* tiles, int n_tiles, const int* singles, int n_singles, int n_positions, int H, int KVH, int HD_,
                                          int VD_, int NV, int PS, float scale, int window, int chunk, int keep, float softcap, const float* slopes,
                                          const float* sinks, int splits, float* workspace, int max_keys, hipStream_t stream) {
   LEV_REQUIRE(HD_ == HD && VD_ == VD, "attention: this library was built for head sizes %d / %d, not %d / %d", HD, VD, HD_, VD_);
@@ -682,7 +682,7 @@ extern "C" int lev_attention_values_mfma(const void* q, long q_stride, float* ou
   LEV_REQUIRE(splits >= 1 && splits <= MERGE_MAX_SPLITS, "attention: %d splits (at most %d)", splits, MERGE_MAX_SPLITS);
   const bool merged = n_singles > 0 && av_merged(n_singles, splits, H, KVH, NV, window, chunk, keep, max_keys);
   LEV_REQUIRE(splits == 1 || merged || workspace, "attention: %d splits (at most %d) need scratch memory", splits, MERGE_MAX_SPLITS);
-  LEV_REQUIRE(n_tiles >= 0 && n_singles >= 0 && (n_tiles == 0 || tiles) && (n_singles == 0 || singles), "attention: bad work lists");
+  LEV_REQUIRE(n_tiles >= 0 && n_singles >= 0 && (n_tiles == 0 || tiles) && (n_singles == 0 || (singles && n_positions > 0)), "attention: bad work lists");
   LEV_REQUIRE(((uintptr_t)q & 15) == 0 && q_stride % 8 == 0 && ((uintptr_t)k_pages & 15) == 0 && ((uintptr_t)v_pages & 15) == 0 &&
                   ((uintptr_t)out & 15) == 0,
               "attention: operands must be 16-byte aligned");
@@ -698,7 +698,7 @@ extern "C" int lev_attention_values_mfma(const void* q, long q_stride, float* ou
         LEV_REQUIRE(e == hipSuccess, "attention: %zu bytes of LDS a workgroup: %s", lds, hipGetErrorString(e));                                         \
       }                                                                                                                                                 \
       attention_values_mfma_kernel<SINGLE, NC, WAVES><<<GRID, WAVES > 1 ? 64 * SPLITS : 64, lds, stream>>>(                                             \
-          (const bf16_t*)q, q_stride, out, (const bf16_t*)k_pages, (const bf16_t*)v_pages, positions, token_seq, block_tables, bt_stride, WORK, H, KVH, \
+          (const bf16_t*)q, q_stride, out, (const bf16_t*)k_pages, (const bf16_t*)v_pages, positions, token_seq, block_tables, bt_stride, WORK, n_positions, H, KVH, \
           NV, PS, scale, window, chunk, keep, softcap, slopes, SPLITS, PART_O, PART_ML, sinks);                                                         \
     }
 #define AV_NO_LDS(NC) 0

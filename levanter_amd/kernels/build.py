@@ -92,7 +92,7 @@ def attention_values_unit(head_dim: int, value_dim: int) -> str:
         if head_dim % 16 or value_dim % 16 or not (16 <= head_dim <= 256 and 16 <= value_dim <= 256):
             raise ValueError(f"no matrix-core attention for head sizes {head_dim} / {value_dim}")
         register_unit(name, [("attention_values_mfma.hip", [f"-DLEV_HD={head_dim}", f"-DLEV_VD={value_dim}"], f"attention_values_mfma_hd{head_dim}_vd{value_dim}.o")],
-                      signatures={"lev_attention_values_mfma": [_P, _L, _P, _P, _P, _P, _P, _P, _I, _P, _I, _P, _I] + [_I] * 6 + [_F, _I, _I, _I, _F, _P, _P, _I, _P, _I, _P],
+                      signatures={"lev_attention_values_mfma": [_P, _L, _P, _P, _P, _P, _P, _P, _I, _P, _I, _P, _I] + [_I] * 7 + [_F, _I, _I, _I, _F, _P, _P, _I, _P, _I, _P],
                                   "lev_attention_values_mfma_workspace": [_I] * 9})
     return name
 
@@ -335,7 +335,7 @@ register_unit("core", ["errors.hip", "elementwise.hip", "layer_ops.hip", "gemm_s
     "lev_linear_f32_normed_takes": [_I, _I, _I],
     "lev_linear_simple": [_P, _L, _P, _P, _P, _L, _P, _L] + [_I] * 6 + [_P],
     "lev_attention_simple": [_P, _L, _P, _L, _P, _P, _P, _P, _P] + [_I] * 6 + [_F, _I, _I, _F, _P, _I, _P],
-    "lev_attention_f32": [_P, _L, _P, _L, _P, _P, _P, _P, _P, _I, _P, _I, _I, _P, _I, _P, _P, _L, _P] + [_I] * 4 + [_F, _I, _F, _P, _I, _P],
+    "lev_attention_f32": [_P, _L, _P, _L, _P, _P, _P, _P, _P, _I, _P, _I, _I, _P, _I, _I, _P, _P, _L, _P] + [_I] * 4 + [_F, _I, _F, _P, _I, _P],
     "lev_attention_mfma_workspace": [_I] * 5,
 })
 register_unit("gemm_mfma", ["gemm_mfma.hip", "gemm_ring.hip", "gemm_norm.hip"], signatures={

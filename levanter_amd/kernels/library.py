@@ -799,7 +799,7 @@ class HipKernels:
             self._check(lib.lev_attention_values_mfma(
                 _ptr(q), _rows(q, "attention_values: q"), _ptr(out), _ptr(k_pages), _ptr(v_pages), _ptr(meta.positions), _ptr(meta.token_seq),
                 _ptr(block_tables), block_tables.shape[1], _ptr(meta.prefill_tiles), meta.n_prefill_tiles, _ptr(meta.decode_tokens),
-                meta.n_decode, n_heads, n_kv_heads, head_dim, value_dim, nv, page_size, float(scale), int(window) if window else 0,
+                meta.n_decode, T, n_heads, n_kv_heads, head_dim, value_dim, nv, page_size, float(scale), int(window) if window else 0,
                 int(chunk) if chunk else 0, int(keep_first), float(softcap) if softcap else 0.0, _ptr(slopes), _ptr(sinks), splits, _ptr(ws), int(meta.max_kv_len), self._s()))
             return
         self._check(self.lib.lev_attention_values(
@@ -1395,7 +1395,7 @@ class HipKernels:
             return k_new is not None
         if dt == torch.float32:
             rc = self.lib.lev_attention_f32(_ptr(q), qs, _ptr(out), os_, _ptr(k_pages), _ptr(v_pages), pos_ptr, seq_ptr, bt_ptr, bt_width, tiles_ptr,
-                                            meta.n_prefill_tiles, self.prefill_tile_rows, decode_ptr, meta.n_decode, _ptr(k_new), _ptr(v_new), kvs,
+                                            meta.n_prefill_tiles, self.prefill_tile_rows, decode_ptr, meta.n_decode, T, _ptr(k_new), _ptr(v_new), kvs,
                                             _ptr(dest) if k_new is not None else None, n_heads, n_kv_heads, head_dim, page_size,
                                             float(scale), w, cap, _ptr(score_bias), bias_len, self._s())
             if rc <= 0:
