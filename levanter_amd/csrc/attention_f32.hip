@@ -6,8 +6,10 @@
 //
 // A workgroup of W waves owns 16 columns: 16 consecutive query rows of one head (runs of several tokens), or up to 16 query heads of one
 // key/value head (single tokens). Its waves take the blocks of 16 KB keys in turn and merge through LDS in wave order.
-// What bounds it: prompts, the matrix pipe half of the time and the round trips between its batches the rest (777 rows of 16 heads of 64:
-// 35 us, 1.2 GFLOP of visible products); single tokens, the chain of one block's loads, products and merge (4 tokens of 12 heads over
+// What bounds it: prompts, the vector instructions and round trips between a block's two products, and the waves there are to fill the matrix pipe meanwhile:
+// blocks of 16 keys (KB = 1) leave registers for three waves on a SIMD at head size 64 and two at 128, where blocks of 64 and 32 keys left two and one, and a
+// prompt's last keys fill them better (777 rows of 16 heads of 64, 1.2 GFLOP of visible products: 35.0 -> 25.4 us; 4 x 777 rows: 106 -> 81; 8 key/value
+// heads of 128, 4 x 777 rows: 225 -> 152; the next block's keys and values loaded ahead take the registers instead: 54 us at 777 rows); single tokens, the chain of one block's loads, products and merge (4 tokens of 12 heads over
 // 200 keys: 9.6 us). The plain kernel gives a wave one query row, reads keys 4 bytes at a time and walks the values key by key:
 // 1,187 us and 70 us. A step of single tokens alone brings its new keys and values along: the wave whose keys they are takes them from the projection's output, and
 // the wave behind it, which has none in a short context, writes them to their page; the kernel that wrote them first took 4 us a layer (GPT-2 small, 4 requests of
@@ -31,8 +33,18 @@ struct AttentionF32Args {
   const int* dest;  // where they go, by token: page * PS + offset
 };
 
+// over the four lanes of a column, neighbouring groups of 16 first; register swaps, where the shuffles of two numbers would wait for LDS four times a block
+template <class Op>
+static __device__ __forceinline__ float af_over_groups(float v, Op op) {
+  typedef __attribute__((ext_vector_type(2))) unsigned pair_t;
+  const pair_t a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);  // {groups 0 0 2 2, groups 1 1 3 3}
+  v = op(__uint_as_float(a.x), __uint_as_float(a.y));
+  const pair_t b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);  // {lower half twice, upper half twice}
+  return op(__uint_as_float(b.x), __uint_as_float(b.y));
+}
+
 template <int HD, int KB, int W, bool RUNS>
-__global__ void __launch_bounds__(64 * W)
+__global__ void __launch_bounds__(64 * W, RUNS ? 8 / W : 1)  /* runs: two waves on a SIMD, all they need are 137 registers at head size 64 and 256 at 128 */
 attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows) per tile of the list; single tokens: their indexes
                      const int* __restrict__ positions, const int* __restrict__ token_seq, const int* __restrict__ block_tables, int bt_stride, int H, int KVH, int PS,
                      int tile_rows, int columns, int n_positions,  // rows of a tile of the list (runs); columns in use (single tokens: query heads of a key/value head, at most 16)
@@ -136,6 +148,15 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
 #pragma unroll
         for (int e = 0; e < 4; ++e) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[t][d][e], q[d][e], s[t], 0, 0, 0);
     }
+    if (p.score_bias || p.softcap > 0.f) {
+#pragma unroll
+      for (int t = 0; t < KB; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (p.score_bias) s[t][r] += p.score_bias[(size_t)head * p.bias_len + min(max(pos - (t0 + t) * 16 - 4 * g - r, 0), p.bias_len - 1)];
+          if (p.softcap > 0.f) s[t][r] = p.softcap * tanhf(s[t][r] / p.softcap);
+        }
+    }
     float mx = -INFINITY;
     bool masked = false;  // some column does not see some key of the block
 #pragma unroll
@@ -143,16 +164,12 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int key = (t0 + t) * 16 + 4 * g + r;
-        float x = s[t][r];
-        if (p.score_bias) x += p.score_bias[(size_t)head * p.bias_len + min(max(pos - key, 0), p.bias_len - 1)];
-        if (p.softcap > 0.f) x = p.softcap * tanhf(x / p.softcap);
         const bool live = key <= pos && key >= first && page[t] >= 0;
         masked |= !live;
-        s[t][r] = live ? x : -INFINITY;
+        s[t][r] = live ? s[t][r] : -INFINITY;
         mx = fmaxf(mx, s[t][r]);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = af_over_groups(mx, [](float a, float b) { return fmaxf(a, b); });
     const float m_new = fmaxf(m, mx);
     const float corr = m == -INFINITY ? 0.f : expf(m - m_new);
     float sum = 0.f;
@@ -164,8 +181,7 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
         s[t][r] = e;
         sum += e;
       }
-    sum += __shfl_xor(sum, 16, 64);
-    sum += __shfl_xor(sum, 32, 64);
+    sum = af_over_groups(sum, [](float a, float b) { return a + b; });
     l = l * corr + sum;
     m = m_new;
 #pragma unroll
@@ -260,15 +276,31 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
   }
 }
 
+template <int HD, int W>
+static int attention_f32_runs(const AttentionF32Args& p, const int* positions, const int* token_seq, const int* block_tables, int bt_stride, int H, int KVH, int PS,
+                              const int* tiles, long blocks, int tile_rows, int n_positions, hipStream_t stream) {
+  constexpr int lds = W * (HD / 16) * 4 * 16 * 16 + 2 * W * 16 * 4 + W * 1024;
+  if (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute((const void*)attention_f32_kernel<HD, 1, W, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    LEV_REQUIRE(e == hipSuccess, "attention: %d bytes of LDS a workgroup: %s", lds, hipGetErrorString(e));
+  }
+  attention_f32_kernel<HD, 1, W, true><<<(unsigned)blocks, 64 * W, lds, stream>>>(tiles, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tile_rows, 16, n_positions, p);
+  return 0;
+}
+
 template <int HD>
 static int attention_f32_launch(const AttentionF32Args& p, const int* positions, const int* token_seq, const int* block_tables, int bt_stride, int H, int KVH, int PS,
                                 const int* tiles, int n_tiles, int tile_rows, const int* tokens, int n_tokens, int n_positions, hipStream_t stream) {
-  constexpr int DT = HD / 16, KB = HD <= 64 ? 4 : 2, KB1 = HD <= 96 ? 2 : 1;  // as many tiles of keys as fit the registers
+    constexpr int DT = HD / 16, KB1 = HD <= 96 ? 2 : 1;  // single tokens: as many tiles of keys as fit the registers
   if (n_tiles > 0) {
-    constexpr int W = 4, lds = W * DT * 4 * 16 * 16 + 2 * W * 16 * 4 + W * 1024;
     const long blocks = (long)n_tiles * ((tile_rows + 15) / 16) * H;
     LEV_REQUIRE(blocks <= 0x7fffffffL, "attention: too many tiles (%ld)", blocks);
-    attention_f32_kernel<HD, KB, W, true><<<(unsigned)blocks, 64 * W, lds, stream>>>(tiles, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tile_rows, 16, n_positions, p);
+    // Eight waves a workgroup up to one and a half for a CU (not all rows of a tile are there): the keys are then walked in half the steps (65 rows behind 935 keys, 16 heads of 64: 21.2 us
+    // with four, 18.8 with eight; 256 rows, 12 heads: 8.3 and 8.1; 3 x 64 rows, 16 heads of 128: 8.8 and 7.2; 500 rows, 8 heads of 32: 10.1 and 8.8). With more of them the merges cost more than that
+    // (777 rows, 16 heads of 64: 25.4 and 31.3; 300 + 500 rows, 16 heads of 112: 28.7 and 36.4).
+    const int rc = blocks <= 384 ? attention_f32_runs<HD, 8>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tiles, blocks, tile_rows, n_positions, stream)
+                                 : attention_f32_runs<HD, 4>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tiles, blocks, tile_rows, n_positions, stream);
+    if (rc) return rc;
   }
   if (n_tokens > 0) {
     constexpr int W = 8;  // at most 256 registers a lane: head size 128 keeps 52 bytes of them in scratch memory

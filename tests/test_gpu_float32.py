@@ -236,6 +236,13 @@ def test_attention_float32(K, H, KVH, HD, PS, runs, window):
         torch.testing.assert_close(got.cpu().double(), want, rtol=2e-5, atol=2e-5)
 
 
+# runs in workgroups of four waves: more than 384 of them (tiles x 8 x heads) at every head size; key ranges that end and begin inside, at and behind a wave's block of 16
+@pytest.mark.parametrize("HD", range(16, 129, 16))
+@pytest.mark.parametrize("window", [None, 33])
+def test_attention_float32_of_many_heads(K, HD, window):
+    test_attention_float32(K, 32, 8, HD, 16, [(15, 63), (33, 64), (17, 81), (1, 40)], window)
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 def test_attention_float32_values_that_are_not_seen_do_not_count(K, bad):
     """Token 20's value is not a number: queries before it are what they are without it, the ones from it on carry it. A single token whose block
