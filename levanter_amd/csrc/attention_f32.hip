@@ -44,7 +44,7 @@ static __device__ __forceinline__ float af_over_groups(float v, Op op) {
 }
 
 template <int HD, int KB, int W, bool RUNS>
-__global__ void __launch_bounds__(64 * W, RUNS ? 8 / W : 1)  /* runs: two waves on a SIMD, all they need are 137 registers at head size 64 and 256 at 128 */
+__global__ void __launch_bounds__(64 * W, 8 / W)  /* two waves on a SIMD, runs need 137 registers at head size 64 and 256 at 128 */
 attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows) per tile of the list; single tokens: their indexes
                      const int* __restrict__ positions, const int* __restrict__ token_seq, const int* __restrict__ block_tables, int bt_stride, int H, int KVH, int PS,
                      int tile_rows, int columns, int n_positions,  // rows of a tile of the list (runs); columns in use (single tokens: query heads of a key/value head, at most 16)
@@ -87,11 +87,13 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
   const int* bt = block_tables + (size_t)seq * bt_stride;
   const size_t head_elems = (size_t)HD * PS;
   const float* qr = p.q + (size_t)token * p.q_stride + (size_t)head * HD;
-  af_f32x4 q[DT], o_acc[DT];
+  constexpr int SUMS = !RUNS && W == 4 ? KB : 1;  // four waves have longer chains of sums than eight: a tile of a block to each keeps their roundings
+  af_f32x4 q[DT], o_acc[SUMS][DT];
 #pragma unroll
   for (int d = 0; d < DT; ++d) {
     q[d] = *reinterpret_cast<const af_f32x4*>(qr + 16 * d + 4 * g) * p.scale;
-    o_acc[d] = af_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int a = 0; a < SUMS; ++a) o_acc[a][d] = af_f32x4{0.f, 0.f, 0.f, 0.f};
   }
   float* ml = af_lds + (size_t)W * DT * 4 * nc * 4;
   float* weights = ml + 2 * W * 16 + wave * 256;
@@ -185,7 +187,9 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
     l = l * corr + sum;
     m = m_new;
 #pragma unroll
-    for (int d = 0; d < DT; ++d) o_acc[d] *= corr;
+    for (int a = 0; a < SUMS; ++a)
+#pragma unroll
+      for (int d = 0; d < DT; ++d) o_acc[a][d] *= corr;
     const bool any_masked = __any(masked);
 #pragma unroll
     for (int t = 0; t < KB; ++t) {
@@ -221,7 +225,7 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
                 asm volatile("" : "+v"(row));  // one address, moved on: the compiler would keep one for each of the sums
-                if (live) o_acc[d][e] = fmaf(weight, *row, o_acc[d][e]);
+                if (live) o_acc[t % SUMS][d][e] = fmaf(weight, *row, o_acc[t % SUMS][d][e]);
                 row += e < 3 ? next : 13 * next;
               }
           }
@@ -232,8 +236,12 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
 #pragma unroll
       for (int d = 0; d < DT; ++d)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o_acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][d][e], s[t][e], o_acc[d], 0, 0, 0);
+        for (int e = 0; e < 4; ++e) o_acc[t % SUMS][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][d][e], s[t][e], o_acc[t % SUMS][d], 0, 0, 0);
     }
+  }
+  if (SUMS == 2) {
+#pragma unroll
+    for (int d = 0; d < DT; ++d) o_acc[0][d] += o_acc[SUMS - 1][d];
   }
   // the new key and value go to their page: read by later steps only. By the wave behind the one with the last keys, which has none where there are few
   if (!RUNS && to >= 0 && blockIdx.x % ((group + 15) / 16) == 0 && wave == ((t_last - lo / 16) / KB + 1) % W) {
@@ -247,7 +255,7 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
   }
   if (col < nc) {
 #pragma unroll
-    for (int d = 0; d < DT; ++d) *reinterpret_cast<af_f32x4*>(af_lds + ((size_t)((wave * DT + d) * 4 + g) * nc + col) * 4) = o_acc[d];
+    for (int d = 0; d < DT; ++d) *reinterpret_cast<af_f32x4*>(af_lds + ((size_t)((wave * DT + d) * 4 + g) * nc + col) * 4) = o_acc[0][d];
   }
   if (g == 0) ml[wave * 16 + col] = m, ml[(W + wave) * 16 + col] = l;
   __syncthreads();
@@ -288,6 +296,19 @@ static int attention_f32_runs(const AttentionF32Args& p, const int* positions, c
   return 0;
 }
 
+template <int HD, int KB, int W>
+static int attention_f32_singles(const AttentionF32Args& p, const int* positions, const int* token_seq, const int* block_tables, int bt_stride, int H, int KVH, int PS,
+                                 const int* tokens, long blocks, int n_positions, hipStream_t stream) {
+  const int group = H / KVH, columns = group < 16 ? group : 16;
+  const int lds = W * (HD / 16) * 4 * columns * 16 + 2 * W * 16 * 4 + W * 1024;
+  if (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute((const void*)attention_f32_kernel<HD, KB, W, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    LEV_REQUIRE(e == hipSuccess, "attention: %d bytes of LDS a workgroup: %s", lds, hipGetErrorString(e));
+  }
+  attention_f32_kernel<HD, KB, W, false><<<(unsigned)blocks, 64 * W, lds, stream>>>(tokens, positions, token_seq, block_tables, bt_stride, H, KVH, PS, 0, columns, n_positions, p);
+  return 0;
+}
+
 template <int HD>
 static int attention_f32_launch(const AttentionF32Args& p, const int* positions, const int* token_seq, const int* block_tables, int bt_stride, int H, int KVH, int PS,
                                 const int* tiles, int n_tiles, int tile_rows, const int* tokens, int n_tokens, int n_positions, hipStream_t stream) {
@@ -303,16 +324,17 @@ static int attention_f32_launch(const AttentionF32Args& p, const int* positions,
     if (rc) return rc;
   }
   if (n_tokens > 0) {
-    constexpr int W = 8;  // at most 256 registers a lane: head size 128 keeps 52 bytes of them in scratch memory
-    const int group = H / KVH, sets = (group + 15) / 16, columns = group < 16 ? group : 16;
-    const int lds = W * DT * 4 * columns * 16 + 2 * W * 16 * 4 + W * 1024;
+    const int sets = (H / KVH + 15) / 16;
     const long blocks = (long)n_tokens * KVH * sets;
     LEV_REQUIRE(blocks <= 0x7fffffffL, "attention: too many single tokens (%ld)", blocks);
-    if (lds > 64 * 1024) {
-      const hipError_t e = hipFuncSetAttribute((const void*)attention_f32_kernel<HD, KB1, W, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-      LEV_REQUIRE(e == hipSuccess, "attention: %d bytes of LDS a workgroup: %s", lds, hipGetErrorString(e));
-    }
-    attention_f32_kernel<HD, KB1, W, false><<<(unsigned)blocks, 64 * W, lds, stream>>>(tokens, positions, token_seq, block_tables, bt_stride, H, KVH, PS, 0, columns, n_positions, p);
+    // Eight waves use up a CU's registers, so that a grid of more workgroups than CUs came in rounds; four leave room for two workgroups (24 tokens of 12 heads of 64
+    // over 150 keys: 16.9 -> 13.0 us; 16 of 25 over 200: 19.0 -> 15.7; 32 of 25 over 1,000: 96.9 -> 88.0; 64 of 16 heads of 96 over 200: 51.8 -> 42.2; 64 of 12 over
+    // 600: level). With no more workgroups than CUs the shorter walk over the keys is the better one (20 of 12 over 150: 10.3 and 11.3; 2 of 12 over 1,000: 20.2 and
+    // 26.7). Head sizes of 112 and 128 have no registers for a second set of sums, without which four waves' error is 2 - 15 % larger.
+    const bool four = KB1 == 2 && blocks > 256;
+    const int rc = four ? attention_f32_singles<HD, KB1, KB1 == 2 ? 4 : 8>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tokens, blocks, n_positions, stream)
+                        : attention_f32_singles<HD, KB1, 8>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tokens, blocks, n_positions, stream);
+    if (rc) return rc;
   }
   return lev_check_launch("attention (32-bit)");
 }

@@ -243,6 +243,13 @@ def test_attention_float32_of_many_heads(K, HD, window):
     test_attention_float32(K, 32, 8, HD, 16, [(15, 63), (33, 64), (17, 81), (1, 40)], window)
 
 
+# single tokens in workgroups of four waves (head sizes up to 96): more than 256 of them (tokens x key/value heads); key ranges of less than a wave's block of 32 keys to several rounds
+@pytest.mark.parametrize("HD", range(16, 97, 16))
+@pytest.mark.parametrize("window", [None, 50])
+def test_attention_float32_of_many_single_tokens(K, HD, window):
+    test_attention_float32(K, 16, 16, HD, 16, [(1, n) for n in (1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 160, 161, 255, 300)], window)
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 def test_attention_float32_values_that_are_not_seen_do_not_count(K, bad):
     """Token 20's value is not a number: queries before it are what they are without it, the ones from it on carry it. A single token whose block

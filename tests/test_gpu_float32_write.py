@@ -41,3 +41,9 @@ def test_written_on_the_way(K, H, KVH, HD, PS, lens, window, odd):
     assert K.paged_attention(q, out2, k2, v2, meta, k_new=k, v_new=v, dest=dest, **args) is True
     torch.testing.assert_close(out2, out1, rtol=0, atol=0, equal_nan=True)
     assert torch.equal(k1.view(torch.int32), k2.view(torch.int32)) and torch.equal(v1.view(torch.int32), v2.view(torch.int32))
+
+
+@pytest.mark.parametrize("odd", [False, True])
+def test_written_on_the_way_by_four_waves(K, odd):
+    """More than 256 workgroups have four waves each: the one behind the last keys' wave is the writer, also where that is the first again."""
+    test_written_on_the_way(K, 16, 16, 64, 16, [1, 5, 31, 32, 33, 64, 65, 96, 97, 127, 128, 129, 160, 161, 255, 256, 300], None, odd)
