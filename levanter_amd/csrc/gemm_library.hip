@@ -7,7 +7,7 @@
 // runs the hand-written kernel. Which of the library's kernels runs a shape is not left to its heuristic alone: for
 // 256 rows and more the heuristic's candidates are timed once (its first choice is up to twice slower than its best on row
 // counts that are no multiple of the tile, 2,052 rows for instance); the other row counts up to the same multiple of 64 try
-// only that kernel against the heuristic's first. In the library's column-major terms the row-major problem is
+// only that kernel against the heuristic's first, where that cannot change the result. In the library's column-major terms the row-major problem is
 //   D^T [N x M] = w_cm^T [N x K] . a_cm [K x M]  (+ C^T),  with w_cm = w seen as K x N (ld K), a_cm = a seen as K x M (ld lda),
 // so that the bias, one value per row of D^T, is the per-output-column bias of the row-major result.
 #include <hipblaslt/hipblaslt.h>
@@ -126,8 +126,21 @@ int tune_level() {
 }
 
 // A buffer larger than the caches (32 MB of L2, 256 MB behind them), one per device, kept for the life of the process:
-// sweeping it between two timed runs leaves nothing of the operands in a cache.
+// sweeping it between two timed runs leaves nothing of the operands in a cache. It holds pairs of bfloat16 numbers of either sign, 1/4 to 4, all bits
+// of which vary: operands, too, on which the kernels' sums are told apart.
 #define LEV_LIB_FLUSH_BYTES ((size_t)512 << 20)
+__global__ void __launch_bounds__(256) fill_kernel(uint4* to, uint32_t n) {
+  auto mixed = [](uint32_t x) {
+    x *= 0x9e3779b1u, x ^= x >> 15, x *= 0x85ebca77u, x ^= x >> 13;
+    const uint32_t raise = x >> 1 & 0x01000100u;  // exponents 125 and 126, 127 and 128
+    return (x & 0x80ff80ffu) + 0x3e803e80u + raise;
+  };
+  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) to[i] = uint4{mixed(4 * i), mixed(4 * i + 1), mixed(4 * i + 2), mixed(4 * i + 3)};
+}
+bool fill(void* flush, hipStream_t stream) {
+  fill_kernel<<<2048, 256, 0, stream>>>((uint4*)flush, (uint32_t)(LEV_LIB_FLUSH_BYTES / sizeof(uint4)));
+  return hipGetLastError() == hipSuccess;
+}
 void* flush_buffer() {
   static std::map<int, void*> buffers;
   int dev = 0;
@@ -140,20 +153,64 @@ void* flush_buffer() {
   return p;
 }
 
-// Times the given kernels on the call's own operands, writing to a buffer of its own (a product into the residual stream
-// adds to its output, so the real output cannot take repeated runs), and gives the plan the fastest. The heuristic's order
+// What tells two results' bits apart: their sum, each word times an odd number of its place.
+template <class Word>
+__global__ void __launch_bounds__(256) bits_kernel(const Word* __restrict__ y, int M, int N, long ldo, unsigned long long* sum) {
+  unsigned long long t = 0;
+  for (int m = blockIdx.x; m < M; m += gridDim.x)
+    for (int n = threadIdx.x; n < N; n += 256) t += y[(size_t)m * ldo + n] * (((unsigned long long)m * N + n) * 0x9e3779b97f4a7c16ull + 1);
+  for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+  if ((threadIdx.x & 63) == 0) atomicAdd(sum, t);
+}
+
+// Of n kernels with the given bits and times (negative: did not run) the one to keep, or -1. Kernels that deal a product's last tiles out over the CUs along K add its sums up in
+// another order than those that do not, so that the choice decides the result's last bits, and these are not to hang on a stopwatch. So: an order of sums that a single
+// kernel has counts only where no two share one, and one order is preferred to another only where its fastest kernel is ahead by more than LEV_LIB_AHEAD; otherwise
+// the one that more kernels have, then the one of the heuristic's earlier kernel. Over 77 shapes of 257 .. 2,070 rows the orders that are left are 4.3 % apart or more
+// where there is more than one (mostly all sixteen kernels share one), while the kernels were down to 0.2 %: 4096 x 16384 at 1,088 rows takes 176 us with two of the kernels, 183 and 188
+// with one each, 198 with three that do not split; it was the one product of the 7B sizes whose bits went by the process. What this gives away: 50257 x 4096 from 900 rows on 4 - 6 %.
+#define LEV_LIB_AHEAD 1.02f
+extern "C" int lev_linear_library_keeps(const unsigned long long* bits, const float* us, int n) {
+  struct Order { int kernels, first, best; };
+  std::vector<Order> orders;
+  for (int i = 0; i < n; ++i) {
+    if (us[i] < 0.0f) continue;
+    size_t at = 0;
+    while (at < orders.size() && bits[orders[at].first] != bits[i]) ++at;
+    if (at == orders.size()) orders.push_back({0, i, i});
+    Order& o = orders[at];
+    ++o.kernels;
+    if (us[i] < us[o.best]) o.best = i;
+  }
+  bool shared = false;
+  for (const Order& o : orders) shared |= o.kernels > 1;
+  float fastest = -1.0f;
+  for (const Order& o : orders)
+    if ((!shared || o.kernels > 1) && (fastest < 0.0f || us[o.best] < fastest)) fastest = us[o.best];
+  const Order* kept = nullptr;
+  for (const Order& o : orders)
+    if ((!shared || o.kernels > 1) && us[o.best] <= fastest * LEV_LIB_AHEAD && (!kept || o.kernels > kept->kernels)) kept = &o;
+  return kept ? kept->best : -1;
+}
+
+// Times the plan's candidates on the call's own operands, writing to a buffer of its own (a product into the residual stream
+// adds to its output, so the real output cannot take repeated runs), and gives the plan the one to keep. The heuristic's order
 // is a table look-up by size; on this chip its first kernel is often not the fastest one for the shape at hand.
+// likely: the library's index of a kernel that another row count keeps, or -1 where none has been timed: where all that may be kept add up in one order, only that kernel and the
+// heuristic's first are timed (a kernel that won at 264 rows can lose at 320, where its tiles divide the rows differently), if it is among them.
 // Allocates and synchronises: called only outside a stream capture. Returns the library's index of the kernel kept, or -1.
-int time_candidates(hipblasLtHandle_t handle, Plan* p, const std::vector<hipblasLtMatmulHeuristicResult_t>& candidates, const void* a,
-                    const void* w, const float* residual, void* workspace, int M, int N, long ldo, int out_dtype, hipStream_t stream) {
+int time_candidates(hipblasLtHandle_t handle, Plan* p, int likely, const void* a, long lda, const void* w, const float* bias, const float* residual, long ldr,
+                    void* workspace, int M, int N, int K, long ldo, int out_dtype, hipStream_t stream) {
   p->timed = true;
-  if (candidates.size() < 2) return -1;
+  const std::vector<hipblasLtMatmulHeuristicResult_t>& candidates = p->candidates;
+  const int n = (int)candidates.size();
+  if (n < 2) return -1;
   auto t_begin = std::chrono::steady_clock::now();
-  const size_t bytes = (size_t)M * (size_t)ldo * (out_dtype == LEV_F32 ? 4 : 2);
+  const size_t bytes = ((size_t)M * (size_t)ldo * (out_dtype == LEV_F32 ? 4 : 2) + 255) / 256 * 256;
   void* scratch = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
-  if (hipMalloc(&scratch, bytes) != hipSuccess) { (void)hipGetLastError(); return -1; }
-  void* flush = flush_buffer();  // null if it could not be had: the runs are then timed on a warm weight
+  if (hipMalloc(&scratch, bytes + LEV_LIB_CANDIDATES * sizeof(unsigned long long)) != hipSuccess) { (void)hipGetLastError(); return -1; }
+  void* flush = flush_buffer();  // null if it could not be had: the runs are then timed on a warm weight, and all on the call's operands
   if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
     (void)hipGetLastError();
     if (e0) (void)hipEventDestroy(e0);
@@ -161,49 +218,85 @@ int time_candidates(hipblasLtHandle_t handle, Plan* p, const std::vector<hipblas
     return -1;
   }
   const float alpha = 1.0f, beta = residual ? 1.0f : 0.0f;
-  const void* c = residual ? (const void*)residual : (const void*)scratch;
-  float best = -1.0f;
-  int best_i = 0;
-  for (size_t i = 0; i < candidates.size(); ++i) {
-    const hipblasLtMatmulHeuristicResult_t& cand = candidates[i];
+  unsigned long long* sums = (unsigned long long*)((char*)scratch + bytes);
+  auto run = [&](int i, const void* a_, const void* w_, const void* c_) {
+    return hipblasLtMatmul(handle, p->desc, &alpha, w_, p->lw, a_, p->la, &beta, residual ? c_ : scratch, p->lc, scratch, p->ld, &candidates[i].algo, workspace,
+                           candidates[i].workspaceSize, stream) == HIPBLAS_STATUS_SUCCESS;
+  };
+  auto bias_at = [&](const void* b) {
+    return !bias || hipblasLtMatmulDescSetAttribute(p->desc, HIPBLASLT_MATMUL_DESC_BIAS_POINTER, &b, sizeof(b)) == HIPBLAS_STATUS_SUCCESS;
+  };
+  // Every kernel once (which loads it), on the buffer's numbers where it has enough of them (the call's may be zeros, on which all are alike): a weight from another place than the
+  // rows, which it may overlap
+  const size_t w_at = ((size_t)1 << 20) + 4096;
+  const bool ours = flush && fill(flush, stream) && ((size_t)M * lda) * 2 <= LEV_LIB_FLUSH_BYTES && w_at + (size_t)N * K * 2 <= LEV_LIB_FLUSH_BYTES &&
+                    (size_t)M * ldr * 4 <= LEV_LIB_FLUSH_BYTES && bias_at(flush);
+  unsigned long long bits[LEV_LIB_CANDIDATES];
+  float us[LEV_LIB_CANDIDATES];
+  bool all = hipMemsetAsync(sums, 0, LEV_LIB_CANDIDATES * sizeof(unsigned long long), stream) == hipSuccess;
+  for (int i = 0; i < n; ++i) {
+    us[i] = all && (ours ? run(i, flush, (const char*)flush + w_at, flush) : run(i, a, w, residual)) ? 0.0f : -1.0f;
+    if (us[i] < 0.0f) { (void)hipGetLastError(); continue; }
+    if (out_dtype == LEV_F32) bits_kernel<uint32_t><<<1024, 256, 0, stream>>>((const uint32_t*)scratch, M, N, ldo, sums + i);
+    else bits_kernel<uint16_t><<<1024, 256, 0, stream>>>((const uint16_t*)scratch, M, N, ldo, sums + i);
+  }
+  all = all && hipMemcpyAsync(bits, sums, sizeof(bits), hipMemcpyDeviceToHost, stream) == hipSuccess && hipStreamSynchronize(stream) == hipSuccess;
+  all = bias_at(bias) && all;
+  // Timed are all whose order of sums may be kept; where that is one order and another row count keeps one of them, two.
+  auto share = [&](int i, int j) { return i != j && us[i] >= 0.0f && us[j] >= 0.0f && bits[i] == bits[j]; };
+  bool shared = false, alone[LEV_LIB_CANDIDATES];
+  for (int i = 0; i < n; ++i) {
+    alone[i] = true;
+    for (int j = 0; j < n; ++j) alone[i] &= !share(i, j);
+    shared |= !alone[i];
+  }
+  int first = -1, known = -1;
+  bool one_order = true;
+  for (int i = 0; i < n; ++i) {
+    if (!all || (shared && alone[i])) us[i] = -1.0f;
+    if (us[i] < 0.0f) continue;
+    if (first < 0) first = i;
+    one_order &= bits[i] == bits[first];
+    hipblasLtMatmulAlgo_t algo = candidates[i].algo;
+    if (likely >= 0 && hipblaslt_ext::getIndexFromAlgo(algo) == likely) known = i;
+  }
+  const bool two = one_order && known >= 0;
+  for (int i = 0; i < n; ++i) {
+    if (us[i] < 0.0f) continue;
+    if (two && i != first && i != known) { us[i] = -1.0f; continue; }
+    if (two && first == known) continue;
     bool ok = true;
     float ms = -1.0f;
     // Every timed run behind a sweep over a buffer larger than the caches: in a model's step a product's weight has not
     // been touched since the step before, and the kernel that is fastest on a weight that waits in the last-level cache
     // (what a plain loop over one weight measures) is often not the fastest on one that comes from memory. The fastest
     // of the runs counts.
-    for (int run = 0; run <= LEV_LIB_TUNE_RUNS && ok; ++run) {  // run 0 loads the kernel and is not timed
-      if (run > 0) ok = (!flush || hipMemsetAsync(flush, run, LEV_LIB_FLUSH_BYTES, stream) == hipSuccess) &&
-                        hipEventRecord(e0, stream) == hipSuccess;
-      ok = ok && hipblasLtMatmul(handle, p->desc, &alpha, w, p->lw, a, p->la, &beta, c, p->lc, scratch, p->ld, &cand.algo, workspace,
-                                 cand.workspaceSize, stream) == HIPBLAS_STATUS_SUCCESS;
-      if (run > 0) {
-        float t = 0.0f;
-        ok = ok && hipEventRecord(e1, stream) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
-             hipEventElapsedTime(&t, e0, e1) == hipSuccess;
-        if (ok && (ms < 0.0f || t < ms)) ms = t;
-      }
+    for (int r = 0; r < LEV_LIB_TUNE_RUNS && ok; ++r) {
+      float t = 0.0f;
+      ok = (!flush || fill(flush, stream)) && hipEventRecord(e0, stream) == hipSuccess && run(i, a, w, residual) && hipEventRecord(e1, stream) == hipSuccess &&
+           hipEventSynchronize(e1) == hipSuccess && hipEventElapsedTime(&t, e0, e1) == hipSuccess;
+      if (ok && (ms < 0.0f || t < ms)) ms = t;
     }
-    if (!ok || ms < 0.0f) { (void)hipGetLastError(); (void)hipStreamSynchronize(stream); continue; }
+    us[i] = ok ? ms * 1000.0f : -1.0f;
+    if (!ok) { (void)hipGetLastError(); (void)hipStreamSynchronize(stream); continue; }
     if (tune_level() >= 2) {
-      hipblasLtMatmulAlgo_t algo = cand.algo;
-      fprintf(stderr, "linear (library) M=%d N=%d: candidate %zu (kernel %d) %.1f us\n", M, N, i, hipblaslt_ext::getIndexFromAlgo(algo),
-              ms * 1000.0f);
+      hipblasLtMatmulAlgo_t algo = candidates[i].algo;
+      fprintf(stderr, "linear (library) M=%d N=%d K=%d: candidate %d (kernel %d, bits %016llx) %.1f us\n", M, N, K, i, hipblaslt_ext::getIndexFromAlgo(algo), bits[i], us[i]);
     }
-    if (best < 0.0f || ms < best) { best = ms; best_i = (int)i; }
   }
-  if (best >= 0.0f) {
-    p->algo = candidates[best_i].algo;
-    p->workspace = candidates[best_i].workspaceSize;
+  const int best = lev_linear_library_keeps(bits, us, n);
+  if (best >= 0) {
+    p->algo = candidates[best].algo;
+    p->workspace = candidates[best].workspaceSize;
     if (tune_level() >= 2)
-      fprintf(stderr, "linear (library) M=%d N=%d: kept candidate %d after %.1f ms\n", M, N, best_i,
+      fprintf(stderr, "linear (library) M=%d N=%d K=%d: kept candidate %d after %.1f ms\n", M, N, K, best,
               std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_begin).count());
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   (void)hipStreamSynchronize(stream);
   (void)hipFree(scratch);
-  return best >= 0.0f ? hipblaslt_ext::getIndexFromAlgo(p->algo) : -1;
+  return best >= 0 ? hipblaslt_ext::getIndexFromAlgo(p->algo) : -1;
 }
 
 // The kernel that timing chose for another row count of the plan's bucket, if the heuristic offers it for this row count
@@ -258,33 +351,17 @@ extern "C" int lev_linear_library(const void* a, long lda, const void* w, const 
     const bool may_time = capturing == hipStreamCaptureStatusNone;
     const PlanKey bucket(dev, rows_bucket(M), N, K, lda, residual ? ldr : 0, ldo, (int)epilogue, out_dtype, residual ? 1 : 0);
     auto known = g_timed_index.find(bucket);
-    if (known == g_timed_index.end()) {
-      if (may_time)
-        g_timed_index[bucket] = time_candidates(handle, &plan, plan.candidates, a, w, residual, workspace, M, N, ldo, out_dtype, stream);
-      else
-        plan.timed = true;  // recorded into a graph with the heuristic's first kernel: eager calls of this shape keep it too,
-                            // so that a replay and an eager run of the same product give the same bits
+    if (may_time) {
+      const int index = time_candidates(handle, &plan, known == g_timed_index.end() ? -1 : known->second, a, lda, w, bias, residual, ldr, workspace, M, N, K, ldo, out_dtype, stream);
+      if (known == g_timed_index.end()) g_timed_index[bucket] = index;
     } else {
-      // Another row count of the bucket has been timed: its kernel against the heuristic's first for this row count (a
-      // kernel that won at 264 rows can lose at 320, where its tiles divide the rows differently), not all sixteen again.
-      plan.timed = true;  // whether the bucket's kernel is on offer or not: the plan is settled
-      const hipblasLtMatmulHeuristicResult_t* theirs = known->second >= 0 ? candidate_of_index(&plan, known->second) : nullptr;
-      if (tune_level() >= 2)
-        fprintf(stderr, "linear (library) M=%d N=%d K=%d: kernel %d of its bucket is %s\n", M, N, K, known->second,
-                theirs == &plan.candidates[0] ? "the heuristic's first" : (theirs ? "on offer" : "not on offer"));
-      if (theirs && theirs != &plan.candidates[0]) {
-        if (may_time) {
-          std::vector<hipblasLtMatmulHeuristicResult_t> two = {*theirs, plan.candidates[0]};
-          time_candidates(handle, &plan, two, a, w, residual, workspace, M, N, ldo, out_dtype, stream);
-        } else {
+      plan.timed = true;  // recorded into a graph with the heuristic's first kernel, or the one its bucket keeps: eager calls of this shape keep it
+                          // too, so that a replay and an eager run of the same product give the same bits
+      if (known != g_timed_index.end() && known->second >= 0)
+        if (const hipblasLtMatmulHeuristicResult_t* theirs = candidate_of_index(&plan, known->second)) {
           plan.algo = theirs->algo;
           plan.workspace = theirs->workspaceSize;
         }
-      } else if (!theirs && may_time) {
-        // the bucket's kernel is not offered for this row count: its own candidates then (the heuristic's first was up to
-        // a third slower than their best at 304 and 320 rows of a 1600-wide layer, whose bucket was timed at 272)
-        time_candidates(handle, &plan, plan.candidates, a, w, residual, workspace, M, N, ldo, out_dtype, stream);
-      }
     }
   }
   if (plan.workspace > 0 && !workspace)

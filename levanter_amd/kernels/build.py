@@ -354,6 +354,7 @@ register_unit("gemm_mfma", ["gemm_mfma.hip", "gemm_ring.hip", "gemm_norm.hip"], 
 register_unit("gemm_library", ["gemm_library.hip"], link_flags=["-lhipblaslt"], signatures={
     "lev_linear_library": [_P, _L, _P, _P, _P, _L, _P, _L, _P, _L] + [_I] * 5 + [_P],
     "lev_linear_library_workspace": [],
+    "lev_linear_library_keeps": [_P, _P, _I],
 })
 for _hd in MFMA_ATTENTION_HEAD_DIMS:
     register_unit(attention_unit(_hd), [("attention_mfma.hip", [f"-DLEV_HD={_hd}"], f"attention_mfma_hd{_hd}.o"),

@@ -48,6 +48,47 @@ def test_the_tiles_of_the_experts_products_are_the_faster_ones(experts, width, i
     assert taken <= 1.05 * min(few, many)
 
 
+# rows, outputs, inputs; for each of the library's kernels the order in which it adds up (0: the first kernel's bits, and so on) and its microseconds
+STOPWATCH = (1088, 4096, 16384, (0, 0, 0, 1, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 4, 3),
+             (201.1, 204.9, 213.5, 320.8, 313.0, 329.9, 180.4, 309.8, 200.0, 290.2, 319.9, 191.0, 187.3, 184.2, 315.0, 254.4))
+
+
+@pytest.fixture(scope="module")
+def keeps(core):
+    library = ctypes.CDLL(build.ensure_built("gemm_library"))
+
+    def kept(bits, us):
+        n = len(bits)
+        return library.lev_linear_library_keeps((ctypes.c_ulonglong * n)(*bits), (ctypes.c_float * n)(*us), n)
+
+    return kept
+
+
+def test_the_order_of_the_librarys_sums_does_not_hang_on_a_stopwatch(keeps):
+    """Times that are off by up to 2 %, as those of two processes are: always a kernel with the same bits. Of these the fastest."""
+    import random
+
+    *_, bits, us = STOPWATCH
+    rng = random.Random(1)
+    noisy = [[t * rng.uniform(0.98, 1.02) for t in us] for _ in range(500)]
+    assert {bits[min(range(len(us)), key=t.__getitem__)] for t in noisy} == {3, 10}  # what the fastest alone gives
+    assert {bits[keeps(bits, t)] for t in noisy} == {3}
+    assert keeps(bits, us) == 6
+
+
+@pytest.mark.parametrize("bits,us,kept", [
+    ((0, 1, 2), (216.0, 216.5, 205.8), 2),                          # nobody shares an order: the fastest
+    ((0, 1, 2), (206.0, 216.5, 205.8), 0),                          # within the stopwatch's error: the heuristic's earlier one
+    ((0, 0, 1, 1, 1), (99.0, 104.0, 103.0, 99.5, 99.9), 3),         # the one that more kernels have
+    ((0, 0, 1, 1, 1), (97.0, 104.0, 103.0, 99.5, 99.9), 0),         # unless it is behind
+    ((0, 1, 1, 2), (90.0, 104.0, 103.0, 80.0), 2),                  # one kernel's own order is left out
+    ((0, 0, 0), (100.0, 99.9, 99.8), 2), ((0, 0), (-1.0, 7.0), 1),  # one order: the fastest that ran
+    ((0, 0, 1), (-1.0, 7.0, 9.0), 1), ((5,), (3.0,), 0), ((0, 1), (-1.0, -1.0), -1),
+])
+def test_which_of_the_librarys_kernels_is_kept(keeps, bits, us, kept):
+    assert keeps(bits, us) == kept
+
+
 # the 32-bit products, over weights that no cache holds
 TILES = [  # rows, outputs, inputs, microseconds of the tiles in the order of the kernels' two lists
     (100, 5120, 6400, (203.6, 171.7, 172.8, 180.6, 143.5, 150.0, 112.8, 119.1, 129.8, 129.3, 137.8, 165.4, 205.6)),
