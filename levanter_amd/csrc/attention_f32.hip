@@ -97,6 +97,8 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
   }
   float* ml = af_lds + (size_t)W * DT * 4 * nc * 4;
   float* weights = ml + 2 * W * 16 + wave * 256;
+  // l: of the weights of this lane's keys, every fourth four. Four sums of a quarter each have half the roundings of one over the column that each block joins (1 / the sum of 16,384 weights,
+  // rms in 2^-24, over the block's lanes first / so: runs of four waves 2.1 / 1.3, of eight 1.5 / 1.1, single tokens of four 1.6 / 1.1, of eight 1.4 / 1.1; times level)
   float m = -INFINITY, l = 0.f;
   const int t_last = last / 16;
   const bool fused = !RUNS && p.k_new != nullptr;
@@ -174,7 +176,7 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
     mx = af_over_groups(mx, [](float a, float b) { return fmaxf(a, b); });
     const float m_new = fmaxf(m, mx);
     const float corr = m == -INFINITY ? 0.f : expf(m - m_new);
-    float sum = 0.f;
+    float sum = 0.f;  // this lane's keys
 #pragma unroll
     for (int t = 0; t < KB; ++t)
 #pragma unroll
@@ -183,7 +185,6 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
         s[t][r] = e;
         sum += e;
       }
-    sum = af_over_groups(sum, [](float a, float b) { return a + b; });
     l = l * corr + sum;
     m = m_new;
 #pragma unroll
@@ -257,6 +258,7 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
 #pragma unroll
     for (int d = 0; d < DT; ++d) *reinterpret_cast<af_f32x4*>(af_lds + ((size_t)((wave * DT + d) * 4 + g) * nc + col) * 4) = o_acc[0][d];
   }
+  l = af_over_groups(l, [](float a, float b) { return a + b; });
   if (g == 0) ml[wave * 16 + col] = m, ml[(W + wave) * 16 + col] = l;
   __syncthreads();
   if (!mine) return;

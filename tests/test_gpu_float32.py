@@ -250,6 +250,40 @@ def test_attention_float32_of_many_single_tokens(K, HD, window):
     test_attention_float32(K, 16, 16, HD, 16, [(1, n) for n in (1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 160, 161, 255, 300)], window)
 
 
+# the kernels of runs with four and eight waves, of single tokens with four and eight; (rows of) requests, heads
+@pytest.mark.parametrize("runs,H,bound", [([64], 64, 1.6), ([17], 16, 1.4), ([1] * 260, 16, 1.3), ([1] * 60, 16, 1.3)])
+@pytest.mark.parametrize("HD", [64, 128])
+def test_attention_float32_denominators_of_long_contexts(K, runs, H, bound, HD):
+    """Scores are exact, the only value is the first key's, whose weight is 1 throughout: an output is 1 / the sum of 16,384 weights. Its error is the exponentials' and
+    the merge's, about one unit of 2^-24, and that of the chain of sums: each lane's of every fourth four keys of a wave's, of n additions, 0.3 sqrt(n / 3) / 2 units.
+    (Measured 1.3, 1.1, 1.1, 1.1; a sum over a block's lanes that joins one over the context: 2.1, 1.5, 1.6, 1.4.)"""
+    from helpers import make_meta
+
+    n, PS = 16384, 16
+    g = torch.Generator().manual_seed(3)
+    x = torch.clamp(torch.round(torch.randn(n, HD, generator=g) * 16) / 16, max=4.0)
+    x[0] = 4.0
+    kd = x.view(n // PS, PS, HD // 8, 8).permute(0, 2, 1, 3).contiguous().to(DEV)
+    vd = torch.zeros(n // PS, HD, PS, device=DEV)
+    vd[0, :, 0] = 1.0
+    T, kv = sum(runs), [n - 37 * (i % 23) for i in range(len(runs))]
+    bt = torch.arange(n // PS, dtype=torch.int32, device=DEV).expand(len(runs), -1).contiguous()
+    scale = torch.tensor([0.5, 0.75, 1.0, 1.25])[torch.arange(T) % 4]
+    q = torch.zeros(T, H, HD)
+    for h in range(H):
+        q[:, h, h] = scale
+    got = torch.empty(T, H * HD, device=DEV)
+    K.paged_attention(q.view(T, -1).to(DEV), got, kd.view(-1), vd.view(-1), make_meta(list(zip(runs, kv)), DEV), n_heads=H, n_kv_heads=1, head_dim=HD, page_size=PS, scale=1.0,
+                      window=None, block_tables=bt)
+    seen = [k - r + i + 1 for r, k in zip(runs, kv) for i in range(r)]
+    xd = x[:, :H].double().to(DEV)
+    want = torch.stack([1 / torch.exp((xd[:m] - 4.0) * float(c)).sum(0) for m, c in zip(seen, scale)])
+    off = (got.view(T, H, HD)[:, :, 5].double() - want) / want
+    rms = float(off.pow(2).mean().sqrt()) / EPS
+    print(f"rms {rms:.3f} of 2^-24")
+    assert rms <= bound
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 def test_attention_float32_values_that_are_not_seen_do_not_count(K, bad):
     """Token 20's value is not a number: queries before it are what they are without it, the ones from it on carry it. A single token whose block
