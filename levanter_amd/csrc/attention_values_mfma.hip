@@ -325,21 +325,39 @@ attention_values_mfma_kernel(const bf16_t* __restrict__ q, long q_stride, float*
 // set of value heads). The keys and values of a block of 64 positions are staged once for all waves: global -> registers
 // (requested a block ahead) -> LDS, with everything beyond the last written key made zero on the way (from the registers, not when they are asked
 // for: that would wait for them).
-// What bounds it: the chain of a block (two barriers, scores, softmax, values) in the workgroups of the longest tiles, few of which share a CU. So the operands of the products
-// come from LDS four at a time, two groups ahead (one, where a workgroup is half a tile) instead of each ahead of its product; a block has no branch for its scores; the maximum goes over the lanes by swaps, and the outputs
-// are scaled only when one was raised. The next block is asked for in one set of registers: of two sets, one of which a branch picked, the loads went to a third, were waited for
-// and copied there, in every block.
-// Before / now, microseconds a layer, 16 heads of 128 / 64, 256 / 224, 64 / 32: 1,000 tokens 38 / 24, 60 / 49, 30 / 20; two of 1,015 41 / 31, 64 / 54, 31 / 24; 2,000 70 / 54, 111 / 87, 54 / 41; twelve of 150
-// 12.8 / 11.4, 27 / 29, 9.9 / 9.4. (Wide heads take the registers of two workgroups of which one is left a CU: many runs of one to three blocks are 4 - 15 % slower there.)
+// What bounds it: the chain of a block (two barriers, scores, softmax, values) in the workgroups of the longest tiles, few of which share a CU; in short runs the trips to memory ahead of the first
+// block. So the operands of the products come from LDS four at a time, a group ahead, instead of each ahead of its product; a block has no branch for its scores; the maximum goes over the lanes by swaps, and the outputs
+// are scaled only when one was raised. The next block is asked for in one set of registers (of two sets, one of which a branch picked, the loads went to a third, were waited for
+// and copied there, in every block), behind the last none; the queries are asked for under no condition: in a branch each, they were waited for one by one (wide heads, twelve runs of 150: 29 -> 24 us).
+// Microseconds a layer, 16 heads, two sets of registers and each operand ahead of its product / all that now:
+//                    128 / 64      64 / 64      144 / 112    256 / 224
+//   1,000 tokens     36.9 / 23.8   31.6 / 22.4  44.3 / 33.2  58.8 / 45.4
+//   two of 1,015     40.1 / 30.8   33.8 / 26.5  47.3 / 34.7  62.7 / 48.6
+//   six of 1,000     79.5 / 67     68.3 / 59    130 / 99     176 / 137
+//   twelve of 150    12.6 / 11.1   10.7 / 10.4  18.6 / 17.5  26.6 / 23.8
+//   32 of 60          9.5 /  9.1    9.3 /  9.2  13.0 / 12.2  18.8 / 17.4
+//   64 of 30         13.7 / 12.6   12.2 / 12.0  18.8 / 17.2  29.1 / 26.6
+//   32 of 70, 200 keys  16.8 / 14.9  15.9 / 14.3  27.3 / 23.4  37.7 / 31.7
 #define RUN_MAX_LDS (80 * 1024)  // bytes a workgroup may take: two workgroups a CU
 #define RUN_PAGES 2048  // page ids of a tile's key range that are kept in LDS
 
-// Waves of a workgroup, 16 query tokens each: half a tile's, where three such workgroups fit a CU's registers (heads of 128 / 64, microseconds, whole tiles / halves: 1,000 tokens 28.3 / 24.5, six
-// of 1,000 82 / 68, two of 1,015 30.7 / 30.4; of 256 / 224 two of 1,015 55 / 100: the loads of a block are twice as many registers a thread).
-#define RUN_WAVES(NC) ((NC) == 1 && HD + VD <= 192 ? PF_WAVES / 2 : PF_WAVES)
+// Waves of a workgroup, 16 query tokens each: half a tile's, where three such workgroups fit a CU's registers (heads of 128 / 64, microseconds, whole tiles / halves: 1,000 tokens 28.3 / 24.5,
+// two of 1,015 30.7 / 30.4; of 256 / 224 two of 1,015 55 / 100: the loads of a block are twice as many registers a thread).
+#define RUN_WAVES (HD + VD <= 192 ? PF_WAVES / 2 : PF_WAVES)
+
+// Whole tiles whose operands are read without a group ahead, in registers for two workgroups a CU (of 16 heads of 128 / 64, us, so / as above): where tiles are half empty, so that so
+// are the halves (64 runs of 30: 12.6 / 15.9; of 30 behind 60 keys 17.0 / 22.6), and where there are more of them than the 768 halves that three a CU are (32 of 70, 200 keys 14.9 / 21.1; 32 of 128 12.8 / 16.2; 24 of 128
+// still 11.6 / 11.2; eight of 1,000 79 / 88), but for the smallest heads, of whose halves a CU holds four (12 heads of 64 / 32, 64 runs of 96: 14.1 / 12.5). Heads beyond 192 numbers, which have no halves: where tiles are half
+// empty and contexts short (144 / 112, 64 runs of 30: 17.2 / 21.5; 16 of 64 over 1,000 keys 32.3 / 29.7); beyond 256 never: their registers leave one workgroup a CU either way (256 / 224, 64 of 30: 27.3 / 26.6).
+static bool av_whole_tiles(int n_tiles, int tokens, int H, int max_keys) {
+  const bool half_empty = tokens <= PF_ROWS / 2 * n_tiles;
+  if (HD + VD > 192) return HD + VD <= 256 && half_empty && max_keys <= 256;
+  return half_empty || (HD + VD >= 128 && (long)n_tiles * H > 384);
+}
 
 // NC: value heads that a wave has room for, as above: 1, or NVC for layers with more
-template <int NC, int WAVES>
+// D - 1: groups of operands that are read ahead
+template <int NC, int WAVES, int D>
 __global__ void __launch_bounds__(64 * WAVES, WAVES == PF_WAVES ? 2 : 3)
 attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, float* __restrict__ out, const bf16_t* __restrict__ k_pages,
                                   const bf16_t* __restrict__ v_pages, const int* __restrict__ positions, const int* __restrict__ token_seq,
@@ -352,6 +370,7 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
   bf16_t* ks = reinterpret_cast<bf16_t*>(av_smem);  // [HD/8][64][8]
   bf16_t* vs = ks + HD * 64;                        // [8 chunks][n_c VD][8]
   __shared__ int pages_s[RUN_PAGES];                // page ids of the blocks that the tile's keys lie in
+  __shared__ __attribute__((aligned(16))) bf16_t zeros[HD % 32 != 0 ? 3 * 128 + 8 : 8];  // keys' dimensions beyond HD, read from as far apart as those of keys are
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, g = lane >> 4;
   const int tile = blockIdx.x / PARTS, skip = (blockIdx.x - tile * PARTS) * 16 * WAVES;
   const int first = tiles[2 * tile] + skip, n = min(tiles[2 * tile + 1] - skip, 16 * WAVES);
@@ -402,9 +421,7 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
   u32x4 qf[NKS];
 #pragma unroll
   for (int s = 0; s < NKS; ++s) {
-    qf[s] = u32x4{0u, 0u, 0u, 0u};
-    if (valid && 32 * s + 8 * g < HD)
-      qf[s] = *reinterpret_cast<const u32x4*>(q + (size_t)tok * q_stride + (size_t)head * HD + 32 * s + 8 * g);
+    qf[s] = *reinterpret_cast<const u32x4*>(q + (size_t)tok * q_stride + (size_t)head * HD + (HD % 32 == 0 ? 32 * s + 8 * g : min(32 * s + 8 * g, HD - 8)));
   }
   f32x4 o[NC][NDT];
 #pragma unroll
@@ -420,6 +437,7 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
   // order but for a turn by twice the chunk's number: 16 lanes' reads, and what neighbouring lanes write, fall on all banks.
   const int v_rows = NC == 1 ? VD : n_c * VD;
   const bf16_t* ks_get = ks + (g * 64 + col) * 8;
+  const bf16_t* ks_get_last = 32 * (NKS - 1) + 8 * g < HD ? ks_get + 4 * (NKS - 1) * 64 * 8 : zeros;
   const bf16_t* vs_get[2] = {vs + (g * v_rows + (col ^ 2 * g)) * 8, vs + ((4 + g) * v_rows + (col ^ (8 + 2 * g))) * 8};
   bf16_t* ks_put = ks + ((tid & ~63) + (tid & 32) + 16 * (tid >> 2 & 1) + 4 * (tid >> 3 & 3) + (tid & 3)) * 8;
   u32x4 kst[K_STAGE], vst[V_STAGE];  // the next block, on its way
@@ -460,18 +478,19 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
     }
   };
 
+  if (HD % 32 != 0 && tid < 4 * 8) zeros[(tid >> 3) * 128 + (tid & 7)] = 0;
   fetch(lev_block_key(0, n_kept, first_block));
+  if (HD % 32 != 0 && 32 * (NKS - 1) + 8 * g >= HD) qf[NKS - 1] = u32x4{0u, 0u, 0u, 0u};
   for (int it = 0; it < n_blocks; ++it) {
     const int key0 = lev_block_key(it, n_kept, first_block);
     lds_barrier();  // the block before has been read by every wave (a barrier for LDS only: the loads on their way stay there)
     stage(key0);
-    fetch(lev_block_key(min(it + 1, n_blocks - 1), n_kept, first_block));  // under no condition: behind the last the last again
+    if (it + 1 < n_blocks) fetch(lev_block_key(it + 1, n_kept, first_block));  // the same for the workgroup
     lds_barrier();
     if (!active || key0 > p_max || (key0 + 63 < lo_min && key0 >= keep)) continue;  // none of this wave's rows sees a key of this block
     // Four operands at a time come from LDS, two such groups ahead of the products: keys (a score tile and up to four k-steps; the tiles in turn), then values (two tiles of 16
     // dimensions), the first of them before the softmax.
     constexpr int KC = (NKS + 3) / 4, NGK = 4 * KC, NGV1 = (NDT + 1) / 2, NGV = NC * NGV1;
-    constexpr int D = WAVES == PF_WAVES ? 3 : 2;
     u32x4 fr[D][4];
     f32x4 st[2][2];
     auto read = [&](int group) __attribute__((always_inline)) {
@@ -481,9 +500,7 @@ attention_values_mfma_runs_kernel(const bf16_t* __restrict__ q, long q_stride, f
         for (int e = 0; e < 4; ++e) {
           const int s = group / 4 * 4 + e;
           if (s >= NKS) break;
-          const bool in = HD % 32 == 0 || 32 * s + 8 * g < HD;  // beyond: read at another place, and zeros
-          to[e] = *reinterpret_cast<const u32x4*>(ks_get + ((in ? 4 * s * 64 : 0) + 16 * (group % 4)) * 8);
-          if (!in) to[e] = u32x4{0u, 0u, 0u, 0u};
+          to[e] = *reinterpret_cast<const u32x4*>((HD % 32 != 0 && s == NKS - 1 ? ks_get_last : ks_get + 4 * s * 64 * 8) + 16 * (group % 4) * 8);
         }
       } else if (group < NGK + NGV) {
         const int c = (group - NGK) / NGV1, dt0 = (group - NGK) % NGV1 * 2;
@@ -718,19 +735,21 @@ extern "C" int lev_attention_values_mfma(const void* q, long q_stride, float* ou
     long reach = window > 0 && window < max_keys ? window : max_keys;
     if (chunk > 0 && chunk < reach) reach = chunk;
     reach += PF_ROWS + 64 + (keep > 0 ? keep + 64 + PS : 0);
-    const size_t all_lds = lds + RUN_PAGES * sizeof(int);
-    if (all_lds > 64 * 1024 && all_lds <= RUN_MAX_LDS) {  // more than a kernel gets unasked
-      hipError_t e = hipFuncSetAttribute(NV == 1 ? (const void*)attention_values_mfma_runs_kernel<1, RUN_WAVES(1)> : (const void*)attention_values_mfma_runs_kernel<NVC, RUN_WAVES(NVC)>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      LEV_REQUIRE(e == hipSuccess, "attention: %zu bytes of LDS a workgroup: %s", all_lds, hipGetErrorString(e));
-    }
-#define AV_RUNS(NC)                                                                                                                                    \
-  attention_values_mfma_runs_kernel<NC, RUN_WAVES(NC)><<<dim3(n_tiles * (PF_WAVES / RUN_WAVES(NC)), H, chunks), 64 * RUN_WAVES(NC), lds, stream>>>(    \
-      (const bf16_t*)q, q_stride, out, (const bf16_t*)k_pages, (const bf16_t*)v_pages, positions, token_seq, block_tables, bt_stride, tiles, H, KVH, NV, PS, scale, window, \
-      chunk, keep, softcap, slopes, sinks)
+    const size_t all_lds = lds + RUN_PAGES * sizeof(int) + (HD % 32 != 0 ? 1024 : 0);
+#define AV_RUNS(NC, WAVES, D)                                                                                                                          \
+  do {                                                                                                                                                 \
+    if (all_lds > 64 * 1024) { /* more than a kernel gets unasked */                                                                                   \
+      hipError_t e = hipFuncSetAttribute((const void*)attention_values_mfma_runs_kernel<NC, WAVES, (D)>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+      LEV_REQUIRE(e == hipSuccess, "attention: %zu bytes of LDS a workgroup: %s", all_lds, hipGetErrorString(e));                                      \
+    }                                                                                                                                                  \
+    attention_values_mfma_runs_kernel<NC, WAVES, (D)><<<dim3(n_tiles * (PF_WAVES / (WAVES)), H, chunks), 64 * (WAVES), lds, stream>>>(                   \
+        (const bf16_t*)q, q_stride, out, (const bf16_t*)k_pages, (const bf16_t*)v_pages, positions, token_seq, block_tables, bt_stride, tiles, H, KVH, NV, PS, scale, window, \
+        chunk, keep, softcap, slopes, sinks);                                                                                                          \
+  } while (0)
     if (all_lds <= RUN_MAX_LDS && reach / PS + 2 <= RUN_PAGES) {
-      if (NV == 1) AV_RUNS(1);
-      else AV_RUNS(NVC);
+      if (NV > 1) AV_RUNS(NVC, PF_WAVES, 2);
+      else if (av_whole_tiles(n_tiles, n_positions - n_singles, H, max_keys)) AV_RUNS(1, PF_WAVES, HD + VD <= 256 ? 1 : 2);
+      else AV_RUNS(1, RUN_WAVES, 2);
     }
 #undef AV_RUNS
     else  // the longest ranges: every wave by itself, operands straight from the pages

@@ -34,9 +34,19 @@ def _step(runs):
                                                   (128, 64, 4, 4, True), (48, 32, 4, 2, True), (64, 48, 2, 2, True)])
 @pytest.mark.parametrize("window,softcap", [(None, None), (70, None), (None, 4.0)])
 def test_runs(dk, dv, H, G, all_values, window, softcap):
+    _check([(63, 63), (64, 64), (65, 129), (127, 140), (128, 128), (129, 193), (2, 300), (200, 391)], dk, dv, H, G, all_values, window, softcap)
+
+
+# half empty tiles, contexts of up to 256 keys and longer ones, and more tiles than half tiles would be on the chip at once (400 and 448 of a tile and a head): whole tiles a workgroup
+@pytest.mark.parametrize("dk,dv,H,G", [(128, 64, 4, 2), (16, 16, 2, 1), (48, 32, 2, 2), (144, 112, 2, 1), (256, 224, 2, 1), (128, 128, 2, 1)])
+@pytest.mark.parametrize("runs,many", [([(2, 2), (63, 63), (64, 64), (65, 129), (17, 256), (16, 80)], 1), ([(31, 300), (64, 391), (2, 65)], 1), ([(128, 128), (66, 66), (127, 140), (129, 193), (100, 391)], 32)])
+def test_runs_in_whole_tiles(dk, dv, H, G, runs, many):
+    _check(runs, dk, dv, H * many, G, False, 70, None)
+
+
+def _check(runs, dk, dv, H, G, all_values, window, softcap):
     from levanter_amd.kernels import get_kernels
 
-    runs = [(63, 63), (64, 64), (65, 129), (127, 140), (128, 128), (129, 193), (2, 300), (200, 391)]
     meta, bt, pages = _step(runs)
     g = torch.Generator(device=DEV).manual_seed(dk + dv)
     rnd = lambda *s: torch.randn(*s, device=DEV, generator=g)
