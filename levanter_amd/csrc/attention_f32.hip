@@ -47,7 +47,7 @@ template <int HD, int KB, int W, bool RUNS>
 __global__ void __launch_bounds__(64 * W, 8 / W)  /* two waves on a SIMD, runs need 137 registers at head size 64 and 256 at 128 */
 attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows) per tile of the list; single tokens: their indexes
                      const int* __restrict__ positions, const int* __restrict__ token_seq, const int* __restrict__ block_tables, int bt_stride, int H, int KVH, int PS,
-                     int tile_rows, int columns, int n_positions,  // rows of a tile of the list (runs); columns in use (single tokens: query heads of a key/value head, at most 16)
+                     int tile_rows, int columns, int n_positions,  // rows of a tile of the list (runs); columns in use (single tokens: query heads of a key/value head, at most 16); entries of positions (single tokens)
                      const AttentionF32Args p) {  // all before p is in registers when the waves start
   extern __shared__ __attribute__((aligned(16))) float af_lds[];  // [W][HD/16][4][columns] of four outputs, then maxima and sums [2][W][16] and a tile's weights [W][16][16]
   constexpr int DT = HD / 16;
@@ -288,13 +288,13 @@ attention_f32_kernel(const int* __restrict__ work,  // runs: (first token, rows)
 
 template <int HD, int W>
 static int attention_f32_runs(const AttentionF32Args& p, const int* positions, const int* token_seq, const int* block_tables, int bt_stride, int H, int KVH, int PS,
-                              const int* tiles, long blocks, int tile_rows, int n_positions, hipStream_t stream) {
+                              const int* tiles, long blocks, int tile_rows, hipStream_t stream) {
   constexpr int lds = W * (HD / 16) * 4 * 16 * 16 + 2 * W * 16 * 4 + W * 1024;
   if (lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute((const void*)attention_f32_kernel<HD, 1, W, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     LEV_REQUIRE(e == hipSuccess, "attention: %d bytes of LDS a workgroup: %s", lds, hipGetErrorString(e));
   }
-  attention_f32_kernel<HD, 1, W, true><<<(unsigned)blocks, 64 * W, lds, stream>>>(tiles, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tile_rows, 16, n_positions, p);
+  attention_f32_kernel<HD, 1, W, true><<<(unsigned)blocks, 64 * W, lds, stream>>>(tiles, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tile_rows, 16, 0, p);
   return 0;
 }
 
@@ -314,15 +314,15 @@ static int attention_f32_singles(const AttentionF32Args& p, const int* positions
 template <int HD>
 static int attention_f32_launch(const AttentionF32Args& p, const int* positions, const int* token_seq, const int* block_tables, int bt_stride, int H, int KVH, int PS,
                                 const int* tiles, int n_tiles, int tile_rows, const int* tokens, int n_tokens, int n_positions, hipStream_t stream) {
-    constexpr int DT = HD / 16, KB1 = HD <= 96 ? 2 : 1;  // single tokens: as many tiles of keys as fit the registers
+  constexpr int KB1 = HD <= 96 ? 2 : 1;  // single tokens: as many tiles of keys as fit the registers
   if (n_tiles > 0) {
     const long blocks = (long)n_tiles * ((tile_rows + 15) / 16) * H;
     LEV_REQUIRE(blocks <= 0x7fffffffL, "attention: too many tiles (%ld)", blocks);
     // Eight waves a workgroup up to one and a half for a CU (not all rows of a tile are there): the keys are then walked in half the steps (65 rows behind 935 keys, 16 heads of 64: 21.2 us
     // with four, 18.8 with eight; 256 rows, 12 heads: 8.3 and 8.1; 3 x 64 rows, 16 heads of 128: 8.8 and 7.2; 500 rows, 8 heads of 32: 10.1 and 8.8). With more of them the merges cost more than that
     // (777 rows, 16 heads of 64: 25.4 and 31.3; 300 + 500 rows, 16 heads of 112: 28.7 and 36.4).
-    const int rc = blocks <= 384 ? attention_f32_runs<HD, 8>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tiles, blocks, tile_rows, n_positions, stream)
-                                 : attention_f32_runs<HD, 4>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tiles, blocks, tile_rows, n_positions, stream);
+    const int rc = blocks <= 384 ? attention_f32_runs<HD, 8>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tiles, blocks, tile_rows, stream)
+                                 : attention_f32_runs<HD, 4>(p, positions, token_seq, block_tables, bt_stride, H, KVH, PS, tiles, blocks, tile_rows, stream);
     if (rc) return rc;
   }
   if (n_tokens > 0) {

@@ -1,5 +1,6 @@
 // y = act(a . w^T + bias) + residual in 32 bits for some hundred rows and more, on the bfloat16 matrix instruction, which multiplies sixteen times as fast as the
-// 32-bit one. Every number is the sum of three bfloat16 numbers of 8 bits each, 24 in all, the products of bfloat16 numbers are exact in 32 bits and are added up in
+// 32-bit one (splitting as in Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for higher-precision computations", 2019). Every number is the sum of
+// three bfloat16 numbers of 8 bits each, 24 in all, the products of bfloat16 numbers are exact in 32 bits and are added up in
 // 32 bits, and six of the nine partial products are taken: the three left out are at most 2^-23 of a product, 2^-26 in the mean and of either sign. The products of the first parts
 // have sums of their own, which join the total every 128 numbers (256 of long sums); the others, a hundredth as large, go to a second sum, so that a total of K numbers has
 // K / 16 + K / 128 roundings of its size. Errors against 64 bits of 300 shapes of 32 .. 2,048 rows and 256 .. 16,384 numbers a sum, normal numbers and positive ones: 0.12 .. 0.99 of
@@ -44,7 +45,8 @@ template <int RT, int NT, int WM, int WN, int KG>
 __global__ void __launch_bounds__(64 * WM * WN * KG, RT * NT * KG == 1 ? 4 : 2)
 gemm_f32_split_kernel(const float* __restrict__ a, long lda, const float* __restrict__ w, const float* __restrict__ bias, const float* residual, long ldr,
                       float* out, long ldo, int M, int N, int K, int act, int n_rows, int n_cols, int vec) {
-  constexpr int BM = 32 * RT * WM, BN = 32 * NT * WN, ROWS = BM + BN, TG = 64 * WM * WN, PASS = TG / 8, NR = (ROWS + PASS - 1) / PASS;
+  constexpr int BM = 32 * RT * WM, BN = 32 * NT * WN, ROWS = BM + BN, TG = 64 * WM * WN, PASS = TG / 8, NR = ROWS / PASS;
+  static_assert(ROWS % PASS == 0, "whole passes of loads");
   constexpr int AHEAD = RT * NT * KG == 1 ? 1 : 2;  // steps whose loads are on their way; two workgroups a CU have registers for one each
   constexpr int BUF = ROWS * GS_K * 3;
   extern __shared__ __attribute__((aligned(16))) uint16_t gs_lds[];  // [KG][2][ROWS / 16][3 parts][4 chunks of 8 numbers][16 rows][8]
@@ -66,7 +68,7 @@ gemm_f32_split_kernel(const float* __restrict__ a, long lda, const float* __rest
     const bool of_a = PASS * i + 8 * wave < BM;
     const int r = PASS * i + row;
     base[i] = of_a ? a0 : w0;
-    at[i] = of_a ? (uint32_t)(min(r, M - 1 - m0) * (int)lda + kc) * 4u : (uint32_t)(min(min(r, ROWS - 1) - BM, N - 1 - o0) * K + kc) * 4u;
+    at[i] = of_a ? (uint32_t)(min(r, M - 1 - m0) * (int)lda + kc) * 4u : (uint32_t)(min(r - BM, N - 1 - o0) * K + kc) * 4u;
   }
   uint16_t* mine = gs_lds + (size_t)kgroup * 2 * BUF;
   // a chunk's rows lie 16 bytes apart, turned by twice the chunk's number: what neighbouring lanes write and read falls on all banks
@@ -85,7 +87,6 @@ gemm_f32_split_kernel(const float* __restrict__ a, long lda, const float* __rest
     for (int i = 0; i < NR; ++i) to[i] = *reinterpret_cast<const gf_f32x4*>(base[i] + k * 4 + at[i]);
   };
   auto stage = [&](gf_f32x4 v, int i, int buf) __attribute__((always_inline)) {
-    if (ROWS % PASS != 0 && i == NR - 1 && PASS * i + 8 * wave >= ROWS) return;  // the whole wave
     gs_u32x2 p[3];
     gs_split(v, p);
 #pragma unroll

@@ -513,7 +513,8 @@ sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
     }
     __builtin_amdgcn_sched_barrier(0);
     if (more) fetch_tiles(tb + SC_Q);
-    // through a buffer of the wave's 16 rows, beyond whose end nothing is written: a branch round a store makes the next block's loads wait for it
+    // through a buffer of the wave's 16 rows (of at most 65,535 heads of 256 channels, which is all that is let in: 2^30 bytes), beyond whose end nothing is written: a branch round a store makes
+    // the next block's loads wait for it
     const auto rows = __builtin_amdgcn_make_buffer_rsrc(o + (size_t)(tb + 16 * wave) * s.H * dv, 0, 16 * s.H * dv * (int)sizeof(float), 0x00027000);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -547,7 +548,6 @@ int sr_chunks_launch(int rule, const bf16_t* u, const float* scal, float* state,
                      const SrShape& s, hipStream_t stream) {
   const int vec = s.C % 8 == 0 && s.dk % 8 == 0 && s.k_off % 8 == 0 && s.q_off % 8 == 0 && ((uintptr_t)u & 15) == 0;
   const int n_blocks = (s.Tn + SC_Q - 1) / SC_Q;
-  LEV_REQUIRE((long)s.H * s.dv < (1L << 25), "state recurrence: rows of %ld numbers are too long", (long)s.H * s.dv);
   LEV_REQUIRE(max_runs <= 65535 && n_blocks <= 65535 && ((uintptr_t)workspace & 15) == 0, "state recurrence: too many runs (%d) or tokens (%d)", max_runs, s.Tn);
   float* P = workspace;
   float* T = workspace + (size_t)n_blocks * s.H * 10 * 256;
