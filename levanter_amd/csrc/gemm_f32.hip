@@ -128,8 +128,9 @@ gemm_f32_kernel(const float* __restrict__ w, const float* __restrict__ a, uint32
 // go to SETS sums in turn (so many that none waits for the one before it), which join the tile's sum every 128 or 256 k, below GF_SHORT every 64: chains of
 // 128, 128 and 64 numbers for 1, 2 and 4 sets, in short sums of 64, 32 and 16, no more than a quarter of K as in the kernel above (errors against
 // 64 bits at 777 rows, that kernel's / this one's: K = 1,024 2.9e-7 / 2.1e-7; 4,096 5.7e-7 / 2.1e-7; 256 1.5e-7 / 1.1e-7 - 1.5e-7, with chains of 128 2.05e-7).
-// What bounds it: the matrix pipe (64 x 128 tiles, 4096 x 4096 at 2,048 rows 495 us, 139 TFLOP/s; before 531), of some hundred rows the last round of
-// tiles. A mask on the chunks in the loop cost it 15 %: it waited for loads that had just gone out.
+// What bounds it: the matrix pipe (4096 x 252 at 1,500 rows 34 us, 91 TFLOP/s; 1697 x 1060 at 743 35, 76), of some hundred rows the last round of
+// tiles. Larger products, long sums into many outputs above all, go to gemm_f32_split.hip by the rule at this file's end; this kernel has those of less than 256 inputs, those whose few tiles or steps
+// would leave the other one's larger tiles idle, and rows too far apart for it. A mask on the chunks in the loop cost it 15 %: it waited for loads that had just gone out.
 #define GF_LD 36
 #define GF_SHORT 512  // inputs: below, single chains of 128 would be less exact than the split of K
 template <int RT, int NT, int SETS>
@@ -322,9 +323,8 @@ gemm_f32_few_kernel(const float* __restrict__ w, const float* __restrict__ a, ui
 // CU (a lone workgroup of 32 x 96 at what it takes with weights that no cache holds; 0.44 us a step with weights in the last cache made it the choice where it is up to
 // 15 % behind: 5120 x 6400 at 100 rows 129 us, 64 x 64 of the first 113). Checked over 1,386 shapes of 512 inputs and more, weights that no cache holds: 0.3 % behind the
 // best tile on average, 18 by more than 5 %, and behind the first kernel's best alone by 4 - 7 % at six, where the second's shorter chains are taken (6400 x 3072 at 100 rows 65 us, the
-// first 61). The ends: 16 x 16 for 16 rows of 768 x 768, 64 x 128 of the second for 4096 x 4096 at 2,048 rows (520 us; 16 x 16 of the first 1,790). Before the second kernel /
-// now: 3072 x 1024 at 777 rows 66 / 54 us, 4096 x 1024 76 / 65, 1024 x 1024 24 / 21, 50257 x 1024 751 / 673, 3072 x 768 at 606 rows 41 / 30, 4096 x 4096 at 404 rows 172 / 135.
-// Below about 100 rows and for long sums into few outputs the first stays ahead: its waves split K (1024 x 4096 at 203 rows 32 us, the second 61; at 777 rows 74 and 76).
+// first 61). (Shapes that the kernel of split operands takes by the rule below are among them.) The ends: 16 x 16 for 16 rows of 768 x 768; 64 x 64 of the second for 2304 x 256 at 777 rows, 64 x 96 for 1697 x
+// 1060 at 743. Below about 100 rows and for long sums into few outputs the first stays ahead of the second: its waves split K (1024 x 4096 at 203 rows 32 us, the second 61; 768 x 3072 at 606 35).
 struct GemmF32Tile {
   int rt, nt, w;
   float pipe;   // share of the matrix pipe that the tile reaches
@@ -337,10 +337,10 @@ struct GemmF32LineTile {
   float start;
 };
 static const GemmF32LineTile GEMM_F32_LINE_TILES[] = {{1, 1, 4, 0.32f, 0.155f, 0.f},  {1, 2, 2, 0.37f, 0.28f, 0.5f}, {1, 3, 2, 0.6f, 0.395f, 1.f},
-                                                      {2, 2, 1, 0.6f, 0.5f, 1.f},     {2, 3, 1, 0.76f, 0.73f, 2.f},  {2, 4, 1, 0.98f, 0.96f, 2.5f}};
+                                                      {2, 2, 1, 0.6f, 0.5f, 1.f},     {2, 3, 1, 0.76f, 0.73f, 2.f}};
 #define GEMM_F32_N_TILES (int)(sizeof(GEMM_F32_TILES) / sizeof(GEMM_F32_TILES[0]))
 
-static int gemm_f32_choose(int M, int N, int K, double* estimate = nullptr) {  // an index into the first list, or behind its end into the second
+static int gemm_f32_choose(int M, int N, int K, double* estimate) {  // an index into the first list, or behind its end into the second
   int best = 0;
   double best_us = 1e30;
   const double memory = 4.0 * N * K / 5.2e6;
@@ -360,7 +360,7 @@ static int gemm_f32_choose(int M, int N, int K, double* estimate = nullptr) {  /
     const double us = t.start + fmax(memory, (K + 31) / 32 * fmax(t.alone + 0.15 * (n - 1) * t.among, n * t.among));
     if (us < best_us) best_us = us, best = GEMM_F32_N_TILES + i;
   }
-  if (estimate) *estimate = best_us;
+  *estimate = best_us;
   return best;
 }
 
@@ -379,28 +379,35 @@ static int gemm_f32_few(int M, int N, int K) {
 }
 
 // the kernel of a product on the 32-bit instruction: 0 less the few-row kernel's room, or the tile's place in the two lists, one behind the other
-extern "C" int lev_linear_f32_choice(int M, int N, int K) {
+static int gemm_f32_choice(int M, int N, int K, double* us) {
   const int few = gemm_f32_few(M, N, K);
-  return few > 0 ? -few : gemm_f32_choose(M, N, K);
+  return few > 0 ? -few : gemm_f32_choose(M, N, K, us);
+}
+extern "C" int lev_linear_f32_choice(int M, int N, int K) {
+  double us;
+  return gemm_f32_choice(M, N, K, &us);
 }
 
-// The tile of the kernel that splits its operands into bfloat16 numbers (gemm_f32_split.hip), or -1 where the kernels above are not behind by an estimate as theirs, fitted
+// The tile of the kernel that splits its operands into bfloat16 numbers (gemm_f32_split.hip), or -1 where the kernels above, which take `us` by their estimate, are not behind by an estimate as theirs, fitted
 // to 208 shapes of 70 .. 2,048 rows (0.2 % behind the best on average, 14 % at worst: 2048 x 256 at 1,000 rows 13.4 us, 11.8 with 64 x 128; none behind the kernels above). Below 256
 // inputs those stay ahead of it, or level; and it knows no rows more than GEMM_F32_SPLIT_MOST apart. Kernels above / this one, microseconds: 4096 x 1024 at 777 rows 62 / 47, 1024 x 4096 72 / 63,
 // 50257 x 768 at 300 rows 209 / 166, 4096 x 4096 at 2,048 502 / 366, 1600 x 1600 at 512 34 / 27; not taken: 768 x 3072 at 606 rows 35 / 47, 1024 x 1024 at 404 15 / 19.
-extern "C" int lev_linear_f32_split(int M, int N, int K) {
-  if (K % 4 != 0 || K < 256 || K > GEMM_F32_SPLIT_MOST || lev_linear_f32_choice(M, N, K) < 0) return -1;
-  double us, best_us;
-  gemm_f32_choose(M, N, K, &best_us);
-  best_us *= 0.949;  // the estimates' own errors: of 190 shapes none is slower than before
+static int gemm_f32_split_tile(int M, int N, int K, int choice, double us) {
+  if (K % 4 != 0 || K < 256 || K > GEMM_F32_SPLIT_MOST || choice < 0) return -1;
+  us *= 0.949;  // the estimates' own errors: of 190 shapes none is slower than before
   int best = -1;
   for (int i = 0; i < GEMM_F32_N_SPLIT_TILES; ++i) {
     const GemmF32SplitTile& t = GEMM_F32_SPLIT_TILES[i];
     const double n = ceil((double)((M + t.rows - 1) / t.rows) * ((N + t.outputs - 1) / t.outputs) / 256.0);
-    us = t.start + fmax(4.0 * N * K / 5.2e6, ((K + 31) / 32 + t.groups - 1) / t.groups * (n <= 1.0 ? t.alone : n * t.among));
-    if (us < best_us) best_us = us, best = i;
+    const double own = t.start + fmax(4.0 * N * K / 5.2e6, ((K + 31) / 32 + t.groups - 1) / t.groups * (n <= 1.0 ? t.alone : n * t.among));
+    if (own < us) us = own, best = i;
   }
   return best;
+}
+extern "C" int lev_linear_f32_split(int M, int N, int K) {
+  double us;
+  const int choice = gemm_f32_choice(M, N, K, &us);
+  return gemm_f32_split_tile(M, N, K, choice, us);
 }
 
 // 1: not for these operands (nothing has been launched): 16-byte loads need rows of a multiple of 4 numbers at 16-byte addresses
@@ -408,9 +415,10 @@ int lev_gemm_f32(const float* a, long lda, const float* w, const float* bias, co
                  int act, hipStream_t stream) {
   if (K % 4 != 0 || lda % 4 != 0 || ((uintptr_t)a & 15) != 0 || ((uintptr_t)w & 15) != 0) return 1;
   const int vec = ldo % 4 == 0 && ((uintptr_t)out & 15) == 0 && (!bias || ((uintptr_t)bias & 15) == 0) && (!residual || (ldr % 4 == 0 && ((uintptr_t)residual & 15) == 0));
-  const int split = lda <= GEMM_F32_SPLIT_MOST ? lev_linear_f32_split(M, N, K) : -1;
+  double us;
+  const int choice = gemm_f32_choice(M, N, K, &us), split = lda <= GEMM_F32_SPLIT_MOST ? gemm_f32_split_tile(M, N, K, choice, us) : -1;
   if (split >= 0) return lev_gemm_f32_split(split, a, lda, w, bias, residual, ldr, out, ldo, M, N, K, act, vec, stream);
-  const int choice = lev_linear_f32_choice(M, N, K), few = -choice, line = choice - GEMM_F32_N_TILES;
+  const int few = -choice, line = choice - GEMM_F32_N_TILES;
   if (few > 0) {
 #define GEMM_F32_FEW(MR) \
   if (few == MR) gemm_f32_few_kernel<MR><<<(N + GF_FEW_OUT - 1) / GF_FEW_OUT, 512, 0, stream>>>(w, a, (uint32_t)(lda / 4), K, N, M, bias, residual, out, ldr, ldo, act)
@@ -443,7 +451,6 @@ int lev_gemm_f32(const float* a, long lda, const float* w, const float* bias, co
   else GEMM_F32_LINE_CASE(1, 3, 2);
   else GEMM_F32_LINE_CASE(2, 2, 1);
   else GEMM_F32_LINE_CASE(2, 3, 1);
-  else GEMM_F32_LINE_CASE(2, 4, 1);
 #undef GEMM_F32_LINE_CASE
 #undef GEMM_F32_CASE
   return lev_check_launch("linear (32-bit)");

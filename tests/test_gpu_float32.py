@@ -24,21 +24,28 @@ def _rand(*shape, seed=0):
 # 16 x 32 and (15, 264, 11531) 16 x 64. That all kernels are among them is a test below.
 LINEAR = [(1, 4, 1), (1, 64, 50), (3, 768, 768), (16, 100, 48), (17, 772, 33), (31, 1024, 130), (33, 20, 65), (64, 256, 4096), (65, 300, 1024), (129, 1028, 257),
           (203, 516, 1000), (400, 128, 1030), (777, 260, 1024), (1031, 96, 3000), (15, 264, 11531), (13, 264, 50257), (5, 6, 40), (70, 333, 129)]
-# the tiles whose operands come through LDS (32 x 32, 32 x 64, 32 x 96, 64 x 64, 64 x 96, 64 x 128): ends inside a tile, K of one step, with a short one, of
-# odd and even numbers of steps, of pieces of 128 and 256 and one step more
+# the tiles whose operands come through LDS (32 x 32, 32 x 64, 32 x 96, 64 x 64, 64 x 96): ends inside a tile, K of one step, with a short one, of
+# odd and even numbers of steps, of pieces of 128 and 256 and one step more; and tiles of split operands (more below)
 LINEAR += [(404, 768, 3072), (289, 100, 2051), (1031, 32, 3001), (801, 1028, 1030), (777, 300, 3072), (2047, 292, 4097), (609, 516, 2310), (2047, 260, 2310),
-           (1000, 260, 4097), (1030, 1028, 4100), (2047, 516, 3071)]
+           (1000, 260, 4097), (1030, 1028, 4100), (2047, 516, 3071), (1153, 284, 1602), (1153, 284, 2303), (511, 412, 3202), (1353, 276, 2199), (447, 1060, 3454),
+           (1406, 1252, 961), (1665, 1236, 863), (777, 1028, 4100)]
 # up to eight rows and four outputs a workgroup: 1, 2, 4 and 8 rows' room full and not, outputs that end inside a workgroup, K of less than a thread each,
 # one stretch of 2,048, two, a short one more; and shapes that the rule gives to the tiles
 LINEAR += [(1, 8196, 64), (2, 1028, 3001), (3, 4100, 130), (4, 2048, 1601), (5, 2052, 33), (8, 1024, 777), (7, 4096, 1600), (8, 1020, 40), (4, 1600, 1601), (1, 100, 6401)]
 
-# 64 x 64 straight from memory: rows and outputs that end inside a tile, K with a short last step, of short and long sums
+# 64 x 64 straight from memory: rows and outputs that end inside a tile, K with a short last step (of 256 inputs and more the tiles of split operands have these)
 LINEAR += [(935, 228, 8317), (129, 3396, 4949), (195, 3364, 3558), (777, 4100, 1030)]
 
 
+def _kernel(K, M, Ki, N):
+    """Which kernel runs a product of aligned rows: "split" and the tile, or the place of the 32-bit instruction's kernel."""
+    split = K.lib.lev_linear_f32_split(M, N, Ki)
+    return ("split", split) if split >= 0 else K.lib.lev_linear_f32_choice(M, N, Ki)
+
+
 def test_every_kernel_is_among_the_shapes(K):
-    """Room for 8, 4, 2 and 1 rows (-8 .. -1), seven tiles straight from memory, six through LDS."""
-    assert {K.lib.lev_linear_f32_choice(M, N, Ki) for M, Ki, N in LINEAR if Ki % 4 == 0} == {-8, -4, -2, -1, *range(13)}
+    """Room for 8, 4, 2 and 1 rows (-8 .. -1), seven tiles straight from memory, five through LDS, three of split operands."""
+    assert {_kernel(K, *s) for s in LINEAR if s[1] % 4 == 0} == {-8, -4, -2, -1, *range(12), ("split", 0), ("split", 1), ("split", 2)}
 
 
 @pytest.mark.parametrize("M,Ki,N", LINEAR)
@@ -90,10 +97,12 @@ def test_linear_float32_keeps_infinities_where_they_are(K):
     torch.testing.assert_close(out[keep], want[keep], rtol=1e-5, atol=52 * EPS * 50)
 
 
-@pytest.mark.parametrize("M,Ki,N", [(289, 100, 2051), (609, 516, 2310), (1030, 1028, 4100), (129, 3396, 4949), (1, 8196, 64), (3, 4100, 130), (8, 1028, 777)])
-def test_linear_float32_keeps_infinities_where_they_are_in_every_kernel(K, M, Ki, N):
-    """Tiles through LDS with a short step of one, two and four sums, 64 x 64 straight from memory, and rooms for 1, 4 and 8 rows whose last stretch is short: an infinite last
-    input reaches its own row, an infinite last weight its own output, and nothing else is anything but finite."""
+@pytest.mark.parametrize("kernel,M,Ki,N", [(7, 289, 100, 2051), (9, 609, 516, 2310), (10, 1153, 284, 2303), (11, 1406, 1252, 961), (6, 935, 228, 8317), (-1, 1, 8196, 64), (-4, 3, 4100, 130), (-8, 8, 1028, 777),
+                                           (("split", 1), 1030, 1028, 4100), (("split", 2), 129, 3396, 4949)])
+def test_linear_float32_keeps_infinities_where_they_are_in_every_kernel(K, kernel, M, Ki, N):
+    """Tiles through LDS with a short step of one, two and four sums, 64 x 64 straight from memory, rooms for 1, 4 and 8 rows whose last stretch is short, and tiles of split operands: an infinite
+    last input reaches its own row, an infinite last weight its own output, and nothing else is anything but finite."""
+    assert _kernel(K, M, Ki, N) == kernel
     a, w = _rand(M, Ki, seed=1).to(DEV), _rand(N, Ki, seed=2).to(DEV)
     row, col = M // 2, N // 2
     a[row, Ki - 1] = float("inf")
@@ -156,7 +165,7 @@ def test_split_products_of_the_smallest_and_largest_numbers(K, tile, M, Ki, N):
     assert bool(((got.double() - want.double()).abs() <= (Ki + 6) * EPS * size)[fine].all())
 
 
-@pytest.mark.parametrize("choice,M,Ki,N", [(8, 273, 772, 9001), (9, 129, 516, 9001), (10, 177, 516, 9001), (11, 465, 256, 9001), (12, 417, 772, 9001)])
+@pytest.mark.parametrize("choice,M,Ki,N", [(8, 273, 772, 9001), (9, 129, 516, 9001), (10, 177, 516, 9001), (11, 465, 256, 9001)])
 def test_rows_too_far_apart_to_be_split(K, choice, M, Ki, N):
     """Rows more than 2^22 numbers apart: the tiles through LDS on the 32-bit instruction."""
     assert K.lib.lev_linear_f32_choice(M, N, Ki) == choice

@@ -91,31 +91,31 @@ def test_which_of_the_librarys_kernels_is_kept(keeps, bits, us, kept):
 
 # the 32-bit products, over weights that no cache holds
 TILES = [  # rows, outputs, inputs, microseconds of the tiles in the order of the kernels' two lists
-    (100, 5120, 6400, (203.6, 171.7, 172.8, 180.6, 143.5, 150.0, 112.8, 119.1, 129.8, 129.3, 137.8, 165.4, 205.6)),
-    (203, 3072, 6400, (223.6, 199.9, 175.6, 181.5, 143.9, 147.5, 114.1, 113.5, 125.5, 126.3, 133.5, 163.5, 205.1)),
-    (256, 3072, 4096, (171.0, 132.7, 133.3, 117.1, 94.4, 97.1, 76.3, 75.8, 81.8, 81.9, 84.9, 107.0, 133.8)),
-    (777, 768, 6400, (220.3, 171.0, 172.6, 173.5, 139.5, 139.6, 110.9, 103.7, 117.0, 122.4, 129.8, 162.1, 203.5)),
-    (404, 1600, 4096, (156.0, 127.5, 131.1, 113.9, 91.5, 93.6, 75.0, 70.7, 77.6, 79.3, 83.8, 106.1, 133.8)),
-    (512, 1200, 6400, (221.8, 171.7, 174.0, 174.7, 142.9, 140.0, 112.3, 105.7, 117.7, 122.2, 130.4, 162.5, 204.2)),
-    (160, 4096, 4096, (145.7, 111.9, 113.8, 117.7, 96.2, 97.3, 76.7, 75.3, 82.6, 83.7, 86.7, 106.6, 134.3)),
-    (33, 10240, 2048, (58.2, 57.9, 47.7, 44.9, 49.3, 51.8, 42.5, 43.0, 46.8, 47.2, 49.5, 57.9, 70.8)),
-    (100, 5120, 3072, (99.0, 83.5, 85.3, 89.7, 71.5, 75.0, 59.2, 59.1, 64.4, 64.5, 68.7, 81.9, 102.8)),
-    (1500, 400, 4096, (142.2, 109.5, 110.0, 112.8, 90.7, 90.2, 74.8, 67.5, 77.1, 78.0, 83.8, 105.2, 132.9)),
-    (100, 6400, 3072, (121.6, 115.0, 101.3, 93.9, 93.3, 75.5, 61.0, 67.4, 65.2, 81.0, 69.2, 82.8, 102.7)),
-    (777, 3072, 1024, (132.0, 105.5, 103.6, 102.4, 78.2, 62.2, 66.4, 54.6, 47.5, 53.8, 53.7, 53.5, 68.0)),
-    (404, 768, 3072, (56.8, 51.7, 52.4, 58.5, 46.2, 39.4, 58.3, 49.8, 55.3, 60.9, 65.0, 80.6, 101.0)),
-    (1024, 4096, 4096, (896.8, 680.4, 683.6, 585.4, 467.6, 360.1, 335.2, 347.4, 311.2, 311.7, 266.2, 286.0, 255.4)),
-    (64, 768, 768, (5.5, 6.9, 7.0, 10.5, 8.3, 11.7, 18.8, 10.5, 12.0, 13.9, 16.8, 23.1, 29.0)),
-    (17, 1600, 1600, (8.7, 11.1, 12.3, 19.0, 14.8, 23.1, 30.5, 28.1, 31.6, 35.0, 36.7, 44.3, 54.8)),
-    (203, 2304, 768, (24.8, 20.6, 20.6, 19.8, 15.6, 13.1, 19.4, 15.2, 16.6, 18.4, 19.7, 24.1, 29.7)),
-    (1500, 10240, 1600, (1287.5, 994.4, 999.2, 813.1, 663.3, 532.5, 482.6, 497.8, 432.4, 411.3, 390.7, 407.8, 395.3)),
-    (48, 400, 6400, (25.2, 36.7, 38.8, 68.5, 48.7, 76.4, 108.9, 101.5, 113.0, 124.5, 132.9, 161.6, 202.2)),
-    (777, 25000, 96, (134.3, 161.8, 152.5, 106.5, 86.0, 74.8, 90.6, 58.2, 50.8, 50.6, 49.0, 53.0, 55.7)),
-    (777, 1600, 384, (30.9, 26.3, 25.7, 20.2, 18.6, 18.3, 23.0, 13.5, 14.3, 14.7, 17.0, 14.7, 18.0)),
-    (777, 1024, 4096, (183.3, 149.5, 151.0, 146.5, 117.8, 90.2, 74.2, 80.1, 76.3, 105.2, 84.1, 105.9, 133.7)),
-    (777, 1024, 1024, (47.7, 40.3, 39.6, 41.3, 32.5, 26.5, 23.7, 22.3, 21.4, 29.5, 21.7, 29.9, 38.1)),
-    (777, 50257, 1024, (2115.1, 1670.5, 1652.2, 1539.1, 1188.0, 926.8, 844.0, 833.1, 747.2, 737.3, 706.9, 696.5, 672.6)),
-    (662, 25055, 96, (117.7, 148.5, 145.4, 99.1, 86.6, 77.5, 88.2, 59.4, 54.0, 53.3, 55.3, 58.2, 66.1)),
+    (100, 5120, 6400, (203.6, 171.7, 172.8, 180.6, 143.5, 150.0, 112.8, 119.1, 129.8, 129.3, 137.8, 165.4)),
+    (203, 3072, 6400, (223.6, 199.9, 175.6, 181.5, 143.9, 147.5, 114.1, 113.5, 125.5, 126.3, 133.5, 163.5)),
+    (256, 3072, 4096, (171.0, 132.7, 133.3, 117.1, 94.4, 97.1, 76.3, 75.8, 81.8, 81.9, 84.9, 107.0)),
+    (777, 768, 6400, (220.3, 171.0, 172.6, 173.5, 139.5, 139.6, 110.9, 103.7, 117.0, 122.4, 129.8, 162.1)),
+    (404, 1600, 4096, (156.0, 127.5, 131.1, 113.9, 91.5, 93.6, 75.0, 70.7, 77.6, 79.3, 83.8, 106.1)),
+    (512, 1200, 6400, (221.8, 171.7, 174.0, 174.7, 142.9, 140.0, 112.3, 105.7, 117.7, 122.2, 130.4, 162.5)),
+    (160, 4096, 4096, (145.7, 111.9, 113.8, 117.7, 96.2, 97.3, 76.7, 75.3, 82.6, 83.7, 86.7, 106.6)),
+    (33, 10240, 2048, (58.2, 57.9, 47.7, 44.9, 49.3, 51.8, 42.5, 43.0, 46.8, 47.2, 49.5, 57.9)),
+    (100, 5120, 3072, (99.0, 83.5, 85.3, 89.7, 71.5, 75.0, 59.2, 59.1, 64.4, 64.5, 68.7, 81.9)),
+    (1500, 400, 4096, (142.2, 109.5, 110.0, 112.8, 90.7, 90.2, 74.8, 67.5, 77.1, 78.0, 83.8, 105.2)),
+    (100, 6400, 3072, (121.6, 115.0, 101.3, 93.9, 93.3, 75.5, 61.0, 67.4, 65.2, 81.0, 69.2, 82.8)),
+    (777, 3072, 1024, (132.0, 105.5, 103.6, 102.4, 78.2, 62.2, 66.4, 54.6, 47.5, 53.8, 53.7, 53.5)),
+    (404, 768, 3072, (56.8, 51.7, 52.4, 58.5, 46.2, 39.4, 58.3, 49.8, 55.3, 60.9, 65.0, 80.6)),
+    (1024, 4096, 4096, (896.8, 680.4, 683.6, 585.4, 467.6, 360.1, 335.2, 347.4, 311.2, 311.7, 266.2, 286.0)),
+    (64, 768, 768, (5.5, 6.9, 7.0, 10.5, 8.3, 11.7, 18.8, 10.5, 12.0, 13.9, 16.8, 23.1)),
+    (17, 1600, 1600, (8.7, 11.1, 12.3, 19.0, 14.8, 23.1, 30.5, 28.1, 31.6, 35.0, 36.7, 44.3)),
+    (203, 2304, 768, (24.8, 20.6, 20.6, 19.8, 15.6, 13.1, 19.4, 15.2, 16.6, 18.4, 19.7, 24.1)),
+    (1500, 10240, 1600, (1287.5, 994.4, 999.2, 813.1, 663.3, 532.5, 482.6, 497.8, 432.4, 411.3, 390.7, 407.8)),
+    (48, 400, 6400, (25.2, 36.7, 38.8, 68.5, 48.7, 76.4, 108.9, 101.5, 113.0, 124.5, 132.9, 161.6)),
+    (777, 25000, 96, (134.3, 161.8, 152.5, 106.5, 86.0, 74.8, 90.6, 58.2, 50.8, 50.6, 49.0, 53.0)),
+    (777, 1600, 384, (30.9, 26.3, 25.7, 20.2, 18.6, 18.3, 23.0, 13.5, 14.3, 14.7, 17.0, 14.7)),
+    (777, 1024, 4096, (183.3, 149.5, 151.0, 146.5, 117.8, 90.2, 74.2, 80.1, 76.3, 105.2, 84.1, 105.9)),
+    (777, 1024, 1024, (47.7, 40.3, 39.6, 41.3, 32.5, 26.5, 23.7, 22.3, 21.4, 29.5, 21.7, 29.9)),
+    (777, 50257, 1024, (2115.1, 1670.5, 1652.2, 1539.1, 1188.0, 926.8, 844.0, 833.1, 747.2, 737.3, 706.9, 696.5)),
+    (662, 25055, 96, (117.7, 148.5, 145.4, 99.1, 86.6, 77.5, 88.2, 59.4, 54.0, 53.3, 55.3, 58.2)),
 ]
 # of one to eight rows
 FEW_ROWS = [  # rows, outputs, inputs, microseconds of the few-row kernel and of the tiles
