@@ -165,6 +165,22 @@ def test_split_products_of_the_smallest_and_largest_numbers(K, tile, M, Ki, N):
     assert bool(((got.double() - want.double()).abs() <= (Ki + 6) * EPS * size)[fine].all())
 
 
+@pytest.mark.parametrize("tile,M,Ki,N", [(0, 513, 284, 6401), (1, 609, 516, 3071), (2, 404, 796, 2051)])
+@pytest.mark.parametrize("terms", [1, 2])
+def test_split_products_of_a_few_terms(K, tile, M, Ki, N, terms):
+    """Rows with one and two inputs that are not zero, where no long sum hides a product's own error. Of numbers in [1, 2) the second and third bfloat16 parts are at most 2^-8 and 2^-17,
+    so that the three partial products left out are at most 2^-24 + 2^-34 of a product; the sums' roundings are one for each term and, of the other parts (2^-7), an eighth in all."""
+    assert K.lib.lev_linear_f32_split(M, N, Ki) == tile
+    g = torch.Generator().manual_seed(tile)
+    at = torch.stack([torch.randperm(Ki, generator=g)[:terms] for _ in range(M)])
+    a = torch.zeros(M, Ki).scatter_(1, at, (1 + torch.rand(M, terms, generator=g)) * 2.0 ** torch.randint(-20, 20, (M, terms), generator=g)).to(DEV)
+    w = ((1 + torch.rand(N, Ki, generator=g)) * (torch.randint(0, 2, (N, Ki), generator=g) * 2 - 1)).to(DEV)
+    got = torch.empty(M, N, device=DEV)
+    K.linear(a, w, None, got)
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    assert bool(((got.double() - want).abs() <= (1 + terms + 0.125) * EPS * size).all())
+
+
 @pytest.mark.parametrize("choice,M,Ki,N", [(8, 273, 772, 9001), (9, 129, 516, 9001), (10, 177, 516, 9001), (11, 465, 256, 9001)])
 def test_rows_too_far_apart_to_be_split(K, choice, M, Ki, N):
     """Rows more than 2^22 numbers apart: the tiles through LDS on the 32-bit instruction."""
