@@ -268,6 +268,13 @@ def test_attention_float32_of_many_heads(K, HD, window):
     test_attention_float32(K, 32, 8, HD, 16, [(15, 63), (33, 64), (17, 81), (1, 40)], window)
 
 
+# the same over many rounds of the waves
+@pytest.mark.parametrize("HD", [16, 64, 128])
+@pytest.mark.parametrize("window", [None, 333])
+def test_attention_float32_of_many_heads_over_long_contexts(K, HD, window):
+    test_attention_float32(K, 64, 8, HD, 16, [(18, 611), (2, 1030), (1, 700)], window)
+
+
 # single tokens in workgroups of four waves (head sizes up to 96): more than 256 of them (tokens x key/value heads); key ranges of less than a wave's block of 32 keys to several rounds
 @pytest.mark.parametrize("HD", range(16, 97, 16))
 @pytest.mark.parametrize("window", [None, 50])
@@ -361,3 +368,33 @@ def test_attention_float32_values_outside_the_window_do_not_count(K, bad, HD, H)
     assert bool((~torch.isfinite(heads) == hit).all())
     # the other sums of such a tile go key by key: another order of at most 10 terms of at most 5, each off by 2^-24 of it
     torch.testing.assert_close(heads[~hit], clean.view(T, H, HD)[~hit], rtol=0, atol=10 * 5 * EPS)
+
+
+# more than 384 workgroups of runs and more than 256 of single tokens (head sizes up to 96): four waves each, of single tokens with a sum for each of a block's two tiles of 16 keys. Key 20 stands in the second tile
+# of a window that begins below key 16, in the first of one that begins at 16 to 20, and behind the window of a block's other keys
+@pytest.mark.parametrize("HD,H", [(16, 64), (64, 64), (96, 64)])
+@pytest.mark.parametrize("window", [10, 60])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_attention_float32_values_outside_the_window_do_not_count_in_four_waves(K, bad, window, HD, H):
+    from helpers import make_meta
+    from test_gpu_kernels import _fill_cache
+
+    KVH, PS = 16, 16
+    kv = [90, *range(18, 35), 79, 80, 81, 100]
+    runs = [(90, 90)] + [(1, n) for n in kv[1:]]
+    bt, kp, vp, kd, vd, _, _ = _fill_cache(K, torch.float32, kv, KVH, HD, PS, sum(-(-n // PS) for n in kv) + 3, seed=7)
+    T = sum(n for n, _ in runs)
+    q = _rand(T, H * HD, seed=8).to(DEV)
+    args = dict(n_heads=H, n_kv_heads=KVH, head_dim=HD, page_size=PS, scale=HD ** -0.5, window=window, block_tables=bt.to(DEV))
+    clean, got = torch.empty(T, H * HD, device=DEV), torch.empty(T, H * HD, device=DEV)
+    K.paged_attention(q, clean, kd, vd, make_meta(runs, DEV), **args)
+    for s in range(len(runs)):
+        vd.view(-1, KVH, HD, PS)[int(bt[s, 1]), :, 5, 4] = bad
+    K.paged_attention(q, got, kd, vd, make_meta(runs, DEV), **args)
+    pos = torch.tensor([*range(90), *(n - 1 for n in kv[1:])], device=DEV)
+    hit = torch.zeros(T, H, HD, dtype=torch.bool, device=DEV)
+    hit[(pos >= 20) & (pos < 20 + window), :, 5] = True
+    heads = got.view(T, H, HD)
+    assert bool((~torch.isfinite(heads) == hit).all())
+    # the other sums of such a tile go key by key: another order of at most `window` terms of at most 5, each off by 2^-24 of it
+    torch.testing.assert_close(heads[~hit], clean.view(T, H, HD)[~hit], rtol=0, atol=window * 5 * EPS)
