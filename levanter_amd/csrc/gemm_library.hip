@@ -126,8 +126,8 @@ int tune_level() {
 }
 
 // A buffer larger than the caches (32 MB of L2, 256 MB behind them), one per device, kept for the life of the process:
-// sweeping it between two timed runs leaves nothing of the operands in a cache. It holds pairs of bfloat16 numbers of either sign, 1/4 to 4, all bits
-// of which vary: operands, too, on which the kernels' sums are told apart.
+// sweeping it between two timed runs leaves nothing of the operands in a cache. Ahead of them it holds bfloat16 numbers of either sign, 1/4 to 4, all bits
+// of which vary: operands on which the kernels' sums are told apart.
 #define LEV_LIB_FLUSH_BYTES ((size_t)512 << 20)
 __global__ void __launch_bounds__(256) fill_kernel(uint4* to, uint32_t n) {
   auto mixed = [](uint32_t x) {
@@ -273,7 +273,7 @@ int time_candidates(hipblasLtHandle_t handle, Plan* p, int likely, const void* a
     // of the runs counts.
     for (int r = 0; r < LEV_LIB_TUNE_RUNS && ok; ++r) {
       float t = 0.0f;
-      ok = (!flush || fill(flush, stream)) && hipEventRecord(e0, stream) == hipSuccess && run(i, a, w, residual) && hipEventRecord(e1, stream) == hipSuccess &&
+      ok = (!flush || hipMemsetAsync(flush, r, LEV_LIB_FLUSH_BYTES, stream) == hipSuccess) && hipEventRecord(e0, stream) == hipSuccess && run(i, a, w, residual) && hipEventRecord(e1, stream) == hipSuccess &&
            hipEventSynchronize(e1) == hipSuccess && hipEventElapsedTime(&t, e0, e1) == hipSuccess;
       if (ok && (ms < 0.0f || t < ms)) ms = t;
     }
