@@ -236,7 +236,7 @@ sc_inner_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, co
 // Runs of several tokens begin first: behind 31 single tokens, as a step has them, one of 1,000 would begin last and its chain be the end of the step (with all that stands around the kernel, 16 columns / 64 / 64 and
 // long runs first: 246 / 254 / 188; of 3,000 406 / 484 / 365; 32 of 40 to 150, in a scan that reads every slot once, 386 / 306 / 282). DELTA stays at 16: its products with two 32-bit sides are four times as long.
 template <int DKM, int RULE, bool VEC, int CT>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, (DKM == 64 && CT == 4) || (DKM == 128 && RULE == SR_DELTA && !VEC) ? 2 : 1)  // else 260 and 257 registers would leave one workgroup a CU; others lose 2 - 7 % by the bound
 sc_chunk_kernel(const bf16_t* __restrict__ u, const float* __restrict__ scal, const float* __restrict__ P_in, const float* __restrict__ T_in,
                 const float2* __restrict__ E_in, float* __restrict__ state, const int* __restrict__ token_slots, float* __restrict__ o, SrShape s) {
   constexpr int LDK = DKM + 8, KS = DKM / 32, NTW = DKM / 64, KI = DKM / 64, QI = DKM / 32;
