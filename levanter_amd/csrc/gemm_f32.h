@@ -8,9 +8,11 @@ typedef __attribute__((ext_vector_type(4))) float gf_f32x4;
 #define GEMM_F32_SPLIT_MOST (1 << 22)
 struct GemmF32SplitTile {
   int rows, outputs, groups;   // groups of waves that share the steps of 32 inputs
-  float start, alone, among;   // microseconds: before and behind the products, of a step of the one workgroup on a CU, and of one among several
+  float start, alone, among;   // microseconds: before and behind the products, of a step of the one workgroup on a CU, and of one among several,
+  float odd, single;           // what a step takes longer where the last of several is left alone, and a tile whose outputs are stored one by one (N no multiple of 4)
 };
-static const GemmF32SplitTile GEMM_F32_SPLIT_TILES[] = {{128, 128, 1, 5.789f, 0.998f, 1.051f}, {64, 128, 1, 4.353f, 0.732f, 0.579f}, {64, 64, 2, 4.205f, 0.644f, 1.135f}};
+static const GemmF32SplitTile GEMM_F32_SPLIT_TILES[] = {{128, 128, 1, 5.093f, 1.048f, 1.257f, 0.125f, 2.561f}, {64, 128, 1, 2.216f, 0.768f, 0.689f, 0.256f, 1.586f},
+                                                        {64, 64, 2, 5.049f, 0.651f, 1.132f, 0.052f, 1.553f}};
 #define GEMM_F32_N_SPLIT_TILES (int)(sizeof(GEMM_F32_SPLIT_TILES) / sizeof(GEMM_F32_SPLIT_TILES[0]))
 extern "C" int lev_linear_f32_choice(int M, int N, int K);
 extern "C" int lev_linear_f32_split(int M, int N, int K);

@@ -389,17 +389,19 @@ extern "C" int lev_linear_f32_choice(int M, int N, int K) {
 }
 
 // The tile of the kernel that splits its operands into bfloat16 numbers (gemm_f32_split.hip), or -1 where the kernels above, which take `us` by their estimate, are not behind by an estimate as theirs, fitted
-// to 208 shapes of 70 .. 2,048 rows (0.2 % behind the best on average, 14 % at worst: 2048 x 256 at 1,000 rows 13.4 us, 11.8 with 64 x 128; none behind the kernels above). Below 256
-// inputs those stay ahead of it, or level; and it knows no rows more than GEMM_F32_SPLIT_MOST apart. Kernels above / this one, microseconds: 4096 x 1024 at 777 rows 62 / 47, 1024 x 4096 72 / 63,
-// 50257 x 768 at 300 rows 209 / 166, 4096 x 4096 at 2,048 502 / 366, 1600 x 1600 at 512 34 / 27; not taken: 768 x 3072 at 606 rows 35 / 47, 1024 x 1024 at 404 15 / 19.
+// to 700 shapes of 17 .. 2,200 rows and 256 .. 6,800 inputs: it is taken at 263 of them, the kernels above are up to 2 % faster at five of these, and what is kept is 0.4 % behind the best on average. Outputs
+// that are stored one by one and a last workgroup alone on a CU have their terms: without them 14 of 480 shapes lost 2 - 19 % (50257 x 576 at 92 rows 62 us above, 74 here; 3072 x 1192 at 1,451 91, 97). Below 256
+// inputs the kernels above stay ahead of it, or level; and it knows no rows more than GEMM_F32_SPLIT_MOST apart. Kernels above / this one, microseconds: 4096 x 1024 at 777 rows 64 / 50, 1024 x 4096 74 / 64,
+// 50257 x 768 at 300 rows 209 / 166, 4096 x 4096 at 2,048 502 / 366, 1600 x 1600 at 512 34 / 27; not taken: 768 x 3072 at 606 rows 36 / 46, 1024 x 1024 at 404 15 / 19.
 static int gemm_f32_split_tile(int M, int N, int K, int choice, double us) {
   if (K % 4 != 0 || K < 256 || K > GEMM_F32_SPLIT_MOST || choice < 0) return -1;
-  us *= 0.949;  // the estimates' own errors: of 190 shapes none is slower than before
+  us *= 0.92;  // the estimates' own errors (0.964 would take 20 more of the shapes, two of them 2 - 4 % slower)
   int best = -1;
   for (int i = 0; i < GEMM_F32_N_SPLIT_TILES; ++i) {
     const GemmF32SplitTile& t = GEMM_F32_SPLIT_TILES[i];
     const double n = ceil((double)((M + t.rows - 1) / t.rows) * ((N + t.outputs - 1) / t.outputs) / 256.0);
-    const double own = t.start + fmax(4.0 * N * K / 5.2e6, ((K + 31) / 32 + t.groups - 1) / t.groups * (n <= 1.0 ? t.alone : n * t.among));
+    const double step = n <= 1.0 ? t.alone : n * t.among + fmod(n, 2.0) * t.odd;
+    const double own = t.start + fmax(4.0 * N * K / 5.2e6, ((K + 31) / 32 + t.groups - 1) / t.groups * step) + (N % 4 != 0 ? n * t.single : 0.0);
     if (own < us) us = own, best = i;
   }
   return best;

@@ -98,7 +98,7 @@ def test_linear_float32_keeps_infinities_where_they_are(K):
 
 
 @pytest.mark.parametrize("kernel,M,Ki,N", [(7, 289, 100, 2051), (9, 609, 516, 2310), (10, 1153, 284, 2303), (11, 1406, 1252, 961), (6, 935, 228, 8317), (-1, 1, 8196, 64), (-4, 3, 4100, 130), (-8, 8, 1028, 777),
-                                           (("split", 1), 1030, 1028, 4100), (("split", 2), 129, 3396, 4949)])
+                                           (11, 1030, 1028, 4100), (("split", 1), 513, 516, 6530), (("split", 2), 129, 3396, 4949)])
 def test_linear_float32_keeps_infinities_where_they_are_in_every_kernel(K, kernel, M, Ki, N):
     """Tiles through LDS with a short step of one, two and four sums, 64 x 64 straight from memory, rooms for 1, 4 and 8 rows whose last stretch is short, and tiles of split operands: an infinite
     last input reaches its own row, an infinite last weight its own output, and nothing else is anything but finite."""
@@ -117,8 +117,8 @@ def test_linear_float32_keeps_infinities_where_they_are_in_every_kernel(K, kerne
 
 # products whose operands are split into bfloat16 numbers: tiles of 128 x 128, 64 x 128 and 64 x 64 outputs that end inside a tile, whole steps of 32 inputs, a partial one of 4 and of 28,
 # odd and even numbers of steps, numbers that the two groups of a 64 x 64 tile share unevenly, sums that are joined once and often, and long ones
-SPLIT = [(0, 777, 260, 4097), (0, 513, 284, 6401), (0, 1030, 288, 3071), (0, 1030, 4100, 2051), (1, 1030, 256, 3071), (1, 513, 516, 3071), (1, 257, 540, 6401), (1, 609, 516, 3071), (2, 777, 772, 1030),
-         (2, 100, 1028, 6401), (2, 65, 3396, 6401), (2, 777, 4100, 1030), (2, 404, 796, 2051)]
+SPLIT = [(0, 1025, 260, 3457), (0, 511, 284, 7171), (0, 1151, 288, 3326), (0, 1153, 4100, 2053), (1, 514, 256, 6404), (1, 1410, 256, 8325), (1, 513, 516, 6530), (1, 385, 540, 8831), (1, 385, 284, 4476),
+         (2, 321, 1028, 2244), (2, 127, 1052, 6204), (2, 65, 3396, 5503), (2, 193, 1316, 3582), (2, 66, 4100, 5566), (2, 770, 2052, 961)]
 
 
 @pytest.mark.parametrize("tile,M,Ki,N", SPLIT)
@@ -140,7 +140,7 @@ def test_split_products(K, tile, M, Ki, N):
     assert float((got.double() - exact).norm() / exact.norm()) <= 1.15 * 0.42 * EPS * (64 + Ki / 256) ** 0.5
 
 
-@pytest.mark.parametrize("tile,M,Ki,N", [(0, 513, 284, 6401), (1, 609, 516, 3071), (2, 404, 796, 2051)])
+@pytest.mark.parametrize("tile,M,Ki,N", [(0, 511, 284, 7171), (1, 513, 516, 6530), (2, 193, 1316, 3582)])
 def test_split_products_of_the_smallest_and_largest_numbers(K, tile, M, Ki, N):
     """Powers of two on the operands change nothing, down to numbers whose last bits are the smallest there are and up to the largest, which have no bfloat16 parts."""
     assert K.lib.lev_linear_f32_split(M, N, Ki) == tile
@@ -165,7 +165,7 @@ def test_split_products_of_the_smallest_and_largest_numbers(K, tile, M, Ki, N):
     assert bool(((got.double() - want.double()).abs() <= (Ki + 6) * EPS * size)[fine].all())
 
 
-@pytest.mark.parametrize("tile,M,Ki,N", [(0, 513, 284, 6401), (1, 609, 516, 3071), (2, 404, 796, 2051)])
+@pytest.mark.parametrize("tile,M,Ki,N", [(0, 511, 284, 7171), (1, 513, 516, 6530), (2, 193, 1316, 3582)])
 @pytest.mark.parametrize("terms", [1, 2])
 def test_split_products_of_a_few_terms(K, tile, M, Ki, N, terms):
     """Rows with one and two inputs that are not zero, where no long sum hides a product's own error. Of numbers in [1, 2) the second and third bfloat16 parts are at most 2^-8 and 2^-17,

@@ -117,6 +117,16 @@ TILES = [  # rows, outputs, inputs, microseconds of the tiles in the order of th
     (777, 50257, 1024, (2115.1, 1670.5, 1652.2, 1539.1, 1188.0, 926.8, 844.0, 833.1, 747.2, 737.3, 706.9, 696.5)),
     (662, 25055, 96, (117.7, 148.5, 145.4, 99.1, 86.6, 77.5, 88.2, 59.4, 54.0, 53.3, 55.3, 58.2)),
 ]
+SPLIT = [  # rows, outputs, inputs, microseconds on the 32-bit instruction and of the three tiles of split operands
+    (92, 50257, 576, 62.7, (74.1, 76.1, 99.1)), (149, 8535, 6212, 180.2, (224.9, 205.8, 192.2)), (349, 9882, 256, 22.9, (26.7, 25.8, 36.7)), (548, 7246, 1024, 77.8, (95.2, 87.2, 101.4)),
+    (1254, 3204, 4292, 297.2, (347.1, 326.6, 300.1)), (264, 8243, 680, 37.6, (40.7, 40.5, 46.2)), (1853, 2304, 1972, 144.3, (170.9, 155.5, 178.2)), (1451, 3072, 1192, 92.0, (108.7, 96.7, 119.7)),
+    (1207, 3528, 2292, 168.7, (195.1, 178.2, 197.7)), (860, 6787, 308, 42.7, (51.1, 44.9, 60.8)), (1274, 1200, 6400, 182.2, (222.5, 189.5, 189.5)), (1510, 3072, 720, 58.4, (71.2, 60.6, 82.3)),
+    (777, 4096, 1024, 63.8, (49.8, 53.4, 77.8)), (777, 1024, 4096, 74.3, (144.1, 105.3, 64.0)), (777, 3072, 1024, 47.1, (44.6, 49.1, 58.4)), (777, 1024, 1024, 21.8, (42.4, 29.2, 20.2)),
+    (606, 3072, 768, 29.8, (34.3, 25.6, 31.9)), (2000, 11063, 1600, 563.4, (490.3, 507.7, 694.1)), (925, 2148, 3072, 103.8, (113.0, 92.9, 109.8)), (846, 3072, 900, 49.4, (43.0, 46.2, 55.8)),
+    (1969, 3072, 496, 57.7, (55.8, 48.0, 76.5)), (123, 6191, 3072, 65.2, (115.4, 102.9, 54.5)), (708, 11626, 1244, 199.6, (192.8, 181.1, 231.5)), (2052, 768, 3596, 120.1, (132.2, 107.7, 117.0)),
+    (103, 5451, 3072, 58.8, (114.3, 102.1, 48.8)), (1166, 2262, 3636, 177.7, (150.3, 173.6, 185.3)), (290, 768, 3096, 21.6, (112.5, 87.7, 46.2)), (298, 1024, 1768, 18.9, (67.6, 47.1, 29.0)),
+    (512, 768, 3072, 35.8, (109.3, 83.8, 45.9)), (400, 768, 3072, 35.5, (109.9, 83.7, 45.6)),
+]
 # of one to eight rows
 FEW_ROWS = [  # rows, outputs, inputs, microseconds of the few-row kernel and of the tiles
     (8, 1600, 2048, 12.4, 9.0), (5, 1200, 2048, 11.6, 8.3), (5, 1200, 3072, 12.5, 10.8), (8, 1600, 4096, 14.9, 14.8), (8, 1000, 2048, 7.3, 8.9),
@@ -138,6 +148,13 @@ def test_the_tile_of_a_32_bit_product_is_among_the_fastest(core, M, N, K, us):
     """Within 8 % of the fastest that is no less exact than a split of K in four: 32 x 64 and 32 x 96 tiles (places 8, 9) from 128 inputs on, larger ones from 256."""
     allowed = [t for i, t in enumerate(us) if i < 8 or K >= 256 or (K >= 128 and i < 10)]
     assert us[core.lev_linear_f32_choice(M, N, K)] <= 1.08 * min(allowed)
+
+
+@pytest.mark.parametrize("M,N,K,whole,split", SPLIT)
+def test_operands_are_split_only_where_that_is_faster(core, M, N, K, whole, split):
+    tile = core.lev_linear_f32_split(M, N, K)
+    taken = split[tile] if tile >= 0 else whole
+    assert taken <= 1.02 * whole and taken <= 1.12 * min(whole, *split)
 
 
 @pytest.mark.parametrize("M,N,K,few,tiles", FEW_ROWS)
