@@ -12,12 +12,14 @@
 // so that the bias, one value per row of D^T, is the per-output-column bias of the row-major result.
 #include <hipblaslt/hipblaslt.h>
 #include <hipblaslt/hipblaslt-ext.hpp>
+#include <algorithm>
 #include <chrono>
 
 #include <cstdio>
 #include <cstdlib>
 #include <map>
 #include <mutex>
+#include <string>
 #include <tuple>
 #include <vector>
 
@@ -49,9 +51,13 @@ typedef std::tuple<int, int, int, int, long, long, long, int, int, int> PlanKey;
 std::mutex g_mutex;
 hipblasLtHandle_t g_handle[LEV_LIB_MAX_DEVICES];
 std::map<PlanKey, Plan> g_plans;
-// What timing chose, by PlanKey with the row count replaced by its bucket (rows_bucket): the library's index of the kernel.
-// Row counts of one bucket share it, so a serving run whose steps differ by a few rows times once, not once a row count.
-std::map<PlanKey, int> g_timed_index;
+// What timing chose, by PlanKey with the row count replaced by its bucket (rows_bucket): the library's index of the kernel, the row count it was timed at, and
+// the indices of all kernels that add up in the same order there. Row counts of one bucket share it, so a serving run whose steps differ by a few rows times once, not once a row count.
+struct Kept {
+  int index = -1, rows = 0;
+  std::vector<int> order;
+};
+std::map<PlanKey, Kept> g_kept;
 
 int rows_bucket(int M) { return (M + LEV_LIB_ROW_BUCKET - 1) / LEV_LIB_ROW_BUCKET; }
 
@@ -193,110 +199,182 @@ extern "C" int lev_linear_library_keeps(const unsigned long long* bits, const fl
   return kept ? kept->best : -1;
 }
 
-// Times the plan's candidates on the call's own operands, writing to a buffer of its own (a product into the residual stream
-// adds to its output, so the real output cannot take repeated runs), and gives the plan the one to keep. The heuristic's order
-// is a table look-up by size; on this chip its first kernel is often not the fastest one for the shape at hand.
-// likely: the library's index of a kernel that another row count keeps, or -1 where none has been timed: where all that may be kept add up in one order, only that kernel and the
-// heuristic's first are timed (a kernel that won at 264 rows can lose at 320, where its tiles divide the rows differently), if it is among them.
-// Allocates and synchronises: called only outside a stream capture. Returns the library's index of the kernel kept, or -1.
-int time_candidates(hipblasLtHandle_t handle, Plan* p, int likely, const void* a, long lda, const void* w, const float* bias, const float* residual, long ldr,
-                    void* workspace, int M, int N, int K, long ldo, int out_dtype, hipStream_t stream) {
-  p->timed = true;
-  const std::vector<hipblasLtMatmulHeuristicResult_t>& candidates = p->candidates;
-  const int n = (int)candidates.size();
-  if (n < 2) return -1;
-  auto t_begin = std::chrono::steady_clock::now();
-  const size_t bytes = ((size_t)M * (size_t)ldo * (out_dtype == LEV_F32 ? 4 : 2) + 255) / 256 * 256;
-  void* scratch = nullptr;
+int index_of(hipblasLtMatmulAlgo_t algo) { return hipblaslt_ext::getIndexFromAlgo(algo); }
+
+// Rows of the call that a tile of the kernel has, from its name (_MT<outputs>x<rows>x<depth>_), or 0.
+int tile_rows(hipblasLtHandle_t handle, hipblasLtMatmulAlgo_t algo) {
+  const std::string name = hipblaslt_ext::getSolutionNameFromAlgo(handle, algo);
+  const size_t at = name.find("_MT");
+  int outputs, rows;
+  return at != std::string::npos && sscanf(name.c_str() + at, "_MT%dx%dx", &outputs, &rows) == 2 && rows > 0 ? rows : 0;
+}
+
+// Runs of a plan's candidates on a call's operands, writing to a buffer of their own (a product into the residual stream adds to its output, so the real output
+// cannot take repeated runs). Allocates and synchronises: used only outside a stream capture.
+struct Trial {
+  hipblasLtHandle_t handle;
+  Plan* plan;
+  const void *a, *w;
+  const float *bias, *residual;
+  void* workspace;
+  int M, N, K, out_dtype;
+  long lda, ldr, ldo;
+  hipStream_t stream;
+  void *scratch = nullptr, *flush = nullptr;
+  unsigned long long* sums = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
-  if (hipMalloc(&scratch, bytes + LEV_LIB_CANDIDATES * sizeof(unsigned long long)) != hipSuccess) { (void)hipGetLastError(); return -1; }
-  void* flush = flush_buffer();  // null if it could not be had: the runs are then timed on a warm weight, and all on the call's operands
-  if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
-    (void)hipGetLastError();
-    if (e0) (void)hipEventDestroy(e0);
-    (void)hipFree(scratch);
-    return -1;
-  }
-  const float alpha = 1.0f, beta = residual ? 1.0f : 0.0f;
-  unsigned long long* sums = (unsigned long long*)((char*)scratch + bytes);
-  auto run = [&](int i, const void* a_, const void* w_, const void* c_) {
-    return hipblasLtMatmul(handle, p->desc, &alpha, w_, p->lw, a_, p->la, &beta, residual ? c_ : scratch, p->lc, scratch, p->ld, &candidates[i].algo, workspace,
-                           candidates[i].workspaceSize, stream) == HIPBLAS_STATUS_SUCCESS;
-  };
-  auto bias_at = [&](const void* b) {
-    return !bias || hipblasLtMatmulDescSetAttribute(p->desc, HIPBLASLT_MATMUL_DESC_BIAS_POINTER, &b, sizeof(b)) == HIPBLAS_STATUS_SUCCESS;
-  };
-  // Every kernel once (which loads it), on the buffer's numbers where it has enough of them (the call's may be zeros, on which all are alike): a weight from another place than the
-  // rows, which it may overlap
-  const size_t w_at = ((size_t)1 << 20) + 4096;
-  const bool ours = flush && fill(flush, stream) && ((size_t)M * lda) * 2 <= LEV_LIB_FLUSH_BYTES && w_at + (size_t)N * K * 2 <= LEV_LIB_FLUSH_BYTES &&
-                    (size_t)M * ldr * 4 <= LEV_LIB_FLUSH_BYTES && bias_at(flush);
   unsigned long long bits[LEV_LIB_CANDIDATES];
-  float us[LEV_LIB_CANDIDATES];
-  bool all = hipMemsetAsync(sums, 0, LEV_LIB_CANDIDATES * sizeof(unsigned long long), stream) == hipSuccess;
-  for (int i = 0; i < n; ++i) {
-    us[i] = all && (ours ? run(i, flush, (const char*)flush + w_at, flush) : run(i, a, w, residual)) ? 0.0f : -1.0f;
-    if (us[i] < 0.0f) { (void)hipGetLastError(); continue; }
-    if (out_dtype == LEV_F32) bits_kernel<uint32_t><<<1024, 256, 0, stream>>>((const uint32_t*)scratch, M, N, ldo, sums + i);
-    else bits_kernel<uint16_t><<<1024, 256, 0, stream>>>((const uint16_t*)scratch, M, N, ldo, sums + i);
+  float us[LEV_LIB_CANDIDATES];  // microseconds; 0: ran, not timed; negative: did not run, or is not asked for
+  bool loaded[LEV_LIB_CANDIDATES] = {};
+
+  bool begin() {
+    const size_t bytes = ((size_t)M * (size_t)ldo * (out_dtype == LEV_F32 ? 4 : 2) + 255) / 256 * 256;
+    for (float& t : us) t = -1.0f;
+    if (hipMalloc(&scratch, bytes + sizeof(bits)) != hipSuccess) { (void)hipGetLastError(); scratch = nullptr; return false; }
+    sums = (unsigned long long*)((char*)scratch + bytes);
+    flush = flush_buffer();  // null if it could not be had: the runs are then timed on a warm weight, and all on the call's operands
+    if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) { (void)hipGetLastError(); return false; }
+    return true;
   }
-  all = all && hipMemcpyAsync(bits, sums, sizeof(bits), hipMemcpyDeviceToHost, stream) == hipSuccess && hipStreamSynchronize(stream) == hipSuccess;
-  all = bias_at(bias) && all;
-  // Timed are all whose order of sums may be kept; where that is one order and another row count keeps one of them, two.
-  auto share = [&](int i, int j) { return i != j && us[i] >= 0.0f && us[j] >= 0.0f && bits[i] == bits[j]; };
-  bool shared = false, alone[LEV_LIB_CANDIDATES];
-  for (int i = 0; i < n; ++i) {
-    alone[i] = true;
-    for (int j = 0; j < n; ++j) alone[i] &= !share(i, j);
-    shared |= !alone[i];
+  ~Trial() {
+    if (e0) (void)hipEventDestroy(e0);
+    if (e1) (void)hipEventDestroy(e1);
+    if (!scratch) return;
+    (void)hipStreamSynchronize(stream);
+    (void)hipFree(scratch);
   }
-  int first = -1, known = -1;
-  bool one_order = true;
-  for (int i = 0; i < n; ++i) {
-    if (!all || (shared && alone[i])) us[i] = -1.0f;
-    if (us[i] < 0.0f) continue;
-    if (first < 0) first = i;
-    one_order &= bits[i] == bits[first];
-    hipblasLtMatmulAlgo_t algo = candidates[i].algo;
-    if (likely >= 0 && hipblaslt_ext::getIndexFromAlgo(algo) == likely) known = i;
+  bool run(int i, const void* a_, const void* w_, const void* c_) {
+    const float alpha = 1.0f, beta = residual ? 1.0f : 0.0f;
+    loaded[i] = true;
+    return hipblasLtMatmul(handle, plan->desc, &alpha, w_, plan->lw, a_, plan->la, &beta, residual ? c_ : scratch, plan->lc, scratch, plan->ld, &plan->candidates[i].algo, workspace,
+                           plan->candidates[i].workspaceSize, stream) == HIPBLAS_STATUS_SUCCESS;
   }
-  const bool two = one_order && known >= 0;
-  for (int i = 0; i < n; ++i) {
-    if (us[i] < 0.0f) continue;
-    if (two && i != first && i != known) { us[i] = -1.0f; continue; }
-    if (two && first == known) continue;
-    bool ok = true;
+  bool bias_at(const void* b) {
+    return !bias || hipblasLtMatmulDescSetAttribute(plan->desc, HIPBLASLT_MATMUL_DESC_BIAS_POINTER, &b, sizeof(b)) == HIPBLAS_STATUS_SUCCESS;
+  }
+  // The bits of the given kernels' results, on the buffer's numbers where it has enough of them (the call's may be zeros, on which all are alike): a weight from another place
+  // than the rows, which it may overlap. us becomes 0 where there are some.
+  void tell_apart(const std::vector<int>& which) {
+    const size_t w_at = ((size_t)1 << 20) + 4096;
+    const bool ours = flush && fill(flush, stream) && ((size_t)M * lda) * 2 <= LEV_LIB_FLUSH_BYTES && w_at + (size_t)N * K * 2 <= LEV_LIB_FLUSH_BYTES &&
+                      (size_t)M * ldr * 4 <= LEV_LIB_FLUSH_BYTES && bias_at(flush);
+    bool all = hipMemsetAsync(sums, 0, sizeof(bits), stream) == hipSuccess;
+    for (int i : which) {
+      us[i] = all && (ours ? run(i, flush, (const char*)flush + w_at, flush) : run(i, a, w, residual)) ? 0.0f : -1.0f;
+      if (us[i] < 0.0f) { (void)hipGetLastError(); continue; }
+      if (out_dtype == LEV_F32) bits_kernel<uint32_t><<<1024, 256, 0, stream>>>((const uint32_t*)scratch, M, N, ldo, sums + i);
+      else bits_kernel<uint16_t><<<1024, 256, 0, stream>>>((const uint16_t*)scratch, M, N, ldo, sums + i);
+    }
+    all = all && hipMemcpyAsync(bits, sums, sizeof(bits), hipMemcpyDeviceToHost, stream) == hipSuccess && hipStreamSynchronize(stream) == hipSuccess;
+    all = bias_at(bias) && all;
+    if (!all)
+      for (int i : which) us[i] = -1.0f;
+  }
+  // Every timed run behind a sweep over a buffer larger than the caches: in a model's step a product's weight has not
+  // been touched since the step before, and the kernel that is fastest on a weight that waits in the last-level cache
+  // (what a plain loop over one weight measures) is often not the fastest on one that comes from memory. The fastest
+  // of the runs counts; a kernel's first run loads it and does not.
+  void time(int i) {
+    bool ok = loaded[i] || run(i, a, w, residual);
     float ms = -1.0f;
-    // Every timed run behind a sweep over a buffer larger than the caches: in a model's step a product's weight has not
-    // been touched since the step before, and the kernel that is fastest on a weight that waits in the last-level cache
-    // (what a plain loop over one weight measures) is often not the fastest on one that comes from memory. The fastest
-    // of the runs counts.
-    for (int r = 0; r < LEV_LIB_TUNE_RUNS && ok; ++r) {
+    for (int r = 1; r <= LEV_LIB_TUNE_RUNS && ok; ++r) {
       float t = 0.0f;
-      ok = (!flush || hipMemsetAsync(flush, r, LEV_LIB_FLUSH_BYTES, stream) == hipSuccess) && hipEventRecord(e0, stream) == hipSuccess && run(i, a, w, residual) && hipEventRecord(e1, stream) == hipSuccess &&
-           hipEventSynchronize(e1) == hipSuccess && hipEventElapsedTime(&t, e0, e1) == hipSuccess;
+      ok = (!flush || hipMemsetAsync(flush, r, LEV_LIB_FLUSH_BYTES, stream) == hipSuccess) && hipEventRecord(e0, stream) == hipSuccess && run(i, a, w, residual) &&
+           hipEventRecord(e1, stream) == hipSuccess && hipEventSynchronize(e1) == hipSuccess && hipEventElapsedTime(&t, e0, e1) == hipSuccess;
       if (ok && (ms < 0.0f || t < ms)) ms = t;
     }
     us[i] = ok ? ms * 1000.0f : -1.0f;
-    if (!ok) { (void)hipGetLastError(); (void)hipStreamSynchronize(stream); continue; }
-    if (tune_level() >= 2) {
-      hipblasLtMatmulAlgo_t algo = candidates[i].algo;
-      fprintf(stderr, "linear (library) M=%d N=%d K=%d: candidate %d (kernel %d, bits %016llx) %.1f us\n", M, N, K, i, hipblaslt_ext::getIndexFromAlgo(algo), bits[i], us[i]);
+    if (!ok) { (void)hipGetLastError(); (void)hipStreamSynchronize(stream); return; }
+    if (tune_level() >= 2) fprintf(stderr, "linear (library) M=%d N=%d K=%d: candidate %d (kernel %d) %.1f us\n", M, N, K, i, index_of(plan->candidates[i].algo), us[i]);
+  }
+};
+
+// Gives the plan the kernel to keep. The heuristic's order is a table look-up by size; on this chip its first kernel is often not the fastest one for the shape at hand.
+//
+// known: what another row count of the bucket keeps, or null. All kernels again would be most of a first call's time (12288 x 4096: 17 ms); the order of sums is that which two of
+// the first three kernels of the known order have here too, and only the known kernel, where it has it, and the heuristic's first, where it has too, are timed (a kernel that won at 264 rows can lose at
+// 320, where its tiles divide the rows differently). A kernel with as many rows of tiles as there deals them out as there: where that is so of all that count, nothing is run to tell them apart. All are
+// tried again where the known kernel is not on offer or has another order (the heuristic's first was up to a third slower than the best at 304 and 320 rows of a 1600-wide layer, whose bucket was timed at 272).
+Kept time_candidates(Trial& trial, const Kept* known) {
+  Plan* p = trial.plan;
+  p->timed = true;
+  const std::vector<hipblasLtMatmulHeuristicResult_t>& candidates = p->candidates;
+  const int n = (int)candidates.size();
+  Kept kept;
+  kept.rows = trial.M;
+  if (n < 2) return kept;
+  auto t_begin = std::chrono::steady_clock::now();
+  auto keep = [&](int i) {
+    p->algo = candidates[i].algo;
+    p->workspace = candidates[i].workspaceSize;
+    kept.index = index_of(p->algo);
+    if (tune_level() >= 2)
+      fprintf(stderr, "linear (library) M=%d N=%d K=%d: kept candidate %d after %.1f ms\n", trial.M, trial.N, trial.K, i,
+              std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_begin).count());
+    return kept;
+  };
+  auto place = [&](int index) {
+    for (int i = 0; i < n; ++i)
+      if (index_of(candidates[i].algo) == index) return i;
+    return -1;
+  };
+  std::vector<int> members;  // of the known order
+  if (known)
+    for (size_t j = 0; j < known->order.size() && members.size() < 3; ++j)
+      if (const int i = place(known->order[j]); i >= 0) members.push_back(i);
+  const int theirs = known ? place(known->index) : -1;
+  bool begun = false;
+  if (theirs >= 0 && members.size() >= 2) {
+    auto alike = [&](int i) {
+      const int t = tile_rows(trial.handle, candidates[i].algo);
+      return t > 0 && (trial.M + t - 1) / t == (known->rows + t - 1) / t;
+    };
+    bool all = alike(theirs), they = all, first = false;  // the known kernel has the order here, the heuristic's first has
+    for (int i : members) all &= alike(i);
+    if (all) {
+      first = std::find(known->order.begin(), known->order.end(), index_of(candidates[0].algo)) != known->order.end() && alike(0);
+    } else {
+      they = false;
+      if (!(begun = trial.begin())) return kept;
+      std::vector<int> which = members;
+      for (int i : {theirs, 0})
+        if (std::find(which.begin(), which.end(), i) == which.end()) which.push_back(i);
+      trial.tell_apart(which);
+      auto same = [&](int i, int j) { return trial.us[i] >= 0.0f && trial.us[j] >= 0.0f && trial.bits[i] == trial.bits[j]; };
+      for (size_t j = 0; j + 1 < members.size() && !they; ++j)
+        for (size_t k = j + 1; k < members.size() && !they; ++k)
+          if (same(members[j], members[k])) they = same(theirs, members[j]), first = same(0, members[j]);
+    }
+    if (they && (!first || theirs == 0)) return keep(theirs);
+    if (they) {
+      if (!begun && !(begun = trial.begin())) return kept;
+      trial.time(theirs), trial.time(0);
+      const float x = trial.us[theirs], y = trial.us[0];
+      if (x >= 0.0f || y >= 0.0f) return keep(y < 0.0f || (x >= 0.0f && x <= y) ? theirs : 0);
+      return kept;
     }
   }
-  const int best = lev_linear_library_keeps(bits, us, n);
-  if (best >= 0) {
-    p->algo = candidates[best].algo;
-    p->workspace = candidates[best].workspaceSize;
-    if (tune_level() >= 2)
-      fprintf(stderr, "linear (library) M=%d N=%d K=%d: kept candidate %d after %.1f ms\n", M, N, K, best,
-              std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_begin).count());
+  if (!begun && !(begun = trial.begin())) return kept;
+  std::vector<int> which;
+  for (int i = 0; i < n; ++i) which.push_back(i);
+  trial.tell_apart(which);
+  bool shared = false, alone[LEV_LIB_CANDIDATES];
+  for (int i = 0; i < n; ++i) {
+    alone[i] = true;
+    for (int j = 0; j < n; ++j) alone[i] &= !(i != j && trial.us[i] >= 0.0f && trial.us[j] >= 0.0f && trial.bits[i] == trial.bits[j]);
+    shared |= !alone[i];
   }
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  (void)hipStreamSynchronize(stream);
-  (void)hipFree(scratch);
-  return best >= 0 ? hipblaslt_ext::getIndexFromAlgo(p->algo) : -1;
+  bool ran[LEV_LIB_CANDIDATES];
+  for (int i = 0; i < n; ++i) {
+    ran[i] = trial.us[i] >= 0.0f;
+    if (ran[i] && shared && alone[i]) trial.us[i] = -1.0f;  // not to be kept
+    else if (ran[i]) trial.time(i);
+  }
+  const int best = lev_linear_library_keeps(trial.bits, trial.us, n);
+  if (best < 0) return kept;
+  for (int i = 0; i < n; ++i)
+    if (ran[i] && trial.bits[i] == trial.bits[best]) kept.order.push_back(index_of(candidates[i].algo));
+  return keep(best);
 }
 
 // The kernel that timing chose for another row count of the plan's bucket, if the heuristic offers it for this row count
@@ -350,15 +428,16 @@ extern "C" int lev_linear_library(const void* a, long lda, const void* w, const 
     if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) { (void)hipGetLastError(); capturing = hipStreamCaptureStatusActive; }
     const bool may_time = capturing == hipStreamCaptureStatusNone;
     const PlanKey bucket(dev, rows_bucket(M), N, K, lda, residual ? ldr : 0, ldo, (int)epilogue, out_dtype, residual ? 1 : 0);
-    auto known = g_timed_index.find(bucket);
+    auto known = g_kept.find(bucket);
     if (may_time) {
-      const int index = time_candidates(handle, &plan, known == g_timed_index.end() ? -1 : known->second, a, lda, w, bias, residual, ldr, workspace, M, N, K, ldo, out_dtype, stream);
-      if (known == g_timed_index.end()) g_timed_index[bucket] = index;
+      Trial trial{handle, &plan, a, w, bias, residual, workspace, M, N, K, out_dtype, lda, ldr, ldo, stream};
+      Kept kept = time_candidates(trial, known == g_kept.end() ? nullptr : &known->second);
+      if (known == g_kept.end()) g_kept[bucket] = kept;
     } else {
       plan.timed = true;  // recorded into a graph with the heuristic's first kernel, or the one its bucket keeps: eager calls of this shape keep it
                           // too, so that a replay and an eager run of the same product give the same bits
-      if (known != g_timed_index.end() && known->second >= 0)
-        if (const hipblasLtMatmulHeuristicResult_t* theirs = candidate_of_index(&plan, known->second)) {
+      if (known != g_kept.end() && known->second.index >= 0)
+        if (const hipblasLtMatmulHeuristicResult_t* theirs = candidate_of_index(&plan, known->second.index)) {
           plan.algo = theirs->algo;
           plan.workspace = theirs->workspaceSize;
         }
