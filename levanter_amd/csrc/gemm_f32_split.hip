@@ -193,7 +193,8 @@ gemm_f32_split_kernel(const float* __restrict__ a, long lda, const float* __rest
 #pragma unroll
   for (int i = 0; i < RT * NT * 16; ++i) sum[i / 16 / NT][i / 16 % NT][i % 16] *= GS_DOWN;
   // An infinity or NaN has no parts: every sum that it meets comes out infinite or NaN, and so does no sum of finite numbers unless it is too large. A wave with
-  // such a sum multiplies its tiles again, as they are, on the 32-bit instruction.
+  // such a sum multiplies its tiles again, as they are, on the 32-bit instruction, from memory: slow, for what no working model has (4096 x 1024 at 777 rows 53 us, with one infinite input 112, with all sums
+  // beyond 2^80, which the scaled parts cannot hold, 152; the 32-bit kernels 73 either way).
   bool finite = true;
 #pragma unroll
   for (int i = 0; i < RT * NT * 16; ++i) finite &= fabsf(sum[i / 16 / NT][i / 16 % NT][i % 16]) < INFINITY;
